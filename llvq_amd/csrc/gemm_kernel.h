@@ -204,21 +204,6 @@ struct SliceWalk {
   uint32_t piece;               // which of the band's partial sums this workgroup's run of slices feeds
 };
 
-// Stage timestamps of tuning builds (-DLLVQ_PHASE_TIMING): lane 0 of EVERY wavefront stores the realtime counter at
-// the boundaries of the workgroup's stage kGemmStampStage.  Producers: 0 stage begins, 1 its share of the slice
-// unranked, 2 its share of the next slice classified, 3 through the barrier.  Consumers: 0 stage begins, 1 its K-steps
-// multiplied, 3 through the barrier.
-#ifdef LLVQ_PHASE_TIMING
-constexpr uint32_t kGemmStampStage = 3;
-__device__ unsigned long long g_gemm_stamps[1024 * 16 * 4];
-#define LLVQ_GSTAMP(k)                                                                                                 \
-  do {                                                                                                                 \
-    if (lane == 0 && stage_no == kGemmStampStage) g_gemm_stamps[((size_t)blockIdx.x * 16 + wave) * 4 + (k)] = wall_clock64(); \
-  } while (0)
-#else
-#define LLVQ_GSTAMP(k) do {} while (0)
-#endif
-
 // A launch covers up to four matrices that share their activations (q/k/v, gate/up): their
 // bands are numbered through, matrix i owning bands [band_begin, next band_begin).
 constexpr int kGemmMaxGroup = 4;
@@ -400,22 +385,12 @@ __global__ __launch_bounds__(kWgThreads) void gemm_tiles_kernel(GemmArgs a) {
     classify(view(w0, 0));
     wg_barrier();
     uint32_t g = 0;
-#ifdef LLVQ_PHASE_TIMING
-    uint32_t stage_no = 0;
-#endif
     while (live(w0)) {
-#ifdef LLVQ_PHASE_TIMING
-      ++stage_no;
-#endif
-      LLVQ_GSTAMP(0);
       if (live(w2)) stage_raw((g + 2u) % 3u, pre);
       prefetch(w3, pre);
       unrank(view(w0, g));
-      LLVQ_GSTAMP(1);
       if (live(w1)) classify(view(w1, g + 1u));
-      LLVQ_GSTAMP(2);
       wg_barrier();
-      LLVQ_GSTAMP(3);
       ++g;
       w0 = w1;
       w1 = w2;
@@ -494,14 +469,7 @@ __global__ __launch_bounds__(kWgThreads) void gemm_tiles_kernel(GemmArgs a) {
           for (int j = 0; j < 16; ++j) acc[rt][ct][j] = 0.f;
     };
     clear_acc();
-#ifdef LLVQ_PHASE_TIMING
-    uint32_t stage_no = 1;
-#endif
     while (live(w)) {
-#ifdef LLVQ_PHASE_TIMING
-      ++stage_no;
-#endif
-      LLVQ_GSTAMP(0);
       const bool last_of_unit = w.si + 1 == w.run_len;  // the band ends, or this workgroup's share of it
       // The loads run ahead into the unit's next slice.  At the unit's end they re-read this
       // slice (the ring starts afresh behind the epilogue, which needs the registers).
@@ -555,9 +523,7 @@ __global__ __launch_bounds__(kWgThreads) void gemm_tiles_kernel(GemmArgs a) {
             ring[1][ct][f] = t;
           }
       }
-      LLVQ_GSTAMP(1);
       consumer_barrier();
-      LLVQ_GSTAMP(3);
 
       const SliceWalk done = w;
       advance(w);

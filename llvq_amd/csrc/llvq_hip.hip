@@ -1,10 +1,7 @@
 // C ABI and gfx950 kernels of the fused Leech-lattice dequant-GEMV.
 //
-// Data layout in HBM, per matrix: the packed code stream exactly as the file
-// holds it (6 bytes per block, big-endian (idx << 1) | gain, rows
-// back to back), f32 row scales, f32 tail columns, two f32 gain centroids.
-// Per runtime: one 45 KB table image (Golay words, class records, class ends,
-// reciprocals) that every workgroup copies into LDS.
+// Data in HBM, per matrix: the lattice points of its code stream as tiles of 13 bytes per block, with the row scales and
+// tail columns (tiles.h; the stream is unranked once, at upload).  Per runtime: the tables of the unranking.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <type_traits>
@@ -128,18 +125,6 @@ __device__ __forceinline__ float wave_sum(float v) {
          __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32)) + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
 }
 
-// Inclusive prefix sum over the wavefront's lanes: four shifts inside each row of 16 lanes, then the
-// rows' totals are handed on (row 0 to row 1 and row 2 to row 3, then rows 0-1 to rows 2-3).
-__device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t v) {
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true);  // row_shr:1
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true);  // row_shr:2
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true);  // row_shr:4
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true);  // row_shr:8
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, true);  // row_bcast:15 into rows 1 and 3
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, true);  // row_bcast:31 into rows 2 and 3
-  return v;
-}
-
 constexpr uint32_t kDenseBits = 49;  // bits per block at shell cap 13: a 48-bit index and the gain bit
 
 // ---- parity probe: unrank records to points -----------------------------------
@@ -185,47 +170,10 @@ __global__ __launch_bounds__(256) void decode_blocks_kernel(GlobalTables g, cons
   }
 }
 
-// ---- fused dequant-GEMV ---------------------------------------------------------
-// One persistent 1024-lane workgroup per CU.  The rows of up to four matrices
-// that share an activation are cut into tiles of at most kTileBlocks blocks; a
-// workgroup takes tiles round-robin and runs four phases on each:
-//   P0  every lane loads its own four consecutive 6-byte records from HBM into
-//       registers (issued a tile ahead; the records never pass through LDS);
-//   P1  the lane parses them, finds each block's class (two table probes and a
-//       comparison) and queues the block with its rank within the class: odd
-//       coset, even coset, and even-coset classes with a second free kind each
-//       have a queue, because they are different straight-line programs and
-//       binning keeps every lane of a wavefront on the same one; blocks of the
-//       rare generic classes go to two small side queues;
-//   P2  wavefronts take 64 queued blocks at a time, unrank them to 8-bit
-//       coordinates, reduce them against the activation with integer dot
-//       products and write one partial sum per block;
-//   P3  sixteen lanes per row add the row's partial sums in a fixed order,
-//       apply the row scale and the tail columns, and store y.
-// Results do not depend on the queue order, so they are reproducible.
-//
-// The activation is held in LDS as block-scaled fixed point: per 24-column
-// block a power-of-two scale and three signed byte planes (x = scale *
-// (65536 d2 + 256 d1 + d0), |65536 d2 + ...| <= 2^22), i.e. every binary16
-// value within 2^12 of its block's largest is exact and the rest round at
-// 2^-23 of that largest.  Integer sums of 24 products are exact; the three
-// plane sums are combined and scaled in f32.
+// ---- what the product kernels share -----------------------------------------------
 constexpr int kWgThreads = 1024;
-constexpr int kWaves = kWgThreads / 64;
-constexpr int kTileBlocks = 4096;  // default tile capacity; the kernel is instantiated per capacity
 constexpr int kMaxGroup = 4;
-constexpr int kPlaneDwords = 18;  // 3 planes x 6 dwords per 24-column block
 constexpr int kGenericSlots = 64; // queue of blocks that take the generic walk
-
-struct MatArg {
-  const uint8_t* codes;
-  const float* rscale;
-  const float* tail;
-  void* y;
-  float g0, g1;
-  uint32_t d_out;
-  uint32_t tile_begin;  // first tile of this matrix in the launch
-};
 
 // What a launch may do to produce its activation before the product.
 enum : uint32_t {
@@ -235,26 +183,21 @@ enum : uint32_t {
                            // x[i] = f16(r / sqrt(mean(r^2) + eps) * norm_w[i])  (model.rs:781, :827-829)
 };
 
-struct GroupArgs {
-  GlobalTables tables;
+// Where a launch's activation comes from, and what it may do to produce it before the product.
+struct ActivationIn {
   const __half* x;
   const float* x_f32;  // when set, the activation is these f32 values (a rotated activation) and x is unused
   const __half* x2;
   const __half* norm_w;
-  __half* resid_out;  // written by workgroup 0 only; must not alias x
+  __half* resid_out;   // written by workgroup 0 only; must not alias x
   float eps;
-  uint32_t prologue;
-  uint32_t nblocks, tail_w, n_mats, rows_per_tile, n_tiles;
-  float inv_nblocks;  // 1 / nblocks, for the block -> column split
-  // the basis of these matrices, when they are stored rotated and the launch rotates its
-  // own activation (rot_m = 0: no rotation; see rotate_lds)
+  uint32_t prologue;   // kPrologue*
+  // the basis of the matrices, when they are stored rotated and the launch rotates its own activation (see rotate_lds)
   const uint32_t* rot_signbits;
   const float* rot_small;
   float rot_inv;
   uint32_t rot_m, rot_k;
-  MatArg m[kMaxGroup];
 };
-
 
 // x <- (S (x) I_m)(I_k (x) H_m / sqrt m) x in place on n = k m f32 values in LDS whose
 // signs D are already applied (llvq-quant/src/rotation.rs:97-105; f32 like the reference's
@@ -365,18 +308,6 @@ __device__ __forceinline__ void rotate_lds(float* v, uint32_t n, uint32_t m, uin
   }
 }
 
-constexpr int kSmallTileBlocks = 2048;  // tile of the variant for rows too wide for the full tile's LDS
-constexpr int kSecSlots = 384;          // queue of even-coset blocks whose class has a second free kind (7.6 % of uniform draws)
-// Per queue slot an 8-byte entry and its 2-byte block number, per tile slot a partial sum; the 32
-// bytes between them keep the area at least as large as a derived activation's staging needs it
-// (see prologue_fits / rotation_fits).
-__host__ __device__ constexpr size_t gemv_stage_bytes(uint32_t tile) { return ((size_t)tile + kSecSlots) * 10 + 32 + (size_t)tile * 4; }
-__host__ __device__ constexpr size_t gemv_lds_bytes(uint32_t nblocks, uint32_t tile = kTileBlocks,
-                                                    size_t image_bytes = kLdsImageBytes) {
-  return image_bytes + (size_t)nblocks * (kPlaneDwords + 1) * 4 + (32 + (nblocks & 1u)) * 4 + gemv_stage_bytes(tile) +
-         2 * (size_t)kGenericSlots * 10 + 32;
-}
-
 template <typename OutT>
 __device__ __forceinline__ void store_out(void* y, uint32_t r, float v);
 template <>
@@ -406,248 +337,6 @@ __device__ __forceinline__ void store_half(__half* p, __half v) {
   else
     *p = v;
 }
-
-// One 24-column block of the activation -> scale and byte planes.
-template <bool kDeviceScope = false>
-__device__ __forceinline__ void load_block_f16(const __half* x, float (&v)[kDim]) {
-  if constexpr (kDeviceScope) {
-    if ((reinterpret_cast<uintptr_t>(x) & 3) == 0) {
-      const uint32_t* src = reinterpret_cast<const uint32_t*>(x);
-#pragma unroll
-      for (int k = 0; k < kDim / 2; ++k) {
-        const uint32_t w = __hip_atomic_load(src + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        v[2 * k] = __half2float(__ushort_as_half((unsigned short)(w & 0xFFFFu)));
-        v[2 * k + 1] = __half2float(__ushort_as_half((unsigned short)(w >> 16)));
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < kDim; ++j) v[j] = __half2float(load_half<true>(x + j));
-    }
-    return;
-  }
-  if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-    const uint4* src = reinterpret_cast<const uint4*>(x);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const uint4 u = src[k];
-      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[8 * k + 2 * j] = __half2float(__ushort_as_half((unsigned short)(w[j] & 0xFFFFu)));
-        v[8 * k + 2 * j + 1] = __half2float(__ushort_as_half((unsigned short)(w[j] >> 16)));
-      }
-    }
-  } else {  // the activation of a batched row need not be 16-byte aligned
-#pragma unroll
-    for (int j = 0; j < kDim; ++j) v[j] = __half2float(x[j]);
-  }
-}
-
-// PLANES = 3: x = scale (65536 d2 + 256 d1 + d0), |...| <= 2^22, for results stored as f32; PLANES = 2: x = scale (256 d1 + d0),
-// |...| <= 2^14, for results stored as binary16 — an activation is then rounded at 2^-15 of its block's largest value,
-// a sixteenth of the half ulp the stored result carries anyway, and a block costs a third fewer dot products.
-template <int PLANES>
-__device__ __forceinline__ void quantize_values(const float (&v)[kDim], uint32_t* planes, float* scale);
-
-template <int PLANES>
-__device__ __forceinline__ void quantize_block(const __half* x, uint32_t* planes, float* scale) {
-  float v[kDim];
-  load_block_f16(x, v);
-  quantize_values<PLANES>(v, planes, scale);
-}
-
-// f32 activation (a rotated one, fused_cuda.rs:384): same block-scaled fixed point
-template <int PLANES>
-__device__ __forceinline__ void quantize_block_f32(const float* x, uint32_t* planes, float* scale) {
-  float v[kDim];
-#pragma unroll
-  for (int j = 0; j < kDim; ++j) v[j] = x[j];
-  quantize_values<PLANES>(v, planes, scale);
-}
-
-template <int PLANES>
-__device__ __forceinline__ void quantize_values(const float (&v)[kDim], uint32_t* planes, float* scale) {
-  static_assert(PLANES == 2 || PLANES == 3, "two or three byte planes");
-  constexpr int kBits = PLANES == 3 ? 22 : 14;
-  float amax = 0.f;
-#pragma unroll
-  for (int j = 0; j < kDim; ++j) amax = fmaxf(amax, fabsf(v[j]));
-  bool bad = false;
-#pragma unroll
-  for (int j = 0; j < kDim; ++j) bad |= !(fabsf(v[j]) <= 3.4028234e38f);  // inf or NaN
-  int e = 0;
-  (void)frexpf(amax, &e);  // amax = m 2^e, m in [0.5, 1)
-  const float up = ldexpf(1.f, kBits - e);
-  *scale = bad ? __builtin_nanf("") : (amax == 0.f ? 0.f : ldexpf(1.f, e - kBits));
-  uint32_t p0[6], p1[6], p2[6];
-#pragma unroll
-  for (int q = 0; q < 6; ++q) p0[q] = p1[q] = p2[q] = 0;
-#pragma unroll
-  for (int j = 0; j < kDim; ++j) {
-    const int xq = (amax == 0.f || bad) ? 0 : (int)rintf(v[j] * up);  // |xq| <= 2^kBits
-    const int d0 = (int)(int8_t)(xq & 0xFF);
-    const int x1 = (xq - d0) >> 8;
-    const int d1 = (int)(int8_t)(x1 & 0xFF);
-    const int d2 = (x1 - d1) >> 8;  // zero with two planes: |x1| <= 64
-    p0[j >> 2] |= (uint32_t)(d0 & 0xFF) << (8 * (j & 3));
-    p1[j >> 2] |= (uint32_t)(d1 & 0xFF) << (8 * (j & 3));
-    p2[j >> 2] |= (uint32_t)(d2 & 0xFF) << (8 * (j & 3));
-  }
-#pragma unroll
-  for (int q = 0; q < 6; ++q) {
-    planes[q] = p0[q];
-    planes[6 + q] = p1[q];
-    if (PLANES == 3) planes[12 + q] = p2[q];
-  }
-}
-
-template <int PLANES>
-__device__ __forceinline__ float planes_to_float(int d0, int d1, int d2) {
-  if (PLANES == 2) return fmaf((float)d1, 256.f, (float)d0);
-  return fmaf((float)d2, 65536.f, fmaf((float)d1, 256.f, (float)d0));
-}
-
-__device__ __forceinline__ void tile_of(const GroupArgs& a, uint32_t tile, MatArg& M, uint32_t& r0, uint32_t& rows) {
-  M = a.m[0];  // constant indices only: a dynamic one would move the arguments to scratch
-#pragma unroll
-  for (uint32_t k = 1; k < kMaxGroup; ++k)
-    if (k < a.n_mats && tile >= a.m[k].tile_begin) M = a.m[k];
-  r0 = (tile - M.tile_begin) * a.rows_per_tile;
-  rows = min(a.rows_per_tile, M.d_out - r0);
-}
-
-// A lane's share of a tile's code bytes: NB consecutive 6-byte records, 3 NB / 2 dwords, from the
-// byte the first of them starts at.  A tile starts on a row boundary, i.e. at an even byte (a
-// multiple of four whenever rows-per-tile x blocks-per-row is even), so these are vector loads at
-// two- or four-byte alignment; consecutive lanes read consecutive memory.  Unconditional: a lane
-// past the tile's end reads the tile's first records again and ignores them — a guarded load is
-// merged with the register's old value at once, and that merge waits for the load.
-template <int NB>
-struct LaneRecords {
-  static_assert(NB == 2 || NB == 4, "a lane takes two or four records");
-  uint32_t w[NB * 3 / 2];
-};
-typedef uint32_t dwords4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t dwords3_a2 __attribute__((ext_vector_type(3), aligned(2)));
-typedef uint32_t dwords2_a2 __attribute__((ext_vector_type(2), aligned(2)));
-template <int NB>
-__device__ __forceinline__ void prefetch_records(const GroupArgs& a, uint32_t tile, uint32_t tid, LaneRecords<NB>& r) {
-  if (tile >= a.n_tiles || a.nblocks == 0) return;  // rows of tail columns only have no code bytes
-  MatArg M;
-  uint32_t r0, rows;
-  tile_of(a, tile, M, r0, rows);
-  // a lane whose records all lie past the tile's end re-reads the tile's first ones: every byte read lies
-  // inside the tile or within 6 NB bytes behind it, which the 64 bytes of slack behind a matrix's last
-  // record cover
-  const uint32_t share = (uint32_t)NB * 6u;
-  const uint32_t at = tid * (uint32_t)NB < rows * a.nblocks ? tid * share : 0u;
-  const uint8_t* src = M.codes + (size_t)r0 * a.nblocks * 6 + at;
-  // streaming loads: the code bytes are read once
-  if constexpr (NB == 4) {
-    const dwords4_a2 lo = __builtin_nontemporal_load(reinterpret_cast<const dwords4_a2*>(src));
-    const dwords2_a2 hi = __builtin_nontemporal_load(reinterpret_cast<const dwords2_a2*>(src + 16));
-    r.w[0] = lo.x; r.w[1] = lo.y; r.w[2] = lo.z; r.w[3] = lo.w; r.w[4] = hi.x; r.w[5] = hi.y;
-  } else {
-    const dwords3_a2 v = __builtin_nontemporal_load(reinterpret_cast<const dwords3_a2*>(src));
-    r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z;
-  }
-}
-
-// Record j of a lane's share as the 48-bit big-endian number it is: one byte permute for its
-// low 32 bits, one for its high 16.
-template <int NB>
-__device__ __forceinline__ void lane_record(const LaneRecords<NB>& r, int j, uint32_t& lo32, uint32_t& hi16) {
-  const int d = 3 * (j / 2) + (j & 1);
-  const uint32_t a = r.w[d], b = r.w[d + 1];  // the record's bytes lie in these two dwords
-  if (j & 1) {  // starts at byte 2 of a
-    lo32 = __builtin_amdgcn_perm(b, a, 0x04050607u);
-    hi16 = __builtin_amdgcn_perm(b, a, 0x0c0c0203u);
-  } else {      // starts at byte 0 of a
-    lo32 = __builtin_amdgcn_perm(b, a, 0x02030405u);
-    hi16 = __builtin_amdgcn_perm(b, a, 0x0c0c0001u);
-  }
-}
-
-// ---- records of the cap-13 ball: 49 bits per block in a dense stream -------------------------------
-// At shell cap 13 an index takes 48 bits (N(13) < 2^48), so a block is 49 bits — index, then the gain bit,
-// most significant bit first — and blocks follow one another without padding (llvq-search/src/pack.rs:48-82,
-// llvq-artifact/src/format.rs:87-89): block b of a matrix starts at bit 49 b of its code stream.  A lane takes
-// four consecutive blocks, 196 bits, from the eight dwords that hold them: the stream position of its first
-// block, cut to a dword boundary, plus the bits `s0` left over.  Unconditional loads, as for the 6-byte records:
-// a lane past the tile's end reads the tile's first blocks again; every byte read lies inside the tile or within
-// 32 bytes behind it, which the slack behind a matrix's code stream covers.
-struct DenseRecords {
-  uint32_t w[8];
-  uint32_t s0;  // bits of w[0] ahead of the lane's first block (0..31)
-};
-typedef uint32_t dwords4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ void prefetch_records(const GroupArgs& a, uint32_t tile, uint32_t tid, DenseRecords& r) {
-  if (tile >= a.n_tiles || a.nblocks == 0) return;
-  MatArg M;
-  uint32_t r0, rows;
-  tile_of(a, tile, M, r0, rows);
-  const uint64_t tile_bit = (uint64_t)r0 * a.nblocks * kDenseBits;    // the tile's first bit in the matrix's stream
-  const uint64_t tile_base = (tile_bit >> 3) & ~(uint64_t)3;           // ... cut to a dword
-  const uint32_t rem = (uint32_t)(tile_bit - 8u * tile_base);           // 0..31
-  const uint32_t first = tid * 4u < rows * a.nblocks ? tid * 4u : 0u;  // the lane's first block in the tile
-  const uint32_t lane_bit = rem + first * kDenseBits;
-  const uint8_t* src = M.codes + tile_base + (size_t)(lane_bit >> 5) * 4;
-  const dwords4_a4 lo = __builtin_nontemporal_load(reinterpret_cast<const dwords4_a4*>(src));
-  const dwords4_a4 hi = __builtin_nontemporal_load(reinterpret_cast<const dwords4_a4*>(src + 16));
-  r.w[0] = lo.x; r.w[1] = lo.y; r.w[2] = lo.z; r.w[3] = lo.w; r.w[4] = hi.x; r.w[5] = hi.y; r.w[6] = hi.z; r.w[7] = hi.w;
-  r.s0 = lane_bit & 31u;
-}
-
-// The index (ilo, ihi) and gain bit of record i of a lane's share.  6-byte records: 47 bits of index.
-template <int NB>
-__device__ __forceinline__ const LaneRecords<NB>& prepared_records(const LaneRecords<NB>& rec) { return rec; }
-template <int NB>
-__device__ __forceinline__ void record_index(const LaneRecords<NB>& rec, int i, uint32_t& ilo, uint32_t& ihi, uint32_t& gain) {
-  uint32_t lo32, hi16;
-  lane_record(rec, i, lo32, hi16);
-  gain = lo32 & 1u;
-  ilo = __builtin_amdgcn_alignbit(hi16, lo32, 1);
-  ihi = hi16 >> 1;
-}
-// 49-bit blocks: the dwords become big-endian words and the lane's bits are moved to the front of them, once;
-// block j is then the 49 bits from bit 49 j on.  48 bits of index.
-struct DenseWords {
-  uint32_t n[7];
-};
-__device__ __forceinline__ DenseWords prepared_records(const DenseRecords& rec) {
-  uint32_t be[8];
-  DenseWords d;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) be[i] = __builtin_bswap32(rec.w[i]);
-#pragma unroll
-  for (int i = 0; i < 7; ++i) d.n[i] = (uint32_t)((((uint64_t)be[i] << 32) | be[i + 1]) >> (32u - rec.s0));
-  return d;
-}
-__device__ __forceinline__ void record_index(const DenseWords& r, int j, uint32_t& ilo, uint32_t& ihi, uint32_t& gain) {
-  constexpr uint32_t kW = kDenseBits;
-  const int d = (int)(kW * (uint32_t)j) >> 5;
-  const uint32_t sh = (kW * (uint32_t)j) & 31u;
-  const uint64_t top = (((uint64_t)r.n[d] << 32) | r.n[d + 1]);
-  const uint64_t x = sh ? (top << sh) | (uint64_t)(r.n[d + 2 > 6 ? 6 : d + 2] >> (32u - sh)) : top;  // 64 bits from the block's first
-  const uint64_t v = x >> (64u - kW);                                                                  // the block: index << 1 | gain
-  gain = (uint32_t)v & 1u;
-  ilo = (uint32_t)(v >> 1);
-  ihi = (uint32_t)(v >> 33);
-}
-template <class Rec> struct RecordTraits { static constexpr bool kWide = false; };
-template <> struct RecordTraits<DenseRecords> { static constexpr bool kWide = true; };
-
-// Phase timestamps for tuning builds (-DLLVQ_PHASE_TIMING): wave 0 of each
-// workgroup stores the realtime counter at every phase boundary of its first tile.
-#ifdef LLVQ_PHASE_TIMING
-__device__ unsigned long long g_phase_stamps[1024 * 8];
-#define LLVQ_STAMP(k)                                                                     \
-  do {                                                                                    \
-    if (threadIdx.x == 0 && tile == blockIdx.x) g_phase_stamps[blockIdx.x * 8 + (k)] = wall_clock64(); \
-  } while (0)
-#else
-#define LLVQ_STAMP(k) do {} while (0)
-#endif
 
 // The same number as one the compiler can relate to nothing it knows.  Used where what it would derive costs
 // more than the plain form: the address of an element of a second array with the same index (formed from the
@@ -800,703 +489,6 @@ __device__ __forceinline__ void classify_and_bin(const DecodeTables& T, uint32_t
   }
 }
 
-// ---- P1 of the GEMV kernel --------------------------------------------------------------
-// Each lane classifies the NB consecutive records it loaded itself and queues them with
-// everything P2 needs, so that the record is parsed once:
-//   qa[slot] = { local rank, bits 0..31;  local rank, bits 32..44 | class << 13 | gain << 22 | flags }
-//   qf[slot] = the block's number in the tile (row * blocks per row + column)
-// (the largest class holds fewer than 2^45 indices).  Three queues — the odd coset from the bottom
-// of qa / qf, the even coset from their top, and even-coset classes with a second free kind in a
-// small queue of their own (what does not fit there rides in the even queue, flagged) — because the
-// three are different straight-line programs.  Blocks of the rare generic classes go to two small
-// queues, by coset; what does not fit rides in the odd queue, flagged.
-constexpr uint32_t kQaClassShift = 13, kQaGainShift = 22;
-constexpr uint32_t kQaSecond = 0x40000000u;
-enum : uint32_t { kCtrlOdd = 0, kCtrlEven = 1, kCtrlGenOdd = 2, kCtrlTicket = 3, kCtrlSec = 4, kCtrlGenEven = 5, kCtrlWords = 8 };
-
-struct GemvQueues {
-  uint2* qa;        // [tile + kSecSlots]: the odd queue from 0 up, the even queue from tile - 1 down, the small even queue from tile up
-  uint16_t* qf;     // [tile + kSecSlots]
-  uint2* gqa;       // [2][kGenericSlots]: odd-coset generic blocks, then even-coset ones
-  uint16_t* gqf;
-  uint32_t* ctrl;   // [kCtrlWords]
-  float* partial;   // [tile]
-};
-
-// What a lane knows of its NB blocks after classification and before they are queued: the two
-// words of each block's queue entry and, packed in `where`, bits 2i..2i+1 = the queue block i joins
-// (0 odd, 1 even, 2 the small even queue, 3 none), bit 8 + i = block i is the origin, bit 12 + i =
-// block i is a generic block of the even coset.
-template <int NB>
-struct Classified {
-  uint32_t e0[NB], e1[NB];
-  uint32_t where;
-};
-
-// First half of P1: table reads only, nothing is written — it may run while another tile's queues are in use.
-template <int NB, class Rec>
-__device__ __forceinline__ void classify_records(const DecodeTables& T, const Rec& rec, uint32_t nblk, Classified<NB>& c,
-                                                 uint32_t tid = threadIdx.x) {
-  constexpr bool kWide = RecordTraits<Rec>::kWide;
-  // Every LDS read below is unconditional, from a valid slot, so that the NB reads of a step go
-  // out together (a guarded read is waited for where it is issued).  A lane past the tile's end
-  // walks the tables with whatever bytes follow the tile and queues nothing.
-  uint32_t zlo[NB], zhi[NB], gain[NB], ci[NB], kind[NB];
-  uint64_t start[NB];
-  bool live[NB];  // a block of the tile that is not the origin (which decodes to zero whatever the gain, index.rs:335-337)
-  uint32_t where = 0;
-  bool any_origin = false;
-  const auto& records = prepared_records(rec);
-  const uint32_t share = nblk > tid * NB ? nblk - tid * NB : 0u;  // this lane's blocks are its first `share` (NB or more: all)
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    uint32_t ilo, ihi;  // the 47-bit (48-bit) index
-    record_index(records, i, ilo, ihi, gain[i]);
-    // The tables are keyed on the index as the record holds it.  A 48-bit field can hold numbers past N(13):
-    // the host refuses such a matrix, and a lane past the tile's end, which reads whatever bits follow, must
-    // still walk the tables inside them: such a number counts as the origin
-    if (kWide) {
-      const uint64_t v = ((uint64_t)ihi << 32) | ilo;
-      const bool inside = v <= kN13;
-      ilo = inside ? ilo : 0u;
-      ihi = inside ? ihi : 0u;
-    }
-    const bool origin = (ilo | ihi) == 0u, mine = (uint32_t)i < share;
-    live[i] = mine && !origin;
-    any_origin |= mine && origin;
-    zlo[i] = ilo;
-    zhi[i] = ihi;
-  }
-  if (__any(any_origin)) {  // rare: a block at the origin is flagged for settle_origins
-    asm volatile("");       // (a branch, not selects on the common path)
-#pragma unroll
-    for (int i = 0; i < NB; ++i) where |= ((uint32_t)i < share && (zlo[i] | zhi[i]) == 0u) ? 1u << (8 + i) : 0u;
-  }
-  find_classes<NB, kWide>(T, zlo, zhi, ci, start, kind);
-  // Which queue a block joins.  A generic block (rare) joins none here: it is settled when the block is queued
-  // (its coset's small queue, or the odd queue, flagged, when that one is full).
-  bool any_generic = false;
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const uint64_t li = (((uint64_t)zhi[i] << 32) | zlo[i]) - start[i];
-    c.e0[i] = (uint32_t)li;
-    c.e1[i] = (uint32_t)(li >> 32) | (ci[i] << kQaClassShift) | (gain[i] << kQaGainShift);
-    where |= (live[i] ? kind[i] : 3u) << (2 * i);
-    any_generic |= live[i] && kind[i] == kLutKindGeneric;
-  }
-  static_assert(kLutKindGeneric == 3u, "a generic block and a block that joins no queue share the code 3");
-  if (__any(any_generic)) {
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if (live[i] && kind[i] == kLutKindGeneric) where |= (1u << (16 + i)) | ((T.fast[ci[i]].meta & kMetaOdd) ? 0u : 1u << (12 + i));
-  }
-  c.where = where;
-}
-
-// Second half of P1: the lane's classified blocks go to the tile's queues (LDS writes and counters).
-template <int NB>
-__device__ __forceinline__ void queue_classified(Classified<NB>& c, uint32_t capacity, const GemvQueues& Q, uint32_t tid = threadIdx.x) {
-  const uint32_t lane = tid & 63u;
-  uint32_t kq[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) kq[i] = (c.where >> (2 * i)) & 3u;
-  if (__any((c.where >> 16) & 15u)) {  // generic blocks: to the small queue of their coset while it has room
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if ((c.where >> (16 + i)) & 1u) {
-        const uint32_t even = (c.where >> (12 + i)) & 1u;
-        const uint32_t slot = atomicAdd(&Q.ctrl[even ? kCtrlGenEven : kCtrlGenOdd], 1u);
-        c.e1[i] |= 0x80000000u;  // the walk, not a fast decoder
-        if (slot < (uint32_t)kGenericSlots) {
-          Q.gqa[even * kGenericSlots + slot] = make_uint2(c.e0[i], c.e1[i]);
-          Q.gqf[even * kGenericSlots + slot] = (uint16_t)(tid * NB + (uint32_t)i);
-        } else {
-          kq[i] = 0u;  // rides in the odd queue, flagged
-        }
-      }
-  }
-  // A block's rank in its queue among the wavefront's blocks.  Three 10-bit counters packed in a
-  // dword (a wavefront classifies at most 256 blocks): a lane's own blocks in order, behind the
-  // blocks of the lanes below it — one prefix sum over the wavefront by lane shifts.
-  uint32_t sh[NB], running[NB], total = 0;
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    sh[i] = __umul24(kq[i], 10u);
-    running[i] = total;
-    total += (1u << sh[i]) & 0x3FFFFFFFu;  // a block that joins no queue (3) counts nowhere
-  }
-  const uint32_t through = wave_prefix_sum(total);  // this lane's blocks included
-  const uint32_t below = through - total;
-  const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)through, 63);
-  const uint32_t n_o = all & 1023u, n_e = (all >> 10) & 1023u, n_s = (all >> 20) & 1023u;
-  uint32_t base_o = 0, base_e = 0, base_s = 0;
-  if (lane == 0) {
-    base_o = atomicAdd(&Q.ctrl[kCtrlOdd], n_o);
-    base_s = atomicAdd(&Q.ctrl[kCtrlSec], n_s);
-    // what the small queue cannot take rides in the even queue behind this wavefront's own entries
-    const uint32_t spill = base_s + n_s > (uint32_t)kSecSlots ? base_s + n_s - max(base_s, (uint32_t)kSecSlots) : 0u;
-    base_e = atomicAdd(&Q.ctrl[kCtrlEven], n_e + spill);
-  }
-  base_o = __builtin_amdgcn_readfirstlane(base_o);
-  base_e = __builtin_amdgcn_readfirstlane(base_e);
-  base_s = __builtin_amdgcn_readfirstlane(base_s);
-  // odd from the bottom, even from the top, the small queue behind both
-  const uint32_t top = capacity - 1u - base_e, small = capacity + base_s;
-  const bool spills = base_s + n_s > (uint32_t)kSecSlots;  // wavefront-uniform, rare
-  auto place = [&](int i, uint32_t pos, uint32_t e1) {
-    if (kq[i] != 3u) {
-      Q.qa[pos] = make_uint2(c.e0[i], e1);
-      Q.qf[detached(pos)] = (uint16_t)(tid * NB + (uint32_t)i);
-    }
-  };
-  if (!spills) {  // a branch of its own: the rare case's arithmetic stays out of the common one
-    // the three queues' first slots in vector registers, formed once, and a signed step: the even queue runs down
-    const uint32_t v_odd = detached(base_o), v_top = detached(top), v_small = detached(small);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const uint32_t rank = __builtin_amdgcn_ubfe(below + running[i], sh[i], 10);
-      const uint32_t first = kq[i] == 1u ? v_top : (kq[i] == 2u ? v_small : v_odd);
-      const int step = kq[i] == 1u ? -1 : 1;
-      place(i, (uint32_t)__mul24((int)rank, step) + first, c.e1[i]);
-    }
-  } else {
-    const uint32_t fits = base_s >= (uint32_t)kSecSlots ? 0u : (uint32_t)kSecSlots - base_s;  // small-queue ranks below this fit
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const uint32_t rank = __builtin_amdgcn_ubfe(below + running[i], sh[i], 10);
-      const uint32_t up = base_o + rank, down = top - rank, behind = small + rank;
-      uint32_t pos = kq[i] == 1u ? down : up;
-      pos = kq[i] == 2u ? behind : pos;
-      const bool out = kq[i] == 2u && rank >= fits;
-      place(i, out ? top - (n_e + (rank - fits)) : pos, c.e1[i] | (out ? kQaSecond : 0u));
-    }
-  }
-}
-
-// The origin blocks of a lane's share decode to zero: their partial sums are written here.
-template <int NB>
-__device__ __forceinline__ void settle_origins(uint32_t where, float* partial, uint32_t tid = threadIdx.x) {
-  if (__any((where >> 8) & 15u)) {
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if ((where >> (8 + i)) & 1u) partial[tid * NB + (uint32_t)i] = 0.f;
-  }
-}
-
-template <int NB, class Rec>
-__device__ __forceinline__ void classify_stream(const DecodeTables& T, const Rec& rec, uint32_t nblk, uint32_t capacity,
-                                                const GemvQueues& Q) {
-  Classified<NB> c;
-  classify_records<NB>(T, rec, nblk, c);
-  settle_origins<NB>(c.where, Q.partial);
-  queue_classified<NB>(c, capacity, Q);
-}
-
-// P2 of the GEMV kernels: unrank the tile's queued blocks and reduce them against the activation planes.
-// Chunks of 64 queued blocks are handed out through a counter: the two generic chunks first (longest),
-// then the chunks of the three fast decoders.  `hook(done, last, state)` (kHook) runs in every wavefront before
-// each of its chunks of the fast decoders, with the number it has finished, and once more (last = true) when
-// there is none left for it: where a caller puts work that does not depend on this tile and fills the issue
-// slots this tile's decoders leave.  `state` is 0 at first and then whatever the hook returned last; the
-// function returns the final one.
-struct UnrankOperands {
-  const uint32_t* xplanes;  // [nb][kPlaneDwords]
-  const float* xscale;      // [nb]
-  uint32_t nb;              // blocks per row
-  float inv_nb;             // 1 / nb, for the block -> column split
-  float g0, g1;             // the matrix's gain centroids
-  uint32_t hook_state = 0;  // the state the hook is first called with
-};
-
-template <int TILE, bool kHook, int PLANES, class Hook>
-__device__ __forceinline__ uint32_t unrank_tile(const DecodeTables& T, const GemvQueues& Q, const UnrankOperands& op, Hook&& hook) {
-  constexpr int kTileBlocks = TILE;
-  uint32_t tid = threadIdx.x;
-  // inside a persistent loop over tiles: lane-derived values are formed here, per call, not carried around that loop
-  if constexpr (kHook) asm volatile("" : "+v"(tid));
-  const uint32_t lane = tid & 63u;
-  uint32_t* ctrl = Q.ctrl;
-  float* partial = Q.partial;
-  const uint32_t* xplanes = op.xplanes;
-  const float* xscale = op.xscale;
-  const uint32_t nb = op.nb;
-  const uint32_t n_odd = ctrl[kCtrlOdd], n_even = ctrl[kCtrlEven], n_sec = min(ctrl[kCtrlSec], (uint32_t)kSecSlots);
-  const uint32_t n_gen_o = min(ctrl[kCtrlGenOdd], (uint32_t)kGenericSlots), n_gen_e = min(ctrl[kCtrlGenEven], (uint32_t)kGenericSlots);
-  const uint32_t c_gen_o = n_gen_o ? 1u : 0u, c_gen_e = n_gen_e ? 1u : 0u, c_gen = c_gen_o + c_gen_e;
-  const uint32_t c_odd = (n_odd + 63u) >> 6, c_even = (n_even + 63u) >> 6, c_sec = (n_sec + 63u) >> 6;
-  auto ticket = [&]() {
-    uint32_t t = 0;
-    if (lane == 0) t = atomicAdd(&ctrl[kCtrlTicket], 1u);
-    return (uint32_t)__shfl(t, 0, 64);
-  };
-  // what every decoder starts from: the block's local rank, class, column and scale
-  struct Block {
-    uint64_t li;
-    uint32_t f, ci, col;
-    float g;
-  };
-  auto open_block = [&](uint2 e, uint32_t f) {
-    Block b;
-    b.li = ((uint64_t)(e.y & 0x1FFFu) << 32) | e.x;
-    b.ci = (e.y >> kQaClassShift) & 0x1FFu;
-    b.f = f;
-    const uint32_t row = (uint32_t)(((float)f + 0.5f) * op.inv_nb);
-    b.col = f - __umul24(row, nb);  // both below 2^24: the full-rate multiply
-    b.g = (e.y >> kQaGainShift) & 1u ? op.g1 : op.g0;
-    return b;
-  };
-  // generic walk of one queued block (rare classes): coordinates packed four to a dword, then
-  // the same integer dot products as the fast paths
-  auto generic_block = [&](uint2 e, uint32_t f) {
-    const Block b = open_block(e, f);
-    const uint32_t* xp = xplanes + __umul24(b.col, (uint32_t)kPlaneDwords);
-    const DevClass c = T.cls[b.ci];
-    uint32_t w[6] = {0, 0, 0, 0, 0, 0};
-    auto emit = [&](int p, int v) { w[p >> 2] |= ((uint32_t)v & 0xFFu) << (8 * (p & 3)); };
-    if (c.meta & kMetaOdd) decode_odd(T, c, b.li, emit);
-    else decode_even(T, c, b.li, emit);
-    int d0 = 0, d1 = 0, d2 = 0;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-      d0 = __builtin_amdgcn_sdot4((int)w[q], (int)xp[q], d0, false);
-      d1 = __builtin_amdgcn_sdot4((int)w[q], (int)xp[6 + q], d1, false);
-      if (PLANES == 3) d2 = __builtin_amdgcn_sdot4((int)w[q], (int)xp[12 + q], d2, false);
-    }
-    partial[b.f] = planes_to_float<PLANES>(d0, d1, d2) * xscale[b.col] * (c.inv_norm * b.g);
-  };
-  auto odd_block = [&](uint2 e, uint32_t f) {
-    const Block b = open_block(e, f);
-    const uint32_t* xp = xplanes + __umul24(b.col, (uint32_t)kPlaneDwords);
-    const FastClass fc = T.fast[b.ci];
-    int d0 = 0, d1 = 0, d2 = 0;
-    odd_codes(T, fc, b.li, [&](int q, uint32_t sel) {
-      const int w = (int)__builtin_amdgcn_perm(fc.tab_hi, fc.tab_lo, sel);
-      d0 = __builtin_amdgcn_sdot4(w, (int)xp[q], d0, false);
-      d1 = __builtin_amdgcn_sdot4(w, (int)xp[6 + q], d1, false);
-      if (PLANES == 3) d2 = __builtin_amdgcn_sdot4(w, (int)xp[12 + q], d2, false);
-    });
-    partial[b.f] = planes_to_float<PLANES>(d0, d1, d2) * xscale[b.col] * (fc.inv_norm * b.g);
-  };
-  auto even_block = [&](uint2 e, uint32_t f, auto second) {
-    constexpr bool kSecond = decltype(second)::value;
-    const Block b = open_block(e, f);
-    const uint32_t* xp = xplanes + __umul24(b.col, (uint32_t)kPlaneDwords);
-    const FastClass fc = T.fast[b.ci];
-    const uint32_t fv1 = fc.u0 >> 16;
-    const uint32_t tab2_lo = fv1 << 8, tab2_hi = ((0u - fv1) & 0xFFu) << 8;
-    int d0 = 0, d1 = 0, d2 = 0;
-    even_codes<kSecond>(T, fc, b.li, [&](int q, uint32_t sel, uint32_t sel2) {
-      int w = (int)__builtin_amdgcn_perm(fc.tab_hi, fc.tab_lo, sel);
-      if (kSecond) w |= (int)__builtin_amdgcn_perm(tab2_hi, tab2_lo, sel2);
-      d0 = __builtin_amdgcn_sdot4(w, (int)xp[q], d0, false);
-      d1 = __builtin_amdgcn_sdot4(w, (int)xp[6 + q], d1, false);
-      if (PLANES == 3) d2 = __builtin_amdgcn_sdot4(w, (int)xp[12 + q], d2, false);
-    });
-    partial[b.f] = planes_to_float<PLANES>(d0, d1, d2) * xscale[b.col] * (fc.inv_norm * b.g);
-  };
-  uint32_t chunk = ticket();
-  // the generic chunks, kept out of the loop below: their code and registers are not the hot path's
-  while (chunk < c_gen) {
-    const uint32_t even = (chunk == 1u || !c_gen_o) ? 1u : 0u;
-    if (lane < (even ? n_gen_e : n_gen_o)) generic_block(Q.gqa[even * kGenericSlots + lane], Q.gqf[even * kGenericSlots + lane]);
-    chunk = ticket();
-  }
-  // Even and odd chunks alternate while both queues last: the even coset waits for tables in L2,
-  // the odd one issues arithmetic, and wavefronts on either kind at the same time overlap the two.
-  // The chunks of the small even queue come first (their queue ends in a partial chunk as well).
-  const uint32_t c_pair = min(c_odd, c_even);
-  const uint32_t c_all = c_gen + c_sec + c_odd + c_even;
-  uint32_t done = 0, hook_state = op.hook_state;
-  for (;; ++done, chunk = ticket()) {
-    if constexpr (kHook) hook_state = hook(done, chunk >= c_all, hook_state);
-    if (chunk >= c_all) break;
-    const uint32_t ts = chunk - c_gen;
-    if (ts < c_sec) {
-      const uint32_t k = ts * 64u + lane;
-      if (k < n_sec) even_block(Q.qa[kTileBlocks + k], Q.qf[detached(kTileBlocks + k)], std::true_type{});
-      continue;
-    }
-    const uint32_t t = ts - c_sec;
-    const bool paired = t < 2u * c_pair;
-    const bool is_odd = paired ? (t & 1u) != 0u : c_odd > c_even;
-    const uint32_t ordinal = paired ? t >> 1 : t - c_pair;
-    const uint32_t k = ordinal * 64u + lane;
-    if (is_odd) {
-      const uint32_t at = min(k, (uint32_t)kTileBlocks - 1u);
-      const uint2 e = Q.qa[at];
-      // generic blocks that found their small queue full wait for the pass below
-      if (k < n_odd && !(e.y >> 31)) odd_block(e, Q.qf[detached(at)]);
-    } else {
-      const uint32_t at = kTileBlocks - 1 - min(k, (uint32_t)kTileBlocks - 1u);
-      const uint2 e = Q.qa[at];
-      const bool mine = k < n_even;
-      // blocks with a second free kind that found their queue full ride here, flagged
-      if (__any(mine && (e.y & kQaSecond))) {
-        if (mine) even_block(e, Q.qf[at], std::true_type{});
-      } else {
-        if (mine) even_block(e, Q.qf[at], std::false_type{});
-      }
-    }
-  }
-  if (ctrl[kCtrlGenOdd] > (uint32_t)kGenericSlots || ctrl[kCtrlGenEven] > (uint32_t)kGenericSlots) {
-    // more generic blocks than the small queues hold (hostile input): the rest sit flagged in the odd queue
-    for (uint32_t k = tid; k < n_odd; k += kWgThreads) {
-      const uint2 e = Q.qa[k];
-      if (e.y >> 31) generic_block(e, Q.qf[k]);
-    }
-  }
-  return hook_state;
-}
-
-// Where a launch's activation comes from, and what it may do to produce it before the product.
-struct ActivationSource {
-  const __half* x;
-  const float* x_f32;  // when set, the activation is these f32 values (a rotated activation) and x is unused
-  const __half* x2;
-  const __half* norm_w;
-  __half* resid_out;
-  float eps;
-  uint32_t prologue;   // kPrologue*
-  uint32_t nb, tail_w;
-  const uint32_t* rot_signbits;
-  const float* rot_small;
-  float rot_inv;
-  uint32_t rot_m, rot_k;
-  bool writes_resid;   // this workgroup is the one that stores the new residual
-  bool device_scope = false;  // a finished activation is read at device scope (another workgroup of this launch stored it)
-};
-
-// Fills the activation planes, scales and tail values in LDS from `a`, by every lane of the workgroup.
-// `raw` (the tile's queue entries, block numbers and partial sums, free at this point) is the staging
-// area of a derived or rotated activation; `request` is called once, right behind the loads of the
-// activation's operands (the caller's first code bytes go out there).  Returns whether the staging
-// area was used: the caller then needs a barrier before the area becomes queues again.  kInPlace: `raw` is the
-// planes' own memory (rows of at most as many blocks as the workgroup has lanes, natural basis only).
-template <int TILE, bool ROT, int PLANES, bool kInPlace = false, class Request>
-__device__ __forceinline__ bool stage_activation(const ActivationSource& a, uint32_t* xplanes, float* xscale, float* xtail, uint8_t* raw,
-                                                 float* partial, Request&& request_first_tile) {
-  constexpr int kTileBlocks = TILE;
-  constexpr int kRawBytes = TILE * 6 + 32;  // what a derived binary16 activation may take of the staging area
-  uint32_t tid = threadIdx.x;
-  // staged from inside a loop over tiles: lane-derived indices are formed here, not carried through the loop in registers
-  if constexpr (kInPlace) asm volatile("" : "+v"(tid));
-  const uint32_t lane = tid & 63u, wave = tid >> 6;
-  const uint32_t nb = a.nb;
-  const __half* xsrc = a.x;
-  // A launch over matrices stored in a rotated basis rotates its activation itself: the
-  // values go, signs applied, as f32 to the area the first tile's queues and
-  // partial sums will use (free until then), are rotated there and quantised from there.
-  const bool rotated = ROT && a.rot_m != 0;
-  float* xf = reinterpret_cast<float*>(raw);
-  const uint32_t d_in = nb * kDim + a.tail_w;
-  auto signed_f32 = [&](uint32_t i, float v) { return ((a.rot_signbits[i >> 5] >> (i & 31u)) & 1u) ? -v : v; };
-  if (a.prologue != kPrologueNone) {
-    // Every workgroup derives the activation for itself (a few thousand values)
-    // instead of waiting for a kernel of its own; it is staged, as binary16, where
-    // the tile's queues will go.
-    __half* xs = reinterpret_cast<__half*>(raw);
-    // All of a lane's values are requested before the first is used (a load and its use per loop
-    // iteration would pay the memory latency once per iteration): the rounds are counted at compile
-    // time (3 covers 3072 values, 6 and 12 the wider rows), their loads are unconditional (a lane past
-    // the row's end reads its last value) and a scheduling barrier keeps them ahead of the arithmetic.
-    constexpr int kPerMax = (kRawBytes / 2 + kWgThreads - 1) / kWgThreads;
-    const bool silu = a.prologue == kPrologueSiluMul;
-    const __half* src1 = a.x2 ? a.x2 : a.x;
-    const __half* src2 = silu ? a.x : a.norm_w;
-    auto derive = [&](auto rounds, uint32_t base) {
-      constexpr int kPer = decltype(rounds)::value;
-      __half in0[kPer], in1[kPer], in2[kPer];
-#pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        const uint32_t i = min(base + tid + (uint32_t)k * kWgThreads, d_in - 1u);
-        in0[k] = load_half<kInPlace>(a.x + i);
-        in1[k] = load_half<kInPlace>(src1 + i);
-        in2[k] = src2[i];  // the norm's gains are constants (with SiLU this is x again, and unused)
-      }
-      request_first_tile();
-      __builtin_amdgcn_sched_barrier(0);
-      if (silu) {
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-          const uint32_t i = base + tid + (uint32_t)k * kWgThreads;
-          if (i < d_in) {
-            const float g = __half2float(in1[k]);
-            const float sg = __half2float(__float2half_rn(g / (1.0f + __expf(-g))));
-            const __half h = __float2half_rn(sg * __half2float(in0[k]));
-            if (rotated) xf[i] = signed_f32(i, __half2float(h));
-            else xs[i] = h;
-          }
-        }
-      } else {
-        float* red = partial + kTileBlocks - kWaves;  // the end of the partial sums: beyond the f32 staging of a rotated launch
-        float v[kPer];
-        float ss = 0.f;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-          const uint32_t i = base + tid + (uint32_t)k * kWgThreads;
-          v[k] = 0.f;
-          if (i < d_in) {
-            float r = __half2float(in0[k]);
-            if (a.x2) r = __half2float(__float2half_rn(r + __half2float(in1[k])));
-            if (a.resid_out && a.writes_resid) store_half<kInPlace>(a.resid_out + i, __float2half_rn(r));
-            v[k] = r;
-            ss += r * r;
-          }
-        }
-        ss = wave_sum(ss);
-        if (lane == 0) red[wave] = ss;
-        __syncthreads();
-        float total = 0.f;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) total += red[w];
-        const float inv = 1.0f / sqrtf(total / (float)d_in + a.eps);
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-          const uint32_t i = base + tid + (uint32_t)k * kWgThreads;
-          if (i < d_in) {
-            const __half h = __float2half_rn(v[k] * inv * __half2float(in2[k]));
-            if (rotated) xf[i] = signed_f32(i, __half2float(h));
-            else xs[i] = h;
-          }
-        }
-      }
-    };
-    const uint32_t n_per = (d_in + kWgThreads - 1) / kWgThreads;
-    if constexpr (kInPlace) {
-      // at most six rounds of operands in registers at a time: the wider SiLU rows go in runs of 6144 values
-      // (a row sum of squares over more than 6144 values is refused by the host for this variant)
-      if (n_per <= 3) derive(std::integral_constant<int, 3>{}, 0u);
-      else
-        for (uint32_t base = 0; base < d_in; base += 6u * kWgThreads) derive(std::integral_constant<int, 6>{}, base);
-    } else {
-      if (n_per <= 3) derive(std::integral_constant<int, kPerMax < 3 ? kPerMax : 3>{}, 0u);
-      else if (n_per <= 6) derive(std::integral_constant<int, kPerMax < 6 ? kPerMax : 6>{}, 0u);
-      else derive(std::integral_constant<int, kPerMax>{}, 0u);
-    }
-    __syncthreads();
-    xsrc = xs;
-  } else if (rotated) {
-    request_first_tile();
-    // eight values per lane and pass; a width that is not a multiple of eight ends one value at a time
-    const uint32_t n8 = d_in & ~7u;
-    for (uint32_t i = tid * 8u; i < n8; i += kWgThreads * 8u) {
-      const uint4 h = *reinterpret_cast<const uint4*>(a.x + i);
-      const uint32_t sg = a.rot_signbits[i >> 5] >> (i & 31u);
-      const uint32_t w[4] = {h.x, h.y, h.z, h.w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float lo = __half2float(__ushort_as_half((unsigned short)(w[q] & 0xFFFFu)));
-        const float hi = __half2float(__ushort_as_half((unsigned short)(w[q] >> 16)));
-        xf[i + 2 * q] = ((sg >> (2 * q)) & 1u) ? -lo : lo;
-        xf[i + 2 * q + 1] = ((sg >> (2 * q + 1)) & 1u) ? -hi : hi;
-      }
-    }
-    for (uint32_t i = n8 + tid; i < d_in; i += kWgThreads) xf[i] = signed_f32(i, __half2float(a.x[i]));
-    __syncthreads();
-  }
-  if (rotated) {
-    rotate_lds(xf, d_in, a.rot_m, a.rot_k, a.rot_inv, a.rot_small);
-    __syncthreads();
-    for (uint32_t col = tid; col < nb; col += kWgThreads)
-      quantize_block_f32<PLANES>(xf + (size_t)col * kDim, xplanes + (size_t)col * kPlaneDwords, xscale + col);
-    if (tid < a.tail_w) xtail[tid] = xf[(size_t)nb * kDim + tid];
-  } else if (a.prologue != kPrologueNone) {
-    if constexpr (kInPlace) {
-      // the staging area is the planes' own: every lane reads its block before any lane writes (nb <= lanes)
-      float v[kDim];
-      load_block_f16(xsrc + (size_t)min(tid, nb ? nb - 1u : 0u) * kDim, v);
-      const float tail_v = tid < a.tail_w ? __half2float(xsrc[(size_t)nb * kDim + tid]) : 0.f;
-      __syncthreads();
-      if (tid < nb) quantize_values<PLANES>(v, xplanes + (size_t)tid * kPlaneDwords, xscale + tid);
-      if (tid < a.tail_w) xtail[tid] = tail_v;
-    } else {
-      for (uint32_t col = tid; col < nb; col += kWgThreads)
-        quantize_block<PLANES>(xsrc + (size_t)col * kDim, xplanes + (size_t)col * kPlaneDwords, xscale + col);
-      if (tid < a.tail_w) xtail[tid] = __half2float(xsrc[(size_t)nb * kDim + tid]);
-    }
-  } else {
-    // a finished activation from global memory: this lane's block is requested, then the first tile's
-    // code bytes, then the block is quantised (rows wider than 1024 blocks take further rounds)
-    float v[kDim];
-#pragma unroll
-    for (int j = 0; j < kDim; ++j) v[j] = 0.f;
-    if ((tid & ~63u) < nb) {  // wavefronts with a block to read (a row of tail columns only has none)
-      const uint32_t c0 = min(tid, nb - 1u);
-      if (a.x_f32) {
-#pragma unroll
-        for (int j = 0; j < kDim; ++j) v[j] = a.x_f32[(size_t)c0 * kDim + j];
-      } else {
-        // (an activation another workgroup of this launch stored is read at device scope; any other through the caches)
-        if (kInPlace && a.device_scope) load_block_f16<true>(xsrc + (size_t)c0 * kDim, v);
-        else load_block_f16<false>(xsrc + (size_t)c0 * kDim, v);
-      }
-    }
-    float tail_v = 0.f;
-    if (tid < a.tail_w) {
-      if (a.x_f32) tail_v = a.x_f32[(size_t)nb * kDim + tid];
-      else if (kInPlace && a.device_scope) tail_v = __half2float(load_half<true>(xsrc + (size_t)nb * kDim + tid));
-      else tail_v = __half2float(xsrc[(size_t)nb * kDim + tid]);
-    }
-    request_first_tile();
-    __builtin_amdgcn_sched_barrier(0);
-    if (tid < nb) quantize_values<PLANES>(v, xplanes + (size_t)tid * kPlaneDwords, xscale + tid);
-    if (tid < a.tail_w) xtail[tid] = tail_v;
-    for (uint32_t col = tid + kWgThreads; col < nb; col += kWgThreads) {
-      if (a.x_f32) quantize_block_f32<PLANES>(a.x_f32 + (size_t)col * kDim, xplanes + (size_t)col * kPlaneDwords, xscale + col);
-      else quantize_block<PLANES>(xsrc + (size_t)col * kDim, xplanes + (size_t)col * kPlaneDwords, xscale + col);
-    }
-  }
-  return a.prologue != kPrologueNone || rotated;
-}
-
-// LEAN: the Golay words and the support-arrangement table stay in L2, which leaves
-// room for the full tile beside the activation planes of a very wide row.
-// ROT: the launch can rotate its own activation (GroupArgs::rot_m); kept out of the other
-// instantiations, whose hot loop it would otherwise cost registers and a few per cent.
-// WIDE: the matrices are cap-13 ones (49-bit blocks in a dense stream, 48-bit indices): a lane extracts its blocks
-// from the stream, and the class tables a 47-bit index cannot reach are read from device memory.
-template <typename OutT, int TILE = kTileBlocks, bool LEAN = false, bool ROT = false, bool WIDE = false>
-__global__ __launch_bounds__(kWgThreads) void gemv_tiles_kernel(GroupArgs a) {
-  static_assert(!WIDE || (TILE == 4 * kWgThreads && !ROT), "the dense-stream variant takes four blocks per lane and no in-launch rotation");
-  // the tile capacity of this instantiation (these shadow the namespace-level defaults)
-  constexpr int kTileBlocks = TILE;
-  constexpr int kP1Blocks = TILE / kWgThreads;
-  constexpr int kPlanes = std::is_same<OutT, __half>::value ? 2 : 3;  // byte planes of the activation (quantize_values)
-  extern __shared__ __align__(16) uint8_t smem[];
-#ifdef LLVQ_PHASE_TIMING
-  if (threadIdx.x == 0) g_phase_stamps[blockIdx.x * 8 + 3] = wall_clock64();
-#endif
-  const DecodeTables T = stage_tables<!LEAN, true, WIDE>(smem, a.tables);
-  // A lane loads the records it classifies itself, HBM -> registers; the next tile's loads are
-  // issued while the current one is being decoded.  The first tile's are issued right behind the
-  // loads of the activation: the memory counter retires in order, so whatever is requested
-  // after them would wait for HBM with them, and they are not needed before the activation is.
-  typename std::conditional<WIDE, DenseRecords, LaneRecords<kP1Blocks>>::type pre;
-#pragma unroll
-  for (int k = 0; k < (int)(sizeof(pre.w) / sizeof(pre.w[0])); ++k) pre.w[k] = 0;
-  if constexpr (WIDE) pre.s0 = 0;
-  auto request_first_tile = [&]() { prefetch_records(a, blockIdx.x, threadIdx.x, pre); };
-  const uint32_t nb = a.nblocks;
-  uint32_t* xplanes = reinterpret_cast<uint32_t*>(smem + (LEAN ? kLdsImageBytesLean : kLdsImageBytes));
-  float* xscale = reinterpret_cast<float*>(xplanes + (size_t)nb * kPlaneDwords);
-  float* xtail = xscale + nb;
-  // queue entries | block numbers | 32 bytes | partial sums: also the staging area of a derived or rotated activation
-  uint8_t* raw = reinterpret_cast<uint8_t*>(xtail + 32 + (nb & 1u));  // 8-byte aligned: the queue entries are read as 64-bit words
-  GemvQueues Q;
-  Q.qa = reinterpret_cast<uint2*>(raw);
-  Q.qf = reinterpret_cast<uint16_t*>(Q.qa + kTileBlocks + kSecSlots);
-  Q.partial = reinterpret_cast<float*>(Q.qf + kTileBlocks + kSecSlots + 16);
-  Q.gqa = reinterpret_cast<uint2*>(Q.partial + kTileBlocks);
-  Q.gqf = reinterpret_cast<uint16_t*>(Q.gqa + 2 * kGenericSlots);
-  Q.ctrl = reinterpret_cast<uint32_t*>(Q.gqf + 2 * kGenericSlots);
-  float* partial = Q.partial;
-  uint32_t* ctrl = Q.ctrl;
-  static_assert((kTileBlocks + kSecSlots) % 4 == 0 && kGenericSlots % 2 == 0, "the arrays behind the 16-bit ones stay 8-byte aligned");
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const ActivationSource src{a.x, a.x_f32, a.x2, a.norm_w, a.resid_out, a.eps, a.prologue, nb, a.tail_w,
-                             a.rot_signbits, a.rot_small, a.rot_inv, a.rot_m, a.rot_k, blockIdx.x == 0};
-  if (stage_activation<kTileBlocks, ROT, kPlanes>(src, xplanes, xscale, xtail, raw, partial, request_first_tile))
-    __syncthreads();  // the staging area becomes the tile's queues
-
-#ifdef LLVQ_PHASE_TIMING
-  if (threadIdx.x == 0) g_phase_stamps[blockIdx.x * 8 + 7] = wall_clock64();
-#endif
-  for (uint32_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
-    LLVQ_STAMP(0);
-    MatArg M;
-    uint32_t r0, rows;
-    tile_of(a, tile, M, r0, rows);
-    const uint32_t nblk = rows * nb;
-
-    if (tid < (uint32_t)kCtrlWords) ctrl[tid] = 0;
-    // P3 operands (row scales, tail weights): fetched now, used after the decode
-    const uint32_t sub = lane >> 4, l16 = lane & 15u;
-    constexpr int kP3Rounds = 2;  // 64 rows per round cover every tile of the usual shapes
-    float rs_pre[kP3Rounds], tl_pre[kP3Rounds][2];
-#pragma unroll
-    for (int j = 0; j < kP3Rounds; ++j) {
-      const uint32_t row = (wave * 4 + sub) + (uint32_t)j * (kWaves * 4);
-      const bool ok = row < rows;
-      rs_pre[j] = ok ? M.rscale[r0 + row] : 0.f;
-      tl_pre[j][0] = (ok && l16 < a.tail_w) ? M.tail[(size_t)(r0 + row) * a.tail_w + l16] : 0.f;
-      tl_pre[j][1] = (ok && l16 + 16 < a.tail_w) ? M.tail[(size_t)(r0 + row) * a.tail_w + l16 + 16] : 0.f;
-    }
-    __syncthreads();
-    LLVQ_STAMP(1);
-
-    // P1: classify and bin (a tile of tail-only rows has no blocks: its queues stay empty)
-    if (nblk != 0) classify_stream<kP1Blocks>(T, pre, nblk, kTileBlocks, Q);
-    __syncthreads();
-    LLVQ_STAMP(2);
-    prefetch_records(a, tile + gridDim.x, tid, pre);
-
-    // P2: unrank and reduce
-    unrank_tile<kTileBlocks, false, kPlanes>(T, Q, UnrankOperands{xplanes, xscale, nb, a.inv_nblocks, M.g0, M.g1}, [](uint32_t, bool, uint32_t) { return 0u; });
-    LLVQ_STAMP(4);
-    __syncthreads();
-    LLVQ_STAMP(5);
-    // P3: 16 lanes per row, fixed summation order
-    for (uint32_t base = 0; base < rows; base += kWaves * 4) {
-      const uint32_t j = base / (kWaves * 4);
-      const uint32_t row = base + wave * 4 + sub;
-      const bool ok = row < rows;
-      float s = 0.f;
-      if (ok)
-        for (uint32_t b = l16; b < nb; b += 16u) s += partial[row * nb + b];  // fixed order per lane
-      float rs, t0, t1;
-      if (j < (uint32_t)kP3Rounds) {
-        rs = j == 0 ? rs_pre[0] : rs_pre[1];
-        t0 = j == 0 ? tl_pre[0][0] : tl_pre[1][0];
-        t1 = j == 0 ? tl_pre[0][1] : tl_pre[1][1];
-      } else {
-        rs = ok ? M.rscale[r0 + row] : 0.f;
-        t0 = (ok && l16 < a.tail_w) ? M.tail[(size_t)(r0 + row) * a.tail_w + l16] : 0.f;
-        t1 = (ok && l16 + 16 < a.tail_w) ? M.tail[(size_t)(r0 + row) * a.tail_w + l16 + 16] : 0.f;
-      }
-      float v = s * rs;
-      v = fmaf(t0, l16 < a.tail_w ? xtail[l16] : 0.f, v);
-      v = fmaf(t1, l16 + 16 < a.tail_w ? xtail[l16 + 16] : 0.f, v);
-#pragma unroll
-      for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 16);  // fixed tree inside each group of 16 lanes
-      if (ok && l16 == 0) store_out<OutT>(M.y, r0 + row, v);
-    }
-    __syncthreads();
-    LLVQ_STAMP(6);
-  }
-}
-
-
-// The instantiations of gemv_tiles_kernel by (f32 output, tile, lean image, in-launch rotation).
-template <typename OutT, bool ROT>
-__host__ const void* gemv_kernel_of(uint32_t tile, bool lean) {
-  if (lean) return reinterpret_cast<const void*>(gemv_tiles_kernel<OutT, kTileBlocks, true, ROT>);
-  if (tile == (uint32_t)kTileBlocks) return reinterpret_cast<const void*>(gemv_tiles_kernel<OutT, kTileBlocks, false, ROT>);
-  return reinterpret_cast<const void*>(gemv_tiles_kernel<OutT, kSmallTileBlocks, false, ROT>);
-}
-__host__ const void* gemv_kernel(bool f32, uint32_t tile, bool lean, bool rot) {
-  if (f32) return rot ? gemv_kernel_of<float, true>(tile, lean) : gemv_kernel_of<float, false>(tile, lean);
-  return rot ? gemv_kernel_of<__half, true>(tile, lean) : gemv_kernel_of<__half, false>(tile, lean);
-}
-// ... and for cap-13 matrices (full tile only, with the whole or the lean table image, no in-launch rotation)
-__host__ const void* gemv_kernel_wide(bool f32, bool lean) {
-  if (f32) return lean ? reinterpret_cast<const void*>(gemv_tiles_kernel<float, kTileBlocks, true, false, true>)
-                       : reinterpret_cast<const void*>(gemv_tiles_kernel<float, kTileBlocks, false, false, true>);
-  return lean ? reinterpret_cast<const void*>(gemv_tiles_kernel<__half, kTileBlocks, true, false, true>)
-              : reinterpret_cast<const void*>(gemv_tiles_kernel<__half, kTileBlocks, false, false, true>);
-}
-template <class Fn>
-__host__ void for_each_gemv_kernel(Fn&& fn) {
-  for (int f32 = 0; f32 < 2; ++f32) {
-    for (int rot = 0; rot < 2; ++rot) {
-      fn(gemv_kernel(f32, kTileBlocks, false, rot));
-      fn(gemv_kernel(f32, kSmallTileBlocks, false, rot));
-      fn(gemv_kernel(f32, kTileBlocks, true, rot));
-    }
-    fn(gemv_kernel_wide(f32, false));
-    fn(gemv_kernel_wide(f32, true));
-  }
-}
-
 // ---- incoherence rotation of an activation ----------------------------------------
 // x' = Q x for Q = (S (x) I_m)(I_k (x) H_m / sqrt m) D (llvq-quant/src/rotation.rs:97-105),
 // in f32 like the reference's device rotation (llvq-cuda/kernels/llvq_rot.cuh): signs on
@@ -1535,6 +527,7 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
 
 }  // namespace llvq
 
+#include "tiles.h"
 #include "gemv_seq.h"
 #include "gemm_kernel.h"
 #include "decoder.h"
@@ -1571,6 +564,9 @@ struct llvq_rt {
   // a batch's activations in K-step tiles [n_steps, m_pad, 32] (pipelined batched kernel)
   __half* gemm_xt = nullptr;
   size_t gemm_xt_bytes = 0;
+  // where an upload's code stream lands before it is unranked into a matrix's tiles (at most kUploadBytes of codes)
+  uint8_t* upload_buf = nullptr;
+  size_t upload_bytes = 0;
 };
 
 struct llvq_mat {
@@ -1578,6 +574,7 @@ struct llvq_mat {
   uint32_t d_out = 0, d_in = 0, nblocks = 0, tail_w = 0;
   uint32_t record_bits = 48;  // 48: 6-byte records (shell cap 12); 49: the dense stream of shell cap 13
   float g[2] = {0, 0};
+  uint8_t* tiles = nullptr;  // device: scale table and records (tiles.h)
   uint8_t* codes = nullptr;  // device
   float* rscale = nullptr;   // device
   float* tail = nullptr;     // device
@@ -1589,10 +586,10 @@ struct llvq_mat {
 };
 
 struct llvq_seq {
-  uint8_t* blob = nullptr;  // one device allocation: tiles | items | counters | status
+  uint8_t* blob = nullptr;  // one device allocation: units | items | runs | counters | status
   SeqArgs args{};
-  uint32_t tile = 0, grid = 0, n_items = 0;
-  bool lean = false, f32 = false, wide = false;
+  const void* kernel = nullptr;
+  uint32_t grid = 0, n_items = 0;
   size_t lds = 0;
   uint32_t* own_status = nullptr;  // the status word inside `blob` (args.status may point at a word several sequences share)
 };
@@ -1728,6 +725,7 @@ void llvq_hip_runtime_destroy(llvq_rt* rt) {
   (void)hipFree(rt->gemm_xt);
   (void)hipFree(rt->rot_scratch);
   (void)hipFree(rt->rot_rows);
+  (void)hipFree(rt->upload_buf);
   for (auto* r : rt->rotations) {
     (void)hipFree(r->signbits);
     (void)hipFree(r->small);
@@ -1735,17 +733,6 @@ void llvq_hip_runtime_destroy(llvq_rt* rt) {
   }
   delete rt;
 }
-
-#ifdef LLVQ_PHASE_TIMING
-// Tuning builds only: the phase timestamps of the last gemv_tiles_kernel launch ([workgroup][8]) and the stage
-// timestamps of the last gemm_tiles_kernel launch ([workgroup][wavefront][4]).
-int llvq_hip_debug_phase_stamps(unsigned long long* out, size_t n) {
-  return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(g_phase_stamps), n * sizeof(unsigned long long));
-}
-int llvq_hip_debug_gemm_stamps(unsigned long long* out, size_t n) {
-  return (int)hipMemcpyFromSymbol(out, HIP_SYMBOL(g_gemm_stamps), n * sizeof(unsigned long long));
-}
-#endif
 
 int llvq_hip_synchronize(llvq_rt* rt) {
   if (!rt) return fail(LLVQ_ERR_INVALID_ARGUMENT, "synchronize: runtime is null");
@@ -1785,6 +772,60 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
   rt->rotations.push_back(r);
   *out = r;
   return LLVQ_OK;
+}
+
+// Grows a device buffer of the runtime to `need` bytes (contents are not kept).
+static hipError_t grow_device(uint8_t** buf, size_t* have, size_t need) {
+  if (need <= *have) return hipSuccess;
+  (void)hipFree(*buf);
+  *buf = nullptr;
+  *have = 0;
+  const hipError_t e = hipMalloc(reinterpret_cast<void**>(buf), need);
+  if (e == hipSuccess) *have = need;
+  return e;
+}
+
+// Code stream, scales and tail -> the matrix's tiles (tiles.h), through the runtime's staging buffer, kUploadRows worth
+// of code bytes at a time.  Blocks until done: the host arrays may go, and the staging buffer is free for the next one.
+constexpr size_t kUploadBytes = 32u << 20;
+static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids, const float* rscale, const float* tail, const uint8_t* codes) {
+  const uint32_t nb = m->nblocks, stride = tile_stride(nb, m->tail_w), n_tiles = tile_count(m->d_out);
+  const size_t row_bits = (size_t)nb * m->record_bits;  // eight rows are whole bytes whatever the record width
+  uint32_t rows_per = row_bits ? (uint32_t)std::min<size_t>(m->d_out, std::max<size_t>(8, kUploadBytes * 8 / row_bits / 8 * 8)) : m->d_out;
+  rows_per = std::min(rows_per, (1u << 20));
+  float table[32];
+  for (uint32_t i = 0; i < 32; ++i) {
+    const uint32_t shell = i & 15u;
+    table[i] = shell ? (float)centroids[i >> 4] * (float)(1.0 / std::sqrt(16.0 * shell)) : 0.f;
+  }
+  hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->tiles), kTileTableBytes + (size_t)n_tiles * stride + kStepBytes + 256);  // a record's last step may reach past it
+  if (e != hipSuccess) return e;
+  const size_t code_room = ((row_bits * rows_per + 7) / 8 + 16 + 255) & ~(size_t)255;
+  const size_t scale_room = ((size_t)rows_per * 4 + 255) & ~(size_t)255, tail_room = (size_t)rows_per * m->tail_w * 4;
+  if ((e = grow_device(&rt->upload_buf, &rt->upload_bytes, code_room + scale_room + tail_room)) != hipSuccess) return e;
+  uint8_t* d_codes = rt->upload_buf;
+  float* d_scale = reinterpret_cast<float*>(d_codes + code_room);
+  float* d_tail = reinterpret_cast<float*>(d_codes + code_room + scale_room);
+  if ((e = hipMemcpyAsync(m->tiles, table, sizeof table, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
+  const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
+  for (uint32_t r0 = 0; r0 < m->d_out; r0 += rows_per) {
+    const uint32_t rows = std::min(rows_per, m->d_out - r0);
+    uint8_t* out = m->tiles + kTileTableBytes + (size_t)(r0 / kTileRows) * stride;
+    const size_t bytes = (row_bits * rows + 7) / 8;
+    if (bytes && (e = hipMemcpyAsync(d_codes, codes + row_bits * r0 / 8, bytes, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
+    if ((e = hipMemcpyAsync(d_scale, rscale + r0, (size_t)rows * 4, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
+    if (m->tail_w && (e = hipMemcpyAsync(d_tail, tail + (size_t)r0 * m->tail_w, (size_t)rows * m->tail_w * 4, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
+    const uint32_t heads = tile_count(rows) * kTileRows * (1u + m->tail_w);
+    hipLaunchKernelGGL(tile_heads_kernel, dim3((heads + 255u) / 256u), dim3(256), 0, rt->stream, d_scale, d_tail, out, rows, nb, m->tail_w);
+    if (nb) {
+      const uint64_t blocks = (uint64_t)tile_count(rows) * kTileRows * nb;
+      const uint32_t grid = (uint32_t)std::min<uint64_t>((blocks + 511) / 512, 2ull * cus);
+      if (m->record_bits == 48) hipLaunchKernelGGL(transcode_kernel<false>, dim3(grid), dim3(512), kLdsImageBytes, rt->stream, rt->tables, d_codes, out, rows, nb, m->tail_w);
+      else hipLaunchKernelGGL(transcode_kernel<true>, dim3(grid), dim3(512), kLdsImageBytes, rt->stream, rt->tables, d_codes, out, rows, nb, m->tail_w);
+    }
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  return hipStreamSynchronize(rt->stream);
 }
 
 static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uint32_t d_in,
@@ -1851,6 +892,7 @@ static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uin
   const size_t code_alloc = ((code_len + 3) & ~(size_t)3) + 64;  // slack so wide loads may run past the last record
   const size_t tail_len = (size_t)d_out * tail_w * sizeof(float);
   auto cleanup = [&](hipError_t e, const char* what) {
+    (void)hipFree(m->tiles);
     (void)hipFree(m->codes);
     (void)hipFree(m->rscale);
     (void)hipFree(m->tail);
@@ -1858,6 +900,7 @@ static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uin
     return hip_fail(e, what);
   };
   hipError_t e;
+  if ((e = upload_tiles(rt, m, centroids, rs.data(), tail, codes)) != hipSuccess) return cleanup(e, "upload_tiles");
   if ((e = hipMalloc(reinterpret_cast<void**>(&m->codes), code_alloc)) != hipSuccess) return cleanup(e, "hipMalloc(codes)");
   if ((e = hipMemset(m->codes, 0, code_alloc)) != hipSuccess) return cleanup(e, "hipMemset(codes)");
   if (code_len && (e = hipMemcpy(m->codes, codes, code_len, hipMemcpyHostToDevice)) != hipSuccess) return cleanup(e, "hipMemcpy(codes)");
@@ -1972,6 +1015,7 @@ int llvq_hip_matrix_from_record(llvq_rt* rt, const uint8_t* buf, size_t len, siz
 void llvq_hip_matrix_free(llvq_rt* rt, llvq_mat* m) {
   if (!m) return;
   if (rt) (void)hipSetDevice(rt->device);
+  (void)hipFree(m->tiles);
   (void)hipFree(m->codes);
   (void)hipFree(m->rscale);
   (void)hipFree(m->tail);
@@ -1991,68 +1035,6 @@ int llvq_hip_matrix_info(const llvq_mat* m, uint32_t* d_out, uint32_t* d_in, uin
 
 const char* llvq_hip_matrix_name(const llvq_mat* m) { return m ? m->name.c_str() : ""; }
 
-// Rows per tile.  The workgroups take tiles in rounds of `grid`; a launch lasts rounds x (a tile's
-// blocks + what a tile costs whatever its size: barriers, row sums, the wait for its first code
-// bytes, taken as kTileFixedBlocks blocks' worth).  For k = 1, 2, ... rounds the best tile is the
-// smallest that needs no more than k rounds; the cheapest of those that fit the tile capacity wins
-// (7168 rows of 213 blocks on 256 CUs: 14 rows in exactly 2 rounds, not 19 rows in 1.5).
-constexpr uint32_t kTileFixedBlocks = 400;
-static uint32_t pick_rows_per_tile(const llvq_mat* const* mats, int n, uint32_t nblocks, uint32_t grid, uint32_t tile) {
-  const uint32_t cap = nblocks ? (tile / nblocks ? tile / nblocks : 1u) : 0xFFFFFFFFu;
-  uint64_t total = 0;
-  for (int i = 0; i < n; ++i) total += mats[i]->d_out;
-  auto tiles_at = [&](uint32_t r) {
-    uint64_t t = 0;
-    for (int i = 0; i < n; ++i) t += (mats[i]->d_out + r - 1) / r;
-    return t;
-  };
-  uint32_t best = cap == 0xFFFFFFFFu ? (uint32_t)((total + grid - 1) / grid) : cap;
-  if (best < 1) best = 1;
-  uint64_t best_cost = ((tiles_at(best) + grid - 1) / grid) * ((uint64_t)best * nblocks + kTileFixedBlocks);
-  for (uint32_t k = 1; k <= 16; ++k) {
-    uint32_t r = (uint32_t)((total + (uint64_t)k * grid - 1) / ((uint64_t)k * grid));
-    if (r < 1) r = 1;
-    for (uint32_t tries = 0; tries < 64 && r <= cap && tiles_at(r) > (uint64_t)k * grid; ++tries) ++r;
-    if (r > cap || tiles_at(r) > (uint64_t)k * grid) continue;
-    const uint64_t cost = (uint64_t)k * ((uint64_t)r * nblocks + kTileFixedBlocks);
-    if (cost < best_cost || (cost == best_cost && r > best)) {
-      best_cost = cost;
-      best = r;
-    }
-  }
-  return best;
-}
-
-// Whether a launch over rows of this width can stage a derived activation where
-// its first tile's queues go.
-struct GemvShape {
-  uint32_t tile;
-  bool lean;
-  size_t lds;
-};
-
-// The kernel variant for rows of nblocks blocks: the full tile with the whole table
-// image in LDS where that fits, else the full tile with the lean image, else the half tile.
-static GemvShape pick_gemv_shape(uint32_t nblocks) {
-  GemvShape s{(uint32_t)kTileBlocks, false, gemv_lds_bytes(nblocks, kTileBlocks)};
-  if (s.lds <= 160 * 1024) return s;
-  s = GemvShape{(uint32_t)kTileBlocks, true, gemv_lds_bytes(nblocks, kTileBlocks, kLdsImageBytesLean)};
-  if (s.lds <= 160 * 1024) return s;
-  return GemvShape{(uint32_t)kSmallTileBlocks, false, gemv_lds_bytes(nblocks, kSmallTileBlocks)};
-}
-
-static bool prologue_fits(const llvq_mat* m0) {
-  return (size_t)m0->d_in * 2 <= (size_t)pick_gemv_shape(m0->nblocks).tile * 6 + 32;
-}
-
-// Whether a launch over rows of this width can rotate its own activation: the f32
-// values take the place of the first tile's queues and partial sums.
-static bool rotation_fits(const llvq_mat* m0) {
-  if (m0->record_bits != 48) return false;  // the dense-stream kernels have no in-launch rotation: a kernel of its own rotates
-  const size_t tile = pick_gemv_shape(m0->nblocks).tile;
-  return (size_t)m0->d_in * 4 + 64 <= tile * 6 + 32 + tile * 8;
-}
-
 struct Prologue {
   uint32_t kind = kPrologueNone;
   const void* x2 = nullptr;
@@ -2061,65 +1043,56 @@ struct Prologue {
   float eps = 0.f;
 };
 
+// Whether the digit planes of rows this wide fit LDS beside what else a launch keeps there.
+static bool gemv_fits(const llvq_mat* m, bool f32_out, bool rotated) {
+  return m->nblocks <= kGemvMaxBlocks && gemv_tiles_lds_bytes(m->nblocks, m->d_in, f32_out, rotated) <= 160 * 1024;
+}
+
+// One launch of gemv_tiles_kernel over n <= kMaxGroup matrices of equal d_in and basis.
 static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, void* const* y,
                         int y_dtype, const Prologue* pro = nullptr, const float* x_f32 = nullptr,
                         const llvq_rt::DevRotation* rot = nullptr) {
   const llvq_mat* m0 = mats[0];
   if (y_dtype != LLVQ_F32 && y_dtype != LLVQ_F16) return fail(LLVQ_ERR_INVALID_ARGUMENT, "gemv: unknown output dtype");
-  const GemvShape shape = pick_gemv_shape(m0->nblocks);
-  const uint32_t tile = shape.tile;
-  const size_t lds = shape.lds;
-  if (lds > 160 * 1024 || m0->nblocks > tile)
+  const bool f32 = y_dtype == LLVQ_F32, rotated = rot || x_f32;
+  if (!gemv_fits(m0, f32, rot != nullptr))
     return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": d_in " + std::to_string(m0->d_in) + " does not fit the LDS activation tile");
-  // as many workgroups as fit a CU's 160 KB of LDS side by side
-  const uint32_t per_cu = (uint32_t)((160 * 1024) / lds) < 1u ? 1u : (uint32_t)((160 * 1024) / lds);
-  const uint32_t wg_per_cu = per_cu > (uint32_t)(2048 / kWgThreads) ? (uint32_t)(2048 / kWgThreads) : per_cu;
-  const uint32_t grid_cap = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256) * wg_per_cu;
-  GroupArgs a{};
-  a.tables = rt->tables;
-  a.x = reinterpret_cast<const __half*>(x);
-  a.x_f32 = x_f32;
+  GemvArgs a{};
+  a.in.x = reinterpret_cast<const __half*>(x);
+  a.in.x_f32 = x_f32;
   if (pro) {
-    if ((size_t)m0->d_in * 2 > (size_t)tile * 6 + 32)
-      return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": d_in too wide for a fused activation prologue");
-    a.prologue = pro->kind;
-    a.x2 = reinterpret_cast<const __half*>(pro->x2);
-    a.norm_w = reinterpret_cast<const __half*>(pro->norm_w);
-    a.resid_out = reinterpret_cast<__half*>(pro->resid_out);
-    a.eps = pro->eps;
+    a.in.prologue = pro->kind;
+    a.in.x2 = reinterpret_cast<const __half*>(pro->x2);
+    a.in.norm_w = reinterpret_cast<const __half*>(pro->norm_w);
+    a.in.resid_out = reinterpret_cast<__half*>(pro->resid_out);
+    a.in.eps = pro->eps;
   }
   if (rot) {
-    if (!rotation_fits(m0) || rot->n != m0->d_in)
-      return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": d_in too wide for a rotation inside the launch");
-    a.rot_signbits = rot->signbits;
-    a.rot_small = rot->small;
-    a.rot_inv = rot->inv;
-    a.rot_m = rot->m;
-    a.rot_k = rot->k;
+    a.in.rot_signbits = rot->signbits;
+    a.in.rot_small = rot->small;
+    a.in.rot_inv = rot->inv;
+    a.in.rot_m = rot->m;
+    a.in.rot_k = rot->k;
   }
-  a.nblocks = m0->nblocks;
+  a.nb = m0->nblocks;
   a.tail_w = m0->tail_w;
   a.n_mats = (uint32_t)n;
-  a.inv_nblocks = m0->nblocks ? 1.0f / (float)m0->nblocks : 0.f;
-  a.rows_per_tile = pick_rows_per_tile(mats, n, m0->nblocks, grid_cap, tile);
-  uint32_t tiles = 0;
+  a.split_shift = gemv_split_shift(m0->nblocks);
   for (int i = 0; i < n; ++i) {
-    a.m[i] = MatArg{mats[i]->codes, mats[i]->rscale, mats[i]->tail, y[i], mats[i]->g[0], mats[i]->g[1],
-                    mats[i]->d_out, tiles};
-    tiles += (mats[i]->d_out + a.rows_per_tile - 1) / a.rows_per_tile;
+    a.m[i] = TileMat{mats[i]->tiles, y[i], mats[i]->d_out, a.n_tiles};
+    a.n_tiles += tile_count(mats[i]->d_out);
   }
-  a.n_tiles = tiles;
-  const uint32_t grid = tiles < grid_cap ? tiles : grid_cap;
-  const bool wide = m0->record_bits != 48;
-  for (int i = 1; i < n; ++i)
-    if (mats[i]->record_bits != m0->record_bits)
-      return fail(LLVQ_ERR_INVALID_ARGUMENT, mats[i]->name + ": matrices of one launch must share their shell cap");
-  if (wide && (tile != (uint32_t)kTileBlocks || rot))
-    return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": rows too wide for the cap-13 kernels");
-  const void* kernel = wide ? gemv_kernel_wide(y_dtype == LLVQ_F32, shape.lean) : gemv_kernel(y_dtype == LLVQ_F32, tile, shape.lean, rot != nullptr);
+  // Teams go to as many CUs as there are records for, then to the same CU, up to sixteen wavefronts: a small launch
+  // is short because every CU has a part of it, a large one because a CU keeps sixteen wavefronts' loads in flight.
+  // The in-launch rotation and the wide rows are written for a full workgroup.
+  const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), most = kGemvMaxWaves >> a.split_shift;
+  uint32_t teams = (a.n_tiles + cus - 1u) / cus;
+  if (teams > most || rotated || gemv_wide(a.nb)) teams = most;
+  const uint32_t grid = std::min(cus, (a.n_tiles + teams - 1u) / teams);
+  const int src = rotated ? kSrcRotated : a.in.prologue == kPrologueSiluMul ? kSrcSiluMul : a.in.prologue == kPrologueAddRmsNorm ? kSrcAddRmsNorm : kSrcF16;
   void* params[] = {&a};
-  HIP_TRY(hipLaunchKernel(kernel, dim3(grid), dim3(kWgThreads), params, lds, rt->stream));
-  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipLaunchKernel(gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(grid), dim3((teams << a.split_shift) * 64u), params,
+                          gemv_tiles_lds_bytes(a.nb, m0->d_in, f32, rot != nullptr), rt->stream));
   return LLVQ_OK;
 }
 
@@ -2143,7 +1116,7 @@ static int launch_rotate(llvq_rt* rt, const llvq_rt::DevRotation* rot, const voi
 }
 
 static bool same_basis(const llvq_mat* a, const llvq_mat* b) {
-  return a->record_bits == b->record_bits && a->has_rotation == b->has_rotation && (!a->has_rotation || a->rotation_seed == b->rotation_seed);
+  return a->has_rotation == b->has_rotation && (!a->has_rotation || a->rotation_seed == b->rotation_seed);
 }
 
 // One activation through projections that share it: consecutive matrices in the
@@ -2158,7 +1131,7 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
     int j = i + 1;
     while (j < n && j - i < kMaxGroup && same_basis(mats[i], mats[j])) ++j;
     const float* xr = nullptr;
-    if (mats[i]->has_rotation && rotation_fits(mats[i])) {
+    if (mats[i]->has_rotation && gemv_fits(mats[i], y_dtype == LLVQ_F32, true)) {
       const int rc = launch_group(rt, mats + i, j - i, x, y + i, y_dtype, pro, nullptr, mats[i]->rot);
       if (rc) return rc;
       i = j;
@@ -2246,36 +1219,10 @@ struct SeqSpec {
   Prologue pro{};
 };
 
-// three byte planes of the activation for f32 results, two for binary16 results, as gemv_tiles_kernel
-static const void* seq_kernel(uint32_t tile, bool lean, bool f32, bool wide) {
-  if (wide) {  // cap-13 matrices: full tiles only
-    if (f32) return lean ? reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, true, 3, true>) : reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, false, 3, true>);
-    return lean ? reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, true, 2, true>) : reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, false, 2, true>);
-  }
-  if (f32) {
-    if (lean) return reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, true, 3>);
-    if (tile == (uint32_t)kTileBlocks) return reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, false, 3>);
-    return reinterpret_cast<const void*>(gemv_seq_kernel<kSmallTileBlocks, false, 3>);
-  }
-  if (lean) return reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, true, 2>);
-  if (tile == (uint32_t)kTileBlocks) return reinterpret_cast<const void*>(gemv_seq_kernel<kTileBlocks, false, 2>);
-  return reinterpret_cast<const void*>(gemv_seq_kernel<kSmallTileBlocks, false, 2>);
-}
-
-// The kernel variant for a sequence whose widest rows have max_nb blocks (as pick_gemv_shape).
-static GemvShape pick_seq_shape(uint32_t max_nb) {
-  GemvShape s{(uint32_t)kTileBlocks, false, gemv_seq_lds_bytes(max_nb, kTileBlocks, kLdsImageBytes)};
-  if (s.lds <= 160 * 1024) return s;
-  s = GemvShape{(uint32_t)kTileBlocks, true, gemv_seq_lds_bytes(max_nb, kTileBlocks, kLdsImageBytesLean)};
-  if (s.lds <= 160 * 1024) return s;
-  return GemvShape{(uint32_t)kSmallTileBlocks, false, gemv_seq_lds_bytes(max_nb, kSmallTileBlocks, kLdsImageBytes)};
-}
-
 constexpr uint32_t kSeqSpinLimit = 1u << 20;  // polls of a wait before it gives up (about a second)
 
 static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) {
   if (n <= 0) return fail(LLVQ_ERR_INVALID_ARGUMENT, "sequence_create: no items");
-  uint32_t max_nb = 0;
   bool dependent = false;
   for (int i = 0; i < n; ++i) {
     const SeqSpec& sp = specs[i];
@@ -2291,27 +1238,27 @@ static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) 
       if (m->record_bits != specs[0].mats[0]->record_bits) return fail(LLVQ_ERR_UNSUPPORTED, m->name + ": the matrices of a sequence share one shell cap");
     }
     if (sp.mats[0]->nblocks > 1024u) return fail(LLVQ_ERR_UNSUPPORTED, sp.mats[0]->name + ": rows wider than 24 576 columns do not fit a sequence");
-    max_nb = std::max(max_nb, sp.mats[0]->nblocks);
     dependent |= sp.after_previous;
   }
-  const GemvShape shape = pick_seq_shape(max_nb);
-  if (shape.lds > 160 * 1024 || max_nb > shape.tile) return fail(LLVQ_ERR_UNSUPPORTED, "sequence_create: the widest rows do not fit the LDS activation tile");
-  const bool wide = specs[0].mats[0]->record_bits != 48;
-  if (wide && shape.tile != (uint32_t)kTileBlocks) return fail(LLVQ_ERR_UNSUPPORTED, "sequence_create: rows this wide do not fit a sequence of cap-13 matrices");
-  for (int i = 0; i < n; ++i)
-    if (specs[i].pro.kind == kPrologueAddRmsNorm && specs[i].mats[0]->d_in > 6u * kWgThreads)
-      return fail(LLVQ_ERR_UNSUPPORTED, specs[i].mats[0]->name + ": d_in too wide for a fused norm inside a sequence");
+  const bool f32 = specs[0].y_dtype == LLVQ_F32;
+  bool prologue = false, wide = false;
+  uint32_t max_blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    prologue |= specs[i].pro.kind != kPrologueNone;
+    wide |= gemv_wide(specs[i].mats[0]->nblocks);
+    max_blocks = std::max(max_blocks, gemv_plane_blocks(specs[i].mats[0]->nblocks));
+  }
+  const size_t lds = gemv_seq_lds_bytes(max_blocks, f32);
+  if (lds > 160 * 1024) return fail(LLVQ_ERR_UNSUPPORTED, "sequence_create: the widest rows do not fit the LDS activation tile");
   const uint32_t grid_cap = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
-  std::vector<SeqTile> tiles;
+  std::vector<SeqUnit> units;
   std::vector<SeqItem> items((size_t)n);
+  std::vector<uint64_t> cost;  // bytes of the units so far, behind each unit
+  uint64_t bytes = 0;
   for (int i = 0; i < n; ++i) {
     const SeqSpec& sp = specs[i];
     const llvq_mat* m0 = sp.mats[0];
-    const uint32_t nb = m0->nblocks;
-    // Ordered items, and an item that is a launch by itself, are balanced one by one, like launches (everyone waits
-    // for an item's slowest workgroup); independent items fill their tiles, because the round-robin runs on across
-    // item boundaries.
-    uint32_t rpt = (dependent || n == 1) ? pick_rows_per_tile(sp.mats, sp.n, nb, grid_cap, shape.tile) : (nb ? std::max(1u, shape.tile / nb) : 256u);
+    const uint32_t nb = m0->nblocks, stride = tile_stride(nb, m0->tail_w), per = (kGemvMaxWaves >> gemv_split_shift(nb)) * kTileRows;
     SeqItem& I = items[(size_t)i];
     std::memset(&I, 0, sizeof I);
     I.x = reinterpret_cast<const __half*>(sp.x);
@@ -2322,75 +1269,79 @@ static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) 
     I.prologue = sp.pro.kind;
     I.nb = nb;
     I.tail_w = m0->tail_w;
-    I.inv_nb = nb ? 1.0f / (float)nb : 0.f;
-    I.y_f16 = sp.y_dtype == LLVQ_F16 ? 1u : 0u;
-    I.first_tile = (uint32_t)tiles.size();
+    I.first_unit = (uint32_t)units.size();
     I.wait_item = sp.after_previous ? (uint32_t)(i - 1) : kSeqNoWait;
     I.signals = (i + 1 < n && specs[i + 1].after_previous) ? 1u : 0u;
-    const size_t ysz = sp.y_dtype == LLVQ_F16 ? 2 : 4;
+    const size_t ysz = f32 ? 4 : 2;
     for (int j = 0; j < sp.n; ++j) {
       const llvq_mat* m = sp.mats[j];
-      for (uint32_t r0 = 0; r0 < m->d_out; r0 += rpt) {
-        SeqTile t{};
-        t.rows = std::min(rpt, m->d_out - r0);
-        t.nblk = t.rows * nb;
-        const uint64_t first_bit = (uint64_t)r0 * nb * m->record_bits;  // 6-byte records begin on a byte; dense 49-bit blocks need not
-        t.codes = m->codes + (first_bit >> 3);
-        t.bit0 = (uint32_t)(first_bit & 7u);
-        t.rscale = m->rscale + r0;
-        t.tail = m->tail + (size_t)r0 * m->tail_w;
+      // Ordered items are spread over all workgroups as a launch of their own would be: everyone waits for the slowest.
+      uint32_t rows_per = per;
+      if (dependent) rows_per = std::min(per, std::max(1u, (tile_count(m->d_out) + grid_cap - 1u) / grid_cap) * kTileRows);
+      for (uint32_t r0 = 0; r0 < m->d_out; r0 += rows_per) {
+        SeqUnit t{};
+        t.rec = m->tiles + kTileTableBytes + (size_t)(r0 / kTileRows) * stride;
+        t.table = reinterpret_cast<const uint32_t*>(m->tiles);
         t.y = reinterpret_cast<uint8_t*>(sp.y[j]) + (size_t)r0 * ysz;
-        t.g0 = m->g[0];
-        t.g1 = m->g[1];
+        t.rows = std::min(rows_per, m->d_out - r0);
         t.item = (uint32_t)i;
-        tiles.push_back(t);
+        units.push_back(t);
+        bytes += (uint64_t)tile_count(t.rows) * stride + 1024u;
+        cost.push_back(bytes);
       }
     }
   }
-  if (tiles.size() > 0x7FFFFFFFu) return fail(LLVQ_ERR_UNSUPPORTED, "sequence_create: too many tiles");
-  const uint32_t n_tiles = (uint32_t)tiles.size();
-  const uint32_t grid = std::min(n_tiles, grid_cap);
+  if (units.size() > 0x7FFFFFFFu) return fail(LLVQ_ERR_UNSUPPORTED, "sequence_create: too many units");
+  const uint32_t n_units = (uint32_t)units.size();
+  const uint32_t grid = std::min(n_units, grid_cap);
   for (int i = 0; i < n; ++i) {
-    const uint32_t t0 = items[(size_t)i].first_tile, t1 = i + 1 < n ? items[(size_t)i + 1].first_tile : n_tiles;
+    const uint32_t t0 = items[(size_t)i].first_unit, t1 = i + 1 < n ? items[(size_t)i + 1].first_unit : n_units;
     items[(size_t)i].expected = std::min(t1 - t0, grid);
   }
   for (int i = 0; i < n; ++i)
     if (items[(size_t)i].wait_item != kSeqNoWait) items[(size_t)i].wait_expected = items[items[(size_t)i].wait_item].expected;
+  // runs of equal bytes: workgroup b ends where the units before its end make up (b + 1) / grid of all bytes
+  std::vector<uint32_t> runs((size_t)grid + 1);
+  for (uint32_t b = 0, at = 0; b < grid; ++b) {
+    runs[b] = at;
+    const uint64_t want = bytes * (b + 1) / grid;
+    while (at < n_units && (b + 1 == grid || cost[at] <= want)) ++at;
+  }
+  runs[grid] = n_units;
   HIP_TRY(hipSetDevice(rt->device));
   auto* q = new llvq_seq();
-  const size_t off_items = tiles.size() * sizeof(SeqTile);
-  const size_t off_counters = (off_items + items.size() * sizeof(SeqItem) + 255) & ~(size_t)255;
+  const size_t off_items = units.size() * sizeof(SeqUnit);
+  const size_t off_runs = off_items + items.size() * sizeof(SeqItem);
+  const size_t off_counters = (off_runs + runs.size() * 4 + 255) & ~(size_t)255;
   const size_t off_status = off_counters + (((size_t)n * 4 + 255) & ~(size_t)255);
   const size_t total = off_status + 256;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&q->blob), total);
   if (e == hipSuccess) e = hipMemset(q->blob, 0, total);
-  if (e == hipSuccess) e = hipMemcpy(q->blob, tiles.data(), off_items, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(q->blob, units.data(), off_items, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(q->blob + off_items, items.data(), items.size() * sizeof(SeqItem), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(q->blob + off_runs, runs.data(), runs.size() * 4, hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     (void)hipFree(q->blob);
     delete q;
     return hip_fail(e, "sequence tables");
   }
-  q->args.tables = rt->tables;
-  q->args.tiles = reinterpret_cast<const SeqTile*>(q->blob);
+  q->args.units = reinterpret_cast<const SeqUnit*>(q->blob);
   q->args.items = reinterpret_cast<const SeqItem*>(q->blob + off_items);
-  q->args.n_tiles = n_tiles;
-  q->args.max_nb = max_nb;
+  q->args.runs = dependent ? nullptr : reinterpret_cast<const uint32_t*>(q->blob + off_runs);
+  q->args.n_units = n_units;
+  q->args.max_blocks = max_blocks;
   q->args.counters = reinterpret_cast<uint32_t*>(q->blob + off_counters);
   q->args.status = reinterpret_cast<uint32_t*>(q->blob + off_status);
   q->own_status = q->args.status;
   q->args.run = 0;
   q->args.spin_limit = kSeqSpinLimit;
   q->args.hold_item = kSeqNoWait;
-  q->args.stamps = nullptr;
-  q->args.item0 = items[0];
-  q->tile = shape.tile;
-  q->lean = shape.lean;
-  q->f32 = specs[0].y_dtype == LLVQ_F32;
-  q->wide = wide;
+  const int mode = prologue ? (wide ? kSeqPrologueWide : kSeqPrologue)
+                            : dependent ? (wide ? kSeqPrologueWide : kSeqOrdered) : (wide ? kSeqIndependentWide : kSeqIndependent);
+  q->kernel = f32 ? seq_kernel_of<float>(mode) : seq_kernel_of<__half>(mode);
   // the activation planes of a wide row push dynamic LDS past the 64 KB default
-  (void)hipFuncSetAttribute(seq_kernel(shape.tile, shape.lean, q->f32, q->wide), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  q->lds = shape.lds;
+  (void)hipFuncSetAttribute(q->kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  q->lds = lds;
   q->grid = grid;
   q->n_items = (uint32_t)n;
   *out = q;
@@ -2401,12 +1352,11 @@ static int seq_run(llvq_rt* rt, llvq_seq* q) {
   q->args.run += 1;
   SeqArgs a = q->args;
   void* params[] = {&a};
-  const void* kernel = seq_kernel(q->tile, q->lean, q->f32, q->wide);
-  // An ordinary launch, also with ordered items: at most one workgroup per CU (by its LDS) and no more workgroups than
+  // An ordinary launch, also with ordered items: sixteen wavefronts a workgroup and no more workgroups than
   // CUs, so on a device this stream has to itself every workgroup is resident and the waits end.  (A cooperative launch
   // would guarantee it, but costs some 200 us per launch here: 4B decode fell from 237 to 85 tokens/s with it.)  Should
   // another queue hold CUs for longer than the bounded wait, the run gives up and says so; it cannot hang.
-  HIP_TRY(hipLaunchKernel(kernel, dim3(q->grid), dim3(kWgThreads), params, q->lds, rt->stream));
+  HIP_TRY(hipLaunchKernel(q->kernel, dim3(q->grid), dim3(1024), params, q->lds, rt->stream));
   HIP_TRY(hipGetLastError());
   q->args.hold_item = kSeqNoWait;
   return LLVQ_OK;
@@ -2453,16 +1403,6 @@ int llvq_hip_sequence_status(llvq_rt* rt, llvq_seq* seq) {
   if (rc) return rc;
   return fail(LLVQ_ERR_DEVICE, "sequence: a workgroup gave up waiting for an item; the run's outputs are incomplete");
 }
-
-#ifdef LLVQ_SEQ_STAMPS
-// Tuning builds only: where the next runs of `seq` store their phase timestamps (device memory of
-// grid x kSeqStampTiles x 8 64-bit words, or null).
-extern "C" int llvq_hip_sequence_debug(llvq_seq* seq, void* stamps_dev, uint32_t* grid) {
-  seq->args.stamps = reinterpret_cast<unsigned long long*>(stamps_dev);
-  if (grid) *grid = seq->grid;
-  return LLVQ_OK;
-}
-#endif
 
 int llvq_hip_sequence_tune(llvq_seq* seq, uint32_t spin_limit, int hold_item) {
   if (!seq) return fail(LLVQ_ERR_INVALID_ARGUMENT, "sequence_tune: null sequence");
@@ -3034,8 +1974,8 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   // their prologue runs as a kernel of its own.
   auto project = [&](const llvq_mat* const* mats, int n, const __half* x, void* const* outs, const Prologue& pro) -> int {
     // every launch of the group can derive (and, in a rotated basis, rotate) the activation itself
-    bool fused = prologue_fits(mats[0]);
-    for (int i = 0; i < n; ++i) fused &= !mats[i]->has_rotation || rotation_fits(mats[i]);
+    bool fused = true;
+    for (int i = 0; i < n; ++i) fused &= gemv_fits(mats[i], false, mats[i]->has_rotation);
     if (fused) return forward_group(rt, mats, n, x, outs, LLVQ_F16, &pro);
     const __half* staged = nullptr;
     if (pro.kind == kPrologueAddRmsNorm) {
@@ -3580,11 +2520,5 @@ int llvq_hip_decoder_prefill(llvq_decoder* d, const uint32_t* tokens, size_t n, 
   HIP_TRY(hipStreamSynchronize(d->rt->stream));
   return LLVQ_OK;
 }
-
-#ifdef LLVQ_SEQ_STAMPS
-llvq_seq* llvq_hip_decoder_debug_sequence(llvq_decoder* d, int index) {
-  return d && index >= 0 && (size_t)index < d->seqs.size() ? d->seqs[(size_t)index] : nullptr;
-}
-#endif
 
 }  // extern "C"
