@@ -1,6 +1,6 @@
-// How a batched launch shares its K-slices out over the workgroups: plain integer
-// arithmetic, used by the kernels, by the host code that sizes the workspace, and by
-// the host tests.
+// How a batched launch's K-slices are shared out over a fixed number of workgroups: plain integer
+// arithmetic.  The partial sums of this sharing are what llvq_hip_gemm_static's limit on shapes is
+// stated in (static_admission_bytes).
 //
 // A band (64 weight rows) is `spb` slices.  Where a launch has at least as many bands as
 // workgroups, every workgroup first walks `whole` bands alone, from the first slice to the

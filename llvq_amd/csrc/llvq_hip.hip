@@ -55,25 +55,15 @@ struct GlobalTables {
   const uint16_t* wide_lut2;
 };
 
-constexpr size_t kLdsImageBytesLean = offsetof(TableImage, golay);  // without the Golay words and the support-arrangement table
-static_assert(kLdsImageBytesLean % 16 == 0, "LDS part of the table image is copied in 16-byte units");
-constexpr size_t kLdsImageBytesLeanest = offsetof(TableImage, lut);  // without the class lookup table either
-static_assert(kLdsImageBytesLeanest % 16 == 0, "LDS part of the table image is copied in 16-byte units");
-
-// kFull: the whole image goes to LDS; otherwise its last two tables (33 KB) are
-// read through L2, for a kernel that needs the LDS for something else.  kLut = false
-// leaves the 4 KB class lookup table (one read per block) in L2 as well.
 // kWide: for 48-bit indices the class records, class starts and class-find tables are the full ones in device
 // memory (read through L2); the LDS copies cover what a 47-bit index reaches.
-template <bool kFull = true, bool kLut = true, bool kWide = false>
+template <bool kWide = false>
 __device__ __forceinline__ DecodeTables stage_tables(uint8_t* smem, const GlobalTables& g) {
-  static_assert(kLut || !kFull, "the tables that stay in L2 are the image's last ones");
   const uint4* src = reinterpret_cast<const uint4*>(g.image);
   uint4* dst = reinterpret_cast<uint4*>(smem);
-  constexpr size_t kBytes = kFull ? sizeof(TableImage) : (kLut ? kLdsImageBytesLean : kLdsImageBytesLeanest);
   // five loads per lane in flight at a time (one pass for a 1024-lane workgroup): a load and its
   // store per loop iteration would pay the L2 latency once per iteration
-  constexpr uint32_t kUnits = (uint32_t)(kBytes / 16), kLast = kUnits - 1u;
+  constexpr uint32_t kUnits = (uint32_t)(sizeof(TableImage) / 16), kLast = kUnits - 1u;
   const uint32_t st = blockDim.x;
   for (uint32_t i0 = threadIdx.x; i0 < kUnits; i0 += 5u * st) {
     const uint32_t i1 = i0 + st, i2 = i1 + st, i3 = i2 + st, i4 = i3 + st;
@@ -86,11 +76,10 @@ __device__ __forceinline__ DecodeTables stage_tables(uint8_t* smem, const Global
     if (i4 < kUnits) dst[i4] = r4;
   }
   const TableImage* s = reinterpret_cast<const TableImage*>(smem);
-  const TableImage* far = kFull ? s : g.image;
   if constexpr (kWide)
-    return DecodeTables{far->golay, g.cls, g.wide_fast, g.starts, g.starts, g.wide_lut, g.wide_lut2, s->rcp, far->on_lut, g.off_lut,
+    return DecodeTables{s->golay, g.cls, g.wide_fast, g.starts, g.starts, g.wide_lut, g.wide_lut2, s->rcp, s->on_lut, g.off_lut,
                         g.expand, s->pdep4, s->step - kTailSlots * 25 * 2, s->tail_meta, g.tail_codes};
-  return DecodeTables{far->golay, g.cls, s->fast, s->starts, g.starts, kLut ? s->lut : g.image->lut, kLut ? s->lut2 : g.image->lut2, s->rcp, far->on_lut, g.off_lut,
+  return DecodeTables{s->golay, g.cls, s->fast, s->starts, g.starts, s->lut, s->lut2, s->rcp, s->on_lut, g.off_lut,
                       g.expand, s->pdep4, s->step - kTailSlots * 25 * 2, s->tail_meta, g.tail_codes};
 }
 
@@ -134,7 +123,7 @@ __global__ __launch_bounds__(256) void decode_blocks_kernel(GlobalTables g, cons
                                                             uint8_t* __restrict__ gains,
                                                             uint8_t* __restrict__ shells) {
   extern __shared__ __align__(16) uint8_t smem[];
-  const DecodeTables T = stage_tables<true, true, WIDE>(smem, g);
+  const DecodeTables T = stage_tables<WIDE>(smem, g);
   __syncthreads();
   if constexpr (WIDE) {
     // 49-bit blocks of a dense stream (shell cap 13): block b is the 49 bits from bit 49 b on, read byte by byte
@@ -171,9 +160,7 @@ __global__ __launch_bounds__(256) void decode_blocks_kernel(GlobalTables g, cons
 }
 
 // ---- what the product kernels share -----------------------------------------------
-constexpr int kWgThreads = 1024;
 constexpr int kMaxGroup = 4;
-constexpr int kGenericSlots = 64; // queue of blocks that take the generic walk
 
 // What a launch may do to produce its activation before the product.
 enum : uint32_t {
@@ -338,157 +325,6 @@ __device__ __forceinline__ void store_half(__half* p, __half v) {
     *p = v;
 }
 
-// The same number as one the compiler can relate to nothing it knows.  Used where what it would derive costs
-// more than the plain form: the address of an element of a second array with the same index (formed from the
-// first element's address by a 64-bit multiply-add), a table key re-shaped into three instructions, a 16-bit
-// entry zero-extended again.
-__device__ __forceinline__ uint32_t detached(uint32_t v) {
-  asm("" : "+v"(v));
-  return v;
-}
-
-static_assert(kLutFinal == 0x8000u, "the final flag is the top bit of a 16-bit entry");
-
-// Classes of NB indices as records hold them (1 .. N, below 2^47; 0 walks the tables harmlessly) side by side:
-// the class, its first index and its decoder
-// (kLutKind*).  Two table probes and one comparison each, every read unconditional so that the NB
-// reads of a step go out together; the indices whose bucket meets several class starts (0.09 % of
-// uniform draws) take the halving search afterwards, under a wavefront-wide test.
-template <int NB, bool WIDE = false>
-__device__ __forceinline__ void find_classes(const DecodeTables& T, const uint32_t (&zlo)[NB], const uint32_t (&zhi)[NB],
-                                             uint32_t (&ci)[NB], uint64_t (&start)[NB], uint32_t (&kind)[NB]) {
-  uint32_t e[NB], e2[NB];
-  // (48-bit indices reach the whole first-level table; T's class-find tables are then the full ones, in device memory)
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    // a bit-field extract and a scaled add; the entry as the 32-bit word the load returns (upper half zero)
-    const uint32_t key = detached(__builtin_amdgcn_ubfe(zhi[i], kLutShift - 32, WIDE ? 12 : 11));
-    e[i] = detached(T.lut[key]);
-  }
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    // a first-level entry that is not final is where its second-level table begins, a multiple of the span
-    const uint32_t at = (__builtin_amdgcn_alignbit(zhi[i], zlo[i], kLut2Shift) & (uint32_t)(kLut2Span - 1)) | e[i];
-    e2[i] = T.lut2[e[i] < kLutFinal ? at : 0u];  // the flag is the entry's top bit: one comparison
-  }
-  uint64_t s0[NB], s1[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    e[i] = e[i] < kLutFinal ? e2[i] : e[i];
-    s0[i] = T.starts[e[i] & 511u];
-    s1[i] = T.starts[(e[i] & 511u) + 1u];
-  }
-  uint32_t wide = 0;
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const uint64_t z = ((uint64_t)zhi[i] << 32) | zlo[i];
-    const bool up = s1[i] <= z;
-    ci[i] = (e[i] & 511u) + (up ? 1u : 0u);
-    start[i] = up ? s1[i] : s0[i];
-    kind[i] = (e[i] >> (up ? 11 : 9)) & 3u;
-    wide |= e[i] & kLutWide;
-  }
-  if (__any(wide != 0u)) {
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if (e[i] & kLutWide) {
-        const uint32_t c = class_from_entry(T, e[i], ((uint64_t)zhi[i] << 32) | zlo[i]);
-        const uint32_t meta = T.fast[c].meta, path = (meta >> kMetaPathShift) & 3u;
-        ci[i] = c;
-        start[i] = T.starts_far[c];
-        kind[i] = path == kPathOdd ? (uint32_t)kLutKindOdd
-                                   : path == kPathEven ? ((meta & kMetaSecondFree) ? (uint32_t)kLutKindEvenSecond : (uint32_t)kLutKindEven)
-                                                       : (uint32_t)kLutKindGeneric;
-      }
-  }
-}
-
-// P1 of the GEMV and GEMM kernels: each of the LANES lanes taking part (the first
-// LANES of the workgroup) classifies up to NB blocks of the tile and bins them: slots first, first + LANES, ...
-// (`first` is the lane's index in the workgroup unless the caller hands out the slots itself).
-// `record(f)` returns the 48-bit record of tile slot f < nblk;
-// `origin(f)` is called for an origin block (index 0) and returns whether the
-// block must still be queued (flagged, with the odd-coset blocks) or is settled.
-// Queue entry: slot (12 bits) | class << 16 | gain << 25 | origin << 30 | generic walk << 31.
-// The halving searches of a lane's blocks run side by side (independent LDS
-// chains); a wavefront claims queue space with one atomic per queue.  Blocks of
-// the rare generic classes take ~2000 dependent instructions: they go to a
-// small queue that P2 hands out first; what does not fit rides in the odd queue.
-constexpr uint32_t kEntryOrigin = 0x40000000u, kEntryGeneric = 0x80000000u;
-template <int NB, int LANES = kWgThreads, typename RecordFn, typename OriginFn>
-__device__ __forceinline__ void classify_and_bin(const DecodeTables& T, uint32_t nblk, uint32_t capacity, uint32_t* queue,
-                                                 uint32_t* gqueue, uint32_t* ctrl, RecordFn record, OriginFn origin,
-                                                 uint32_t first = threadIdx.x) {
-  const uint32_t tid = first, lane = threadIdx.x & 63u;
-  uint32_t entry[NB], ci[NB];
-  uint64_t zi[NB];  // the record's index, ~0 when the lane has no block / an origin
-  bool queued_origin[NB];
-  // Every LDS read of this phase is unconditional (a lane without a block reads a valid slot and
-  // ignores it), so that the NB reads of a step go out together: a guarded read is waited for
-  // where it is issued, and the phase is a chain of dependent reads.
-  uint64_t recs[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) recs[i] = record(min(tid + (uint32_t)i * LANES, nblk - 1u));
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const uint32_t f = tid + (uint32_t)i * LANES;
-    zi[i] = ~0ULL;
-    entry[i] = 0;
-    ci[i] = 0;
-    queued_origin[i] = false;
-    if (f < nblk) {
-      const uint64_t rec = recs[i];
-      entry[i] = f | ((uint32_t)(rec & 1) << 25);
-      if ((rec >> 1) == 0) {  // the origin decodes to zero whatever the gain (index.rs:335-337)
-        queued_origin[i] = origin(f);
-        if (queued_origin[i]) entry[i] |= kEntryOrigin;
-      } else {
-        zi[i] = rec >> 1;
-      }
-    }
-  }
-  uint32_t zlo[NB], zhi[NB], kind[NB];
-  uint64_t start[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {  // a lane without a block, or with an origin, walks the tables with index 0
-    zlo[i] = zi[i] != ~0ULL ? (uint32_t)zi[i] : 0u;
-    zhi[i] = zi[i] != ~0ULL ? (uint32_t)(zi[i] >> 32) : 0u;
-  }
-  find_classes<NB>(T, zlo, zhi, ci, start, kind);
-  uint32_t path[NB], odd_rank[NB], even_rank[NB], n_o = 0, n_e = 0;
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const uint32_t decoder = kind[i] == kLutKindOdd ? (uint32_t)kPathOdd : kind[i] == kLutKindGeneric ? (uint32_t)kPathGeneric : (uint32_t)kPathEven;
-    path[i] = zi[i] != ~0ULL ? decoder : (queued_origin[i] ? (uint32_t)kPathOdd : 3u);
-    entry[i] |= ci[i] << 16;
-    if (path[i] == kPathGeneric) {
-      entry[i] |= kEntryGeneric;
-      const uint32_t slot = atomicAdd(&ctrl[2], 1u);
-      if (slot < (uint32_t)kGenericSlots) {
-        gqueue[slot] = entry[i];
-        path[i] = 3u;  // placed
-      }
-    }
-    const uint64_t mo = __ballot(path[i] == kPathOdd || path[i] == kPathGeneric), me = __ballot(path[i] == kPathEven);
-    odd_rank[i] = n_o + __builtin_amdgcn_mbcnt_hi((uint32_t)(mo >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mo, 0));
-    even_rank[i] = n_e + __builtin_amdgcn_mbcnt_hi((uint32_t)(me >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)me, 0));
-    n_o += (uint32_t)__popcll(mo);
-    n_e += (uint32_t)__popcll(me);
-  }
-  uint32_t base_o = 0, base_e = 0;
-  if (lane == 0) {
-    base_o = atomicAdd(&ctrl[0], n_o);
-    base_e = atomicAdd(&ctrl[1], n_e);
-  }
-  base_o = __shfl(base_o, 0, 64);
-  base_e = __shfl(base_e, 0, 64);
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    if (path[i] == kPathOdd || path[i] == kPathGeneric) queue[base_o + odd_rank[i]] = entry[i];  // odd from the bottom
-    if (path[i] == kPathEven) queue[capacity - 1 - (base_e + even_rank[i])] = entry[i];          // even from the top
-  }
-}
-
 // ---- incoherence rotation of an activation ----------------------------------------
 // x' = Q x for Q = (S (x) I_m)(I_k (x) H_m / sqrt m) D (llvq-quant/src/rotation.rs:97-105),
 // in f32 like the reference's device rotation (llvq-cuda/kernels/llvq_rot.cuh): signs on
@@ -530,6 +366,7 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
 #include "tiles.h"
 #include "gemv_seq.h"
 #include "gemm_kernel.h"
+#include "gemm_share.h"
 #include "decoder.h"
 
 // =================================================================================
@@ -575,9 +412,6 @@ struct llvq_mat {
   uint32_t record_bits = 48;  // 48: 6-byte records (shell cap 12); 49: the dense stream of shell cap 13
   float g[2] = {0, 0};
   uint8_t* tiles = nullptr;  // device: scale table and records (tiles.h)
-  uint8_t* codes = nullptr;  // device
-  float* rscale = nullptr;   // device
-  float* tail = nullptr;     // device
   uint64_t device_bytes = 0;
   uint64_t encoded_bytes = 0;
   bool has_rotation = false;
@@ -711,8 +545,8 @@ int llvq_hip_runtime_create(int device, void* hip_stream, llvq_rt** out) {
   for_each_gemv_kernel([&](const void* kernel) { (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds); });
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rotate_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rotate_kernel<__half>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<8>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<12>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<1, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   *out = rt;
   return LLVQ_OK;
 }
@@ -889,29 +723,14 @@ static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uin
   std::vector<float> rs(d_out);
   for (uint32_t r = 0; r < d_out; ++r) rs[r] = (float)row_scales[r];  // fused.rs:1210
   const size_t code_len = (size_t)((total_blocks * record_bits + 7) / 8);
-  const size_t code_alloc = ((code_len + 3) & ~(size_t)3) + 64;  // slack so wide loads may run past the last record
   const size_t tail_len = (size_t)d_out * tail_w * sizeof(float);
-  auto cleanup = [&](hipError_t e, const char* what) {
+  const hipError_t e = upload_tiles(rt, m, centroids, rs.data(), tail, codes);
+  if (e != hipSuccess) {
     (void)hipFree(m->tiles);
-    (void)hipFree(m->codes);
-    (void)hipFree(m->rscale);
-    (void)hipFree(m->tail);
     delete m;
-    return hip_fail(e, what);
-  };
-  hipError_t e;
-  if ((e = upload_tiles(rt, m, centroids, rs.data(), tail, codes)) != hipSuccess) return cleanup(e, "upload_tiles");
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->codes), code_alloc)) != hipSuccess) return cleanup(e, "hipMalloc(codes)");
-  if ((e = hipMemset(m->codes, 0, code_alloc)) != hipSuccess) return cleanup(e, "hipMemset(codes)");
-  if (code_len && (e = hipMemcpy(m->codes, codes, code_len, hipMemcpyHostToDevice)) != hipSuccess) return cleanup(e, "hipMemcpy(codes)");
-  // 64 floats of slack: the batched kernel reads the scales of a whole 64-row band, four at a time
-  rs.resize((size_t)d_out + 64, 0.f);
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->rscale), rs.size() * sizeof(float))) != hipSuccess) return cleanup(e, "hipMalloc(rscale)");
-  if ((e = hipMemcpy(m->rscale, rs.data(), rs.size() * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess) return cleanup(e, "hipMemcpy(rscale)");
-  // zero-length arrays become one-element dummies (fused_cuda.rs:1084-1098)
-  if ((e = hipMalloc(reinterpret_cast<void**>(&m->tail), tail_len ? tail_len : sizeof(float))) != hipSuccess) return cleanup(e, "hipMalloc(tail)");
-  if (tail_len && (e = hipMemcpy(m->tail, tail, tail_len, hipMemcpyHostToDevice)) != hipSuccess) return cleanup(e, "hipMemcpy(tail)");
-  m->device_bytes = code_alloc + rs.size() * sizeof(float) + (tail_len ? tail_len : sizeof(float));
+    return hip_fail(e, "upload_tiles");
+  }
+  m->device_bytes = kTileTableBytes + (uint64_t)tile_count(d_out) * tile_stride(nblocks, tail_w);
   m->encoded_bytes = code_len + (uint64_t)d_out * 8 + tail_len + 16;
   *out = m;
   return LLVQ_OK;
@@ -1016,9 +835,6 @@ void llvq_hip_matrix_free(llvq_rt* rt, llvq_mat* m) {
   if (!m) return;
   if (rt) (void)hipSetDevice(rt->device);
   (void)hipFree(m->tiles);
-  (void)hipFree(m->codes);
-  (void)hipFree(m->rscale);
-  (void)hipFree(m->tail);
   delete m;
 }
 
@@ -1433,10 +1249,6 @@ static int grow_buffer(void** buf, size_t* have, size_t need) {
   return LLVQ_OK;
 }
 
-// Batches of up to this many activation rows leave the matrix cores little to do:
-// twelve of the sixteen wavefronts unrank and four multiply (four consumers cover 256 rows).
-constexpr uint32_t kGemmNarrowRows = 256;
-
 // Where a batched call's device workspaces come from: the runtime's buffers, grown with
 // hipMalloc on first use of a larger shape, or (fixed != null) a region the caller of this
 // file's helpers provides, which is carved up and never outgrown.
@@ -1459,25 +1271,61 @@ static int workspace_take(llvq_rt* rt, GemmWorkspace* w, void** runtime_buf, siz
   return LLVQ_OK;
 }
 
-// Workspace bytes of one batched launch (launch_gemm) over these matrices at M rows: the partial
-// sums and the K-step-tiled copy of the activations.
-static void gemm_workspace_bytes(const llvq_rt* rt, const llvq_mat* const* mats, int n, uint32_t M, size_t* ws_bytes, size_t* xt_bytes) {
-  const uint32_t grid_cap = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
-  const llvq_mat* m0 = mats[0];
-  uint32_t n_bands = 0;
-  for (int i = 0; i < n; ++i) n_bands += (mats[i]->d_out + kGemmRows - 1) / kGemmRows;
-  const uint32_t consumers = M <= kGemmNarrowRows ? 4u : 8u;
-  uint32_t ct_shift = 0;
-  while (((uint32_t)kGemmColTile << ct_shift) < M) ++ct_shift;
-  const uint32_t kparts = consumers >> ct_shift;
-  const uint32_t spb = (m0->nblocks + kGemmKb - 1) / kGemmKb;
-  const GemmShare share = gemm_share(n_bands ? n_bands : 1, spb ? spb : 1, grid_cap);
-  // bands walked by one workgroup alone are finished in the launch when every consumer owns its tile's every K-step
-  const uint32_t ws_band0 = kparts == 1 ? share.shared0 : 0u;
-  const uint32_t m_pad = (M + kGemmColTile - 1) / kGemmColTile * kGemmColTile;
-  const uint32_t n_steps = spb * (kGemmKb * 24 / 32);
-  *ws_bytes = (size_t)(n_bands - (ws_band0 < n_bands ? ws_band0 : n_bands)) * share.max_pieces * kparts * M * kGemmRows * sizeof(float);
-  *xt_bytes = (size_t)n_steps * m_pad * 64;
+// Rows of activations one batched launch takes; more go out as further launches.
+constexpr int kGemmMaxM = 1024;
+
+// How a batched launch over these matrices at M rows is cut up, and the workspaces it needs.
+struct GemmPlan {
+  uint32_t small;                // 1: up to 16 rows, 2: up to 64 (gemm_tiles_kernel), 0: gemm_wide_kernel
+  uint32_t wm, rows_per_tile;    // the wide kernel's shape, and weight rows of a workgroup
+  uint32_t n_tiles, m_pad, m_tiles, splits, steps_per_split, n_oct;
+  size_t ws_bytes, xt_bytes;
+};
+// The wide kernel's partial sums are kept below this: more column splits than that allows would cost more in memory
+// traffic than they gain in filled CUs.
+constexpr size_t kGemmWsCap = 32u << 20;
+static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n, uint32_t M) {
+  const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), nb = mats[0]->nblocks;
+  GemmPlan p{};
+  p.small = M <= 16u ? 1u : M <= kGemmSmallRows ? 2u : 0u;
+  p.n_oct = (nb + 3u) / 4u * 12u;
+  p.splits = 1;
+  p.m_tiles = 1;
+  auto count_tiles = [&](uint32_t rows) {
+    p.rows_per_tile = rows;
+    p.n_tiles = 0;
+    for (int i = 0; i < n; ++i) p.n_tiles += (mats[i]->d_out + rows - 1u) / rows;
+  };
+  if (p.small) {
+    count_tiles(p.small * 16u);
+    p.m_pad = p.small == 1u ? 16u : 64u;
+  } else {
+    // 128 activation rows per wavefront; two wavefronts side by side where that wastes no column of them
+    const uint32_t m128 = (M + 127u) / 128u;
+    p.wm = m128 % 2u == 0u ? 2u : 1u;
+    count_tiles(64u * (4u / p.wm));
+    p.m_tiles = m128 / p.wm;
+    p.m_pad = p.m_tiles * 128u * p.wm;
+    // Column splits: enough workgroups for two per CU, as long as each keeps eight steps of 48 columns.  The time of a
+    // launch is rounds of resident workgroups times steps, and what the partial sums cost on their way through memory
+    // (measured: a step of two workgroups sharing a CU 0.8 us, partial sums about 4 bytes per ps).
+    const uint32_t steps = (nb + 1u) / 2u, tiles = p.n_tiles * p.m_tiles;
+    const size_t one = (size_t)p.m_pad * p.n_tiles * p.rows_per_tile * sizeof(float);
+    double best = 1e30;
+    for (uint32_t sp = 1; sp <= 16u && (sp == 1u || (steps / sp >= 8u && one * sp <= kGemmWsCap)); ++sp) {
+      const uint32_t per = (steps + sp - 1u) / sp, wgs = tiles * ((steps + per - 1u) / per);
+      const double rounds = (double)((wgs + cus - 1u) / cus);
+      const double cost = rounds * per * 0.4 + (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
+      if (cost < best) {
+        best = cost;
+        p.splits = (steps + per - 1u) / per;
+        p.steps_per_split = per;
+      }
+    }
+    if (p.splits > 1u) p.ws_bytes = one * p.splits;
+  }
+  p.xt_bytes = (size_t)p.n_oct * p.m_pad * 16;
+  return p;
 }
 
 // Sizes the runtime's batched-path buffers for calls over these matrices (grouped as
@@ -1495,13 +1343,12 @@ static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint
     bool six_byte = true;
     for (int i = i0; i < i1; ++i) six_byte &= mats[i]->record_bits == 48;
     if (mats[i0]->nblocks && six_byte) {  // (cap-13 matrices take the row loop, which has no workspace)
-      // every row count up to the chunk: the partial-sum layout is not monotone in M where the consumers' split changes
-      for (uint32_t M : {chunk, (uint32_t)64, (uint32_t)128, (uint32_t)256}) {
-        if (M > chunk) continue;
-        size_t w = 0, x = 0;
-        gemm_workspace_bytes(rt, mats + i0, i1 - i0, M, &w, &x);
-        ws = w > ws ? w : ws;
-        xt = x > xt ? x : xt;
+      // every row count up to the chunk: the splits, and so the partial sums, are not monotone in it
+      for (uint32_t M = 16;; M = M < 64u ? M + 48u : M < 128u ? 128u : M + 128u) {
+        const GemmPlan p = gemm_plan(rt, mats + i0, i1 - i0, M < chunk ? M : chunk);
+        ws = p.ws_bytes > ws ? p.ws_bytes : ws;
+        xt = p.xt_bytes > xt ? p.xt_bytes : xt;
+        if (M >= chunk) break;
       }
     }
     if (mats[i0]->has_rotation) {
@@ -1520,99 +1367,78 @@ static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint
 // (already in the matrices' basis), M <= kGemmMaxM rows.
 static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, uint32_t M, void* const* y,
                        int y_dtype, GemmWorkspace* wsp = nullptr) {
-  const uint32_t grid_cap = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
-  const bool f32 = y_dtype == LLVQ_F32;
   const llvq_mat* m0 = mats[0];
   const __half* xh = reinterpret_cast<const __half*>(x);
-  GemmArgs a{};
-  GemmReduceArgs r{};
-  a.tables = rt->tables;
-  a.n_mats = r.n_mats = (uint32_t)n;
-  for (int i = 0; i < n; ++i) {
-    a.mat[i] = GemmMat{mats[i]->codes, mats[i]->rscale, mats[i]->tail, y[i], mats[i]->g[0], mats[i]->g[1], mats[i]->d_out, a.n_bands};
-    r.mat[i] = GemmReduceMat{mats[i]->rscale, mats[i]->tail, y[i], mats[i]->d_out, a.n_bands};
-    a.n_bands += (mats[i]->d_out + kGemmRows - 1) / kGemmRows;
-  }
-  a.y_f32 = f32 ? 1u : 0u;
-  a.x = xh;
-  a.ldx = m0->d_in;
-  a.tail_w = m0->tail_w;
-  a.M = M;
-  a.m_pad = (M + kGemmColTile - 1) / kGemmColTile * kGemmColTile;
-  a.nblocks = m0->nblocks;
-  // the consumer wavefronts over the batch's 64-row tiles, the count rounded up to a power of two
-  const uint32_t consumers = M <= kGemmNarrowRows ? 4u : 8u;
-  a.ct_shift = 0;
-  while (((uint32_t)kGemmColTile << a.ct_shift) < M) ++a.ct_shift;
-  const uint32_t kparts = consumers >> a.ct_shift;
-  // The launch's slices, band by band, are shared out evenly over the workgroups (one per CU): a
-  // band whose slices fall to several of them leaves one partial sum per workgroup.
-  a.spb = (m0->nblocks + kGemmKb - 1) / kGemmKb;
-  const uint64_t total = (uint64_t)a.n_bands * a.spb;
-  if (total > 0xFFFFFFFFull) return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": too many K-slices for one batched launch");
-  const GemmShare share = gemm_share(a.n_bands, a.spb, grid_cap);
-  if (!gemm_share_exact(share, a.n_bands, a.spb)) return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": rows too wide for the batched launch's slice arithmetic");
-  const uint32_t n_wg = share.n_wg;
-  a.share = share;
-  a.ws_band0 = kparts == 1 ? share.shared0 : 0u;
-  const uint32_t ws_bands = a.n_bands - a.ws_band0;  // bands with partial sums in the workspace
+  const GemmPlan p = gemm_plan(rt, mats, n, M);
   void* ws_buf = nullptr;
   void* xt_buf = nullptr;
   const size_t mark = wsp ? wsp->used : 0;  // a launch's carvings are released when it has been enqueued: the stream orders the next
-  size_t ws_bytes = 0, xt_bytes = 0;
-  gemm_workspace_bytes(rt, mats, n, M, &ws_bytes, &xt_bytes);
-  if (ws_bytes != (size_t)ws_bands * share.max_pieces * kparts * M * kGemmRows * sizeof(float))
-    return fail(LLVQ_ERR_DEVICE, "gemm: workspace sizing disagrees with the launch");
   int rc = LLVQ_OK;
-  if (ws_bytes) rc = workspace_take(rt, wsp, reinterpret_cast<void**>(&rt->gemm_ws), &rt->gemm_ws_bytes, ws_bytes, &ws_buf);
+  if (p.ws_bytes) rc = workspace_take(rt, wsp, reinterpret_cast<void**>(&rt->gemm_ws), &rt->gemm_ws_bytes, p.ws_bytes, &ws_buf);
   if (rc) return rc;
-  // every slice has all its twelve K-steps in the tiled copy, zeros past the matrix's last block
-  const uint32_t n_steps = (m0->nblocks + kGemmKb - 1) / kGemmKb * (kGemmKb * 24 / 32);
-  if (xt_bytes != (size_t)n_steps * a.m_pad * 64) return fail(LLVQ_ERR_DEVICE, "gemm: activation-copy sizing disagrees with the launch");
-  // the kernel reads the copy through a buffer descriptor: 32-bit offsets
-  if (xt_bytes >= (1ull << 32)) return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": rows too wide for the batched launch's 32-bit activation offsets");
-  rc = workspace_take(rt, wsp, reinterpret_cast<void**>(&rt->gemm_xt), &rt->gemm_xt_bytes, xt_bytes, &xt_buf);
+  rc = workspace_take(rt, wsp, reinterpret_cast<void**>(&rt->gemm_xt), &rt->gemm_xt_bytes, p.xt_bytes, &xt_buf);
   if (rc) return rc;
   if (wsp) wsp->used = mark;
-  hipLaunchKernelGGL(tile_activations_kernel, dim3((uint32_t)((xt_bytes / 16 + 255) / 256)), dim3(256), 0, rt->stream, xh, M,
-                     m0->d_in, m0->nblocks * 24u, a.m_pad, n_steps, reinterpret_cast<uint4*>(xt_buf));
-  HIP_TRY(hipGetLastError());
-  a.xt = reinterpret_cast<__half*>(xt_buf);
+  GemmReduceArgs r{};
+  GemmArgs& a = r.g;
+  a.xt = reinterpret_cast<const uint4*>(xt_buf);
+  a.x = xh;
   a.ws = reinterpret_cast<float*>(ws_buf);
-  const dim3 grid(n_wg), wg(kWgThreads);
-  if (consumers == 4) hipLaunchKernelGGL(gemm_tiles_kernel<12>, grid, wg, gemm_lds_bytes(), rt->stream, a);
-  else hipLaunchKernelGGL(gemm_tiles_kernel<8>, grid, wg, gemm_lds_bytes(), rt->stream, a);
-  HIP_TRY(hipGetLastError());
-  r.ws = a.ws;
-  r.x = xh;
-  r.M = M;
-  r.ldx = m0->d_in;
-  r.nblocks = m0->nblocks;
-  r.tail_w = m0->tail_w;
-  r.n_bands = a.n_bands;
-  r.spb = a.spb;
-  r.share = share;
-  r.ws_band0 = a.ws_band0;
-  r.kparts = kparts;
-  if (ws_bands == 0) return LLVQ_OK;  // every band was finished by the workgroup that walked it
-  const uint32_t rgrid = ws_bands * ((M + kReduceRowsM - 1) / kReduceRowsM);
-  if (f32) hipLaunchKernelGGL(gemm_reduce_kernel<float>, dim3(rgrid), dim3(256), 0, rt->stream, r);
-  else hipLaunchKernelGGL(gemm_reduce_kernel<__half>, dim3(rgrid), dim3(256), 0, rt->stream, r);
+  a.n_mats = (uint32_t)n;
+  for (int i = 0; i < n; ++i) {
+    a.mat[i] = GemmMat{mats[i]->tiles, y[i], mats[i]->d_out, a.n_tiles};
+    a.n_tiles += (mats[i]->d_out + p.rows_per_tile - 1u) / p.rows_per_tile;
+  }
+  a.y_f32 = y_dtype == LLVQ_F32 ? 1u : 0u;
+  a.ldx = m0->d_in;
+  a.tail_w = m0->tail_w;
+  a.M = M;
+  a.m_pad = p.m_pad;
+  a.nb = m0->nblocks;
+  a.m_tiles = p.m_tiles;
+  a.splits = p.splits;
+  a.steps_per_split = p.steps_per_split;
+  const uint32_t oct_waves = (p.n_oct + 7u) / 8u * (p.m_pad / 8u);
+  hipLaunchKernelGGL(tile_activations_kernel, dim3((oct_waves + 3u) / 4u), dim3(256), 0, rt->stream, xh, M, a.ldx, a.nb * 24u, p.m_pad, p.n_oct,
+                     reinterpret_cast<uint4*>(xt_buf));
+  if (p.small == 1u) hipLaunchKernelGGL((gemm_tiles_kernel<1, 1>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<1, 1>()), rt->stream, a);
+  else if (p.small) hipLaunchKernelGGL((gemm_tiles_kernel<2, 4>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<2, 4>()), rt->stream, a);
+  else if (p.wm == 1u) hipLaunchKernelGGL(gemm_wide_kernel<1>, dim3(a.n_tiles * p.m_tiles * p.splits), dim3(256), gemm_wide_lds<1>(), rt->stream, a);
+  else hipLaunchKernelGGL(gemm_wide_kernel<2>, dim3(a.n_tiles * p.m_tiles * p.splits), dim3(256), gemm_wide_lds<2>(), rt->stream, a);
+  if (p.splits > 1u) {
+    r.rows_per_tile = p.rows_per_tile;
+    r.row_chunks = (a.n_tiles * p.rows_per_tile + 255u) / 256u;
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3(r.row_chunks * ((M + kReduceM - 1u) / kReduceM)), dim3(256), 0, rt->stream, r);
+  }
   HIP_TRY(hipGetLastError());
   return LLVQ_OK;
 }
 
-// Matrices [0, n) of one group: same d_in, same basis.  The matrix-core kernel reads activations as
-// 16-byte vectors; a single row, or a shape that breaks that alignment, runs as GEMV launches instead.
+// What llvq_hip_gemm_static admits.  The bound is part of its contract (callers choose their fallback by it), so it stays
+// the one of the partial-sum layout the entry point was specified with (gemm_share.h: a band's K-slices shared out over
+// the workgroups, 64 x 64 sums per piece, and a tiled copy of the activations), which is above what the kernels take now.
+static size_t static_admission_bytes(const llvq_rt* rt, const llvq_mat* m, uint32_t M) {
+  const uint32_t grid_cap = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), consumers = M <= 256u ? 4u : 8u;
+  const uint32_t bands = (m->d_out + 63u) / 64u, spb = (m->nblocks + 15u) / 16u;
+  uint32_t ct_shift = 0;
+  while ((64u << ct_shift) < M) ++ct_shift;
+  const uint32_t kparts = consumers >> ct_shift;
+  const GemmShare share = gemm_share(bands ? bands : 1, spb ? spb : 1, grid_cap);
+  const uint32_t band0 = kparts == 1 ? share.shared0 : 0u;
+  const size_t sums = (size_t)(bands - (band0 < bands ? band0 : bands)) * share.max_pieces * kparts * M * 64 * sizeof(float);
+  return ((sums + 255) & ~(size_t)255) + (size_t)spb * 12 * ((M + 63) / 64 * 64) * 64;
+}
+
+// Matrices [0, n) of one group: same d_in, same basis.  A single row runs as GEMV launches instead, as do matrices
+// without a whole block and cap-13 matrices, whose rows keep the bits of the single-row product.
 static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, int M, void* const* y, int y_dtype,
                            GemmWorkspace* wsp = nullptr) {
   const llvq_mat* m0 = mats[0];
   const size_t esz = y_dtype == LLVQ_F32 ? 4 : 2;
   const uint8_t* xb = reinterpret_cast<const uint8_t*>(x);
-  bool six_byte = true;  // the matrix-core kernel's producers read 6-byte records: cap-13 matrices take the row loop
+  bool six_byte = true;
   for (int i = 0; i < n; ++i) six_byte &= mats[i]->record_bits == 48;
-  const bool mfma_ok = M >= 2 && m0->d_in % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && m0->nblocks > 0 && six_byte;
-  if (!mfma_ok) {
+  if (M < 2 || m0->nblocks == 0 || !six_byte) {
     for (int i = 0; i < n; ++i)
       for (int r = 0; r < M; ++r) {
         const int rc = launch_gemv(rt, mats[i], xb + (size_t)r * m0->d_in * 2, reinterpret_cast<uint8_t*>(y[i]) + (size_t)r * mats[i]->d_out * esz, y_dtype);
@@ -1621,21 +1447,17 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
     return LLVQ_OK;
   }
   if (wsp && wsp->fixed) {
-    // a caller-provided region is never outgrown part-way: every launch's carvings (released once it is enqueued)
-    // are sized before the first launch, since a short last chunk can need more than a full one, and a call
-    // that does not fit is refused whole
+    // a call that does not fit is refused whole, before its first launch
     auto after = [](size_t used, size_t bytes) { return ((used + 255) & ~(size_t)255) + bytes; };
     const size_t base = m0->has_rotation ? after(wsp->used, (size_t)M * m0->d_in * sizeof(__half)) : wsp->used;
     size_t need = base;
-    for (int m_lo = 0; m_lo < M; m_lo += kGemmMaxM) {
-      const uint32_t mc = (uint32_t)(M - m_lo < kGemmMaxM ? M - m_lo : kGemmMaxM);
+    for (int m_lo = 0; m_lo < M; m_lo += 512)
+      for (int i = 0; i < n; ++i) need = std::max(need, after(base, static_admission_bytes(rt, mats[i], (uint32_t)std::min(M - m_lo, 512))));
+    for (int m_lo = 0; m_lo < M; m_lo += kGemmMaxM)
       for (int i0 = 0; i0 < n; i0 += kGemmMaxGroup) {
-        size_t ws = 0, xt = 0;
-        gemm_workspace_bytes(rt, mats + i0, n - i0 < kGemmMaxGroup ? n - i0 : kGemmMaxGroup, mc, &ws, &xt);
-        const size_t top = after(ws ? after(base, ws) : base, xt);
-        if (top > need) need = top;
+        const GemmPlan p = gemm_plan(rt, mats + i0, std::min(n - i0, kGemmMaxGroup), (uint32_t)std::min(M - m_lo, kGemmMaxM));
+        need = std::max(need, after(p.ws_bytes ? after(base, p.ws_bytes) : base, p.xt_bytes));
       }
-    }
     if (need > wsp->fixed_bytes)
       return fail(LLVQ_ERR_UNSUPPORTED, "gemm_static: this shape needs " + std::to_string(need) +
                                             " bytes of workspace, the static one holds " + std::to_string(wsp->fixed_bytes));

@@ -39,7 +39,7 @@ template <bool WIDE>
 __global__ __launch_bounds__(512) void transcode_kernel(GlobalTables g, const uint8_t* __restrict__ codes, uint8_t* __restrict__ tiles,
                                                         uint32_t rows, uint32_t nb, uint32_t tail_w) {
   extern __shared__ __align__(16) uint8_t smem[];
-  const DecodeTables T = stage_tables<true, true, WIDE>(smem, g);
+  const DecodeTables T = stage_tables<WIDE>(smem, g);
   __syncthreads();
   const uint32_t stride = tile_stride(nb, tail_w), head = tile_head_bytes(tail_w);
   const uint64_t padded = (uint64_t)tile_count(rows) * kTileRows * nb;
