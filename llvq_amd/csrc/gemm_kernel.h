@@ -6,7 +6,7 @@
 // exactly what a lane hands to a 16-deep (32 x 32) or 32-deep (16 x 16) product step, so a wavefront turns the 12 bytes
 // its lanes load into its own fragments: no weights pass through LDS, and the order in which the products walk the
 // columns is the order the blocks lie in (the lane groups of a fragment hold the same octet of two or four neighbouring
-// blocks).  17 instructions per eight weights.
+// blocks).  19 instructions per eight weights.
 //
 // The activations come as octets: xt[c][m] = columns 8 c .. 8 c + 7 of row m, 16 bytes, m_pad rows to a column octet, so
 // that the fragments of 16 or 32 rows are runs of 256 or 512 bytes (tile_activations_kernel; in x they would be 16-byte
@@ -50,42 +50,56 @@ __global__ __launch_bounds__(256) void tile_activations_kernel(const __half* __r
 }
 
 // ---- weights ---------------------------------------------------------------------------------------
-// A block's scale factors for a lane: an unpacked nibble is n in one half of a dword's nibble pairs and 16 n in the other.
-struct BlockScale {
-  float c, c16, odd;  // 2 s, s / 8, and s if the block's coordinates are odd
-};
-__device__ __forceinline__ BlockScale block_scale(uint32_t meta_dword, uint32_t r, uint32_t table) {
-  const uint32_t meta = meta_dword >> (8u * (r & 3u));
-  const float s = __int_as_float(__builtin_amdgcn_ds_bpermute((int)(meta & 0x7Cu), (int)table));
-  return BlockScale{2.f * s, 0.125f * s, (meta & 1u) ? s : 0.f};
+// The matrix's table of scales for dequant_octet: a lane keeps entry lane % 32 as the sum of two binary16 numbers (low
+// half: the entry rounded, high half: what that left), a power of two taken out first that puts the largest entry into
+// [8, 16), so that neither number nor an eighth of it leaves the normal range by more than the precision can spare.
+// `unit` is that power of two; it goes back in with the row scales.
+__device__ __forceinline__ uint32_t split_table(float entry, float& unit) {
+  uint32_t e = __float_as_uint(entry) & 0x7F800000u;
+#pragma unroll
+  for (int k = 1; k < 32; k <<= 1) e = max(e, (uint32_t)__shfl_xor((int)e, k));
+  const int ex = min(max((int)(e >> 23) - 130, -100), 100);  // (a table of zeros or with an infinity in it: any power will do)
+  unit = ldexpf(1.f, ex);
+  const float v = entry * ldexpf(1.f, -ex);
+  const _Float16 hi = (_Float16)v;
+  const _Float16 lo = (_Float16)(v - (float)hi);
+  return __builtin_bit_cast(uint32_t, half2_t{hi, lo});
 }
-// One dword of nibbles -> eight weights.  1024 + u is a binary16 number whose low bits are u; taking 1032 away leaves
-// n = u - 8 exactly (the nibble's top bit is flipped on the way: two's complement to offset), and 16 n likewise; one
-// fused multiply-add in f32 per weight, rounded to binary16 once.
-// The eight of those are one block of assembly: the compiler does not form them from source, and it does not know what
-// an assembly statement does to the registers a matrix instruction reads, so the two wait states that are due between a
-// vector write and that read stand at the block's end (and the halves of a register are written four apart).
+// What a block's meta byte gives a lane: the two parts of its scale (and an eighth of them), and its parity bit where
+// dequant_octet wants it.
+struct BlockScale {
+  half2_t c, c8;
+  uint32_t odd, odd8;
+};
+__device__ __forceinline__ uint32_t block_meta(uint32_t meta_dword, uint32_t r) { return meta_dword >> (8u * (r & 3u)); }
+__device__ __forceinline__ uint32_t scale_parts(uint32_t meta, uint32_t table) {
+  return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(meta & 0x7Cu), (int)table);
+}
+__device__ __forceinline__ BlockScale block_scale(uint32_t meta, uint32_t parts) {
+  const half2_t c = __builtin_bit_cast(half2_t, parts);
+  const uint32_t p = (uint32_t)((int32_t)(meta << 31) >> 31);
+  uint32_t odd = (p & 0x00010001u) ^ 0x64106410u, odd8 = (p & 0x00080008u) ^ 0x64806480u;
+  asm("" : "+v"(odd), "+v"(odd8));  // (kept whole: taken apart again, a mask and it would no longer be one operation)
+  return BlockScale{c, c * half2_t{(_Float16)0.125f, (_Float16)0.125f}, odd, odd8};
+}
+// One dword of nibbles -> eight weights.  A binary16 number of the form 1024 + k has k in its low bits: with the nibble's
+// top bit flipped (two's complement to offset) and the parity bit below it that is 1024 + 16 + v, or 1024 + 128 + 8 v
+// where the nibble lies four bits higher.  v (hi + lo) is rounded once: v lo is small enough for its own rounding to be
+// lost in that of the sum.  19 instructions, all of which run beside the matrix cores; the mixed-precision
+// multiply-add (two fewer) does not: 4 products and 20 of those took 103 ns of a SIMD, with packed or f32 ones 70.
 __device__ __forceinline__ half8_t dequant_octet(uint32_t w, const BlockScale& s) {
-  const uint32_t v = w >> 8;
-  const uint32_t t[4] = {(w & 0x000F000Fu) ^ 0x64086408u, (w & 0x00F000F0u) ^ 0x64806480u, (v & 0x000F000Fu) ^ 0x64086408u, (v & 0x00F000F0u) ^ 0x64806480u};
-  uint32_t n[4], o[4];
+  const uint32_t t[4] = {((w << 1) & 0x001E001Eu) ^ s.odd, (w & 0x00F000F0u) ^ s.odd8, ((w >> 7) & 0x001E001Eu) ^ s.odd, ((w >> 8) & 0x00F000F0u) ^ s.odd8};
+  half8_t out;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const half2_t bias = (i & 1) ? half2_t{(_Float16)1152.f, (_Float16)1152.f} : half2_t{(_Float16)1032.f, (_Float16)1032.f};
-    n[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, t[i]) - bias);
+    const half2_t bias = (i & 1) ? half2_t{(_Float16)1152.f, (_Float16)1152.f} : half2_t{(_Float16)1040.f, (_Float16)1040.f};
+    const half2_t v = __builtin_bit_cast(half2_t, t[i]) - bias;
+    const half2_t c = (i & 1) ? s.c8 : s.c;
+    const half2_t y = __builtin_elementwise_fma(v, half2_t{c.x, c.x}, v * half2_t{c.y, c.y});
+    out[2 * i] = y.x;
+    out[2 * i + 1] = y.y;
   }
-  asm("v_fma_mixlo_f16 %0, %4, %8, %10 op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixlo_f16 %1, %5, %9, %10 op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixlo_f16 %2, %6, %8, %10 op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixlo_f16 %3, %7, %9, %10 op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixhi_f16 %0, %4, %8, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixhi_f16 %1, %5, %9, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixhi_f16 %2, %6, %8, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixhi_f16 %3, %7, %9, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-      "s_nop 1"
-      : "=&v"(o[0]), "=&v"(o[1]), "=&v"(o[2]), "=&v"(o[3])
-      : "v"(n[0]), "v"(n[1]), "v"(n[2]), "v"(n[3]), "v"(s.c), "v"(s.c16), "v"(s.odd));
-  return __builtin_bit_cast(half8_t, o);
+  return out;
 }
 
 struct GemmMat {
@@ -161,7 +175,7 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   const uint8_t* recs = t.base + kTileTableBytes + (size_t)(t.row0 / kTileRows) * stride;
   const uint32_t last_rec = tile_count(t.d_out) - 1u - t.row0 / kTileRows;  // records past the matrix's last repeat it
   const uint32_t r = lane & 7u, g = lane >> 4, m16 = lane & 15u;
-  const uint32_t table = reinterpret_cast<const uint32_t*>(t.base)[lane & 31u];
+  const float entry = reinterpret_cast<const float*>(t.base)[lane & 31u];
   uint32_t rec_off[RG];
 #pragma unroll
   for (int k = 0; k < RG; ++k) rec_off[k] = min((uint32_t)k * 2u + ((lane >> 3) & 1u), last_rec) * stride + head + g * kTileBlockBytes;
@@ -206,6 +220,8 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   load_w(q, q < n_quads);
 #pragma unroll
   for (uint32_t j = 0; j < 3; ++j) load_x(j, q, q < n_quads);
+  float unit;
+  const uint32_t table = split_table(entry, unit);
   acc4_t acc[RG][MT];
 #pragma unroll
   for (int k = 0; k < RG; ++k)
@@ -216,7 +232,10 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
     const bool live = qn < n_quads;
     BlockScale s[RG];
 #pragma unroll
-    for (int k = 0; k < RG; ++k) s[k] = block_scale(W[k].meta, r, table);
+    for (int k = 0; k < RG; ++k) {
+      const uint32_t meta = block_meta(W[k].meta, r);
+      s[k] = block_scale(meta, scale_parts(meta, table));
+    }
 #pragma unroll
     for (uint32_t j = 0; j < 3; ++j) {
       half8_t w[RG];
@@ -239,7 +258,7 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
     }
   }
   if (op_col < a.tail_w) tw[op_row * 24u + op_col] = op_w;
-  else if (op_col == 24u) scale_s[op_row] = op_w;
+  else if (op_col == 24u) scale_s[op_row] = op_w * unit;
   if (a.tail_w) {
 #pragma unroll
     for (uint32_t i = 0; i < 2; ++i) {
@@ -271,171 +290,312 @@ template <int RG, int MT>
 __host__ constexpr size_t gemm_small_lds() { return (size_t)(16 * RG * MT * 256 + RG * 16 * 25 + MT * 16 * 24) * 4; }
 static_assert(gemm_small_lds<2, 4>() <= 160 * 1024, "partial sums of sixteen wavefronts fit a CU's LDS");
 
+// A lane's sixteen results of one activation row (weight rows row + 8 g + 4 h .. + 3, g < 4) into y + at: where y and its
+// rows lie on 16-byte boundaries, and one by one.
+struct StoreF32 {
+  static __device__ __forceinline__ void store(void* y, size_t at, uint32_t row, uint32_t h, uint32_t, const acc16_t& v) {
+    float* out = reinterpret_cast<float*>(y) + at + row + 4u * h;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) *reinterpret_cast<float4*>(out + g * 8) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+  }
+};
+struct StoreF16 {
+  static __device__ __forceinline__ void store(void* y, size_t at, uint32_t row, uint32_t h, uint32_t, const acc16_t& v) {
+    uint32_t p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = __builtin_bit_cast(uint32_t, half2_t{(_Float16)v[2 * i], (_Float16)v[2 * i + 1]});
+    _Float16* out = reinterpret_cast<_Float16*>(y) + at + row;
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {  // the upper half's group g for the lower half's group g + 1: eight rows in a row each
+      const auto a = __builtin_amdgcn_permlane32_swap(p[2 * g], p[2 * g + 2], false, false);
+      const auto b = __builtin_amdgcn_permlane32_swap(p[2 * g + 1], p[2 * g + 3], false, false);
+      *reinterpret_cast<u32x4_t*>(out + (g + h) * 8u) = u32x4_t{a[0], b[0], a[1], b[1]};
+    }
+  }
+};
+template <typename Y>
+struct StoreEach {
+  static __device__ __forceinline__ void store(void* y, size_t at, uint32_t row, uint32_t h, uint32_t d_out, const acc16_t& v) {
+    Y* out = reinterpret_cast<Y*>(y) + at;
+#pragma unroll
+    for (uint32_t e = 0; e < 16; ++e) {
+      const uint32_t r = row + 8u * (e >> 2) + 4u * h + (e & 3u);
+      if (r < d_out) out[r] = (Y)v[e];
+    }
+  }
+};
+
 // ---- more activation rows ----------------------------------------------------------------------------
-// What bounds it: the matrix cores (a 64 x 128 tile of a wavefront is 24 steps of 32 cycles per 48 columns, its two
-// weight fragments 120 vector instructions beside them).  A workgroup of four wavefronts takes 64 (4 / WM) weight rows by
-// 128 WM activation rows: each wavefront unpacks its own 64 rows (two 32-row fragments, from memory to registers) against
-// 128 activation rows (four fragments, from LDS, which the workgroup fills a step of 48 columns ahead from the octets,
-// whose order is the fragments' own: a run of 512 bytes each).  128 accumulators and a step's operands fit 256 registers,
-// so two workgroups share a CU and one unpacks while the other multiplies.
+// What bounds it: the matrix cores, and the issue slots they share with the unpacking (38 instructions for every 2 CF
+// products).  A workgroup of four wavefronts takes 256 weight rows by 32 CF activation rows; a wavefront unpacks 64 rows
+// (two fragments) against all of the activation rows (CF fragments).  CF = 8: 256 accumulators and one wavefront on a
+// SIMD, half the unpacking and a workgroup on every CU (1.28 us a step, where the products alone take 0.85 on numbers
+// like these); CF = 4: half of that, two workgroups on a CU (0.69 us a step each) or one (0.8), for batches and matrices
+// that do not fill the other.
+// Octets and tiles go from memory to LDS without passing through registers, two to three steps of 48 columns (two
+// blocks) ahead.
 // Launches with too few tiles to fill the chip split the columns (`splits`): partial sums go to the workspace and
 // gemm_reduce_kernel adds them in order; otherwise the tile is finished here.
-constexpr uint32_t kWideStepBlocks = 2;  // blocks per step: the halves of a wavefront hold one each
-template <int WM>
-__host__ __device__ constexpr uint32_t gemm_wide_rows() { return 64u * (4u / WM); }
-template <int WM>
-__host__ __device__ constexpr uint32_t gemm_wide_cols() { return 128u * WM; }
+// Gate and up of an 8B layer (24576 x 4096) at 512 rows: 158 -> 116 us, 886 TFLOP/s; a plain f16 product of that size
+// by the vendor's library runs at 1151 on this card, whose clock follows the power the products draw (on random numbers
+// a loop of nothing else reaches 1650).
+constexpr uint32_t kWideRows = 256;
+constexpr uint32_t kWideTileBytes = 1024;  // four records, two blocks of each (832 bytes) and what the lanes behind them bring
+constexpr uint32_t kWideDepth = 4;         // LDS buffers, a step each
+template <int CF>
+__host__ __device__ constexpr uint32_t gemm_wide_x_bytes() { return 6u * 32u * CF * 16u; }
+template <int CF>
+__host__ __device__ constexpr uint32_t gemm_wide_buf() { return gemm_wide_x_bytes<CF>() + 8u * kWideTileBytes; }
+template <int CF>
+__host__ constexpr size_t gemm_wide_lds() { return (size_t)kWideDepth * gemm_wide_buf<CF>(); }
+static_assert(kWideDepth * gemm_wide_buf<4>() >= (kWideRows + 128u) * kDim * 4u && kWideDepth * gemm_wide_buf<8>() >= (kWideRows + 256u) * kDim * 4u,
+              "the tail's operands fit the buffers");
 
-// Sixteen results of a lane (one weight row, activation rows 8 (e / 4) + e % 4 from m on) into y.
-template <typename Y>
-__device__ __forceinline__ void store_fragment(Y* y, uint32_t ldy, const acc16_t& v, uint32_t m, uint32_t M) {
-#pragma unroll
-  for (uint32_t e = 0; e < 16; ++e) {
-    const uint32_t me = m + 8u * (e >> 2) + (e & 3u);
-    if (me < M) y[(size_t)me * ldy] = (Y)v[e];
-  }
+// 16 bytes per lane from base + offset to LDS, lane after lane from `lds` on.  In assembly because the compiler, which
+// cannot tell the buffers apart, would have every read of LDS wait for all of these; the counting is done by hand
+// (wide_wait), and there are no other loads in flight where it is.
+__device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t offset, const uint8_t* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory");
 }
+template <int N>
+__device__ __forceinline__ void wide_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-template <int WM>
-__global__ __launch_bounds__(256, 2) void gemm_wide_kernel(GemmArgs a) {
-  constexpr uint32_t kCols = gemm_wide_cols<WM>(), kRows = gemm_wide_rows<WM>();
-  constexpr uint32_t kPieces = kCols * 6u;            // 16-byte pieces of a step: two blocks of three octets
-  constexpr uint32_t kPer = kPieces / 256u;           // of them a lane moves to LDS
-  extern __shared__ __align__(16) uint8_t smem[];
-  u32x4_t* buf = reinterpret_cast<u32x4_t*>(smem);    // [2][2 blocks][3 octets][kCols]
+template <int CF>
+__global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArgs a) {
+  constexpr uint32_t kCols = 32u * CF, kBuf = gemm_wide_buf<CF>();
+  constexpr int kLoadsX = 3 * CF / 4, kLoadsW = 2, kLoads = kLoadsX + kLoadsW;  // of a wavefront in a step
+  extern __shared__ __align__(16) uint8_t smem[];     // [kWideDepth] x { [6 octets][kCols] 16 bytes, [8] x 32 rows of tiles }
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t l32 = lane & 31u, h = lane >> 5, r = lane & 7u;
-  const uint32_t wm = wave % WM, wr = wave / WM;
   // tiles of one row group are neighbours in the grid: they read the same weights
   const uint32_t mt = blockIdx.x % a.m_tiles, rest = blockIdx.x / a.m_tiles;
   const uint32_t tile = rest % a.n_tiles, split = rest / a.n_tiles;
   const uint32_t nb = a.nb, stride = tile_stride(nb, a.tail_w), head = tile_head_bytes(a.tail_w);
-  const GemmTile t = gemm_tile_at(a, tile, kRows);
-  const uint32_t row0 = t.row0 + wr * 64u;            // this wavefront's first row
+  const GemmTile t = gemm_tile_at(a, tile, kWideRows);
+  const uint32_t row0 = t.row0 + wave * 64u;            // this wavefront's first row
   const uint32_t n_rec = tile_count(t.d_out);
-  const uint8_t* recs = t.base + kTileTableBytes;
-  const uint32_t table = reinterpret_cast<const uint32_t*>(t.base)[lane & 31u];
+  const float entry = reinterpret_cast<const float*>(t.base)[lane & 31u];
   const uint32_t n_steps = (nb + 1u) >> 1;
   const uint32_t s0 = split * a.steps_per_split, s1 = min(s0 + a.steps_per_split, n_steps);
+  const uint8_t* rec0 = uniform_global(t.base + kTileTableBytes + (size_t)(t.row0 / kTileRows) * stride);
   // records past the matrix's last repeat it: their rows are not stored
-  const uint32_t rec0 = min(row0 / kTileRows, n_rec - 1u);
-  const uint8_t* wave_rec = recs + (size_t)rec0 * stride;
-  uint32_t rec_off[2];
+  auto record = [&](uint32_t row) __attribute__((always_inline)) { return (min(row / kTileRows, n_rec - 1u) - t.row0 / kTileRows) * stride; };
+  // a load of tiles takes four records, 13 lanes each; a load of octets 64 activation rows of one
+  uint32_t w_off[kLoadsW], x_off[kLoadsX];
+  const uint32_t w_rec = min(lane, 51u) / 13u, w_piece = min(lane, 51u) - w_rec * 13u;
 #pragma unroll
-  for (uint32_t k = 0; k < 2; ++k) rec_off[k] = (min(row0 / kTileRows + k * 4u + (l32 >> 3), n_rec - 1u) - rec0) * stride;
-  const uint32_t in_step = head + h * kTileBlockBytes;
-  const uint32_t w_off[2] = {rec_off[0] + in_step + r * 12u, rec_off[1] + in_step + r * 12u};
-  const uint32_t meta_off[2] = {rec_off[0] + in_step + 96u + (r & 4u), rec_off[1] + in_step + 96u + (r & 4u)};
-
-  struct __attribute__((packed, aligned(4))) W3 { uint32_t w[3]; };
-  StepWords Wa[2], Wb[2];  // of the even and the odd steps
-  u32x4_t pre[kPer];
-  // piece p of a step: octet p / kCols of the step's six, activation row p % kCols of the tile
-  const uint8_t* xt = reinterpret_cast<const uint8_t*>(a.xt + (size_t)mt * kCols);
-  uint32_t x_off[kPer];
+  for (uint32_t k = 0; k < (uint32_t)kLoadsW; ++k) w_off[k] = record(t.row0 + (wave * (uint32_t)kLoadsW + k) * 32u + w_rec * 8u) + head + w_piece * 16u;
 #pragma unroll
-  for (uint32_t i = 0; i < kPer; ++i) x_off[i] = ((tid + i * 256u) / kCols * a.m_pad + (tid + i * 256u) % kCols) * 16u;
-  auto load_x = [&](uint32_t s) __attribute__((always_inline)) {
-    const uint8_t* xs = uniform_global(xt + (size_t)s * 6u * a.m_pad * 16u);
+  for (uint32_t i = 0; i < (uint32_t)kLoadsX; ++i) {
+    const uint32_t k = i * 4u + wave, o = k / (kCols / 64u), m = k % (kCols / 64u) * 64u + lane;
+    x_off[i] = (o * a.m_pad + mt * kCols + m) * 16u;
+  }
+  const uint32_t x_step = 6u * a.m_pad * 16u, smem_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  const uint8_t* xt = reinterpret_cast<const uint8_t*>(a.xt);
+  auto load = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) {
+    s = min(s, s1 - 1u);  // (steps past the last are loaded too, so that the count of loads in flight is always the same)
+    const uint32_t at = smem_at + buffer;
+    const uint8_t* xs = uniform_global(xt + (size_t)s * x_step);
+    const uint8_t* ws = uniform_global(rec0 + (size_t)s * (2u * kTileBlockBytes));
 #pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) pre[i] = *reinterpret_cast<const u32x4_t*>(xs + lane_offset(x_off[i]));
+    for (uint32_t i = 0; i < (uint32_t)kLoadsX; ++i) load_to_lds(at + (i * 4u + wave) * 1024u, x_off[i], xs);
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)kLoadsW; ++k) load_to_lds(at + gemm_wide_x_bytes<CF>() + (wave * (uint32_t)kLoadsW + k) * kWideTileBytes, w_off[k], ws);
   };
-  auto load_w = [&](StepWords (&W)[2], uint32_t s) __attribute__((always_inline)) {
-    const uint8_t* ws = uniform_global(wave_rec + s * (2u * kTileBlockBytes));
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const W3 w = *reinterpret_cast<const W3*>(ws + lane_offset(w_off[k]));
-      W[k] = StepWords{w.w[0], w.w[1], w.w[2], *reinterpret_cast<const uint32_t*>(ws + lane_offset(meta_off[k]))};
-    }
-  };
-  acc16_t acc[2][4];
+  acc16_t acc[2][CF];
 #pragma unroll
   for (int k = 0; k < 2; ++k)
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < CF; ++c)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[k][c][e] = 0.f;
-  // One step: the octets fetched during the one before go to LDS, those of the next are fetched, and so are the weights
-  // two steps on once this step's are unpacked.
-  auto step = [&](StepWords (&W)[2], uint32_t s, u32x4_t* b) __attribute__((always_inline)) {
+  float unit;
+  const uint32_t table = split_table(entry, unit);
+  // One step: three rounds of eight products, in whose shadow the weights of the round after are unpacked and its
+  // activations read.  Behind the first round every wavefront waits for its loads of the next step and then for the
+  // others; the step before has been read by then, and its buffer is filled again.  In the second the next step's tiles
+  // are read, in the third unpacked.
+  struct W3 { uint32_t w[3]; };
+  typedef __attribute__((address_space(3))) uint32_t lds_u32;
+  half8_t w[2], x[CF];
+  W3 W[2], Wn[2];
+  uint32_t meta[2], parts[2];
+  BlockScale sc[2];
+  auto unpack = [&](uint32_t j) __attribute__((always_inline)) {
 #pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) b[tid + i * 256u] = pre[i];
-    lds_barrier();  // (the other buffer was last read before the previous barrier)
-    __builtin_amdgcn_sched_barrier(0);
-    load_x(min(s + 1u, s1 - 1u));
-    __builtin_amdgcn_sched_barrier(0);
-    BlockScale sc[2];
+    for (int k = 0; k < 2; ++k) w[k] = dequant_octet(W[k].w[j], sc[k]);
+  };
+  const uint32_t x_at = (h * 3u * kCols + l32) * 16u;
+  const uint32_t block_at = gemm_wide_x_bytes<CF>() + wave * 2u * kWideTileBytes + (l32 >> 3) * (2u * kTileBlockBytes) + h * kTileBlockBytes;
+  const uint32_t w_at = block_at + r * 12u, meta_at = block_at + 96u + r;
+  auto read_x = [&](uint32_t buffer, uint32_t j) __attribute__((always_inline)) {
+    const u32x4_t* f = reinterpret_cast<const u32x4_t*>(smem + (buffer + x_at)) + j * kCols;
 #pragma unroll
-    for (int k = 0; k < 2; ++k) sc[k] = block_scale(W[k].meta, r, table);
-    const u32x4_t* bx = b + h * 3u * kCols + wm * 128u + l32;
-    half8_t w[2];
+    for (int c = 0; c < CF; ++c) x[c] = __builtin_bit_cast(half8_t, f[(uint32_t)c * 32u]);
+  };
+  auto read_w = [&](uint32_t buffer) __attribute__((always_inline)) {
 #pragma unroll
-    for (uint32_t j = 0; j < 3; ++j) {
-      half8_t x[4];
+    for (int k = 0; k < 2; ++k) meta[k] = smem[(buffer + meta_at) + k * kWideTileBytes];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) x[c] = __builtin_bit_cast(half8_t, bx[j * kCols + (uint32_t)c * 32u]);
+    for (int k = 0; k < 2; ++k) {
+      // (dword by dword: merged into one read of 12 bytes at 4-byte alignment they took 60 cycles of LDS, not 6)
+      const volatile lds_u32* f = (const volatile lds_u32*)(lds_u32*)(smem + (buffer + w_at) + k * (int)kWideTileBytes);
+      Wn[k] = W3{{f[0], f[1], f[2]}};
+    }
+  };
+  auto look_up = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int k = 0; k < 2; ++k) w[k] = dequant_octet(j == 0 ? W[k].w0 : j == 1 ? W[k].w1 : W[k].w2, sc[k]);
-      if (j == 2u) {
-        __builtin_amdgcn_sched_barrier(0);
-        load_w(W, min(s + 2u, s1 - 1u));
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    for (int k = 0; k < 2; ++k) parts[k] = scale_parts(meta[k], table);
+  };
+  auto scales = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < 2; ++k) {
+      sc[k] = block_scale(meta[k], parts[k]);
+      W[k] = Wn[k];
+    }
+  };
+  auto round = [&](uint32_t buffer, uint32_t next, auto round_j) __attribute__((always_inline)) {
+    constexpr uint32_t j = decltype(round_j)::value;
+    const half8_t w0[2] = {w[0], w[1]};
+    half8_t x0[CF];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[k][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[c], w[k], acc[k][c], 0, 0, 0);
+    for (int c = 0; c < CF; ++c) x0[c] = x[c];
+    if (j < 2u) {
+      read_x(buffer, j + 1u);
+      unpack(j + 1u);
+    } else {
+      read_x(next, 0);
+      scales();
+      unpack(0);
+    }
+#pragma unroll
+    for (int c = 0; c < CF; ++c)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) acc[k][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w0[k], x0[c], acc[k][c], 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < CF; ++c) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read,
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product,
+      __builtin_amdgcn_sched_group_barrier(0x002, CF == 8 ? 3 : 5, 0);  // vector instructions
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, CF == 8 ? 3 : 5, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  load_x(s0);
-  __builtin_amdgcn_sched_barrier(0);
-  load_w(Wa, s0);
-  load_w(Wb, min(s0 + 1u, s1 - 1u));
-  for (uint32_t s = s0;;) {
-    step(Wa, s, buf);
-    if (++s >= s1) break;
-    step(Wb, s, buf + kPieces);
-    if (++s >= s1) break;
-  }
-  // element e of a lane: activation row 8 (e / 4) + 4 h + e % 4 of the fragment, weight row l32 of it
-  const uint32_t m0 = mt * kCols + wm * 128u;
-  if (a.splits > 1u) {
-    const uint32_t n_rows = a.n_tiles * kRows;
-    float* out = a.ws + (size_t)split * a.m_pad * n_rows + tile * kRows + wr * 64u + l32;
+  load(s0, 0);
+  load(s0 + 1u, kBuf);
+  load(s0 + 2u, 2u * kBuf);
+  wide_wait<2 * kLoads>();
+  lds_barrier();
+  read_w(0);
+  look_up();
+  read_x(0, 0);
+  scales();
+  unpack(0);
+  uint32_t buffer = 0, next = kBuf, last = 3u * kBuf, s = s0;
+  do {  // (a split has at least one step)
+    round(buffer, next, std::integral_constant<uint32_t, 0>{});
+    wide_wait<kLoads>();
+    lds_barrier();
+    load(s + 3u, last);
+    read_w(next);
+    __builtin_amdgcn_sched_barrier(0);
+    round(buffer, next, std::integral_constant<uint32_t, 1>{});
+    look_up();
+    __builtin_amdgcn_sched_barrier(0);
+    round(buffer, next, std::integral_constant<uint32_t, 2>{});
+    last = buffer;
+    buffer = next;
+    next = next + kBuf == kWideDepth * kBuf ? 0u : next + kBuf;
+  } while (++s < s1);
+  wide_wait<0>();
+  if constexpr (CF == 8) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) store_fragment(out + k * 32, n_rows, acc[k][c], m0 + (uint32_t)c * 32u + 4u * h, a.M);
+      for (int c = 0; c < CF; ++c) asm volatile("" : "+a"(acc[k][c]));  // one by one from here: all of them would not fit the vector registers
+  }
+  // A lane's activation row is l32 of a fragment; element e is weight row 8 (e / 4) + 4 h + e % 4 of it.
+  // (From the lane's number anew: nothing of this may occupy registers during the loop.)
+  const uint32_t lane_e = lane_offset(lane), l32e = lane_e & 31u, he = lane_e >> 5;
+  const uint32_t m0 = mt * kCols + l32e;
+  if (a.splits > 1u) {
+    const uint32_t n_rows = a.n_tiles * kWideRows;
+    float* out = a.ws + (size_t)split * a.m_pad * n_rows;
+#pragma unroll
+    for (int c = 0; c < CF; ++c)
+      if (m0 + (uint32_t)c * 32u < a.M) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          StoreF32::store(out, (size_t)(m0 + (uint32_t)c * 32u) * n_rows, tile * kWideRows + wave * 64u + (uint32_t)k * 32u, he, 0, acc[k][c] * unit);
+      }
     return;
   }
+  // The tail's operands to LDS, columns of all rows: a lane would wait for each of its loads in turn.
+  float* w_tail = reinterpret_cast<float*>(smem);
+  float* x_tail = w_tail + kWideRows * kDim;
+  if (a.tail_w) {
+    __syncthreads();
+    for (uint32_t c0 = 0; c0 < a.tail_w; c0 += 8u) {
+      float v[8];
+      const uint32_t row = tid % kWideRows, m = mt * kCols + tid % kCols;
+      // (the columns are shared out where there are two threads to a row)
+      const float* rec = reinterpret_cast<const float*>(rec0 + record(t.row0 + row) + 32u) + (row & 7u);
+      const __half* tx = a.x + (size_t)min(m, a.M - 1u) * a.ldx + nb * kDim;
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const float* rec = reinterpret_cast<const float*>(wave_rec + rec_off[k]);
-    const float scale = rec[r];
-    const uint32_t row = row0 + (uint32_t)k * 32u + l32;
+      for (uint32_t i = 0; i < 8; ++i) v[i] = rec[min(c0 + i, a.tail_w - 1u) * 8u];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      acc16_t v = acc[k][c];
+      for (uint32_t i = 0; i < 8; ++i)
+        if (tid < kWideRows && c0 + i < a.tail_w) w_tail[(c0 + i) * kWideRows + row] = v[i];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) v[e] *= scale;
-      // f32 tail columns, two at a time: lane half h holds column i + h
-      const __half* tx = a.x + (size_t)min(m0 + (uint32_t)c * 32u + l32, a.M - 1u) * a.ldx + nb * kDim;
-      for (uint32_t i = 0; i < a.tail_w; i += 2u) {
-        const uint32_t col = min(i + h, a.tail_w - 1u);
-        const float keep = i + h < a.tail_w ? 1.f : 0.f;
-        v = __builtin_amdgcn_mfma_f32_32x32x2f32(__half2float(tx[col]), keep * rec[8u + col * 8u + r], v, 0, 0, 0);
-      }
-      if (row >= t.d_out) continue;
-      const uint32_t m = m0 + (uint32_t)c * 32u + 4u * h;
-      if (a.y_f32) store_fragment(reinterpret_cast<float*>(t.y) + row, t.d_out, v, m, a.M);
-      else store_fragment(reinterpret_cast<_Float16*>(t.y) + row, t.d_out, v, m, a.M);
+      for (uint32_t i = 0; i < 8; ++i) v[i] = __half2float(tx[min(c0 + i, a.tail_w - 1u)]);
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i)
+        if (tid < kCols && c0 + i < a.tail_w) x_tail[(c0 + i) * kCols + tid] = v[i];
     }
+    __syncthreads();
+  }
+  auto finish = [&](auto to) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t row = row0 + (uint32_t)k * 32u;
+      float scale[16];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 v = *reinterpret_cast<const float4*>(rec0 + record(row + g * 8u) + he * 16u);
+        scale[4 * g] = v.x * unit;
+        scale[4 * g + 1] = v.y * unit;
+        scale[4 * g + 2] = v.z * unit;
+        scale[4 * g + 3] = v.w * unit;
+      }
+#pragma unroll
+      for (int c = 0; c < CF; ++c) {
+        acc16_t v = acc[k][c];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] *= scale[e];
+        // f32 tail columns, two at a time: the halves hold one each
+        for (uint32_t i = 0; i < a.tail_w; i += 2u) {
+          const uint32_t col = min(i + he, a.tail_w - 1u);
+          const float keep = i + he < a.tail_w ? 1.f : 0.f;
+          v = __builtin_amdgcn_mfma_f32_32x32x2f32(keep * w_tail[col * kWideRows + wave * 64u + (uint32_t)k * 32u + l32e],
+                                                   x_tail[col * kCols + (uint32_t)c * 32u + l32e], v, 0, 0, 0);
+        }
+        const uint32_t m = m0 + (uint32_t)c * 32u;
+        if (m < a.M) decltype(to)::store(t.y, (size_t)m * t.d_out, row, he, t.d_out, v);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  const bool whole = row0 + 64u <= t.d_out && ((reinterpret_cast<uintptr_t>(t.y) | t.d_out * (a.y_f32 ? 4u : 2u)) & 15u) == 0;
+  if (a.y_f32) {
+    if (whole) finish(StoreF32{});
+    else finish(StoreEach<float>{});
+  } else {
+    if (whole) finish(StoreF16{});
+    else finish(StoreEach<_Float16>{});
   }
 }
-template <int WM>
-__host__ constexpr size_t gemm_wide_lds() { return 2ull * gemm_wide_cols<WM>() * 6 * 16; }
 
 // The partial sums of the column splits, added in order; row scale and tail columns.  A lane takes one weight row and
 // kReduceM activation rows, so that the row's tail is read once for them.

@@ -547,6 +547,8 @@ int llvq_hip_runtime_create(int device, void* hip_stream, llvq_rt** out) {
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rotate_kernel<__half>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<1, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_wide_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_wide_kernel<8>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   *out = rt;
   return LLVQ_OK;
 }
@@ -1272,12 +1274,16 @@ static int workspace_take(llvq_rt* rt, GemmWorkspace* w, void** runtime_buf, siz
 }
 
 // Rows of activations one batched launch takes; more go out as further launches.
-constexpr int kGemmMaxM = 1024;
+constexpr uint32_t kGemmMaxM = 1024;
+
+// Measured times of one step (48 columns) of the wide kernel in us: 256 activation rows; 128, two workgroups sharing a
+// CU, each; and one of those alone.
+constexpr double kWideStep = 1.28, kWideHalfStep = 0.69, kWideHalfStepAlone = 0.8;
 
 // How a batched launch over these matrices at M rows is cut up, and the workspaces it needs.
 struct GemmPlan {
   uint32_t small;                // 1: up to 16 rows, 2: up to 64 (gemm_tiles_kernel), 0: gemm_wide_kernel
-  uint32_t wm, rows_per_tile;    // the wide kernel's shape, and weight rows of a workgroup
+  uint32_t cf, rows_per_tile;    // the wide kernel's form, and weight rows of a workgroup
   uint32_t n_tiles, m_pad, m_tiles, splits, steps_per_split, n_oct;
   size_t ws_bytes, xt_bytes;
 };
@@ -1288,41 +1294,37 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
   const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), nb = mats[0]->nblocks;
   GemmPlan p{};
   p.small = M <= 16u ? 1u : M <= kGemmSmallRows ? 2u : 0u;
-  p.n_oct = (nb + 3u) / 4u * 12u;
   p.splits = 1;
   p.m_tiles = 1;
-  auto count_tiles = [&](uint32_t rows) {
-    p.rows_per_tile = rows;
-    p.n_tiles = 0;
-    for (int i = 0; i < n; ++i) p.n_tiles += (mats[i]->d_out + rows - 1u) / rows;
-  };
+  p.rows_per_tile = p.small ? p.small * 16u : kWideRows;
+  for (int i = 0; i < n; ++i) p.n_tiles += (mats[i]->d_out + p.rows_per_tile - 1u) / p.rows_per_tile;
+  p.n_oct = (nb + 3u) / 4u * 12u;
   if (p.small) {
-    count_tiles(p.small * 16u);
     p.m_pad = p.small == 1u ? 16u : 64u;
-  } else {
-    // 128 activation rows per wavefront; two wavefronts side by side where that wastes no column of them
-    const uint32_t m128 = (M + 127u) / 128u;
-    p.wm = m128 % 2u == 0u ? 2u : 1u;
-    count_tiles(64u * (4u / p.wm));
-    p.m_tiles = m128 / p.wm;
-    p.m_pad = p.m_tiles * 128u * p.wm;
-    // Column splits: enough workgroups for two per CU, as long as each keeps eight steps of 48 columns.  The time of a
-    // launch is rounds of resident workgroups times steps, and what the partial sums cost on their way through memory
-    // (measured: a step of two workgroups sharing a CU 0.8 us, partial sums about 4 bytes per ps).
-    const uint32_t steps = (nb + 1u) / 2u, tiles = p.n_tiles * p.m_tiles;
-    const size_t one = (size_t)p.m_pad * p.n_tiles * p.rows_per_tile * sizeof(float);
-    double best = 1e30;
+    p.xt_bytes = (size_t)p.n_oct * p.m_pad * 16;
+    return p;
+  }
+  // The form and the column splits by the time they should take: rounds of resident workgroups times steps of a
+  // workgroup's share of a CU, and for the splits what the partial sums cost on their way through memory.
+  const uint32_t steps = (nb + 1u) / 2u;
+  double best = 1e30;
+  for (uint32_t cf = 8; cf >= 4u; cf -= 4u) {
+    const uint32_t m_tiles = (M + 32u * cf - 1u) / (32u * cf), tiles = p.n_tiles * m_tiles, m_pad = m_tiles * 32u * cf;
+    const size_t one = (size_t)m_pad * p.n_tiles * kWideRows * sizeof(float);
     for (uint32_t sp = 1; sp <= 16u && (sp == 1u || (steps / sp >= 8u && one * sp <= kGemmWsCap)); ++sp) {
-      const uint32_t per = (steps + sp - 1u) / sp, wgs = tiles * ((steps + per - 1u) / per);
-      const double rounds = (double)((wgs + cus - 1u) / cus);
-      const double cost = rounds * per * 0.4 + (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
+      const uint32_t per = (steps + sp - 1u) / sp, wgs = tiles * ((steps + per - 1u) / per), per_cu = (wgs + cus - 1u) / cus;
+      const double cost = (cf == 8u ? per_cu * kWideStep : per_cu == 1u ? kWideHalfStepAlone : per_cu * kWideHalfStep) * per +
+                          (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
       if (cost < best) {
         best = cost;
+        p.cf = cf;
+        p.m_tiles = m_tiles;
+        p.m_pad = m_pad;
         p.splits = (steps + per - 1u) / per;
         p.steps_per_split = per;
+        p.ws_bytes = p.splits > 1u ? one * p.splits : 0;
       }
     }
-    if (p.splits > 1u) p.ws_bytes = one * p.splits;
   }
   p.xt_bytes = (size_t)p.n_oct * p.m_pad * 16;
   return p;
@@ -1334,7 +1336,6 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
 static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint32_t max_rows) {
   if (n <= 0 || max_rows < 2) return LLVQ_OK;
   size_t ws = 0, xt = 0, rows = 0;
-  const uint32_t chunk = max_rows < (uint32_t)kGemmMaxM ? max_rows : (uint32_t)kGemmMaxM;
   for (int i0 = 0; i0 < n;) {
     int i1 = i0 + 1;
     while (i1 < n && i1 - i0 < kGemmMaxGroup && mats[i1]->has_rotation == mats[i0]->has_rotation &&
@@ -1343,6 +1344,7 @@ static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint
     bool six_byte = true;
     for (int i = i0; i < i1; ++i) six_byte &= mats[i]->record_bits == 48;
     if (mats[i0]->nblocks && six_byte) {  // (cap-13 matrices take the row loop, which has no workspace)
+      const uint32_t chunk = std::min(max_rows, kGemmMaxM);
       // every row count up to the chunk: the splits, and so the partial sums, are not monotone in it
       for (uint32_t M = 16;; M = M < 64u ? M + 48u : M < 128u ? 128u : M + 128u) {
         const GemmPlan p = gemm_plan(rt, mats + i0, i1 - i0, M < chunk ? M : chunk);
@@ -1401,10 +1403,11 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   const uint32_t oct_waves = (p.n_oct + 7u) / 8u * (p.m_pad / 8u);
   hipLaunchKernelGGL(tile_activations_kernel, dim3((oct_waves + 3u) / 4u), dim3(256), 0, rt->stream, xh, M, a.ldx, a.nb * 24u, p.m_pad, p.n_oct,
                      reinterpret_cast<uint4*>(xt_buf));
+  const dim3 wide_grid(a.n_tiles * p.m_tiles * p.splits);
   if (p.small == 1u) hipLaunchKernelGGL((gemm_tiles_kernel<1, 1>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<1, 1>()), rt->stream, a);
   else if (p.small) hipLaunchKernelGGL((gemm_tiles_kernel<2, 4>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<2, 4>()), rt->stream, a);
-  else if (p.wm == 1u) hipLaunchKernelGGL(gemm_wide_kernel<1>, dim3(a.n_tiles * p.m_tiles * p.splits), dim3(256), gemm_wide_lds<1>(), rt->stream, a);
-  else hipLaunchKernelGGL(gemm_wide_kernel<2>, dim3(a.n_tiles * p.m_tiles * p.splits), dim3(256), gemm_wide_lds<2>(), rt->stream, a);
+  else if (p.cf == 4u) hipLaunchKernelGGL(gemm_wide_kernel<4>, wide_grid, dim3(256), gemm_wide_lds<4>(), rt->stream, a);
+  else hipLaunchKernelGGL(gemm_wide_kernel<8>, wide_grid, dim3(256), gemm_wide_lds<8>(), rt->stream, a);
   if (p.splits > 1u) {
     r.rows_per_tile = p.rows_per_tile;
     r.row_chunks = (a.n_tiles * p.rows_per_tile + 255u) / 256u;
@@ -1446,6 +1449,7 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
       }
     return LLVQ_OK;
   }
+  const int chunk = std::min(M, (int)kGemmMaxM);
   if (wsp && wsp->fixed) {
     // a call that does not fit is refused whole, before its first launch
     auto after = [](size_t used, size_t bytes) { return ((used + 255) & ~(size_t)255) + bytes; };
@@ -1453,9 +1457,9 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
     size_t need = base;
     for (int m_lo = 0; m_lo < M; m_lo += 512)
       for (int i = 0; i < n; ++i) need = std::max(need, after(base, static_admission_bytes(rt, mats[i], (uint32_t)std::min(M - m_lo, 512))));
-    for (int m_lo = 0; m_lo < M; m_lo += kGemmMaxM)
+    for (int m_lo = 0; m_lo < M; m_lo += chunk)
       for (int i0 = 0; i0 < n; i0 += kGemmMaxGroup) {
-        const GemmPlan p = gemm_plan(rt, mats + i0, std::min(n - i0, kGemmMaxGroup), (uint32_t)std::min(M - m_lo, kGemmMaxM));
+        const GemmPlan p = gemm_plan(rt, mats + i0, std::min(n - i0, kGemmMaxGroup), (uint32_t)std::min(M - m_lo, chunk));
         need = std::max(need, after(p.ws_bytes ? after(base, p.ws_bytes) : base, p.xt_bytes));
       }
     if (need > wsp->fixed_bytes)
@@ -1472,8 +1476,8 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
     if (rc) return rc;
     xb = reinterpret_cast<const uint8_t*>(rows);
   }
-  for (int m_lo = 0; m_lo < M; m_lo += kGemmMaxM) {
-    const uint32_t mc = (uint32_t)(M - m_lo < kGemmMaxM ? M - m_lo : kGemmMaxM);
+  for (int m_lo = 0; m_lo < M; m_lo += chunk) {
+    const uint32_t mc = (uint32_t)std::min(M - m_lo, chunk);
     for (int i0 = 0; i0 < n; i0 += kGemmMaxGroup) {
       const int cnt = n - i0 < kGemmMaxGroup ? n - i0 : kGemmMaxGroup;
       void* ys[kGemmMaxGroup];
