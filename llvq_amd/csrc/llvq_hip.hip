@@ -186,111 +186,180 @@ struct ActivationIn {
   uint32_t rot_m, rot_k;
 };
 
-// x <- (S (x) I_m)(I_k (x) H_m / sqrt m) x in place on n = k m f32 values in LDS whose
-// signs D are already applied (llvq-quant/src/rotation.rs:97-105; f32 like the reference's
-// device rotation, llvq-cuda/kernels/llvq_rot.cuh).  `small` is the k x k block in device
-// memory.  Every thread of a 1024-thread workgroup calls it; the values are final after
-// the caller's next barrier.
-//  * Walsh-Hadamard levels: for m >= 512 a wavefront takes a run of 512 values, eight per
-//    lane, and does nine levels without a barrier (three in registers, six by lane
-//    exchange); the levels above 512, and every level of a narrower m, are radix-2
-//    passes over LDS (groups are contiguous, so one pass covers all of them).
-//  * the k x k block across groups, with the 1/sqrt m factor applied first, is a small
-//    dense product S (k x k) . C (k x m): a wavefront takes 32 columns of C at a time and
-//    runs it as f32 matrix-core steps of depth 2 (S padded with zeros to 32 x 32); it reads
-//    its columns whole before it writes them, and no other wavefront touches them.
+// A workgroup barrier that orders LDS accesses only: loads from memory stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Eight binary16 values at any 2-byte alignment (one 16-byte load).
+struct __attribute__((packed, aligned(2))) HalfOctet { uint32_t w[4]; };
+__device__ __forceinline__ float half_lo(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w & 0xFFFFu))); }
+__device__ __forceinline__ float half_hi(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w >> 16))); }
+
+// The rotation x' = (S (x) I_m)(I_k (x) H_m / sqrt m) D x of an activation of n = k m values, by a workgroup of 1024
+// lanes (llvq-quant/src/rotation.rs:97-105; f32 like the reference's device rotation, llvq-cuda/kernels/llvq_rot.cuh).
+//
+// Every workgroup of a batch-1 product rotates its own activation, so a rotation is a chain that a launch waits for.
+// With a value per lane and load, lane exchanges through LDS and a pass over LDS per level above 512 it took 12 us of
+// the 19.2 of a 2560 x 9728 product.  Here a lane holds eight neighbouring values from the load on (one 16-byte load and
+// a byte of signs, all of a wavefront's requested together) and does nine levels in registers: three inside the lane, six by
+// lane moves of the vector unit (19.2 -> 15.7 us).  The values meet LDS once, rotate_octets_to; the levels above 512 are one pass of
+// register butterflies and the k x k block one pass of f32 matrix-core steps, rotate_rest.
+// Where an octet spans groups (m < 8) the signed values are put into LDS instead and every level is a pass there.
+constexpr uint32_t kRotOctetM = 8;    // the narrowest m that takes the octets
+constexpr uint32_t kRotRun = 512;     // values of a wavefront's run
+__device__ __forceinline__ float flip_sign(float v, uint32_t bits, int j) {  // bit j of `bits` is the sign of D
+  return __uint_as_float(__float_as_uint(v) ^ (((bits >> j) & 1u) << 31));
+}
+// Sum and difference with the lane L away: lower lanes get own + other, upper ones other - own (sgn = -1 there).
+template <int L>
+__device__ __forceinline__ float lane_butterfly(float v, float sgn) {
+  const int i = (int)__float_as_uint(v);
+  if constexpr (L == 16) {  // the swaps leave the lower and the upper lane's value in both
+    const auto p = __builtin_amdgcn_permlane16_swap((uint32_t)i, (uint32_t)i, false, false);
+    return fmaf(sgn, __uint_as_float(p[1]), __uint_as_float(p[0]));
+  } else if constexpr (L == 32) {
+    const auto p = __builtin_amdgcn_permlane32_swap((uint32_t)i, (uint32_t)i, false, false);
+    return fmaf(sgn, __uint_as_float(p[1]), __uint_as_float(p[0]));
+  } else {
+    int o;
+    if constexpr (L == 1) o = __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, false);
+    if constexpr (L == 2) o = __builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, false);
+    if constexpr (L == 4) {  // lane ^ 7, then lane ^ 3
+      o = __builtin_amdgcn_update_dpp(0, i, 0x141, 0xF, 0xF, false);
+      o = __builtin_amdgcn_update_dpp(0, o, 0x1B, 0xF, 0xF, false);
+    }
+    if constexpr (L == 8) o = __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, false);
+    return fmaf(sgn, v, __uint_as_float((uint32_t)o));
+  }
+}
+template <int L>
+__device__ __forceinline__ void lane_level(float (&r)[8], uint32_t lane, uint32_t m) {
+  if (m >= 16u * (uint32_t)L) {
+    const float sgn = (lane & (uint32_t)L) ? -1.f : 1.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = lane_butterfly<L>(r[i], sgn);
+  }
+}
+// The levels below min(m, 512) of the signed values at `at` (lane-contiguous octets of a run), into LDS where at < n.
+__device__ __forceinline__ void rotate_octets_to(float* v, float (&r)[8], uint32_t at, uint32_t n, uint32_t m, uint32_t k, float inv) {
+  const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+  for (int l = 1; l < 8; l <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & l)) {
+        const float u = r[i], w = r[i | l];
+        r[i] = u + w;
+        r[i | l] = u - w;
+      }
+  lane_level<1>(r, lane, m);
+  lane_level<2>(r, lane, m);
+  lane_level<4>(r, lane, m);
+  lane_level<8>(r, lane, m);
+  lane_level<16>(r, lane, m);
+  lane_level<32>(r, lane, m);
+  if (k == 1 && m <= kRotRun) {  // nothing follows but the factor
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] *= inv;
+  }
+  if (at < n) {
+    float4* dst = reinterpret_cast<float4*>(v + at);
+    dst[0] = make_float4(r[0], r[1], r[2], r[3]);
+    dst[1] = make_float4(r[4], r[5], r[6], r[7]);
+  }
+}
+// log2 R levels from 2^lg on, by all lanes: butterflies over R values 2^lg apart.
+template <uint32_t R>
+__device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t lg, float factor) {
+  for (uint32_t p = threadIdx.x; p < n / R; p += 1024u) {
+    float* at = v + (p >> lg) * (R << lg) + (p & ((1u << lg) - 1u));
+    float r[R];
+#pragma unroll
+    for (uint32_t i = 0; i < R; ++i) r[i] = at[i << lg];
+#pragma unroll
+    for (uint32_t l = 1; l < R; l <<= 1)
+#pragma unroll
+      for (uint32_t i = 0; i < R; ++i)
+        if (!(i & l)) {
+          const float u = r[i], w = r[i | l];
+          r[i] = u + w;
+          r[i | l] = u - w;
+        }
+#pragma unroll
+    for (uint32_t i = 0; i < R; ++i) at[i << lg] = r[i] * factor;
+  }
+}
+
+// The part of S a lane multiplies with, S[l32][2 s + lh]: loaded before the levels, so that it is there when they are done.
 typedef float rot_acc_t __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ void rotate_lds(float* v, uint32_t n, uint32_t m, uint32_t k, float inv,
-                                           const float* __restrict__ small) {
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t l32 = lane & 31u, lh = lane >> 5;
-  const uint32_t steps = (k + 1u) >> 1;  // depth-2 steps that cover k
-  // S[l32][2 s + lh], requested before the butterflies so that the loads are back by the time they are used
-  float s_frag[kRotKMax / 2];
+struct RotBlock { float s[kRotKMax / 2]; };
+__device__ __forceinline__ RotBlock load_rot_block(const float* __restrict__ small, uint32_t k) {
+  const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, lh = lane >> 5;
+  RotBlock b;
 #pragma unroll
   for (uint32_t s = 0; s < kRotKMax / 2; ++s) {
     const uint32_t t = 2u * s + lh;
-    s_frag[s] = (k > 1 && m >= 32 && l32 < k && t < k) ? small[l32 * k + t] : 0.f;
+    const bool in = l32 < k && t < k;
+    const float e = small[in ? l32 * k + t : 0u];  // always a valid address, so the loads go out together
+    b.s[s] = in ? e : 0.f;
   }
-  uint32_t len0 = 1;
-  if (m >= 512) {
-    for (uint32_t c = wave; c < (n >> 9); c += 16) {
-      float4* src = reinterpret_cast<float4*>(v + (c << 9) + lane * 8u);
-      const float4 lo = src[0], hi = src[1];
-      float r[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  return b;
+}
+
+// What is left once the levels below 512 are in LDS (every level, `put_levels`, where the octets were not taken): the values
+// are final after the caller's next barrier.  Called behind a barrier.
+__device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, uint32_t k, float inv, const float* __restrict__ small,
+                                            const RotBlock& S, bool put_levels) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t l32 = lane & 31u, lh = lane >> 5;
+  // three levels to a pass, what is over in the last
+  for (uint32_t lg = put_levels ? 0u : 31u - (uint32_t)__builtin_clz(kRotRun); (1u << lg) < m; lg += 3u) {
+    const bool last = (8u << lg) >= m;
+    const float factor = last && k == 1 ? inv : 1.f;
+    if ((m >> lg) >= 8u) rotate_levels<8>(v, n, lg, factor);
+    else if ((m >> lg) == 4u) rotate_levels<4>(v, n, lg, factor);
+    else rotate_levels<2>(v, n, lg, factor);
+    if (!last || k > 1) lds_barrier();
+  }
+  if (k == 1 && m == 1) {  // (a row of one value)
+    if (tid == 0) v[0] *= inv;
+  }
+  if (k == 1) return;
+  // S (k x k) . C (k x m), the 1 / sqrt m factor first: a wavefront takes 32 columns of C at a time as f32 matrix-core
+  // steps of depth 2 (S padded with zeros to 32 x 32; lanes past a narrow m repeat its first column); it reads its columns
+  // whole before it writes them, and no other wavefront touches them.
+  const uint32_t steps = (k + 1u) >> 1;
+  for (uint32_t tile = wave; tile * 32u < m; tile += 16) {
+    const uint32_t j = tile * 32u + l32;
+    rot_acc_t acc;
 #pragma unroll
-      for (int l = 1; l < 8; l <<= 1)
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    uint32_t rows = k - lh;  // 2 s < rows: step s has a row for this half
+    asm volatile("" : "+v"(rows));  // (compared in each tile: kept across tiles, sixteen masks would crowd the scalar registers)
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (!(i & l)) {
-            const float u = r[i], w = r[i | l];
-            r[i] = u + w;
-            r[i | l] = u - w;
-          }
+    for (uint32_t s0 = 0; s0 < kRotKMax / 2; s0 += 8u) {  // half the steps at a time: the weights in flight leave registers for that
+      if (s0 >= steps) break;
+      float c_frag[8];
 #pragma unroll
-      for (int l = 1; l < 64; l <<= 1) {
-        const bool upper = (lane & (uint32_t)l) != 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float other = __shfl_xor(r[i], l, 64);
-          r[i] = upper ? other - r[i] : r[i] + other;
-        }
+      for (uint32_t i = 0; i < 8u; ++i) {
+        const uint32_t t = 2u * (s0 + i);
+        const float x = v[(t < rows ? (t + lh) * m : 0u) + (j < m ? j : 0u)];  // always a valid address, so the reads go out together
+        c_frag[i] = t < rows ? x * inv : 0.f;
       }
-      src[0] = make_float4(r[0], r[1], r[2], r[3]);
-      src[1] = make_float4(r[4], r[5], r[6], r[7]);
+#pragma unroll
+      for (uint32_t i = 0; i < 8u; ++i)
+        if (s0 + i < steps) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(S.s[s0 + i], c_frag[i], acc, 0, 0, 0);
     }
-    len0 = 512;
-  }
-  __syncthreads();
-  for (uint32_t len = len0; len < m; len <<= 1) {
-    for (uint32_t p = tid; p < (n >> 1); p += 1024) {
-      const uint32_t j = (p / len) * (len << 1) + (p % len);
-      const float u = v[j], w = v[j + len];
-      v[j] = u + w;
-      v[j + len] = u - w;
-    }
-    __syncthreads();
-  }
-  if (k == 1) {
-    for (uint32_t i = tid; i < n; i += 1024) v[i] = v[i] * inv;
-    return;
-  }
-  if (m >= 32) {
-    for (uint32_t tile = wave; tile < (m >> 5); tile += 16) {
-      const uint32_t j = (tile << 5) + l32;
-      float c_frag[kRotKMax / 2];
+    // acc[r] is row 8 (r / 4) + 4 lh + r % 4 of column j
+    uint32_t left = j < m && k > 4u * lh ? k - 4u * lh : 0u;  // rows of the block from this half's first on
+    asm volatile("" : "+v"(left));
 #pragma unroll
-      for (uint32_t s = 0; s < kRotKMax / 2; ++s) {
-        const uint32_t t = 2u * s + lh;
-        const float x = v[(t < k ? t * m : 0u) + j];  // always a valid address, so the reads go out together
-        c_frag[s] = t < k ? x * inv : 0.f;
-      }
-      rot_acc_t acc;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-#pragma unroll
-      for (uint32_t s = 0; s < kRotKMax / 2; ++s)
-        if (s < steps) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s_frag[s], c_frag[s], acc, 0, 0, 0);
-      // acc[r] is row 8 (r / 4) + 4 lh + r % 4 of column j
-#pragma unroll
-      for (uint32_t r = 0; r < 16; ++r) {
-        const uint32_t g = 8u * (r >> 2) + 4u * lh + (r & 3u);
-        if (g < k) v[g * m + j] = acc[r];
-      }
-    }
-    return;
-  }
-  // narrow groups (m < 32): one thread per column
-  for (uint32_t j = tid; j < m; j += 1024) {
-    float col[kRotKMax];
-#pragma unroll
-    for (uint32_t t = 0; t < kRotKMax; ++t) col[t] = t < k ? v[t * m + j] * inv : 0.f;
-    for (uint32_t g = 0; g < k; ++g) {
-      float acc = 0.f;
-#pragma unroll
-      for (uint32_t t = 0; t < kRotKMax; ++t)
-        if (t < k) acc = fmaf(small[g * k + t], col[t], acc);
-      v[g * m + j] = acc;
+    for (uint32_t r = 0; r < 16; ++r) {
+      const uint32_t g = 8u * (r >> 2) + (r & 3u);
+      if (g < left) v[(g + 4u * lh) * m + j] = acc[r];
     }
   }
 }
@@ -326,10 +395,7 @@ __device__ __forceinline__ void store_half(__half* p, __half v) {
 }
 
 // ---- incoherence rotation of an activation ----------------------------------------
-// x' = Q x for Q = (S (x) I_m)(I_k (x) H_m / sqrt m) D (llvq-quant/src/rotation.rs:97-105),
-// in f32 like the reference's device rotation (llvq-cuda/kernels/llvq_rot.cuh): signs on
-// load, radix-2 Walsh-Hadamard butterflies inside each group of m, then the k x k block
-// across groups with the 1/sqrt m factor applied first.  One workgroup per activation row.
+// One workgroup per activation row.
 struct RotArgs {
   const __half* x;        // [rows, n]
   void* out;              // [rows, n] f32 or f16
@@ -350,14 +416,50 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
   extern __shared__ __align__(16) float rot_s[];
   const uint32_t tid = threadIdx.x, n = a.n, m = a.m, k = a.k;
   const __half* x = a.x + (size_t)blockIdx.x * n;
-  for (uint32_t i = tid; i < n; i += 1024) {
-    const float v = __half2float(x[i]);
-    rot_s[i] = ((a.signbits[i >> 5] >> (i & 31u)) & 1u) ? -v : v;
+  const RotBlock S = load_rot_block(a.small, k);
+  if (m >= kRotOctetM) {
+    const uint8_t* signs = reinterpret_cast<const uint8_t*>(a.signbits);
+    constexpr int kRuns = 2;  // of a wavefront at a time
+    for (uint32_t at0 = (tid >> 6) * kRotRun; at0 < n; at0 += kRuns * 16u * kRotRun) {
+      HalfOctet o[kRuns];
+      uint32_t sg[kRuns];
+#pragma unroll
+      for (int p = 0; p < kRuns; ++p) {
+        const uint32_t at = at0 + (uint32_t)p * 16u * kRotRun + (tid & 63u) * 8u, from = at < n ? at : 0u;
+        o[p] = *reinterpret_cast<const HalfOctet*>(x + from);
+        sg[p] = signs[from >> 3];
+      }
+#pragma unroll
+      for (int p = 0; p < kRuns; ++p) {
+        const uint32_t at = at0 + (uint32_t)p * 16u * kRotRun + (tid & 63u) * 8u;
+        float r[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          r[2 * j] = flip_sign(half_lo(o[p].w[j]), sg[p], 2 * j);
+          r[2 * j + 1] = flip_sign(half_hi(o[p].w[j]), sg[p], 2 * j + 1);
+        }
+        rotate_octets_to(rot_s, r, at, n, m, k, a.inv);
+      }
+    }
+  } else {
+    for (uint32_t i = tid; i < n; i += 1024) rot_s[i] = flip_sign(__half2float(x[i]), a.signbits[i >> 5] >> (i & 31u), 0);
   }
   __syncthreads();
-  rotate_lds(rot_s, n, m, k, a.inv, a.small);
+  rotate_rest(rot_s, n, m, k, a.inv, a.small, S, m < kRotOctetM);
   __syncthreads();
   OutT* out = reinterpret_cast<OutT*>(a.out) + (size_t)blockIdx.x * n;
+  if constexpr (std::is_same<OutT, __half>::value) {
+    if (m >= kRotOctetM) {
+      for (uint32_t i = tid * 8u; i < n; i += 8192) {
+        HalfOctet o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(rot_s[i + 2 * j])) | (uint32_t)__half_as_ushort(__float2half_rn(rot_s[i + 2 * j + 1])) << 16;
+        *reinterpret_cast<HalfOctet*>(out + i) = o;
+      }
+      return;
+    }
+  }
   for (uint32_t i = tid; i < n; i += 1024) out[i] = (OutT)rot_s[i];
 }
 

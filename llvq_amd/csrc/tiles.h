@@ -115,13 +115,6 @@ __device__ __forceinline__ T* uniform_global(T* p) {
 // In LDS a block is 3 dwords per digit, the sum of its integers (v = 2 n + p: sum v x = 2 sum n x + p sum x) and the scale.
 template <int DIG> struct XPlanes { static constexpr uint32_t kDwords = 3 * DIG + 2; };
 
-// A workgroup barrier that orders LDS accesses only: loads from memory stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // An inclusive maximum of the lanes' |f32| bit patterns over a quad (integers: a NaN is larger than anything).
 __device__ __forceinline__ uint32_t quad_max(uint32_t v) {
   v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));
@@ -259,11 +252,7 @@ __device__ __forceinline__ GemvLds gemv_lds(uint8_t* smem, uint32_t plane_blocks
   return L;
 }
 
-// Eight binary16 values at any 2-byte alignment (one 16-byte load).
-struct __attribute__((packed, aligned(2))) HalfOctet { uint32_t w[4]; };
 struct __attribute__((packed, aligned(4))) FloatOctet { float v[8]; };
-__device__ __forceinline__ float half_lo(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w & 0xFFFFu))); }
-__device__ __forceinline__ float half_hi(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w >> 16))); }
 __device__ __forceinline__ float round_half(float v) { return __half2float(__float2half_rn(v)); }
 __device__ __forceinline__ float silu_mul(float gate, float up) { return round_half(round_half(gate / (1.0f + __expf(-gate))) * up); }
 
@@ -300,37 +289,103 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
   if (tid < 32u) L.xtail[tid] = 0.f;
   for (uint32_t i = tid; i < 8u * kStr; i += n_thr) L.planes[pad * kStr + i] = 0u;  // the step of zeros
   if constexpr (SRC == kSrcRotated) {
-    // Signs applied, the values go to LDS as f32, are rotated there and quantised from there.
-    // (A finished f32 activation is quantised from where it is.)
+    // The activation is rotated into LDS and quantised from there (a finished f32 one from where it is).
+    // A launch in a rotated basis has 1024 lanes.
     float* xf = L.xf;
     if (in.x_f32) {
       request();
     } else {
-      auto put = [&](uint32_t i, float v) { xf[i] = ((in.rot_signbits[i >> 5] >> (i & 31u)) & 1u) ? -v : v; };
-      if (in.prologue == kPrologueAddRmsNorm) {
-        float ss = 0.f;
-        for (uint32_t i = tid; i < d_in; i += n_thr) {
-          float r = __half2float(in.x[i]);
-          if (in.x2) r = round_half(r + __half2float(in.x2[i]));
-          if (in.resid_out && store_resid) in.resid_out[i] = __float2half_rn(r);
-          xf[i] = r;
-          ss += r * r;
-        }
-        request();
+      const RotBlock S = load_rot_block(in.rot_small, in.rot_k);
+      const bool norm = in.prologue == kPrologueAddRmsNorm, silu = in.prologue == kPrologueSiluMul;
+      auto norm_scale = [&](float ss) {
         ss = wave_sum(ss);
         if (lane == 0) L.red[wave] = ss;
         lds_barrier();
         float total = 0.f;
         for (uint32_t w = 0; w < (n_thr >> 6); ++w) total += L.red[w];
-        const float inv = 1.0f / sqrtf(total / (float)d_in + in.eps);
-        for (uint32_t i = tid; i < d_in; i += n_thr) put(i, round_half(xf[i] * inv * __half2float(in.norm_w[i])));
+        return 1.0f / sqrtf(total / (float)d_in + in.eps);
+      };
+      if (in.rot_m >= kRotOctetM) {
+        // every operand of the wavefront's runs is requested before the first is used; one that is not there reads x
+        constexpr int kRuns = PMAX > 2 ? 3 : 2;  // of 16: rows past 512 blocks, or not
+        const __half* second = in.x2 ? in.x2 : in.x;
+        const __half* third = norm ? in.norm_w : in.x;
+        const uint8_t* signs = reinterpret_cast<const uint8_t*>(in.rot_signbits);
+        HalfOctet a[kRuns], b[kRuns], g[kRuns];
+        uint32_t sg[kRuns];
+        auto octet_at = [&](int p) { return ((uint32_t)p * 16u + wave) * kRotRun + lane * 8u; };
+#pragma unroll
+        for (int p = 0; p < kRuns; ++p) {
+          const uint32_t from = octet_at(p) < d_in ? octet_at(p) : 0u;
+          a[p] = *reinterpret_cast<const HalfOctet*>(in.x + from);
+          b[p] = *reinterpret_cast<const HalfOctet*>(second + from);
+          g[p] = *reinterpret_cast<const HalfOctet*>(third + from);
+          sg[p] = signs[from >> 3];
+        }
+        if constexpr (kRuns == 2) request();
+        __builtin_amdgcn_sched_barrier(0);
+        float inv = 0.f;
+        if (norm) {
+          float ss = 0.f;
+#pragma unroll
+          for (int p = 0; p < kRuns; ++p) {
+            if (octet_at(p) >= d_in) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              float lo = half_lo(a[p].w[j]), hi = half_hi(a[p].w[j]);
+              if (in.x2) {
+                lo = round_half(lo + half_lo(b[p].w[j]));
+                hi = round_half(hi + half_hi(b[p].w[j]));
+              }
+              a[p].w[j] = (uint32_t)__half_as_ushort(__float2half_rn(lo)) | (uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16;
+              ss = fmaf(lo, lo, fmaf(hi, hi, ss));
+            }
+            if (in.resid_out && store_resid) *reinterpret_cast<HalfOctet*>(in.resid_out + octet_at(p)) = a[p];
+          }
+          inv = norm_scale(ss);
+        }
+#pragma unroll
+        for (int p = 0; p < kRuns; ++p) {
+          if (((uint32_t)p * 16u + wave) * kRotRun >= d_in) break;
+          float v[8];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float lo = half_lo(a[p].w[j]), hi = half_hi(a[p].w[j]);
+            if (silu) {
+              lo = silu_mul(half_lo(b[p].w[j]), lo);
+              hi = silu_mul(half_hi(b[p].w[j]), hi);
+            } else if (norm) {
+              lo = round_half(lo * inv * half_lo(g[p].w[j]));
+              hi = round_half(hi * inv * half_hi(g[p].w[j]));
+            }
+            v[2 * j] = flip_sign(lo, sg[p], 2 * j);
+            v[2 * j + 1] = flip_sign(hi, sg[p], 2 * j + 1);
+          }
+          rotate_octets_to(xf, v, octet_at(p), d_in, in.rot_m, in.rot_k, in.rot_inv);
+        }
+        if constexpr (kRuns > 2) request();  // (no registers for a wide step beside the operands)
       } else {
-        for (uint32_t i = tid; i < d_in; i += n_thr)
-          put(i, in.prologue == kPrologueSiluMul ? silu_mul(__half2float(in.x2[i]), __half2float(in.x[i])) : __half2float(in.x[i]));
-        request();
+        auto put = [&](uint32_t i, float v) { xf[i] = flip_sign(v, in.rot_signbits[i >> 5] >> (i & 31u), 0); };
+        if (norm) {
+          float ss = 0.f;
+          for (uint32_t i = tid; i < d_in; i += n_thr) {
+            float r = __half2float(in.x[i]);
+            if (in.x2) r = round_half(r + __half2float(in.x2[i]));
+            if (in.resid_out && store_resid) in.resid_out[i] = __float2half_rn(r);
+            xf[i] = r;
+            ss += r * r;
+          }
+          request();
+          const float inv = norm_scale(ss);
+          for (uint32_t i = tid; i < d_in; i += n_thr) put(i, round_half(xf[i] * inv * __half2float(in.norm_w[i])));
+        } else {
+          for (uint32_t i = tid; i < d_in; i += n_thr)
+            put(i, silu ? silu_mul(__half2float(in.x2[i]), __half2float(in.x[i])) : __half2float(in.x[i]));
+          request();
+        }
       }
       lds_barrier();
-      rotate_lds(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, in.rot_small);
+      rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, in.rot_small, S, in.rot_m < kRotOctetM);
       lds_barrier();
     }
     for (uint32_t p = 0; p < passes; ++p) {

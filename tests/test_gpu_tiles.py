@@ -57,3 +57,27 @@ def test_batched_products(gpu_rt, orc, nb, tail, d_out, M):
     assert _check(Y32.cpu().numpy(), Y_ref, A_ref) < 3e-4  # weights are rounded to binary16
     _check(Y16.float().cpu().numpy(), Y_ref, A_ref, out_rounding=2.0 ** -11)
     assert torch.equal(again, Y32)
+
+
+# Rotations: octets that span groups (m < 8), groups of an octet up to one run of 512, levels above it in one pass of 2, 4
+# or 8 and in two, blocks of every depth; rows whose last run is short.  Bound: a rounding per level and per term of the
+# k x k block, at most 2^-24 of the row's norm each.
+@pytest.mark.parametrize("n", [5, 6, 12, 8, 16, 24, 31 * 8, 31 * 32, 1024, 3 * 1024, 29 * 512, 17 * 1024, 7 * 2048, 3 * 4096, 16384, 32768])
+def test_rotations(gpu_rt, orc, n):
+    import torch
+
+    raw = synth.make_matrix(f"model.layers.0.rot{n}.weight", 9, n, seed=n)
+    raw.rotation_seed = 77 + n
+    X = synth.make_activation(n, seed=n, rows=3)
+    want = np.stack([orc.Rotation(n, 77 + n).apply(x.astype(np.float64)) for x in X])
+    proj = gpu_rt.upload(raw)
+    try:
+        xr = np.stack([gpu_rt.rotate(proj, x).cpu().numpy().reshape(-1) for x in _x16(X)])
+        levels = (n & -n).bit_length() + n // (n & -n) + 1
+        assert np.linalg.norm(xr - want, axis=1).max() <= levels * 2.0 ** -24 * np.linalg.norm(want, axis=1).max()
+        if 24 <= n <= 24 * 1024:
+            one = gpu_rt.forward(proj, _x16(X)[0], out_dtype=torch.float32).reshape(-1)
+            two = gpu_rt.forward_rotated(proj, gpu_rt.rotate(proj, _x16(X)[0]), out_dtype=torch.float32).reshape(-1)
+            assert torch.equal(one, two)
+    finally:
+        gpu_rt.free(proj)
