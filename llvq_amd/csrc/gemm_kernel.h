@@ -599,40 +599,68 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
 
 // The partial sums of the column splits, added in order; row scale and tail columns.  A lane takes one weight row and
 // kReduceM activation rows, so that the row's tail is read once for them.
+// What bounds it is how many round trips to memory a lane makes: the sums and the tail columns are read four splits and
+// eight columns at a time, the activations' tail comes to LDS with the first of them.  (One by one 11.3 us for 500
+// rows of 2560 with 8 or 16 tail columns and 14.9 for 6144; so 9.0 and 10.3.)
 constexpr uint32_t kReduceM = 8;
+constexpr uint32_t kReduceSplits = 4;
 struct GemmReduceArgs {
   GemmArgs g;
   uint32_t rows_per_tile, row_chunks;
 };
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
+  __shared__ float x_tail[kReduceM][32];
+  static_assert(kReduceM * 32u == 256u && kDim <= 32, "a value of the activations' tail per lane");
   const GemmArgs& a = ra.g;
   const uint32_t n_rows = a.n_tiles * ra.rows_per_tile;
   const uint32_t chunk = blockIdx.x % ra.row_chunks, m0 = blockIdx.x / ra.row_chunks * kReduceM;
-  const uint32_t out_row = chunk * 256u + threadIdx.x;
-  if (out_row >= n_rows) return;
+  const uint32_t mine = chunk * 256u + threadIdx.x, out_row = min(mine, n_rows - 1u);  // lanes past the last row repeat it
   const GemmTile t = gemm_tile_at(a, out_row / ra.rows_per_tile, ra.rows_per_tile);
-  const uint32_t row = t.row0 + out_row % ra.rows_per_tile;
-  if (row >= t.d_out) return;
+  const uint32_t my_row = t.row0 + out_row % ra.rows_per_tile, row = min(my_row, t.d_out - 1u);
   const uint32_t stride = tile_stride(a.nb, a.tail_w);
   const uint8_t* rec = t.base + kTileTableBytes + (size_t)(row / kTileRows) * stride;
-  const uint32_t r = row & 7u;
+  const uint32_t r = row & 7u, tail_w = a.tail_w;
+  if (tail_w) {
+    const uint32_t m = min(m0 + threadIdx.x / 32u, a.M - 1u), c = min(threadIdx.x % 32u, tail_w - 1u);
+    x_tail[threadIdx.x / 32u][threadIdx.x % 32u] = __half2float(a.x[(size_t)m * a.ldx + a.nb * kDim + c]);
+  }
+  const float scale = reinterpret_cast<const float*>(rec)[r];
   float s[kReduceM];
 #pragma unroll
   for (uint32_t k = 0; k < kReduceM; ++k) s[k] = 0.f;
-  for (uint32_t p = 0; p < a.splits; ++p)
+  for (uint32_t p0 = 0; p0 < a.splits; p0 += kReduceSplits) {
+    float v[kReduceSplits][kReduceM];
 #pragma unroll
-    for (uint32_t k = 0; k < kReduceM; ++k) s[k] += a.ws[((size_t)p * a.m_pad + min(m0 + k, a.M - 1u)) * n_rows + out_row];
-  const float scale = reinterpret_cast<const float*>(rec)[r];
+    for (uint32_t p = 0; p < kReduceSplits; ++p)
 #pragma unroll
-  for (uint32_t k = 0; k < kReduceM; ++k) s[k] *= scale;
-  for (uint32_t c = 0; c < a.tail_w; ++c) {
-    const float tw = reinterpret_cast<const float*>(rec + 32)[c * 8u + r];
+      for (uint32_t k = 0; k < kReduceM; ++k)
+        v[p][k] = a.ws[((size_t)min(p0 + p, a.splits - 1u) * a.m_pad + min(m0 + k, a.M - 1u)) * n_rows + out_row];
 #pragma unroll
-    for (uint32_t k = 0; k < kReduceM; ++k) s[k] = fmaf(tw, __half2float(a.x[(size_t)min(m0 + k, a.M - 1u) * a.ldx + a.nb * kDim + c]), s[k]);
+    for (uint32_t p = 0; p < kReduceSplits; ++p)
+#pragma unroll
+      for (uint32_t k = 0; k < kReduceM; ++k) s[k] = p0 + p < a.splits ? s[k] + v[p][k] : s[k];
   }
 #pragma unroll
-  for (uint32_t k = 0; k < kReduceM; ++k)
-    if (m0 + k < a.M) store_y(t.y, (size_t)(m0 + k) * t.d_out + row, s[k], a.y_f32);
+  for (uint32_t k = 0; k < kReduceM; ++k) s[k] *= scale;
+  if (tail_w) {
+    lds_barrier();
+    for (uint32_t c0 = 0; c0 < tail_w; c0 += 8u) {
+      float tw[8];
+#pragma unroll
+      for (uint32_t c = 0; c < 8u; ++c) tw[c] = reinterpret_cast<const float*>(rec + 32)[min(c0 + c, tail_w - 1u) * 8u + r];
+#pragma unroll
+      for (uint32_t c = 0; c < 8u; ++c)
+        if (c0 + c < tail_w) {
+#pragma unroll
+          for (uint32_t k = 0; k < kReduceM; ++k) s[k] = fmaf(tw[c], x_tail[k][c0 + c], s[k]);
+        }
+    }
+  }
+  if (mine < n_rows && my_row < t.d_out) {
+#pragma unroll
+    for (uint32_t k = 0; k < kReduceM; ++k)
+      if (m0 + k < a.M) store_y(t.y, (size_t)(m0 + k) * t.d_out + row, s[k], a.y_f32);
+  }
 }
 
 }  // namespace llvq
