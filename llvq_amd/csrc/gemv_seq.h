@@ -244,10 +244,7 @@ __global__ __launch_bounds__(1024) void gemv_seq_kernel(SeqArgs s) {
         if (((n + 1u) & (split - 1u)) == 0u) {
           p -= w * 8u;
           q -= w * 8u;
-          float sum = 0.f, t = 0.f;
-          for (uint32_t k = 0; k < split; ++k) sum += p[k * 8u + r];
-          for (uint32_t k = 0; k < tail_waves; ++k) t += q[k * 8u + r];
-          const float v = fmaf(sum, row_scale, t);
+          const float v = team_sum(p, q, row_scale, split, tail_waves, lane);
           const uint32_t row = team * kTileRows + r;
           if (lane < 8u && row < cur.rows) {
             if constexpr (kWaits) {  // a later item of this launch may read it from another XCD
