@@ -127,21 +127,28 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
+// The served width, head_dim = 128: a lane's two elements (lane, lane + 64) are a rotation pair, so nothing crosses lanes but
+// the sum of squares, and a caller can request the operands of several heads before it finishes the first.
+struct HeadOperands { __half x1, x2, w1, w2; };
+struct RopeAngle { __half c, s; };
+__device__ __forceinline__ HeadOperands head_operands_128(const __half* __restrict__ src, const __half* __restrict__ w, uint32_t a, uint32_t b) {
+  return HeadOperands{src[a], src[b], w[a], w[b]};
+}
+__device__ __forceinline__ float2 norm_rope_128(const HeadOperands& h, const RopeAngle& a, float eps) {
+  const float x1 = __half2float(h.x1), x2 = __half2float(h.x2), c = __half2float(a.c), sn = __half2float(a.s);
+  const float ss = wave_sum(x1 * x1 + x2 * x2);
+  const float inv = 1.0f / sqrtf(ss / 128.0f + eps);
+  const float n1 = __half2float(__float2half_rn(x1 * inv * __half2float(h.w1))), n2 = __half2float(__float2half_rn(x2 * inv * __half2float(h.w2)));
+  return make_float2(__half2float(__float2half_rn(n1 * c - n2 * sn)), __half2float(__float2half_rn(n1 * sn + n2 * c)));
+}
 __device__ __forceinline__ void norm_rope_wave(const __half* __restrict__ src, const __half* __restrict__ w,
                                                const __half* __restrict__ cos_t, const __half* __restrict__ sin_t,
                                                uint32_t pos, uint32_t head_dim, float eps, float* stage, uint32_t lane) {
   const uint32_t half_d = head_dim >> 1;
   if (head_dim == 128) {
-    // the served width: a lane's two elements (lane, lane + 64) are a rotation pair, so nothing
-    // crosses lanes but the sum of squares, and every load goes out before the first use
-    const float x1 = __half2float(src[lane]), x2 = __half2float(src[lane + 64]);
-    const float w1 = __half2float(w[lane]), w2 = __half2float(w[lane + 64]);
-    const float c = __half2float(cos_t[(size_t)pos * 64 + lane]), sn = __half2float(sin_t[(size_t)pos * 64 + lane]);
-    const float ss = wave_sum(x1 * x1 + x2 * x2);
-    const float inv = 1.0f / sqrtf(ss / 128.0f + eps);
-    const float n1 = __half2float(__float2half_rn(x1 * inv * w1)), n2 = __half2float(__float2half_rn(x2 * inv * w2));
-    stage[lane] = __half2float(__float2half_rn(n1 * c - n2 * sn));
-    stage[lane + 64] = __half2float(__float2half_rn(n1 * sn + n2 * c));
+    const float2 r = norm_rope_128(head_operands_128(src, w, lane, lane + 64u), RopeAngle{cos_t[(size_t)pos * 64 + lane], sin_t[(size_t)pos * 64 + lane]}, eps);
+    stage[lane] = r.x;
+    stage[lane + 64] = r.y;
     wave_lds_sync();
     return;
   }
@@ -402,25 +409,33 @@ __global__ __launch_bounds__(64) void attn_rows_kernel(const __half* __restrict_
 //   O^T += V^T P^T   8 x the same MFMA; B = the probabilities just computed, rounded to
 //                    binary16 in the lanes that hold them (no cross-lane movement: the K
 //                    index of the product is permuted to match, V^T is stored in that order).
+// H = 2: a second set of wavefronts walks every other tile, and the two sets' sums are joined at the end: the walk is a
+// chain (16 tiles for the last rows of a 500-row prompt), and a prompt's workgroups leave CUs idle.  31 -> 22 us for 500 rows of 32 heads.
 // Scores, maxima, sums and O stay in f32; the context is rounded once.  The next tile's K and
 // V rows are requested before the current tile is multiplied.  Positions past the pass's last
 // row are read as that row (their probabilities are zero; the values must be finite).
 constexpr int kAttnTile = 32;
 constexpr int kAttnKPitch = 128 + 8;   // binary16 elements per K row in LDS
 constexpr int kAttnVPitch = 32 + 8;    // per V^T row
-template <bool Q8, int G>
-__global__ __launch_bounds__(G * 64) void attn_rows_mfma_kernel(const __half* __restrict__ q, const __half* __restrict__ kcache,
+template <bool Q8, int G, int H>
+__global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half* __restrict__ q, const __half* __restrict__ kcache,
                                                                 const __half* __restrict__ vcache, KvQ8 q8,
                                                                 __half* __restrict__ ctx, uint32_t n_heads, uint32_t n_kv,
                                                                 uint32_t pos0, uint32_t n_rows, uint32_t max_pos, float scale) {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   typedef float f16v __attribute__((ext_vector_type(16)));
-  constexpr uint32_t kDimH = 128, kThreads = G * 64;
+  constexpr uint32_t kDimH = 128, kThreads = G * 64;  // threads of a part
   constexpr int CH = (kAttnTile * kDimH / 8 + kThreads - 1) / kThreads;  // 16-byte pieces of a tile per lane
-  __shared__ __align__(16) _Float16 kt[kAttnTile * kAttnKPitch];
-  __shared__ __align__(16) _Float16 vt[kDimH * kAttnVPitch];
+  struct __align__(16) Tile {
+    _Float16 k[kAttnTile * kAttnKPitch];
+    _Float16 v[kDimH * kAttnVPitch];
+  };
+  __shared__ Tile tiles[H];
+  static_assert(H == 1 || (H == 2 && sizeof(tiles) >= G * 64 * 16 * sizeof(float)), "the parts meet in the tiles' memory");
   const uint32_t kvh = blockIdx.x, row0 = blockIdx.y * kAttnTile;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t part = H == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kThreads));
+  const uint32_t tid = threadIdx.x - part * kThreads, lane = tid & 63u, wave = tid >> 6;
+  _Float16 *kt = tiles[part].k, *vt = tiles[part].v;
   const uint32_t groups = n_heads / n_kv;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
   const bool has_head = wave < groups;
@@ -429,7 +444,7 @@ __global__ __launch_bounds__(G * 64) void attn_rows_mfma_kernel(const __half* __
   const uint32_t qpos = pos0 + my_row;
   const uint32_t last_pos = pos0 + n_rows - 1u;              // last cached position
   const uint32_t t_end = pos0 + min(row0 + kAttnTile - 1u, n_rows - 1u);
-  const uint32_t n_tiles = t_end / kAttnTile + 1u;
+  const uint32_t n_tiles = t_end / kAttnTile + 1u;           // a part takes every H-th; one past the last is masked whole
   const size_t base = (size_t)kvh * max_pos;
   constexpr uint32_t kvgroups = kDimH / kKvGroup;
 
@@ -502,12 +517,12 @@ __global__ __launch_bounds__(G * 64) void attn_rows_mfma_kernel(const __half* __
     }
   };
 
-  request(0);
-  for (uint32_t tile = 0; tile < n_tiles; ++tile) {
+  request(part);
+  for (uint32_t tile = part; tile < n_tiles + part; tile += H) {  // as many turns for every part
     __syncthreads();  // the previous tile has been read by every wavefront
     deposit();
     __syncthreads();
-    if (tile + 1 < n_tiles) request(tile + 1);
+    if (tile + H < n_tiles + part) request(tile + H);
     // S^T = K Q^T
     f16v sacc;
 #pragma unroll
@@ -554,6 +569,36 @@ __global__ __launch_bounds__(G * 64) void attn_rows_mfma_kernel(const __half* __
       }
     }
   }
+  if constexpr (H == 2) {  // the second part's sums join the first's, a quarter of the dims at a time
+    float* meet = reinterpret_cast<float*>(tiles) + wave * 1024u + lane;
+    __syncthreads();
+    if (part) {
+      meet[0] = m_run;
+      meet[64] = l_run;
+    }
+    __syncthreads();
+    float w0 = 1.f, w1 = 0.f;
+    if (!part) {
+      const float m1 = meet[0], l1 = meet[64], m = fmaxf(m_run, m1);  // the first part has seen position 0
+      w0 = __expf(m_run - m);
+      w1 = __expf(m1 - m);
+      l_run = fmaf(l_run, w0, l1 * w1);
+    }
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      __syncthreads();
+      if (part) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) meet[j * 64] = o[dt][j];
+      }
+      __syncthreads();
+      if (!part) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) o[dt][j] = fmaf(o[dt][j], w0, meet[j * 64] * w1);
+      }
+    }
+    if (part) return;
+  }
   // o[dt][j] = O[q = l32][dim 32 dt + 8 (j / 4) + 4 h + j % 4]
   if (has_head && row0 + l32 < n_rows) {
     const float inv = 1.0f / l_run;
@@ -578,17 +623,23 @@ __global__ __launch_bounds__(G * 64) void attn_rows_mfma_kernel(const __half* __
 // (and, for the int8 cache, rebuilt) once per group.  The range is walked once:
 // sixteen position classes (four per wavefront, 16 lanes x 8 dims each) keep a
 // running maximum, a sum of exponentials and a weighted V sum per query head,
-// with the K and V rows of four positions requested together; the classes meet
-// in LDS and the workgroup leaves an unnormalised partial per query head.  The
-// workgroup that arrives last at the kv head's counter merges the partials in
-// split order and rounds the context once.  Scores, softmax and sums stay in
+// with the K and V rows of four positions requested together; a wavefront's
+// four classes meet by lane moves, the wavefronts in LDS, and the workgroup
+// leaves an unnormalised partial per query head.  The workgroup that arrives
+// last at the kv head's counter merges the partials in split order and rounds
+// the context once.  At the lengths of a chat (one batch of rows per class) a
+// launch is a chain of round trips: operands and rows, partials to memory, the
+// counter, partials from memory.  So all operands of the new position's heads
+// are requested in front of the rows, and partials are stored and loaded at
+// device scope (past the XCDs' own L2s) instead of between fences, which write
+// back and empty an L2.  Scores, softmax and sums stay in
 // f32.  head_dim <= 128, a multiple of 8; G >= query heads per kv head sizes
 // the register arrays.
 template <bool Q8, int G>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, const __half* __restrict__ kcache,
                                                                    const __half* __restrict__ vcache, KvQ8 q8,
                                                                    __half* __restrict__ ctx,
-                                                                   float* __restrict__ part, uint32_t* __restrict__ counters,
+                                                                   float* part, uint32_t* __restrict__ counters,
                                                                    uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
                                                                    uint32_t T, uint32_t max_pos, float scale, uint32_t n_splits,
                                                                    uint32_t merge_inline) {
@@ -602,7 +653,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
   const uint32_t chunk = (T + n_splits - 1) / n_splits;
   const uint32_t j0 = min(T, split * chunk), j1 = min(T, j0 + chunk), nj = j1 - j0;
   float* qs = att_smem;                         // [groups][head_dim]
-  float* cls = qs + groups * head_dim;          // [16 classes][groups][head_dim + 2]: running max, sum, weighted V sums
+  float* cls = qs + groups * head_dim;          // the wavefronts' results
   const __half* K = kcache + (size_t)kvh * max_pos * head_dim;
   const __half* V = vcache + (size_t)kvh * max_pos * head_dim;
   const uint32_t kvgroups = head_dim / kKvGroup;
@@ -648,9 +699,31 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
       }
     }
   };
+  // head_dim = 128: the operands of the wavefront's query heads and of the new k and v, in front of the rows
+  constexpr int kHeads = (G + kAttnWaves - 1) / kAttnWaves;  // query heads of a wavefront
+  const bool d128 = head_dim == 128u;
+  // (of another width: what these read is valid, and not used)
+  const uint32_t lane_a = d128 ? lane : 0u, lane_b = d128 ? lane + 64u : 0u, angle_at = d128 ? pos * 64u + lane : 0u;
+  const RopeAngle angle{nw.cos_t[angle_at], nw.sin_t[angle_at]};
+  HeadOperands qop[kHeads];
+#pragma unroll
+  for (int i = 0; i < kHeads; ++i)
+    qop[i] = head_operands_128(nw.q_raw + (size_t)(kvh * groups + min(wave + (uint32_t)i * kAttnWaves, groups - 1u)) * head_dim, nw.qn, lane_a, lane_b);
+  const HeadOperands kop = head_operands_128(nw.k_raw + (size_t)kvh * head_dim, nw.kn, lane_a, lane_b);
+  const uint16_t v1 = reinterpret_cast<const uint16_t*>(nw.v_raw)[(size_t)kvh * head_dim + lane_a], v2 = reinterpret_cast<const uint16_t*>(nw.v_raw)[(size_t)kvh * head_dim + lane_b];
   request(c);
   // the query heads of this kv head: norm, rotate, scale
-  for (uint32_t g = wave; g < groups; g += kAttnWaves) {
+  if (d128) {
+#pragma unroll
+    for (int i = 0; i < kHeads; ++i) {
+      const uint32_t g = wave + (uint32_t)i * kAttnWaves;
+      if (g < groups) {
+        const float2 r = norm_rope_128(qop[i], angle, nw.eps);
+        qs[g * 128u + lane] = r.x * scale;
+        qs[g * 128u + 64u + lane] = r.y * scale;
+      }
+    }
+  } else for (uint32_t g = wave; g < groups; g += kAttnWaves) {
     norm_rope_wave(nw.q_raw + (size_t)(kvh * groups + g) * head_dim, nw.qn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps,
                    stage[wave], lane);
     for (uint32_t i = lane; i < head_dim; i += 64) qs[g * head_dim + i] = stage[wave][i] * scale;
@@ -660,7 +733,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
   // cache for later positions, and to LDS, in the form the cache gives back,
   // for this one (nothing else reads that cache row during this launch).
   if (has_new && wave == 0) {
-    norm_rope_wave(nw.k_raw + (size_t)kvh * head_dim, nw.kn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage[0], lane);
+    if (d128) {
+      const float2 r = norm_rope_128(kop, angle, nw.eps);
+      stage[0][lane] = r.x;
+      stage[0][lane + 64] = r.y;
+      wave_lds_sync();
+    } else {
+      norm_rope_wave(nw.k_raw + (size_t)kvh * head_dim, nw.kn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage[0], lane);
+    }
     const size_t row = (size_t)kvh * max_pos + pos;
     if constexpr (Q8) {
       for (uint32_t g = 0; g < kvgroups; ++g) {
@@ -684,7 +764,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
     const size_t row = (size_t)kvh * max_pos + pos;
     if constexpr (Q8) {
       for (uint32_t g = 0; g < kvgroups; ++g) {
-        const float x = __half2float(nw.v_raw[(size_t)kvh * head_dim + g * kKvGroup + lane]);
+        const float x = d128 ? __half2float(__ushort_as_half(g ? v2 : v1)) : __half2float(nw.v_raw[(size_t)kvh * head_dim + g * kKvGroup + lane]);
         __half sh, bh;
         const uint8_t code = kv_quantize_group(x, &sh, &bh);
         q8.vq[row * head_dim + g * kKvGroup + lane] = code;
@@ -696,7 +776,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
       }
     } else {
       for (uint32_t i = lane; i < head_dim; i += 64) {
-        const __half x = nw.v_raw[(size_t)kvh * head_dim + i];
+        const __half x = __ushort_as_half(d128 ? (i < 64u ? v1 : v2) : __half_as_ushort(nw.v_raw[(size_t)kvh * head_dim + i]));
         nw.vcache[row * head_dim + i] = x;
         vnew[i] = __half2float(x);
       }
@@ -758,125 +838,166 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
       }
     }
     if (jb + 16u * U < nj) request(jb + 16u * U);
+    // the batch's maximum first, so that its exponentials do not wait for each other
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (jb + 16u * u < nj) {
+    for (int g = 0; g < G; ++g) {
+      float mn = m[g];
 #pragma unroll
-        for (int g = 0; g < G; ++g)
-          if ((uint32_t)g < groups) {
-            const float d = sc[u][g];
-            const float mn = fmaxf(m[g], d);
-            const float e0 = __expf(m[g] - mn), p = __expf(d - mn);  // e0 = 0 on the first position (m = -inf)
-            l[g] = fmaf(l[g], e0, p);
-#pragma unroll
-            for (int t = 0; t < 8; ++t) acc[g][t] = fmaf(acc[g][t], e0, p * vfs[u][t]);
-            m[g] = mn;
-          }
+      for (int u = 0; u < U; ++u) {
+        sc[u][g] = jb + 16u * u < nj ? sc[u][g] : -INFINITY;
+        mn = fmaxf(mn, sc[u][g]);
       }
-  }
-  // the classes' results meet in LDS
+      const float e0 = __expf(m[g] - mn);  // 0 on the first batch (m = -inf)
+      float p[U];
+      l[g] *= e0;
 #pragma unroll
-  for (int g = 0; g < G; ++g)
-    if ((uint32_t)g < groups) {
-      float* dst = cls + ((size_t)c * groups + g) * stride;
+      for (int u = 0; u < U; ++u) {
+        p[u] = __expf(sc[u][g] - mn);
+        l[g] += p[u];
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        acc[g][t] *= e0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc[g][t] = fmaf(p[u], vfs[u][t], acc[g][t]);
+      }
+      m[g] = mn;
+    }
+  }
+  // A wavefront's four classes meet by lane moves; every sixteen lanes then hold the sums, and lanes 16 (g mod 4) on put
+  // head g's down.  (A class with no position: maximum -inf, weight 0.)
+  float* wmax = cls;                                       // [4 wavefronts][groups] running maximum,
+  float* wsum = wmax + kAttnWaves * groups;                // sum of exponentials,
+  float* wacc = qs + ((groups * head_dim + 2u * kAttnWaves * groups + 3u) & ~3u);  // [4][groups][head_dim] weighted V sums
+  // (Heads four at a time: a move across half the wavefront leaves each half two heads of both, one across a quarter
+  // each quarter its own head of all four.)
+  auto swap32 = [](float a, float b, auto op) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  };
+  auto swap16 = [](float a, float b, auto op) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  };
+  auto add = [](float a, float b) { return a + b; };
+  auto larger = [](float a, float b) { return fmaxf(a, b); };
+#pragma unroll
+  for (int g0 = 0; g0 < G; g0 += 4) {
+    float wgt[4], M = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      wgt[k] = 0.f;
+      if (g0 + k < G) {
+        const int g = g0 + k;
+        float mk = swap32(m[g], m[g], larger);
+        mk = swap16(mk, mk, larger);
+        wgt[k] = m[g] == -INFINITY ? 0.f : __expf(m[g] - mk);
+        M = pj == (uint32_t)k ? mk : M;
+      }
+    }
+    auto quarters = [&](auto value) {  // value(k): head k's; the lane's quarter's own, summed over the classes
+      const float lo = swap32(value(0), value(2), add), hi = swap32(value(1), value(3), add);
+      return swap16(lo, hi, add);
+    };
+    const float Lsum = quarters([&](int k) { return g0 + k < G ? l[g0 + k < G ? g0 + k : 0] * wgt[k] : 0.f; });
+    float s[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) s[t] = quarters([&](int k) { return g0 + k < G ? acc[g0 + k < G ? g0 + k : 0][t] * wgt[k] : 0.f; });
+    const uint32_t g = (uint32_t)g0 + pj;
+    if (g < groups) {
       if (sub == 0) {
-        dst[0] = m[g];
-        dst[1] = l[g];
+        wmax[wave * groups + g] = M;
+        wsum[wave * groups + g] = Lsum;
       }
       if (active) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) dst[2 + i0 + t] = acc[g][t];
+        float4* dst = reinterpret_cast<float4*>(wacc + ((size_t)wave * groups + g) * head_dim + i0);
+        dst[0] = make_float4(s[0], s[1], s[2], s[3]);
+        dst[1] = make_float4(s[4], s[5], s[6], s[7]);
       }
     }
-  __syncthreads();
-  // ---- this workgroup's partial: the sixteen classes merged in class order ----
-  // per query head: the maximum over the classes, then each class's weight, once, into its slot for the maximum
-  if (tid < groups) {
-    float M = -INFINITY;
-#pragma unroll
-    for (int cc = 0; cc < 16; ++cc) M = fmaxf(M, cls[((size_t)cc * groups + tid) * stride]);
-    float Lsum = 0.f;
-#pragma unroll
-    for (int cc = 0; cc < 16; ++cc) {
-      float* src = cls + ((size_t)cc * groups + tid) * stride;
-      const float wgt = src[0] == -INFINITY ? 0.f : __expf(src[0] - M);  // a class with no position
-      Lsum = fmaf(src[1], wgt, Lsum);
-      src[0] = wgt;
-    }
-    float* dst = part + ((size_t)(kvh * groups + tid) * n_splits + split) * stride;
-    dst[0] = M;  // -inf for an empty range
-    dst[1] = Lsum;
   }
   __syncthreads();
+  // ---- this workgroup's partial: the wavefronts merged in order ----
+  auto put = [&](float* at, float v) {  // read by another workgroup of this launch, or by attn_merge_kernel
+    __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   for (uint32_t o = tid; o < groups * head_dim; o += kAttnThreads) {
     const uint32_t g = o / head_dim, i = o - g * head_dim;
-    float A = 0.f;
+    float w[kAttnWaves], M = -INFINITY, L = 0.f, A = 0.f;
 #pragma unroll
-    for (int cc = 0; cc < 16; ++cc) {
-      const float* src = cls + ((size_t)cc * groups + g) * stride;
-      A = fmaf(src[2 + i], src[0], A);
+    for (int k = 0; k < kAttnWaves; ++k) {
+      w[k] = wmax[k * groups + g];
+      M = fmaxf(M, w[k]);
     }
-    part[((size_t)(kvh * groups + g) * n_splits + split) * stride + 2 + i] = A;
+#pragma unroll
+    for (int k = 0; k < kAttnWaves; ++k) {
+      w[k] = w[k] == -INFINITY ? 0.f : __expf(w[k] - M);
+      L = fmaf(wsum[k * groups + g], w[k], L);
+      A = fmaf(wacc[((size_t)k * groups + g) * head_dim + i], w[k], A);
+    }
+    float* dst = part + ((size_t)(kvh * groups + g) * n_splits + split) * stride;
+    if (i == 0) {
+      put(dst, M);  // -inf for an empty range
+      put(dst + 1, L);
+    }
+    put(dst + 2 + i, A);
   }
   if (!merge_inline) return;  // attn_merge_kernel finishes (long caches: many partials, merged chip-wide)
-  // publish, and let the last workgroup of this kv head merge (one lane's
-  // device-scope release / acquire stands for the workgroup, ordered by the barriers)
+  // Let the last workgroup of this kv head merge: a lane's partials have arrived in memory before it reaches the barrier,
+  // and only then is the workgroup counted.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (tid == 0) arrived = __hip_atomic_fetch_add(&counters[kvh], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) arrived = __hip_atomic_fetch_add(&counters[kvh], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   if (arrived != n_splits - 1) return;
-  // Merge (at most kAttnInlineSplits ranges).  The partials come from the other XCDs' writes,
-  // i.e. from memory, so latency is what matters: the (max, sum) pairs and the first partial
-  // vectors are requested together, every load unconditional (a lane past the end re-reads a
-  // valid element and gives it weight zero).  Each lane then forms its head's weights from
-  // the pairs in LDS for itself; sums run in range order.
-  float* mx = att_smem;                // [groups][n_splits] running maxima (the staging of this launch is dead)
-  float* sm = mx + groups * n_splits;  // [groups][n_splits] sums of exponentials
-  const uint32_t n_pairs = groups * n_splits, n_out = groups * head_dim;
-  auto fetch = [&](uint32_t o, float (&v)[kAttnInlineSplits]) {
-    o = min(o, n_out - 1u);
-    const uint32_t g = o / head_dim, i = o - g * head_dim;
-    const float* src = part + (size_t)(kvh * groups + g) * n_splits * stride + 2 + i;
-#pragma unroll
-    for (int u = 0; u < kAttnInlineSplits; ++u) v[u] = src[(size_t)min((uint32_t)u, n_splits - 1u) * stride];
+  // Merge (at most kAttnInlineSplits = 16 ranges): sixteen lanes hold the ranges of a head, form its weights and leave
+  // them in LDS; a lane then sums two neighbouring elements.  The first elements are requested together with the
+  // (max, sum) pairs, every load unconditional (past the end: a valid one again, of weight zero).  Sums run in range order.
+  float* wts = att_smem;                            // [groups][16] weights (the staging of this launch is dead)
+  float* tot = wts + groups * kAttnInlineSplits;    // [groups] sums of exponentials
+  static_assert(kAttnInlineSplits == 16 && kAttnMaxGroup <= kAttnWaves * 4, "a range per lane of a row, a head per row");
+  const uint32_t n_pairs = groups * (head_dim >> 1);
+  auto load2 = [&](uint32_t at) {
+    return __hip_atomic_load(reinterpret_cast<uint64_t*>(part + at), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
-  float v[kAttnInlineSplits], vn[kAttnInlineSplits];
-  float2 pair[(kAttnMaxGroup * kAttnInlineSplits + kAttnThreads - 1) / kAttnThreads];
+  const uint32_t hg = wave * 4u + pj;
+  const uint64_t pair = load2(((kvh * groups + min(hg, groups - 1u)) * n_splits + min(sub, n_splits - 1u)) * stride);
+  uint64_t v[kAttnInlineSplits];
+  auto fetch = [&](uint32_t o) {
+    o = min(o, n_pairs - 1u);
+    const uint32_t g = o / (head_dim >> 1), i = (o - g * (head_dim >> 1)) * 2u;
+    const uint32_t at = (kvh * groups + g) * n_splits * stride + 2u + i;
 #pragma unroll
-  for (uint32_t r = 0; r < sizeof(pair) / sizeof(pair[0]); ++r) {
-    const uint32_t o = min(tid + r * kAttnThreads, n_pairs - 1u);
-    const uint32_t g = o / n_splits, sp = o - g * n_splits;
-    pair[r] = *reinterpret_cast<const float2*>(part + ((size_t)(kvh * groups + g) * n_splits + sp) * stride);
-  }
-  fetch(tid, v);
+    for (int u = 0; u < kAttnInlineSplits; ++u) v[u] = load2(at + min((uint32_t)u, n_splits - 1u) * stride);
+  };
+  fetch(tid);
+  {
+    const float mx = sub < n_splits ? __uint_as_float((uint32_t)pair) : -INFINITY;
+    float M = mx;
 #pragma unroll
-  for (uint32_t r = 0; r < sizeof(pair) / sizeof(pair[0]); ++r) {
-    const uint32_t o = tid + r * kAttnThreads;
-    if (o < n_pairs) {
-      mx[o] = pair[r].x;
-      sm[o] = pair[r].y;
+    for (int k = 1; k < 16; k <<= 1) M = fmaxf(M, __shfl_xor(M, k));
+    const float w = mx == -INFINITY ? 0.f : __expf(mx - M);  // 0 for an empty range too
+    float L = w * (sub < n_splits ? __uint_as_float((uint32_t)(pair >> 32)) : 0.f);
+    L = row16_sum(L);
+    if (hg < groups) {
+      wts[hg * kAttnInlineSplits + sub] = w;
+      if (sub == 0) tot[hg] = L;
     }
   }
   __syncthreads();
-  for (uint32_t o = tid; o < n_out; o += kAttnThreads) {
-    fetch(o + kAttnThreads, vn);
-    const uint32_t g = o / head_dim, i = o - g * head_dim;
-    float w[kAttnInlineSplits], M = -INFINITY;
+#pragma unroll 1
+  for (uint32_t o = tid; o < n_pairs; o += kAttnThreads) {
+    const uint32_t g = o / (head_dim >> 1), i = (o - g * (head_dim >> 1)) * 2u;
+    float A = 0.f, B = 0.f;
 #pragma unroll
     for (int u = 0; u < kAttnInlineSplits; ++u) {
-      w[u] = mx[g * n_splits + min((uint32_t)u, n_splits - 1u)];
-      M = fmaxf(M, w[u]);
+      const float w = wts[g * kAttnInlineSplits + u];
+      A = fmaf(__uint_as_float((uint32_t)v[u]), w, A);
+      B = fmaf(__uint_as_float((uint32_t)(v[u] >> 32)), w, B);
     }
-    float L = 0.f, A = 0.f;
-#pragma unroll
-    for (int u = 0; u < kAttnInlineSplits; ++u) {
-      w[u] = (uint32_t)u < n_splits ? __expf(w[u] - M) : 0.f;  // 0 for an empty range too
-      L = fmaf(sm[g * n_splits + min((uint32_t)u, n_splits - 1u)], w[u], L);
-      A = fmaf(v[u], w[u], A);
-    }
-    ctx[(size_t)(kvh * groups + g) * head_dim + i] = __float2half_rn(A / L);
-#pragma unroll
-    for (int u = 0; u < kAttnInlineSplits; ++u) v[u] = vn[u];
+    const float L = tot[g];
+    reinterpret_cast<__half2*>(ctx + (size_t)(kvh * groups + g) * head_dim + i)[0] = __floats2half2_rn(A / L, B / L);
+    if (o + kAttnThreads < n_pairs) fetch(o + kAttnThreads);
   }
   if (tid == 0) counters[kvh] = 0;  // ready for the next launch
 }

@@ -224,15 +224,15 @@ __device__ __forceinline__ float lane_butterfly(float v, float sgn) {
     const auto p = __builtin_amdgcn_permlane32_swap((uint32_t)i, (uint32_t)i, false, false);
     return fmaf(sgn, __uint_as_float(p[1]), __uint_as_float(p[0]));
   } else {
-    int o;
-    if constexpr (L == 1) o = __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, false);
-    if constexpr (L == 2) o = __builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, false);
+    int o = i;
+    if constexpr (L == 1) o = __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, true);
+    if constexpr (L == 2) o = __builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, true);
     if constexpr (L == 4) {  // lane ^ 7, then lane ^ 3
-      o = __builtin_amdgcn_update_dpp(0, i, 0x141, 0xF, 0xF, false);
-      o = __builtin_amdgcn_update_dpp(0, o, 0x1B, 0xF, 0xF, false);
+      o = __builtin_amdgcn_update_dpp(0, i, 0x141, 0xF, 0xF, true);
+      o = __builtin_amdgcn_update_dpp(0, o, 0x1B, 0xF, 0xF, true);
     }
-    if constexpr (L == 8) o = __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, false);
-    return fmaf(sgn, v, __uint_as_float((uint32_t)o));
+    if constexpr (L == 8) o = __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, true);
+    return __uint_as_float((uint32_t)o) + sgn * v;  // (exact products: the same as one rounding)
   }
 }
 template <int L>
@@ -274,6 +274,7 @@ __device__ __forceinline__ void rotate_octets_to(float* v, float (&r)[8], uint32
 // log2 R levels from 2^lg on, by all lanes: butterflies over R values 2^lg apart.
 template <uint32_t R>
 __device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t lg, float factor) {
+#pragma unroll 1
   for (uint32_t p = threadIdx.x; p < n / R; p += 1024u) {
     float* at = v + (p >> lg) * (R << lg) + (p & ((1u << lg) - 1u));
     float r[R];
@@ -332,6 +333,7 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
   // steps of depth 2 (S padded with zeros to 32 x 32; lanes past a narrow m repeat its first column); it reads its columns
   // whole before it writes them, and no other wavefront touches them.
   const uint32_t steps = (k + 1u) >> 1;
+#pragma unroll 1
   for (uint32_t tile = wave; tile * 32u < m; tile += 16) {
     const uint32_t j = tile * 32u + l32;
     rot_acc_t acc;
@@ -1889,10 +1891,8 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   uint32_t n_splits = (T + 63) / 64;
   if (n_splits > (uint32_t)kAttnMaxSplits) n_splits = kAttnMaxSplits;
   const uint32_t groups_per_kv = d->n_heads / d->n_kv;
-  // the queries and the sixteen position classes' running results
-  size_t attn_lds = ((size_t)groups_per_kv * d->head_dim + (size_t)16 * groups_per_kv * (d->head_dim + 2)) * sizeof(float);
-  const size_t merge_lds = (size_t)groups_per_kv * 2 * n_splits * sizeof(float);  // the merge reuses the staging area
-  if (attn_lds < merge_lds) attn_lds = merge_lds;
+  // the queries and the wavefronts' running results
+  const size_t attn_lds = ((size_t)groups_per_kv * d->head_dim + (size_t)kAttnWaves * groups_per_kv * (d->head_dim + 2) + 4) * sizeof(float);
   const size_t group_layer = cache_layer / kKvGroup;
   // few partials: the last workgroup of a kv head merges them; many: a chip-wide merge kernel does
   const uint32_t merge_inline = n_splits <= (uint32_t)kAttnInlineSplits ? 1u : 0u;
@@ -2070,7 +2070,8 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(kernel, agrid, dim3(64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->head_dim, d->pos, d->max_pos, scale);
     };
     const uint32_t grp = d->n_heads / d->n_kv;
-    // 32 rows per workgroup on the matrix cores where the head width is the one that kernel is built for
+    // 32 rows per workgroup on the matrix cores where the head width is the one that kernel is built for, the cache walked
+    // by two sets of wavefronts (more than five heads to a set leave it too few registers for that)
     const bool on_mfma = d->head_dim == 128 && grp <= (uint32_t)kAttnMaxGroup;
     const dim3 mgrid(d->n_kv, (n + kAttnTile - 1) / kAttnTile);
     auto attend_mfma = [&](auto kernel, uint32_t waves) {
@@ -2080,10 +2081,10 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<true>, hgrid, dim3(64), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos);
       if (on_mfma) {
-        if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<true, 2>, 2);
-        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<true, 4>, 4);
-        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<true, 5>, 5);
-        else attend_mfma(attn_rows_mfma_kernel<true, kAttnMaxGroup>, kAttnMaxGroup);
+        if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<true, 2, 2>, 2 * 2);
+        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<true, 4, 2>, 2 * 4);
+        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<true, 5, 2>, 2 * 5);
+        else attend_mfma(attn_rows_mfma_kernel<true, kAttnMaxGroup, 1>, kAttnMaxGroup);
       } else if (grp <= 2) attend(attn_rows_kernel<true, 2>);
       else if (grp <= 4) attend(attn_rows_kernel<true, 4>);
       else if (grp <= 5) attend(attn_rows_kernel<true, 5>);
@@ -2092,10 +2093,10 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<false>, hgrid, dim3(64), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos);
       if (on_mfma) {
-        if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<false, 2>, 2);
-        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<false, 4>, 4);
-        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<false, 5>, 5);
-        else attend_mfma(attn_rows_mfma_kernel<false, kAttnMaxGroup>, kAttnMaxGroup);
+        if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<false, 2, 2>, 2 * 2);
+        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<false, 4, 2>, 2 * 4);
+        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<false, 5, 2>, 2 * 5);
+        else attend_mfma(attn_rows_mfma_kernel<false, kAttnMaxGroup, 1>, kAttnMaxGroup);
       } else if (grp <= 2) attend(attn_rows_kernel<false, 2>);
       else if (grp <= 4) attend(attn_rows_kernel<false, 4>);
       else if (grp <= 5) attend(attn_rows_kernel<false, 5>);
