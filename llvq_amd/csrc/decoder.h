@@ -33,10 +33,10 @@ __device__ __forceinline__ float block_sum_1024(float v, float* red) {
   return s;
 }
 
-// h[row] = embed[token[row]], row = blockIdx.y
-__global__ __launch_bounds__(256) void embed_kernel(const __half* __restrict__ table, const uint32_t* __restrict__ token,
+// h[row] = embed[token[row]], row = blockIdx.y (token null: the one token `value`)
+__global__ __launch_bounds__(256) void embed_kernel(const __half* __restrict__ table, const uint32_t* __restrict__ token, uint32_t value,
                                                     uint32_t vocab, uint32_t hidden, __half* __restrict__ h) {
-  const uint32_t t = min(token[blockIdx.y], vocab - 1u);
+  const uint32_t t = min(token ? token[blockIdx.y] : value, vocab - 1u);
   h += (size_t)blockIdx.y * hidden;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < hidden; i += gridDim.x * blockDim.x)
     h[i] = table[(size_t)t * hidden + i];
@@ -1110,9 +1110,9 @@ __device__ __forceinline__ float q8_weight(uint32_t q, float s, float b) {
 }
 
 // h = f16(embedding row of *token)   (emb_q8_gather)
-__global__ __launch_bounds__(256) void embed_q8_kernel(QuantRows e, const uint32_t* __restrict__ token, uint32_t vocab,
+__global__ __launch_bounds__(256) void embed_q8_kernel(QuantRows e, const uint32_t* __restrict__ token, uint32_t value, uint32_t vocab,
                                                        uint32_t hidden, __half* __restrict__ h) {
-  const uint32_t t = min(token[blockIdx.y], vocab - 1u);
+  const uint32_t t = min(token ? token[blockIdx.y] : value, vocab - 1u);
   h += (size_t)blockIdx.y * hidden;
   const uint32_t gpr = (hidden + kEmbedGroup - 1) / kEmbedGroup;
   for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < hidden; c += gridDim.x * blockDim.x) {
@@ -1195,7 +1195,5 @@ __global__ __launch_bounds__(1024) void argmax_final_kernel(const float* __restr
     if (history) history[slot] = si[0];
   }
 }
-
-__global__ void set_token_kernel(uint32_t* token, uint32_t value) { *token = value; }
 
 }  // namespace llvq
