@@ -181,7 +181,7 @@ struct ActivationIn {
   uint32_t prologue;   // kPrologue*
   // the basis of the matrices, when they are stored rotated and the launch rotates its own activation (see rotate_lds)
   const uint32_t* rot_signbits;
-  const float* rot_small;
+  const void* rot_fragments;  // [64] RotFragments
   float rot_inv;
   uint32_t rot_m, rot_k;
 };
@@ -201,29 +201,46 @@ __device__ __forceinline__ float half_hi(uint32_t w) { return __half2float(__ush
 // The rotation x' = (S (x) I_m)(I_k (x) H_m / sqrt m) D x of an activation of n = k m values, by a workgroup of 1024
 // lanes (llvq-quant/src/rotation.rs:97-105; f32 like the reference's device rotation, llvq-cuda/kernels/llvq_rot.cuh).
 //
-// Every workgroup of a batch-1 product rotates its own activation, so a rotation is a chain that a launch waits for.
-// With a value per lane and load, lane exchanges through LDS and a pass over LDS per level above 512 it took 12 us of
-// the 19.2 of a 2560 x 9728 product.  Here a lane holds eight neighbouring values from the load on (one 16-byte load and
-// a byte of signs, all of a wavefront's requested together) and does nine levels in registers: three inside the lane, six by
-// lane moves of the vector unit (19.2 -> 15.7 us).  The values meet LDS once, rotate_octets_to; the levels above 512 are one pass of
-// register butterflies and the k x k block one pass of f32 matrix-core steps, rotate_rest.
+// Every workgroup of a batch-1 product rotates its own activation, and with sixteen wavefronts on a CU an instruction of
+// each costs 7 ns: what bounds a rotation is their number.  (With a value per lane and load, lane exchanges through LDS and a
+// pass over LDS per level above 512 a 2560 x 9728 product took 19.2 us; it takes 12.7.)  So:
+//  * The five lowest levels are two matrix-core steps: what is rotated is binary16, the entries of H are 0 and +-1, so
+//    the products are exact and the sums f32, as butterflies would have them.  A wavefront takes 1024 values; a column of
+//    its 32 x 32 result is 32 neighbouring ones, requested by two lanes as two octets each (with their signs).
+//  * The next four are lane moves between columns, on the sixteen results a lane holds; the values meet LDS once.
+//  * The levels above 512 are passes over LDS, three levels to a pass, the k x k block is f32 matrix-core steps (rotate_rest).
+// A lane's parts of both matrices lie together in a table (RotFragments).
 // Where an octet spans groups (m < 8) the signed values are put into LDS instead and every level is a pass there.
 constexpr uint32_t kRotOctetM = 8;    // the narrowest m that takes the octets
-constexpr uint32_t kRotRun = 512;     // values of a wavefront's run
+constexpr uint32_t kRotRun = 512;     // values that the levels before LDS reach across
+constexpr uint32_t kRotTile = 1024;   // values of a wavefront
+typedef _Float16 rot_h8_t __attribute__((ext_vector_type(8)));
+typedef float rot_acc_t __attribute__((ext_vector_type(16)));
+struct RotFragments {   // of lane l: (l32, lh) = (l % 32, l / 32)
+  float s[kRotKMax / 2];  // S[l32][2 i + lh], zero past k
+  rot_h8_t h[2];          // H[l32][16 i + 8 lh + e], H the transform inside groups of min(m, 32)
+};
+static_assert(sizeof(RotFragments) == 96, "six 16-byte loads");
 __device__ __forceinline__ float flip_sign(float v, uint32_t bits, int j) {  // bit j of `bits` is the sign of D
   return __uint_as_float(__float_as_uint(v) ^ (((bits >> j) & 1u) << 31));
 }
+// Two binary16 values and bits 2 j and 2 j + 1 of their octet's signs.
+__device__ __forceinline__ uint32_t flip_signs(uint32_t pair, uint32_t bits, int j) {
+  return pair ^ (((bits << (15 - 2 * j)) | (bits << (30 - 2 * j))) & 0x80008000u);
+}
+// Where a lane's octet i of a tile lies.
+__device__ __forceinline__ uint32_t rot_octet_at(uint32_t tile, uint32_t i) {
+  const uint32_t lane = threadIdx.x & 63u;
+  return tile * kRotTile + (lane & 31u) * 32u + i * 16u + (lane >> 5) * 8u;
+}
 // Sum and difference with the lane L away: lower lanes get own + other, upper ones other - own (sgn = -1 there).
 template <int L>
-__device__ __forceinline__ float lane_butterfly(float v, float sgn) {
-  const int i = (int)__float_as_uint(v);
-  if constexpr (L == 16) {  // the swaps leave the lower and the upper lane's value in both
-    const auto p = __builtin_amdgcn_permlane16_swap((uint32_t)i, (uint32_t)i, false, false);
-    return fmaf(sgn, __uint_as_float(p[1]), __uint_as_float(p[0]));
-  } else if constexpr (L == 32) {
-    const auto p = __builtin_amdgcn_permlane32_swap((uint32_t)i, (uint32_t)i, false, false);
-    return fmaf(sgn, __uint_as_float(p[1]), __uint_as_float(p[0]));
-  } else {
+__device__ __forceinline__ void lane_level(rot_acc_t& v, uint32_t lane, uint32_t m) {
+  if (m < 64u * (uint32_t)L) return;
+  const float sgn = (lane & (uint32_t)L) ? -1.f : 1.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int i = (int)__float_as_uint(v[r]);
     int o = i;
     if constexpr (L == 1) o = __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, true);
     if constexpr (L == 2) o = __builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, true);
@@ -232,44 +249,32 @@ __device__ __forceinline__ float lane_butterfly(float v, float sgn) {
       o = __builtin_amdgcn_update_dpp(0, o, 0x1B, 0xF, 0xF, true);
     }
     if constexpr (L == 8) o = __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, true);
-    return __uint_as_float((uint32_t)o) + sgn * v;  // (exact products: the same as one rounding)
+    v[r] = __uint_as_float((uint32_t)o) + sgn * v[r];  // (exact product)
   }
 }
-template <int L>
-__device__ __forceinline__ void lane_level(float (&r)[8], uint32_t lane, uint32_t m) {
-  if (m >= 16u * (uint32_t)L) {
-    const float sgn = (lane & (uint32_t)L) ? -1.f : 1.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = lane_butterfly<L>(r[i], sgn);
-  }
-}
-// The levels below min(m, 512) of the signed values at `at` (lane-contiguous octets of a run), into LDS where at < n.
-__device__ __forceinline__ void rotate_octets_to(float* v, float (&r)[8], uint32_t at, uint32_t n, uint32_t m, uint32_t k, float inv) {
+// The levels below min(m, 512) of a tile whose signed octets a lane holds (zeros past n), into LDS.
+__device__ __forceinline__ void rotate_tile_to(float* v, const uint32_t (&x0)[4], const uint32_t (&x1)[4], const RotFragments& F, uint32_t tile,
+                                               uint32_t n, uint32_t m, uint32_t k, float inv) {
   const uint32_t lane = threadIdx.x & 63u;
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  rot_acc_t acc;
 #pragma unroll
-  for (int l = 1; l < 8; l <<= 1)
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (!(i & l)) {
-        const float u = r[i], w = r[i | l];
-        r[i] = u + w;
-        r[i | l] = u - w;
-      }
-  lane_level<1>(r, lane, m);
-  lane_level<2>(r, lane, m);
-  lane_level<4>(r, lane, m);
-  lane_level<8>(r, lane, m);
-  lane_level<16>(r, lane, m);
-  lane_level<32>(r, lane, m);
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F.h[0], __builtin_bit_cast(rot_h8_t, u4{x0[0], x0[1], x0[2], x0[3]}), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F.h[1], __builtin_bit_cast(rot_h8_t, u4{x1[0], x1[1], x1[2], x1[3]}), acc, 0, 0, 0);
+  // acc[r] is value 8 (r / 4) + 4 lh + r % 4 of column l32
+  lane_level<1>(acc, lane, m);
+  lane_level<2>(acc, lane, m);
+  lane_level<4>(acc, lane, m);
+  lane_level<8>(acc, lane, m);
   if (k == 1 && m <= kRotRun) {  // nothing follows but the factor
 #pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] *= inv;
+    for (int r = 0; r < 16; ++r) acc[r] *= inv;
   }
-  if (at < n) {
-    float4* dst = reinterpret_cast<float4*>(v + at);
-    dst[0] = make_float4(r[0], r[1], r[2], r[3]);
-    dst[1] = make_float4(r[4], r[5], r[6], r[7]);
-  }
+  const uint32_t at = tile * kRotTile + (lane & 31u) * 32u + (lane >> 5) * 4u;
+#pragma unroll
+  for (uint32_t q = 0; q < 4u; ++q)
+    if (at + 8u * q < n) *reinterpret_cast<float4*>(v + at + 8u * q) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
 }
 // log2 R levels from 2^lg on, by all lanes: butterflies over R values 2^lg apart.
 template <uint32_t R>
@@ -294,26 +299,10 @@ __device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t lg,
   }
 }
 
-// The part of S a lane multiplies with, S[l32][2 s + lh]: loaded before the levels, so that it is there when they are done.
-typedef float rot_acc_t __attribute__((ext_vector_type(16)));
-struct RotBlock { float s[kRotKMax / 2]; };
-__device__ __forceinline__ RotBlock load_rot_block(const float* __restrict__ small, uint32_t k) {
-  const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, lh = lane >> 5;
-  RotBlock b;
-#pragma unroll
-  for (uint32_t s = 0; s < kRotKMax / 2; ++s) {
-    const uint32_t t = 2u * s + lh;
-    const bool in = l32 < k && t < k;
-    const float e = small[in ? l32 * k + t : 0u];  // always a valid address, so the loads go out together
-    b.s[s] = in ? e : 0.f;
-  }
-  return b;
-}
-
 // What is left once the levels below 512 are in LDS (every level, `put_levels`, where the octets were not taken): the values
 // are final after the caller's next barrier.  Called behind a barrier.
-__device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, uint32_t k, float inv, const float* __restrict__ small,
-                                            const RotBlock& S, bool put_levels) {
+__device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, uint32_t k, float inv,
+                                            const float (&S)[kRotKMax / 2], bool put_levels) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
   // three levels to a pass, what is over in the last
@@ -332,36 +321,39 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
   // S (k x k) . C (k x m), the 1 / sqrt m factor first: a wavefront takes 32 columns of C at a time as f32 matrix-core
   // steps of depth 2 (S padded with zeros to 32 x 32; lanes past a narrow m repeat its first column); it reads its columns
   // whole before it writes them, and no other wavefront touches them.
-  const uint32_t steps = (k + 1u) >> 1;
 #pragma unroll 1
   for (uint32_t tile = wave; tile * 32u < m; tile += 16) {
+    // (in each tile anew: what the steps compare and multiply with would otherwise be formed ahead of the loop and spilled)
+    asm volatile("" : "+s"(k), "+s"(m));
+    const uint32_t steps = (k + 1u) >> 1;  // k is odd: the last one has no row for the upper half
     const uint32_t j = tile * 32u + l32;
+    const float* col = v + (j < m ? j : 0u);
     rot_acc_t acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    uint32_t rows = k - lh;  // 2 s < rows: step s has a row for this half
-    asm volatile("" : "+v"(rows));  // (compared in each tile: kept across tiles, sixteen masks would crowd the scalar registers)
 #pragma unroll
     for (uint32_t s0 = 0; s0 < kRotKMax / 2; s0 += 8u) {  // half the steps at a time: the weights in flight leave registers for that
       if (s0 >= steps) break;
-      float c_frag[8];
+      float c[8];
+#pragma unroll
+      for (uint32_t i = 0; i < 8u; ++i) c[i] = col[min((2u * (s0 + i) + lh) * m, (k - 1u) * m)];  // always valid, so the reads go out together
 #pragma unroll
       for (uint32_t i = 0; i < 8u; ++i) {
-        const uint32_t t = 2u * (s0 + i);
-        const float x = v[(t < rows ? (t + lh) * m : 0u) + (j < m ? j : 0u)];  // always a valid address, so the reads go out together
-        c_frag[i] = t < rows ? x * inv : 0.f;
+        if (s0 + i >= steps) break;
+        float x = c[i] * inv;
+        if (s0 + i + 1u == steps) x = lh ? 0.f : x;
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(S[s0 + i], x, acc, 0, 0, 0);
       }
-#pragma unroll
-      for (uint32_t i = 0; i < 8u; ++i)
-        if (s0 + i < steps) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(S.s[s0 + i], c_frag[i], acc, 0, 0, 0);
     }
     // acc[r] is row 8 (r / 4) + 4 lh + r % 4 of column j
-    uint32_t left = j < m && k > 4u * lh ? k - 4u * lh : 0u;  // rows of the block from this half's first on
-    asm volatile("" : "+v"(left));
+    if (j < m) {
+      float* out = v + j + lh * 4u * m;
 #pragma unroll
-    for (uint32_t r = 0; r < 16; ++r) {
-      const uint32_t g = 8u * (r >> 2) + (r & 3u);
-      if (g < left) v[(g + 4u * lh) * m + j] = acc[r];
+      for (uint32_t r = 0; r < 16; ++r) {
+        const uint32_t g = 8u * (r >> 2) + (r & 3u);
+        if (g + 4u < k) out[g * m] = acc[r];
+        else if (g < k && !lh) out[g * m] = acc[r];
+      }
     }
   }
 }
@@ -402,7 +394,7 @@ struct RotArgs {
   const __half* x;        // [rows, n]
   void* out;              // [rows, n] f32 or f16
   const uint32_t* signbits;
-  const float* small;     // k x k
+  const void* fragments;  // [64] RotFragments
   uint32_t n, m, k;
   float inv;
 };
@@ -418,36 +410,30 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
   extern __shared__ __align__(16) float rot_s[];
   const uint32_t tid = threadIdx.x, n = a.n, m = a.m, k = a.k;
   const __half* x = a.x + (size_t)blockIdx.x * n;
-  const RotBlock S = load_rot_block(a.small, k);
+  const RotFragments F = reinterpret_cast<const RotFragments*>(a.fragments)[tid & 63u];
   if (m >= kRotOctetM) {
     const uint8_t* signs = reinterpret_cast<const uint8_t*>(a.signbits);
-    constexpr int kRuns = 2;  // of a wavefront at a time
-    for (uint32_t at0 = (tid >> 6) * kRotRun; at0 < n; at0 += kRuns * 16u * kRotRun) {
-      HalfOctet o[kRuns];
-      uint32_t sg[kRuns];
+#pragma unroll 1
+    for (uint32_t tile = tid >> 6; tile * kRotTile < n; tile += 16u) {
+      HalfOctet o[2];
+      uint32_t sg[2];
 #pragma unroll
-      for (int p = 0; p < kRuns; ++p) {
-        const uint32_t at = at0 + (uint32_t)p * 16u * kRotRun + (tid & 63u) * 8u, from = at < n ? at : 0u;
-        o[p] = *reinterpret_cast<const HalfOctet*>(x + from);
-        sg[p] = signs[from >> 3];
+      for (uint32_t i = 0; i < 2u; ++i) {
+        const uint32_t at = rot_octet_at(tile, i), from = at < n ? at : 0u;
+        o[i] = *reinterpret_cast<const HalfOctet*>(x + from);
+        sg[i] = signs[from >> 3];
       }
 #pragma unroll
-      for (int p = 0; p < kRuns; ++p) {
-        const uint32_t at = at0 + (uint32_t)p * 16u * kRotRun + (tid & 63u) * 8u;
-        float r[8];
+      for (uint32_t i = 0; i < 2u; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          r[2 * j] = flip_sign(half_lo(o[p].w[j]), sg[p], 2 * j);
-          r[2 * j + 1] = flip_sign(half_hi(o[p].w[j]), sg[p], 2 * j + 1);
-        }
-        rotate_octets_to(rot_s, r, at, n, m, k, a.inv);
-      }
+        for (int j = 0; j < 4; ++j) o[i].w[j] = rot_octet_at(tile, i) < n ? flip_signs(o[i].w[j], sg[i], j) : 0u;
+      rotate_tile_to(rot_s, o[0].w, o[1].w, F, tile, n, m, k, a.inv);
     }
   } else {
     for (uint32_t i = tid; i < n; i += 1024) rot_s[i] = flip_sign(__half2float(x[i]), a.signbits[i >> 5] >> (i & 31u), 0);
   }
   __syncthreads();
-  rotate_rest(rot_s, n, m, k, a.inv, a.small, S, m < kRotOctetM);
+  rotate_rest(rot_s, n, m, k, a.inv, F.s, m < kRotOctetM);
   __syncthreads();
   OutT* out = reinterpret_cast<OutT*>(a.out) + (size_t)blockIdx.x * n;
   if constexpr (std::is_same<OutT, __half>::value) {
@@ -492,7 +478,7 @@ struct llvq_rt {
     uint64_t seed = 0;
     float inv = 1.f;
     uint32_t* signbits = nullptr;
-    float* small = nullptr;
+    void* fragments = nullptr;  // [64] RotFragments
   };
   std::vector<DevRotation*> rotations;
   float* rot_scratch = nullptr;   // one rotated activation, f32
@@ -668,7 +654,7 @@ void llvq_hip_runtime_destroy(llvq_rt* rt) {
   (void)hipFree(rt->upload_buf);
   for (auto* r : rt->rotations) {
     (void)hipFree(r->signbits);
-    (void)hipFree(r->small);
+    (void)hipFree(r->fragments);
     delete r;
   }
   delete rt;
@@ -694,8 +680,23 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
   r->n = t.n; r->m = t.m; r->k = t.k; r->seed = seed; r->inv = t.inv;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&r->signbits), t.signbits.size() * 4);
   if (e == hipSuccess) e = hipMemcpy(r->signbits, t.signbits.data(), t.signbits.size() * 4, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&r->small), t.small.size() * 4);
-  if (e == hipSuccess) e = hipMemcpy(r->small, t.small.data(), t.small.size() * 4, hipMemcpyHostToDevice);
+  std::vector<RotFragments> frag(64);
+  const uint32_t inside = std::min(t.m, 32u) - 1u;  // the bits of a column that the transform mixes
+  for (uint32_t l = 0; l < 64u; ++l) {
+    const uint32_t row = l & 31u, lh = l >> 5;
+    for (uint32_t i = 0; i < kRotKMax / 2; ++i) {
+      const uint32_t c = 2u * i + lh;
+      frag[l].s[i] = row < t.k && c < t.k ? t.small[(size_t)row * t.k + c] : 0.f;
+    }
+    for (uint32_t i = 0; i < 2u; ++i)
+      for (uint32_t e8 = 0; e8 < 8u; ++e8) {
+        const uint32_t c = 16u * i + 8u * lh + e8;
+        const bool same = ((row ^ c) & ~inside) == 0;
+        frag[l].h[i][e8] = (_Float16)(!same ? 0.f : __builtin_popcount(row & c & inside) & 1 ? -1.f : 1.f);
+      }
+  }
+  if (e == hipSuccess) e = hipMalloc(&r->fragments, frag.size() * sizeof(RotFragments));
+  if (e == hipSuccess) e = hipMemcpy(r->fragments, frag.data(), frag.size() * sizeof(RotFragments), hipMemcpyHostToDevice);
   if (e == hipSuccess && n > rt->rot_scratch_elems) {
     (void)hipFree(rt->rot_scratch);
     rt->rot_scratch = nullptr;
@@ -705,7 +706,7 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
   }
   if (e != hipSuccess) {
     (void)hipFree(r->signbits);
-    (void)hipFree(r->small);
+    (void)hipFree(r->fragments);
     delete r;
     return hip_fail(e, "rotation tables");
   }
@@ -991,7 +992,7 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   }
   if (rot) {
     a.in.rot_signbits = rot->signbits;
-    a.in.rot_small = rot->small;
+    a.in.rot_fragments = rot->fragments;
     a.in.rot_inv = rot->inv;
     a.in.rot_m = rot->m;
     a.in.rot_k = rot->k;
@@ -1025,7 +1026,7 @@ static int launch_rotate(llvq_rt* rt, const llvq_rt::DevRotation* rot, const voi
   a.x = reinterpret_cast<const __half*>(x_f16);
   a.out = out;
   a.signbits = rot->signbits;
-  a.small = rot->small;
+  a.fragments = rot->fragments;
   a.n = rot->n;
   a.m = rot->m;
   a.k = rot->k;

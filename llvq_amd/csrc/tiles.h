@@ -295,7 +295,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
     if (in.x_f32) {
       request();
     } else {
-      const RotBlock S = load_rot_block(in.rot_small, in.rot_k);
+      const RotFragments F = reinterpret_cast<const RotFragments*>(in.rot_fragments)[lane];
       const bool norm = in.prologue == kPrologueAddRmsNorm, silu = in.prologue == kPrologueSiluMul;
       auto norm_scale = [&](float ss) {
         ss = wave_sum(ss);
@@ -306,78 +306,67 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
         return 1.0f / sqrtf(total / (float)d_in + in.eps);
       };
       if (in.rot_m >= kRotOctetM) {
-        // every operand of the wavefront's runs is requested before the first is used; one that is not there reads x
-        constexpr int kRuns = PMAX > 2 ? 3 : 2;  // of 16: rows past 512 blocks, or not
+        // Every operand of a wavefront's tile is requested before the first is used; one that is not there reads x.
+        // (Rows past sixteen tiles: a second turn.  Those have no norm in front: a decoder's hidden size ends at 8192.)
         const __half* second = in.x2 ? in.x2 : in.x;
         const __half* third = norm ? in.norm_w : in.x;
         const uint8_t* signs = reinterpret_cast<const uint8_t*>(in.rot_signbits);
-        HalfOctet a[kRuns], b[kRuns], g[kRuns];
-        uint32_t sg[kRuns];
-        auto octet_at = [&](int p) { return ((uint32_t)p * 16u + wave) * kRotRun + lane * 8u; };
+        HalfOctet a[2], b[2], g[2];
+        uint32_t sg[2];
+        auto load_tile = [&](uint32_t tile) {
 #pragma unroll
-        for (int p = 0; p < kRuns; ++p) {
-          const uint32_t from = octet_at(p) < d_in ? octet_at(p) : 0u;
-          a[p] = *reinterpret_cast<const HalfOctet*>(in.x + from);
-          b[p] = *reinterpret_cast<const HalfOctet*>(second + from);
-          g[p] = *reinterpret_cast<const HalfOctet*>(third + from);
-          sg[p] = signs[from >> 3];
-        }
-        if constexpr (kRuns == 2) request();
+          for (uint32_t i = 0; i < 2u; ++i) {
+            const uint32_t from = rot_octet_at(tile, i) < d_in ? rot_octet_at(tile, i) : 0u;
+            a[i] = *reinterpret_cast<const HalfOctet*>(in.x + from);
+            b[i] = *reinterpret_cast<const HalfOctet*>(second + from);
+            g[i] = *reinterpret_cast<const HalfOctet*>(third + from);
+            sg[i] = signs[from >> 3];
+          }
+        };
+        auto pack = [](float lo, float hi) { return (uint32_t)__half_as_ushort(__float2half_rn(lo)) | (uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16; };
+        load_tile(wave);
+        if constexpr (PMAX <= 2) request();
         __builtin_amdgcn_sched_barrier(0);
         float inv = 0.f;
         if (norm) {
           float ss = 0.f;
 #pragma unroll
-          for (int p = 0; p < kRuns; ++p) {
-            if (octet_at(p) >= d_in) continue;
+          for (uint32_t i = 0; i < 2u; ++i) {
+            if (rot_octet_at(wave, i) >= d_in) continue;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              float lo = half_lo(a[p].w[j]), hi = half_hi(a[p].w[j]);
+              float lo = half_lo(a[i].w[j]), hi = half_hi(a[i].w[j]);
               if (in.x2) {
-                lo = round_half(lo + half_lo(b[p].w[j]));
-                hi = round_half(hi + half_hi(b[p].w[j]));
+                lo = round_half(lo + half_lo(b[i].w[j]));
+                hi = round_half(hi + half_hi(b[i].w[j]));
               }
-              a[p].w[j] = (uint32_t)__half_as_ushort(__float2half_rn(lo)) | (uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16;
+              a[i].w[j] = pack(lo, hi);
               ss = fmaf(lo, lo, fmaf(hi, hi, ss));
             }
-            if (in.resid_out && store_resid) *reinterpret_cast<HalfOctet*>(in.resid_out + octet_at(p)) = a[p];
+            if (in.resid_out && store_resid) *reinterpret_cast<HalfOctet*>(in.resid_out + rot_octet_at(wave, i)) = a[i];
           }
           inv = norm_scale(ss);
         }
-        // (one copy of the code for all runs, whose operands move up)
 #pragma unroll 1
-        for (uint32_t c = wave; c * kRotRun < d_in; c += 16u) {
-          float v[8];
+        for (uint32_t tile = wave; tile * kRotTile < d_in; tile += 16u) {
+          if (tile != wave) load_tile(tile);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            v[2 * j] = half_lo(a[0].w[j]);
-            v[2 * j + 1] = half_hi(a[0].w[j]);
-          }
-          if (silu) {
+          for (uint32_t i = 0; i < 2u; ++i) {
+            if (silu) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              v[2 * j] = silu_mul(half_lo(b[0].w[j]), v[2 * j]);
-              v[2 * j + 1] = silu_mul(half_hi(b[0].w[j]), v[2 * j + 1]);
+              for (int j = 0; j < 4; ++j)
+                a[i].w[j] = pack(silu_mul(half_lo(b[i].w[j]), half_lo(a[i].w[j])), silu_mul(half_hi(b[i].w[j]), half_hi(a[i].w[j])));
+            } else if (norm) {
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                a[i].w[j] = pack(half_lo(a[i].w[j]) * inv * half_lo(g[i].w[j]), half_hi(a[i].w[j]) * inv * half_hi(g[i].w[j]));
             }
-          } else if (norm) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              v[2 * j] = round_half(v[2 * j] * inv * half_lo(g[0].w[j]));
-              v[2 * j + 1] = round_half(v[2 * j + 1] * inv * half_hi(g[0].w[j]));
-            }
+            for (int j = 0; j < 4; ++j) a[i].w[j] = rot_octet_at(tile, i) < d_in ? flip_signs(a[i].w[j], sg[i], j) : 0u;
           }
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = flip_sign(v[j], sg[0], j);
-#pragma unroll
-          for (int p = 0; p + 1 < kRuns; ++p) {
-            a[p] = a[p + 1];
-            b[p] = b[p + 1];
-            g[p] = g[p + 1];
-            sg[p] = sg[p + 1];
-          }
-          rotate_octets_to(xf, v, c * kRotRun + lane * 8u, d_in, in.rot_m, in.rot_k, in.rot_inv);
+          rotate_tile_to(xf, a[0].w, a[1].w, F, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
         }
-        if constexpr (kRuns > 2) request();  // (no registers for a wide step beside the operands)
+        if constexpr (PMAX > 2) request();  // (no registers for a wide step beside the operands)
       } else {
         auto put = [&](uint32_t i, float v) { xf[i] = flip_sign(v, in.rot_signbits[i >> 5] >> (i & 31u), 0); };
         if (norm) {
@@ -399,7 +388,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
         }
       }
       lds_barrier();
-      rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, in.rot_small, S, in.rot_m < kRotOctetM);
+      rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, F.s, in.rot_m < kRotOctetM);
       lds_barrier();
     }
 #pragma unroll 1
