@@ -19,19 +19,8 @@
 
 namespace llvq {
 
-constexpr int kNormThreads = 1024;
-
-__device__ __forceinline__ float block_sum_1024(float v, float* red) {
-  v = wave_sum(v);
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  __syncthreads();  // red may still be read from a previous call
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  float s = 0.f;
-#pragma unroll
-  for (int w = 0; w < kNormThreads / 64; ++w) s += red[w];  // same order in every lane
-  return s;
-}
+// Eight binary16 values per lane of a row's workgroup (rows of up to 8192, a multiple of 8).
+__host__ inline uint32_t norm_threads(uint32_t n) { return (n / 8u + 63u) / 64u * 64u; }
 
 // h[row] = embed[token[row]], row = blockIdx.y (token null: the one token `value`)
 __global__ __launch_bounds__(256) void embed_kernel(const __half* __restrict__ table, const uint32_t* __restrict__ token, uint32_t value,
@@ -45,37 +34,41 @@ __global__ __launch_bounds__(256) void embed_kernel(const __half* __restrict__ t
 // r = f16(h + delta) when delta is given (else h), written to h_out when that is given
 // (it may be h itself); normed = f16(r / sqrt(mean(r^2) + eps) * w)
 // (candle_nn::RmsNorm: f32 inside, one rounding on the way out).
-__global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(const __half* h, const __half* __restrict__ delta,
-                                                                   const __half* __restrict__ w, __half* h_out,
-                                                                   __half* __restrict__ normed, uint32_t n, float eps) {
-  __shared__ float red[kNormThreads / 64];
-  // one workgroup per row of n values
-  h += (size_t)blockIdx.x * n;
-  if (delta) delta += (size_t)blockIdx.x * n;
-  if (h_out) h_out += (size_t)blockIdx.x * n;
-  normed += (size_t)blockIdx.x * n;
-  constexpr int kPer = 8;  // n <= 8192
-  float v[kPer];
+// One workgroup of norm_threads(n) lanes per row of n values; 16 bytes of an operand per lane: with two bytes, and four
+// wavefronts where one has work, 500 rows of 2560 took 5.2 us.
+__global__ __launch_bounds__(1024) void add_rmsnorm_kernel(const __half* h, const __half* __restrict__ delta, const __half* __restrict__ w,
+                                                           __half* h_out, __half* __restrict__ normed, uint32_t n, float eps) {
+  __shared__ float red[16];
+  const uint32_t at = threadIdx.x * 8u, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const size_t row = (size_t)blockIdx.x * n;
+  const bool in = at < n;
+  const uint32_t from = in ? at : 0u;
+  HalfOctet x = *reinterpret_cast<const HalfOctet*>(h + row + from);
+  const HalfOctet g = *reinterpret_cast<const HalfOctet*>(w + from);
+  if (delta) {  // the residual stream is binary16
+    const HalfOctet d = *reinterpret_cast<const HalfOctet*>(delta + row + from);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      x.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(half_lo(x.w[j]) + half_lo(d.w[j]))) |
+               (uint32_t)__half_as_ushort(__float2half_rn(half_hi(x.w[j]) + half_hi(d.w[j]))) << 16;
+  }
+  if (h_out && in) *reinterpret_cast<HalfOctet*>(h_out + row + at) = x;
   float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const uint32_t i = threadIdx.x + (uint32_t)k * kNormThreads;
-    v[k] = 0.f;
-    if (i < n) {
-      float x = __half2float(h[i]);
-      if (delta) x = __half2float(__float2half_rn(x + __half2float(delta[i])));  // the residual stream is binary16
-      if (h_out) h_out[i] = __float2half_rn(x);
-      v[k] = x;
-      ss += x * x;
-    }
-  }
-  const float total = block_sum_1024(ss, red);
+  for (int j = 0; j < 4; ++j) ss = fmaf(half_lo(x.w[j]), half_lo(x.w[j]), fmaf(half_hi(x.w[j]), half_hi(x.w[j]), ss));
+  ss = wave_sum(in ? ss : 0.f);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  float total = 0.f;
+  for (uint32_t k = 0; k < (blockDim.x >> 6); ++k) total += red[k];  // same order in every lane
   const float inv = 1.0f / sqrtf(total / (float)n + eps);
+  if (!in) return;
+  HalfOctet o;
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const uint32_t i = threadIdx.x + (uint32_t)k * kNormThreads;
-    if (i < n) normed[i] = __float2half_rn(v[k] * inv * __half2float(w[i]));
-  }
+  for (int j = 0; j < 4; ++j)
+    o.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(half_lo(x.w[j]) * inv * half_lo(g.w[j]))) |
+             (uint32_t)__half_as_ushort(__float2half_rn(half_hi(x.w[j]) * inv * half_hi(g.w[j]))) << 16;
+  *reinterpret_cast<HalfOctet*>(normed + row + at) = o;
 }
 
 // int8 KV cache (llvq-llm/src/kvq.rs:110-165): asymmetric 8-bit codes per group
@@ -217,16 +210,19 @@ constexpr int kAttnMaxGroup = 8;    // query heads per kv head
 constexpr int kAttnInlineSplits = 16;  // up to this many ranges, the workgroup that finishes last merges them itself
 
 // ---- rows of positions at once (prompt processing through the batched product) ----
-// One wavefront per (head, row): q heads are normed and rotated in place, k heads are
+// One wavefront per (head, row), four to a workgroup: q heads are normed and rotated in place, k heads are
 // normed, rotated and appended to the cache at position pos0 + row, v heads are appended.
-// Grid (n_heads + 2 n_kv, rows).  Same arithmetic as the one-position path.
+// Grid (a quarter of n_heads + 2 n_kv, rows).  Same arithmetic as the one-position path.
 template <bool Q8>
-__global__ __launch_bounds__(64) void norm_rope_append_rows_kernel(__half* __restrict__ q, const __half* __restrict__ k,
+__global__ __launch_bounds__(256) void norm_rope_append_rows_kernel(__half* __restrict__ q, const __half* __restrict__ k,
                                                                    const __half* __restrict__ v, AttnNew nw, KvQ8 q8,
                                                                    uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
                                                                    uint32_t pos0, uint32_t max_pos) {
-  __shared__ float stage[256];
-  const uint32_t head = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
+  __shared__ float stages[4][256];
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t head = blockIdx.x * 4u + wave, row = blockIdx.y, lane = threadIdx.x & 63u;
+  if (head >= n_heads + 2u * n_kv) return;
+  float* stage = stages[wave];
   const uint32_t pos = pos0 + row, kvgroups = head_dim / kKvGroup;
   if (head < n_heads) {
     __half* qh = q + ((size_t)row * n_heads + head) * head_dim;
@@ -1045,13 +1041,20 @@ __global__ __launch_bounds__(128) void attn_merge_kernel(const float* __restrict
 }
 
 // act = f16(f16(silu(gate)) * up)   (model.rs:831: gu[0].apply(act).mul(gu[1]))
+// Eight values per lane and turn (two bytes at a time 500 rows of 9728 took 6.9 us); what is over eight goes one by one.
 __global__ __launch_bounds__(256) void silu_mul_kernel(const __half* __restrict__ gate, const __half* __restrict__ up,
                                                        __half* __restrict__ out, uint32_t n) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const float g = __half2float(gate[i]);
-    const float s = __half2float(__float2half_rn(g / (1.0f + __expf(-g))));
-    out[i] = __float2half_rn(s * __half2float(up[i]));
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n / 8u; i += gridDim.x * blockDim.x) {
+    const HalfOctet g = *reinterpret_cast<const HalfOctet*>(gate + i * 8u), u = *reinterpret_cast<const HalfOctet*>(up + i * 8u);
+    HalfOctet o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(silu_mul(half_lo(g.w[j]), half_lo(u.w[j])))) |
+               (uint32_t)__half_as_ushort(__float2half_rn(silu_mul(half_hi(g.w[j]), half_hi(u.w[j])))) << 16;
+    *reinterpret_cast<HalfOctet*>(out + i * 8u) = o;
   }
+  const uint32_t i = (n & ~7u) + threadIdx.x;
+  if (blockIdx.x == 0 && i < n) out[i] = __float2half_rn(silu_mul(__half2float(gate[i]), __half2float(up[i])));
 }
 
 // logits = f16(E h) for a dense binary16 head (Head::project, model.rs:578-587);

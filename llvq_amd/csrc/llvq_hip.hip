@@ -1912,12 +1912,12 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     if (fused) return forward_group(rt, mats, n, x, outs, LLVQ_F16, &pro);
     const __half* staged = nullptr;
     if (pro.kind == kPrologueAddRmsNorm) {
-      hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(kNormThreads), 0, st, x, reinterpret_cast<const __half*>(pro.x2),
+      hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, x, reinterpret_cast<const __half*>(pro.x2),
                          reinterpret_cast<const __half*>(pro.norm_w), reinterpret_cast<__half*>(pro.resid_out), d->normed,
                          d->hidden, pro.eps);
       staged = d->normed;
     } else {
-      hipLaunchKernelGGL(silu_mul_kernel, dim3((d->inter + 255) / 256), dim3(256), 0, st, reinterpret_cast<const __half*>(pro.x2),
+      hipLaunchKernelGGL(silu_mul_kernel, dim3((d->inter / 8 + 256) / 256), dim3(256), 0, st, reinterpret_cast<const __half*>(pro.x2),
                          x, d->act, d->inter);
       staged = d->act;
     }
@@ -2024,7 +2024,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   }
   phase_mark(d);
   if (want_logits) {
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(kNormThreads), 0, st, h, d->down, d->fnorm, h, d->normed, d->hidden, d->eps);
+    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, h, d->down, d->fnorm, h, d->normed, d->hidden, d->eps);
     launch_head(d, history_slot, record);
   }
   HIP_TRY(hipGetLastError());
@@ -2075,7 +2075,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
   for (uint32_t L = 0; L < d->n_layers; ++L) {
     const llvq_mat* const* P = d->proj.data() + (size_t)L * 7;
     // residual + previous MLP branch, then the input norm (the branch of layer 0 is absent)
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(n), dim3(kNormThreads), 0, st, ph, L ? d->pdown : (const __half*)nullptr,
+    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(n), dim3(norm_threads(d->hidden)), 0, st, ph, L ? d->pdown : (const __half*)nullptr,
                        d->ln1 + (size_t)L * d->hidden, L ? ph_alt : (__half*)nullptr, d->pnormed, d->hidden, d->eps);
     if (L) std::swap(ph, ph_alt);
     void* const qkv[3] = {d->pq, d->pk, d->pv};
@@ -2096,7 +2096,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     nw.kcache = kc;
     nw.vcache = vc;
     nw.eps = d->eps;
-    const dim3 hgrid(d->n_heads + 2 * d->n_kv, n), agrid(d->n_kv, n);
+    const dim3 hgrid((d->n_heads + 2 * d->n_kv + 3) / 4, n), agrid(d->n_kv, n);
     auto attend = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, agrid, dim3(64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->head_dim, d->pos, d->max_pos, scale);
     };
@@ -2109,7 +2109,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(kernel, mgrid, dim3(waves * 64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->pos, n, d->max_pos, scale);
     };
     if (d->kv_q8) {
-      hipLaunchKernelGGL(norm_rope_append_rows_kernel<true>, hgrid, dim3(64), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
+      hipLaunchKernelGGL(norm_rope_append_rows_kernel<true>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos);
       if (on_mfma) {
         if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<true, 2, 2>, 2 * 2);
@@ -2121,7 +2121,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       else if (grp <= 5) attend(attn_rows_kernel<true, 5>);
       else attend(attn_rows_kernel<true, kAttnMaxGroup>);
     } else {
-      hipLaunchKernelGGL(norm_rope_append_rows_kernel<false>, hgrid, dim3(64), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
+      hipLaunchKernelGGL(norm_rope_append_rows_kernel<false>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos);
       if (on_mfma) {
         if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<false, 2, 2>, 2 * 2);
@@ -2135,20 +2135,20 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     }
     rc = rows(P[3], d->pctx, d->po);
     if (rc) return rc;
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(n), dim3(kNormThreads), 0, st, ph, d->po, d->ln2 + (size_t)L * d->hidden, ph_alt,
+    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(n), dim3(norm_threads(d->hidden)), 0, st, ph, d->po, d->ln2 + (size_t)L * d->hidden, ph_alt,
                        d->pnormed, d->hidden, d->eps);
     std::swap(ph, ph_alt);
     void* const gate_up[2] = {d->pgate, d->pup};
     rc = llvq_hip_gemm_group(rt, P + 4, 2, d->pnormed, (int)n, gate_up, LLVQ_F16);
     if (rc) return rc;
     const uint32_t na = n * d->inter;
-    hipLaunchKernelGGL(silu_mul_kernel, dim3((na + 255) / 256 < 4096u ? (na + 255) / 256 : 4096u), dim3(256), 0, st, d->pgate, d->pup, d->pact, na);
+    hipLaunchKernelGGL(silu_mul_kernel, dim3(std::min((na / 8u + 256u) / 256u, 4096u)), dim3(256), 0, st, d->pgate, d->pup, d->pact, na);
     rc = rows(P[6], d->pact, d->pdown);
     if (rc) return rc;
   }
   if (want_logits) {
     const size_t last = (size_t)(n - 1) * d->hidden;
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(kNormThreads), 0, st, ph + last, d->pdown + last, d->fnorm, d->h, d->normed,
+    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, ph + last, d->pdown + last, d->fnorm, d->h, d->normed,
                        d->hidden, d->eps);
     launch_head(d, history_slot, record);
   }
