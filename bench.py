@@ -504,8 +504,8 @@ def main():
             "traffic": int(prof["traffic_bytes_per_launch"]) if prof_ok and "traffic_bytes_per_launch" in prof else None,
             "traffic_source": TRAFFIC_PROFILE if prof_ok else None,
             "profiled_kernel_avg_us": prof.get("kernel_avg_us"),
-            # what actually binds: the unranking arithmetic on the vector ALUs, not HBM (rocprofv3 SQ counters, same file)
-            "limited_by": "valu",
+            # what binds: the tiles' way from memory, 13 bytes per block where the encoding has 6
+            "limited_by": "hbm",
             "valu_slots_per_block": prof.get("valu_slots_per_block") if prof_ok else None,
             "valu_busy_frac": prof.get("valu_busy_frac") if prof_ok else None,
             "avg_launch_us": round(avg_launch_us, 3),
