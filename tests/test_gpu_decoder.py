@@ -461,6 +461,27 @@ def test_prompt_attention_on_the_matrix_cores(gpu_rt, orc, heads, kv, kv_mode, s
         dec.close()
 
 
+@pytest.mark.parametrize("heads,kv,kv_mode", [(4, 2, "f16"), (8, 2, "q8"), (10, 2, "f16"), (8, 1, "q8")])
+def test_attention_where_its_split_turns(gpu_rt, orc, heads, kv, kv_mode):
+    """Prompts that end a row block or a cache tile, one short of it and one past it (an odd count of tiles leaves the second
+    set of wavefronts one that is masked whole), and decoded positions where another range begins (64, 128) and where the
+    ranges leave the merge inside the launch (1024): the prompt path against the position-by-position path, whose
+    attention kernels share nothing."""
+    cfg = _wide(heads, kv, kv_mode)
+    cfg.max_positions = 1040
+    dec, _ = _build(gpu_rt, orc, cfg, 21, prefill_rows=512)
+    try:
+        tokens = np.random.default_rng(22).integers(0, cfg.vocab_size, size=1026)
+        one_by_one = [dec.forward_token(int(t))[0] for t in tokens]
+        for n in (1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 511, 1023, 1024, 1025, 1026):
+            dec.reset()
+            got, _best = dec.prefill(tokens[:n])
+            want = one_by_one[n - 1]
+            assert np.abs(got - want).max() < 2e-3 * np.abs(want).max(), n  # binary16 weights, as above
+    finally:
+        dec.close()
+
+
 @pytest.mark.parametrize("fixture_name,cfg,max_positions", [
     ("qwen3_4b_synthetic_greedy.json", decoder.QWEN3_4B, 768),
     ("qwen3_14b_q8kv_synthetic_greedy.json", decoder.QWEN3_14B, 128),

@@ -39,10 +39,10 @@ def usage(tmp_path_factory):
 
 def test_no_kernel_spills(usage):
     gemv = {k: v for k, v in usage.items() if "gemv_tiles_kernel" in k}
-    # 2 output types x ((full tile, half tile, lean image) x (natural, rotated basis) + cap-13 stream x (whole, lean image))
+    # 2 output types x 4 sources of the activation x (rows of up to 512 blocks, wider ones)
     assert len(gemv) == 16
     seq = {k: v for k, v in usage.items() if "gemv_seq_kernel" in k}
-    assert len(seq) == 10  # (full tile, lean image, half tile; full and lean again for the dense 49-bit blocks) x (two, three activation planes)
+    assert len(seq) == 10  # 2 output types x (independent, the same wide, ordered, with prologues, the same wide)
     gemv.update(seq)
     for name, u in usage.items():
         assert u["ScratchSize"] == 0, f"{name} spills {u['ScratchSize']} bytes per lane"
@@ -52,10 +52,9 @@ def test_no_kernel_spills(usage):
 
 
 def test_the_batched_kernel_does_not_spill_either(usage):
-    """Producers and consumers are separate branches of gemm_tiles_kernel, so the consumers' 64
-    accumulators and the producers' decode state share the 128 registers instead of adding up."""
+    """Sixteen wavefronts share a tile: 128 registers each."""
     gemm = {k: v for k, v in usage.items() if "gemm_tiles_kernel" in k}
-    assert len(gemm) == 2  # 8 or 12 producer wavefronts
+    assert len(gemm) == 2  # up to 16 activation rows, up to 64
     for name, u in gemm.items():
         assert u["ScratchSize"] == 0, (name, u)
         assert u["VGPRs"] + u.get("AGPRs", 0) <= 128, (name, u)
