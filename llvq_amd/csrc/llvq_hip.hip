@@ -734,10 +734,10 @@ static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids
   const size_t row_bits = (size_t)nb * m->record_bits;  // eight rows are whole bytes whatever the record width
   uint32_t rows_per = row_bits ? (uint32_t)std::min<size_t>(m->d_out, std::max<size_t>(8, kUploadBytes * 8 / row_bits / 8 * 8)) : m->d_out;
   rows_per = std::min(rows_per, (1u << 20));
-  float table[32];
+  TileTable table;
   for (uint32_t i = 0; i < 32; ++i) {
     const uint32_t shell = i & 15u;
-    table[i] = shell ? (float)centroids[i >> 4] * (float)(1.0 / std::sqrt(16.0 * shell)) : 0.f;
+    table.v[i] = shell ? (float)centroids[i >> 4] * (float)(1.0 / std::sqrt(16.0 * shell)) : 0.f;
   }
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->tiles), kTileTableBytes + (size_t)n_tiles * stride + kStepBytes + 256);  // a record's last step may reach past it
   if (e != hipSuccess) return e;
@@ -747,7 +747,6 @@ static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids
   uint8_t* d_codes = rt->upload_buf;
   float* d_scale = reinterpret_cast<float*>(d_codes + code_room);
   float* d_tail = reinterpret_cast<float*>(d_codes + code_room + scale_room);
-  if ((e = hipMemcpyAsync(m->tiles, table, sizeof table, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
   const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
   for (uint32_t r0 = 0; r0 < m->d_out; r0 += rows_per) {
     const uint32_t rows = std::min(rows_per, m->d_out - r0);
@@ -757,7 +756,8 @@ static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids
     if ((e = hipMemcpyAsync(d_scale, rscale + r0, (size_t)rows * 4, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
     if (m->tail_w && (e = hipMemcpyAsync(d_tail, tail + (size_t)r0 * m->tail_w, (size_t)rows * m->tail_w * 4, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
     const uint32_t heads = tile_count(rows) * kTileRows * (1u + m->tail_w);
-    hipLaunchKernelGGL(tile_heads_kernel, dim3((heads + 255u) / 256u), dim3(256), 0, rt->stream, d_scale, d_tail, out, rows, nb, m->tail_w);
+    hipLaunchKernelGGL(tile_heads_kernel, dim3((heads + 255u) / 256u), dim3(256), 0, rt->stream, table,
+                       r0 ? (float*)nullptr : reinterpret_cast<float*>(m->tiles), d_scale, d_tail, out, rows, nb, m->tail_w);
     if (nb) {
       const uint64_t blocks = (uint64_t)tile_count(rows) * kTileRows * nb;
       const uint32_t grid = (uint32_t)std::min<uint64_t>((blocks + 511) / 512, 2ull * cus);

@@ -80,9 +80,12 @@ __global__ __launch_bounds__(512) void transcode_kernel(GlobalTables g, const ui
   }
 }
 
-// Row scales and tail columns into the records' heads (zeros for rows past the last).
-__global__ __launch_bounds__(256) void tile_heads_kernel(const float* __restrict__ rscale, const float* __restrict__ tail, uint8_t* __restrict__ tiles,
+// Row scales and tail columns into the records' heads (zeros for rows past the last), the matrix's block scales to
+// `table_out` where that is given (as an argument: a copy of 128 bytes from the host costs an upload 15 us).
+struct TileTable { float v[kTileTableBytes / 4]; };
+__global__ __launch_bounds__(256) void tile_heads_kernel(TileTable table, float* table_out, const float* __restrict__ rscale, const float* __restrict__ tail, uint8_t* __restrict__ tiles,
                                                          uint32_t rows, uint32_t nb, uint32_t tail_w) {
+  if (table_out && blockIdx.x == 0 && threadIdx.x < kTileTableBytes / 4) table_out[threadIdx.x] = table.v[threadIdx.x];
   const uint32_t per = kTileRows * (1u + tail_w), stride = tile_stride(nb, tail_w);
   const uint32_t total = tile_count(rows) * per;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
