@@ -800,6 +800,12 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t jj = jb + 16u * u;
+      // A row past the range is one of the row this launch is about to write: whatever an earlier use of the cache left.
+      // Its weight is zero, and its values have to be as well: 0 x infinity would reach the sums.
+      if (jj >= nj) {
+        vraw[u] = make_uint4(0, 0, 0, 0);
+        vsc[u] = vbi[u] = 0.f;
+      }
       float kf[8];
       if (j0 + jj == newj) {  // the row appended by this launch: from LDS, as the cache returns it
 #pragma unroll

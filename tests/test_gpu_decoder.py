@@ -595,3 +595,32 @@ def test_config4_widths_and_context_against_the_oracle(gpu_rt):
             assert worst < 1e-3, f"batched={batched}: max |dlogit| / max|logit| = {worst:.3e}"
     finally:
         dec.close()
+
+
+@pytest.mark.parametrize("kv_mode,head_dim", [("f16", 64), ("f16", 128), ("q8", 64), ("q8", 128)])
+def test_a_decoder_recovers_from_a_non_finite_run(gpu_rt, kv_mode, head_dim):
+    """A token with an infinite embedding value leaves NaN in every cache row from its position on.  After a reset the
+    same decoder gives the logits of a fresh one, bit for bit: what an earlier run left at positions that are not yet
+    written reaches nothing."""
+    import dataclasses
+
+    cfg = dataclasses.replace(SMALL, num_hidden_layers=2, head_dim=head_dim, kv_mode=kv_mode, tie_word_embeddings=False)
+    weights = decoder.synthetic_weights(cfg, 12)
+    weights.embed[7, 3] = np.inf
+    tokens = [int(t) for t in np.random.default_rng(12).integers(8, cfg.vocab_size, size=70)]
+    projs = [[gpu_rt.upload(m) for m in layer] for layer in decoder.synthetic_projections(cfg, 12)]
+    used, fresh = decoder.Decoder(gpu_rt, cfg, projs, weights), decoder.Decoder(gpu_rt, cfg, projs, weights)
+    try:
+        assert np.isnan(used.forward_token(7)[0]).all()
+        for t in tokens:
+            used.forward_token(t, want_logits=False)
+        used.reset()
+        for t in tokens:
+            got, want = used.forward_token(t)[0], fresh.forward_token(t)[0]
+            assert np.isfinite(want).all() and np.array_equal(got, want)
+    finally:
+        used.close()
+        fresh.close()
+        for layer in projs:
+            for p in layer:
+                gpu_rt.free(p)
