@@ -409,7 +409,9 @@ __global__ __launch_bounds__(64) void attn_rows_kernel(const __half* __restrict_
 // chain (16 tiles for the last rows of a 500-row prompt), and a prompt's workgroups leave CUs idle.  31 -> 22 us for 500 rows of 32 heads.
 // Scores, maxima, sums and O stay in f32; the context is rounded once.  The next tile's K and
 // V rows are requested before the current tile is multiplied.  Positions past the pass's last
-// row are read as that row (their probabilities are zero; the values must be finite).
+// row are read as that row.  Inside a tile a masked position has probability zero and is multiplied
+// all the same, so a value that is not finite reaches the rows of its own block of 32 that come
+// before it; rows of earlier blocks never meet it.
 constexpr int kAttnTile = 32;
 constexpr int kAttnKPitch = 128 + 8;   // binary16 elements per K row in LDS
 constexpr int kAttnVPitch = 32 + 8;    // per V^T row
@@ -440,7 +442,7 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
   const uint32_t qpos = pos0 + my_row;
   const uint32_t last_pos = pos0 + n_rows - 1u;              // last cached position
   const uint32_t t_end = pos0 + min(row0 + kAttnTile - 1u, n_rows - 1u);
-  const uint32_t n_tiles = t_end / kAttnTile + 1u;           // a part takes every H-th; one past the last is masked whole
+  const uint32_t n_tiles = t_end / kAttnTile + 1u;           // a part takes every H-th; one past the last is staged and not multiplied
   const size_t base = (size_t)kvh * max_pos;
   constexpr uint32_t kvgroups = kDimH / kKvGroup;
 
@@ -519,6 +521,7 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
     deposit();
     __syncthreads();
     if (tile + H < n_tiles + part) request(tile + H);
+    if (H == 2 && tile >= n_tiles) continue;  // past every row of this block: nothing of it may reach their sums, not even times zero
     // S^T = K Q^T
     f16v sacc;
 #pragma unroll

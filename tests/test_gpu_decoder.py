@@ -624,3 +624,30 @@ def test_a_decoder_recovers_from_a_non_finite_run(gpu_rt, kv_mode, head_dim):
         for layer in projs:
             for p in layer:
                 gpu_rt.free(p)
+
+
+@pytest.mark.parametrize("heads,kv_mode", [(4, "f16"), (8, "q8"), (10, "f16"), (12, "q8")])
+def test_a_non_finite_row_stays_out_of_earlier_blocks_of_a_prompt(gpu_rt, heads, kv_mode):
+    """Prompt attention takes 32 rows at a time.  A token with an infinite embedding value at position 40 (the second
+    block, whose first rows and all later ones it spoils) must leave the cache rows of positions 0 to 31 as a prompt
+    without it does: the logits of a token decoded behind them are the same bit for bit."""
+    import dataclasses
+
+    cfg = dataclasses.replace(SMALL, num_hidden_layers=3, num_attention_heads=heads, head_dim=128, kv_mode=kv_mode, tie_word_embeddings=False)
+    weights = decoder.synthetic_weights(cfg, 13)
+    weights.embed[7, 3] = -np.inf
+    dec = decoder.Decoder(gpu_rt, cfg, decoder.synthetic_projections(cfg, 13), weights, prefill_rows=90)
+    try:
+        prompt = np.random.default_rng(13).integers(8, cfg.vocab_size, size=90)
+        got = []
+        for poison in (False, True):
+            p = prompt.copy()
+            p[40] = 7 if poison else p[40]
+            dec.reset()
+            last = dec.prefill(p)[0]
+            assert np.isnan(last).all() if poison else np.isfinite(last).all()
+            dec.seek(32)
+            got.append(dec.forward_token(11)[0])
+        assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
+    finally:
+        dec.close()
