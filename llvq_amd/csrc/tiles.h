@@ -138,7 +138,9 @@ __device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub
 #pragma unroll
   for (int j = 0; j < 8; ++j) m = max(m, __float_as_uint(v[j]) & 0x7FFFFFFFu);
   m = quad_max(m);
-  const uint32_t e = max(m >> 23, 64u);  // biased exponent of the block's largest; 2^-63 and below count as zero
+  // Biased exponent of the block's largest, at least the one below which `scale` would leave the normal range (2^-105 with
+  // six digits, 2^-113 with four): smaller blocks are quantised at that scale.
+  const uint32_t e = max(m >> 23, (uint32_t)kBits);
   const bool bad = m >= 0x7F800000u;     // inf or NaN: the block's products are NaN
   const float up = bad ? 0.f : __uint_as_float((253u + (uint32_t)kBits - e) << 23);
   const float scale = bad ? __builtin_nanf("") : __uint_as_float((e + 1u - (uint32_t)kBits) << 23);

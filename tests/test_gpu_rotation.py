@@ -138,3 +138,20 @@ def test_decoder_with_rotated_projections(gpu_rt, orc):
         assert worst < 2e-2
     finally:
         dec.close()
+
+
+@pytest.mark.parametrize("k", [-40, -64, -75, -90, 60])
+@pytest.mark.parametrize("d_in", [248, 13000])  # 13 000: rows past 512 blocks
+def test_a_power_of_two_goes_through_a_rotated_product_unchanged(gpu_rt, k, d_in):
+    """The activation is quantised per block relative to the block's largest value, so a power of two in front of an f32
+    activation is one in front of an f32 result, bit for bit, as long as nothing leaves the normal range (|k| <= 90)."""
+    import torch
+
+    proj = gpu_rt.upload(synth.make_matrix(f"model.layers.0.scaled.{d_in}.weight", 40, d_in, seed=4))
+    try:
+        xr = torch.from_numpy(synth.make_activation(d_in, seed=9)[0].astype(np.float32)).cuda().reshape(1, -1)
+        one = gpu_rt.forward_rotated(proj, xr, out_dtype=torch.float32).double()
+        got = gpu_rt.forward_rotated(proj, xr * 2.0 ** k, out_dtype=torch.float32)
+        assert torch.equal(got.double(), one * 2.0 ** k)
+    finally:
+        gpu_rt.free(proj)
