@@ -212,7 +212,11 @@ void llvq_hip_sequence_destroy(llvq_rt* rt, llvq_seq* seq);
 int llvq_hip_sequence_tune(llvq_seq* seq, uint32_t spin_limit, int hold_item);
 
 /* The row loop of group_forward (model.rs:521-529) as one batched product:
- * Y[M, d_out] = X[M, d_in] W^T, X row-major binary16. */
+ * Y[M, d_out] = X[M, d_in] W^T, X row-major binary16.
+ * Precision (M >= 2, shell cap 12): where d_in is a multiple of 8 and X starts on a 16-byte boundary, weights are
+ * rounded to binary16 once (and rotated rows to binary16): about 2e-4 of the results' norm.  All other rows, and all
+ * cap-13 matrices, are as good as llvq_hip_gemv is row by row (about 1e-7 with f32 results); such rows in a rotated
+ * basis, and cap-13 matrices, run row by row.  Tail columns, row scales and sums are f32 or better everywhere. */
 int llvq_hip_gemm(llvq_rt* rt, const llvq_mat* m, const void* x_f16_dev, int M, void* y_dev,
                   int y_dtype);
 
@@ -239,7 +243,9 @@ int llvq_hip_reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, in
  * copy of the activations and (rotated matrices) the rotated rows live in one static device
  * array of LLVQ_STATIC_SCRATCH_BYTES per GPU instead of buffers the runtime grows, and the
  * call makes no hipMalloc / hipFree.  A shape whose workspaces do not fit is refused with
- * LLVQ_ERR_UNSUPPORTED (the message names the bytes needed).  Every call on a GPU shares that
+ * LLVQ_ERR_UNSUPPORTED (the message names the bytes needed).  That limit is one of rows of a multiple of 8 values
+ * from a 16-byte boundary on; other rows, and cap-13 matrices, are taken whatever M is, up to the widest rows
+ * llvq_hip_gemv takes.  Every call on a GPU shares that
  * GPU's array: calls that overlap on one GPU (two streams, two runtimes) race. */
 #define LLVQ_STATIC_SCRATCH_BYTES (64u << 20)
 int llvq_hip_gemm_static(llvq_rt* rt, const llvq_mat* m, const void* x_f16_dev, int M, void* y_dev,

@@ -2,7 +2,10 @@
 // llvq_hip.hip after it.  The reference runs a row loop of matrix-vector products (llvq-llm/src/model.rs:521-529).
 //
 // Weights are multiplied as binary16: v centroid[gain] / sqrt(16 shell) rounded once; sums are f32; row scale and tail
-// columns are applied in f32 at the end.  A dword of a block's nibbles is eight consecutive columns of a row, which is
+// columns are applied in f32 at the end.  The PAIR variants of the kernels multiply what that rounding took as well and keep
+// their sums in f64 (of f32 sums over 32 or 48 columns), for the rows whose results are f32 exact (llvq_hip.hip,
+// gemm_same_basis).  Relative error of f32 results in norm, 2561 x 1000 at 65 rows: 2.1e-4 with one term, 1.01e-7 with two,
+// 0.97e-7 for rows one by one; 13000 columns: 2.2e-4, 1.37e-7, 1.38e-7.  Two terms alone, summed in f32, left up to 6e-7.  A dword of a block's nibbles is eight consecutive columns of a row, which is
 // exactly what a lane hands to a 16-deep (32 x 32) or 32-deep (16 x 16) product step, so a wavefront turns the 12 bytes
 // its lanes load into its own fragments: no weights pass through LDS, and the order in which the products walk the
 // columns is the order the blocks lie in (the lane groups of a fragment hold the same octet of two or four neighbouring
@@ -102,6 +105,31 @@ __device__ __forceinline__ half8_t dequant_octet(uint32_t w, const BlockScale& s
   return out;
 }
 
+// The same with what the rounding took as a second binary16 number each: the two make the weight to 2^-22 of it.  (A nibble
+// that lies four bits higher is brought down by the operation that takes the bias off, so both halves are v itself; what is
+// left of v hi after the first rounding is exact, and v lo joins it in one more.)  27 instructions.
+struct WeightPair {
+  half8_t hi, lo;
+};
+__device__ __forceinline__ WeightPair dequant_octet_pair(uint32_t w, const BlockScale& s) {
+  const uint32_t t[4] = {((w << 1) & 0x001E001Eu) ^ s.odd, (w & 0x00F000F0u) ^ s.odd8, ((w >> 7) & 0x001E001Eu) ^ s.odd, ((w >> 8) & 0x00F000F0u) ^ s.odd8};
+  const half2_t hi = half2_t{s.c.x, s.c.x}, lo = half2_t{s.c.y, s.c.y};
+  WeightPair out;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const half2_t u = __builtin_bit_cast(half2_t, t[i]);
+    const half2_t v = (i & 1) ? __builtin_elementwise_fma(u, half2_t{(_Float16)0.125f, (_Float16)0.125f}, half2_t{(_Float16)-144.f, (_Float16)-144.f})
+                              : u - half2_t{(_Float16)1040.f, (_Float16)1040.f};
+    const half2_t y = __builtin_elementwise_fma(v, hi, v * lo);
+    const half2_t r = __builtin_elementwise_fma(v, lo, __builtin_elementwise_fma(v, hi, -y));
+    out.hi[2 * i] = y.x;
+    out.hi[2 * i + 1] = y.y;
+    out.lo[2 * i] = r.x;
+    out.lo[2 * i + 1] = r.y;
+  }
+  return out;
+}
+
 struct GemmMat {
   const uint8_t* base;  // the matrix (table, then records)
   void* y;
@@ -159,7 +187,10 @@ __device__ __forceinline__ uint32_t lane_offset(uint32_t v) {
 // fragments, whose way from L2 would bind otherwise).
 // 2560 x 2560 at 5 rows: 35.9 -> 10.4 us; rotated q, k, v of 2560 columns at 64 rows, rotation included: 58.1 -> 21.7 us
 // (before: codes unranked in the product, partial sums through memory).
-template <int RG, int MT>
+// PAIR: both terms of the weights (dequant_octet_pair), 32 columns to a product sum that starts from zero, those added in
+// f64; RG = 1 always, two row groups would not fit the registers.  4097 columns, 1024 rows by 64: 16 -> 14 us (twice the
+// workgroups), 5000 by 33: 15 -> 22 us.
+template <int RG, int MT, bool PAIR>
 __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   extern __shared__ __align__(16) uint8_t smem[];
   constexpr uint32_t kRows = RG * 16, kCols = MT * 16;
@@ -222,11 +253,12 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   for (uint32_t j = 0; j < 3; ++j) load_x(j, q, q < n_quads);
   float unit;
   const uint32_t table = split_table(entry, unit);
-  acc4_t acc[RG][MT];
+  typedef double sum4_t __attribute__((ext_vector_type(4)));
+  typename std::conditional<PAIR, sum4_t, acc4_t>::type acc[RG][MT];
 #pragma unroll
   for (int k = 0; k < RG; ++k)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[k][mt] = acc4_t{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; ++mt) acc[k][mt] = 0;
   for (; q < n_quads; q += 16u) {
     const uint32_t qn = q + 16u;
     const bool live = qn < n_quads;
@@ -238,9 +270,18 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
     }
 #pragma unroll
     for (uint32_t j = 0; j < 3; ++j) {
-      half8_t w[RG];
+      half8_t w[RG], w2[RG];
 #pragma unroll
-      for (int k = 0; k < RG; ++k) w[k] = dequant_octet(j == 0 ? W[k].w0 : j == 1 ? W[k].w1 : W[k].w2, s[k]);
+      for (int k = 0; k < RG; ++k) {
+        const uint32_t nibbles = j == 0 ? W[k].w0 : j == 1 ? W[k].w1 : W[k].w2;
+        if constexpr (PAIR) {
+          const WeightPair p = dequant_octet_pair(nibbles, s[k]);
+          w[k] = p.hi;
+          w2[k] = p.lo;
+        } else {
+          w[k] = dequant_octet(nibbles, s[k]);
+        }
+      }
       // a register is asked for again as soon as its contents are used, and not moved from there
       if (j == 2u) {
         __builtin_amdgcn_sched_barrier(0);
@@ -250,8 +291,15 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int k = 0; k < RG; ++k)
-          acc[k][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, X[j][mt]), w[k], acc[k][mt], 0, 0, 0);
+        for (int k = 0; k < RG; ++k) {
+          if constexpr (PAIR) {
+            const acc4_t lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, X[j][mt]), w2[k], acc4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            const acc4_t one = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, X[j][mt]), w[k], lo, 0, 0, 0);
+            acc[k][mt] += __builtin_convertvector(one, sum4_t);
+          } else {
+            acc[k][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, X[j][mt]), w[k], acc[k][mt], 0, 0, 0);
+          }
+        }
       __builtin_amdgcn_sched_barrier(0);
       load_x(j, qn, live);
       __builtin_amdgcn_sched_barrier(0);
@@ -271,19 +319,20 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   for (int k = 0; k < RG; ++k)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      *reinterpret_cast<acc4_t*>(part + (((wave * RG + k) * MT + mt) * 64u + lane) * 4u) = acc[k][mt];
+      *reinterpret_cast<acc4_t*>(part + (((wave * RG + k) * MT + mt) * 64u + lane) * 4u) = __builtin_convertvector(acc[k][mt], acc4_t);
   __syncthreads();
   for (uint32_t o = tid; o < kRows * kCols; o += 1024u) {
     const uint32_t row = o % kRows, m = o / kRows;
     if (m >= a.M || t.row0 + row >= t.d_out) continue;
     const uint32_t l = (row & 15u) + 16u * ((m & 15u) >> 2), e = m & 3u;
     const float* p = part + (((row >> 4) * MT + (m >> 4)) * 64u + l) * 4u + e;
-    float s = 0.f;
+    typedef typename std::conditional<PAIR, double, float>::type sum_t;
+    sum_t s = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < 16; ++k) s += p[k * RG * MT * 256];
+    for (uint32_t k = 0; k < 16; ++k) s += (sum_t)p[k * RG * MT * 256];
     float tl = 0.f;
     for (uint32_t c = 0; c < a.tail_w; ++c) tl = fmaf(tw[row * 24u + c], tx[m * 24u + c], tl);
-    store_y(t.y, (size_t)m * t.d_out + t.row0 + row, fmaf(s, scale_s[row], tl), a.y_f32);
+    store_y(t.y, (size_t)m * t.d_out + t.row0 + row, fmaf((float)s, scale_s[row], tl), a.y_f32);
   }
 }
 template <int RG, int MT>
@@ -334,6 +383,8 @@ struct StoreEach {
 // that do not fill the other.
 // Octets and tiles go from memory to LDS without passing through registers, two to three steps of 48 columns (two
 // blocks) ahead.
+// PAIR: both terms of the weights against the same activations, 2 CF more products a round; every step's sums go to f64
+// ones (512 registers: CF = 4 and one wavefront on a SIMD).  2.4 us a step; 13000 x 5121 at 600 rows 115 -> 250 us.
 // Launches with too few tiles to fill the chip split the columns (`splits`): partial sums go to the workspace and
 // gemm_reduce_kernel adds them in order; otherwise the tile is finished here.
 // Gate and up of an 8B layer (24576 x 4096) at 512 rows: 158 -> 116 us, 886 TFLOP/s; a plain f16 product of that size
@@ -360,8 +411,8 @@ __device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t offset, const
 template <int N>
 __device__ __forceinline__ void wide_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-template <int CF>
-__global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArgs a) {
+template <int CF, bool PAIR>
+__global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel(GemmArgs a) {
   constexpr uint32_t kCols = 32u * CF, kBuf = gemm_wide_buf<CF>();
   constexpr int kLoadsX = 3 * CF / 4, kLoadsW = 2, kLoads = kLoadsX + kLoadsW;  // of a wavefront in a step
   extern __shared__ __align__(16) uint8_t smem[];     // [kWideDepth] x { [6 octets][kCols] 16 bytes, [8] x 32 rows of tiles }
@@ -410,6 +461,15 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
     for (int c = 0; c < CF; ++c)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[k][c][e] = 0.f;
+  double sum[PAIR ? 2 : 1][PAIR ? CF : 1][16];  // of the steps, with PAIR
+  if constexpr (PAIR) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int c = 0; c < CF; ++c)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum[k][c][e] = 0.;
+  }
   float unit;
   const uint32_t table = split_table(entry, unit);
   // One step: three rounds of eight products, in whose shadow the weights of the round after are unpacked and its
@@ -418,13 +478,21 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
   // are read, in the third unpacked.
   struct W3 { uint32_t w[3]; };
   typedef __attribute__((address_space(3))) uint32_t lds_u32;
-  half8_t w[2], x[CF];
+  half8_t w[2], w2[2], x[CF];
   W3 W[2], Wn[2];
   uint32_t meta[2], parts[2];
   BlockScale sc[2];
   auto unpack = [&](uint32_t j) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) w[k] = dequant_octet(W[k].w[j], sc[k]);
+    for (int k = 0; k < 2; ++k) {
+      if constexpr (PAIR) {
+        const WeightPair p = dequant_octet_pair(W[k].w[j], sc[k]);
+        w[k] = p.hi;
+        w2[k] = p.lo;
+      } else {
+        w[k] = dequant_octet(W[k].w[j], sc[k]);
+      }
+    }
   };
   const uint32_t x_at = (h * 3u * kCols + l32) * 16u;
   const uint32_t block_at = gemm_wide_x_bytes<CF>() + wave * 2u * kWideTileBytes + (l32 >> 3) * (2u * kTileBlockBytes) + h * kTileBlockBytes;
@@ -457,7 +525,7 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
   };
   auto round = [&](uint32_t buffer, uint32_t next, auto round_j) __attribute__((always_inline)) {
     constexpr uint32_t j = decltype(round_j)::value;
-    const half8_t w0[2] = {w[0], w[1]};
+    const half8_t w0[2] = {w[0], w[1]}, w20[2] = {w2[0], w2[1]};
     half8_t x0[CF];
 #pragma unroll
     for (int c = 0; c < CF; ++c) x0[c] = x[c];
@@ -469,6 +537,12 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
       scales();
       unpack(0);
     }
+    if constexpr (PAIR) {
+#pragma unroll
+      for (int c = 0; c < CF; ++c)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) acc[k][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w20[k], x0[c], acc[k][c], 0, 0, 0);
+    }
 #pragma unroll
     for (int c = 0; c < CF; ++c)
 #pragma unroll
@@ -476,10 +550,11 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
 #pragma unroll
     for (int c = 0; c < CF; ++c) {
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read,
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product,
-      __builtin_amdgcn_sched_group_barrier(0x002, CF == 8 ? 3 : 5, 0);  // vector instructions
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, CF == 8 ? 3 : 5, 0);
+#pragma unroll
+      for (int i = 0; i < (PAIR ? 4 : 2); ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product,
+        __builtin_amdgcn_sched_group_barrier(0x002, PAIR ? (CF == 8 ? 2 : 4) : (CF == 8 ? 3 : 5), 0);  // vector instructions
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -508,7 +583,26 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
     last = buffer;
     buffer = next;
     next = next + kBuf == kWideDepth * kBuf ? 0u : next + kBuf;
+    if constexpr (PAIR) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int c = 0; c < CF; ++c)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            sum[k][c][e] += (double)acc[k][c][e];
+            acc[k][c][e] = 0.f;
+          }
+    }
   } while (++s < s1);
+  if constexpr (PAIR) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int c = 0; c < CF; ++c)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[k][c][e] = (float)sum[k][c][e];
+  }
   wide_wait<0>();
   if constexpr (CF == 8) {
 #pragma unroll
@@ -571,15 +665,20 @@ __global__ __launch_bounds__(256, CF == 8 ? 1 : 2) void gemm_wide_kernel(GemmArg
       }
 #pragma unroll
       for (int c = 0; c < CF; ++c) {
-        acc16_t v = acc[k][c];
+        // f32 tail columns, two at a time: the halves hold one each.  (One by one on top of the blocks' sum each costs that a
+        // rounding: with PAIR they are summed by themselves and meet it last.)
+        acc16_t v;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] *= scale[e];
-        // f32 tail columns, two at a time: the halves hold one each
+        for (int e = 0; e < 16; ++e) v[e] = PAIR ? 0.f : acc[k][c][e] * scale[e];
         for (uint32_t i = 0; i < a.tail_w; i += 2u) {
           const uint32_t col = min(i + he, a.tail_w - 1u);
           const float keep = i + he < a.tail_w ? 1.f : 0.f;
           v = __builtin_amdgcn_mfma_f32_32x32x2f32(keep * w_tail[col * kWideRows + wave * 64u + (uint32_t)k * 32u + l32e],
                                                    x_tail[col * kCols + (uint32_t)c * 32u + l32e], v, 0, 0, 0);
+        }
+        if constexpr (PAIR) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) v[e] = fmaf(acc[k][c][e], scale[e], v[e]);
         }
         const uint32_t m = m0 + (uint32_t)c * 32u;
         if (m < a.M) decltype(to)::store(t.y, (size_t)m * t.d_out, row, he, t.d_out, v);
@@ -608,7 +707,10 @@ struct GemmReduceArgs {
   GemmArgs g;
   uint32_t rows_per_tile, row_chunks;
 };
+// With PAIR the splits are added in f64 and the tail by itself.
+template <bool PAIR>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
+  typedef typename std::conditional<PAIR, double, float>::type sum_t;
   __shared__ float x_tail[kReduceM][32];
   static_assert(kReduceM * 32u == 256u && kDim <= 32, "a value of the activations' tail per lane");
   const GemmArgs& a = ra.g;
@@ -625,9 +727,9 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
     x_tail[threadIdx.x / 32u][threadIdx.x % 32u] = __half2float(a.x[(size_t)m * a.ldx + a.nb * kDim + c]);
   }
   const float scale = reinterpret_cast<const float*>(rec)[r];
-  float s[kReduceM];
+  sum_t s[kReduceM];
 #pragma unroll
-  for (uint32_t k = 0; k < kReduceM; ++k) s[k] = 0.f;
+  for (uint32_t k = 0; k < kReduceM; ++k) s[k] = 0;
   for (uint32_t p0 = 0; p0 < a.splits; p0 += kReduceSplits) {
     float v[kReduceSplits][kReduceM];
 #pragma unroll
@@ -638,10 +740,11 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
 #pragma unroll
     for (uint32_t p = 0; p < kReduceSplits; ++p)
 #pragma unroll
-      for (uint32_t k = 0; k < kReduceM; ++k) s[k] = p0 + p < a.splits ? s[k] + v[p][k] : s[k];
+      for (uint32_t k = 0; k < kReduceM; ++k) s[k] = p0 + p < a.splits ? s[k] + (sum_t)v[p][k] : s[k];
   }
+  float out[kReduceM];
 #pragma unroll
-  for (uint32_t k = 0; k < kReduceM; ++k) s[k] *= scale;
+  for (uint32_t k = 0; k < kReduceM; ++k) out[k] = PAIR ? 0.f : (float)s[k] * scale;
   if (tail_w) {
     lds_barrier();
     for (uint32_t c0 = 0; c0 < tail_w; c0 += 8u) {
@@ -652,14 +755,14 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
       for (uint32_t c = 0; c < 8u; ++c)
         if (c0 + c < tail_w) {
 #pragma unroll
-          for (uint32_t k = 0; k < kReduceM; ++k) s[k] = fmaf(tw[c], x_tail[k][c0 + c], s[k]);
+          for (uint32_t k = 0; k < kReduceM; ++k) out[k] = fmaf(tw[c], x_tail[k][c0 + c], out[k]);
         }
     }
   }
   if (mine < n_rows && my_row < t.d_out) {
 #pragma unroll
     for (uint32_t k = 0; k < kReduceM; ++k)
-      if (m0 + k < a.M) store_y(t.y, (size_t)(m0 + k) * t.d_out + row, s[k], a.y_f32);
+      if (m0 + k < a.M) store_y(t.y, (size_t)(m0 + k) * t.d_out + row, PAIR ? fmaf((float)s[k], scale, out[k]) : out[k], a.y_f32);
   }
 }
 

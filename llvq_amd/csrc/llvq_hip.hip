@@ -635,10 +635,11 @@ int llvq_hip_runtime_create(int device, void* hip_stream, llvq_rt** out) {
   for_each_gemv_kernel([&](const void* kernel) { (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds); });
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rotate_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rotate_kernel<__half>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<1, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<2, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_wide_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_wide_kernel<8>), hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+  for (const void* kernel : {reinterpret_cast<const void*>(gemm_tiles_kernel<1, 1, false>), reinterpret_cast<const void*>(gemm_tiles_kernel<1, 1, true>),
+                             reinterpret_cast<const void*>(gemm_tiles_kernel<2, 4, false>), reinterpret_cast<const void*>(gemm_tiles_kernel<1, 4, true>),
+                             reinterpret_cast<const void*>(gemm_wide_kernel<4, false>), reinterpret_cast<const void*>(gemm_wide_kernel<4, true>),
+                             reinterpret_cast<const void*>(gemm_wide_kernel<8, false>)})
+    (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   *out = rt;
   return LLVQ_OK;
 }
@@ -1378,14 +1379,19 @@ static int workspace_take(llvq_rt* rt, GemmWorkspace* w, void** runtime_buf, siz
   return LLVQ_OK;
 }
 
-// Rows of activations one batched launch takes; more go out as further launches.
+// Rows of activations one batched launch takes; more go out as further launches.  With both terms of the weights (pair)
+// half as many where the rows are so wide that their octets would exceed 32 MiB: up to the widest rows a batch-1 product
+// takes, such a launch's octets and partial sums (kGemmWsCap) then fit LLVQ_STATIC_SCRATCH_BYTES.
 constexpr uint32_t kGemmMaxM = 1024;
+static uint32_t gemm_chunk(uint32_t nb, bool pair) { return pair && (nb + 3u) / 4u * 12u > 2048u ? kGemmMaxM / 2 : kGemmMaxM; }
+static_assert((kGemvMaxBlocks + 3) / 4 * 12 * (kGemmMaxM / 2) * 16 <= (32u << 20) && 2048u * kGemmMaxM * 16 <= (32u << 20), "octets of a launch");
 
 // Measured times of one step (48 columns) of the wide kernel in us: 256 activation rows; 128, two workgroups sharing a
-// CU, each; and one of those alone.
-constexpr double kWideStep = 1.28, kWideHalfStep = 0.69, kWideHalfStepAlone = 0.8;
+// CU, each; one of those alone; and 128 with both terms of the weights.
+constexpr double kWideStep = 1.28, kWideHalfStep = 0.69, kWideHalfStepAlone = 0.8, kWidePairStep = 2.4;
 
-// How a batched launch over these matrices at M rows is cut up, and the workspaces it needs.
+// How a batched launch over these matrices at M rows is cut up, and the workspaces it needs.  pair: with both terms of
+// the weights (gemm_same_basis says when).
 struct GemmPlan {
   uint32_t small;                // 1: up to 16 rows, 2: up to 64 (gemm_tiles_kernel), 0: gemm_wide_kernel
   uint32_t cf, rows_per_tile;    // the wide kernel's form, and weight rows of a workgroup
@@ -1395,13 +1401,13 @@ struct GemmPlan {
 // The wide kernel's partial sums are kept below this: more column splits than that allows would cost more in memory
 // traffic than they gain in filled CUs.
 constexpr size_t kGemmWsCap = 32u << 20;
-static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n, uint32_t M) {
+static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n, uint32_t M, bool pair) {
   const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), nb = mats[0]->nblocks;
   GemmPlan p{};
   p.small = M <= 16u ? 1u : M <= kGemmSmallRows ? 2u : 0u;
   p.splits = 1;
   p.m_tiles = 1;
-  p.rows_per_tile = p.small ? p.small * 16u : kWideRows;
+  p.rows_per_tile = !p.small ? kWideRows : pair ? 16u : p.small * 16u;
   for (int i = 0; i < n; ++i) p.n_tiles += (mats[i]->d_out + p.rows_per_tile - 1u) / p.rows_per_tile;
   p.n_oct = (nb + 3u) / 4u * 12u;
   if (p.small) {
@@ -1413,12 +1419,12 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
   // workgroup's share of a CU, and for the splits what the partial sums cost on their way through memory.
   const uint32_t steps = (nb + 1u) / 2u;
   double best = 1e30;
-  for (uint32_t cf = 8; cf >= 4u; cf -= 4u) {
+  for (uint32_t cf = pair ? 4u : 8u; cf >= 4u; cf -= 4u) {
     const uint32_t m_tiles = (M + 32u * cf - 1u) / (32u * cf), tiles = p.n_tiles * m_tiles, m_pad = m_tiles * 32u * cf;
     const size_t one = (size_t)m_pad * p.n_tiles * kWideRows * sizeof(float);
     for (uint32_t sp = 1; sp <= 16u && (sp == 1u || (steps / sp >= 8u && one * sp <= kGemmWsCap)); ++sp) {
       const uint32_t per = (steps + sp - 1u) / sp, wgs = tiles * ((steps + per - 1u) / per), per_cu = (wgs + cus - 1u) / cus;
-      const double cost = (cf == 8u ? per_cu * kWideStep : per_cu == 1u ? kWideHalfStepAlone : per_cu * kWideHalfStep) * per +
+      const double cost = (pair ? per_cu * kWidePairStep : cf == 8u ? per_cu * kWideStep : per_cu == 1u ? kWideHalfStepAlone : per_cu * kWideHalfStep) * per +
                           (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
       if (cost < best) {
         best = cost;
@@ -1449,13 +1455,16 @@ static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint
     bool six_byte = true;
     for (int i = i0; i < i1; ++i) six_byte &= mats[i]->record_bits == 48;
     if (mats[i0]->nblocks && six_byte) {  // (cap-13 matrices take the row loop, which has no workspace)
-      const uint32_t chunk = std::min(max_rows, kGemmMaxM);
-      // every row count up to the chunk: the splits, and so the partial sums, are not monotone in it
-      for (uint32_t M = 16;; M = M < 64u ? M + 48u : M < 128u ? 128u : M + 128u) {
-        const GemmPlan p = gemm_plan(rt, mats + i0, i1 - i0, M < chunk ? M : chunk);
-        ws = p.ws_bytes > ws ? p.ws_bytes : ws;
-        xt = p.xt_bytes > xt ? p.xt_bytes : xt;
-        if (M >= chunk) break;
+      for (const bool pair : {false, true}) {
+        if (pair ? mats[i0]->has_rotation : mats[i0]->d_in % 8 != 0) continue;  // no call takes it (gemm_same_basis)
+        const uint32_t chunk = std::min(max_rows, gemm_chunk(mats[i0]->nblocks, pair));
+        // every row count up to the chunk: the splits, and so the partial sums, are not monotone in it
+        for (uint32_t M = 16;; M = M < 64u ? M + 48u : M < 128u ? 128u : M + 128u) {
+          const GemmPlan p = gemm_plan(rt, mats + i0, i1 - i0, M < chunk ? M : chunk, pair);
+          ws = p.ws_bytes > ws ? p.ws_bytes : ws;
+          xt = p.xt_bytes > xt ? p.xt_bytes : xt;
+          if (M >= chunk) break;
+        }
       }
     }
     if (mats[i0]->has_rotation) {
@@ -1473,10 +1482,10 @@ static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint
 // One launch over n <= kGemmMaxGroup matrices of equal d_in that take the same activations
 // (already in the matrices' basis), M <= kGemmMaxM rows.
 static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, uint32_t M, void* const* y,
-                       int y_dtype, GemmWorkspace* wsp = nullptr) {
+                       int y_dtype, bool pair, GemmWorkspace* wsp = nullptr) {
   const llvq_mat* m0 = mats[0];
   const __half* xh = reinterpret_cast<const __half*>(x);
-  const GemmPlan p = gemm_plan(rt, mats, n, M);
+  const GemmPlan p = gemm_plan(rt, mats, n, M, pair);
   void* ws_buf = nullptr;
   void* xt_buf = nullptr;
   const size_t mark = wsp ? wsp->used : 0;  // a launch's carvings are released when it has been enqueued: the stream orders the next
@@ -1509,14 +1518,21 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   hipLaunchKernelGGL(tile_activations_kernel, dim3((oct_waves + 3u) / 4u), dim3(256), 0, rt->stream, xh, M, a.ldx, a.nb * 24u, p.m_pad, p.n_oct,
                      reinterpret_cast<uint4*>(xt_buf));
   const dim3 wide_grid(a.n_tiles * p.m_tiles * p.splits);
-  if (p.small == 1u) hipLaunchKernelGGL((gemm_tiles_kernel<1, 1>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<1, 1>()), rt->stream, a);
-  else if (p.small) hipLaunchKernelGGL((gemm_tiles_kernel<2, 4>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<2, 4>()), rt->stream, a);
-  else if (p.cf == 4u) hipLaunchKernelGGL(gemm_wide_kernel<4>, wide_grid, dim3(256), gemm_wide_lds<4>(), rt->stream, a);
-  else hipLaunchKernelGGL(gemm_wide_kernel<8>, wide_grid, dim3(256), gemm_wide_lds<8>(), rt->stream, a);
+  auto product = [&](auto pair) {
+    constexpr bool kPair = decltype(pair)::value;
+    if (p.small == 1u) hipLaunchKernelGGL((gemm_tiles_kernel<1, 1, kPair>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<1, 1>()), rt->stream, a);
+    else if (p.small) hipLaunchKernelGGL((gemm_tiles_kernel<kPair ? 1 : 2, 4, kPair>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<kPair ? 1 : 2, 4>()), rt->stream, a);
+    else if (p.cf == 4u) hipLaunchKernelGGL((gemm_wide_kernel<4, kPair>), wide_grid, dim3(256), gemm_wide_lds<4>(), rt->stream, a);
+    else if constexpr (!kPair) hipLaunchKernelGGL((gemm_wide_kernel<8, false>), wide_grid, dim3(256), gemm_wide_lds<8>(), rt->stream, a);
+  };
+  if (pair) product(std::true_type{});
+  else product(std::false_type{});
   if (p.splits > 1u) {
     r.rows_per_tile = p.rows_per_tile;
     r.row_chunks = (a.n_tiles * p.rows_per_tile + 255u) / 256u;
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3(r.row_chunks * ((M + kReduceM - 1u) / kReduceM)), dim3(256), 0, rt->stream, r);
+    const dim3 grid(r.row_chunks * ((M + kReduceM - 1u) / kReduceM));
+    if (pair) hipLaunchKernelGGL(gemm_reduce_kernel<true>, grid, dim3(256), 0, rt->stream, r);
+    else hipLaunchKernelGGL(gemm_reduce_kernel<false>, grid, dim3(256), 0, rt->stream, r);
   }
   HIP_TRY(hipGetLastError());
   return LLVQ_OK;
@@ -1537,8 +1553,15 @@ static size_t static_admission_bytes(const llvq_rt* rt, const llvq_mat* m, uint3
   return ((sums + 255) & ~(size_t)255) + (size_t)spb * 12 * ((M + 63) / 64 * 64) * 64;
 }
 
-// Matrices [0, n) of one group: same d_in, same basis.  A single row runs as GEMV launches instead, as do matrices
-// without a whole block and cap-13 matrices, whose rows keep the bits of the single-row product.
+// Matrices [0, n) of one group: same d_in, same basis.  What such a call has always been good to decides its way:
+//   * rows of a multiple of 8 values from a 16-byte boundary on: weights rounded to binary16 once (error 2e-4 of the
+//     results' norm);
+//   * other rows, natural basis: both terms of the weights (1e-7 with f32 results, which is what a row by itself has).
+//     A second product costs the matrix cores twice the time (13000 x 5121 at 600 rows 250 us for 115) and a loop of
+//     single rows many times that (27 900 us before there were tiles);
+//   * row by row, as batch-1 products: a single row, other rows in a rotated basis (the products above take them as
+//     binary16, a row by itself in f32; such widths end at 124), matrices without a whole block, and cap-13 matrices,
+//     whose rows keep the bits of the single-row product.
 static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, int M, void* const* y, int y_dtype,
                            GemmWorkspace* wsp = nullptr) {
   const llvq_mat* m0 = mats[0];
@@ -1546,7 +1569,8 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
   const uint8_t* xb = reinterpret_cast<const uint8_t*>(x);
   bool six_byte = true;
   for (int i = 0; i < n; ++i) six_byte &= mats[i]->record_bits == 48;
-  if (M < 2 || m0->nblocks == 0 || !six_byte) {
+  const bool pair = m0->d_in % 8 != 0 || (reinterpret_cast<uintptr_t>(x) & 15) != 0;
+  if (M < 2 || m0->nblocks == 0 || !six_byte || (pair && m0->has_rotation)) {
     for (int i = 0; i < n; ++i)
       for (int r = 0; r < M; ++r) {
         const int rc = launch_gemv(rt, mats[i], xb + (size_t)r * m0->d_in * 2, reinterpret_cast<uint8_t*>(y[i]) + (size_t)r * mats[i]->d_out * esz, y_dtype);
@@ -1554,17 +1578,18 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
       }
     return LLVQ_OK;
   }
-  const int chunk = std::min(M, (int)kGemmMaxM);
+  const int chunk = std::min(M, (int)gemm_chunk(m0->nblocks, pair));
   if (wsp && wsp->fixed) {
     // a call that does not fit is refused whole, before its first launch
     auto after = [](size_t used, size_t bytes) { return ((used + 255) & ~(size_t)255) + bytes; };
     const size_t base = m0->has_rotation ? after(wsp->used, (size_t)M * m0->d_in * sizeof(__half)) : wsp->used;
     size_t need = base;
-    for (int m_lo = 0; m_lo < M; m_lo += 512)
-      for (int i = 0; i < n; ++i) need = std::max(need, after(base, static_admission_bytes(rt, mats[i], (uint32_t)std::min(M - m_lo, 512))));
+    if (!pair)  // (rows that pair takes have no such bound, and fit: gemm_chunk)
+      for (int m_lo = 0; m_lo < M; m_lo += 512)
+        for (int i = 0; i < n; ++i) need = std::max(need, after(base, static_admission_bytes(rt, mats[i], (uint32_t)std::min(M - m_lo, 512))));
     for (int m_lo = 0; m_lo < M; m_lo += chunk)
       for (int i0 = 0; i0 < n; i0 += kGemmMaxGroup) {
-        const GemmPlan p = gemm_plan(rt, mats + i0, std::min(n - i0, kGemmMaxGroup), (uint32_t)std::min(M - m_lo, chunk));
+        const GemmPlan p = gemm_plan(rt, mats + i0, std::min(n - i0, kGemmMaxGroup), (uint32_t)std::min(M - m_lo, chunk), pair);
         need = std::max(need, after(p.ws_bytes ? after(base, p.ws_bytes) : base, p.xt_bytes));
       }
     if (need > wsp->fixed_bytes)
@@ -1587,7 +1612,7 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
       const int cnt = n - i0 < kGemmMaxGroup ? n - i0 : kGemmMaxGroup;
       void* ys[kGemmMaxGroup];
       for (int i = 0; i < cnt; ++i) ys[i] = reinterpret_cast<uint8_t*>(y[i0 + i]) + (size_t)m_lo * mats[i0 + i]->d_out * esz;
-      const int rc = launch_gemm(rt, mats + i0, cnt, xb + (size_t)m_lo * m0->d_in * 2, mc, ys, y_dtype, wsp);
+      const int rc = launch_gemm(rt, mats + i0, cnt, xb + (size_t)m_lo * m0->d_in * 2, mc, ys, y_dtype, pair, wsp);
       if (rc) return rc;
     }
   }

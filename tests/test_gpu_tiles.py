@@ -81,3 +81,66 @@ def test_rotations(gpu_rt, orc, n):
             assert torch.equal(one, two)
     finally:
         gpu_rt.free(proj)
+
+
+# Rows that do not start on 16-byte boundaries: widths that are no multiple of 8 (every tail length's parity, blocks that
+# end inside a quad and inside a step), or a first row one value past a boundary (`off`).  Sizes: the edges of the three
+# kernels (16, 64, 128 rows), row tiles with something over, column splits, more rows than a launch takes.
+# Bar: what rounds is a weight's block scale (twice), its two terms, the row scale and the sums, 2^-24 of the weight each:
+# eight of those.  (A weight rounded to binary16 once is 2e-4 off.)
+@pytest.mark.parametrize("nb,tail,d_out,M,off", [
+    (1, 1, 9, 2, 0), (16, 17, 1024, 3, 0), (41, 19, 33, 16, 0), (63, 23, 100, 17, 0), (170, 17, 70, 64, 0), (65, 5, 257, 65, 0), (106, 17, 1000, 129, 0),
+    (541, 15, 300, 200, 0), (3, 4, 70, 700, 0), (20, 2, 31, 1030, 0), (684, 3, 24, 515, 0), (32, 0, 40, 5, 1), (64, 8, 70, 40, 3), (85, 16, 300, 300, 1)])
+def test_batched_rows_off_their_boundaries_are_as_good_as_single_rows(gpu_rt, orc, nb, tail, d_out, M, off):
+    import torch
+
+    d_in = nb * 24 + tail
+    raw = synth.make_matrix(f"model.layers.0.tiles.{d_out}x{d_in}.weight", d_out, d_in, seed=nb + M)
+    X = synth.make_activation(d_in, seed=M, rows=M)
+    Y_ref, _ = _reference(orc, raw, X)
+    proj = gpu_rt.upload(raw)
+    try:
+        buf = torch.empty(M * d_in + 8, dtype=torch.float16, device="cuda")
+        x = buf[off:off + M * d_in].view(M, d_in)
+        x.copy_(_x16(X))
+        Y32, again = (torch.empty((M, d_out), dtype=torch.float32, device="cuda") for _ in range(2))
+        Y16 = torch.empty((M, d_out), dtype=torch.float16, device="cuda")
+        gpu_rt.forward_batched_into(proj, x, Y32)
+        gpu_rt.forward_batched_into(proj, x, again)
+        gpu_rt.forward_batched_into(proj, x, Y16)
+        rows = sorted({0, 1, M // 2, M - 1})
+        single = torch.stack([gpu_rt.forward(proj, x[r], out_dtype=torch.float32) for r in rows])
+    finally:
+        gpu_rt.free(proj)
+
+    def error(Y, want):
+        return np.linalg.norm(Y.double().cpu().numpy() - want) / np.linalg.norm(want)
+
+    print(f"OBSERVED {d_out}x{d_in} M={M} off={off}: {error(Y32, Y_ref):.2e}, single rows {error(single, Y_ref[rows]):.2e}")
+    assert error(single, Y_ref[rows]) < 8 * 2.0 ** -24
+    assert error(Y32, Y_ref) < 8 * 2.0 ** -24
+    assert torch.equal(Y32, again)
+    # the same sums, to the nearest binary16: half a unit in the last place, 2^-11 of the value (and 2^-25 below the normal
+    # range), and a rounding of the f32 sum itself, which a fused conversion does not have
+    off16 = (Y16.double() - Y32.double()).abs()
+    assert bool((off16 <= (2.0 ** -11 + 2.0 ** -23) * Y32.double().abs() + 2.0 ** -25).all())
+
+
+# In a rotated basis such rows go one by one, as they always have: rotated in f32, the bits of the single-row product.
+@pytest.mark.parametrize("n,M,off", [(100, 5, 0), (124, 70, 0), (26, 3, 0), (256, 17, 1), (960, 3, 1)])
+def test_rotated_rows_off_their_boundaries_go_one_by_one(gpu_rt, n, M, off):
+    import torch
+
+    raw = synth.make_matrix(f"model.layers.0.tiles.rot{n}.weight", 40, n, seed=n)
+    raw.rotation_seed = n
+    proj = gpu_rt.upload(raw)
+    try:
+        buf = torch.empty(M * n + 8, dtype=torch.float16, device="cuda")
+        x = buf[off:off + M * n].view(M, n)
+        x.copy_(_x16(synth.make_activation(n, seed=M, rows=M)))
+        for dt in (torch.float32, torch.float16):
+            y = torch.empty((M, 40), dtype=dt, device="cuda")
+            gpu_rt.forward_batched_into(proj, x, y)
+            assert torch.equal(y, torch.stack([gpu_rt.forward(proj, x[r], out_dtype=dt) for r in range(M)]))
+    finally:
+        gpu_rt.free(proj)

@@ -104,3 +104,25 @@ def test_static_workspace_refuses_the_whole_call(gpu_rt):
         assert bool(torch.isfinite(y[:512]).all()) and bool(torch.isnan(y[512:]).all())
     finally:
         gpu_rt.free(proj)
+
+
+@pytest.mark.parametrize("d_out,d_in,M,off", [(12288, 4097, 512, 0), (8000, 16391, 1024, 0), (6000, 24599, 600, 0), (12288, 4096, 512, 1)])
+def test_static_workspace_takes_rows_off_their_boundaries(gpu_rt, d_out, d_in, M, off):
+    """The limit above is one of rows of a multiple of 8 values on a 16-byte boundary.  Any other rows are taken whatever
+    their number (up to the widest a single-row product takes), with the results of llvq_hip_gemm."""
+    import torch
+
+    raw = synth.make_matrix(f"model.layers.0.static.{d_out}x{d_in}.weight", d_out, d_in, seed=15)
+    proj = gpu_rt.upload(raw)
+    try:
+        buf = torch.empty(M * d_in + 8, dtype=torch.float16, device="cuda")
+        x = buf[off:off + M * d_in].view(M, d_in)
+        x.copy_(torch.randn(M, d_in, generator=torch.Generator().manual_seed(3)).half())
+        want = torch.empty((M, d_out), dtype=torch.float32, device="cuda")
+        got = torch.full_like(want, float("nan"))
+        gpu_rt.forward_batched_into(proj, x, want)
+        gpu_rt.forward_batched_static_into(proj, x, got)
+        gpu_rt.synchronize()
+        assert torch.equal(got, want)
+    finally:
+        gpu_rt.free(proj)
