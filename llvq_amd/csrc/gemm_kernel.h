@@ -671,10 +671,12 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
 #pragma unroll
         for (int e = 0; e < 16; ++e) v[e] = PAIR ? 0.f : acc[k][c][e] * scale[e];
         for (uint32_t i = 0; i < a.tail_w; i += 2u) {
-          const uint32_t col = min(i + he, a.tail_w - 1u);
-          const float keep = i + he < a.tail_w ? 1.f : 0.f;
-          v = __builtin_amdgcn_mfma_f32_32x32x2f32(keep * w_tail[col * kWideRows + wave * 64u + (uint32_t)k * 32u + l32e],
-                                                   x_tail[col * kCols + (uint32_t)c * 32u + l32e], v, 0, 0, 0);
+          // (Without PAIR they are an even number.  With it a column past the last is zero in both operands: zero times the last
+          // one again is not zero where that is infinite.)
+          const uint32_t col = PAIR ? min(i + he, a.tail_w - 1u) : i + he;
+          const bool there = !PAIR || i + he < a.tail_w;
+          const float tw = w_tail[col * kWideRows + wave * 64u + (uint32_t)k * 32u + l32e], tx = x_tail[col * kCols + (uint32_t)c * 32u + l32e];
+          v = __builtin_amdgcn_mfma_f32_32x32x2f32(there ? tw : 0.f, there ? tx : 0.f, v, 0, 0, 0);
         }
         if constexpr (PAIR) {
 #pragma unroll

@@ -144,3 +144,34 @@ def test_rotated_rows_off_their_boundaries_go_one_by_one(gpu_rt, n, M, off):
             assert torch.equal(y, torch.stack([gpu_rt.forward(proj, x[r], out_dtype=dt) for r in range(M)]))
     finally:
         gpu_rt.free(proj)
+
+
+# A row that is not finite spoils itself and no other, whatever repeats or pads it: the last row of a batch and one inside,
+# in a block's column and in the last tail column (odd and even tails), through each of the kernels.
+@pytest.mark.parametrize("nb,tail,d_out,M", [(9, 8, 40, 5), (9, 7, 40, 5), (70, 16, 50, 60), (70, 1, 50, 60), (9, 16, 300, 300), (9, 23, 300, 300),
+                                             (65, 8, 257, 70), (65, 5, 257, 70)])
+def test_rows_that_are_not_finite_spoil_no_others(gpu_rt, nb, tail, d_out, M):
+    import torch
+
+    d_in = nb * 24 + tail
+    raw = synth.make_matrix(f"model.layers.0.tiles.{d_out}x{d_in}.weight", d_out, d_in, seed=nb)
+    X = _x16(synth.make_activation(d_in, seed=M, rows=M))
+    proj = gpu_rt.upload(raw)
+    try:
+        for dt in (torch.float32, torch.float16):
+            clean = gpu_rt.forward_batched(proj, X, out_dtype=dt)
+            assert bool(torch.isfinite(clean).all())
+            for column, value in ((nb * 24 - 1, float("inf")), (3, float("nan")), (d_in - 1, float("-inf")), (d_in - 1, float("nan"))):
+                bad = [M // 3, M - 1]
+                x = X.clone()
+                x[bad, column] = value
+                y = gpu_rt.forward_batched(proj, x, out_dtype=dt)
+                good = [r for r in range(M) if r not in bad]
+                assert torch.equal(y[good], clean[good]), (column, value)
+                if column == d_in - 1 and value < 0:  # an infinite value in f32 columns: infinite by the weight's sign
+                    want = -np.sign(raw.tail.reshape(d_out, tail)[:, -1]) * np.inf
+                    assert np.array_equal(y[bad].double().cpu().numpy(), np.broadcast_to(want, (2, d_out)))
+                else:
+                    assert not bool(torch.isfinite(y[bad]).any())
+    finally:
+        gpu_rt.free(proj)
