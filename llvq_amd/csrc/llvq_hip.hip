@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -491,7 +492,10 @@ struct llvq_rt {
   // a batch's activations in K-step tiles [n_steps, m_pad, 32] (pipelined batched kernel)
   __half* gemm_xt = nullptr;
   size_t gemm_xt_bytes = 0;
-  // where an upload's code stream lands before it is unranked into a matrix's tiles (at most kUploadBytes of codes)
+  // Uploads may come from several threads; launches come from one (llvq_hip.h).  Held while an upload uses what follows
+  // and `rotations`.
+  std::mutex uploads;
+  // where an upload's codes, scales and tail land before they become a matrix's tiles (kUploadBytes at most, kept for the next)
   uint8_t* upload_buf = nullptr;
   size_t upload_bytes = 0;
 };
@@ -668,7 +672,7 @@ int llvq_hip_synchronize(llvq_rt* rt) {
 }
 
 // The device tables of rotation (n, seed), built once per runtime.  Also makes
-// sure the f32 scratch holds n values.
+// sure the f32 scratch holds n values.  Called with rt->uploads held.
 static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_rt::DevRotation** out) {
   for (auto* r : rt->rotations)
     if (r->n == n && r->seed == seed) { *out = r; return LLVQ_OK; }
@@ -727,14 +731,14 @@ static hipError_t grow_device(uint8_t** buf, size_t* have, size_t need) {
   return e;
 }
 
-// Code stream, scales and tail -> the matrix's tiles (tiles.h), through the runtime's staging buffer, kUploadRows worth
-// of code bytes at a time.  Blocks until done: the host arrays may go, and the staging buffer is free for the next one.
+// Code stream, scales and tail -> the matrix's tiles (tiles.h), through the runtime's staging buffer, kUploadBytes of them
+// at a time.  Blocks until done: the host arrays may go, and the staging buffer is free for the next one.  Called with
+// rt->uploads held: another upload's copies between this one's and its kernels would end up in this matrix.
 constexpr size_t kUploadBytes = 32u << 20;
 static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids, const float* rscale, const float* tail, const uint8_t* codes) {
   const uint32_t nb = m->nblocks, stride = tile_stride(nb, m->tail_w), n_tiles = tile_count(m->d_out);
   const size_t row_bits = (size_t)nb * m->record_bits;  // eight rows are whole bytes whatever the record width
-  uint32_t rows_per = row_bits ? (uint32_t)std::min<size_t>(m->d_out, std::max<size_t>(8, kUploadBytes * 8 / row_bits / 8 * 8)) : m->d_out;
-  rows_per = std::min(rows_per, (1u << 20));
+  const uint32_t rows_per = (uint32_t)std::min<size_t>(m->d_out, std::max<size_t>(8, kUploadBytes * 8 / (row_bits + 32u * (1u + m->tail_w)) / 8 * 8));
   TileTable table;
   for (uint32_t i = 0; i < 32; ++i) {
     const uint32_t shell = i & 15u;
@@ -767,7 +771,13 @@ static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  return hipStreamSynchronize(rt->stream);
+  e = hipStreamSynchronize(rt->stream);
+  if (rt->upload_bytes > kUploadBytes + 1024) {  // eight rows that exceed it by themselves: not kept
+    (void)hipFree(rt->upload_buf);
+    rt->upload_buf = nullptr;
+    rt->upload_bytes = 0;
+  }
+  return e;
 }
 
 static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uint32_t d_in,
@@ -811,6 +821,7 @@ static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uin
   }
 
   HIP_TRY(hipSetDevice(rt->device));
+  std::lock_guard<std::mutex> one_at_a_time(rt->uploads);
   const llvq_rt::DevRotation* rot = nullptr;
   if (has_rotation) {
     const int rc = runtime_rotation(rt, d_in, rotation_seed, &rot);

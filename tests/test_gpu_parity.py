@@ -420,3 +420,48 @@ def test_full_size_properties_linearity_and_scaling(gpu_rt):
     if bool(exact.all()):
         assert torch.allclose(yz, lin, rtol=1e-4, atol=1e-6)
     gpu_rt.free(proj)
+
+
+def test_uploads_from_several_threads(gpu_rt):
+    """Uploads to one runtime may come from several threads at once (ctypes gives up the interpreter's lock for the call):
+    every matrix gets its own codes, scales, tail and rotation, as the same matrices uploaded one after the other show."""
+    import threading
+
+    import torch
+
+    shapes = [(600, 2560), (1000, 1040), (64, 401), (3000, 256)]
+    x = {d: _x16(synth.make_activation(d, seed=d)[0]) for _, d in shapes}
+    mats = []
+    for t in range(4):
+        mats.append([synth.make_matrix(f"model.layers.{t}.threads{k}.weight", do, di, seed=10 * t + k) for k, (do, di) in enumerate(shapes)])
+        for k in (0, 3):  # (widths that rotate)
+            mats[t][k].rotation_seed = 1000 + 10 * t + k if t % 2 else None
+    got, errors = [[] for _ in mats], []
+    start = threading.Barrier(len(mats))
+
+    def work(t):
+        try:
+            start.wait()
+            for _ in range(6):
+                got[t] += [gpu_rt.upload(m) for m in mats[t]]
+        except Exception as e:  # noqa: BLE001 (shown below)
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(len(mats))]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    try:
+        assert not errors, errors
+        for t, layer in enumerate(mats):
+            for k, m in enumerate(layer):
+                alone = gpu_rt.upload(m)
+                want = gpu_rt.forward(alone, x[m.d_in], out_dtype=torch.float32)
+                gpu_rt.free(alone)
+                for p in got[t][k::len(shapes)]:
+                    assert torch.equal(gpu_rt.forward(p, x[m.d_in], out_dtype=torch.float32), want), (t, k)
+    finally:
+        for ps in got:
+            for p in ps:
+                gpu_rt.free(p)
