@@ -472,18 +472,17 @@ struct llvq_rt {
   uint8_t* static_scratch = nullptr;  // this device's copy of `scratch` (kStaticScratchBytes)
   GlobalTables tables{};
   int cu_count = 0;
-  // rotations by (width, seed) — shared by every matrix that consumes the same activation
-  // (llvq-llm/src/fused.rs:672-674) — and the scratch rotated activations land in
+  // rotations by (width, seed), shared by every matrix that consumes the same activation
+  // (llvq-llm/src/fused.rs:672-674); an upload may add one, none is changed or moved while launches use it
   struct DevRotation {
     uint32_t n = 0, m = 0, k = 0;
     uint64_t seed = 0;
     float inv = 1.f;
     uint32_t* signbits = nullptr;
     void* fragments = nullptr;  // [64] RotFragments
+    float* scratch = nullptr;   // one rotated activation, f32, where rows are too wide to be rotated in a product's launch
   };
   std::vector<DevRotation*> rotations;
-  float* rot_scratch = nullptr;   // one rotated activation, f32
-  size_t rot_scratch_elems = 0;
   __half* rot_rows = nullptr;     // rotated batch rows, f16 (matrix-core path)
   size_t rot_rows_bytes = 0;
   // workspace of the batched kernels: partial sums [S, n_bands, M, 64]
@@ -654,12 +653,12 @@ void llvq_hip_runtime_destroy(llvq_rt* rt) {
   (void)hipFree(rt->blob);
   (void)hipFree(rt->gemm_ws);
   (void)hipFree(rt->gemm_xt);
-  (void)hipFree(rt->rot_scratch);
   (void)hipFree(rt->rot_rows);
   (void)hipFree(rt->upload_buf);
   for (auto* r : rt->rotations) {
     (void)hipFree(r->signbits);
     (void)hipFree(r->fragments);
+    (void)hipFree(r->scratch);
     delete r;
   }
   delete rt;
@@ -671,8 +670,12 @@ int llvq_hip_synchronize(llvq_rt* rt) {
   return LLVQ_OK;
 }
 
-// The device tables of rotation (n, seed), built once per runtime.  Also makes
-// sure the f32 scratch holds n values.  Called with rt->uploads held.
+// Whether the digit planes of rows this wide fit LDS beside what else a launch keeps there.
+static bool gemv_fits(uint32_t d_in, bool f32_out, bool rotated) {
+  return d_in / kDim <= kGemvMaxBlocks && gemv_tiles_lds_bytes(d_in / kDim, d_in, f32_out, rotated) <= 160 * 1024;
+}
+
+// The device tables of rotation (n, seed), built once per runtime.  Called with rt->uploads held.
 static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_rt::DevRotation** out) {
   for (auto* r : rt->rotations)
     if (r->n == n && r->seed == seed) { *out = r; return LLVQ_OK; }
@@ -702,13 +705,8 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
   }
   if (e == hipSuccess) e = hipMalloc(&r->fragments, frag.size() * sizeof(RotFragments));
   if (e == hipSuccess) e = hipMemcpy(r->fragments, frag.data(), frag.size() * sizeof(RotFragments), hipMemcpyHostToDevice);
-  if (e == hipSuccess && n > rt->rot_scratch_elems) {
-    (void)hipFree(rt->rot_scratch);
-    rt->rot_scratch = nullptr;
-    rt->rot_scratch_elems = 0;
-    e = hipMalloc(reinterpret_cast<void**>(&rt->rot_scratch), (size_t)n * sizeof(float));
-    if (e == hipSuccess) rt->rot_scratch_elems = n;
-  }
+  // (f32 results have the larger planes: where those fit, all do)
+  if (e == hipSuccess && !gemv_fits(n, true, true)) e = hipMalloc(reinterpret_cast<void**>(&r->scratch), (size_t)n * sizeof(float));
   if (e != hipSuccess) {
     (void)hipFree(r->signbits);
     (void)hipFree(r->fragments);
@@ -978,11 +976,6 @@ struct Prologue {
   float eps = 0.f;
 };
 
-// Whether the digit planes of rows this wide fit LDS beside what else a launch keeps there.
-static bool gemv_fits(const llvq_mat* m, bool f32_out, bool rotated) {
-  return m->nblocks <= kGemvMaxBlocks && gemv_tiles_lds_bytes(m->nblocks, m->d_in, f32_out, rotated) <= 160 * 1024;
-}
-
 // One launch of gemv_tiles_kernel over n <= kMaxGroup matrices of equal d_in and basis.
 static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, void* const* y,
                         int y_dtype, const Prologue* pro = nullptr, const float* x_f32 = nullptr,
@@ -990,7 +983,7 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   const llvq_mat* m0 = mats[0];
   if (y_dtype != LLVQ_F32 && y_dtype != LLVQ_F16) return fail(LLVQ_ERR_INVALID_ARGUMENT, "gemv: unknown output dtype");
   const bool f32 = y_dtype == LLVQ_F32, rotated = rot || x_f32;
-  if (!gemv_fits(m0, f32, rot != nullptr))
+  if (!gemv_fits(m0->d_in, f32, rot != nullptr))
     return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": d_in " + std::to_string(m0->d_in) + " does not fit the LDS activation tile");
   GemvArgs a{};
   a.in.x = reinterpret_cast<const __half*>(x);
@@ -1057,7 +1050,7 @@ static bool same_basis(const llvq_mat* a, const llvq_mat* b) {
 // One activation through projections that share it: consecutive matrices in the
 // same basis go out as one launch (at most kMaxGroup).  A launch in a rotated basis
 // rotates the activation itself (`pro`, when given, derives it first); rows too wide
-// for that get it rotated once, into the runtime's scratch, by a kernel of its own
+// for that get it rotated once, into the rotation's scratch, by a kernel of its own
 // (never together with `pro`: the caller stages the activation first then).
 static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, void* const* y, int y_dtype,
                          const Prologue* pro = nullptr) {
@@ -1066,7 +1059,7 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
     int j = i + 1;
     while (j < n && j - i < kMaxGroup && same_basis(mats[i], mats[j])) ++j;
     const float* xr = nullptr;
-    if (mats[i]->has_rotation && gemv_fits(mats[i], y_dtype == LLVQ_F32, true)) {
+    if (mats[i]->has_rotation && gemv_fits(mats[i]->d_in, y_dtype == LLVQ_F32, true)) {
       const int rc = launch_group(rt, mats + i, j - i, x, y + i, y_dtype, pro, nullptr, mats[i]->rot);
       if (rc) return rc;
       i = j;
@@ -1075,9 +1068,9 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
     if (pro && mats[i]->has_rotation) return fail(LLVQ_ERR_UNSUPPORTED, mats[i]->name + ": prologue with a rotation outside the launch");
     if (mats[i]->has_rotation) {
       // the scratch may still hold this very rotation if the previous run used it; rotating again is cheap and always right
-      const int rc = launch_rotate(rt, mats[i]->rot, x, 1, rt->rot_scratch, false);
+      const int rc = launch_rotate(rt, mats[i]->rot, x, 1, mats[i]->rot->scratch, false);
       if (rc) return rc;
-      xr = rt->rot_scratch;
+      xr = mats[i]->rot->scratch;
     }
     const int rc = launch_group(rt, mats + i, j - i, x, y + i, y_dtype, pro, xr);
     if (rc) return rc;
@@ -1944,7 +1937,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   auto project = [&](const llvq_mat* const* mats, int n, const __half* x, void* const* outs, const Prologue& pro) -> int {
     // every launch of the group can derive (and, in a rotated basis, rotate) the activation itself
     bool fused = true;
-    for (int i = 0; i < n; ++i) fused &= gemv_fits(mats[i], false, mats[i]->has_rotation);
+    for (int i = 0; i < n; ++i) fused &= gemv_fits(mats[i]->d_in, false, mats[i]->has_rotation);
     if (fused) return forward_group(rt, mats, n, x, outs, LLVQ_F16, &pro);
     const __half* staged = nullptr;
     if (pro.kind == kPrologueAddRmsNorm) {

@@ -155,3 +155,29 @@ def test_a_power_of_two_goes_through_a_rotated_product_unchanged(gpu_rt, k, d_in
         assert torch.equal(got.double(), one * 2.0 ** k)
     finally:
         gpu_rt.free(proj)
+
+
+def test_rows_too_wide_to_be_rotated_in_the_launch(gpu_rt, orc):
+    """20 480 columns with f32 results and 24 576 with either do not fit LDS beside their digit planes: the activation is
+    rotated by a kernel of its own, into memory that belongs to the rotation.  An upload between two products (which
+    brings another such rotation) changes nothing about the first."""
+    import torch
+
+    first = _rotated("model.layers.0.wide.0.weight", 9, 20480, 3, 41)
+    x = {n: _x16(synth.make_activation(n, seed=n)[0]) for n in (20480, 24576)}
+    projs = [gpu_rt.upload(first)]
+    try:
+        one = gpu_rt.forward(projs[0], x[20480], out_dtype=torch.float32)
+        projs += [gpu_rt.upload(_rotated("model.layers.0.wide.1.weight", 9, 24576, 4, 42)),
+                  gpu_rt.upload(_rotated("model.layers.0.wide.2.weight", 9, 20480, 5, 43))]
+        for p in projs:
+            for dt in (torch.float32, torch.float16):
+                y = gpu_rt.forward(p, x[p.d_in], out_dtype=dt).reshape(-1)
+                assert torch.equal(y, gpu_rt.forward_rotated(p, gpu_rt.rotate(p, x[p.d_in]), out_dtype=dt).reshape(-1))
+        assert torch.equal(gpu_rt.forward(projs[0], x[20480], out_dtype=torch.float32), one)
+        om, _ = orc.read_matrix_raw(artifact.write_matrix_raw(first))
+        y_ref, a_ref = om.fused_product(synth.make_activation(20480, seed=20480)[0].astype(np.float64))
+        assert (np.abs(one.cpu().numpy().reshape(-1) - y_ref) / a_ref).max() < 1e-5
+    finally:
+        for p in projs:
+            gpu_rt.free(p)
