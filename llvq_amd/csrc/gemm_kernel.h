@@ -404,9 +404,10 @@ static_assert(kWideDepth * gemm_wide_buf<4>() >= (kWideRows + 128u) * kDim * 4u 
 
 // 16 bytes per lane from base + offset to LDS, lane after lane from `lds` on.  In assembly because the compiler, which
 // cannot tell the buffers apart, would have every read of LDS wait for all of these; the counting is done by hand
-// (wide_wait), and there are no other loads in flight where it is.
+// (wide_wait), and there are no other loads in flight where it is.  M0, where the place in LDS goes, is an operand: the
+// compiler writes it, and knows that it did.
 __device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t offset, const uint8_t* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(lds), "v"(offset), "s"(base) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wide_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
