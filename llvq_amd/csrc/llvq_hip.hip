@@ -2092,7 +2092,6 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
   llvq_rt* rt = d->rt;
   hipStream_t st = rt->stream;
   if (d->pos + n > d->max_pos) return fail(LLVQ_ERR_INVALID_ARGUMENT, "decoder_prefill: positions past max_positions");
-  const uint32_t qd = d->n_heads * d->head_dim;
   __half *ph = d->ph, *ph_alt = d->ph_alt;  // by local name: a pass that fails part-way leaves the decoder as it found it
   if (d->embed_q8)
     hipLaunchKernelGGL(embed_q8_kernel, dim3((d->hidden + 255) / 256, n), dim3(256), 0, st, d->embed_q, d->ptokens, 0u, d->vocab, d->hidden, ph);
@@ -2183,7 +2182,6 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
   }
   HIP_TRY(hipGetLastError());
   d->pos += n;
-  (void)qd;
   return LLVQ_OK;
 }
 

@@ -257,7 +257,6 @@ __device__ __forceinline__ GemvLds gemv_lds(uint8_t* smem, uint32_t plane_blocks
   return L;
 }
 
-struct __attribute__((packed, aligned(4))) FloatOctet { float v[8]; };
 __device__ __forceinline__ float round_half(float v) { return __half2float(__float2half_rn(v)); }
 __device__ __forceinline__ float silu_mul(float gate, float up) { return round_half(round_half(gate / (1.0f + __expf(-gate))) * up); }
 
