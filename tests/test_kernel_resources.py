@@ -58,3 +58,15 @@ def test_the_batched_kernel_does_not_spill_either(usage):
     for name, u in gemm.items():
         assert u["ScratchSize"] == 0, (name, u)
         assert u["VGPRs"] + u.get("AGPRs", 0) <= 128, (name, u)
+
+
+def test_the_wide_batched_kernel_keeps_its_workgroups_on_a_cu(usage):
+    """Four wavefronts to a workgroup, one on each SIMD: two workgroups share a CU's 512 registers a lane where a tile has
+    128 activation rows, one has them for itself at 256 rows or with both terms of the weights."""
+    wide = {k: v for k, v in usage.items() if "gemm_wide_kernel" in k}
+    bound = {"ILi4ELb0E": 256, "ILi4ELb1E": 512, "ILi8ELb0E": 512}
+    assert len(wide) == len(bound)
+    for name, u in wide.items():
+        limit = next(v for k, v in bound.items() if k in name)
+        assert u["ScratchSize"] == 0 and u["VGPRs"] + u.get("AGPRs", 0) <= limit, (name, u)
+        assert u["Occupancy"] >= 512 // limit, (name, u)
