@@ -1421,12 +1421,14 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
   }
   // The form and the column splits by the time they should take: rounds of resident workgroups times steps of a
   // workgroup's share of a CU, and for the splits what the partial sums cost on their way through memory.
-  const uint32_t steps = (nb + 1u) / 2u;
+  // (Rows of a multiple of 8 values that lie off a boundary are not split: what is reserved for such matrices at their usual
+  // place holds the octets of either plan, and needs no partial sums for rows that hardly ever come.)
+  const uint32_t steps = (nb + 1u) / 2u, most = pair && mats[0]->d_in % 8 == 0 ? 1u : 16u;
   double best = 1e30;
   for (uint32_t cf = pair ? 4u : 8u; cf >= 4u; cf -= 4u) {
     const uint32_t m_tiles = (M + 32u * cf - 1u) / (32u * cf), tiles = p.n_tiles * m_tiles, m_pad = m_tiles * 32u * cf;
     const size_t one = (size_t)m_pad * p.n_tiles * kWideRows * sizeof(float);
-    for (uint32_t sp = 1; sp <= 16u && (sp == 1u || (steps / sp >= 8u && one * sp <= kGemmWsCap)); ++sp) {
+    for (uint32_t sp = 1; sp <= most && (sp == 1u || (steps / sp >= 8u && one * sp <= kGemmWsCap)); ++sp) {
       const uint32_t per = (steps + sp - 1u) / sp, wgs = tiles * ((steps + per - 1u) / per), per_cu = (wgs + cus - 1u) / cus;
       const double cost = (pair ? per_cu * kWidePairStep : cf == 8u ? per_cu * kWideStep : per_cu == 1u ? kWideHalfStepAlone : per_cu * kWideHalfStep) * per +
                           (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
@@ -1459,16 +1461,14 @@ static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint
     bool six_byte = true;
     for (int i = i0; i < i1; ++i) six_byte &= mats[i]->record_bits == 48;
     if (mats[i0]->nblocks && six_byte) {  // (cap-13 matrices take the row loop, which has no workspace)
-      for (const bool pair : {false, true}) {
-        if (pair ? mats[i0]->has_rotation : mats[i0]->d_in % 8 != 0) continue;  // no call takes it (gemm_same_basis)
-        const uint32_t chunk = std::min(max_rows, gemm_chunk(mats[i0]->nblocks, pair));
-        // every row count up to the chunk: the splits, and so the partial sums, are not monotone in it
-        for (uint32_t M = 16;; M = M < 64u ? M + 48u : M < 128u ? 128u : M + 128u) {
-          const GemmPlan p = gemm_plan(rt, mats + i0, i1 - i0, M < chunk ? M : chunk, pair);
-          ws = p.ws_bytes > ws ? p.ws_bytes : ws;
-          xt = p.xt_bytes > xt ? p.xt_bytes : xt;
-          if (M >= chunk) break;
-        }
+      const bool pair = mats[i0]->d_in % 8 != 0;
+      const uint32_t chunk = std::min(max_rows, gemm_chunk(mats[i0]->nblocks, pair));
+      // every row count up to the chunk: the splits, and so the partial sums, are not monotone in it
+      for (uint32_t M = 16;; M = M < 64u ? M + 48u : M < 128u ? 128u : M + 128u) {
+        const GemmPlan p = gemm_plan(rt, mats + i0, i1 - i0, M < chunk ? M : chunk, pair);
+        ws = p.ws_bytes > ws ? p.ws_bytes : ws;
+        xt = p.xt_bytes > xt ? p.xt_bytes : xt;
+        if (M >= chunk) break;
       }
     }
     if (mats[i0]->has_rotation) {

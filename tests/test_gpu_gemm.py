@@ -344,3 +344,29 @@ def test_reserved_workspaces_change_nothing(gpu_rt):
     finally:
         for p in projs:
             gpu_rt.free(p)
+
+
+def test_reserved_workspaces_hold_rows_off_their_boundaries(gpu_rt):
+    """Rows whose first value lies off a 16-byte boundary, and rows of an odd length, take device memory no more than others
+    once llvq_hip_reserve_batched has been told of the group."""
+    import torch
+
+    rt = type(gpu_rt)(device=0)  # a runtime that has reserved nothing yet
+    projs = [rt.upload(synth.make_matrix(f"model.layers.0.reserve.off.{d_in}.weight", 200, d_in, seed=50)) for d_in in (4096, 4097)]
+    try:
+        for p in projs:
+            rt.reserve_batched([p], 700)
+        buf = torch.randn(700 * 4097 + 8, device="cuda").half()
+        ys = {M: torch.empty((M, 200), dtype=torch.float32, device="cuda") for M in (700, 300, 130, 40, 5)}
+        rt.synchronize()
+        free_before = torch.cuda.mem_get_info()[0]
+        for p in projs:
+            for off in (0, 1):
+                for M, y in ys.items():
+                    rt.forward_batched_into(p, buf[off:off + M * p.d_in].view(M, p.d_in), y)
+        rt.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free_before
+    finally:
+        for p in projs:
+            rt.free(p)
+        rt.close()
