@@ -681,7 +681,11 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
         }
         if constexpr (PAIR) {
 #pragma unroll
-          for (int e = 0; e < 16; ++e) v[e] = fmaf(acc[k][c][e], scale[e], v[e]);
+          for (int e = 0; e < 16; ++e) {
+            float y = fmaf(acc[k][c][e], scale[e], v[e]);
+            asm("" : "+v"(y));  // (an f32 value in every store: where they convert one by one it would be one operation, rounded once)
+            v[e] = y;
+          }
         }
         const uint32_t m = m0 + (uint32_t)c * 32u;
         if (m < a.M) decltype(to)::store(t.y, (size_t)m * t.d_out, row, he, t.d_out, v);

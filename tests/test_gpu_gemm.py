@@ -370,3 +370,26 @@ def test_reserved_workspaces_hold_rows_off_their_boundaries(gpu_rt):
         for p in projs:
             rt.free(p)
         rt.close()
+
+
+@pytest.mark.parametrize("d_in", [480, 488, 489])  # weights of one term without and with a tail, of two; 20 blocks: not split over columns
+@pytest.mark.parametrize("d_out,M", [(1024, 70), (9000, 300), (1020, 130), (1022, 130)])  # whole tiles, and rows of y on 8 and 4 bytes
+def test_gemm_wide_stores_into_an_output_that_is_only_element_aligned(gpu_rt, d_in, d_out, M):
+    """The wide kernel stores sixteen bytes a lane where y and its rows lie on such boundaries and one value at a time where
+    they do not: the same bits either way, and nothing outside y."""
+    import torch
+
+    proj = gpu_rt.upload(synth.make_matrix("model.layers.3.self_attn.v_proj.weight", d_out, d_in, seed=4))
+    try:
+        X = _x16(synth.make_activation(d_in, seed=6, rows=M))
+        for dt in (torch.float16, torch.float32):
+            want = gpu_rt.forward_batched(proj, X, out_dtype=dt)
+            buf = torch.full((M * d_out + 8,), float("nan"), dtype=dt, device="cuda")
+            y = buf[1:1 + M * d_out].view(M, d_out)
+            assert y.data_ptr() % 16 != 0
+            gpu_rt.forward_batched_into(proj, X, y)
+            gpu_rt.synchronize()
+            assert torch.equal(y, want)
+            assert bool(torch.isnan(buf[0])) and bool(torch.isnan(buf[1 + M * d_out:]).all())
+    finally:
+        gpu_rt.free(proj)
