@@ -61,8 +61,8 @@ def test_gemv_cap13_matches_the_oracle(gpu_rt, orc, d_out, d_in):
 
 
 def test_gemv_cap13_kernel_unranks_every_coordinate_exactly(gpu_rt, orc, boundary_indices):
-    """One-hot activations read a cap-13 matrix back column by column through the product kernel's own stream
-    extraction, class find and decoders: all 24 coordinates of 61 440 blocks — every class boundary of the ball,
+    """One-hot activations read a cap-13 matrix back column by column, as the products read it from the layout that an
+    upload unranks its dense stream into: all 24 coordinates of 61 440 blocks — every class boundary of the ball,
     uniform draws over it (60 % of them on shell 13), origins, both gain bits — are the oracle's integers."""
     import torch
 
@@ -96,8 +96,8 @@ def test_gemv_cap13_kernel_unranks_every_coordinate_exactly(gpu_rt, orc, boundar
 
 
 def test_cap13_groups_rotation_and_batched_rows(gpu_rt, orc):
-    """A group of cap-13 matrices in one call; a call that mixes caps (one launch per cap); a cap-13 matrix stored
-    in a rotated basis (a kernel of its own rotates the activation); batched rows (a loop over the rows' products)."""
+    """A group of cap-13 matrices in one call; a call that mixes caps; a cap-13 matrix stored
+    in a rotated basis; batched rows (a loop over the rows' products)."""
     import torch
 
     mk = lambda name, do, cap: synth.make_matrix(f"model.layers.1.{name}.weight", do, 2560, seed=6, shell_cap=cap)

@@ -3,8 +3,9 @@ CPU oracle: Y = X W^T with W the oracle's decoded matrix, in f64.
 
 Bar: |y - y_ref| / sum|w_i x_i| < 1e-3.  Weights enter the matrix cores as
 binary16 (one rounding of value * centroid / sqrt(16 shell), 2^-11 relative per
-weight), accumulation is f32; row scale and tail columns are applied in f32.
-That rounding is of the order of 1e-4 of sum|w_i x_i|, so the plain relative
+weight) where rows are a multiple of 8 values from a 16-byte boundary on, as all rows
+here are (test_gpu_tiles.py has the others); accumulation is f32; row scale and tail
+columns are applied in f32.  That rounding is of the order of 1e-4 of sum|w_i x_i|, so the plain relative
 error of an output is below 1e-3 only where the sum does not cancel
 (|y_ref| >= 0.2 sum|w_i x_i|); both are asserted.
 """
@@ -44,25 +45,26 @@ def _check(Y, Y_ref, A_ref, tol=TOL, out_rounding=0.0):
     return e.max()
 
 
-# d_in must keep activation rows 16-byte aligned (d_in % 8 == 0) for the matrix-core path
+# d_in % 8 == 0: weights of one term
 CASES = [
-    # d_out, d_in, M.  A K-slice is 16 blocks per row; up to 256 activation rows four wavefronts
-    # multiply (64-row tiles, the wavefronts left over share a tile's K-steps), beyond that eight.
-    (64, 480, 16),      # one band, one full and one short K-slice, no tail
-    (72, 184, 16),      # ragged band (72 = 64 + 8), 7 blocks + 16 tail columns
-    (8, 2560, 2),       # tiny band, smallest batch
+    # d_out, d_in, M.  Up to 16 activation rows a workgroup takes 16 weight rows, up to 64 it takes 32 and sixteen
+    # wavefronts share the columns four blocks at a time; beyond that a tile is 256 weight rows by 128 or 256
+    # activation rows and a step two blocks.
+    (64, 480, 16),      # 20 blocks, no tail; a whole tile of activation rows
+    (72, 184, 16),      # ragged rows (72 = 64 + 8), 7 blocks + 16 tail columns
+    (8, 2560, 2),       # half a tile of weight rows, smallest batch
     (128, 2568, 17),    # ragged batch, tail
     (256, 4096, 64),    # 8B hidden size: 170 blocks + 16 tail
-    (64, 384, 65),      # exactly one slice; two 64-row tiles, the second with one row
-    (192, 976, 130),    # three tiles on four multiplying wavefronts: one of them idles
-    (64, 416, 129),     # 17 blocks: a full slice and a slice of one block
-    (64, 1000, 256),    # the widest batch of the four-wavefront variant
-    (64, 376, 257),     # the narrowest of the eight-wavefront variant: 15 blocks, five tiles
-    (320, 800, 300),    # 33 blocks = two full slices and one block; five tiles, three wavefronts idle
-    (19000, 80, 257),   # 297 bands on 256 CUs: workgroups walk several units, short slices throughout
-    (128, 4096, 512),   # eight tiles
+    (64, 384, 65),      # the smallest batch of the wide kernel, a quarter of its weight rows
+    (192, 976, 130),
+    (64, 416, 129),     # 17 blocks: a step of one block
+    (64, 1000, 256),
+    (64, 376, 257),     # 15 blocks
+    (320, 800, 300),    # two tiles of weight rows, the second a quarter full
+    (19000, 80, 257),   # more tiles than CUs, two steps each
+    (128, 4096, 512),
     (64, 376, 511),
-    (64, 488, 600),     # more rows than one launch holds
+    (64, 488, 600),
 ]
 
 
@@ -157,7 +159,8 @@ def test_gemm_matches_gemv_rows(gpu_rt):
 def test_gemm_into_an_output_that_is_only_element_aligned(gpu_rt, M):
     """y as a view one element into a larger buffer (2 bytes off for binary16, 4 for f32): the kernels
     group four results into one store only where y keeps that alignment, and the bits are those of an
-    aligned output either way.  48 rows finish through the partial sums, 512 also inside the launch."""
+    aligned output either way.  48 rows finish in the narrow kernel, 512 of this width through the sum of column splits
+    (the wide kernel's own stores: test_gemm_wide_stores_into_an_output_that_is_only_element_aligned)."""
     import torch
 
     raw = synth.make_matrix("model.layers.3.self_attn.v_proj.weight", 1024, 2560, seed=4)
@@ -178,10 +181,10 @@ def test_gemm_into_an_output_that_is_only_element_aligned(gpu_rt, M):
 
 
 @pytest.mark.parametrize("site,d_out,d_in,M", [
-    ("self_attn.k_proj", 1024, 4096, 64),     # few bands: the block range is split over units
+    ("self_attn.k_proj", 1024, 4096, 64),     # few tiles: sixteen wavefronts share the columns of each
     ("mlp.down_proj", 4096, 12288, 16),
     ("mlp.gate_proj", 12288, 4096, 256),
-    ("self_attn.o_proj", 4096, 4096, 512),    # eight consumer wavefronts, bands shared between workgroups
+    ("self_attn.o_proj", 4096, 4096, 512),    # the columns are split over workgroups
     ("mlp.down_proj", 4096, 12288, 512),
 ])
 def test_gemm_qwen3_8b_shapes(gpu_rt, orc, site, d_out, d_in, M):
@@ -200,8 +203,8 @@ def test_gemm_qwen3_8b_shapes(gpu_rt, orc, site, d_out, d_in, M):
 
 
 def test_gemm_2048_rows_in_chunks(gpu_rt, orc):
-    """More activation rows than one launch holds: four launches of 512 rows, each row of the
-    result against the oracle's on a sample that touches every chunk and its ends."""
+    """More activation rows than one launch holds: two launches of 1024 rows, each row of the
+    result against the oracle's on a sample that touches both and their ends."""
     import torch
 
     d_out, d_in, M = 1024, 4096, 2048
@@ -223,13 +226,13 @@ def test_gemm_2048_rows_in_chunks(gpu_rt, orc):
 
 
 def test_gemm_partial_sums_of_the_call_before_do_not_leak(gpu_rt, orc):
-    """Bands that several workgroups share are summed from a workspace.  Two matrices of one shape
+    """Column splits are summed from a workspace.  Two matrices of one shape
     take turns, so the workspace holds the other one's partial sums at the same addresses whenever a
     call starts: every result must be that of the first call, bit for bit, and the first calls are
     checked against the oracle."""
     import torch
 
-    d_out, d_in, M = 4096, 4096, 256  # 64 bands of 11 slices over 256 workgroups: every band has several pieces
+    d_out, d_in, M = 4096, 4096, 256  # 16 tiles of 256 rows for 256 CUs: the columns are split
     raws = [synth.make_matrix(f"model.layers.{i}.self_attn.o_proj.weight", d_out, d_in, seed=60 + i) for i in range(2)]
     Xs = [synth.make_activation(d_in, seed=70 + i, rows=M) for i in range(2)]
     projs = [gpu_rt.upload(r) for r in raws]
@@ -283,15 +286,12 @@ def test_gemm_group_matches_the_oracle_and_the_single_calls(gpu_rt, orc):
 
 @pytest.mark.parametrize("M", [130, 257])
 def test_gemm_bands_finished_in_the_launch(gpu_rt, orc, M):
-    """More 64-row bands than workgroups: every workgroup walks whole bands alone and, where each
-    multiplying wavefront owns a tile's every K-step (M > 128), finishes them in the launch — row scale,
-    f32 tail, store — while the bands left over go through the workspace and the sum pass.  Three matrices
-    in one call (299 bands, the first 256 walked alone), so that a short last band (6 rows), row counts
-    that are no multiple of four (scalar stores) and tail columns all meet the in-launch epilogue, and a
-    57-row band the sum pass; f32 and f16 outputs against the oracle."""
+    """Too few columns to split: every tile of the wide kernel is finished in the launch (row scale, f32 tail,
+    store).  Three matrices in one call, so that short last tiles, row counts that are no multiple of four (stores
+    one by one) and tail columns all meet that end; f32 and f16 outputs against the oracle."""
     import torch
 
-    d_in = 88  # three blocks and 16 tail columns: one slice per band
+    d_in = 88  # three blocks and 16 tail columns: two steps
     d_outs = [70, 16441, 2500]
     raws = [synth.make_matrix(f"model.layers.0.alone{i}.weight", d, d_in, seed=80 + i) for i, d in enumerate(d_outs)]
     X = synth.make_activation(d_in, seed=M, rows=M)

@@ -184,10 +184,8 @@ def _matrix_of_classes(ranges, d_out, nb, seed, name):
 
 
 def test_gemv_tiles_full_of_rare_class_blocks(gpu_rt, orc):
-    """Every block from a class that takes the generic walk.  2560 rows of 40 blocks make tiles of ten rows:
-    400 such blocks in a tile, six times what the kernel's two side queues for them hold, so the overflow
-    path (the blocks ride in the odd queue, flagged) runs in every tile.  Uniform draws meet these classes
-    0.07 % of the time."""
+    """Every block from a class that the unranking at upload takes the generic walk for; uniform draws meet these
+    classes 0.07 % of the time."""
     import torch
 
     ranges = _class_ranges(orc, _is_rare)
@@ -209,10 +207,9 @@ def test_gemv_tiles_full_of_rare_class_blocks(gpu_rt, orc):
 
 @pytest.mark.parametrize("share", [1.0, 0.5])
 def test_gemv_tiles_full_of_second_free_kind_blocks(gpu_rt, orc, share):
-    """Even-coset classes whose off-support slots hold two magnitudes besides zero have a decoder and a
-    384-slot queue of their own (6 to 8 % of uniform draws, about 300 of a full tile).  2560 rows of 100 blocks
-    make tiles of 1000 blocks: with every block from such a class 616 of them overflow into the even queue,
-    flagged, in every tile; with half of them plain even-coset blocks the even queue's chunks mix the two."""
+    """Even-coset classes whose off-support slots hold two magnitudes besides zero have a decoder of their own (6 to
+    8 % of uniform draws): every block from such a class, and half of them plain even-coset blocks, so that a wavefront
+    mixes the two."""
     import torch
 
     second = _class_ranges(orc, lambda odd, w, vals: not odd and not _is_rare(odd, w, vals)
@@ -238,8 +235,8 @@ def test_gemv_tiles_full_of_second_free_kind_blocks(gpu_rt, orc, share):
 
 
 def test_gemv_kernel_unranks_every_coordinate_exactly(gpu_rt, orc, boundary_indices):
-    """The lattice points as the product kernels themselves unrank them (their own class find, queues and
-    decoders, not the probe kernel's): one-hot activations read the matrix back column by column, and
+    """The lattice points as the products read them from the layout that an upload unranks them into (not the probe
+    kernel's): one-hot activations read the matrix back column by column, and
     every one of the 24 coordinates of 163 840 blocks must be the oracle's integer — class boundaries,
     the rare classes, the classes with a second free kind, uniform cap-12 ranks and ranks over the whole
     47-bit field (shell 13), origins, both gain bits."""
@@ -274,7 +271,7 @@ def test_gemv_kernel_unranks_every_coordinate_exactly(gpu_rt, orc, boundary_indi
         eye = torch.eye(nb * 24, dtype=torch.float16, device="cuda")
         cols = [gpu_rt.forward(proj, eye[c], out_dtype=torch.float32).reshape(-1) for c in range(nb * 24)]
         W = torch.stack(cols).t().contiguous().cpu().numpy().astype(np.float64)  # [d_out, d_in]
-        # the batched kernel's producers unrank on their own: the identity as 960 activation rows reads the matrix back too
+        # the batched kernel unpacks that layout on its own: the identity as 960 activation rows reads the matrix back too
         Wb = gpu_rt.forward_batched(proj, eye, out_dtype=torch.float32).t().contiguous().cpu().numpy().astype(np.float64)
     finally:
         gpu_rt.free(proj)

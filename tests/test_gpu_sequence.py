@@ -67,8 +67,8 @@ def test_independent_items_match_the_separate_calls(gpu_rt, orc, out, widest):
 
 
 def test_hostile_tiles_through_the_sequence(gpu_rt, orc):
-    """Tiles full of generic-class blocks (the side queues overflow), of second-free-kind blocks (their queue
-    overflows) and of origins, one item each, against the separate calls bit for bit."""
+    """Matrices full of generic-class blocks, of second-free-kind blocks and of origins, one item each, against the
+    separate calls bit for bit."""
     import torch
 
     rare = _matrix_of_classes(_class_ranges(orc, _is_rare), 1280, 40, 11, "model.layers.0.rare.weight")

@@ -120,8 +120,8 @@ def test_batched_rows_off_their_boundaries_are_as_good_as_single_rows(gpu_rt, or
     assert error(single, Y_ref[rows]) < 8 * 2.0 ** -24
     assert error(Y32, Y_ref) < 8 * 2.0 ** -24
     assert torch.equal(Y32, again)
-    # the same sums, to the nearest binary16: half a unit in the last place, 2^-11 of the value (and 2^-25 below the normal
-    # range), and a rounding of the f32 sum itself, which a fused conversion does not have
+    # the same sums to the nearest binary16: half a unit in the last place, 2^-11 of the value (and 2^-25 below the normal
+    # range), and a rounding of the f32 sum itself, which a conversion fused with the last operation does not have
     off16 = (Y16.double() - Y32.double()).abs()
     assert bool((off16 <= (2.0 ** -11 + 2.0 ** -23) * Y32.double().abs() + 2.0 ** -25).all())
 

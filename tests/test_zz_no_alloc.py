@@ -2,7 +2,7 @@
 memory — against llvq_hip_gemm, through the C ABI.
 
 Both entry points run the same kernels, so the outputs must be identical bit for bit; the
-static one takes its partial sums, tiled activations and rotated rows from a static device
+static one takes its partial sums, the activations' octets and rotated rows from a static device
 array that keeps the previous call's contents, which is why the second call here is the
 smaller one.  Run last: a failure here must not hide the other tests.
 """
@@ -65,7 +65,7 @@ def test_static_workspace_matches_the_allocating_entry_point(gpu_rt, rotated):
 def test_static_workspace_refuses_what_does_not_fit(gpu_rt):
     import torch
 
-    # 12288 x 4096 at 512 rows needs several hundred MB of partial sums
+    # 12288 x 4096 at 512 rows: beyond the limit the entry point was specified with
     raw = synth.make_matrix("model.layers.0.static.wide.weight", 12288, 4096, seed=13)
     proj = gpu_rt.upload(raw)
     try:
@@ -84,9 +84,8 @@ def test_static_workspace_refuses_what_does_not_fit(gpu_rt):
 
 
 def test_static_workspace_refuses_the_whole_call(gpu_rt):
-    """Rows beyond 512 go out as further launches, and a short last one can need more partial sums than a
-    full one (its consumers split the K-steps): 17000 x 4096 at 576 rows fits its first 512 and not its last
-    64.  The call is refused before anything is enqueued, so no row of y is written."""
+    """The limit is one of 512 rows at a time, and a short last part can need more by it than a full one: 17000 x
+    4096 at 576 rows fits its first 512 and not its last 64.  The call is refused before anything is enqueued, so no row of y is written."""
     import torch
 
     raw = synth.make_matrix("model.layers.0.static.uneven.weight", 17000, 4096, seed=14)
