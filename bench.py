@@ -333,7 +333,7 @@ def measure_gemm(args, torch, llvq_amd, synth, dev, M, n_layers, steps, warmup):
         "blocks_per_s": round(n_blocks * steps / wall, 1),
         "per_shape": per_shape,
         "roofline": {
-            "kernel": "gemm_tiles_kernel",
+            "kernel": "gemm_tiles_kernel" if args.M <= 64 else "gemm_wide_kernel",
             "bound": "mfma",
             "achieved": round(flops * steps / dev_s / 1e12, 2),
             "peak": MFMA_F16_PEAK_TFLOPS,

@@ -57,7 +57,7 @@ typedef struct llvq_mat llvq_mat; /* replaces FusedProj     (fused_cuda.rs:119-1
  * stream at cap 13, format.rs:87-89). All pointers are host memory.
  * Cap 12 and cap 13 are accepted; other caps are refused by name
  * (LLVQ_ERR_UNSUPPORTED).  A cap-13 matrix is served by llvq_hip_gemv,
- * llvq_hip_gemv_group (a call may mix caps: one launch per cap), llvq_hip_rotate /
+ * llvq_hip_gemv_group (a call may mix caps), llvq_hip_rotate /
  * llvq_hip_gemv_rotated, llvq_hip_sequence_* (the matrices of one sequence share
  * their cap), the decode loop and, as a loop over its rows, by llvq_hip_gemm /
  * llvq_hip_gemm_group and the batched prompt path. */
@@ -91,7 +91,9 @@ uint64_t llvq_hip_codebook_fingerprint(void);
 int llvq_hip_host_decode(uint64_t idx, int8_t point[24], int* shell);
 
 /* upload_matrix (fused_cuda.rs:1058): validates, range-checks every index
- * (IndexOutOfRange, format.rs:389-392) and copies the record to the device. */
+ * (IndexOutOfRange, format.rs:389-392), copies the record to the device and unranks its codes there,
+ * once: 13 bytes per block of 24 weights stay on the device.  Waits for the runtime's stream.  May be
+ * called from several threads (uploads of one runtime take turns), also while another thread launches. */
 int llvq_hip_matrix_upload(llvq_rt* rt, const llvq_matrix_desc* desc, llvq_mat** out);
 
 /* read_header (format.rs:588): parses magic, count and, for LVQ4, the
@@ -112,7 +114,7 @@ typedef struct llvq_record_info {
 int llvq_hip_parse_matrix_record(const uint8_t* buf, size_t len, size_t* pos, llvq_record_info* out);
 
 /* read_matrix_raw (format.rs:301) fused with upload: parses one on-disk matrix
- * record at buf[*pos..] and uploads it; the code stream is copied verbatim.
+ * record at buf[*pos..] and uploads it; the code stream goes to the device as it is in the file.
  * *pos is advanced past the record. */
 int llvq_hip_matrix_from_record(llvq_rt* rt, const uint8_t* buf, size_t len, size_t* pos,
                                 llvq_mat** out);
@@ -227,7 +229,7 @@ int llvq_hip_gemm(llvq_rt* rt, const llvq_mat* m, const void* x_f16_dev, int M, 
 int llvq_hip_gemm_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x_f16_dev, int M,
                         void* const* y_dev, int y_dtype);
 
-/* llvq_hip_gemm / llvq_hip_gemm_group keep their partial sums, a tiled copy of the activations and
+/* llvq_hip_gemm / llvq_hip_gemm_group keep their partial sums, a copy of the activations as column octets and
  * (rotated matrices) the rotated rows in buffers of the runtime, which they grow on first use of a
  * larger shape — a hipFree + hipMalloc, i.e. a device-wide wait inside a call that otherwise only
  * enqueues.  This sizes those buffers ahead of time for calls over `mats` (one group, as
@@ -239,8 +241,8 @@ int llvq_hip_reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, in
 
 /* llvq_hip_gemm for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart
- * in the reference.  Same kernels and results as llvq_hip_gemm; the partial sums, the tiled
- * copy of the activations and (rotated matrices) the rotated rows live in one static device
+ * in the reference.  Same kernels and results as llvq_hip_gemm; the partial sums, the copy of
+ * the activations and (rotated matrices) the rotated rows live in one static device
  * array of LLVQ_STATIC_SCRATCH_BYTES per GPU instead of buffers the runtime grows, and the
  * call makes no hipMalloc / hipFree.  A shape whose workspaces do not fit is refused with
  * LLVQ_ERR_UNSUPPORTED (the message names the bytes needed).  That limit is one of rows of a multiple of 8 values
@@ -287,8 +289,8 @@ typedef struct llvq_quant_rows {
 /* How llvq_hip_decoder_* launches the projection groups of a decoded position.  The results are the same bit for bit;
  * the speed is not: a decode position is a chain of dependent products, and an ordered item of a sequence pays about
  * what a launch boundary costs (measured on the Qwen3-4B shape: 600 / 502 / 418 tokens/s in the order below).
- * Models a sequence cannot take (matrices in a rotated basis or of mixed shell caps, hidden > 6144) use LLVQ_LAUNCH_PER_GROUP
- * whatever is asked. */
+ * Models a sequence cannot take (matrices in a rotated basis or of mixed shell caps, rows wider than 24 576 columns) use
+ * LLVQ_LAUNCH_PER_GROUP whatever is asked. */
 typedef enum llvq_launch_mode {
   LLVQ_LAUNCH_PER_GROUP = 0,  /* one llvq_hip_gemv_group launch per group */
   LLVQ_LAUNCH_SINGLE = 1,     /* one single-item sequence (llvq_hip_sequence_*) per group: the sequence kernel's tile loop */

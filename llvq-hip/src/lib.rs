@@ -8,7 +8,7 @@
 //! `CustomOp` does for the CUDA arm (fused_cuda.rs:758-900).
 //!
 //! Nothing here decodes, transcodes or copies weights on the host: the archive's 6-byte
-//! records go to the device verbatim and are unranked by the kernels.
+//! records go to the device verbatim and are unranked there, once, at upload.
 #![allow(clippy::missing_safety_doc)]
 
 use std::ffi::{c_char, c_int, c_void, CStr, CString};
@@ -209,7 +209,7 @@ pub struct HipRuntime {
     rt: *mut LlvqRt,
 }
 
-// The runtime and its matrices are immutable after construction and the library takes launches
+// The runtime and its matrices are immutable after construction, uploads take turns inside the library, and it takes launches
 // from one thread at a time — the contract `Arc<FusedRuntime>` is shared under (model.rs:268-271).
 unsafe impl Send for HipRuntime {}
 unsafe impl Sync for HipRuntime {}

@@ -2,7 +2,7 @@
 
 Host-side mirror of llvq-artifact/src/format.rs (`read_header` :588,
 `read_matrix_raw` :301, `write_matrix_raw` :238, `write_header` :563) with the
-code stream kept packed — the device reads the file's bytes verbatim.  Errors
+code stream kept packed — the device is handed the file's bytes verbatim.  Errors
 are the variants of llvq-artifact/src/error.rs:11-45.
 """
 import struct

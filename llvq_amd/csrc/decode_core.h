@@ -332,7 +332,7 @@ LLVQ_HD void decode_even(const DecodeTables& T, const DevClass& c, uint64_t li, 
 }
 
 // Decodes `idx` and calls emit(position, value) for positions 0..23 in order,
-// taking the same path the GEMV kernel takes for the index's class.  Returns
+// by the path of the index's class.  Returns
 // the class index, -1 for the origin, -2 for an index past N(13) (zeros).
 template <class Emit>
 LLVQ_HD int decode_index(const DecodeTables& T, uint64_t idx, Emit&& emit) {
@@ -357,7 +357,7 @@ LLVQ_HD int decode_index(const DecodeTables& T, uint64_t idx, Emit&& emit) {
         emit(4 * q + j, table_byte(f.tab_lo, f.tab_hi, (sel >> (8 * j)) & 7u) + second);
       }
     };
-    // the two instantiations the GEMV kernel bins even-coset blocks into
+    // most even-coset blocks have one free kind, whose instantiation is the shorter
     if (f.meta & kMetaSecondFree) even_codes<true>(T, f, li, on_codes);
     else even_codes<false>(T, f, li, on_codes);
   } else {

@@ -375,21 +375,21 @@ struct StoreEach {
 };
 
 // ---- more activation rows ----------------------------------------------------------------------------
-// What bounds it: the matrix cores, and the issue slots they share with the unpacking (38 instructions for every 2 CF
-// products).  A workgroup of four wavefronts takes 256 weight rows by 32 CF activation rows; a wavefront unpacks 64 rows
+// What bounds it: the chain of a step, in which the matrix cores are busy half the time (51 % for CF = 8, counters in
+// profiles/; 38 instructions of unpacking run beside every 2 CF products), and tiles that are no multiple of the CUs (192
+// workgroups for gate and up of an 8B layer at 512 rows).  A workgroup of four wavefronts takes 256 weight rows by 32 CF activation rows; a wavefront unpacks 64 rows
 // (two fragments) against all of the activation rows (CF fragments).  CF = 8: 256 accumulators and one wavefront on a
 // SIMD, half the unpacking and a workgroup on every CU (1.28 us a step, where the products alone take 0.85 on numbers
-// like these); CF = 4: half of that, two workgroups on a CU (0.69 us a step each) or one (0.8), for batches and matrices
+// like these in a loop of nothing else); CF = 4: half of that, two workgroups on a CU (0.69 us a step each) or one (0.8), for batches and matrices
 // that do not fill the other.
 // Octets and tiles go from memory to LDS without passing through registers, two to three steps of 48 columns (two
 // blocks) ahead.
 // PAIR: both terms of the weights against the same activations, 2 CF more products a round; every step's sums go to f64
-// ones (512 registers: CF = 4 and one wavefront on a SIMD).  2.4 us a step; 13000 x 5121 at 600 rows 115 -> 250 us.
+// ones (512 registers: CF = 4 and one wavefront on a SIMD).  2.4 us a step; 13000 x 5121 at 600 rows 115 -> 250 to 280 us.
 // Launches with too few tiles to fill the chip split the columns (`splits`): partial sums go to the workspace and
 // gemm_reduce_kernel adds them in order; otherwise the tile is finished here.
 // Gate and up of an 8B layer (24576 x 4096) at 512 rows: 158 -> 116 us, 886 TFLOP/s; a plain f16 product of that size
-// by the vendor's library runs at 1151 on this card, whose clock follows the power the products draw (on random numbers
-// a loop of nothing else reaches 1650).
+// by the vendor's library runs at 1151 on this card (a loop of nothing but products on random numbers reaches 1650).
 constexpr uint32_t kWideRows = 256;
 constexpr uint32_t kWideTileBytes = 1024;  // four records, two blocks of each (832 bytes) and what the lanes behind them bring
 constexpr uint32_t kWideDepth = 4;         // LDS buffers, a step each

@@ -7,7 +7,7 @@
 // workgroup per CU walks its share of them without stopping at an item's end but to stage the next activation.
 //
 //   * Independent items: a workgroup takes one contiguous run of units, the runs equal in bytes, so that it meets two or
-//     three items of a model's 144 and streams the rest.  What bounds it is HBM: 13.x bytes per block; the planes of an
+//     three items of a model's 144 and streams the rest.  What bounds it is HBM: 13.x bytes per block at 4.6 to 5.2 TB/s; the planes of an
 //     item sit in registers, a step's registers are loaded again for the next unit as soon as they have been used
 //     (16 wavefronts x 4 steps x 832 bytes in flight per CU), and the sums over a team's wavefronts need no barrier: the
 //     wavefront that arrives last at a record's counter in LDS adds them up and stores.  A barrier every four units only

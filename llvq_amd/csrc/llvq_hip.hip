@@ -485,10 +485,10 @@ struct llvq_rt {
   std::vector<DevRotation*> rotations;
   __half* rot_rows = nullptr;     // rotated batch rows, f16 (matrix-core path)
   size_t rot_rows_bytes = 0;
-  // workspace of the batched kernels: partial sums [S, n_bands, M, 64]
+  // workspace of the wide batched kernel: partial sums of its column splits [splits][padded rows][weight rows, whole tiles]
   float* gemm_ws = nullptr;
   size_t gemm_ws_bytes = 0;
-  // a batch's activations in K-step tiles [n_steps, m_pad, 32] (pipelined batched kernel)
+  // a batch's activations as column octets [n_oct][m_pad] of 16 bytes
   __half* gemm_xt = nullptr;
   size_t gemm_xt_bytes = 0;
   // Uploads may come from several threads; launches come from one (llvq_hip.h).  Held while an upload uses what follows
@@ -1542,9 +1542,10 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   return LLVQ_OK;
 }
 
-// What llvq_hip_gemm_static admits.  The bound is part of its contract (callers choose their fallback by it), so it stays
-// the one of the partial-sum layout the entry point was specified with (gemm_share.h: a band's K-slices shared out over
-// the workgroups, 64 x 64 sums per piece, and a tiled copy of the activations), which is above what the kernels take now.
+// What llvq_hip_gemm_static admits of rows on 16-byte boundaries.  The bound is part of its contract (callers choose their
+// fallback by it: what it refused stays refused), so it is the one of the partial-sum layout the entry point was specified
+// with (gemm_share.h: a band's K-slices shared out over the workgroups, 64 x 64 sums per piece, and a tiled copy of the
+// activations).  The kernels need less, and nothing else uses that formula.
 static size_t static_admission_bytes(const llvq_rt* rt, const llvq_mat* m, uint32_t M) {
   const uint32_t grid_cap = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), consumers = M <= 256u ? 4u : 8u;
   const uint32_t bands = (m->d_out + 63u) / 64u, spb = (m->nblocks + 15u) / 16u;
@@ -1561,7 +1562,7 @@ static size_t static_admission_bytes(const llvq_rt* rt, const llvq_mat* m, uint3
 //   * rows of a multiple of 8 values from a 16-byte boundary on: weights rounded to binary16 once (error 2e-4 of the
 //     results' norm);
 //   * other rows, natural basis: both terms of the weights (1e-7 with f32 results, which is what a row by itself has).
-//     A second product costs the matrix cores twice the time (13000 x 5121 at 600 rows 250 us for 115) and a loop of
+//     A second product costs the matrix cores twice the time (13000 x 5121 at 600 rows 250 to 280 us for 115) and a loop of
 //     single rows many times that (27 900 us before there were tiles);
 //   * row by row, as batch-1 products: a single row, other rows in a rotated basis (the products above take them as
 //     binary16, a row by itself in f32; such widths end at 124), matrices without a whole block, and cap-13 matrices,
@@ -1930,10 +1931,8 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   const size_t group_layer = cache_layer / kKvGroup;
   // few partials: the last workgroup of a kv head merges them; many: a chip-wide merge kernel does
   const uint32_t merge_inline = n_splits <= (uint32_t)kAttnInlineSplits ? 1u : 0u;
-  // Projections in the natural basis derive their activation in the launch's
-  // prologue; a rotated basis needs the activation as a tensor first (it goes
-  // through the rotation kernel), and so do rows too wide for the staging area:
-  // their prologue runs as a kernel of its own.
+  // Projections derive their activation in the launch's prologue, and rotate it there where their basis
+  // is a rotated one; where rows are too wide for that (gemv_fits) the prologue runs as a kernel of its own.
   auto project = [&](const llvq_mat* const* mats, int n, const __half* x, void* const* outs, const Prologue& pro) -> int {
     // every launch of the group can derive (and, in a rotated basis, rotate) the activation itself
     bool fused = true;

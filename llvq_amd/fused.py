@@ -16,7 +16,7 @@ from .artifact import RawMatrix, read_header, read_matrix_raw, read_sealed
 
 class FusedMatrix:
     """One projection ready to upload (fused.rs:566-588).  The payload is the
-    file's own code stream; there is no load-time transcode on this path."""
+    file's own code stream; the device unranks it at upload, the host never does."""
 
     def __init__(self, raw: RawMatrix):
         # one gain bit is compiled into the kernels (fused.rs:1168-1177)
@@ -306,7 +306,8 @@ class FusedRuntime:
         return FusedSequence(self, handle, outputs, keep)
 
     def forward_batched(self, proj: FusedProj, x, out_dtype=None):
-        """Rows of `x` [M, d_in] through one projection (the row loop of model.rs:521-529)."""
+        """Rows of `x` [M, d_in] through one projection (the row loop of model.rs:521-529).  M >= 2: weights are rounded to
+        binary16 once where d_in is a multiple of 8 and x starts on a 16-byte boundary; otherwise as exact as `forward`."""
         torch = self._torch
         if x.dim() != 2 or x.shape[1] != proj.d_in:
             raise ValueError(f"{proj.name} expects [M, {proj.d_in}], got {list(x.shape)}")
@@ -336,7 +337,7 @@ class FusedRuntime:
 
     def forward_batched_static_into(self, proj: FusedProj, x, y):
         """`forward_batched_into` through llvq_hip_gemm_static: the call allocates no device memory
-        (its workspaces are a static device array); shapes beyond that array raise Unsupported."""
+        (its workspaces are a static device array); shapes beyond its limit (llvq_hip.h) raise Unsupported."""
         torch = self._torch
         if x.dtype != torch.float16 or not x.is_contiguous() or x.dim() != 2 or x.shape[1] != proj.d_in:
             raise ValueError(f"{proj.name} expects a contiguous f16 [M, {proj.d_in}] activation")
