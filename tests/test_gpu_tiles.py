@@ -38,8 +38,10 @@ def test_single_row_products(gpu_rt, orc, nb, tail, d_out):
 
 # Rows of activations: 16, 64 and 128 close a variant or a tile; columns: products of four blocks, of two, steps of
 # the last split that are short, a block beyond them, tails and row strides of any parity; few rows split the columns.
+# (Tails of 8 and 16 columns keep the rows on 16-byte boundaries: weights of one term.  Other tails: of two.)
 @pytest.mark.parametrize("nb,tail,d_out,M", [(1, 0, 1, 2), (5, 7, 31, 16), (63, 0, 33, 17), (64, 1, 16, 64), (65, 23, 70, 65), (170, 16, 255, 128),
-                                             (171, 3, 257, 129), (34, 0, 4100, 256), (16, 5, 200, 257), (512, 0, 64, 1024), (33, 1, 24, 1025)])
+                                             (171, 3, 257, 129), (34, 0, 4100, 256), (16, 5, 200, 257), (512, 0, 64, 1024), (33, 1, 24, 1025),
+                                             (5, 8, 31, 16), (64, 16, 16, 64), (65, 8, 70, 65), (171, 16, 257, 129), (16, 8, 200, 257), (33, 16, 24, 1025)])
 def test_batched_products(gpu_rt, orc, nb, tail, d_out, M):
     import torch
 
