@@ -1066,45 +1066,104 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const __half* __restrict_
   if (blockIdx.x == 0 && i < n) out[i] = __float2half_rn(silu_mul(__half2float(gate[i]), __half2float(up[i])));
 }
 
-// logits = f16(E h) for a dense binary16 head (Head::project, model.rs:578-587);
-// one wavefront per row at a time, 16-byte loads, f32 accumulate.  Every
-// wavefront also leaves its best (value, row), lowest row on ties.
+// ---- head -------------------------------------------------------------------------------
+// Bound by the read of the head.  One row under way in a wavefront, its loads waiting for the sum of the row before, read
+// 151936 rows at 5.5 TB/s (2560 columns in binary16, 140 us) and 5.0 TB/s (5120 in int8, 165 us).  Two rows together, the
+// next chunk's loads ahead of this chunk's products and non-temporal (each line is read once): 116 us and 132 us, 6.7 and
+// 6.3 TB/s.  Three or four rows (122 and 137 us) have more in flight than the memory takes and a longer last turn.
 constexpr int kHeadThreads = 256;
-__global__ __launch_bounds__(kHeadThreads) void lm_head_kernel(const __half* __restrict__ E, const __half* __restrict__ h,
-                                                               uint32_t vocab, uint32_t hidden, float* __restrict__ logits,
-                                                               float* __restrict__ best_val, uint32_t* __restrict__ best_idx) {
-  extern __shared__ __align__(16) float hs[];  // [hidden]
+constexpr uint32_t kHeadRows = 2;
+// Three workgroups a CU: 1024 of them took 120 us and 131 us, 512 140 us and 165 us.
+constexpr uint32_t kHeadGroups = 768;
+typedef uint32_t head_u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ head_u32x4 head_load(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const head_u32x4*>(p));
+}
+
+// logits = f16(E h) and every wavefront's best (value, row), lowest row on ties.  W: kValues a lane holds of a chunk,
+// Piece, load(row, chunk), dot(piece, h, a) in the order of the row.  A wavefront holds kHeadRows rows together; the
+// next chunk's loads, also those of the next rows, leave before this chunk's products.  A row past the end repeats the
+// wavefront's first and is not stored, a lane past the row's end the last chunk, which it does not add.
+template <class W>
+__device__ __forceinline__ void head_rows(const W& w, const __half* __restrict__ h, uint32_t vocab, uint32_t hidden,
+                                          float* __restrict__ hs, float* __restrict__ logits, float* __restrict__ best_val,
+                                          uint32_t* __restrict__ best_idx) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t gw = __builtin_amdgcn_readfirstlane(blockIdx.x * (kHeadThreads / 64) + (threadIdx.x >> 6));
+  const uint32_t nw = gridDim.x * (kHeadThreads / 64);
+  const uint32_t chunks = hidden / W::kValues, rounds = (chunks + 63u) >> 6;
+  typename W::Piece p[kHeadRows];
+  const auto request = [&](uint32_t r0, uint32_t c) {  // r0 < vocab
+    const uint32_t cl = min(c * 64u + lane, chunks - 1u);
+#pragma unroll
+    for (uint32_t i = 0; i < kHeadRows; ++i) {
+      const uint32_t r = r0 + i * nw;
+      p[i] = w.load(r < vocab ? r : r0, cl);
+    }
+  };
+  if (gw < vocab) request(gw, 0);
   for (uint32_t i = threadIdx.x; i < hidden; i += kHeadThreads) hs[i] = __half2float(h[i]);
   __syncthreads();
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t gw = blockIdx.x * (kHeadThreads / 64) + (threadIdx.x >> 6), nw = gridDim.x * (kHeadThreads / 64);
-  const uint32_t chunks = hidden >> 3;  // 16-byte units per row
   float bv = -INFINITY;
   uint32_t bi = 0xFFFFFFFFu;
-  for (uint32_t r = gw; r < vocab; r += nw) {
-    const uint4* row = reinterpret_cast<const uint4*>(E + (size_t)r * hidden);
-    float a = 0.f;
-    for (uint32_t c = lane; c < chunks; c += 64) {
-      const uint4 u = row[c];
-      const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
+  for (uint32_t r0 = gw; r0 < vocab; r0 += kHeadRows * nw) {
+    float a[kHeadRows] = {};
+    for (uint32_t c = 0; c < rounds; ++c) {
+      typename W::Piece now[kHeadRows];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        a = fmaf(__half2float(__ushort_as_half((unsigned short)(wv[j] & 0xFFFFu))), hs[8 * c + 2 * j], a);
-        a = fmaf(__half2float(__ushort_as_half((unsigned short)(wv[j] >> 16))), hs[8 * c + 2 * j + 1], a);
+      for (uint32_t i = 0; i < kHeadRows; ++i) now[i] = p[i];
+      const bool more = c + 1u < rounds;
+      const uint32_t rn = more ? r0 : r0 + kHeadRows * nw;
+      if (rn < vocab) request(rn, more ? c + 1u : 0u);
+      const uint32_t cl = c * 64u + lane;
+      if (cl < chunks) {
+#pragma unroll
+        for (uint32_t i = 0; i < kHeadRows; ++i) a[i] = W::dot(now[i], hs + cl * W::kValues, a[i]);
       }
     }
-    a = wave_sum(a);
-    const float l = __half2float(__float2half_rn(a));
-    if (lane == 0) logits[r] = l;
-    if (l > bv) {  // rows ascend inside a wavefront, so '>' keeps the lowest row of a tie
-      bv = l;
-      bi = r;
+#pragma unroll
+    for (uint32_t i = 0; i < kHeadRows; ++i) {
+      const uint32_t r = r0 + i * nw;
+      const float l = __half2float(__float2half_rn(wave_sum(a[i])));
+      if (r >= vocab) break;
+      if (lane == 0) logits[r] = l;
+      if (l > bv) {  // rows ascend inside a wavefront, so '>' keeps the lowest row of a tie
+        bv = l;
+        bi = r;
+      }
     }
   }
   if (lane == 0) {
     best_val[gw] = bv;
     best_idx[gw] = bi;
   }
+}
+
+// Dense binary16 head (Head::project, model.rs:578-587): eight values a lane and load, f32 accumulate.
+struct HalfHead {
+  static constexpr uint32_t kValues = 8;
+  struct Piece {
+    head_u32x4 u;
+  };
+  const __half* E;
+  uint32_t hidden;
+  __device__ __forceinline__ Piece load(uint32_t r, uint32_t c) const { return {head_load(E + (size_t)r * hidden + c * 8u)}; }
+  static __device__ __forceinline__ float dot(const Piece& p, const float* h, float a) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a = fmaf(half_lo(p.u[j]), h[2 * j], a);
+      a = fmaf(half_hi(p.u[j]), h[2 * j + 1], a);
+    }
+    return a;
+  }
+};
+
+__global__ __launch_bounds__(kHeadThreads) void lm_head_kernel(const __half* __restrict__ E, const __half* __restrict__ h,
+                                                               uint32_t vocab, uint32_t hidden, float* __restrict__ logits,
+                                                               float* __restrict__ best_val, uint32_t* __restrict__ best_idx) {
+  extern __shared__ __align__(16) float hs[];  // [hidden]
+  head_rows(HalfHead{E, hidden}, h, vocab, hidden, hs, logits, best_val, best_idx);
 }
 
 // ---- int8 embedding / head (llvq-llm/kernels/emb_q8.cu) --------------------------------
@@ -1133,43 +1192,34 @@ __global__ __launch_bounds__(256) void embed_q8_kernel(QuantRows e, const uint32
   }
 }
 
-// logits = f16(E h) for the int8 head (tv_q8_h): one wavefront per row at a time,
-// 16 codes per lane and load (a 16-byte run never straddles a group of 64).
+// int8 head (tv_q8_h): 16 codes per lane and load (a 16-byte run never straddles a group of 64).
+struct QuantHead {
+  static constexpr uint32_t kValues = 16;
+  struct Piece {
+    head_u32x4 u;
+    __half s, b;
+  };
+  QuantRows e;
+  uint32_t hidden, gpr;
+  __device__ __forceinline__ Piece load(uint32_t r, uint32_t c) const {
+    const size_t g = (size_t)r * gpr + (c >> 2);
+    return {head_load(e.q + (size_t)r * hidden + c * 16u), e.scales[g], e.biases[g]};
+  }
+  static __device__ __forceinline__ float dot(const Piece& p, const float* h, float a) {
+    const float s = __half2float(p.s), b = __half2float(p.b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a = fmaf(q8_weight((p.u[j] >> (8 * t)) & 0xFFu, s, b), h[4 * j + t], a);
+    return a;
+  }
+};
+
 __global__ __launch_bounds__(kHeadThreads) void lm_head_q8_kernel(QuantRows e, const __half* __restrict__ h, uint32_t vocab,
                                                                   uint32_t hidden, float* __restrict__ logits,
                                                                   float* __restrict__ best_val, uint32_t* __restrict__ best_idx) {
   extern __shared__ __align__(16) float hs[];  // [hidden]
-  for (uint32_t i = threadIdx.x; i < hidden; i += kHeadThreads) hs[i] = __half2float(h[i]);
-  __syncthreads();
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t gw = blockIdx.x * (kHeadThreads / 64) + (threadIdx.x >> 6), nw = gridDim.x * (kHeadThreads / 64);
-  const uint32_t chunks = hidden >> 4, gpr = (hidden + kEmbedGroup - 1) / kEmbedGroup;
-  float bv = -INFINITY;
-  uint32_t bi = 0xFFFFFFFFu;
-  for (uint32_t r = gw; r < vocab; r += nw) {
-    const uint4* row = reinterpret_cast<const uint4*>(e.q + (size_t)r * hidden);
-    float a = 0.f;
-    for (uint32_t c = lane; c < chunks; c += 64) {
-      const uint4 u = row[c];
-      const float s = __half2float(e.scales[(size_t)r * gpr + (c >> 2)]), b = __half2float(e.biases[(size_t)r * gpr + (c >> 2)]);
-      const uint32_t wv[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) a = fmaf(q8_weight((wv[j] >> (8 * t)) & 0xFFu, s, b), hs[16 * c + 4 * j + t], a);
-    }
-    a = wave_sum(a);
-    const float l = __half2float(__float2half_rn(a));
-    if (lane == 0) logits[r] = l;
-    if (l > bv) {
-      bv = l;
-      bi = r;
-    }
-  }
-  if (lane == 0) {
-    best_val[gw] = bv;
-    best_idx[gw] = bi;
-  }
+  head_rows(QuantHead{e, hidden, (hidden + kEmbedGroup - 1) / kEmbedGroup}, h, vocab, hidden, hs, logits, best_val, best_idx);
 }
 
 // token = argmax over the wavefront winners; lowest row on ties

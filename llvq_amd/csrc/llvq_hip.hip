@@ -2243,7 +2243,7 @@ int llvq_hip_decoder_create(llvq_rt* rt, const llvq_decoder_desc* c, llvq_decode
   d->eps = (float)c->rms_eps;
   d->kv_q8 = c->kv_mode == LLVQ_KV_Q8;
   d->proj.assign(c->projections, c->projections + (size_t)c->n_layers * 7);
-  d->head_grid = 1024;
+  d->head_grid = kHeadGroups;
   while (d->head_grid > 1 && (uint64_t)d->head_grid * (kHeadThreads / 64) > c->vocab) d->head_grid >>= 1;
 
   // RoPE tables exactly as Rotary::new builds them (model.rs:163-179): f32 inverse

@@ -651,3 +651,47 @@ def test_a_non_finite_row_stays_out_of_earlier_blocks_of_a_prompt(gpu_rt, heads,
         assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
     finally:
         dec.close()
+
+
+@pytest.mark.parametrize("hidden,vocab,int8", [
+    (64, 3000, False),      # a row of 8 lanes; fewer pairs of rows than wavefronts
+    (520, 6143, False),     # one lane into a second chunk; one row short of two a wavefront
+    (520, 9300, False),     # a second turn, of one row for some wavefronts
+    (1024, 6144, True),     # int8: exactly one chunk, exactly two rows a wavefront
+    (1040, 12290, True),    # one lane into a second chunk; a third turn of two rows
+])
+def test_head_rows_and_chunks(gpu_rt, hidden, vocab, int8):
+    """The head at the edges of its rows and chunks against a product in 64 bits.  Its first rows are the unit vectors, so
+    the logits carry its input; every other logit then lies within the f32 sum's rounding (n + 3 roundings of at most
+    2^-24 of the sum of magnitudes, int8 weights add two) and one binary16 rounding."""
+    import dataclasses
+
+    cfg = dataclasses.replace(SMALL, num_hidden_layers=1, hidden_size=hidden, vocab_size=vocab, tie_word_embeddings=False)
+    weights = decoder.synthetic_weights(cfg, 31)
+    head = weights.lm_head
+    head[:hidden] = np.eye(hidden, dtype=np.float16)
+    mags = np.abs(head.astype(np.float64))
+    if int8:
+        rng = np.random.default_rng(31)
+        n_groups = (hidden + 63) // 64
+        q = rng.integers(0, 256, size=(vocab, hidden), dtype=np.uint8)
+        s = (1e-3 * (1 + rng.random((vocab, n_groups)))).astype(np.float16)
+        b = (-0.1 * rng.random((vocab, n_groups))).astype(np.float16)
+        q[:hidden], s[:hidden], b[:hidden] = np.eye(hidden, dtype=np.uint8), 1, 0
+        weights.lm_head = artifact.RawTensor("lm_head.weight", [vocab, hidden], bits=8, group=64, packed=q.reshape(-1),
+                                             scales=s.reshape(-1).view(np.uint16), biases=b.reshape(-1).view(np.uint16))
+        g = np.arange(hidden) // 64
+        head = q * s.astype(np.float64)[:, g] + b.astype(np.float64)[:, g]
+        mags = q * s.astype(np.float64)[:, g] - b.astype(np.float64)[:, g]
+    dec = decoder.Decoder(gpu_rt, cfg, decoder.synthetic_projections(cfg, 31), weights)
+    try:
+        for t in (5, 2999):
+            got, best = dec.forward_token(t)
+            h = got[:hidden].astype(np.float64)
+            terms = mags @ np.abs(h)
+            want = head.astype(np.float64) @ h
+            bound = (hidden + 5) * 2.0 ** -24 * terms + 2.0 ** -11 * np.abs(want) * 1.001 + 2.0 ** -24
+            assert np.any(h) and np.all(np.abs(got - want) <= bound)
+            assert best == int(np.argmax(got))
+    finally:
+        dec.close()
