@@ -6,10 +6,10 @@
 // their sums in f64 (of f32 sums over 32 or 48 columns), for the rows whose results are f32 exact (llvq_hip.hip,
 // gemm_same_basis).  Relative error of f32 results in norm, 2561 x 1000 at 65 rows: 2.1e-4 with one term, 1.01e-7 with two,
 // 0.97e-7 for rows one by one; 13000 columns: 2.2e-4, 1.37e-7, 1.38e-7.  Two terms alone, summed in f32, left up to 6e-7.  A dword of a block's nibbles is eight consecutive columns of a row, which is
-// exactly what a lane hands to a 16-deep (32 x 32) or 32-deep (16 x 16) product step, so a wavefront turns the 12 bytes
-// its lanes load into its own fragments: no weights pass through LDS, and the order in which the products walk the
+// exactly what a lane hands to a 16-deep (32 x 32) or 32-deep (16 x 16) product step, so a wavefront turns the ten bytes
+// of a block that its lanes load into its own fragments: no weights pass through LDS, and the order in which the products walk the
 // columns is the order the blocks lie in (the lane groups of a fragment hold the same octet of two or four neighbouring
-// blocks).  19 instructions per eight weights.
+// blocks).  17 instructions per eight weights, and 8 per block to put its three octets together.
 //
 // The activations come as octets: xt[c][m] = columns 8 c .. 8 c + 7 of row m, 16 bytes, m_pad rows to a column octet, so
 // that the fragments of 16 or 32 rows are runs of 256 or 512 bytes (tile_activations_kernel; in x they would be 16-byte
@@ -22,7 +22,6 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float acc4_t __attribute__((ext_vector_type(4)));
 typedef float acc16_t __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kGemmMaxGroup = 4;
 constexpr uint32_t kGemmSmallRows = 64;     // activation rows up to which the split kernel (gemm_tiles_kernel) runs
@@ -53,52 +52,104 @@ __global__ __launch_bounds__(256) void tile_activations_kernel(const __half* __r
 }
 
 // ---- weights ---------------------------------------------------------------------------------------
-// The matrix's table of scales for dequant_octet: a lane keeps entry lane % 32 as the sum of two binary16 numbers (low
-// half: the entry rounded, high half: what that left), a power of two taken out first that puts the largest entry into
-// [8, 16), so that neither number nor an eighth of it leaves the normal range by more than the precision can spare.
+// The matrix's table of scales for dequant_octet: a lane keeps its entry (scale_table) as the sum of two binary16 numbers
+// (low half: the entry rounded, high half: what that left), a power of two taken out first that puts the largest entry into
+// [8, 16), so that neither number nor a sixteenth of it leaves the normal range by more than the precision can spare.
 // `unit` is that power of two; it goes back in with the row scales.
-__device__ __forceinline__ uint32_t split_table(float entry, float& unit) {
-  uint32_t e = __float_as_uint(entry) & 0x7F800000u;
-#pragma unroll
-  for (int k = 1; k < 32; k <<= 1) e = max(e, (uint32_t)__shfl_xor((int)e, k));
-  const int ex = min(max((int)(e >> 23) - 130, -100), 100);  // (a table of zeros or with an infinity in it: any power will do)
-  unit = ldexpf(1.f, ex);
-  const float v = entry * ldexpf(1.f, -ex);
+__device__ __forceinline__ float table_unit(float entry) {
+  int e = (int)(__float_as_uint(entry) & 0x7F800000u);  // (two lanes to an entry, eight to a row of lanes)
+  e = max(e, __builtin_amdgcn_update_dpp(0, e, 0x122, 0xF, 0xF, false));  // row_ror 2, 4, 8
+  e = max(e, __builtin_amdgcn_update_dpp(0, e, 0x124, 0xF, 0xF, false));
+  e = max(e, __builtin_amdgcn_update_dpp(0, e, 0x128, 0xF, 0xF, false));
+  e = max(max(__builtin_amdgcn_readlane(e, 0), __builtin_amdgcn_readlane(e, 16)), max(__builtin_amdgcn_readlane(e, 32), __builtin_amdgcn_readlane(e, 48)));
+  return ldexpf(1.f, min(max((e >> 23) - 130, -100), 100));  // (a table of zeros or with an infinity in it: any power will do)
+}
+__device__ __forceinline__ uint32_t split_table(float entry, float unit) {
+  const float v = entry * (1.f / unit);
   const _Float16 hi = (_Float16)v;
   const _Float16 lo = (_Float16)(v - (float)hi);
   return __builtin_bit_cast(uint32_t, half2_t{hi, lo});
 }
-// What a block's meta byte gives a lane: the two parts of its scale (and an eighth of them), and its parity bit where
-// dequant_octet wants it.
-struct BlockScale {
-  half2_t c, c8;
-  uint32_t odd, odd8;
+// A block's octets as the unpacking wants them: v = nibble + 16 (the lowest bit of the next nibble around) + win - 3, that
+// bit for the blocks with one coordinate 16 below (block_code.h), where all others get it and the window goes down by 16.
+// And the two parts of the block's scale.
+struct GemmBlock {
+  uint32_t w[3], parts, meta;
+  int win;
 };
-__device__ __forceinline__ uint32_t block_meta(uint32_t meta_dword, uint32_t r) { return meta_dword >> (8u * (r & 3u)); }
 __device__ __forceinline__ uint32_t scale_parts(uint32_t meta, uint32_t table) {
-  return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(meta & 0x7Cu), (int)table);
+  return (uint32_t)__builtin_amdgcn_ds_bpermute((int)meta, (int)table);
 }
-__device__ __forceinline__ BlockScale block_scale(uint32_t meta, uint32_t parts) {
+// s, m: the {s, meta} dwords of the block's row; k: the block in its unit.
+__device__ __forceinline__ GemmBlock gemm_block(uint32_t d0, uint32_t d1, uint32_t s, uint32_t m, uint32_t k, uint32_t table) {
+  GemmBlock b;
+  block_octets(d0, d1, s << (3u - k), b.w);
+  const uint32_t meta = m >> (8u * k);
+  b.meta = meta & 255u;
+  b.parts = scale_parts(meta, table);
+  b.win = (int)(meta & 7u);
+  return b;
+}
+__device__ __forceinline__ bool is_escape(const GemmBlock& b) { return b.meta >= kBlockEscape; }
+// For all lanes (the scales are in all of them), where any has an escape.
+__device__ __forceinline__ void gemm_escape(GemmBlock& b, uint32_t table) {
+  const bool escape = is_escape(b);
+  const BlockEscape e = block_escape(b.w, b.meta);
+  const uint32_t parts = scale_parts(e.slot << 3, table) ^ (e.negative ? 0x80008000u : 0u);
+  const uint32_t q = e.at & 7u, bit = 1u << (4u * (q == 7u ? 0u : q + 1u));
+  const bool one = e.at < 24u;
+  b.w[0] = escape ? e.w0 : b.w[0];
+#pragma unroll
+  for (uint32_t o = 0; o < 3; ++o) b.w[o] |= escape && one ? 0x11111111u & ~((e.at >> 3) == o ? bit : 0u) : 0u;
+  b.win = escape ? (int)e.win - (one ? 16 : 0) : b.win;
+  b.parts = escape ? parts : b.parts;
+}
+// An escape of a tile's list in the same form, from lane `of` of `e` to lane `to`: a nibble n is 8 less, of which the bit above
+// has 16 and the window the rest.
+__device__ __forceinline__ void gemm_listed(GemmBlock& b, const u32x4_t& e, uint32_t of, uint32_t to, uint32_t lane, uint32_t table) {
+  const bool mine = lane == to;
+#pragma unroll
+  for (int o = 0; o < 3; ++o) {
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)e[o], of), up = ~(n >> 3) & 0x11111111u;
+    const uint32_t w = (((n & 0x77777777u) ^ 0x44444444u) << 1) | (up << 4 | up >> 28);
+    b.w[o] = mine ? w : b.w[o];
+  }
+  const uint32_t key = (uint32_t)__builtin_amdgcn_readlane((int)e.w, of);
+  const uint32_t parts = (uint32_t)__builtin_amdgcn_readlane((int)table, (key & 31u) * 2u);
+  b.parts = mine ? parts : b.parts;
+  b.win = mine ? (int)((key >> 8) & 1u) - 5 : b.win;
+}
+// The parts of a block's scale (and a sixteenth of them), and what takes a nibble's offset off (dequant_octet), in pairs.
+struct BlockScale {
+  half2_t c, c16;
+  uint32_t b, b16;
+};
+__device__ __forceinline__ BlockScale block_scale(int win, uint32_t parts) {
   const half2_t c = __builtin_bit_cast(half2_t, parts);
-  const uint32_t p = (uint32_t)((int32_t)(meta << 31) >> 31);
-  uint32_t odd = (p & 0x00010001u) ^ 0x64106410u, odd8 = (p & 0x00080008u) ^ 0x64806480u;
-  asm("" : "+v"(odd), "+v"(odd8));  // (kept whole: taken apart again, a mask and it would no longer be one operation)
-  return BlockScale{c, c * half2_t{(_Float16)0.125f, (_Float16)0.125f}, odd, odd8};
+  // -(1024 + 11 - win) and -(1024 + 16 (11 - win)) as binary16
+  const uint32_t b = (uint32_t)mad24(win, -0x00010001, (int)0xE40BE40Bu), b16 = (uint32_t)mad24(win, -0x00100010, (int)0xE4B0E4B0u);
+  return BlockScale{c, c * half2_t{(_Float16)0.0625f, (_Float16)0.0625f}, b, b16};
 }
-// One dword of nibbles -> eight weights.  A binary16 number of the form 1024 + k has k in its low bits: with the nibble's
-// top bit flipped (two's complement to offset) and the parity bit below it that is 1024 + 16 + v, or 1024 + 128 + 8 v
-// where the nibble lies four bits higher.  v (hi + lo) is rounded once: v lo is small enough for its own rounding to be
-// lost in that of the sum.  19 instructions, all of which run beside the matrix cores; the mixed-precision
+// One dword of nibbles -> eight weights.  A binary16 number of the form 1024 + k has k in its low bits: a nibble there, its
+// top bit turned over, with the lowest bit of the next one on top of it, makes 1024 + 11 - win + v, or 1024 +
+// 16 (11 - win) + 16 v where it lies four bits higher.
+// v (hi + lo) is rounded once: v lo is small enough for its own rounding to be
+// lost in that of the sum.  17 instructions, all of which run beside the matrix cores; the mixed-precision
 // multiply-add (two fewer) does not: 4 products and 20 of those took 103 ns of a SIMD, with packed or f32 ones 70.
+__device__ __forceinline__ half2_t octet_bits(uint32_t w, int i) {  // nibbles i and i + 4
+  const uint32_t u = i < 2 ? w : __builtin_amdgcn_alignbit(w, w, 8);
+  return __builtin_bit_cast(half2_t, (i & 1) ? (u & 0x01E001E0u) ^ 0x64806480u : (u & 0x001E001Eu) ^ 0x64086408u);
+}
+__device__ __forceinline__ half2_t dequant_two(uint32_t w, const BlockScale& s, int i) {
+  const half2_t v = octet_bits(w, i) + __builtin_bit_cast(half2_t, (i & 1) ? s.b16 : s.b);
+  const half2_t c = (i & 1) ? s.c16 : s.c;
+  return __builtin_elementwise_fma(v, half2_t{c.x, c.x}, v * half2_t{c.y, c.y});
+}
 __device__ __forceinline__ half8_t dequant_octet(uint32_t w, const BlockScale& s) {
-  const uint32_t t[4] = {((w << 1) & 0x001E001Eu) ^ s.odd, (w & 0x00F000F0u) ^ s.odd8, ((w >> 7) & 0x001E001Eu) ^ s.odd, ((w >> 8) & 0x00F000F0u) ^ s.odd8};
   half8_t out;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const half2_t bias = (i & 1) ? half2_t{(_Float16)1152.f, (_Float16)1152.f} : half2_t{(_Float16)1040.f, (_Float16)1040.f};
-    const half2_t v = __builtin_bit_cast(half2_t, t[i]) - bias;
-    const half2_t c = (i & 1) ? s.c8 : s.c;
-    const half2_t y = __builtin_elementwise_fma(v, half2_t{c.x, c.x}, v * half2_t{c.y, c.y});
+    const half2_t y = dequant_two(w, s, i);
     out[2 * i] = y.x;
     out[2 * i + 1] = y.y;
   }
@@ -106,34 +157,103 @@ __device__ __forceinline__ half8_t dequant_octet(uint32_t w, const BlockScale& s
 }
 
 // The same with what the rounding took as a second binary16 number each: the two make the weight to 2^-22 of it.  (A nibble
-// that lies four bits higher is brought down by the operation that takes the bias off, so both halves are v itself; what is
+// that lies four bits higher is brought down by the operation that takes the offset off, so both halves are v itself; what is
 // left of v hi after the first rounding is exact, and v lo joins it in one more.)  27 instructions.
+struct TwoPair {
+  half2_t hi, lo;
+};
+__device__ __forceinline__ TwoPair dequant_two_pair(uint32_t w, const BlockScale& s, int i) {
+  const half2_t hi = half2_t{s.c.x, s.c.x}, lo = half2_t{s.c.y, s.c.y}, u = octet_bits(w, i);
+  // (a sixteenth of -(1024 + 16 k) is -(64 + k): the exponent four lower)
+  const half2_t v = (i & 1) ? __builtin_elementwise_fma(u, half2_t{(_Float16)0.0625f, (_Float16)0.0625f}, __builtin_bit_cast(half2_t, s.b16 - 0x10001000u))
+                            : u + __builtin_bit_cast(half2_t, s.b);
+  const half2_t y = __builtin_elementwise_fma(v, hi, v * lo);
+  return TwoPair{y, __builtin_elementwise_fma(v, lo, __builtin_elementwise_fma(v, hi, -y))};
+}
 struct WeightPair {
   half8_t hi, lo;
 };
 __device__ __forceinline__ WeightPair dequant_octet_pair(uint32_t w, const BlockScale& s) {
-  const uint32_t t[4] = {((w << 1) & 0x001E001Eu) ^ s.odd, (w & 0x00F000F0u) ^ s.odd8, ((w >> 7) & 0x001E001Eu) ^ s.odd, ((w >> 8) & 0x00F000F0u) ^ s.odd8};
-  const half2_t hi = half2_t{s.c.x, s.c.x}, lo = half2_t{s.c.y, s.c.y};
   WeightPair out;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const half2_t u = __builtin_bit_cast(half2_t, t[i]);
-    const half2_t v = (i & 1) ? __builtin_elementwise_fma(u, half2_t{(_Float16)0.125f, (_Float16)0.125f}, half2_t{(_Float16)-144.f, (_Float16)-144.f})
-                              : u - half2_t{(_Float16)1040.f, (_Float16)1040.f};
-    const half2_t y = __builtin_elementwise_fma(v, hi, v * lo);
-    const half2_t r = __builtin_elementwise_fma(v, lo, __builtin_elementwise_fma(v, hi, -y));
-    out.hi[2 * i] = y.x;
-    out.hi[2 * i + 1] = y.y;
-    out.lo[2 * i] = r.x;
-    out.lo[2 * i + 1] = r.y;
+    const TwoPair y = dequant_two_pair(w, s, i);
+    out.hi[2 * i] = y.hi.x;
+    out.hi[2 * i + 1] = y.hi.y;
+    out.lo[2 * i] = y.lo.x;
+    out.lo[2 * i + 1] = y.lo.y;
   }
   return out;
+}
+
+// The wide kernel unpacks by looking up: the weights of the eight values that a block's coordinates can have, binary16, lie
+// in LDS, 16 bytes for each meta byte, in the order of three bits of the coordinates' nibbles, the low bytes of all before
+// the high ones; v_perm_b32 picks four at a time.  12 instructions an octet where arithmetic takes 17 (dequant_octet) and one
+// dword in place of the scale's four.  Meta bytes below kBlockEscape are windows of the matrix's scales, those from
+// there on are of a wavefront's escapes, 16 of them at a time: no point of shells up to 13 has more than eight different coordinates
+// (nine of one parity have squares that add up to 240 or more), so each can be written that way.
+constexpr uint32_t kValueBytes = 256u * 16u;  // with PAIR a second such table, of what the rounding took
+constexpr uint32_t kWaveValues = (256u - kBlockEscape) / 4u;
+struct Values {
+  u32x4_t hi, lo;
+};
+__device__ __forceinline__ void value_to(Values& t, int i, float y) {
+  const _Float16 hi = (_Float16)y, lo = (_Float16)(y - (float)hi);
+  const uint32_t a = __builtin_bit_cast(uint16_t, hi), b = __builtin_bit_cast(uint16_t, lo), at = 8u * ((uint32_t)i & 3u);
+  t.hi[i >> 2] |= (a & 255u) << at;
+  t.hi[2 + (i >> 2)] |= (a >> 8) << at;
+  t.lo[i >> 2] |= (b & 255u) << at;
+  t.lo[2 + (i >> 2)] |= (b >> 8) << at;
+}
+// A block as d0, d1 and its bits of s (in bit 0 of the nibbles) that picks from eight weights of its own.  n: the nibbles of v =
+// 2 n + odd.  About 300 instructions.
+struct ValueBlock {
+  Values t;
+  uint32_t d0, d1, s, at;  // at: where it belongs, of who keeps it
+};
+__device__ __forceinline__ ValueBlock value_block(const uint32_t (&n)[3], uint32_t odd, float scale) {
+  uint32_t there = 0, pick[3] = {0, 0, 0};
+  const uint32_t u[3] = {n[0] ^ 0x88888888u, n[1] ^ 0x88888888u, n[2] ^ 0x88888888u};  // n + 8
+#pragma unroll
+  for (int o = 0; o < 3; ++o)
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) there |= 1u << ((u[o] >> (4u * q)) & 15u);
+#pragma unroll
+  for (int o = 0; o < 3; ++o)
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) pick[o] |= (uint32_t)__builtin_popcount(there & ((1u << ((u[o] >> (4u * q)) & 15u)) - 1u)) << (4u * q);
+  ValueBlock b{{{}, {}}, pick[0] << 1 | (pick[2] & 0x11111111u), pick[1] << 1 | ((pick[2] >> 1) & 0x11111111u), (pick[2] >> 2) & 0x11111111u, 0u};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int v = there ? 2 * ((int)__builtin_ctz(there) - 8) + (int)odd : 0;
+    there &= there - 1u;
+    value_to(b.t, i, (float)v * scale);
+  }
+  return b;
+}
+// A quarter of an octet's unpacking: w's three bits at bit SHIFT of its nibbles.  Quarters 0 and 1 leave the pairs of
+// nibbles (0, 4) and (2, 6), 2 and 3 the others; a quarter's first half hands its bytes to the second.
+struct ValuePick {
+  uint32_t at, high;
+};
+template <uint32_t SHIFT>
+__device__ __forceinline__ void pick_values(uint32_t w, const u32x4_t& t, uint32_t quarter, ValuePick& p, u32x4_t& to) {
+  if ((quarter & 1u) == 0u) {
+    const uint32_t shift = SHIFT + (quarter ? 4u : 0u);
+    p.at = (shift ? w >> shift : w) & 0x07070707u;
+    p.high = __builtin_amdgcn_perm(t[3], t[2], p.at);
+  } else {
+    const uint32_t low = __builtin_amdgcn_perm(t[1], t[0], p.at);
+    to[quarter >> 1] = __builtin_amdgcn_perm(p.high, low, 0x06020400u);
+    to[2 + (quarter >> 1)] = __builtin_amdgcn_perm(p.high, low, 0x07030501u);
+  }
 }
 
 struct GemmMat {
   const uint8_t* base;  // the matrix (table, then records)
   void* y;
   uint32_t d_out, tile_begin;  // first row tile of this matrix in the launch
+  uint32_t stride, slots;      // of its tiles in memory
 };
 struct GemmArgs {
   const uint4* xt;     // [octets][m_pad]
@@ -150,10 +270,10 @@ struct GemmArgs {
 struct GemmTile {
   const uint8_t* base;
   void* y;
-  uint32_t row0, d_out;
+  uint32_t row0, d_out, stride, slots;
 };
 __device__ __forceinline__ GemmTile gemm_tile_at(const GemmArgs& a, uint32_t tile, uint32_t rows_per_tile) {
-  GemmTile t{a.mat[0].base, a.mat[0].y, 0u, a.mat[0].d_out};
+  GemmTile t{a.mat[0].base, a.mat[0].y, 0u, a.mat[0].d_out, a.mat[0].stride, a.mat[0].slots};
   uint32_t begin = 0;
 #pragma unroll
   for (uint32_t k = 1; k < (uint32_t)kGemmMaxGroup; ++k)
@@ -161,6 +281,8 @@ __device__ __forceinline__ GemmTile gemm_tile_at(const GemmArgs& a, uint32_t til
       t.base = a.mat[k].base;
       t.y = a.mat[k].y;
       t.d_out = a.mat[k].d_out;
+      t.stride = a.mat[k].stride;
+      t.slots = a.mat[k].slots;
       begin = a.mat[k].tile_begin;
     }
   t.row0 = (tile - begin) * rows_per_tile;
@@ -201,27 +323,25 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t nb = a.nb, n_quads = (nb + 3u) >> 2;
-  const uint32_t stride = tile_stride(nb, a.tail_w), head = tile_head_bytes(a.tail_w);
   const GemmTile t = gemm_tile_at(a, blockIdx.x, kRows);
+  const uint32_t stride = t.stride, head = tile_head_bytes(a.tail_w);
   const uint8_t* recs = t.base + kTileTableBytes + (size_t)(t.row0 / kTileRows) * stride;
-  const uint32_t last_rec = tile_count(t.d_out) - 1u - t.row0 / kTileRows;  // records past the matrix's last repeat it
-  const uint32_t r = lane & 7u, g = lane >> 4, m16 = lane & 15u;
-  const float entry = reinterpret_cast<const float*>(t.base)[lane & 31u];
-  uint32_t rec_off[RG];
-#pragma unroll
-  for (int k = 0; k < RG; ++k) rec_off[k] = min((uint32_t)k * 2u + ((lane >> 3) & 1u), last_rec) * stride + head + g * kTileBlockBytes;
+  const uint32_t last_rec = tile_count(t.d_out) - 1u - t.row0 / kTileRows;  // tiles past the matrix's last repeat it
+  const uint32_t g = lane >> 4, m16 = lane & 15u;  // the lane's block of a unit, and its row
+  const float entry = __uint_as_float(scale_table(t.base, lane));
+  const uint32_t d_off = head + (m16 & 7u) * 16u + ((m16 >> 3) * 2u + (g >> 1)) * 128u + (g & 1u) * 8u;
+  const uint32_t m_off = head + (m16 & 7u) * 16u + 512u + (m16 >> 3) * 8u;
   const uint32_t x_off = (g * 3u * a.m_pad + m16) * 16u, x_oct = a.m_pad * 16u;
 
-  StepWords W[RG];
+  struct Words { u32x2_t d, m; } W[RG];
   u32x4_t X[3][MT];
-  struct __attribute__((packed, aligned(4))) W3 { uint32_t w[3]; };
   auto load_w = [&](uint32_t q, bool live) {
     const uint32_t keep = live ? 0xFFFFFFFFu : 0u;
-    const uint8_t* p = uniform_global(recs + ((q * 4u * kTileBlockBytes) & keep));
 #pragma unroll
-    for (int k = 0; k < RG; ++k) {
-      const W3 w = *reinterpret_cast<const W3*>(p + lane_offset((rec_off[k] + r * 12u) & keep));
-      W[k] = StepWords{w.w[0], w.w[1], w.w[2], *reinterpret_cast<const uint32_t*>(p + lane_offset((rec_off[k] + 96u + (r & 4u)) & keep))};
+    for (uint32_t k = 0; k < (uint32_t)RG; ++k) {
+      const uint8_t* p = uniform_global(recs + (size_t)min(k, last_rec) * stride + ((q * kUnitBytes) & keep));
+      W[k].d = *reinterpret_cast<const u32x2_t*>(p + lane_offset(d_off & keep));
+      W[k].m = *reinterpret_cast<const u32x2_t*>(p + lane_offset(m_off & keep));
     }
   };
   auto load_x = [&](uint32_t j, uint32_t q, bool live) {
@@ -231,14 +351,13 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) X[j][mt] = *reinterpret_cast<const u32x4_t*>(p + off + (uint32_t)mt * 256u);
   };
-  // The row scales and the tail's operands, needed at the end: asked for first, put down last.
+  // The row scales and the tail's operands, needed at the end: asked for first.
   const uint32_t op_row = tid % kRows, op_col = tid / kRows;  // column 24: the row's scale
   float op_w = 0.f;
   uint32_t op_x[2] = {};
   {
     const uint8_t* rec = recs + (size_t)min(op_row / kTileRows, last_rec) * stride;
-    const uint32_t c = op_col < a.tail_w ? op_col + 1u : 0u;
-    op_w = reinterpret_cast<const float*>(rec)[c * 8u + (op_row & 7u)];
+    op_w = reinterpret_cast<const float*>(rec)[op_col < a.tail_w ? tail_at(op_row & 15u, op_col, a.tail_w) : op_row & 15u];
     if (a.tail_w) {
 #pragma unroll
       for (uint32_t i = 0; i < 2; ++i) {
@@ -247,12 +366,28 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
       }
     }
   }
+  // the tiles' lists of escapes, 32 lanes each
+  u32x4_t listed = {};
+  if (t.slots && (lane >> 5) < (uint32_t)RG)
+    listed = *reinterpret_cast<const u32x4_t*>(recs + (size_t)min(lane >> 5, last_rec) * stride + stride - (t.slots - min(lane & 31u, t.slots - 1u)) * 16u);
+  if ((lane & 31u) >= t.slots) listed.w = 0u;
   uint32_t q = wave;
   load_w(q, q < n_quads);
 #pragma unroll
   for (uint32_t j = 0; j < 3; ++j) load_x(j, q, q < n_quads);
-  float unit;
+  const float unit = table_unit(entry);
   const uint32_t table = split_table(entry, unit);
+  const bool read_codes = t.slots == 0u || __builtin_amdgcn_ballot_w64(listed.w == ~0u) != 0u;
+  // (before the loop: the registers are needed there)
+  if (op_col < a.tail_w) tw[op_row * 24u + op_col] = op_w;
+  else if (op_col == 24u) scale_s[op_row] = op_w * unit;
+  if (a.tail_w) {
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+      const uint32_t k = tid + i * 1024u, m = k / a.tail_w;
+      if (m < kCols) tx[m * 24u + k - m * a.tail_w] = __half2float(__ushort_as_half((unsigned short)op_x[i]));
+    }
+  }
   typedef double sum4_t __attribute__((ext_vector_type(4)));
   typename std::conditional<PAIR, sum4_t, acc4_t>::type acc[RG][MT];
 #pragma unroll
@@ -263,17 +398,37 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
     const uint32_t qn = q + 16u;
     const bool live = qn < n_quads;
     BlockScale s[RG];
+    GemmBlock b[RG];
 #pragma unroll
     for (int k = 0; k < RG; ++k) {
-      const uint32_t meta = block_meta(W[k].meta, r);
-      s[k] = block_scale(meta, scale_parts(meta, table));
+      b[k] = gemm_block(W[k].d.x, W[k].d.y, W[k].m.x, W[k].m.y, g, table);
+      // Escapes from the tiles' lists, where those count: 30 instructions and not 120.  (One of twenty units has one, but so
+      // has nearly every workgroup, and waits for it: 0.1 us of 6.5.)
+      if (__builtin_amdgcn_ballot_w64(is_escape(b[k]))) {
+        if (read_codes) {
+          gemm_escape(b[k], table);
+        } else {
+          for (uint64_t left = __builtin_amdgcn_ballot_w64(((listed.w >> 11) & 0x1FFFFu) == q && (lane >> 5) == (uint32_t)k && listed.w != 0u); left; left &= left - 1u) {
+            const uint32_t of = (uint32_t)__builtin_ctzll(left), key = (uint32_t)__builtin_amdgcn_readlane((int)listed.w, of);
+            gemm_listed(b[k], listed, of, ((key >> 9) & 3u) * 16u + (key >> 28), lane, table);
+          }
+        }
+      }
+      s[k] = block_scale(b[k].win, b[k].parts);
     }
+    // a register is asked for again as soon as its contents are used, and not moved from there
+    auto next_words = [&]() __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(qn, live);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (RG == 1) next_words();
 #pragma unroll
     for (uint32_t j = 0; j < 3; ++j) {
       half8_t w[RG], w2[RG];
 #pragma unroll
       for (int k = 0; k < RG; ++k) {
-        const uint32_t nibbles = j == 0 ? W[k].w0 : j == 1 ? W[k].w1 : W[k].w2;
+        const uint32_t nibbles = b[k].w[j];
         if constexpr (PAIR) {
           const WeightPair p = dequant_octet_pair(nibbles, s[k]);
           w[k] = p.hi;
@@ -282,12 +437,7 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
           w[k] = dequant_octet(nibbles, s[k]);
         }
       }
-      // a register is asked for again as soon as its contents are used, and not moved from there
-      if (j == 2u) {
-        __builtin_amdgcn_sched_barrier(0);
-        load_w(qn, live);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      if (RG != 1 && j == 2u) next_words();  // (two groups' words have no registers beside the blocks' octets before)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -305,23 +455,16 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (op_col < a.tail_w) tw[op_row * 24u + op_col] = op_w;
-  else if (op_col == 24u) scale_s[op_row] = op_w * unit;
-  if (a.tail_w) {
-#pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) {
-      const uint32_t k = tid + i * 1024u, m = k / a.tail_w;
-      if (m < kCols) tx[m * 24u + k - m * a.tail_w] = __half2float(__ushort_as_half((unsigned short)op_x[i]));
-    }
-  }
+  // (From the lane's number anew: nothing of this may occupy registers during the loop.)
+  const uint32_t tid_e = lane_offset(threadIdx.x), lane_e = tid_e & 63u;
   // of a fragment a lane's row is a weight row (lane % 16) and its four elements activation rows 4 (lane / 16) + e
 #pragma unroll
   for (int k = 0; k < RG; ++k)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      *reinterpret_cast<acc4_t*>(part + (((wave * RG + k) * MT + mt) * 64u + lane) * 4u) = __builtin_convertvector(acc[k][mt], acc4_t);
+      *reinterpret_cast<acc4_t*>(part + (((wave * RG + k) * MT + mt) * 64u + lane_e) * 4u) = __builtin_convertvector(acc[k][mt], acc4_t);
   __syncthreads();
-  for (uint32_t o = tid; o < kRows * kCols; o += 1024u) {
+  for (uint32_t o = tid_e; o < kRows * kCols; o += 1024u) {
     const uint32_t row = o % kRows, m = o / kRows;
     if (m >= a.M || t.row0 + row >= t.d_out) continue;
     const uint32_t l = (row & 15u) + 16u * ((m & 15u) >> 2), e = m & 3u;
@@ -390,17 +533,28 @@ struct StoreEach {
 // gemm_reduce_kernel adds them in order; otherwise the tile is finished here.
 // Gate and up of an 8B layer (24576 x 4096) at 512 rows: 158 -> 116 us, 886 TFLOP/s; a plain f16 product of that size
 // by the vendor's library runs at 1151 on this card (a loop of nothing but products on random numbers reaches 1650).
-constexpr uint32_t kWideRows = 256;
-constexpr uint32_t kWideTileBytes = 1024;  // four records, two blocks of each (832 bytes) and what the lanes behind them bring
+template <int RF>
+__host__ __device__ constexpr uint32_t gemm_wide_rows() { return 128u * RF; }
+template <int RF>
+__host__ __device__ constexpr uint32_t gemm_wide_tiles() { return 2u * RF * 384u; }  // {d0, d1} of two blocks of a wavefront's tiles, 256 bytes each; their {s, meta}
 constexpr uint32_t kWideDepth = 4;         // LDS buffers, a step each
 template <int CF>
 __host__ __device__ constexpr uint32_t gemm_wide_x_bytes() { return 6u * 32u * CF * 16u; }
-template <int CF>
-__host__ __device__ constexpr uint32_t gemm_wide_buf() { return gemm_wide_x_bytes<CF>() + 8u * kWideTileBytes; }
-template <int CF>
-__host__ constexpr size_t gemm_wide_lds() { return (size_t)kWideDepth * gemm_wide_buf<CF>(); }
-static_assert(kWideDepth * gemm_wide_buf<4>() >= (kWideRows + 128u) * kDim * 4u && kWideDepth * gemm_wide_buf<8>() >= (kWideRows + 256u) * kDim * 4u,
-              "the tail's operands fit the buffers");
+template <int RF, int CF>
+__host__ __device__ constexpr uint32_t gemm_wide_buf() { return gemm_wide_x_bytes<CF>() + 4u * gemm_wide_tiles<RF>(); }
+template <int RF, int CF, bool PAIR>
+__host__ constexpr size_t gemm_wide_lds() {
+  return (PAIR ? 2u * kValueBytes + 256u * sizeof(ValueBlock) : kValueBytes) + (size_t)kWideDepth * gemm_wide_buf<RF, CF>();
+}
+static_assert(2 * gemm_wide_lds<2, 4, false>() <= 160 * 1024 && gemm_wide_lds<2, 8, false>() <= 160 * 1024 && gemm_wide_lds<3, 4, false>() <= 160 * 1024 &&
+              gemm_wide_lds<2, 4, true>() <= 160 * 1024, "two workgroups of the first, one of the others on a CU");
+// A wavefront's lists of escapes as they come, and those of its split with the tile's number, where the last buffer will be.
+template <int RF>
+__host__ __device__ constexpr uint32_t gemm_wide_lists() { return 2u * RF * kMaxListSlots * 16u; }
+static_assert(gemm_wide_buf<2, 4>() >= 4u * (gemm_wide_lists<2>() + 64u * 20u) && gemm_wide_buf<3, 4>() >= 4u * (gemm_wide_lists<3>() + 64u * 20u), "the lists fit a buffer");
+template <int RF, int CF>
+__host__ constexpr bool gemm_wide_tail_fits() { return kWideDepth * gemm_wide_buf<RF, CF>() >= (gemm_wide_rows<RF>() + 32u * CF) * kDim * 4u; }
+static_assert(gemm_wide_tail_fits<2, 4>() && gemm_wide_tail_fits<2, 8>() && gemm_wide_tail_fits<3, 4>(), "the tail's operands fit the buffers");
 
 // 16 bytes per lane from base + offset to LDS, lane after lane from `lds` on.  In assembly because the compiler, which
 // cannot tell the buffers apart, would have every read of LDS wait for all of these; the counting is done by hand
@@ -409,196 +563,401 @@ static_assert(kWideDepth * gemm_wide_buf<4>() >= (kWideRows + 128u) * kDim * 4u 
 __device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t offset, const uint8_t* base) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(lds), "v"(offset), "s"(base) : "memory");
 }
+// Three of these, 1024 bytes apart in LDS; and two or three, the last by the first LANES lanes only, 512 bytes for each 16 of
+// them behind the first.  An instruction's offset counts in LDS and in memory: the lanes' offsets have it taken off, and
+// kLoadBias put on, which the base is without.  (All lanes are active where these are used; a condition would be a branch,
+// and what is in front of it and behind it could not be moved across.)
+constexpr uint32_t kLoadBias = 4096;
+__device__ __forceinline__ void load_three_to_lds(uint32_t lds, uint32_t o0, uint32_t o1, uint32_t o2, const uint8_t* base) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\tglobal_load_lds_dwordx4 %2, %4 offset:1024\n\tglobal_load_lds_dwordx4 %3, %4 offset:2048"
+               : : "{m0}"(lds), "v"(o0), "v"(o1), "v"(o2), "s"(base) : "memory");
+}
+template <int RF>
+__device__ __forceinline__ void load_tiles_to_lds(uint32_t lds, const uint32_t (&o)[RF], const uint8_t* d, const uint8_t* m) {
+  if constexpr (RF == 2)
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\ts_mov_b32 exec_hi, 0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4 offset:1024\n\ts_mov_b32 exec_hi, -1"
+                 : : "{m0}"(lds), "v"(o[0]), "v"(o[1]), "s"(d), "s"(m) : "memory");
+  else
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\ts_mov_b32 exec_hi, 0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4 offset:1024\n\t"
+                 "s_mov_b32 exec_hi, 0xffff\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %5 offset:1536\n\ts_mov_b32 exec_hi, -1"
+                 : : "{m0}"(lds), "v"(o[0]), "v"(o[1]), "v"(o[2]), "s"(d), "s"(m) : "memory");
+}
+// What a wavefront has read of LDS has come before it writes there, and the other way round.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// At the end of a branch that is seldom taken: the compiler would otherwise have the common way wait for what is in flight there.
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
+// A barrier by itself: what LDS reads of a wavefront are in flight it has not begun to need, and what they read stays.
+__device__ __forceinline__ void wide_barrier() {
+  asm volatile("" : : : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+}
 template <int N>
 __device__ __forceinline__ void wide_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-template <int CF, bool PAIR>
-__global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel(GemmArgs a) {
-  constexpr uint32_t kCols = 32u * CF, kBuf = gemm_wide_buf<CF>();
-  constexpr int kLoadsX = 3 * CF / 4, kLoadsW = 2, kLoads = kLoadsX + kLoadsW;  // of a wavefront in a step
-  extern __shared__ __align__(16) uint8_t smem[];     // [kWideDepth] x { [6 octets][kCols] 16 bytes, [8] x 32 rows of tiles }
+template <int RF, int CF, bool PAIR>
+__device__ __forceinline__ void wide_product(const GemmArgs& a) {
+  constexpr uint32_t kCols = 32u * CF, kRows = gemm_wide_rows<RF>(), kBuf = gemm_wide_buf<RF, CF>();
+  constexpr uint32_t kTileBytes = gemm_wide_tiles<RF>(), kTerms = PAIR ? 2u : 1u;
+  constexpr int kLoadsX = 3 * CF / 4, kLoadsW = RF, kLoads = kLoadsX + kLoadsW;  // of a wavefront in a step
+  static_assert(RF == 2 || RF == 3, "a wavefront's tiles: four, and two more");
+  // (aligned so that an entry's address is its offset or'ed in)
+  extern __shared__ __align__(4096) uint8_t wide_smem[];  // weights of the meta bytes, [kWideDepth] x { [6 octets][kCols] 16 bytes, tiles }
+  uint8_t* const smem = wide_smem + kTerms * kValueBytes;
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-  const uint32_t l32 = lane & 31u, h = lane >> 5, r = lane & 7u;
+  const uint32_t l32 = lane & 31u, h = lane >> 5;
   // tiles of one row group are neighbours in the grid: they read the same weights
   const uint32_t mt = blockIdx.x % a.m_tiles, rest = blockIdx.x / a.m_tiles;
   const uint32_t tile = rest % a.n_tiles, split = rest / a.n_tiles;
-  const uint32_t nb = a.nb, stride = tile_stride(nb, a.tail_w), head = tile_head_bytes(a.tail_w);
-  const GemmTile t = gemm_tile_at(a, tile, kWideRows);
-  const uint32_t row0 = t.row0 + wave * 64u;            // this wavefront's first row
+  const GemmTile t = gemm_tile_at(a, tile, kRows);
+  const uint32_t nb = a.nb, stride = t.stride, head = tile_head_bytes(a.tail_w);
+  const uint32_t row0 = t.row0 + wave * (32u * RF);     // this wavefront's first row
   const uint32_t n_rec = tile_count(t.d_out);
-  const float entry = reinterpret_cast<const float*>(t.base)[lane & 31u];
+  const float entry_f = __uint_as_float(scale_table(t.base, lane));
   const uint32_t n_steps = (nb + 1u) >> 1;
   const uint32_t s0 = split * a.steps_per_split, s1 = min(s0 + a.steps_per_split, n_steps);
   const uint8_t* rec0 = uniform_global(t.base + kTileTableBytes + (size_t)(t.row0 / kTileRows) * stride);
-  // records past the matrix's last repeat it: their rows are not stored
+  // tiles past the matrix's last repeat it: their rows are not stored
   auto record = [&](uint32_t row) __attribute__((always_inline)) { return (min(row / kTileRows, n_rec - 1u) - t.row0 / kTileRows) * stride; };
-  // a load of tiles takes four records, 13 lanes each; a load of octets 64 activation rows of one
+  // a load of tiles takes the lines of two blocks, of four or two tiles, or those of {s, meta} of all of this wavefront's; a load of octets 64 activation rows of one
   uint32_t w_off[kLoadsW], x_off[kLoadsX];
-  const uint32_t w_rec = min(lane, 51u) / 13u, w_piece = min(lane, 51u) - w_rec * 13u;
-#pragma unroll
-  for (uint32_t k = 0; k < (uint32_t)kLoadsW; ++k) w_off[k] = record(t.row0 + (wave * (uint32_t)kLoadsW + k) * 32u + w_rec * 8u) + head + w_piece * 16u;
+  w_off[0] = record(row0 + (lane >> 4) * 16u) + head + ((lane >> 3) & 1u) * 256u + (lane & 7u) * 16u;
+  if constexpr (RF == 3) w_off[1] = record(row0 + (4u + ((lane >> 4) & 1u)) * 16u) + head + ((lane >> 3) & 1u) * 256u + (lane & 7u) * 16u;
+  w_off[RF - 1] = record(row0 + min(lane >> 3, 2u * RF - 1u) * 16u) + head + 512u + (lane & 7u) * 16u;
 #pragma unroll
   for (uint32_t i = 0; i < (uint32_t)kLoadsX; ++i) {
-    const uint32_t k = i * 4u + wave, o = k / (kCols / 64u), m = k % (kCols / 64u) * 64u + lane;
-    x_off[i] = (o * a.m_pad + mt * kCols + m) * 16u;
+    const uint32_t k = wave * kLoadsX + i, o = k / (kCols / 64u), m = k % (kCols / 64u) * 64u + lane;
+    x_off[i] = (o * a.m_pad + mt * kCols + m) * 16u + kLoadBias - i % 3u * 1024u;
   }
-  const uint32_t x_step = 6u * a.m_pad * 16u, smem_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  const uint8_t* xt = reinterpret_cast<const uint8_t*>(a.xt);
-  auto load = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) {
-    s = min(s, s1 - 1u);  // (steps past the last are loaded too, so that the count of loads in flight is always the same)
-    const uint32_t at = smem_at + buffer;
-    const uint8_t* xs = uniform_global(xt + (size_t)s * x_step);
-    const uint8_t* ws = uniform_global(rec0 + (size_t)s * (2u * kTileBlockBytes));
-#pragma unroll
-    for (uint32_t i = 0; i < (uint32_t)kLoadsX; ++i) load_to_lds(at + (i * 4u + wave) * 1024u, x_off[i], xs);
-#pragma unroll
-    for (uint32_t k = 0; k < (uint32_t)kLoadsW; ++k) load_to_lds(at + gemm_wide_x_bytes<CF>() + (wave * (uint32_t)kLoadsW + k) * kWideTileBytes, w_off[k], ws);
+  w_off[0] += kLoadBias;
+  if constexpr (RF == 3) w_off[1] += kLoadBias - 1024u;
+  w_off[RF - 1] += kLoadBias - 512u * RF;
+  const uint32_t x_step = 6u * a.m_pad * 16u, values_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)wide_smem;
+  const uint32_t smem_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+  // where the steps come from, one after the other; steps past the last are loaded too, so that the count of loads in flight is
+  // always the same
+  uint32_t from_left = s1 - 1u - s0, from_odd = (s0 & 1u) * 128u;
+  const uint8_t* from_x = uniform_global(reinterpret_cast<const uint8_t*>(a.xt) + (size_t)s0 * x_step - kLoadBias);
+  const uint8_t* from_unit = uniform_global(rec0 + (size_t)(s0 >> 1) * kUnitBytes - kLoadBias);
+  auto load_x = [&](uint32_t buffer, uint32_t i) __attribute__((always_inline)) {
+    load_three_to_lds(smem_at + buffer + (wave * kLoadsX + 3u * i) * 1024u, x_off[3 * i], x_off[3 * i + 1], x_off[3 * i + 2], from_x);
   };
-  acc16_t acc[2][CF];
+  auto load_w = [&](uint32_t buffer) __attribute__((always_inline)) {  // and on to the next step
+    load_tiles_to_lds<RF>(smem_at + buffer + gemm_wide_x_bytes<CF>() + wave * kTileBytes, w_off, from_unit + from_odd, from_unit);
+    from_x += from_left ? x_step : 0u;
+    from_unit += from_left && from_odd ? kUnitBytes : 0u;
+    from_odd ^= from_left ? 128u : 0u;
+    from_left -= from_left ? 1u : 0u;
+  };
+  auto load = [&](uint32_t buffer) __attribute__((always_inline)) {
 #pragma unroll
-  for (int k = 0; k < 2; ++k)
+    for (uint32_t i = 0; i < (uint32_t)kLoadsX / 3u; ++i) load_x(buffer, i);
+    load_w(buffer);
+  };
+  acc16_t acc[RF][CF];
+  double sum[PAIR ? RF : 1][PAIR ? CF : 1][16];  // of the steps, with PAIR
+  const float unit = table_unit(entry_f), table = entry_f * (1.f / unit);
+  const auto scale_of = [&](uint32_t meta) __attribute__((always_inline)) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)meta, (int)__float_as_uint(table)));
+  };
+  // One step: three rounds of 2 CF products (an octet of columns of two blocks), in whose shadow everything else runs: the
+  // weights of the round after are unpacked, two at a time, and its activations read into the registers of those just used.
+  // In the middle of the first every wavefront waits for its loads of the next step and then for the others; the step before
+  // has been read by then, and its buffer is filled again during the second, which also reads the next step's tiles and puts
+  // their octets together.
+  // w: the next round's weights, [1] what the rounding took of them.  B: the block they are unpacked from, T: the weights it
+  // picks from.  (With PAIR the sums leave no registers for the next one's beside them.)
+  struct Block { uint32_t w[3], meta; };
+  u32x4_t w[kTerms][RF] = {}, T[RF][kTerms], Tn[RF];
+  half8_t x[CF];
+  Block B[RF], Bn[RF];
+  u32x2_t words[RF], metas[RF];
+  const auto unpack_part = [&](auto octet, uint32_t idx, ValuePick (&pick)[kTerms], u32x4_t (&to)[kTerms][RF]) __attribute__((always_inline)) {
+    constexpr uint32_t j = decltype(octet)::value;
+    const uint32_t k = idx >> 2;
+#pragma unroll
+    for (uint32_t p = 0; p < kTerms; ++p) pick_values<j == 2u ? 0u : 1u>(B[k].w[j], T[k][p], idx & 3u, pick[p], to[p][k]);
+  };
+  const uint32_t x_at = (h * 3u * kCols + l32) * 16u;
+  const uint32_t wave_at = gemm_wide_x_bytes<CF>() + wave * kTileBytes;
+  const uint32_t w_at = wave_at + (l32 >> 4) * 256u + ((l32 >> 3) & 1u) * 128u + (l32 & 7u) * 16u + h * 8u;
+  const uint32_t meta_at = wave_at + 512u * RF + (l32 >> 4) * 128u + (l32 & 7u) * 16u + ((l32 >> 3) & 1u) * 8u;
+  auto read_x_part = [&](uint32_t buffer, uint32_t j, uint32_t c) __attribute__((always_inline)) {
+    x[c] = __builtin_bit_cast(half8_t, (reinterpret_cast<const u32x4_t*>(smem + (buffer + x_at)) + j * kCols)[c * 32u]);
+  };
+  auto read_x = [&](uint32_t buffer, uint32_t j) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t c = 0; c < (uint32_t)CF; ++c) read_x_part(buffer, j, c);
+  };
+  auto read_w = [&](uint32_t buffer) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
+      words[k] = *reinterpret_cast<const u32x2_t*>(smem + (buffer + w_at) + k * 512u);
+      metas[k] = *reinterpret_cast<const u32x2_t*>(smem + (buffer + meta_at) + k * 256u);
+    }
+  };
+  // the lane's block of a step is 2 (step & 1) + h of its unit: by how much its bits of the dwords are turned
+  uint32_t turn_s = (2u * (s0 & 1u) + h - 2u) & 31u, turn_m = (8u * (2u * (s0 & 1u) + h) - 4u) & 31u;
+  auto read_values = [&](uint32_t k) __attribute__((always_inline)) {
+    const uint32_t meta = __builtin_amdgcn_alignbit(metas[k].y, metas[k].y, turn_m);
+    Bn[k].meta = meta;
+    const uint32_t from = (meta & 0xFF0u) | values_at;
+    if constexpr (PAIR) {
+#pragma unroll
+      for (uint32_t p = 0; p < kTerms; ++p) T[k][p] = *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)(from + p * kValueBytes);
+    } else {
+      Tn[k] = *(const __attribute__((address_space(3))) u32x4_t*)(uintptr_t)from;
+    }
+  };
+  auto assemble = [&](uint32_t k) __attribute__((always_inline)) {
+    const uint32_t third = __builtin_amdgcn_alignbit(metas[k].x, metas[k].x, turn_s);  // bit 2 of its three
+    Bn[k].w[0] = words[k].x;
+    Bn[k].w[1] = words[k].y;
+    Bn[k].w[2] = bfi32(0x33333333u, bfi32(0x11111111u, words[k].x, words[k].y << 1), third);
+  };
+  auto turn = [&]() __attribute__((always_inline)) {
+    turn_s ^= 30u;
+    turn_m ^= 16u;
+  };
+  // Escapes (block_code.h): a lane keeps one of this wavefront's, from its tiles' lists, as a block that picks from weights of
+  // its own, and puts it in the place of the code in LDS once that has come; where there is none in a step that is one
+  // comparison.  (Their codes read as they came, 120 instructions in one of ten steps and so in a third of a workgroup's, cost
+  // 6 to 10 % of the time, every wavefront waiting for the slowest; weights exchanged where they are unpacked, 7 %.)
+  // at: {d0, d1} and {s, meta} in the wavefront's tiles, 12 bits each, and the block of its unit.  (With PAIR it waits in LDS.)
+  uint32_t own_step = ~0u;
+  ValueBlock own{};
+  ValueBlock* const own_lds = reinterpret_cast<ValueBlock*>(smem + kWideDepth * kBuf) + tid;
+  bool read_codes = false, decode = false;  // a tile's list does not count, or there are more than lanes; this step's are read as they are
+  const uint32_t my_tiles = gemm_wide_x_bytes<CF>() + wave * kTileBytes;
+  auto place_escapes = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) {
+    const uint64_t mine = __builtin_amdgcn_ballot_w64(own_step == s);
+    decode = read_codes;
+    if (mine) {
+      if ((uint32_t)__builtin_popcountll(mine) > kWaveValues) {
+        decode = true;
+      } else if (own_step == s) {
+        const uint32_t v = kBlockEscape + wave * kWaveValues + __builtin_amdgcn_mbcnt_hi((uint32_t)(mine >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mine, 0u));
+        uint8_t* const tiles = smem + buffer + my_tiles;
+        if constexpr (PAIR) own = *own_lds;
+        *reinterpret_cast<u32x2_t*>(tiles + (own.at & 0xFFFu)) = u32x2_t{own.d0, own.d1};
+        uint32_t* const meta = reinterpret_cast<uint32_t*>(tiles + ((own.at >> 12) & 0xFFFu));
+        const uint32_t k = own.at >> 24;
+        __hip_atomic_fetch_and(meta, ~(0x11111111u << k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __hip_atomic_fetch_or(meta, own.s << k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        reinterpret_cast<uint8_t*>(meta + 1)[k] = (uint8_t)v;
+        reinterpret_cast<u32x4_t*>(wide_smem)[v] = own.t.hi;
+        if constexpr (PAIR) reinterpret_cast<u32x4_t*>(wide_smem + kValueBytes)[v] = own.t.lo;
+      }
+    }
+  };
+  auto decode_escapes = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
+      const uint32_t meta = (Bn[k].meta >> 4) & 255u;
+      uint32_t o[3], n[3] = {0, 0, 0};
+      block_octets(Bn[k].w[0], Bn[k].w[1], Bn[k].w[2] << 1, o);
+      const BlockEscape e = block_escape(o, meta);
+      o[0] = e.w0;
+      const int c = (int)e.win - 3;
+      const uint32_t odd = (uint32_t)c & 1u;
+#pragma unroll
+      for (uint32_t q = 0; q < 24u; ++q) {
+        const int v = nibble_at(o[q >> 3], q & 7u) + c - (q == e.at ? 16 : 0);
+        n[q >> 3] |= ((uint32_t)(((e.negative ? -v : v) - (int)odd) >> 1) & 15u) << (4u * (q & 7u));
+      }
+      const ValueBlock b = value_block(n, odd, scale_of(e.slot << 3));
+      if (meta >= kBlockEscape) {
+        Bn[k].w[0] = b.d0;
+        Bn[k].w[1] = b.d1;
+        Bn[k].w[2] = (b.d0 & 0x11111111u) | (b.d1 & 0x11111111u) << 1 | b.s << 2;
+        if constexpr (PAIR) {
+          T[k][0] = b.t.hi;
+          T[k][kTerms - 1u] = b.t.lo;
+        } else {
+          Tn[k] = b.t.hi;
+        }
+      }
+    }
+  };
+  auto round = [&](uint32_t buffer, uint32_t next, uint32_t last, uint32_t s, auto round_j) __attribute__((always_inline)) {
+    constexpr uint32_t j = decltype(round_j)::value, jn = j < 2u ? j + 1u : 0u;  // of the products, and of what is unpacked
+    constexpr uint32_t kParts = (PAIR && j == 1u ? 8u : 4u) * RF / CF;  // (PAIR: T is read anew behind its last use)
+    u32x4_t to[kTerms][RF];
+    ValuePick pick[kTerms];
+    if (j == 1u) {
+      read_w(next);
+      turn();
+    }
+    if (j == 2u) {
+#pragma unroll
+      for (int k = 0; k < RF; ++k) {
+        B[k] = Bn[k];
+        if constexpr (!PAIR) T[k][0] = Tn[k];
+      }
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < (uint32_t)CF; ++c) {
+      if (j == 0u && c == (uint32_t)CF / 2u) {
+        wide_wait<kLoads>();
+        wide_barrier();
+      }
+#pragma unroll
+      for (int p = (int)kTerms - 1; p >= 0; --p)
+#pragma unroll
+        for (int k = 0; k < RF; ++k)
+          acc[k][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, w[p][k]), x[c],
+                                                              PAIR && j == 0u && p == (int)kTerms - 1 ? acc16_t{} : acc[k][c], 0, 0, 0);  // (PAIR: a step's sum)
+      if (j < 2u) read_x_part(buffer, jn, c);
+      else read_x_part(next, 0, c);
+      const uint32_t first = c * kParts, after = min(first + kParts, 4u * RF);
+#pragma unroll
+      for (uint32_t i = first; i < after; ++i) unpack_part(std::integral_constant<uint32_t, jn>{}, i, pick, to);
+      // (here, not where it is used)
+#pragma unroll
+      for (uint32_t p = 0; p < kTerms; ++p)
+        if (first < after) {
+          if (after & 1u) asm volatile("" : "+v"(pick[p].at), "+v"(pick[p].high));
+          else asm volatile("" : "+v"(to[p][(after - 1u) >> 2]));
+        }
+      if (j == 1u) {
+        if (c == CF / 2u) {
+#pragma unroll
+          for (uint32_t k = 0; k < (uint32_t)RF; ++k) read_values(k);
+        }
+        if (c + RF >= (uint32_t)CF) assemble(c + RF - CF);
+        // (three steps ahead)
+        if (c % 2u == 0u && c / 2u < (uint32_t)kLoadsX / 3u) load_x(last, c / 2u);
+        if (c == 2u * (uint32_t)kLoadsX / 3u) load_w(last);
+      }
+#pragma unroll
+      for (int i = 0; i < (PAIR ? 2 * RF : RF); ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product,
+        __builtin_amdgcn_sched_group_barrier(0x002, CF == 8 ? 3 : 4, 0);  // vector instructions
+        if (i == 0) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (j == 0u) place_escapes(s + 1u, next);
+    if (j == 1u && decode) decode_escapes();
+#pragma unroll
+    for (uint32_t p = 0; p < kTerms; ++p)
+#pragma unroll
+      for (int k = 0; k < RF; ++k) w[p][k] = to[p][k];
+  };
+  // the lists first, into the buffer that is filled last: they are put in order while the first step's octets and tiles come
+  const uint32_t slots = t.slots, n_listed = 2u * RF * slots;
+  const uint32_t lists_at = 3u * kBuf + wave * (gemm_wide_lists<RF>() + 64u * 20u);
+  const uint8_t* const lists = uniform_global(rec0 + stride - slots * 16u);
+  for (uint32_t e0 = 0; e0 < n_listed; e0 += 64u) {
+    const uint32_t e = min(e0 + lane, n_listed - 1u), tile_of = e / slots;
+    load_to_lds(smem_at + lists_at + e0 * 16u, record(row0 + tile_of * 16u) + (e - tile_of * slots) * 16u, lists);
+  }
+  load(0);
+  load(kBuf);
+  load(2u * kBuf);
+  {
+    // the weights of meta byte `tid`
+    const float v = scale_of(tid & 255u);
+    Values values{};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) value_to(values, i, (float)(2 * (i < 4 ? i : i - 8) + (int)(tid & 7u) - 3) * v);
+    if (tid < kBlockEscape) {
+      reinterpret_cast<u32x4_t*>(wide_smem)[tid] = values.hi;
+      if constexpr (PAIR) reinterpret_cast<u32x4_t*>(wide_smem + kValueBytes)[tid] = values.lo;
+    }
+  }
+  if (slots) {
+    wide_wait<3 * kLoads>();
+    const u32x4_t* const raw = reinterpret_cast<const u32x4_t*>(smem + lists_at);
+    u32x4_t* const kept = reinterpret_cast<u32x4_t*>(smem + lists_at + gemm_wide_lists<RF>());
+    uint32_t* const kept_tile = reinterpret_cast<uint32_t*>(kept + 64);
+    uint32_t n = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)RF; ++i) {
+      const uint32_t from = min(i * 64u + lane, n_listed - 1u);
+      const u32x4_t e = raw[from];
+      const uint32_t step = (e.w >> 10) & 0x3FFFFu;
+      read_codes |= __builtin_amdgcn_ballot_w64(e.w == ~0u) != 0u;
+      const bool valid = i * 64u + lane < n_listed && e.w != 0u && step >= s0 && step < s1;
+      const uint64_t there = __builtin_amdgcn_ballot_w64(valid);
+      const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(there >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)there, 0u));
+      if (valid && at < 64u) {
+        kept[at] = e;
+        kept_tile[at] = from / slots;
+      }
+      n += (uint32_t)__builtin_popcountll(there);
+    }
+    read_codes |= n > 64u;
+    wave_lds_order();
+    if (n && !read_codes) {
+      const u32x4_t e = kept[lane];
+      const uint32_t tile_of = kept_tile[lane], row = e.w >> 28, blk = (e.w >> 9) & 0x7FFFFu, nibbles[3] = {e.x, e.y, e.z};
+      own = value_block(nibbles, (e.w >> 8) & 1u, scale_of((e.w & 31u) << 3));
+      own.at = (tile_of * 256u + (row >> 3) * 128u + (row & 7u) * 16u + (blk & 1u) * 8u) | (512u * RF + tile_of * 128u + (row & 7u) * 16u + (row >> 3) * 8u) << 12 | (blk & 3u) << 24;
+      own_step = lane < n ? blk >> 1 : ~0u;
+      if constexpr (PAIR) *own_lds = own;
+    }
+  }
+  wide_wait<2 * kLoads>();
+  lds_barrier();
+  place_escapes(s0, 0);
+  read_w(0);
+  read_x(0, 0);
+#pragma unroll
+  for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
+    read_values(k);
+    assemble(k);
+  }
+  if (decode) decode_escapes();
+#pragma unroll
+  for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
+    B[k] = Bn[k];
+    if constexpr (!PAIR) T[k][0] = Tn[k];
+    ValuePick pick[kTerms];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) unpack_part(std::integral_constant<uint32_t, 0>{}, 4u * k + i, pick, w);
+  }
+#pragma unroll
+  for (int k = 0; k < RF; ++k)
 #pragma unroll
     for (int c = 0; c < CF; ++c)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[k][c][e] = 0.f;
-  double sum[PAIR ? 2 : 1][PAIR ? CF : 1][16];  // of the steps, with PAIR
   if constexpr (PAIR) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < RF; ++k)
 #pragma unroll
       for (int c = 0; c < CF; ++c)
 #pragma unroll
         for (int e = 0; e < 16; ++e) sum[k][c][e] = 0.;
   }
-  float unit;
-  const uint32_t table = split_table(entry, unit);
-  // One step: three rounds of eight products, in whose shadow the weights of the round after are unpacked and its
-  // activations read.  Behind the first round every wavefront waits for its loads of the next step and then for the
-  // others; the step before has been read by then, and its buffer is filled again.  In the second the next step's tiles
-  // are read, in the third unpacked.
-  struct W3 { uint32_t w[3]; };
-  typedef __attribute__((address_space(3))) uint32_t lds_u32;
-  half8_t w[2], w2[2], x[CF];
-  W3 W[2], Wn[2];
-  uint32_t meta[2], parts[2];
-  BlockScale sc[2];
-  auto unpack = [&](uint32_t j) __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if constexpr (PAIR) {
-        const WeightPair p = dequant_octet_pair(W[k].w[j], sc[k]);
-        w[k] = p.hi;
-        w2[k] = p.lo;
-      } else {
-        w[k] = dequant_octet(W[k].w[j], sc[k]);
-      }
-    }
-  };
-  const uint32_t x_at = (h * 3u * kCols + l32) * 16u;
-  const uint32_t block_at = gemm_wide_x_bytes<CF>() + wave * 2u * kWideTileBytes + (l32 >> 3) * (2u * kTileBlockBytes) + h * kTileBlockBytes;
-  const uint32_t w_at = block_at + r * 12u, meta_at = block_at + 96u + r;
-  auto read_x = [&](uint32_t buffer, uint32_t j) __attribute__((always_inline)) {
-    const u32x4_t* f = reinterpret_cast<const u32x4_t*>(smem + (buffer + x_at)) + j * kCols;
-#pragma unroll
-    for (int c = 0; c < CF; ++c) x[c] = __builtin_bit_cast(half8_t, f[(uint32_t)c * 32u]);
-  };
-  auto read_w = [&](uint32_t buffer) __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) meta[k] = smem[(buffer + meta_at) + k * kWideTileBytes];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      // (dword by dword: merged into one read of 12 bytes at 4-byte alignment they took 60 cycles of LDS, not 6)
-      const volatile lds_u32* f = (const volatile lds_u32*)(lds_u32*)(smem + (buffer + w_at) + k * (int)kWideTileBytes);
-      Wn[k] = W3{{f[0], f[1], f[2]}};
-    }
-  };
-  auto look_up = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) parts[k] = scale_parts(meta[k], table);
-  };
-  auto scales = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      sc[k] = block_scale(meta[k], parts[k]);
-      W[k] = Wn[k];
-    }
-  };
-  auto round = [&](uint32_t buffer, uint32_t next, auto round_j) __attribute__((always_inline)) {
-    constexpr uint32_t j = decltype(round_j)::value;
-    const half8_t w0[2] = {w[0], w[1]}, w20[2] = {w2[0], w2[1]};
-    half8_t x0[CF];
-#pragma unroll
-    for (int c = 0; c < CF; ++c) x0[c] = x[c];
-    if (j < 2u) {
-      read_x(buffer, j + 1u);
-      unpack(j + 1u);
-    } else {
-      read_x(next, 0);
-      scales();
-      unpack(0);
-    }
-    if constexpr (PAIR) {
-#pragma unroll
-      for (int c = 0; c < CF; ++c)
-#pragma unroll
-        for (int k = 0; k < 2; ++k) acc[k][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w20[k], x0[c], acc[k][c], 0, 0, 0);
-    }
-#pragma unroll
-    for (int c = 0; c < CF; ++c)
-#pragma unroll
-      for (int k = 0; k < 2; ++k) acc[k][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w0[k], x0[c], acc[k][c], 0, 0, 0);
-#pragma unroll
-    for (int c = 0; c < CF; ++c) {
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read,
-#pragma unroll
-      for (int i = 0; i < (PAIR ? 4 : 2); ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product,
-        __builtin_amdgcn_sched_group_barrier(0x002, PAIR ? (CF == 8 ? 2 : 4) : (CF == 8 ? 3 : 5), 0);  // vector instructions
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  load(s0, 0);
-  load(s0 + 1u, kBuf);
-  load(s0 + 2u, 2u * kBuf);
-  wide_wait<2 * kLoads>();
-  lds_barrier();
-  read_w(0);
-  look_up();
-  read_x(0, 0);
-  scales();
-  unpack(0);
   uint32_t buffer = 0, next = kBuf, last = 3u * kBuf, s = s0;
   do {  // (a split has at least one step)
-    round(buffer, next, std::integral_constant<uint32_t, 0>{});
-    wide_wait<kLoads>();
-    lds_barrier();
-    load(s + 3u, last);
-    read_w(next);
-    __builtin_amdgcn_sched_barrier(0);
-    round(buffer, next, std::integral_constant<uint32_t, 1>{});
-    look_up();
-    __builtin_amdgcn_sched_barrier(0);
-    round(buffer, next, std::integral_constant<uint32_t, 2>{});
+    round(buffer, next, last, s, std::integral_constant<uint32_t, 0>{});
+    round(buffer, next, last, s, std::integral_constant<uint32_t, 1>{});
+    round(buffer, next, last, s, std::integral_constant<uint32_t, 2>{});
     last = buffer;
     buffer = next;
     next = next + kBuf == kWideDepth * kBuf ? 0u : next + kBuf;
     if constexpr (PAIR) {
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
+      for (int k = 0; k < RF; ++k)
 #pragma unroll
-        for (int c = 0; c < CF; ++c)
+        for (int c = 0; c < CF; ++c) {
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
             sum[k][c][e] += (double)acc[k][c][e];
-            acc[k][c][e] = 0.f;
           }
+        }
     }
   } while (++s < s1);
   if constexpr (PAIR) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < RF; ++k)
 #pragma unroll
       for (int c = 0; c < CF; ++c)
 #pragma unroll
@@ -607,7 +966,7 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
   wide_wait<0>();
   if constexpr (CF == 8) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < RF; ++k)
 #pragma unroll
       for (int c = 0; c < CF; ++c) asm volatile("" : "+a"(acc[k][c]));  // one by one from here: all of them would not fit the vector registers
   }
@@ -616,33 +975,36 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
   const uint32_t lane_e = lane_offset(lane), l32e = lane_e & 31u, he = lane_e >> 5;
   const uint32_t m0 = mt * kCols + l32e;
   if (a.splits > 1u) {
-    const uint32_t n_rows = a.n_tiles * kWideRows;
+    const uint32_t n_rows = a.n_tiles * kRows;
     float* out = a.ws + (size_t)split * a.m_pad * n_rows;
 #pragma unroll
     for (int c = 0; c < CF; ++c)
       if (m0 + (uint32_t)c * 32u < a.M) {
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-          StoreF32::store(out, (size_t)(m0 + (uint32_t)c * 32u) * n_rows, tile * kWideRows + wave * 64u + (uint32_t)k * 32u, he, 0, acc[k][c] * unit);
+        for (int k = 0; k < RF; ++k)
+          StoreF32::store(out, (size_t)(m0 + (uint32_t)c * 32u) * n_rows, tile * kRows + wave * (32u * RF) + (uint32_t)k * 32u, he, 0, acc[k][c] * unit);
       }
     return;
   }
   // The tail's operands to LDS, columns of all rows: a lane would wait for each of its loads in turn.
   float* w_tail = reinterpret_cast<float*>(smem);
-  float* x_tail = w_tail + kWideRows * kDim;
+  float* x_tail = w_tail + kRows * kDim;
   if (a.tail_w) {
     __syncthreads();
     for (uint32_t c0 = 0; c0 < a.tail_w; c0 += 8u) {
       float v[8];
-      const uint32_t row = tid % kWideRows, m = mt * kCols + tid % kCols;
-      // (the columns are shared out where there are two threads to a row)
-      const float* rec = reinterpret_cast<const float*>(rec0 + record(t.row0 + row) + 32u) + (row & 7u);
+      const uint32_t m = mt * kCols + tid % kCols;
       const __half* tx = a.x + (size_t)min(m, a.M - 1u) * a.ldx + nb * kDim;
 #pragma unroll
-      for (uint32_t i = 0; i < 8; ++i) v[i] = rec[min(c0 + i, a.tail_w - 1u) * 8u];
+      for (uint32_t r0 = 0; r0 < kRows; r0 += 256u) {
+        const uint32_t row = min(r0 + tid, kRows - 1u);
+        const float* rec = reinterpret_cast<const float*>(rec0 + record(t.row0 + row));
 #pragma unroll
-      for (uint32_t i = 0; i < 8; ++i)
-        if (tid < kWideRows && c0 + i < a.tail_w) w_tail[(c0 + i) * kWideRows + row] = v[i];
+        for (uint32_t i = 0; i < 8; ++i) v[i] = rec[tail_at(row & 15u, min(c0 + i, a.tail_w - 1u), a.tail_w)];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i)
+          if (r0 + tid < kRows && c0 + i < a.tail_w) w_tail[(c0 + i) * kRows + row] = v[i];
+      }
 #pragma unroll
       for (uint32_t i = 0; i < 8; ++i) v[i] = __half2float(tx[min(c0 + i, a.tail_w - 1u)]);
 #pragma unroll
@@ -653,12 +1015,12 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
   }
   auto finish = [&](auto to) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < RF; ++k) {
       const uint32_t row = row0 + (uint32_t)k * 32u;
       float scale[16];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float4 v = *reinterpret_cast<const float4*>(rec0 + record(row + g * 8u) + he * 16u);
+      for (uint32_t g = 0; g < 4u; ++g) {
+        const float4 v = *reinterpret_cast<const float4*>(rec0 + record(row + g * 8u) + (g & 1u) * 32u + he * 16u);
         scale[4 * g] = v.x * unit;
         scale[4 * g + 1] = v.y * unit;
         scale[4 * g + 2] = v.z * unit;
@@ -676,7 +1038,7 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
           // one again is not zero where that is infinite.)
           const uint32_t col = PAIR ? min(i + he, a.tail_w - 1u) : i + he;
           const bool there = !PAIR || i + he < a.tail_w;
-          const float tw = w_tail[col * kWideRows + wave * 64u + (uint32_t)k * 32u + l32e], tx = x_tail[col * kCols + (uint32_t)c * 32u + l32e];
+          const float tw = w_tail[col * kRows + wave * (32u * RF) + (uint32_t)k * 32u + l32e], tx = x_tail[col * kCols + (uint32_t)c * 32u + l32e];
           v = __builtin_amdgcn_mfma_f32_32x32x2f32(there ? tw : 0.f, there ? tx : 0.f, v, 0, 0, 0);
         }
         if constexpr (PAIR) {
@@ -693,7 +1055,7 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
       }
     }
   };
-  const bool whole = row0 + 64u <= t.d_out && ((reinterpret_cast<uintptr_t>(t.y) | t.d_out * (a.y_f32 ? 4u : 2u)) & 15u) == 0;
+  const bool whole = row0 + 32u * RF <= t.d_out && ((reinterpret_cast<uintptr_t>(t.y) | t.d_out * (a.y_f32 ? 4u : 2u)) & 15u) == 0;
   if (a.y_f32) {
     if (whole) finish(StoreF32{});
     else finish(StoreEach<float>{});
@@ -702,6 +1064,9 @@ __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel
     else finish(StoreEach<_Float16>{});
   }
 }
+template <int CF, bool PAIR>
+__global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel(GemmArgs a) { wide_product<2, CF, PAIR>(a); }
+__global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmArgs a) { wide_product<3, 4, false>(a); }
 
 // The partial sums of the column splits, added in order; row scale and tail columns.  A lane takes one weight row and
 // kReduceM activation rows, so that the row's tail is read once for them.
@@ -726,14 +1091,22 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
   const uint32_t mine = chunk * 256u + threadIdx.x, out_row = min(mine, n_rows - 1u);  // lanes past the last row repeat it
   const GemmTile t = gemm_tile_at(a, out_row / ra.rows_per_tile, ra.rows_per_tile);
   const uint32_t my_row = t.row0 + out_row % ra.rows_per_tile, row = min(my_row, t.d_out - 1u);
-  const uint32_t stride = tile_stride(a.nb, a.tail_w);
+  const uint32_t stride = t.stride;
   const uint8_t* rec = t.base + kTileTableBytes + (size_t)(row / kTileRows) * stride;
-  const uint32_t r = row & 7u, tail_w = a.tail_w;
+  const uint32_t r = row & 15u, tail_w = a.tail_w;
   if (tail_w) {
     const uint32_t m = min(m0 + threadIdx.x / 32u, a.M - 1u), c = min(threadIdx.x % 32u, tail_w - 1u);
     x_tail[threadIdx.x / 32u][threadIdx.x % 32u] = __half2float(a.x[(size_t)m * a.ldx + a.nb * kDim + c]);
   }
   const float scale = reinterpret_cast<const float*>(rec)[r];
+  // (a class's columns lie together: four of each at a time, the first of them asked for before the sums; what is behind the
+  // last is not used)
+  struct __attribute__((packed, aligned(4))) F4 { float v[4]; } tw[4];
+  const auto read_tail = [&](uint32_t i0) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t c = 0; c < 4u; ++c) tw[c] = *reinterpret_cast<const F4*>(reinterpret_cast<const float*>(rec) + tail_at(r, 4u * i0 + c, tail_w));
+  };
+  if (tail_w) read_tail(0);
   sum_t s[kReduceM];
 #pragma unroll
   for (uint32_t k = 0; k < kReduceM; ++k) s[k] = 0;
@@ -754,16 +1127,17 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
   for (uint32_t k = 0; k < kReduceM; ++k) out[k] = PAIR ? 0.f : (float)s[k] * scale;
   if (tail_w) {
     lds_barrier();
-    for (uint32_t c0 = 0; c0 < tail_w; c0 += 8u) {
-      float tw[8];
+    const uint32_t depth = tail_depth(tail_w);
+    for (uint32_t i0 = 0; i0 < depth; i0 += 4u) {
+      if (i0) read_tail(i0);
 #pragma unroll
-      for (uint32_t c = 0; c < 8u; ++c) tw[c] = reinterpret_cast<const float*>(rec + 32)[min(c0 + c, tail_w - 1u) * 8u + r];
+      for (uint32_t i = 0; i < 4u; ++i)
 #pragma unroll
-      for (uint32_t c = 0; c < 8u; ++c)
-        if (c0 + c < tail_w) {
+        for (uint32_t c = 0; c < 4u; ++c)
+          if (4u * (i0 + i) + c < tail_w) {
 #pragma unroll
-          for (uint32_t k = 0; k < kReduceM; ++k) out[k] = fmaf(tw[c], x_tail[k][c0 + c], out[k]);
-        }
+            for (uint32_t k = 0; k < kReduceM; ++k) out[k] = fmaf(tw[c].v[i], x_tail[k][4u * (i0 + i) + c], out[k]);
+          }
     }
   }
   if (mine < n_rows && my_row < t.d_out) {

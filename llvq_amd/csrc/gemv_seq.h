@@ -2,42 +2,50 @@
 // layout it shares.
 //
 // The reference issues two launches per projection and notes that launch latency is about half of a decode token
-// (llvq-llm/src/fused_cuda.rs:789-795).  Here the records of every item of a list — an item is what one
-// llvq_hip_gemv_group call would be — are cut into units of one workgroup's worth and one persistent 1024-lane
-// workgroup per CU walks its share of them without stopping at an item's end but to stage the next activation.
+// (llvq-llm/src/fused_cuda.rs:789-795).  Here the tiles of every item of a list — an item is what one
+// llvq_hip_gemv_group call would be — are shared out over one persistent 1024-lane workgroup per CU, which walks its share
+// without stopping at an item's end but to stage the next activation.
 //
-//   * Independent items: a workgroup takes one contiguous run of units, the runs equal in bytes, so that it meets two or
-//     three items of a model's 144 and streams the rest.  What bounds it is HBM: 13.x bytes per block at 4.6 to 5.2 TB/s; the planes of an
-//     item sit in registers, a step's registers are loaded again for the next unit as soon as they have been used
-//     (16 wavefronts x 4 steps x 832 bytes in flight per CU), and the sums over a team's wavefronts need no barrier: the
-//     wavefront that arrives last at a record's counter in LDS adds them up and stores.  A barrier every four units only
-//     bounds how far the wavefronts drift apart (eight record slots).
-//   * Ordered items (`wait_item`): the units of an item are dealt round-robin; before a workgroup reads an activation
+//   * Independent items: a workgroup takes one contiguous run of tiles, the runs equal in bytes, so that it meets two or
+//     three items of a model's 144 and streams the rest.  What bounds it is HBM: 10.x bytes per block.  A wavefront takes
+//     up to four steps of a tile at a time (a task); a step's registers are loaded again, piece by piece, for its next
+//     step, in this task or the one after, as soon as they have been used: sixteen wavefronts x 5 KB in flight per CU.
+//     Rows of up to four steps (128 blocks) are a wavefront's own; of wider ones the sums of the steps meet in LDS, the
+//     wavefront that arrives last at a tile's counter adds them up and stores, and a barrier every kSeqDrift tasks
+//     bounds how far the wavefronts drift apart.
+//   * Ordered items (`wait_item`): a step is a task, the tiles are dealt out evenly; before a workgroup reads an activation
 //     that an earlier item stores it waits for that item's counter, which every workgroup bumps when its last rows of
 //     it have arrived in memory (outputs and activations are stored and loaded at device scope, past the XCDs' own L2s).
-//     The first unit's weights are requested before the wait.  A workgroup only ever waits for items below the one it is
+//     The first tasks' weights are requested before the wait.  A workgroup only ever waits for items below the one it is
 //     working on and takes its units in ascending order, so with every workgroup resident (grid <= CUs, one workgroup per
 //     CU, the device otherwise idle) the waits end.  They are bounded all the same: a wait that reaches `spin_limit`
 //     polls sets `*status` and the workgroup returns, which makes every wait behind it give up in turn.
 //
-// Results are those of the per-item launches bit for bit: a record's split over wavefronts and every order of addition
-// depend on the row length alone.
+// Results are those of the per-item launches bit for bit: every order of addition depends on the row length alone.
 #pragma once
 
 namespace llvq {
 
 constexpr uint32_t kSeqNoWait = 0xFFFFFFFFu;
-constexpr uint32_t kSeqSlots = 8;    // records per team whose sums may be pending
-constexpr uint32_t kSeqDrift = 4;    // units between two barriers: half of kSeqSlots
+constexpr uint32_t kSeqWaves = 16;
+constexpr uint32_t kSeqTaskSteps = 4;  // steps of a task of independent items
+constexpr uint32_t kSeqDrift = 4;      // tasks of a wavefront between two barriers, where tiles are shared
+// Tiles whose sums may be pending between two barriers, when a tile is `tasks` >= 2 tasks: those that begin there, and one
+// that is cut at either end.
+__host__ __device__ inline uint32_t seq_slots(uint32_t tasks) { return kSeqDrift * kSeqWaves / tasks + 2u; }
+// Sixteen rows of sums for each of their steps: at the most 4 tasks (64 / tasks + 2) with tasks <= 8.
+constexpr uint32_t kSeqPartSteps = 4 * (kSeqDrift * kSeqWaves + 2 * 8), kSeqMaxSlots = kSeqDrift * kSeqWaves / 2 + 2;
 
-struct SeqUnit {           // up to 16 >> split_shift consecutive records of one matrix
-  const uint8_t* rec;      // the first record
+struct SeqUnit {           // consecutive tiles of one matrix
+  const uint8_t* rec;      // the first tile
   const uint32_t* table;   // the matrix's scales
-  void* y;                 // the first record's first output element
+  void* y;                 // the first tile's first output element
   uint32_t rows;           // rows of the unit
   uint32_t item;
+  uint32_t stride, slots;  // of the matrix's tiles
+  uint32_t pad[2];
 };
-static_assert(sizeof(SeqUnit) == 32, "unit descriptors are read with scalar loads");
+static_assert(sizeof(SeqUnit) == 48, "unit descriptors are read with scalar loads");
 
 struct SeqItem {
   const __half* x;        // the activation, or the prologue's first operand
@@ -52,7 +60,9 @@ struct SeqItem {
   uint32_t expected;      // workgroups that take part in this item
   uint32_t signals;       // a later item waits for this one
   uint32_t wait_expected; // `expected` of wait_item
-  uint32_t pad[3];
+  uint32_t tasks;         // tasks of a tile, its steps shared out evenly
+  uint32_t inv_tasks;     // 2^32 / tasks, rounded up (tasks > 1)
+  uint32_t pad;
 };
 static_assert(sizeof(SeqItem) == 80, "item records are read with scalar loads");
 
@@ -60,7 +70,7 @@ struct SeqArgs {
   const SeqUnit* units;
   const SeqItem* items;
   const uint32_t* runs;  // [grid + 1] where each workgroup's run of units begins, or null: dealt round-robin
-  uint32_t n_units, max_blocks;  // max_blocks: plane blocks of the widest item
+  uint32_t n_units, max_units;  // max_units: plane units of the widest item
   uint32_t* counters;    // per item: workgroups that have finished it, counted on from run to run
   uint32_t* status;      // set to 1 by a workgroup that gave up waiting
   uint32_t run;          // 1, 2, ...: item i is complete in this run at counters[i] == run * expected
@@ -77,9 +87,9 @@ enum : int {
   kSeqPrologueWide = 4      // the same with rows past 512 blocks
 };
 
-__host__ __device__ inline size_t gemv_seq_lds_bytes(uint32_t max_blocks, bool f32_out) {
-  const size_t planes = (size_t)max_blocks * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
-  return gemv_lds_fixed() + planes + 2 * kSeqSlots * kGemvMaxWaves * 8 * 4 + kSeqSlots * kGemvMaxWaves * 4 + 16;
+__host__ __device__ inline size_t gemv_seq_lds_bytes(uint32_t max_units, bool f32_out) {
+  const size_t planes = (size_t)max_units * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
+  return gemv_lds_fixed() + planes + (kSeqPartSteps + 2 * kSeqMaxSlots) * kTileRows * 4 + kSeqMaxSlots * 4 + 16;
 }
 
 // The tables are the same for every lane and no kernel writes them: read through the constant address space, they come by
@@ -107,35 +117,23 @@ __global__ __launch_bounds__(1024) void gemv_seq_kernel(SeqArgs s) {
   constexpr int DIG = std::is_same<OutT, __half>::value ? 4 : 6;
   constexpr bool kWide = MODE == kSeqIndependentWide || MODE == kSeqPrologueWide;
   constexpr bool kWaits = MODE >= kSeqOrdered, kPro = MODE >= kSeqPrologue;
-  constexpr uint32_t kSteps = kWide ? kGemvWideSteps : kGemvSteps;
-  constexpr uint32_t kStr = XPlanes<DIG>::kDwords;
   extern __shared__ __align__(16) uint8_t smem[];
   GemvLds L;
   L.xtail = reinterpret_cast<float*>(smem);
   L.red = L.xtail + 32;
   L.planes = reinterpret_cast<uint32_t*>(L.red + 16);
-  L.part = reinterpret_cast<float*>(L.planes + (size_t)s.max_blocks * kStr);
-  L.tpart = L.part + kSeqSlots * kGemvMaxWaves * 8;
+  L.part = reinterpret_cast<float*>(L.planes + (size_t)s.max_units * XPlanes<DIG>::kDwords);  // [slot][step][16 rows]
   L.xf = nullptr;
-  uint32_t* arrived = reinterpret_cast<uint32_t*>(L.tpart + kSeqSlots * kGemvMaxWaves * 8);  // [slot][team]
-  uint32_t* verdict = arrived + kSeqSlots * kGemvMaxWaves;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 7u, bq = lane >> 3;
+  float* const tpart = L.part + kSeqPartSteps * kTileRows;                                      // [slot][16 rows] what tile_extras gives,
+  float* const scales = tpart + kSeqMaxSlots * kTileRows;                                       // and the row scales
+  uint32_t* arrived = reinterpret_cast<uint32_t*>(scales + kSeqMaxSlots * kTileRows);           // [slot]
+  uint32_t* verdict = arrived + kSeqMaxSlots;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   uint32_t u = s.runs ? scalar_read(s.runs + blockIdx.x) : blockIdx.x;
   const uint32_t u_end = s.runs ? scalar_read(s.runs + blockIdx.x + 1u) : s.n_units, u_step = s.runs ? 1u : gridDim.x;
 
   uint32_t it = kSeqNoWait, it_signals = 0;  // the item whose activation is in LDS
-  uint32_t nb = 0, tail_w = 0, shift = 2, split = 4, team = 0, w = 0, stride = 0, head = 0, n_steps = 0;
-  const LaneOffsets at = lane_offsets(lane);
-  uint32_t tail_c = 0, tail_off = 0, tail_waves = 0;
-  RecordWords<kSteps> W;
-  uint32_t slot = 0;
-  // this wavefront's record of a unit
-  auto request = [&](const SeqUnit& q) {
-    const bool mine = team * kTileRows < q.rows;
-    const uint8_t* rec = q.rec + (mine ? team * stride : 0u);
-    load_record(W, rec, reinterpret_cast<const uint8_t*>(q.table), head, w, split, n_steps, mine, tail_off, lane, at);
-  };
   // Every store of this workgroup for item `it` has arrived in memory: tell the items that wait for it.  (The rows went
   // out as device-scope stores; no fence, which would flush or empty the XCD's L2.)
   auto signal_item = [&]() {
@@ -145,28 +143,79 @@ __global__ __launch_bounds__(1024) void gemv_seq_kernel(SeqArgs s) {
   };
 
   if (u >= u_end) return;  // the same for every lane of the workgroup
-  SeqUnit cur = seq_unit_at(s.units, u);
-  bool last = false;
-  for (;;) {  // an item (everything that decides a branch outside a wavefront's own steps is the same for every lane)
+  SeqUnit first = seq_unit_at(s.units, u);
+  if (tid < kSeqMaxSlots) arrived[tid] = 0;
+  for (;;) {  // an item (everything that decides a branch outside a wavefront's own tasks is the same for every lane)
     if (it != kSeqNoWait) {
       if (kWaits && it_signals) signal_item();
       else lds_barrier();  // the old planes and slots are no longer read
     }
-    const SeqItem I = scalar_read(s.items + cur.item);
-    nb = I.nb;
-    tail_w = I.tail_w;
-    shift = gemv_split_shift(nb);
-    split = 1u << shift;
-    team = wave >> shift;
-    w = wave & (split - 1u);
-    n_steps = (nb + 7u) >> 3;
-    stride = tile_stride(nb, tail_w);
-    head = tile_head_bytes(tail_w);
-    tail_c = w * 8u + bq;
-    tail_off = tail_c < tail_w ? 32u + tail_c * 32u + r * 4u : 0u;
-    tail_waves = (tail_w + 7u) >> 3;
-    if (tid < kSeqSlots * kGemvMaxWaves) arrived[tid] = 0;
-    slot = 0;
+    const SeqItem I = scalar_read(s.items + first.item);
+    const uint32_t nb = I.nb, tail_w = I.tail_w, n_steps = tile_steps(nb), units = tile_units(nb), head = tile_head_bytes(tail_w);
+    const uint32_t tasks = I.tasks, long_steps = n_steps / tasks, long_tasks = n_steps - long_steps * tasks, slots = seq_slots(tasks);
+    it = first.item;
+    it_signals = I.signals;
+    // The workgroup's units of the item, and the tasks in them.
+    auto unit_tiles = [&](const SeqUnit& q) { return (q.rows + kTileRows - 1u) / kTileRows; };
+    uint32_t total = 0, u_next = u;
+    SeqUnit after = first;
+    do {
+      total += unit_tiles(after) * tasks;
+      u_next += u_step;
+      if (u_next >= u_end) break;
+      after = seq_unit_at(s.units, u_next);
+    } while (after.item == it);
+    // Where this wavefront is in them: round r's tasks are the sixteen from 16 r on, its own another one of them each time
+    // (a tile's tasks may differ in length, and their number divide sixteen).
+    SeqUnit at = first;
+    uint32_t at_u = u, at_task = 0, at_tile = 0;  // the unit, and the item's tasks and tiles in front of it
+    struct Task {
+      const uint8_t* rec;
+      const uint8_t* table;
+      uint8_t* y;
+      uint32_t rows;         // of the tile that are there
+      uint32_t step, end;    // steps [step, end)
+      uint32_t part, slot;   // which of the tile's tasks; where its sums meet
+      uint32_t list;         // places in the tile's list of escapes
+      bool live;
+    };
+    auto task_of = [&](uint32_t round) {
+      const uint32_t g = round * kSeqWaves + ((wave + round) & (kSeqWaves - 1u));
+      const bool live = g < total;
+      Task t;
+      if (live)
+        while (g - at_task >= unit_tiles(at) * tasks) {
+          at_task += unit_tiles(at) * tasks;
+          at_tile += unit_tiles(at);
+          at_u += u_step;
+          at = seq_unit_at(s.units, at_u);
+        }
+      const uint32_t k = live ? g - at_task : 0u, tile = tasks == 1u ? k : __umulhi(k, I.inv_tasks);
+      t.part = k - tile * tasks;
+      t.rec = at.rec + (size_t)tile * at.stride;
+      t.list = at.slots;
+      t.table = reinterpret_cast<const uint8_t*>(at.table);
+      t.y = reinterpret_cast<uint8_t*>(at.y) + (size_t)tile * (kTileRows * sizeof(OutT));
+      t.rows = at.rows - tile * kTileRows;
+      t.step = t.part * long_steps + min(t.part, long_tasks);
+      t.end = t.step + long_steps + (t.part < long_tasks ? 1u : 0u);
+      t.slot = (at_tile + tile) % slots;
+      t.live = live;
+      return t;
+    };
+    const uint32_t rounds = (total + kSeqWaves - 1u) / kSeqWaves;
+    StepWords W;
+    uint32_t table;
+    TileExtras extras{};
+    auto load_head = [&](const Task& t) {  // a tile's first task sees to them
+      if (t.live & (t.part == 0u)) extras = load_extras(t.rec, nb, tail_w, t.list, true, lane);
+    };
+    Task cur = task_of(0);
+    auto request = [&]() {
+      table = scale_table(cur.table, lane);
+      load_head(cur);
+      load_step(W, scalar_base(cur.rec), cur.live ? step_offset(cur.step, units, head, lane) : 0u);
+    };
     ActivationIn in{};
     in.x = uniform_global(I.x);
     if constexpr (kPro) {
@@ -177,7 +226,7 @@ __global__ __launch_bounds__(1024) void gemv_seq_kernel(SeqArgs s) {
       in.prologue = I.prologue;
     }
     if constexpr (kWaits) {
-      if constexpr (!kWide) request(cur);  // the weights do not depend on the item before
+      request();  // the weights do not depend on the item before
       if (I.wait_item != kSeqNoWait) {
         if (tid == 0) {
           const uint32_t target = s.run * I.wait_expected + (I.wait_item == s.hold_item ? 1u : 0u);
@@ -194,75 +243,79 @@ __global__ __launch_bounds__(1024) void gemv_seq_kernel(SeqArgs s) {
         if (*verdict == 0) return;  // gave up: every lane leaves, and so will whoever waits for this workgroup
       }
     }
-    auto ask = [&] { if constexpr (!kWaits && !kWide) request(cur); };
+    auto ask = [&] { if constexpr (!kWaits) request(); };
     constexpr int kPasses = kWide ? 4 : 2;
     const bool resid = u == I.first_unit;
     if (kPro && I.prologue == kPrologueSiluMul) stage_x<DIG, kSrcSiluMul, kPasses, kWaits>(in, nb, tail_w, L, resid, ask);
     else if (kPro && I.prologue == kPrologueAddRmsNorm) stage_x<DIG, kSrcAddRmsNorm, kPasses, kWaits>(in, nb, tail_w, L, resid, ask);
     else stage_x<DIG, kSrcF16, kPasses, kWaits>(in, nb, tail_w, L, false, ask);
-    if constexpr (kWide) request(cur);  // (the registers are the staging's until here)
     lds_barrier();
-    it = cur.item;
-    it_signals = I.signals;
-    for (;;) {  // its units
-      const uint32_t un = u + u_step;
-      last = un >= u_end;
-      const SeqUnit next = seq_unit_at(s.units, last ? u : un);
-      if (slot && slot % kSeqDrift == 0) lds_barrier();
-      const bool mine = team * kTileRows < cur.rows;  // whether this wavefront has a record of the unit, and of the next
-      const bool more = !last & (next.item == it) & (team * kTileRows < next.rows);
-      const uint8_t* nrec = next.rec + (more ? team * stride : 0u);
-      const uint32_t table = W.table;
-      const float row_scale = W.scale, tail = W.tail;
-      W.table = next.table[lane & 31u];  // first, so that the next unit waits for them alone
-      W.tail = *reinterpret_cast<const float*>(nrec + (more ? tail_off : 0u));
-      W.scale = reinterpret_cast<const float*>(nrec)[r];
-      float acc = 0.f;
-#pragma unroll
-      for (uint32_t j = 0; j < kSteps; ++j) {
-        const uint32_t step = w + j * split;
-        acc = step_product<DIG>(W.step[j], load_xblock<DIG>(L.planes + (min(step, n_steps) * 8u + bq) * kStr), table, r, acc);
-        __builtin_amdgcn_sched_barrier(0);
-        W.step[j] = load_step(nrec + head, step, more & (step < n_steps), at);
-        __builtin_amdgcn_sched_barrier(0);
+
+    auto store_rows = [&](const Task& t, float v) {
+      const uint32_t row = lane_row(lane);
+      if (lane_class(lane) == 0u && row < t.rows) {
+        if constexpr (kWaits) {  // a later item of this launch may read it from another XCD
+          if constexpr (std::is_same<OutT, __half>::value) store_half<true>(reinterpret_cast<__half*>(t.y) + row, __float2half_rn(v));
+          else __hip_atomic_store(reinterpret_cast<float*>(t.y) + row, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+          store_out<OutT>(t.y, row, v);
+        }
       }
-      acc = row8_sum(acc);
-      if (mine) {
-        float* p = L.part + ((slot % kSeqSlots) * kGemvMaxWaves + wave) * 8u;
-        float* q = L.tpart + ((slot % kSeqSlots) * kGemvMaxWaves + wave) * 8u;
-        if (lane < 8u) p[lane] = acc;
-        if (w < tail_waves) {
-          const float t = row8_sum(tail_c < tail_w ? tail * L.xtail[tail_c] : 0.f);
-          if (lane < 8u) q[lane] = t;
+    };
+    for (uint32_t round = 0; round < rounds; ++round) {
+      if (tasks > 1u && round && round % kSeqDrift == 0) lds_barrier();
+      const Task next = task_of(round + 1u);
+      if (!cur.live) {  // (only in the last round)
+        cur = next;
+        continue;
+      }
+      const uint32_t lanes_table = table;
+      float* const part = L.part + (size_t)(cur.slot * n_steps) * kTileRows;
+      const float row_scale = extras.scale;
+      float t = 0.f;
+      if (cur.part == 0u) t = tile_extras<DIG>(extras, cur.rec, nb, tail_w, cur.list, lanes_table, L, lane);
+      load_head(next);
+      float even = 0.f, odd = 0.f;  // steps 0 and 1 of a tile that is one task, and 2 and 3
+      for (uint32_t step = cur.step; step < cur.end; ++step) {
+        const bool last = step + 1u == cur.end;
+        if (last) table = scale_table(next.table, lane);  // in front of the pieces, so that the next task waits for it alone
+        const uint8_t* base = scalar_base(last ? next.rec : cur.rec);
+        const uint32_t off = last && !next.live ? 0u : step_offset(last ? next.step : step + 1u, units, head, lane);
+        float lo, hi;
+        step_product<DIG>(W, L.planes + (step * kStepUnits + (lane >> 3)) * XPlanes<DIG>::kDwords, lanes_table, lo, hi,
+                          [&](auto piece) __attribute__((always_inline)) { load_piece<decltype(piece)::value>(W, base, off); });
+        const float v = rows_sum(lo, hi);
+        if (tasks == 1u) {
+          if (step & 2u) odd += v;
+          else even += v;
+        } else if (lane_class(lane) == 0u) {
+          part[step * kTileRows + lane_row(lane)] = v;
+        }
+      }
+      if (tasks == 1u) {
+        store_rows(cur, fmaf(even + odd, row_scale, t));
+      } else {
+        if (cur.part == 0u && lane_class(lane) == 0u) {
+          tpart[cur.slot * kTileRows + lane_row(lane)] = t;
+          scales[cur.slot * kTileRows + lane_row(lane)] = row_scale;
         }
         // whoever sees the count complete sees the sums of the wavefronts that counted
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         uint32_t n = 0;
-        if (lane == 0) n = __hip_atomic_fetch_add(arrived + (slot % kSeqSlots) * kGemvMaxWaves + team, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (lane == 0) n = __hip_atomic_fetch_add(arrived + cur.slot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        if (((n + 1u) & (split - 1u)) == 0u) {
-          p -= w * 8u;
-          q -= w * 8u;
-          const float v = team_sum(p, q, row_scale, split, tail_waves, lane);
-          const uint32_t row = team * kTileRows + r;
-          if (lane < 8u && row < cur.rows) {
-            if constexpr (kWaits) {  // a later item of this launch may read it from another XCD
-              if constexpr (std::is_same<OutT, __half>::value) store_half<true>(reinterpret_cast<__half*>(cur.y) + row, __float2half_rn(v));
-              else __hip_atomic_store(reinterpret_cast<float*>(cur.y) + row, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-              store_out<OutT>(cur.y, row, v);
-            }
-          }
+        if (n + 1u == tasks) {
+          const float v = steps_sum<kGemvMaxBlocks / kStepBlocks>(part, n_steps, lane);
+          store_rows(cur, fmaf(v, scales[cur.slot * kTileRows + lane_row(lane)], tpart[cur.slot * kTileRows + lane_row(lane)]));
+          if (lane == 0) __hip_atomic_store(arrived + cur.slot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
       }
-      ++slot;
-      if (last) break;
       cur = next;
-      u = un;
-      if (cur.item != it) break;
     }
-    if (last) break;
+    if (u_next >= u_end) break;
+    u = u_next;
+    first = after;
   }
   if (kWaits && it_signals) signal_item();
 }

@@ -1,6 +1,6 @@
 // C ABI and gfx950 kernels of the fused Leech-lattice dequant-GEMV.
 //
-// Data in HBM, per matrix: the lattice points of its code stream as tiles of 13 bytes per block, with the row scales and
+// Data in HBM, per matrix: the lattice points of its code stream as tiles of 10 bytes per block, with the row scales and
 // tail columns (tiles.h; the stream is unranked once, at upload).  Per runtime: the tables of the unranking.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -504,7 +504,8 @@ struct llvq_mat {
   uint32_t d_out = 0, d_in = 0, nblocks = 0, tail_w = 0;
   uint32_t record_bits = 48;  // 48: 6-byte records (shell cap 12); 49: the dense stream of shell cap 13
   float g[2] = {0, 0};
-  uint8_t* tiles = nullptr;  // device: scale table and records (tiles.h)
+  uint32_t slots = 0, stride = 0;  // places in a tile's list of escapes, bytes of a tile
+  uint8_t* tiles = nullptr;  // device: scale table and tiles (tiles.h)
   uint64_t device_bytes = 0;
   uint64_t encoded_bytes = 0;
   bool has_rotation = false;
@@ -641,7 +642,7 @@ int llvq_hip_runtime_create(int device, void* hip_stream, llvq_rt** out) {
   for (const void* kernel : {reinterpret_cast<const void*>(gemm_tiles_kernel<1, 1, false>), reinterpret_cast<const void*>(gemm_tiles_kernel<1, 1, true>),
                              reinterpret_cast<const void*>(gemm_tiles_kernel<2, 4, false>), reinterpret_cast<const void*>(gemm_tiles_kernel<1, 4, true>),
                              reinterpret_cast<const void*>(gemm_wide_kernel<4, false>), reinterpret_cast<const void*>(gemm_wide_kernel<4, true>),
-                             reinterpret_cast<const void*>(gemm_wide_kernel<8, false>)})
+                             reinterpret_cast<const void*>(gemm_wide_kernel<8, false>), reinterpret_cast<const void*>(gemm_tall_kernel)})
     (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   *out = rt;
   return LLVQ_OK;
@@ -734,15 +735,13 @@ static hipError_t grow_device(uint8_t** buf, size_t* have, size_t need) {
 // rt->uploads held: another upload's copies between this one's and its kernels would end up in this matrix.
 constexpr size_t kUploadBytes = 32u << 20;
 static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids, const float* rscale, const float* tail, const uint8_t* codes) {
-  const uint32_t nb = m->nblocks, stride = tile_stride(nb, m->tail_w), n_tiles = tile_count(m->d_out);
-  const size_t row_bits = (size_t)nb * m->record_bits;  // eight rows are whole bytes whatever the record width
-  const uint32_t rows_per = (uint32_t)std::min<size_t>(m->d_out, std::max<size_t>(8, kUploadBytes * 8 / (row_bits + 32u * (1u + m->tail_w)) / 8 * 8));
-  TileTable table;
-  for (uint32_t i = 0; i < 32; ++i) {
-    const uint32_t shell = i & 15u;
-    table.v[i] = shell ? (float)centroids[i >> 4] * (float)(1.0 / std::sqrt(16.0 * shell)) : 0.f;
-  }
-  hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->tiles), kTileTableBytes + (size_t)n_tiles * stride + kStepBytes + 256);  // a record's last step may reach past it
+  const uint32_t nb = m->nblocks, slots = m->slots, stride = m->stride, n_tiles = tile_count(m->d_out);
+  const size_t row_bits = (size_t)nb * m->record_bits;  // sixteen rows are whole bytes whatever the record width
+  const uint32_t rows_per = (uint32_t)std::min<size_t>(m->d_out, std::max<size_t>(kTileRows, kUploadBytes * 8 / (row_bits + 32u * (1u + m->tail_w)) / kTileRows * kTileRows));
+  TileTable table{};
+  for (uint32_t gain = 0; gain < 2; ++gain)
+    for (uint32_t shell = 2; shell <= (uint32_t)kMaxShell; ++shell) table.v[gain * 12u + shell - 2u] = (float)centroids[gain] * (float)(1.0 / std::sqrt(16.0 * shell));
+  hipError_t e = hipMalloc(reinterpret_cast<void**>(&m->tiles), kTileTableBytes + (size_t)n_tiles * stride + kUnitBytes + 256);  // a tile without a block is read as if it had one
   if (e != hipSuccess) return e;
   const size_t code_room = ((row_bits * rows_per + 7) / 8 + 16 + 255) & ~(size_t)255;
   const size_t scale_room = ((size_t)rows_per * 4 + 255) & ~(size_t)255, tail_room = (size_t)rows_per * m->tail_w * 4;
@@ -758,19 +757,23 @@ static hipError_t upload_tiles(llvq_rt* rt, llvq_mat* m, const double* centroids
     if (bytes && (e = hipMemcpyAsync(d_codes, codes + row_bits * r0 / 8, bytes, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
     if ((e = hipMemcpyAsync(d_scale, rscale + r0, (size_t)rows * 4, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
     if (m->tail_w && (e = hipMemcpyAsync(d_tail, tail + (size_t)r0 * m->tail_w, (size_t)rows * m->tail_w * 4, hipMemcpyHostToDevice, rt->stream)) != hipSuccess) return e;
-    const uint32_t heads = tile_count(rows) * kTileRows * (1u + m->tail_w);
+    const uint32_t heads = tile_count(rows) * kTileRows * (1u + 4u * tail_depth(m->tail_w));
     hipLaunchKernelGGL(tile_heads_kernel, dim3((heads + 255u) / 256u), dim3(256), 0, rt->stream, table,
-                       r0 ? (float*)nullptr : reinterpret_cast<float*>(m->tiles), d_scale, d_tail, out, rows, nb, m->tail_w);
+                       r0 ? (float*)nullptr : reinterpret_cast<float*>(m->tiles), d_scale, d_tail, out, rows, nb, m->tail_w, slots);
     if (nb) {
-      const uint64_t blocks = (uint64_t)tile_count(rows) * kTileRows * nb;
-      const uint32_t grid = (uint32_t)std::min<uint64_t>((blocks + 511) / 512, 2ull * cus);
-      if (m->record_bits == 48) hipLaunchKernelGGL(transcode_kernel<false>, dim3(grid), dim3(512), kLdsImageBytes, rt->stream, rt->tables, d_codes, out, rows, nb, m->tail_w);
-      else hipLaunchKernelGGL(transcode_kernel<true>, dim3(grid), dim3(512), kLdsImageBytes, rt->stream, rt->tables, d_codes, out, rows, nb, m->tail_w);
+      const uint64_t units = (uint64_t)tile_count(rows) * tile_units(nb);
+      const uint32_t grid = (uint32_t)std::min<uint64_t>((units + 7) / 8, 2ull * cus);
+      if (m->record_bits == 48) hipLaunchKernelGGL(transcode_kernel<false>, dim3(grid), dim3(512), kLdsImageBytes, rt->stream, rt->tables, d_codes, out, rows, nb, m->tail_w, slots);
+      else hipLaunchKernelGGL(transcode_kernel<true>, dim3(grid), dim3(512), kLdsImageBytes, rt->stream, rt->tables, d_codes, out, rows, nb, m->tail_w, slots);
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
+  if (slots) {
+    hipLaunchKernelGGL(sort_lists_kernel, dim3((n_tiles + 3u) / 4u), dim3(256), 0, rt->stream, m->tiles + kTileTableBytes, n_tiles, stride, slots);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
   e = hipStreamSynchronize(rt->stream);
-  if (rt->upload_bytes > kUploadBytes + 1024) {  // eight rows that exceed it by themselves: not kept
+  if (rt->upload_bytes > kUploadBytes + 1024) {  // sixteen rows that exceed it by themselves: not kept
     (void)hipFree(rt->upload_buf);
     rt->upload_buf = nullptr;
     rt->upload_bytes = 0;
@@ -835,6 +838,8 @@ static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uin
   m->nblocks = nblocks;
   m->tail_w = tail_w;
   m->record_bits = record_bits;
+  m->slots = list_slots(nblocks, record_bits != 48u);
+  m->stride = tile_stride(nblocks, tail_w, m->slots);
   m->g[0] = (float)centroids[0];  // fused.rs:1209
   m->g[1] = (float)centroids[1];
   std::vector<float> rs(d_out);
@@ -847,7 +852,7 @@ static int upload_impl(llvq_rt* rt, const std::string& name, uint32_t d_out, uin
     delete m;
     return hip_fail(e, "upload_tiles");
   }
-  m->device_bytes = kTileTableBytes + (uint64_t)tile_count(d_out) * tile_stride(nblocks, tail_w);
+  m->device_bytes = kTileTableBytes + (uint64_t)tile_count(d_out) * m->stride;
   m->encoded_bytes = code_len + (uint64_t)d_out * 8 + tail_len + 16;
   *out = m;
   return LLVQ_OK;
@@ -1005,21 +1010,21 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   a.nb = m0->nblocks;
   a.tail_w = m0->tail_w;
   a.n_mats = (uint32_t)n;
-  a.split_shift = gemv_split_shift(m0->nblocks);
+  a.team = gemv_team(m0->nblocks);
   for (int i = 0; i < n; ++i) {
-    a.m[i] = TileMat{mats[i]->tiles, y[i], mats[i]->d_out, a.n_tiles};
+    a.m[i] = TileMat{mats[i]->tiles, y[i], mats[i]->d_out, a.n_tiles, mats[i]->stride, mats[i]->slots};
     a.n_tiles += tile_count(mats[i]->d_out);
   }
-  // Teams go to as many CUs as there are records for, then to the same CU, up to sixteen wavefronts: a small launch
+  // Teams go to as many CUs as there are tiles for, then to the same CU, up to sixteen wavefronts: a small launch
   // is short because every CU has a part of it, a large one because a CU keeps sixteen wavefronts' loads in flight.
-  // The in-launch rotation and the wide rows are written for a full workgroup.
-  const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), most = kGemvMaxWaves >> a.split_shift;
-  uint32_t teams = (a.n_tiles + cus - 1u) / cus;
-  if (teams > most || rotated || gemv_wide(a.nb)) teams = most;
-  const uint32_t grid = std::min(cus, (a.n_tiles + teams - 1u) / teams);
+  // The in-launch rotation and the wide rows are written for a full workgroup, whatever of it has a tile.
+  const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
+  a.teams = std::min((a.n_tiles + cus - 1u) / cus, kGemvMaxWaves / a.team);
+  const uint32_t grid = std::min(cus, (a.n_tiles + a.teams - 1u) / a.teams);
+  const uint32_t waves = rotated || gemv_wide(a.nb) ? kGemvMaxWaves : a.teams * a.team;
   const int src = rotated ? kSrcRotated : a.in.prologue == kPrologueSiluMul ? kSrcSiluMul : a.in.prologue == kPrologueAddRmsNorm ? kSrcAddRmsNorm : kSrcF16;
   void* params[] = {&a};
-  HIP_TRY(hipLaunchKernel(gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(grid), dim3((teams << a.split_shift) * 64u), params,
+  HIP_TRY(hipLaunchKernel(gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(grid), dim3(waves * 64u), params,
                           gemv_tiles_lds_bytes(a.nb, m0->d_in, f32, rot != nullptr), rt->stream));
   return LLVQ_OK;
 }
@@ -1170,23 +1175,34 @@ static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) 
   }
   const bool f32 = specs[0].y_dtype == LLVQ_F32;
   bool prologue = false, wide = false;
-  uint32_t max_blocks = 0;
+  uint32_t max_units = 0;
   for (int i = 0; i < n; ++i) {
     prologue |= specs[i].pro.kind != kPrologueNone;
     wide |= gemv_wide(specs[i].mats[0]->nblocks);
-    max_blocks = std::max(max_blocks, gemv_plane_blocks(specs[i].mats[0]->nblocks));
+    max_units = std::max(max_units, gemv_plane_units(specs[i].mats[0]->nblocks));
   }
-  const size_t lds = gemv_seq_lds_bytes(max_blocks, f32);
+  const size_t lds = gemv_seq_lds_bytes(max_units, f32);
   if (lds > 160 * 1024) return fail(LLVQ_ERR_UNSUPPORTED, "sequence_create: the widest rows do not fit the LDS activation tile");
   const uint32_t grid_cap = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
   std::vector<SeqUnit> units;
   std::vector<SeqItem> items((size_t)n);
-  std::vector<uint64_t> cost;  // bytes of the units so far, behind each unit
-  uint64_t bytes = 0;
+  uint64_t bytes = 0, n_tiles = 0;
+  for (int i = 0; i < n; ++i)
+    for (int j = 0; j < specs[i].n; ++j) {
+      const llvq_mat* m = specs[i].mats[j];
+      n_tiles += tile_count(m->d_out);
+      bytes += (uint64_t)tile_count(m->d_out) * m->stride;
+    }
+  // Independent items: runs of equal bytes, workgroup b's ending at the tile with which all before it make up (b + 1) / grid
+  // of them; a unit is what a workgroup has of a matrix.  Ordered ones are spread over all workgroups as a launch of their
+  // own would be, unit after unit: everyone waits for the slowest.
+  uint32_t grid = (uint32_t)std::min<uint64_t>(n_tiles, grid_cap);
+  std::vector<uint32_t> runs{0};
+  uint64_t done = 0;
   for (int i = 0; i < n; ++i) {
     const SeqSpec& sp = specs[i];
     const llvq_mat* m0 = sp.mats[0];
-    const uint32_t nb = m0->nblocks, stride = tile_stride(nb, m0->tail_w), per = (kGemvMaxWaves >> gemv_split_shift(nb)) * kTileRows;
+    const uint32_t nb = m0->nblocks, steps = tile_steps(nb);
     SeqItem& I = items[(size_t)i];
     std::memset(&I, 0, sizeof I);
     I.x = reinterpret_cast<const __half*>(sp.x);
@@ -1200,42 +1216,44 @@ static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) 
     I.first_unit = (uint32_t)units.size();
     I.wait_item = sp.after_previous ? (uint32_t)(i - 1) : kSeqNoWait;
     I.signals = (i + 1 < n && specs[i + 1].after_previous) ? 1u : 0u;
+    I.tasks = std::max(1u, dependent ? steps : (steps + kSeqTaskSteps - 1u) / kSeqTaskSteps);
+    I.inv_tasks = I.tasks > 1u ? (uint32_t)(((1ull << 32) + I.tasks - 1u) / I.tasks) : 0u;
     const size_t ysz = f32 ? 4 : 2;
     for (int j = 0; j < sp.n; ++j) {
       const llvq_mat* m = sp.mats[j];
-      // Ordered items are spread over all workgroups as a launch of their own would be: everyone waits for the slowest.
-      uint32_t rows_per = per;
-      if (dependent) rows_per = std::min(per, std::max(1u, (tile_count(m->d_out) + grid_cap - 1u) / grid_cap) * kTileRows);
-      for (uint32_t r0 = 0; r0 < m->d_out; r0 += rows_per) {
+      const uint32_t tiles = tile_count(m->d_out), stride = m->stride;
+      for (uint32_t t0 = 0, count; t0 < tiles; t0 += count) {
+        if (dependent) {
+          count = (tiles + grid_cap - 1u) / grid_cap;
+        } else {
+          uint64_t want;  // the end of the run that the tile begins in
+          while ((want = bytes * runs.size() / grid) <= done) runs.push_back((uint32_t)units.size());
+          count = (uint32_t)((want - done + stride - 1u) / stride);
+        }
+        count = std::min(count, tiles - t0);
         SeqUnit t{};
-        t.rec = m->tiles + kTileTableBytes + (size_t)(r0 / kTileRows) * stride;
+        t.rec = m->tiles + kTileTableBytes + (size_t)t0 * stride;
         t.table = reinterpret_cast<const uint32_t*>(m->tiles);
-        t.y = reinterpret_cast<uint8_t*>(sp.y[j]) + (size_t)r0 * ysz;
-        t.rows = std::min(rows_per, m->d_out - r0);
+        t.y = reinterpret_cast<uint8_t*>(sp.y[j]) + (size_t)t0 * kTileRows * ysz;
+        t.rows = std::min(count * kTileRows, m->d_out - t0 * kTileRows);
         t.item = (uint32_t)i;
+        t.stride = stride;
+        t.slots = m->slots;
         units.push_back(t);
-        bytes += (uint64_t)tile_count(t.rows) * stride + 1024u;
-        cost.push_back(bytes);
+        done += (uint64_t)count * stride;
       }
     }
   }
   if (units.size() > 0x7FFFFFFFu) return fail(LLVQ_ERR_UNSUPPORTED, "sequence_create: too many units");
   const uint32_t n_units = (uint32_t)units.size();
-  const uint32_t grid = std::min(n_units, grid_cap);
+  if (dependent) grid = std::min(n_units, grid_cap);
+  runs.resize((size_t)grid + 1, n_units);
   for (int i = 0; i < n; ++i) {
     const uint32_t t0 = items[(size_t)i].first_unit, t1 = i + 1 < n ? items[(size_t)i + 1].first_unit : n_units;
     items[(size_t)i].expected = std::min(t1 - t0, grid);
   }
   for (int i = 0; i < n; ++i)
     if (items[(size_t)i].wait_item != kSeqNoWait) items[(size_t)i].wait_expected = items[items[(size_t)i].wait_item].expected;
-  // runs of equal bytes: workgroup b ends where the units before its end make up (b + 1) / grid of all bytes
-  std::vector<uint32_t> runs((size_t)grid + 1);
-  for (uint32_t b = 0, at = 0; b < grid; ++b) {
-    runs[b] = at;
-    const uint64_t want = bytes * (b + 1) / grid;
-    while (at < n_units && (b + 1 == grid || cost[at] <= want)) ++at;
-  }
-  runs[grid] = n_units;
   HIP_TRY(hipSetDevice(rt->device));
   auto* q = new llvq_seq();
   const size_t off_items = units.size() * sizeof(SeqUnit);
@@ -1257,7 +1275,7 @@ static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) 
   q->args.items = reinterpret_cast<const SeqItem*>(q->blob + off_items);
   q->args.runs = dependent ? nullptr : reinterpret_cast<const uint32_t*>(q->blob + off_runs);
   q->args.n_units = n_units;
-  q->args.max_blocks = max_blocks;
+  q->args.max_units = max_units;
   q->args.counters = reinterpret_cast<uint32_t*>(q->blob + off_counters);
   q->args.status = reinterpret_cast<uint32_t*>(q->blob + off_status);
   q->own_status = q->args.status;
@@ -1390,15 +1408,16 @@ constexpr uint32_t kGemmMaxM = 1024;
 static uint32_t gemm_chunk(uint32_t nb, bool pair) { return pair && (nb + 3u) / 4u * 12u > 2048u ? kGemmMaxM / 2 : kGemmMaxM; }
 static_assert((kGemvMaxBlocks + 3) / 4 * 12 * (kGemmMaxM / 2) * 16 <= (32u << 20) && 2048u * kGemmMaxM * 16 <= (32u << 20), "octets of a launch");
 
-// Measured times of one step (48 columns) of the wide kernel in us: 256 activation rows; 128, two workgroups sharing a
-// CU, each; one of those alone; and 128 with both terms of the weights.
-constexpr double kWideStep = 1.28, kWideHalfStep = 0.69, kWideHalfStepAlone = 0.8, kWidePairStep = 2.4;
+// Measured times of one step (48 columns) of the wide kernel in us (85 steps less 8, back to back): 256 weight rows by 256
+// activation rows; 384 by 128; 256 by 128, two workgroups sharing a CU, each; one of those alone; and with both terms of the
+// weights.
+constexpr double kWideStep = 1.21, kTallStep = 1.12, kWideHalfStep = 0.76, kWideHalfStepAlone = 0.80, kWidePairStep = 2.5;
 
 // How a batched launch over these matrices at M rows is cut up, and the workspaces it needs.  pair: with both terms of
 // the weights (gemm_same_basis says when).
 struct GemmPlan {
   uint32_t small;                // 1: up to 16 rows, 2: up to 64 (gemm_tiles_kernel), 0: gemm_wide_kernel
-  uint32_t cf, rows_per_tile;    // the wide kernel's form, and weight rows of a workgroup
+  uint32_t rf, cf, rows_per_tile;  // the wide kernel's form, and weight rows of a workgroup
   uint32_t n_tiles, m_pad, m_tiles, splits, steps_per_split, n_oct;
   size_t ws_bytes, xt_bytes;
 };
@@ -1411,10 +1430,15 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
   p.small = M <= 16u ? 1u : M <= kGemmSmallRows ? 2u : 0u;
   p.splits = 1;
   p.m_tiles = 1;
-  p.rows_per_tile = !p.small ? kWideRows : pair ? 16u : p.small * 16u;
-  for (int i = 0; i < n; ++i) p.n_tiles += (mats[i]->d_out + p.rows_per_tile - 1u) / p.rows_per_tile;
+  p.rows_per_tile = pair ? 16u : p.small * 16u;
+  const auto tiles_of = [&](uint32_t rows) {
+    uint32_t sum = 0;
+    for (int i = 0; i < n; ++i) sum += (mats[i]->d_out + rows - 1u) / rows;
+    return sum;
+  };
   p.n_oct = (nb + 3u) / 4u * 12u;
   if (p.small) {
+    p.n_tiles = tiles_of(p.rows_per_tile);
     p.m_pad = p.small == 1u ? 16u : 64u;
     p.xt_bytes = (size_t)p.n_oct * p.m_pad * 16;
     return p;
@@ -1425,16 +1449,19 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
   // place holds the octets of either plan, and needs no partial sums for rows that hardly ever come.)
   const uint32_t steps = (nb + 1u) / 2u, most = pair && mats[0]->d_in % 8 == 0 ? 1u : 16u;
   double best = 1e30;
-  for (uint32_t cf = pair ? 4u : 8u; cf >= 4u; cf -= 4u) {
-    const uint32_t m_tiles = (M + 32u * cf - 1u) / (32u * cf), tiles = p.n_tiles * m_tiles, m_pad = m_tiles * 32u * cf;
-    const size_t one = (size_t)m_pad * p.n_tiles * kWideRows * sizeof(float);
-    for (uint32_t sp = 1; sp <= most && (sp == 1u || (steps / sp >= 8u && one * sp <= kGemmWsCap)); ++sp) {
-      const uint32_t per = (steps + sp - 1u) / sp, wgs = tiles * ((steps + per - 1u) / per), per_cu = (wgs + cus - 1u) / cus;
-      const double cost = (pair ? per_cu * kWidePairStep : cf == 8u ? per_cu * kWideStep : per_cu == 1u ? kWideHalfStepAlone : per_cu * kWideHalfStep) * per +
-                          (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
+  const auto weigh = [&](uint32_t rf, uint32_t cf, size_t ws_cap) {
+    const uint32_t rows = 128u * rf, n_tiles = tiles_of(rows), m_tiles = (M + 32u * cf - 1u) / (32u * cf), m_pad = m_tiles * 32u * cf;
+    const size_t one = (size_t)m_pad * n_tiles * rows * sizeof(float);
+    for (uint32_t sp = 1; sp <= most && (sp == 1u || (steps / sp >= 8u && one * sp <= ws_cap)); ++sp) {
+      const uint32_t per = (steps + sp - 1u) / sp, wgs = n_tiles * m_tiles * ((steps + per - 1u) / per), per_cu = (wgs + cus - 1u) / cus;
+      const double step = pair ? kWidePairStep : rf == 3u ? kTallStep : cf == 8u ? kWideStep : per_cu == 1u ? kWideHalfStepAlone : kWideHalfStep;
+      const double cost = per_cu * step * per + (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
       if (cost < best) {
         best = cost;
+        p.rf = rf;
         p.cf = cf;
+        p.rows_per_tile = rows;
+        p.n_tiles = n_tiles;
         p.m_tiles = m_tiles;
         p.m_pad = m_pad;
         p.splits = (steps + per - 1u) / per;
@@ -1442,7 +1469,11 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
         p.ws_bytes = p.splits > 1u ? one * p.splits : 0;
       }
     }
-  }
+  };
+  if (!pair) weigh(2u, 8u, kGemmWsCap);
+  weigh(2u, 4u, kGemmWsCap);
+  // (384 rows never with more workspace than the best of 256: where a call has to fit a given one it fits as before)
+  if (!pair) weigh(3u, 4u, p.ws_bytes);
   p.xt_bytes = (size_t)p.n_oct * p.m_pad * 16;
   return p;
 }
@@ -1506,7 +1537,7 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   a.ws = reinterpret_cast<float*>(ws_buf);
   a.n_mats = (uint32_t)n;
   for (int i = 0; i < n; ++i) {
-    a.mat[i] = GemmMat{mats[i]->tiles, y[i], mats[i]->d_out, a.n_tiles};
+    a.mat[i] = GemmMat{mats[i]->tiles, y[i], mats[i]->d_out, a.n_tiles, mats[i]->stride, mats[i]->slots};
     a.n_tiles += (mats[i]->d_out + p.rows_per_tile - 1u) / p.rows_per_tile;
   }
   a.y_f32 = y_dtype == LLVQ_F32 ? 1u : 0u;
@@ -1526,8 +1557,11 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
     constexpr bool kPair = decltype(pair)::value;
     if (p.small == 1u) hipLaunchKernelGGL((gemm_tiles_kernel<1, 1, kPair>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<1, 1>()), rt->stream, a);
     else if (p.small) hipLaunchKernelGGL((gemm_tiles_kernel<kPair ? 1 : 2, 4, kPair>), dim3(a.n_tiles), dim3(1024), (gemm_small_lds<kPair ? 1 : 2, 4>()), rt->stream, a);
-    else if (p.cf == 4u) hipLaunchKernelGGL((gemm_wide_kernel<4, kPair>), wide_grid, dim3(256), gemm_wide_lds<4>(), rt->stream, a);
-    else if constexpr (!kPair) hipLaunchKernelGGL((gemm_wide_kernel<8, false>), wide_grid, dim3(256), gemm_wide_lds<8>(), rt->stream, a);
+    else if (p.rf == 2u && p.cf == 4u) hipLaunchKernelGGL((gemm_wide_kernel<4, kPair>), wide_grid, dim3(256), (gemm_wide_lds<2, 4, kPair>()), rt->stream, a);
+    else if constexpr (!kPair) {
+      if (p.rf == 3u) hipLaunchKernelGGL(gemm_tall_kernel, wide_grid, dim3(256), (gemm_wide_lds<3, 4, false>()), rt->stream, a);
+      else hipLaunchKernelGGL((gemm_wide_kernel<8, false>), wide_grid, dim3(256), (gemm_wide_lds<2, 8, false>()), rt->stream, a);
+    }
   };
   if (pair) product(std::true_type{});
   else product(std::false_type{});

@@ -2,54 +2,98 @@
 //
 // A code stream is unranked once, on the device, when its matrix is uploaded: unranking costs about 500 vector
 // instructions per block, and a product that repeats it is bound by them at 5 % of what HBM delivers (2.26 ms for the
-// 150.7 M blocks of a 4B model, 434 GB/s of codes).  A lattice point's 24 coordinates are all even or all odd and at
-// most 13 in magnitude, so v = 2 n + p with one bit p per block and n in [-8, 7]: 12 bytes of nibbles and one byte for
-// p, the gain bit and the shell.  Nothing is rounded; what a kernel rebuilds from 13 bytes is the integer point itself.
+// 150.7 M blocks of a 4B model, 434 GB/s of codes).  What is kept of a block are the ten bytes of block_code.h, the
+// integer point itself; 13 (4-bit coordinates and a byte) were 23 % more to read.
 //
-//   matrix: 32 floats (gain centroid / sqrt(16 shell), indexed gain << 4 | shell; shell 0, the origin, gives 0),
-//           then one record per 8 rows:
-//             8 row scales (f32), tail_w x 8 tail values (f32, column by column), nb blocks of 104 bytes
-//   block:  8 rows x 12 bytes of nibbles, then 8 rows x 1 byte (gain << 4 | shell) << 2 | p
-//   nibble q of dword j holds column 8 j + {0, 2, 4, 6, 1, 3, 5, 7}[q], two's complement: nibbles q and q + 4 are
-//           neighbouring columns in the two halves of the dword, which is what a packed binary16 unpack wants, and a
-//           dword is the operand of an 8-wide 4-bit dot product.
+//   matrix: 32 floats (the block scales, centroid / sqrt(16 shell), in the order of block_code.h's slots, zeros behind
+//           them), then one tile per 16 rows:
+//             16 row scales (f32), the number of escapes in it and 60 bytes of nothing; the tail columns (tail_at), 64 lanes
+//             of (tail_w + 3) / 4 floats; the units of four blocks; the list of escapes
+//   unit:   640 bytes, five 128-byte lines of eight 16-byte pieces, piece l of a line being of rows l and l + 8:
+//             {d0, d1} of blocks 0 and 1 of row l; of blocks 2 and 3; the same two lines of row l + 8;
+//             {s, meta} of row l, {s, meta} of row l + 8, four blocks in a dword
+//           nibble q of a dword holds column 8 j + {0, 2, 4, 6, 1, 3, 5, 7}[q]: nibbles q and q + 4 are neighbouring
+//           columns in the two halves of the dword, which is what a packed binary16 unpack wants, and a dword is the
+//           operand of an 8-wide 4-bit dot product.
 //
-// Eight rows of eight consecutive blocks are 832 consecutive bytes: one step of a wavefront, each lane one (row, block).
+//   escape: a block whose code says kBlockEscape or more (block_code.h), as 16 bytes: the nibbles n of v = 2 n + odd, and
+//           row << 28 | block << 9 | odd << 8 | slot, in the order of these, zeros behind them.  The products, in which a
+//           wavefront would take block_escape's path for one of its lanes at a time, take such blocks for zero where they
+//           meet them (their slot's scale is) and make up for it from the list.  Where a tile has more of them than
+//           list_slots (all of them, or by chance) its list does not count and they read the codes.
+//
+// Eight units are a step of a wavefront, 5120 consecutive bytes: lane (l, q) = (lane % 8, lane / 8) loads the five pieces l
+// of unit q.  Every line of memory is asked for by one load, whole, and marked as not to be kept: read like that the card
+// delivers 6.9 TB/s (a loop of nothing else, 8 or 16 wavefronts on a CU), without the mark 6.1, and 5.9 where 12-byte
+// pieces and their bytes of meta are asked for by two loads that share lines (there the mark makes it 5.4).
 #pragma once
+
+#include "block_code.h"
 
 namespace llvq {
 
-constexpr uint32_t kTileRows = 8;
-constexpr uint32_t kTileBlockBytes = 104;
-constexpr uint32_t kTileTableBytes = 128;
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
-__host__ __device__ inline uint32_t tile_head_bytes(uint32_t tail_w) { return 32u + 32u * tail_w; }
-// bytes of one record of eight rows (its blocks start 32-byte aligned)
-__host__ __device__ inline uint32_t tile_stride(uint32_t nb, uint32_t tail_w) {
-  return tile_head_bytes(tail_w) + ((nb * kTileBlockBytes + 31u) & ~31u);
+constexpr uint32_t kTileRows = 16;
+constexpr uint32_t kUnitBytes = 640;
+constexpr uint32_t kStepUnits = 8;
+constexpr uint32_t kStepBlocks = 4 * kStepUnits;
+constexpr uint32_t kTileTableBytes = kScaleSlots * 4;
+
+// Floats of a row's tail columns that a lane of its four holds: column c is the (c / 4)-th of lane class c % 4.
+__host__ __device__ inline uint32_t tail_depth(uint32_t tail_w) { return (tail_w + 3u) >> 2; }
+__host__ __device__ inline uint32_t tile_head_bytes(uint32_t tail_w) { return 128u + 256u * tail_depth(tail_w); }
+__host__ __device__ inline uint32_t tile_units(uint32_t nb) { return (nb + 3u) >> 2; }
+__host__ __device__ inline uint32_t tile_steps(uint32_t nb) { return (nb + kStepBlocks - 1u) / kStepBlocks; }
+// Places in a tile's list, a multiple of eight: of uniformly drawn points of shells 2..12 0.08 % are escapes (with shell 13
+// 0.4 %), so as many as a tile has of them on average and four deviations more.  (Shell 13 takes no batched products, whose
+// kernels have room for 32.)
+constexpr uint32_t kMaxListSlots = 32, kMaxListSlots13 = 64;
+__host__ inline uint32_t list_slots(uint32_t nb, bool shell13) {
+  if (nb == 0) return 0u;
+  const double mean = kTileRows * (double)nb * (shell13 ? 4.1e-3 : 0.85e-3), want = mean + 4. * std::sqrt(mean) + 8.;
+  const uint32_t most = shell13 ? kMaxListSlots13 : kMaxListSlots;
+  return want < most ? (uint32_t)want / 8u * 8u : most;
 }
+// bytes of one tile of sixteen rows, a multiple of 128
+__host__ __device__ inline uint32_t tile_stride(uint32_t nb, uint32_t tail_w, uint32_t slots) {
+  return tile_head_bytes(tail_w) + tile_units(nb) * kUnitBytes + slots * 16u;
+}
+__host__ __device__ inline uint32_t list_at(uint32_t nb, uint32_t tail_w) { return tile_head_bytes(tail_w) + tile_units(nb) * kUnitBytes; }
+constexpr uint32_t kCountAt = 64;  // byte of a tile at which the number of its escapes is
 __host__ __device__ inline uint32_t tile_count(uint32_t d_out) { return (d_out + kTileRows - 1u) / kTileRows; }
+// The lane that holds row r's class c, wherever sixteen rows meet four classes: what two exchanges, across 8 and 16 lanes,
+// add up are the classes of one row.
+__host__ __device__ inline uint32_t row_lane(uint32_t r, uint32_t c) { return (r & 7u) | c << 3 | (r >> 3) << 5; }
+__host__ __device__ inline uint32_t lane_row(uint32_t lane) { return (lane & 7u) | (lane >> 5) << 3; }
+__host__ __device__ inline uint32_t lane_class(uint32_t lane) { return (lane >> 3) & 3u; }
+// float of a tile that holds tail column c of row r
+__host__ __device__ inline uint32_t tail_at(uint32_t r, uint32_t c, uint32_t tail_w) { return 32u + row_lane(r, c & 3u) * tail_depth(tail_w) + (c >> 2); }
 
 // ---- upload: code stream -> tiles ---------------------------------------------------------------
-// One lane per block; lane % 8 is the row inside a record, so that a wavefront writes whole records.  The lanes of a
-// wavefront take both coset programs (about 800 instructions per block, 3 ms for a 4B model's blocks): an upload is
-// bound by the copy of the codes over PCIe, twenty times that.
+// One lane per block, a wavefront a unit: lane % 4 is the block in it, lane / 4 the row.  The lanes of a wavefront take
+// both coset programs (about 800 instructions per block, and 250 for the code, 4 ms for a 4B model's blocks): an upload is
+// bound by the copy of the codes over PCIe, fifteen times that.
 // `rows` rows; codes and tiles are those rows' own.
+__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);
+  return v | (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false);
+}
 template <bool WIDE>
 __global__ __launch_bounds__(512) void transcode_kernel(GlobalTables g, const uint8_t* __restrict__ codes, uint8_t* __restrict__ tiles,
-                                                        uint32_t rows, uint32_t nb, uint32_t tail_w) {
+                                                        uint32_t rows, uint32_t nb, uint32_t tail_w, uint32_t slots) {
   extern __shared__ __align__(16) uint8_t smem[];
   const DecodeTables T = stage_tables<WIDE>(smem, g);
   __syncthreads();
-  const uint32_t stride = tile_stride(nb, tail_w), head = tile_head_bytes(tail_w);
-  const uint64_t padded = (uint64_t)tile_count(rows) * kTileRows * nb;
-  for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < padded; k += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t r = (uint32_t)(k & 7u);
-    const uint64_t tb = k >> 3;
-    const uint32_t tile = (uint32_t)tb / nb, b = (uint32_t)tb - tile * nb;  // the host keeps a launch's blocks below 2^32
-    const uint32_t row = tile * kTileRows + r;
-    uint32_t w0 = 0, w1 = 0, w2 = 0, meta = 0;
-    if (row < rows) {
+  const uint32_t stride = tile_stride(nb, tail_w, slots), head = tile_head_bytes(tail_w), per_tile = tile_units(nb);
+  const uint32_t units = tile_count(rows) * per_tile;  // (the host keeps a launch's blocks below 2^32)
+  const uint32_t lane = threadIdx.x & 63u, k = lane & 3u, r = lane >> 2, waves = blockDim.x >> 6;
+  for (uint32_t u = blockIdx.x * waves + (threadIdx.x >> 6); u < units; u += gridDim.x * waves) {
+    const uint32_t tile = u / per_tile, in_tile = u - tile * per_tile;
+    const uint32_t row = tile * kTileRows + r, b = in_tile * 4u + k;
+    uint32_t w[3] = {0, 0, 0}, par = 0, gain = 0, shell = 0;
+    if (row < rows && b < nb) {
       const uint64_t at = (uint64_t)row * nb + b;
       uint64_t rec;
       if constexpr (WIDE) {  // block `at` is the 49 bits from bit 49 at on; the staged stream has slack behind it
@@ -61,39 +105,67 @@ __global__ __launch_bounds__(512) void transcode_kernel(GlobalTables g, const ui
       } else {
         rec = read_record(codes, 6 * at);
       }
-      uint32_t par = 0;
       const int ci = decode_index(T, rec >> 1, [&](int p, int v) {
         const uint32_t nib = ((uint32_t)(v >> 1) & 15u) << (4u * (((uint32_t)p & 7u) >> 1) + 16u * ((uint32_t)p & 1u));
         par = (uint32_t)v & 1u;
-        if (p < 8) w0 |= nib;
-        else if (p < 16) w1 |= nib;
-        else w2 |= nib;
+        if (p < 8) w[0] |= nib;
+        else if (p < 16) w[1] |= nib;
+        else w[2] |= nib;
       });
-      if (ci >= 0) meta = ((((uint32_t)rec & 1u) << 4) | T.cls[ci].shell) << 2 | par;
+      if (ci >= 0) {
+        gain = (uint32_t)rec & 1u;
+        shell = T.cls[ci].shell;
+      }
     }
-    uint8_t* out = tiles + (size_t)tile * stride + head + (size_t)b * kTileBlockBytes;
-    uint32_t* wout = reinterpret_cast<uint32_t*>(out + r * 12u);
-    wout[0] = w0;
-    wout[1] = w1;
-    wout[2] = w2;
-    out[96u + r] = (uint8_t)meta;
+    BlockCode c;
+    block_encode(w, par, gain, shell, c);
+    const uint32_t s = quad_or(c.s << k), meta = quad_or(c.meta << (8u * k));
+    if (c.meta >= kBlockEscape && slots) {
+      uint8_t* t = tiles + (size_t)tile * stride;
+      const uint32_t e = atomicAdd(reinterpret_cast<uint32_t*>(t + kCountAt), 1u);
+      if (e < slots) *reinterpret_cast<uint4*>(t + stride - slots * 16u + e * 16u) = make_uint4(w[0], w[1], w[2], r << 28 | b << 9 | par << 8 | (gain * 12u + shell - 2u));
+    }
+    uint8_t* out = tiles + (size_t)tile * stride + head + (size_t)in_tile * kUnitBytes + (r & 7u) * 16u;
+    *reinterpret_cast<uint2*>(out + ((r >> 3) * 2u + (k >> 1)) * 128u + (k & 1u) * 8u) = make_uint2(c.d0, c.d1);
+    if (k == 0) *reinterpret_cast<uint2*>(out + 512u + (r >> 3) * 8u) = make_uint2(s, meta);
   }
 }
 
-// Row scales and tail columns into the records' heads (zeros for rows past the last), the matrix's block scales to
-// `table_out` where that is given (as an argument: a copy of 128 bytes from the host costs an upload 15 us).
-struct TileTable { float v[kTileTableBytes / 4]; };
+// The lists in order, behind transcode_kernel, whose lanes put an escape wherever there was room: a wavefront per tile, a
+// lane per escape, which goes where as many lie before it.
+__global__ __launch_bounds__(256) void sort_lists_kernel(uint8_t* __restrict__ tiles, uint32_t n_tiles, uint32_t stride, uint32_t slots) {
+  const uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  if (tile >= n_tiles) return;
+  uint8_t* t = tiles + (size_t)tile * stride;
+  const uint32_t count = *reinterpret_cast<const uint32_t*>(t + kCountAt);
+  uint4* list = reinterpret_cast<uint4*>(t + stride - slots * 16u);
+  if (count > slots) {
+    if (lane == 0) list[0].w = 0xFFFFFFFFu;  // for those who read the list alone
+    return;
+  }
+  const uint4 mine = list[min(lane, slots - 1u)];
+  uint32_t before = 0;
+  for (uint32_t e = 0; e < count; ++e) before += (uint32_t)__shfl((int)mine.w, (int)e) < mine.w ? 1u : 0u;
+  if (lane < count) list[before] = mine;
+  else if (lane < slots) list[lane] = make_uint4(0, 0, 0, 0);
+}
+
+// Row scales, the escapes' counters (zero) and tail columns into the tiles' heads (zeros for rows past the last and columns that are not there), the
+// matrix's block scales to `table_out` where that is given (as an argument: a copy of 128 bytes from the host costs an
+// upload 15 us).
+struct TileTable { float v[kScaleSlots]; };
 __global__ __launch_bounds__(256) void tile_heads_kernel(TileTable table, float* table_out, const float* __restrict__ rscale, const float* __restrict__ tail, uint8_t* __restrict__ tiles,
-                                                         uint32_t rows, uint32_t nb, uint32_t tail_w) {
-  if (table_out && blockIdx.x == 0 && threadIdx.x < kTileTableBytes / 4) table_out[threadIdx.x] = table.v[threadIdx.x];
-  const uint32_t per = kTileRows * (1u + tail_w), stride = tile_stride(nb, tail_w);
+                                                         uint32_t rows, uint32_t nb, uint32_t tail_w, uint32_t slots) {
+  if (table_out && blockIdx.x == 0 && threadIdx.x < kScaleSlots) table_out[threadIdx.x] = table.v[threadIdx.x];
+  const uint32_t per = kTileRows * (1u + 4u * tail_depth(tail_w)), stride = tile_stride(nb, tail_w, slots);
   const uint32_t total = tile_count(rows) * per;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-    const uint32_t tile = i / per, k = i - tile * per, r = k & 7u, j = k >> 3;  // j = 0: the scale, j > 0: tail column j - 1
+    const uint32_t tile = i / per, k = i - tile * per, r = k & 15u, j = k >> 4;  // j = 0: the scale, j > 0: tail column j - 1
     const uint32_t row = tile * kTileRows + r;
     float v = 0.f;
-    if (row < rows) v = j ? tail[(size_t)row * tail_w + j - 1u] : rscale[row];
-    reinterpret_cast<float*>(tiles + (size_t)tile * stride)[k] = v;
+    if (row < rows) v = !j ? rscale[row] : j <= tail_w ? tail[(size_t)row * tail_w + j - 1u] : 0.f;
+    reinterpret_cast<float*>(tiles + (size_t)tile * stride)[j ? tail_at(r, j - 1u, tail_w) : r] = v;
+    if (k == 0) *reinterpret_cast<uint32_t*>(tiles + (size_t)tile * stride + kCountAt) = 0u;
   }
 }
 
@@ -115,8 +187,15 @@ __device__ __forceinline__ T* uniform_global(T* p) {
 // largest, a sixteenth of the half ulp such a result carries anyway), six for f32 results (2^22: every binary16 value
 // within 2^12 of its block's largest is exact).  An 8-wide 4-bit dot product then takes one digit of eight columns
 // against a dword of weights, exactly.
-// In LDS a block is 3 dwords per digit, the sum of its integers (v = 2 n + p: sum v x = 2 sum n x + p sum x) and the scale.
-template <int DIG> struct XPlanes { static constexpr uint32_t kDwords = 3 * DIG + 2; };
+// In LDS the four blocks of a unit lie together: 3 dwords per digit and block, then each block's sum of its integers
+// (v = 2 n + b: sum v x = 2 sum n x + b sum x) and scale.  The pad spreads the eight units of a step over the banks.
+template <int DIG> struct XPlanes {
+  static constexpr uint32_t kBlock = 3 * DIG, kSums = 4 * kBlock, kDwords = kSums + 8 + (DIG == 6 ? 4 : 0);
+};
+template <int DIG>
+__device__ __forceinline__ uint32_t plane_at(uint32_t blk) { return (blk >> 2) * XPlanes<DIG>::kDwords + (blk & 3u) * XPlanes<DIG>::kBlock; }
+template <int DIG>
+__device__ __forceinline__ uint32_t plane_sum_at(uint32_t blk) { return (blk >> 2) * XPlanes<DIG>::kDwords + XPlanes<DIG>::kSums + (blk & 3u) * 2u; }
 
 // An inclusive maximum of the lanes' |f32| bit patterns over a quad (integers: a NaN is larger than anything).
 __device__ __forceinline__ uint32_t quad_max(uint32_t v) {
@@ -129,9 +208,9 @@ __device__ __forceinline__ int quad_sum(int v) {
 }
 
 // Eight values of a block (columns 8 sub .. 8 sub + 7 of it), sub = lane % 4; the quad's fourth lane passes zeros and
-// only takes part in the exchange.  Writes the block's planes at xb.  About 90 instructions for the quad's 24 values.
+// only takes part in the exchange.  Writes the block's planes at xb, its sum and scale at xs.  About 90 instructions for the quad's 24 values.
 template <int DIG>
-__device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub, uint32_t* xb) {
+__device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub, uint32_t* xb, uint32_t* xs) {
   constexpr int kBits = DIG == 4 ? 14 : 22;
   constexpr uint32_t kMagic = 0x4B400000u;  // 1.5 2^23: adding it leaves the rounded integer in the low mantissa bits
   uint32_t m = 0;
@@ -187,32 +266,29 @@ __device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub
       xb[(2 * k + 1) * 3 + sub] = bfi32(0x0F0F0F0Fu, lo[k] >> 4, hi[k]);
     }
   } else {
-    xb[3 * DIG] = (uint32_t)sum;
-    xb[3 * DIG + 1] = __float_as_uint(scale);
+    xs[0] = (uint32_t)sum;
+    xs[1] = __float_as_uint(scale);
   }
 }
 
 // ---- batch-1 product ------------------------------------------------------------------------------
-constexpr uint32_t kGemvSteps = 4;      // steps of 8 blocks a wavefront takes of a record, ...
-constexpr uint32_t kGemvWideSteps = 8;  // ... and of a record wider than 16 wavefronts' worth of those
 constexpr uint32_t kGemvMaxWaves = 16;
-constexpr uint32_t kGemvRounds = 8;     // records per team between two sums over the team's wavefronts
+constexpr uint32_t kGemvWideSteps = 2;  // steps of a wavefront where a row has more than sixteen
+constexpr uint32_t kGemvRounds = 8;     // tiles per team between two sums over the team's wavefronts, at the most
 
-// How a record's blocks are split over wavefronts: 2^shift of them, wavefront w taking the steps w, w + 2^shift, ...
-// It depends on the row length alone, so a matrix gives the same bits whatever it shares a launch with.  The fewest
-// wavefronts, at least four, that leave each at most kGemvSteps steps (16 past 512 blocks, with kGemvWideSteps).
-// Every wavefront runs all its steps, on zeros where the row has ended: a branch around a load would make every wait
-// behind it a wait for all loads in flight.
-__host__ __device__ inline uint32_t gemv_split_shift(uint32_t nb) {
-  const uint32_t steps = (nb + 7u) >> 3;
-  uint32_t s = 2;
-  while (s < 4u && (kGemvSteps << s) < steps) ++s;
-  return s;
+// A tile's steps go to a team of wavefronts, one each (two each past sixteen).  A row is added up in an order that does not
+// depend on that: the lanes of a step (rows_sum), the steps of equal number mod 4 one behind the other, those four sums;
+// so a matrix gives the same bits whatever it shares a launch with.
+__host__ __device__ inline uint32_t gemv_team(uint32_t nb) {
+  const uint32_t steps = tile_steps(nb);
+  return steps > kGemvMaxWaves ? kGemvMaxWaves : steps ? steps : 1u;
 }
-__host__ __device__ inline bool gemv_wide(uint32_t nb) { return nb > 8u * kGemvSteps * kGemvMaxWaves; }
-constexpr uint32_t kGemvMaxBlocks = 8u * kGemvWideSteps * kGemvMaxWaves;
-// Blocks of the planes in LDS: whole steps, and a step of zeros behind them for the wavefronts whose steps end early.
-__host__ __device__ inline uint32_t gemv_plane_blocks(uint32_t nb) { return (((nb + 7u) >> 3) + 1u) * 8u; }
+__host__ __device__ inline bool gemv_wide(uint32_t nb) { return nb > kStepBlocks * kGemvMaxWaves; }
+// ... and so that there is a wavefront for each of the workgroup's
+__host__ __device__ inline uint32_t gemv_batch(uint32_t team) { return team < kGemvRounds ? team : kGemvRounds; }
+constexpr uint32_t kGemvMaxBlocks = kStepBlocks * kGemvMaxWaves * kGemvWideSteps;
+// Units of the planes in LDS: whole steps, and a step of zeros behind them for the wavefronts whose steps end early.
+__host__ __device__ inline uint32_t gemv_plane_units(uint32_t nb) { return (tile_steps(nb) + 1u) * kStepUnits; }
 
 // What a launch's activation is made from.
 enum : int { kSrcF16 = 0, kSrcRotated = 1, kSrcSiluMul = 2, kSrcAddRmsNorm = 3 };
@@ -221,39 +297,38 @@ struct TileMat {
   const uint8_t* base;  // the matrix (table, then records)
   void* y;
   uint32_t d_out;
-  uint32_t tile_begin;  // first record of this matrix in the launch
+  uint32_t tile_begin;  // first tile of this matrix in the launch
+  uint32_t stride, slots;
 };
 struct GemvArgs {
   ActivationIn in;
   uint32_t nb, tail_w, n_mats, n_tiles;
-  uint32_t split_shift;
+  uint32_t team, teams;  // wavefronts of a team, teams of a workgroup (more wavefronts only stage the activation)
   TileMat m[kMaxGroup];
 };
 
 struct GemvLds {
   float* xtail;      // [32]
   float* red;        // [16]
-  uint32_t* planes;  // [plane blocks][XPlanes::kDwords]
-  float* part;       // [kGemvRounds][16][8]
-  float* tpart;      // the same for the tail columns
-  float* scales;     // and the rows' scales
+  uint32_t* planes;  // [plane units][XPlanes::kDwords]
+  float* part;       // [kGemvRounds][16 or 32 steps][16 rows]
   float* xf;         // [d_in] f32 values of a rotated activation
 };
 __host__ __device__ inline uint32_t gemv_lds_fixed() { return 128u + 64u; }
 __host__ __device__ inline size_t gemv_tiles_lds_bytes(uint32_t nb, uint32_t d_in, bool f32_out, bool rotated) {
-  const size_t planes = (size_t)gemv_plane_blocks(nb) * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
-  return gemv_lds_fixed() + planes + 3 * kGemvRounds * kGemvMaxWaves * 8 * 4 + (rotated ? ((size_t)d_in * 4 + 31) / 16 * 16 : 0);
+  const size_t planes = (size_t)gemv_plane_units(nb) * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
+  const size_t sums = kGemvRounds * kGemvMaxWaves * kTileRows * 4;
+  return gemv_lds_fixed() + planes + (gemv_wide(nb) ? kGemvWideSteps : 1u) * sums + (rotated ? ((size_t)d_in * 4 + 31) / 16 * 16 : 0);
 }
-template <int DIG>
-__device__ __forceinline__ GemvLds gemv_lds(uint8_t* smem, uint32_t plane_blocks) {
+template <int DIG, bool WIDE>
+__device__ __forceinline__ GemvLds gemv_lds(uint8_t* smem, uint32_t plane_units) {
+  constexpr uint32_t kSums = kGemvRounds * kGemvMaxWaves * kTileRows;
   GemvLds L;
   L.xtail = reinterpret_cast<float*>(smem);
   L.red = L.xtail + 32;
   L.planes = reinterpret_cast<uint32_t*>(L.red + 16);
-  L.part = reinterpret_cast<float*>(L.planes + (size_t)plane_blocks * XPlanes<DIG>::kDwords);
-  L.tpart = L.part + kGemvRounds * kGemvMaxWaves * 8;
-  L.scales = L.tpart + kGemvRounds * kGemvMaxWaves * 8;
-  L.xf = L.scales + kGemvRounds * kGemvMaxWaves * 8;
+  L.part = reinterpret_cast<float*>(L.planes + (size_t)plane_units * XPlanes<DIG>::kDwords);
+  L.xf = L.part + kSums * (WIDE ? kGemvWideSteps : 1u);
   return L;
 }
 
@@ -280,22 +355,26 @@ __device__ __forceinline__ void load_halves(const __half* p, uint32_t (&w)[4]) {
 }
 
 // Fills the planes and the tail values in LDS from `in`, by every lane of the workgroup.
-// `request` is called once, right behind the loads of the activation's operands: the first weights go out there.
+// `request` is called once, right behind the loads of the activation's operands: the first weights go out there.  (With a
+// barrier in front, so that no wavefront's operands come behind the others' weights, a decode step took 3 % longer.)
 // PMAX: how often the workgroup's quads pass over the padded blocks, at most.  store_resid: this workgroup is the one
 // that stores the new residual.  Ends without a barrier.
 template <int DIG, int SRC, int PMAX, bool kDeviceScope = false, class Request>
 __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uint32_t tail_w, const GemvLds& L, bool store_resid, Request&& request) {
-  constexpr uint32_t kStr = XPlanes<DIG>::kDwords;
   const uint32_t tid = threadIdx.x, n_thr = blockDim.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t sub = tid & 3u, quad = tid >> 2, quads = n_thr >> 2;
-  const uint32_t pad = (nb + 7u) & ~7u, d_in = nb * kDim + tail_w;
+  const uint32_t pad = tile_steps(nb) * kStepBlocks, d_in = nb * kDim + tail_w;
   const uint32_t passes = (pad + quads - 1u) / quads;
-  if (tid < 32u) L.xtail[tid] = 0.f;
-  for (uint32_t i = tid; i < 8u * kStr; i += n_thr) L.planes[pad * kStr + i] = 0u;  // the step of zeros
+  auto quantize = [&](const float (&v)[8], uint32_t blk) { quantize_octet<DIG>(v, sub, L.planes + plane_at<DIG>(blk), L.planes + plane_sum_at<DIG>(blk)); };
+  auto zeros = [&]() {  // past the tail, and the step of zeros
+    if (tid < 32u) L.xtail[tid] = 0.f;
+    for (uint32_t i = tid; i < kStepUnits * XPlanes<DIG>::kDwords; i += n_thr) L.planes[plane_at<DIG>(pad) + i] = 0u;
+  };
   if constexpr (SRC == kSrcRotated) {
     // The activation is rotated into LDS and quantised from there (a finished f32 one from where it is).
     // A launch in a rotated basis has 1024 lanes.
     float* xf = L.xf;
+    zeros();
     if (in.x_f32) {
       request();
     } else {
@@ -412,7 +491,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
           for (int j = 0; j < 8; ++j) v[j] = xf[at + j];
         }
       }
-      quantize_octet<DIG>(v, sub, L.planes + (size_t)blk * kStr);
+      quantize(v, blk);
     }
     if (tid < tail_w) L.xtail[tid] = in.x_f32 ? in.x_f32[nb * kDim + tid] : xf[nb * kDim + tid];
   } else {
@@ -457,11 +536,12 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
         v[2 * j] = ok ? lo : 0.f;
         v[2 * j + 1] = ok ? hi : 0.f;
       }
-      quantize_octet<DIG>(v, sub, L.planes + (size_t)blk * kStr);
+      quantize(v, blk);
     };
     load_operands(0);
     request();
     __builtin_amdgcn_sched_barrier(0);
+    zeros();
     float inv = 0.f;
     if constexpr (SRC == kSrcAddRmsNorm) {
       float ss = 0.f;
@@ -496,7 +576,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
               }
             }
             if constexpr (PMAX > kChunk) {
-              uint32_t* keep = L.planes + (size_t)blk * kStr + sub * 4u;
+              uint32_t* keep = L.planes + plane_at<DIG>(blk) + sub * 4u;
 #pragma unroll
               for (int j = 0; j < 4; ++j) keep[j] = a[k][j];
             }
@@ -529,7 +609,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
         const uint32_t blk = block_of(p);
         if (blk >= pad) break;
         const bool ok = blk < nb && sub < 3u;
-        const uint32_t* kept = L.planes + (size_t)blk * kStr + sub * 4u;
+        const uint32_t* kept = L.planes + plane_at<DIG>(blk) + sub * 4u;
 #pragma unroll
         for (int j = 0; j < 4; ++j) a[0][j] = ok ? kept[j] : 0u;
         load_halves<false>(in.norm_w + (ok ? blk * kDim + sub * 8u : 0u), g[0]);
@@ -558,102 +638,254 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
   }
 }
 
-// A lane's share of a step: the nibbles and the byte of one (row, block).
+// A lane's share of a step: five pieces of a unit, two rows by four blocks.
 struct StepWords {
-  uint32_t w0, w1, w2, meta;  // meta: the dword with the bytes of the lane's row and its three neighbours
+  u32x4_t p[5];
 };
-// step_at: the step's first block; lane_off: block lane / 8 and row lane % 8 behind it (12-byte words), meta_off the dword
-// with the row's byte.  live = false (uniform) sends every lane to one place instead, a load nobody uses: one cache line,
-// and no branch, which would turn every wait behind it into a wait for all loads.
-// A record's last step may reach up to seven blocks past it, into the next record or the allocation's slack: such lanes
-// meet zeros in the planes.
-struct LaneOffsets {
-  uint32_t words, meta;
-};
-__device__ __forceinline__ LaneOffsets lane_offsets(uint32_t lane) {
-  const uint32_t r = lane & 7u, bq = lane >> 3;
-  return LaneOffsets{bq * kTileBlockBytes + r * 12u, bq * kTileBlockBytes + 96u + (r & 4u)};
+// What a lane adds to a tile's address for its unit of a step (units past the last repeat it: they meet zeros in the planes).
+__device__ __forceinline__ uint32_t step_offset(uint32_t step, uint32_t units, uint32_t head, uint32_t lane) {
+  const uint32_t u = min(step * kStepUnits + (lane >> 3), max(units, 1u) - 1u);
+  return head + u * kUnitBytes + (lane & 7u) * 16u;
 }
-constexpr uint32_t kStepBytes = 8u * kTileBlockBytes;
-__device__ __forceinline__ StepWords load_step(const uint8_t* blocks, uint32_t step, bool live, const LaneOffsets& at) {
-  struct __attribute__((packed, aligned(4))) W3 { uint32_t w[3]; };
+// A scalar base the compiler cannot take apart again: loads through it add a 32-bit lane offset.
+__device__ __forceinline__ const uint8_t* scalar_base(const uint8_t* p) {
   typedef const uint8_t __attribute__((address_space(1))) global_u8;
-  const uint32_t keep = live ? 0xFFFFFFFFu : 0u;
-  uint64_t bits = reinterpret_cast<uint64_t>(blocks + ((step * kStepBytes) & keep));
-  asm("" : "+s"(bits));  // a scalar base the compiler cannot take apart again: the loads add a 32-bit lane offset to it
-  const uint8_t* base = (const uint8_t*)reinterpret_cast<global_u8*>(bits);
-  const W3 w = *reinterpret_cast<const W3*>(base + (at.words & keep));
-  // (the byte comes with its dword: a loop-carried byte would be copied, and so waited for, as soon as it is requested)
-  return StepWords{w.w[0], w.w[1], w.w[2], *reinterpret_cast<const uint32_t*>(base + (at.meta & keep))};
+  uint64_t bits = reinterpret_cast<uint64_t>(uniform_global(p));
+  asm("" : "+s"(bits));
+  return (const uint8_t*)reinterpret_cast<global_u8*>(bits);
+}
+template <int P>
+__device__ __forceinline__ void load_piece(StepWords& W, const uint8_t* base, uint32_t off) {
+  W.p[P] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(base + off + P * 128u));
+}
+__device__ __forceinline__ void load_step(StepWords& W, const uint8_t* base, uint32_t off) {
+  load_piece<0>(W, base, off);
+  load_piece<1>(W, base, off);
+  load_piece<2>(W, base, off);
+  load_piece<3>(W, base, off);
+  load_piece<4>(W, base, off);
 }
 
+// The block scales, two lanes to each: a block's meta byte is the address of its own in them (a lane's register is at four
+// times its number, and the two lowest bits don't count).
+__device__ __forceinline__ uint32_t scale_table(const uint8_t* base, uint32_t lane) {
+  return reinterpret_cast<const uint32_t*>(base)[lane >> 1];
+}
+__device__ __forceinline__ float scale_at(uint32_t meta, uint32_t table) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute((int)meta, (int)table));
+}
+
+// first + the sum of a block's digit products, exact, from the top digit down.  (One chain: each step of it waits a little
+// for the one before, which the other wavefronts of a SIMD fill; two side by side take two more instructions.)
 template <int DIG>
-struct XBlock {
-  int d[3 * DIG];
-  int sum;
-  float scale;
+__device__ __forceinline__ int digits_sum(const uint32_t (&w)[3], const int (&x)[3 * DIG], int first) {
+  int t = 0;
+#pragma unroll
+  for (int k = DIG - 1; k >= 0; --k) {
+    if (k != DIG - 1) t = (t << 4) + (k ? 0 : first);
+#pragma unroll
+    for (int o = 0; o < 3; ++o) t = __builtin_amdgcn_sdot8((int)w[o], x[3 * k + o], t, false);
+  }
+  return t;
+}
+// a * b + c, a and b of 24 bits
+__device__ __forceinline__ int mad24_lanes(int a, int b, int c) {
+  int r;  // (the compiler would extend the factors first)
+  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// One block's part in a product: acc + sum of (n + win - 3) x, exact but for the f32 conversion, scaled by the block's weight
+// scale and the activation's.  12 or 18 dot products and about 18 more instructions.
+struct BlockTerm {
+  uint32_t w[3], win;
+  float c;
 };
+// K: the block in its unit; s, m: its row's {s, meta} dwords.  (An escape's scale is zero here: tile_extras sees to it.)
+template <int DIG, int K>
+__device__ __forceinline__ BlockTerm block_term(uint32_t d0, uint32_t d1, uint32_t s, uint32_t m, uint32_t table) {
+  BlockTerm b;
+  block_octets(d0, d1, s << (3 - K), b.w);
+  const uint32_t meta = m >> (8 * K);
+  b.win = meta & 7u;
+  b.c = scale_at(meta, table);
+  return b;
+}
+// sum, less: the sum of the block's integers x, and -3 times that (four digits' sums have 20 bits).
 template <int DIG>
-__device__ __forceinline__ XBlock<DIG> load_xblock(const uint32_t* xb) {
-  XBlock<DIG> x;
-  const uint2* p = reinterpret_cast<const uint2*>(xb);
-#pragma unroll
-  for (int i = 0; i < 3 * DIG / 2; ++i) {
-    const uint2 v = p[i];
-    x.d[2 * i] = (int)v.x;
-    x.d[2 * i + 1] = (int)v.y;
-  }
-  const uint2 v = p[3 * DIG / 2];
-  x.sum = (int)v.x;
-  x.scale = __uint_as_float(v.y);
-  return x;
+__device__ __forceinline__ float block_sum(const BlockTerm& b, const int (&x)[3 * DIG], int sum, int less, float scale, float acc) {
+  const int t = digits_sum<DIG>(b.w, x, DIG == 4 ? mad24_lanes((int)b.win, sum, less) : (int)b.win * sum + less);
+  return fmaf((float)t, b.c * scale, acc);
 }
 
-// acc + (one block's product): exact integer digit products, one f32 conversion, scaled by the block's weight scale and
-// the activation's.  12 or 18 dot products and about 10 more instructions.
-// table: the matrix's 32 scales, one per lane (the byte & 0x7C is the lane's place in bytes).
+// A block's digit planes.
 template <int DIG>
-__device__ __forceinline__ float step_product(const StepWords& w, const XBlock<DIG>& x, uint32_t table, uint32_t r, float acc) {
-  const uint32_t meta = w.meta >> (8u * (r & 3u));
-  int d[DIG];
+__device__ __forceinline__ void load_planes(const uint32_t* xb, int (&x)[3 * DIG]) {
+  if constexpr (DIG == 4) {
 #pragma unroll
-  for (int k = 0; k < DIG; ++k) {
-    d[k] = __builtin_amdgcn_sdot8((int)w.w0, x.d[3 * k], 0, false);
-    d[k] = __builtin_amdgcn_sdot8((int)w.w1, x.d[3 * k + 1], d[k], false);
-    d[k] = __builtin_amdgcn_sdot8((int)w.w2, x.d[3 * k + 2], d[k], false);
+    for (int i = 0; i < 3; ++i) {
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(xb + 4 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[4 * i + j] = (int)v[j];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 3 * DIG / 2; ++i) {
+      const u32x2_t v = *reinterpret_cast<const u32x2_t*>(xb + 2 * i);
+      x[2 * i] = (int)v.x;
+      x[2 * i + 1] = (int)v.y;
+    }
   }
-  int s = d[DIG - 1];
-#pragma unroll
-  for (int k = DIG - 2; k >= 0; --k) s = (s << 4) + d[k];
-  s = (s << 1) + (x.sum & -(int)(meta & 1u));
-  const float scale = __int_as_float(__builtin_amdgcn_ds_bpermute((int)(meta & 0x7Cu), (int)table));
-  return fmaf((float)s, scale * x.scale, acc);
 }
 
-// Sum over the lanes that hold the same row (lane % 8): lanes 8, 16 and 32 apart.
-__device__ __forceinline__ float row8_sum(float v) {
+// A step's products, rows l and l + 8 of the tile: what the lane's four blocks add up to.  xq: the unit's planes.
+// `reload(p)` is called for every piece as soon as its registers are free: what is to be loaded next goes out there.
+template <int DIG, class Reload>
+__device__ __forceinline__ void step_product(const StepWords& W, const uint32_t* xq, uint32_t table, float& lo, float& hi, Reload&& reload) {
+  lo = hi = 0.f;
+  auto block = [&](auto block_k) __attribute__((always_inline)) {
+    constexpr int K = decltype(block_k)::value;
+    int x[3 * DIG];
+    load_planes<DIG>(xq + K * XPlanes<DIG>::kBlock, x);
+    const u32x2_t ss = *reinterpret_cast<const u32x2_t*>(xq + XPlanes<DIG>::kSums + 2 * K);
+    const int sum = (int)ss.x, less = DIG == 4 ? __mul24(sum, -3) : sum * -3;
+    const float scale = __uint_as_float(ss.y);
+    const BlockTerm a = block_term<DIG, K>(W.p[K >> 1][2 * (K & 1)], W.p[K >> 1][2 * (K & 1) + 1], W.p[4].x, W.p[4].y, table);
+    const BlockTerm b = block_term<DIG, K>(W.p[2 + (K >> 1)][2 * (K & 1)], W.p[2 + (K >> 1)][2 * (K & 1) + 1], W.p[4].z, W.p[4].w, table);
+    lo = block_sum<DIG>(a, x, sum, less, scale, lo);
+    hi = block_sum<DIG>(b, x, sum, less, scale, hi);
+    __builtin_amdgcn_sched_barrier(0);  // the registers are free again only now: the loads need no others, and the products of several blocks at once would not fit
+  };
+  block(std::integral_constant<int, 0>{});
+  block(std::integral_constant<int, 1>{});
+  reload(std::integral_constant<int, 0>{});
+  reload(std::integral_constant<int, 2>{});
+  __builtin_amdgcn_sched_barrier(0);
+  block(std::integral_constant<int, 2>{});
+  block(std::integral_constant<int, 3>{});
+  reload(std::integral_constant<int, 1>{});
+  reload(std::integral_constant<int, 3>{});
+  reload(std::integral_constant<int, 4>{});
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The sum over the four classes of a row (row_lane), in every lane of it.
+__device__ __forceinline__ float classes_sum(float v) {
   v += dpp_move<0x128>(v);  // row_ror:8
   const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
-  const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+// The sums over a step's units of rows l (lo) and l + 8 (hi): row lane_row(lane)'s in every lane.
+__device__ __forceinline__ float rows_sum(float lo, float hi) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+  return classes_sum(__uint_as_float(p[0]) + __uint_as_float(p[1]));
 }
 
-// A record's result from what its team's wavefronts left: row lane % 8 in every lane.  part, tpart: 8 floats to a wavefront.
-__device__ __forceinline__ float team_sum(const float* part, const float* tpart, float scale, uint32_t split, uint32_t tail_waves, uint32_t lane) {
-  const uint32_t k = lane >> 3;
-  float v = k < split ? part[lane] : 0.f;
-  if (split > 8u) v += part[64u + lane];
-  v = row8_sum(v);
+// What a tile adds to its rows besides its steps, as one wavefront loads it: the row scales, the tail columns (a lane's
+// share, the neighbours' behind it), the escapes.
+struct TileExtras {
+  float scale;
+  u32x4_t tail;
+  u32x2_t tail2;
+  uint32_t count;
+  u32x4_t escape;
+};
+// (not live: not to be used, and one cache line)
+__device__ __forceinline__ TileExtras load_extras(const uint8_t* rec, uint32_t nb, uint32_t tail_w, uint32_t slots, bool live, uint32_t lane) {
+  struct __attribute__((packed, aligned(4))) W4 { u32x4_t w; };
+  struct __attribute__((packed, aligned(4))) W2 { u32x2_t w; };
+  const uint32_t depth = tail_depth(tail_w), at = live & (depth != 0u) ? 128u + lane * depth * 4u : 0u;
+  TileExtras x;
+  x.scale = reinterpret_cast<const float*>(rec)[live ? lane_row(lane) : 0u];
+  x.count = *reinterpret_cast<const uint32_t*>(rec + kCountAt);
+  x.tail = reinterpret_cast<const W4*>(rec + at)->w;
+  x.tail2 = reinterpret_cast<const W2*>(rec + at + (live & (depth > 4u) ? 16u : 0u))->w;
+  x.escape = *reinterpret_cast<const u32x4_t*>(rec + (live & (slots != 0u) ? list_at(nb, tail_w) + min(lane, slots - 1u) * 16u : 0u));
+  return x;
+}
+// The rows' tail columns and escapes, the latter by the row scales: row lane_row(lane)'s in every lane.  A lane takes an
+// escape of the list, and a row adds up its own in their order.
+template <int DIG>
+__device__ __forceinline__ float tile_extras(const TileExtras& X, const uint8_t* rec, uint32_t nb, uint32_t tail_w, uint32_t slots, uint32_t table,
+                                             const GemvLds& L, uint32_t lane) {
+  const uint32_t depth = tail_depth(tail_w);
   float t = 0.f;
-  if (tail_waves) t = row8_sum(k < tail_waves ? tpart[lane] : 0.f);
-  return fmaf(v, scale, t);
+#pragma unroll
+  for (uint32_t i = 0; i < 6; ++i)
+    if (i < depth) t = fmaf(__uint_as_float(i < 4u ? X.tail[i & 3u] : X.tail2[i & 1u]), L.xtail[4u * i + lane_class(lane)], t);
+  t = classes_sum(t);
+  const uint32_t count = (uint32_t)__builtin_amdgcn_readfirstlane((int)X.count);
+  if (count == 0u) return t;
+  float sum = 0.f;
+  auto add = [&](const uint32_t (&w)[3], uint32_t key, uint32_t n) {  // the escapes of lanes 0 .. n - 1
+    const uint32_t blk = (key >> 9) & 0x7FFFFu;
+    int x[3 * DIG];
+    load_planes<DIG>(L.planes + plane_at<DIG>(blk), x);
+    const u32x2_t ss = *reinterpret_cast<const u32x2_t*>(L.planes + plane_sum_at<DIG>(blk));
+    const int v = (digits_sum<DIG>(w, x, 0) << 1) + ((key >> 8) & 1u ? (int)ss.x : 0);
+    const float f = (float)v * (scale_at((key & 31u) << 3, table) * __uint_as_float(ss.y));
+    for (uint32_t e = 0; e < n; ++e) {
+      const uint32_t row = (uint32_t)__builtin_amdgcn_readlane((int)key, (int)e) >> 28;
+      const float p = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), (int)e));
+      sum += lane_row(lane) == row ? p : 0.f;
+    }
+  };
+  if (count <= slots) {
+    const bool mine = lane < count;  // (the others: any block that is there)
+    add({X.escape.x, X.escape.y, X.escape.z}, mine ? X.escape.w : 0u, count);
+  } else {  // more than there was room for: the tile's blocks one row after the other, 64 at a time
+#pragma unroll 1
+    for (uint32_t r = 0; r < kTileRows; ++r)
+#pragma unroll 1
+      for (uint32_t b0 = 0; b0 < nb; b0 += 64u) {
+        const uint32_t blk = min(b0 + lane, nb - 1u), k = blk & 3u;
+        const uint8_t* unit = rec + tile_head_bytes(tail_w) + (blk >> 2) * kUnitBytes + (r & 7u) * 16u;
+        const u32x2_t d = *reinterpret_cast<const u32x2_t*>(unit + ((r >> 3) * 2u + (k >> 1)) * 128u + (k & 1u) * 8u);
+        const u32x2_t sm = *reinterpret_cast<const u32x2_t*>(unit + 512u + (r >> 3) * 8u);
+        const uint32_t meta = (sm.y >> (8u * k)) & 255u;
+        uint32_t w[3];
+        block_octets(d.x, d.y, sm.x << (3u - k), w);
+        const BlockEscape e = block_escape(w, meta);
+        w[0] = e.w0;
+        int x[3 * DIG];
+        load_planes<DIG>(L.planes + plane_at<DIG>(blk), x);
+        const u32x2_t ss = *reinterpret_cast<const u32x2_t*>(L.planes + plane_sum_at<DIG>(blk));
+        const uint32_t bit = 1u << (4u * (e.at & 7u));  // the coordinate that is 16 below, by itself
+        const uint32_t one[3] = {e.at < 8u ? bit : 0u, (e.at >> 3) == 1u ? bit : 0u, (e.at >> 3) == 2u ? bit : 0u};
+        const int v = digits_sum<DIG>(w, x, ((int)e.win - 3) * (int)ss.x) - (digits_sum<DIG>(one, x, 0) << 4);
+        const float f = (float)(e.negative ? -v : v) * (scale_at(e.slot << 3, table) * __uint_as_float(ss.y));
+        const bool mine = meta >= kBlockEscape && b0 + lane < nb;
+        for (uint64_t left = __builtin_amdgcn_ballot_w64(mine); left; left &= left - 1u) {
+          const float p = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), __builtin_ctzll(left)));
+          sum += lane_row(lane) == r ? p : 0.f;
+        }
+      }
+  }
+  return fmaf(sum, X.scale, t);
 }
 
-__device__ __forceinline__ void tile_mat(const GemvArgs& a, uint32_t tile, const uint8_t*& base, void*& y, uint32_t& row0, uint32_t& d_out) {
+// A row's blocks from what its steps left in LDS (sixteen rows a step).
+template <uint32_t MAX>
+__device__ __forceinline__ float steps_sum(const float* part, uint32_t steps, uint32_t lane) {
+  float v[MAX / 4], t = 0.f;
+#pragma unroll
+  for (uint32_t i = 0; i < MAX / 4; ++i) {
+    const uint32_t s = 4u * i + lane_class(lane);
+    v[i] = part[min(s, MAX - 1u) * kTileRows + lane_row(lane)];
+    v[i] = s < steps ? v[i] : 0.f;
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < MAX / 4; ++i) t += v[i];
+  return classes_sum(t);
+}
+
+__device__ __forceinline__ void tile_mat(const GemvArgs& a, uint32_t tile, const uint8_t*& base, void*& y, uint32_t& row0, uint32_t& d_out,
+                                         uint32_t& stride, uint32_t& slots) {
   base = a.m[0].base;  // constant indices only: a dynamic one would move the arguments to scratch
   y = a.m[0].y;
   d_out = a.m[0].d_out;
+  stride = a.m[0].stride;
+  slots = a.m[0].slots;
   uint32_t begin = 0;
 #pragma unroll
   for (uint32_t k = 1; k < kMaxGroup; ++k)
@@ -661,142 +893,114 @@ __device__ __forceinline__ void tile_mat(const GemvArgs& a, uint32_t tile, const
       base = a.m[k].base;
       y = a.m[k].y;
       d_out = a.m[k].d_out;
+      stride = a.m[k].stride;
+      slots = a.m[k].slots;
       begin = a.m[k].tile_begin;
     }
   row0 = (tile - begin) * kTileRows;
 }
 
-// What a wavefront loads for a record: its steps, its row's scale and a tail column of it, the matrix's block scales (one
-// per lane).
-template <uint32_t STEPS>
-struct RecordWords {
-  StepWords step[STEPS];
-  float scale, tail;
-  uint32_t table;
-};
-// live: whether the wavefront has a record at all; its j-th step is w + j split of n_steps.
-template <uint32_t STEPS>
-__device__ __forceinline__ void load_record(RecordWords<STEPS>& W, const uint8_t* rec, const uint8_t* base, uint32_t head, uint32_t w, uint32_t split,
-                                            uint32_t n_steps, bool live, uint32_t tail_off, uint32_t lane, const LaneOffsets& at) {
-  W.scale = reinterpret_cast<const float*>(rec)[lane & 7u];
-  W.table = reinterpret_cast<const uint32_t*>(base)[lane & 31u];
-  W.tail = *reinterpret_cast<const float*>(rec + (live ? tail_off : 0u));
-#pragma unroll
-  for (uint32_t j = 0; j < STEPS; ++j) W.step[j] = load_step(rec + head, w + j * split, live & (w + j * split < n_steps), at);
-}
-
 // y = W x for the rows of up to four matrices that share an activation.
 //
-// What bounds it: at 13 bytes per block and about 25 vector instructions the weights' way from memory; in a launch of
-// a few microseconds the chain launch -> activation -> planes -> product -> store.  So: a team of 2^split_shift
-// wavefronts takes a record of eight rows, a wavefront a fixed set of its steps; the loads of a record are all in flight
-// before the planes are ready, and each step's registers are loaded again for the team's next record as soon as they have
-// been used, without a branch, so that every wait is for the oldest load only.  For binary16 results a wavefront reads
-// its planes from LDS once and keeps them in registers.  The sums over a team's wavefronts wait in LDS for one barrier
-// per kGemvRounds records.  The host spreads teams over the CUs first (a workgroup has four to sixteen wavefronts),
-// records over teams so that the last, partial round meets every CU.
-// WIDE: rows past 512 blocks, with twice the steps.  Their planes, and the six digits of f32 results, do not fit the
-// registers beside the weights: a step then reads its planes from LDS.
+// What bounds it: at 10 bytes per block and about 35 vector instructions the weights' way from memory; in a launch of
+// a few microseconds the chain launch -> activation -> planes -> product -> store.  So: a team of wavefronts takes a tile of
+// sixteen rows, a wavefront a fixed step of it (two of rows past 512 blocks); a tile's loads are all in flight before the
+// planes are ready, and each piece's registers are loaded again for the team's next tile as soon as they have been used,
+// without a branch, so that every wait is for the oldest load only.  The planes of a unit are read from LDS once for
+// the two rows a lane has.  The sums over a team's wavefronts wait in LDS for one barrier per gemv_batch tiles, behind which
+// every wavefront finishes one.  The host spreads teams over the CUs first, tiles over teams so that the last, partial round
+// meets every CU.
 template <typename OutT, int SRC, bool WIDE>
 __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
   constexpr int DIG = std::is_same<OutT, __half>::value ? 4 : 6;
-  constexpr bool XREG = !WIDE && DIG == 4;
-  constexpr uint32_t kSteps = WIDE ? kGemvWideSteps : kGemvSteps;
-  constexpr uint32_t kStr = XPlanes<DIG>::kDwords;
+  constexpr uint32_t kSteps = WIDE ? kGemvWideSteps : 1u, kMaxSteps = kGemvMaxWaves * kSteps;
   extern __shared__ __align__(16) uint8_t smem[];
-  const GemvLds L = gemv_lds<DIG>(smem, gemv_plane_blocks(a.nb));
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, r = lane & 7u, bq = lane >> 3;
-  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-  const uint32_t split = 1u << a.split_shift, team = wave >> a.split_shift, w = wave & (split - 1u);
-  const uint32_t teams = (blockDim.x >> 6) >> a.split_shift, n_teams = teams * gridDim.x;
-  const uint32_t nb = a.nb, n_steps = (nb + 7u) >> 3;
-  const LaneOffsets at = lane_offsets(lane);
-  const uint32_t stride = tile_stride(nb, a.tail_w), head = tile_head_bytes(a.tail_w);
+  const GemvLds L = gemv_lds<DIG, WIDE>(smem, gemv_plane_units(a.nb));
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), waves = blockDim.x >> 6;
+  const uint32_t team = wave / a.team, w = wave - team * a.team, n_teams = a.teams * gridDim.x;
+  const uint32_t nb = a.nb, n_steps = tile_steps(nb), units = tile_units(nb), head = tile_head_bytes(a.tail_w);
 
-  struct Record { const uint8_t* rec; const uint8_t* base; };
+  struct Record { const uint8_t* rec; const uint8_t* base; uint32_t slots; };
   auto record_of = [&](uint32_t t) {
     const uint8_t* base;
     void* y;
-    uint32_t row0, d_out;
-    tile_mat(a, t, base, y, row0, d_out);
-    return Record{base + kTileTableBytes + (size_t)(row0 / kTileRows) * stride, base};
+    uint32_t row0, d_out, stride, slots;
+    tile_mat(a, t, base, y, row0, d_out, stride, slots);
+    return Record{base + kTileTableBytes + (size_t)(row0 / kTileRows) * stride, base, slots};
   };
-  const uint32_t tail_c = w * 8u + bq;  // the tail column this lane adds for its row
-  const uint32_t tail_off = tail_c < a.tail_w ? 32u + tail_c * 32u + r * 4u : 0u;
-  const uint32_t tail_waves = (a.tail_w + 7u) >> 3;
-
-  uint32_t tile = team * gridDim.x + blockIdx.x;
+  uint32_t off[kSteps];  // (where a wavefront has no step, or no next tile, its loads repeat one: one cache line, and no branch)
+#pragma unroll
+  for (uint32_t j = 0; j < kSteps; ++j) off[j] = step_offset(w + j * kGemvMaxWaves, units, head, lane);
+  uint32_t tile = team < a.teams ? team * gridDim.x + blockIdx.x : 0xFFFFFFFFu;
   Record cur = record_of(min(tile, a.n_tiles - 1u));
-  RecordWords<kSteps> W;
-  stage_x<DIG, SRC, WIDE ? 8 : 2>(a.in, nb, a.tail_w, L, blockIdx.x == 0,
-                                  [&]() { load_record(W, cur.rec, cur.base, head, w, split, n_steps, tile < a.n_tiles, tail_off, lane, at); });
+  StepWords W[kSteps];
+  constexpr uint32_t kFirst = SRC == kSrcRotated ? 1u : kSteps;  // (beside a rotation's operands there are registers for one)
+  uint32_t table;
+  // The tile that this wavefront finishes of those whose rounds begin with r0.
+  const uint32_t batch = gemv_batch(a.team), my_round = wave / a.teams, my_team = wave - my_round * a.teams;
+  TileExtras extras;
+  uint32_t extras_table;
+  auto finished = [&](uint32_t r0) { return my_round < batch ? (r0 + my_round) * n_teams + my_team * gridDim.x + blockIdx.x : 0xFFFFFFFFu; };
+  auto load_finish = [&](uint32_t r0) {
+    const uint32_t t = finished(r0);
+    const Record r = record_of(min(t, a.n_tiles - 1u));
+    extras = load_extras(r.rec, nb, a.tail_w, r.slots, t < a.n_tiles, lane);
+    extras_table = scale_table(r.base, lane);
+  };
+  stage_x<DIG, SRC, WIDE ? 4 : 2>(a.in, nb, a.tail_w, L, blockIdx.x == 0, [&]() {
+    if constexpr (SRC != kSrcRotated) load_finish(0);  // little, and it has a use while the pieces come
+    table = scale_table(cur.base, lane);
+    const uint8_t* base = scalar_base(cur.rec);
+    const uint32_t keep = tile < a.n_tiles ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+    for (uint32_t j = 0; j < kFirst; ++j) load_step(W[j], base, off[j] & keep);
+  });
+  if constexpr (kFirst != kSteps) load_step(W[1], scalar_base(cur.rec), off[1] & (tile < a.n_tiles ? 0xFFFFFFFFu : 0u));
+  if constexpr (SRC == kSrcRotated) load_finish(0);
   lds_barrier();
 
-  XBlock<DIG> X[XREG ? kSteps : 1];
-  if constexpr (XREG) {
-#pragma unroll
-    for (uint32_t j = 0; j < kSteps; ++j) X[j] = load_xblock<DIG>(L.planes + (min(w + j * split, n_steps) * 8u + bq) * kStr);
-  }
-  const float xt = tail_c < a.tail_w ? L.xtail[tail_c] : 0.f;
   const uint32_t rounds = (a.n_tiles + n_teams - 1u) / n_teams;
-  for (uint32_t rd = 0; rd < rounds; ++rd) {
-    const uint32_t next = tile + n_teams;
-    const bool more = next < a.n_tiles;
-    const Record nx = record_of(min(next, a.n_tiles - 1u));
-    const uint32_t table = W.table;
-    const float tail = W.tail, scale = W.scale;
-    W.scale = reinterpret_cast<const float*>(nx.rec)[r];
-    W.table = reinterpret_cast<const uint32_t*>(nx.base)[lane & 31u];  // first again, so that the next round waits for them alone
-    W.tail = *reinterpret_cast<const float*>(nx.rec + (more ? tail_off : 0u));
-    float acc = 0.f;
-    if constexpr (XREG) {
+  for (uint32_t r0 = 0; r0 < rounds; r0 += batch) {
+    const uint32_t r1 = min(r0 + batch, rounds), o_tile = finished(r0);
+    const float o_scale = extras.scale;
+    float o_extra = 0.f;
+    if (o_tile < a.n_tiles) {
+      const Record r = record_of(o_tile);
+      o_extra = tile_extras<DIG>(extras, r.rec, nb, a.tail_w, r.slots, extras_table, L, lane);
+    }
+    if (r1 != rounds) load_finish(r1);
+    for (uint32_t rd = r0; rd < r1 && tile < a.n_tiles; ++rd) {
+      const uint32_t next = tile + n_teams;
+      const bool more = next < a.n_tiles;
+      const Record nx = record_of(min(next, a.n_tiles - 1u));
+      const uint32_t lanes_table = table, keep = more ? 0xFFFFFFFFu : 0u;
+      const uint8_t* base = scalar_base(nx.rec);
+      float* const part = L.part + ((rd - r0) * kMaxSteps + team * a.team) * kTileRows;
+      table = scale_table(nx.base, lane);  // in front of the pieces, so that the next round waits for it alone
 #pragma unroll
       for (uint32_t j = 0; j < kSteps; ++j) {
-        acc = step_product<DIG>(W.step[j], X[j], table, r, acc);
-        __builtin_amdgcn_sched_barrier(0);  // the step's registers are free again only now: the loads need no others
-        W.step[j] = load_step(nx.rec + head, w + j * split, more & (w + j * split < n_steps), at);
-        __builtin_amdgcn_sched_barrier(0);  // step by step: the products of several at once would not fit the registers
+        const uint32_t step = w + j * kGemvMaxWaves;
+        float lo, hi;
+        step_product<DIG>(W[j], L.planes + (min(step, n_steps) * kStepUnits + (lane >> 3)) * XPlanes<DIG>::kDwords, lanes_table, lo, hi,
+                          [&](auto piece) __attribute__((always_inline)) { load_piece<decltype(piece)::value>(W[j], base, off[j] & keep); });
+        const float v = rows_sum(lo, hi);
+        if (lane_class(lane) == 0u) part[step * kTileRows + lane_row(lane)] = v;
       }
-    } else {
-#pragma unroll
-      for (uint32_t j = 0; j < kSteps; ++j) {
-        const uint32_t step = w + j * split;
-        acc = step_product<DIG>(W.step[j], load_xblock<DIG>(L.planes + (min(step, n_steps) * 8u + bq) * kStr), table, r, acc);
-        __builtin_amdgcn_sched_barrier(0);
-        W.step[j] = load_step(nx.rec + head, step, more & (step < n_steps), at);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      tile = next;
     }
-    acc = row8_sum(acc);
-    const uint32_t slot = ((rd % kGemvRounds) * kGemvMaxWaves + wave) * 8u + lane;
-    if (lane < 8u) {
-      L.part[slot] = acc;
-      L.scales[slot] = scale;
-    }
-    if (w < tail_waves) {
-      const float t = row8_sum(tail_c < a.tail_w ? tail * xt : 0.f);
-      if (lane < 8u) L.tpart[slot] = t;
-    }
-    cur = nx;
-    tile = next;
-    if ((rd + 1u) % kGemvRounds != 0u && rd + 1u != rounds) continue;
-    // A wavefront per record of the last rounds: everything but the sums themselves is scalar.  (A lane per row, adding up
-    // to sixteen values one behind the other, took 5300 of the 13700 cycles of a 2560 x 9728 product.)
+    // A wavefront per tile of these rounds: everything but the sums themselves is scalar.
     lds_barrier();
-    const uint32_t r0 = rd / kGemvRounds * kGemvRounds, slots = kGemvMaxWaves >> a.split_shift;  // slots: teams to a round
-    for (uint32_t q = wave; q < ((rd + 1u - r0) << (4u - a.split_shift)); q += teams << a.split_shift) {
-      const uint32_t o_round = q >> (4u - a.split_shift), o_team = q & (slots - 1u);
-      const uint32_t o_tile = (r0 + o_round) * n_teams + o_team * gridDim.x + blockIdx.x;
-      if (o_team >= teams || o_tile >= a.n_tiles) continue;
+    if (o_tile < a.n_tiles) {
       const uint8_t* o_base;
       void* o_y;
-      uint32_t o_row0, o_d_out;
-      tile_mat(a, o_tile, o_base, o_y, o_row0, o_d_out);
-      const uint32_t at0 = (o_round * kGemvMaxWaves + (o_team << a.split_shift)) * 8u;
-      const float v = team_sum(L.part + at0, L.tpart + at0, L.scales[at0 + r], split, tail_waves, lane);
-      if (lane < 8u && o_row0 + lane < o_d_out) store_out<OutT>(o_y, o_row0 + lane, v);
+      uint32_t o_row0, o_d_out, o_stride, o_slots;
+      tile_mat(a, o_tile, o_base, o_y, o_row0, o_d_out, o_stride, o_slots);
+      const float v = steps_sum<kMaxSteps>(L.part + (my_round * kMaxSteps + my_team * a.team) * kTileRows, n_steps, lane);
+      const uint32_t row = o_row0 + lane_row(lane);
+      if (lane_class(lane) == 0u && row < o_d_out) store_out<OutT>(o_y, row, fmaf(v, o_scale, o_extra));
     }
-    if (rd + 1u != rounds) lds_barrier();
+    if (r1 != rounds) lds_barrier();
   }
 }
 
