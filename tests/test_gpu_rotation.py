@@ -181,3 +181,25 @@ def test_rows_too_wide_to_be_rotated_in_the_launch(gpu_rt, orc):
     finally:
         for p in projs:
             gpu_rt.free(p)
+
+
+# Rows that are rotated straight to the products' octets, in a call of its own, against the rotated rows of a group too large for
+# one launch (five matrices): the same values, so the same bits.  m = 8 (the narrowest with octets), tails of 8 and 16 columns;
+# rows around the padding of 16, 64 and 128 and around 256, from where both calls take the second way.
+@pytest.mark.parametrize("n,rows", [(31 * 8, 2), (31 * 8, 17), (1024, 16), (1024, 65), (3 * 1024, 64), (3 * 1024, 130), (4096, 256), (4096, 257)])
+def test_rotated_rows_to_octets(gpu_rt, n, rows):
+    import torch
+
+    projs = [gpu_rt.upload(_rotated(f"model.layers.3.mlp.p{i}.weight", 48, n, 5 + i, 77)) for i in range(5)]
+    try:
+        x = _x16(synth.make_activation(n, seed=n + rows, rows=rows))
+        ys = [torch.empty((rows, 48), dtype=torch.float32, device="cuda") for _ in projs]
+        gpu_rt.forward_batched_group_into(projs, x, ys)
+        junk = torch.full((rows, n), float("nan"), dtype=torch.float16, device="cuda")  # what the octets' padding must not keep
+        gpu_rt.forward_batched(projs[0], junk)
+        alone = [gpu_rt.forward_batched(p, x, out_dtype=torch.float32) for p in projs]
+    finally:
+        for p in projs:
+            gpu_rt.free(p)
+    for y, z in zip(ys, alone):
+        assert torch.isfinite(z).all() and torch.equal(y, z)
