@@ -504,7 +504,7 @@ def main():
             "traffic": int(prof["traffic_bytes_per_launch"]) if prof_ok and "traffic_bytes_per_launch" in prof else None,
             "traffic_source": TRAFFIC_PROFILE if prof_ok else None,
             "profiled_kernel_avg_us": prof.get("kernel_avg_us"),
-            # what binds: the tiles' way from memory, 13 bytes per block where the encoding has 6
+            # what binds: the tiles' way from memory, 10 bytes per block where the encoding has 6
             "limited_by": "hbm",
             "valu_slots_per_block": prof.get("valu_slots_per_block") if prof_ok else None,
             "valu_busy_frac": prof.get("valu_busy_frac") if prof_ok else None,

@@ -92,7 +92,7 @@ int llvq_hip_host_decode(uint64_t idx, int8_t point[24], int* shell);
 
 /* upload_matrix (fused_cuda.rs:1058): validates, range-checks every index
  * (IndexOutOfRange, format.rs:389-392), copies the record to the device and unranks its codes there,
- * once: 13 bytes per block of 24 weights stay on the device.  Waits for the runtime's stream.  May be
+ * once: 10 bytes per block of 24 weights stay on the device.  Waits for the runtime's stream.  May be
  * called from several threads (uploads of one runtime take turns), also while another thread launches. */
 int llvq_hip_matrix_upload(llvq_rt* rt, const llvq_matrix_desc* desc, llvq_mat** out);
 

@@ -9,7 +9,8 @@
 // exactly what a lane hands to a 16-deep (32 x 32) or 32-deep (16 x 16) product step, so a wavefront turns the ten bytes
 // of a block that its lanes load into its own fragments: no weights pass through LDS, and the order in which the products walk the
 // columns is the order the blocks lie in (the lane groups of a fragment hold the same octet of two or four neighbouring
-// blocks).  17 instructions per eight weights, and 8 per block to put its three octets together.
+// blocks).  17 instructions per eight weights, and 8 per block to put its three octets together; 12 and 4 in the wide kernels,
+// which look the weights up.
 //
 // The activations come as octets: xt[c][m] = columns 8 c .. 8 c + 7 of row m, 16 bytes, m_pad rows to a column octet, so
 // that the fragments of 16 or 32 rows are runs of 256 or 512 bytes (tile_activations_kernel; in x they would be 16-byte
@@ -518,21 +519,24 @@ struct StoreEach {
 };
 
 // ---- more activation rows ----------------------------------------------------------------------------
-// What bounds it: the chain of a step, in which the matrix cores are busy half the time (51 % for CF = 8, counters in
-// profiles/; 38 instructions of unpacking run beside every 2 CF products), and tiles that are no multiple of the CUs (192
-// workgroups for gate and up of an 8B layer at 512 rows).  A workgroup of four wavefronts takes 256 weight rows by 32 CF activation rows; a wavefront unpacks 64 rows
-// (two fragments) against all of the activation rows (CF fragments).  CF = 8: 256 accumulators and one wavefront on a
-// SIMD, half the unpacking and a workgroup on every CU (1.28 us a step, where the products alone take 0.85 on numbers
-// like these in a loop of nothing else); CF = 4: half of that, two workgroups on a CU (0.69 us a step each) or one (0.8), for batches and matrices
-// that do not fill the other.
+// What bounds it: a wavefront with a SIMD to itself issues an instruction every four cycles at the most, and a step has 270
+// beside its 48 products of 32 cycles (RF = 2, CF = 8), not all of which fall between those; what it waits for, nothing
+// else fills.  Then power: a loop of nothing but products on random numbers reaches 1650 TFLOP/s, at three quarters of the clock.
+// So what counts is the number of instructions, and where they stand.  A workgroup of four wavefronts takes 128 RF weight rows by 32 CF
+// activation rows; a wavefront unpacks 32 RF rows (RF fragments) against all of the activation rows (CF fragments).  CF = 8, RF = 2:
+// 256 accumulators, half the unpacking for a product (1.21 us a step).  RF = 3, CF = 4 (gemm_tall_kernel): three quarters of
+// that tile, half as much unpacking again for a product (1.12 us), for matrices whose tiles of the other leave CUs idle: gate and up of
+// an 8B layer at 512 rows are 192 of those and 256 of these, 112.6 and 110.2 us; of a 4B layer at 500 rows 152 and 204, 78 and 73 us.
+// CF = 4, RF = 2: two workgroups on a CU (0.76 us a step each) or one (0.80), for batches and matrices that fill neither.
 // Octets and tiles go from memory to LDS without passing through registers, two to three steps of 48 columns (two
 // blocks) ahead.
 // PAIR: both terms of the weights against the same activations, 2 CF more products a round; every step's sums go to f64
-// ones (512 registers: CF = 4 and one wavefront on a SIMD).  2.4 us a step; 13000 x 5121 at 600 rows 115 -> 250 to 280 us.
+// ones (512 registers: CF = 4, RF = 2 and one wavefront on a SIMD).  2.5 us a step, of which moving those sums in and out of the
+// accumulator registers is most; 13000 x 5121 at 600 rows 115 -> 250 to 280 us.
 // Launches with too few tiles to fill the chip split the columns (`splits`): partial sums go to the workspace and
 // gemm_reduce_kernel adds them in order; otherwise the tile is finished here.
-// Gate and up of an 8B layer (24576 x 4096) at 512 rows: 158 -> 116 us, 886 TFLOP/s; a plain f16 product of that size
-// by the vendor's library runs at 1151 on this card (a loop of nothing but products on random numbers reaches 1650).
+// Gate and up of an 8B layer (24576 x 4096) at 512 rows: 116 -> 110 us, 935 TFLOP/s (116 with 17 binary16 operations an octet and
+// 13 bytes a block; 121 with those and ten); a plain f16 product of that size by the vendor's library runs at 1159 on this card.
 template <int RF>
 __host__ __device__ constexpr uint32_t gemm_wide_rows() { return 128u * RF; }
 template <int RF>
@@ -848,7 +852,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
 #pragma unroll
       for (int k = 0; k < RF; ++k) w[p][k] = to[p][k];
   };
-  // the lists first, into the buffer that is filled last: they are put in order while the first step's octets and tiles come
+  // the lists first, into the buffer that is filled last: the lanes take theirs while the first step's octets and tiles come
   const uint32_t slots = t.slots, n_listed = 2u * RF * slots;
   const uint32_t lists_at = 3u * kBuf + wave * (gemm_wide_lists<RF>() + 64u * 20u);
   const uint8_t* const lists = uniform_global(rec0 + stride - slots * 16u);
