@@ -591,8 +591,6 @@ __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-// At the end of a branch that is seldom taken: the compiler would otherwise have the common way wait for what is in flight there.
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 // A barrier by itself: what LDS reads of a wavefront are in flight it has not begun to need, and what they read stays.
 __device__ __forceinline__ void wide_barrier() {
   asm volatile("" : : : "memory");
