@@ -29,6 +29,7 @@
 #pragma once
 
 #include "block_code.h"
+#include "step_sums.h"
 
 namespace llvq {
 
@@ -37,15 +38,12 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr uint32_t kTileRows = 16;
 constexpr uint32_t kUnitBytes = 640;
-constexpr uint32_t kStepUnits = 8;
-constexpr uint32_t kStepBlocks = 4 * kStepUnits;
 constexpr uint32_t kTileTableBytes = kScaleSlots * 4;
 
 // Floats of a row's tail columns that a lane of its four holds: column c is the (c / 4)-th of lane class c % 4.
 __host__ __device__ inline uint32_t tail_depth(uint32_t tail_w) { return (tail_w + 3u) >> 2; }
 __host__ __device__ inline uint32_t tile_head_bytes(uint32_t tail_w) { return 128u + 256u * tail_depth(tail_w); }
 __host__ __device__ inline uint32_t tile_units(uint32_t nb) { return (nb + 3u) >> 2; }
-__host__ __device__ inline uint32_t tile_steps(uint32_t nb) { return (nb + kStepBlocks - 1u) / kStepBlocks; }
 // Places in a tile's list, a multiple of eight: of uniformly drawn points of shells 2..12 0.08 % are escapes (with shell 13
 // 0.4 %), so as many as a tile has of them on average and four deviations more.  (Shell 13 takes no batched products, whose
 // kernels have room for 32.)
@@ -272,21 +270,6 @@ __device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub
 }
 
 // ---- batch-1 product ------------------------------------------------------------------------------
-constexpr uint32_t kGemvMaxWaves = 16;
-constexpr uint32_t kGemvWideSteps = 2;  // steps of a wavefront where a row has more than sixteen
-constexpr uint32_t kGemvRounds = 8;     // tiles per team between two sums over the team's wavefronts, at the most
-
-// A tile's steps go to a team of wavefronts, one each (two each past sixteen).  A row is added up in an order that does not
-// depend on that: the lanes of a step (rows_sum), the steps of equal number mod 4 one behind the other, those four sums;
-// so a matrix gives the same bits whatever it shares a launch with.
-__host__ __device__ inline uint32_t gemv_team(uint32_t nb) {
-  const uint32_t steps = tile_steps(nb);
-  return steps > kGemvMaxWaves ? kGemvMaxWaves : steps ? steps : 1u;
-}
-__host__ __device__ inline bool gemv_wide(uint32_t nb) { return nb > kStepBlocks * kGemvMaxWaves; }
-// ... and so that there is a wavefront for each of the workgroup's
-__host__ __device__ inline uint32_t gemv_batch(uint32_t team) { return team < kGemvRounds ? team : kGemvRounds; }
-constexpr uint32_t kGemvMaxBlocks = kStepBlocks * kGemvMaxWaves * kGemvWideSteps;
 // Units of the planes in LDS: whole steps, and a step of zeros behind them for the wavefronts whose steps end early.
 __host__ __device__ inline uint32_t gemv_plane_units(uint32_t nb) { return (tile_steps(nb) + 1u) * kStepUnits; }
 
@@ -311,7 +294,7 @@ struct GemvLds {
   float* xtail;      // [32]
   float* red;        // [16]
   uint32_t* planes;  // [plane units][XPlanes::kDwords]
-  float* part;       // [kGemvRounds][16 or 32 steps][16 rows]
+  float* part;       // [kGemvRounds][sums_steps][16 rows]
   float* xf;         // [d_in] f32 values of a rotated activation
 };
 __host__ __device__ inline uint32_t gemv_lds_fixed() { return 128u + 64u; }
@@ -871,7 +854,7 @@ __device__ __forceinline__ float steps_sum(const float* part, uint32_t steps, ui
 #pragma unroll
   for (uint32_t i = 0; i < MAX / 4; ++i) {
     const uint32_t s = 4u * i + lane_class(lane);
-    v[i] = part[min(s, MAX - 1u) * kTileRows + lane_row(lane)];
+    v[i] = part[sums_read(i, lane_class(lane), steps) * kTileRows + lane_row(lane)];
     v[i] = s < steps ? v[i] : 0.f;
   }
 #pragma unroll
@@ -913,7 +896,7 @@ __device__ __forceinline__ void tile_mat(const GemvArgs& a, uint32_t tile, const
 template <typename OutT, int SRC, bool WIDE>
 __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
   constexpr int DIG = std::is_same<OutT, __half>::value ? 4 : 6;
-  constexpr uint32_t kSteps = WIDE ? kGemvWideSteps : 1u, kMaxSteps = kGemvMaxWaves * kSteps;
+  constexpr uint32_t kSteps = WIDE ? kGemvWideSteps : 1u;
   extern __shared__ __align__(16) uint8_t smem[];
   const GemvLds L = gemv_lds<DIG, WIDE>(smem, gemv_plane_units(a.nb));
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -976,7 +959,7 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
       const Record nx = record_of(min(next, a.n_tiles - 1u));
       const uint32_t lanes_table = table, keep = more ? 0xFFFFFFFFu : 0u;
       const uint8_t* base = scalar_base(nx.rec);
-      float* const part = L.part + ((rd - r0) * kMaxSteps + team * a.team) * kTileRows;
+      float* const part = L.part + sums_at(rd - r0, team, a.team, WIDE) * kTileRows;
       table = scale_table(nx.base, lane);  // in front of the pieces, so that the next round waits for it alone
 #pragma unroll
       for (uint32_t j = 0; j < kSteps; ++j) {
@@ -996,7 +979,7 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
       void* o_y;
       uint32_t o_row0, o_d_out, o_stride, o_slots;
       tile_mat(a, o_tile, o_base, o_y, o_row0, o_d_out, o_stride, o_slots);
-      const float v = steps_sum<kMaxSteps>(L.part + (my_round * kMaxSteps + my_team * a.team) * kTileRows, n_steps, lane);
+      const float v = steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(my_round, my_team, a.team, WIDE) * kTileRows, n_steps, lane);
       const uint32_t row = o_row0 + lane_row(lane);
       if (lane_class(lane) == 0u && row < o_d_out) store_out<OutT>(o_y, row, fmaf(v, o_scale, o_extra));
     }

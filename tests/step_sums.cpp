@@ -1,0 +1,25 @@
+// Every place of LDS that the batch-1 product's sums over a tile's steps are read from (step_sums.h), for every row length, round
+// and team of a workgroup: one that the tile's own wavefronts wrote.  Prints the first that is not and returns 1.
+#include "step_sums.h"
+
+#include <cstdio>
+
+using namespace llvq;
+
+int main() {
+  for (uint32_t nb = 0; nb <= kGemvMaxBlocks; ++nb) {
+    const bool wide = gemv_wide(nb);
+    const uint32_t steps = tile_steps(nb), team = gemv_team(nb), teams = kGemvMaxWaves / team, room = kGemvRounds * sums_steps(wide);
+    for (uint32_t round = 0; round < gemv_batch(team); ++round)
+      for (uint32_t t = 0; t < teams; ++t)
+        for (uint32_t i = 0; i < sums_steps(wide) / 4u; ++i)
+          for (uint32_t c = 0; c < 4u; ++c) {
+            const uint32_t begin = sums_at(round, t, team, wide), at = begin + sums_read(i, c, steps);
+            if (at >= room || (steps && at >= begin + steps) || (4u * i + c < steps && at != begin + 4u * i + c)) {
+              std::printf("%u blocks, round %u, team %u: read %u of %u\n", nb, round, t, at, room);
+              return 1;
+            }
+          }
+  }
+  return 0;
+}
