@@ -110,8 +110,8 @@ LLVQ_HD void block_octets(uint32_t d0, uint32_t d1, uint32_t s3, uint32_t (&w)[3
 }
 
 // What a code of kBlockEscape or more stands for: the first octet's nibbles with nothing hidden in them, the window, the
-// scale's slot, whether it is the negative, and the coordinate that is 16 below (0..23, more: none).  About 45 instructions,
-// which a wavefront runs for one in twenty of its blocks (where any of its lanes has such a point).
+// scale's slot, whether it is the negative, and the coordinate that is 16 below (0..23, more: none).  About 45 instructions; who
+// puts the coordinates back into a form of its own needs as many again or more (gemm_kernel.h: 120 in gemm_escape, 200 in code_block).
 struct BlockEscape {
   uint32_t w0, win, slot, negative, at;
 };
@@ -133,6 +133,34 @@ LLVQ_HD BlockEscape block_escape(const uint32_t (&w)[3], uint32_t meta) {
   const int norm = squares + 2 * c * total + 24 * c * c + (none ? 0 : 256 - 32 * far);
   x.slot = (k & 1u) * 12u + ((uint32_t)norm >> 4) - 2u;
   return x;
+}
+
+// For who looks a coordinate's three bits up in eight values, at i (as a signed number) 2 i + win - 3: an index that none of
+// the others has, in the nibbles now in the far one's place, and the far one's value (24 places on: no index, 8).  There is one:
+// no point of shells up to 13 has more than eight different coordinates (nine of one parity have squares that add up to 240
+// or more), and the far one is unlike all others.  About 70 instructions.  w: the octets, the first with nothing hidden in it.
+struct EscapePick {
+  uint32_t index;
+  int value;
+};
+LLVQ_HD EscapePick escape_pick(uint32_t (&w)[3], const BlockEscape& e) {
+  uint32_t used = 0;
+  int far = 0;
+#pragma unroll
+  for (uint32_t o = 0; o < 3; ++o) {
+    const bool here = e.at >> 3 == o;
+    const uint32_t at = here ? 15u << (4u * (e.at & 7u)) : 0u;
+    far = here ? nibble_at(w[o], e.at & 7u) : far;
+    const uint32_t others = bfi32(at, w[o] >> 4 | w[o] << 28, w[o]);  // its neighbour's instead
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) used |= 1u << ((others >> (4u * q + 1u)) & 7u);
+  }
+  EscapePick p{8u, far + (int)e.win - 19};
+  if (e.at < 24u) p.index = (uint32_t)__builtin_ctz(~used & 0x1FFu);
+#pragma unroll
+  for (uint32_t o = 0; o < 3; ++o)
+    if (e.at >> 3 == o) w[o] = bfi32(15u << (4u * (e.at & 7u)), (p.index & 7u) << (4u * (e.at & 7u) + 1u), w[o]);
+  return p;
 }
 
 }  // namespace llvq

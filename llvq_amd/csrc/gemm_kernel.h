@@ -648,17 +648,21 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
   auto load_x = [&](uint32_t buffer, uint32_t i) __attribute__((always_inline)) {
     load_three_to_lds(smem_at + buffer + (wave * kLoadsX + 3u * i) * 1024u, x_off[3 * i], x_off[3 * i + 1], x_off[3 * i + 2], from_x);
   };
-  auto load_w = [&](uint32_t buffer) __attribute__((always_inline)) {  // and on to the next step
+  auto load_w = [&](uint32_t buffer) __attribute__((always_inline)) {
     load_tiles_to_lds<RF>(smem_at + buffer + gemm_wide_x_bytes<CF>() + wave * kTileBytes, w_off, from_unit + from_odd, from_unit);
-    from_x += from_left ? x_step : 0u;
-    from_unit += from_left && from_odd ? kUnitBytes : 0u;
-    from_odd ^= from_left ? 128u : 0u;
-    from_left -= from_left ? 1u : 0u;
+  };
+  auto to_next_step = [&](uint32_t part) __attribute__((always_inline)) {  // (in three: between two products there is room for no more)
+    if (part == 0u) from_x += from_left ? x_step : 0u;
+    if (part == 1u) from_unit += from_left && from_odd ? kUnitBytes : 0u;
+    if (part == 2u) from_odd ^= from_left ? 128u : 0u;
+    if (part == 2u) from_left -= from_left ? 1u : 0u;
   };
   auto load = [&](uint32_t buffer) __attribute__((always_inline)) {
 #pragma unroll
     for (uint32_t i = 0; i < (uint32_t)kLoadsX / 3u; ++i) load_x(buffer, i);
     load_w(buffer);
+#pragma unroll
+    for (uint32_t part = 0; part < 3u; ++part) to_next_step(part);
   };
   acc16_t acc[RF][CF];
   double sum[PAIR ? RF : 1][PAIR ? CF : 1][16];  // of the steps, with PAIR
@@ -727,51 +731,101 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
   };
   // Escapes (block_code.h): a lane keeps one of this wavefront's, from its tiles' lists, as a block that picks from weights of
   // its own, and puts it in the place of the code in LDS once that has come; where there is none in a step that is one
-  // comparison.  (Their codes read as they came, 120 instructions in one of ten steps and so in a third of a workgroup's, cost
+  // comparison.  (Their codes read as they came, in one of ten steps and so in a third of a workgroup's, cost
   // 6 to 10 % of the time, every wavefront waiting for the slowest; weights exchanged where they are unpacked, 7 %.)
   // at: {d0, d1} and {s, meta} in the wavefront's tiles, 12 bits each, and the block of its unit.  (With PAIR it waits in LDS.)
   uint32_t own_step = ~0u;
   ValueBlock own{};
   ValueBlock* const own_lds = reinterpret_cast<ValueBlock*>(smem + kWideDepth * kBuf) + tid;
-  bool read_codes = false, decode = false;  // a tile's list does not count, or there are more than lanes; this step's are read as they are
+  // What no lane keeps, because it is past 64 or of a list that does not count, is read from its code, and left_steps says in which
+  // steps that can be: there the codes are counted, and where they are more than lanes keep, every one of them goes to a lane, which reads
+  // it, some 250 instructions, and puts it in its own place likewise.  Steps with more than kWaveValues are for every lane to
+  // read its blocks, 200 instructions a fragment that has one.  Gate and up of a 4B layer at 512 rows, 81 us: with one tile whose
+  // list does not count 101 -> 87 us, with one escape in a hundred blocks 191 -> 124 us; 17408 x 17408 with the escapes of uniform
+  // codes, past 64 in one wavefront of six, 500 -> 360 us, without any 350 (before: from the first of these on every step was read by every
+  // lane, 500 instructions a fragment).
+  bool some_left = false;
+  uint32_t left_steps = 0;  // bit s of the 2048 in the lanes: step s0 + s (+ 2048 ...) may have one of those
   const uint32_t my_tiles = gemm_wide_x_bytes<CF>() + wave * kTileBytes;
-  auto place_escapes = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) {
+  const auto tile_place = [&](uint32_t tile_of, uint32_t row, uint32_t blk) __attribute__((always_inline)) {
+    return (tile_of * 256u + (row >> 3) * 128u + (row & 7u) * 16u + (blk & 1u) * 8u) | (512u * RF + tile_of * 128u + (row & 7u) * 16u + (row >> 3) * 8u) << 12 | (blk & 3u) << 24;
+  };
+  const auto code_block = [&](uint32_t (&o)[3], uint32_t meta) __attribute__((always_inline)) {  // (for all lanes: the scales are in all of them)
+    const BlockEscape e = block_escape(o, meta);
+    o[0] = e.w0;
+    const EscapePick p = escape_pick(o, e);
+    ValueBlock b{{{}, {}}, o[0] | ((o[2] >> 1) & 0x11111111u), o[1] | ((o[2] >> 2) & 0x11111111u), (o[2] >> 3) & 0x11111111u, 0u};
+    const float scale = scale_of(e.slot << 3);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int v = (uint32_t)i == p.index ? p.value : 2 * (i < 4 ? i : i - 8) + (int)e.win - 3;
+      value_to(b.t, i, (float)(e.negative ? -v : v) * scale);
+    }
+    return b;
+  };
+  // b of the lanes in `there`, 16 at the most, into the tiles.
+  const auto place = [&](const ValueBlock& b, uint64_t there, uint8_t* tiles) __attribute__((always_inline)) {
+    const uint32_t v = kBlockEscape + wave * kWaveValues + __builtin_amdgcn_mbcnt_hi((uint32_t)(there >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)there, 0u));
+    *reinterpret_cast<u32x2_t*>(tiles + (b.at & 0xFFFu)) = u32x2_t{b.d0, b.d1};
+    uint32_t* const meta = reinterpret_cast<uint32_t*>(tiles + ((b.at >> 12) & 0xFFFu));
+    const uint32_t k = b.at >> 24;
+    __hip_atomic_fetch_and(meta, ~(0x11111111u << k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    __hip_atomic_fetch_or(meta, b.s << k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    reinterpret_cast<uint8_t*>(meta + 1)[k] = (uint8_t)v;
+    reinterpret_cast<u32x4_t*>(wide_smem)[v] = b.t.hi;
+    if constexpr (PAIR) reinterpret_cast<u32x4_t*>(wide_smem + kValueBytes)[v] = b.t.lo;
+  };
+  uint32_t codes[RF];  // the lane's blocks' of the step after
+  const auto read_codes = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k) codes[k] = (smem + (buffer + meta_at) + k * 256u + 4u)[2u * (s & 1u) + h];
+  };
+  auto place_escapes = [&](auto left_t, uint32_t s, uint32_t buffer) __attribute__((always_inline)) -> bool {  // whether the step is read by every lane
     const uint64_t mine = __builtin_amdgcn_ballot_w64(own_step == s);
-    decode = read_codes;
-    if (mine) {
-      if ((uint32_t)__builtin_popcountll(mine) > kWaveValues) {
-        decode = true;
-      } else if (own_step == s) {
-        const uint32_t v = kBlockEscape + wave * kWaveValues + __builtin_amdgcn_mbcnt_hi((uint32_t)(mine >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mine, 0u));
-        uint8_t* const tiles = smem + buffer + my_tiles;
-        if constexpr (PAIR) own = *own_lds;
-        *reinterpret_cast<u32x2_t*>(tiles + (own.at & 0xFFFu)) = u32x2_t{own.d0, own.d1};
-        uint32_t* const meta = reinterpret_cast<uint32_t*>(tiles + ((own.at >> 12) & 0xFFFu));
-        const uint32_t k = own.at >> 24;
-        __hip_atomic_fetch_and(meta, ~(0x11111111u << k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        __hip_atomic_fetch_or(meta, own.s << k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        reinterpret_cast<uint8_t*>(meta + 1)[k] = (uint8_t)v;
-        reinterpret_cast<u32x4_t*>(wide_smem)[v] = own.t.hi;
-        if constexpr (PAIR) reinterpret_cast<u32x4_t*>(wide_smem + kValueBytes)[v] = own.t.lo;
+    uint8_t* const tiles = smem + buffer + my_tiles;
+    const uint32_t bit = s - s0;
+    if (left_t && s < s1 && ((uint32_t)__builtin_amdgcn_readlane((int)left_steps, (bit >> 5) & 63u) >> (bit & 31u) & 1u)) {
+      if constexpr (!std::is_same<decltype(left_t), std::true_type>::value) read_codes(s, buffer);
+      // lane i's the i-th of the step's escapes: fragment, row and half of a step
+      uint32_t n = 0, at = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
+        for (uint64_t left = __builtin_amdgcn_ballot_w64(codes[k] >= kBlockEscape); left; left &= left - 1u) {
+          const uint32_t l = (uint32_t)__builtin_ctzll(left);
+          at = lane == n ? tile_place(2u * k + ((l & 31u) >> 4), l & 15u, 2u * (s & 1u) + (l >> 5)) : at;
+          ++n;
+        }
+      }
+      if (n > kWaveValues) return true;
+      if (n != (uint32_t)__builtin_popcountll(mine)) {
+        at = lane < n ? at : tile_place(0u, 0u, 0u);
+        const u32x2_t d = *reinterpret_cast<const u32x2_t*>(tiles + (at & 0xFFFu)), sm = *reinterpret_cast<const u32x2_t*>(tiles + ((at >> 12) & 0xFFFu));
+        const uint32_t k = at >> 24;
+        uint32_t o[3];
+        block_octets(d.x, d.y, sm.x << (3u - k), o);
+        ValueBlock b = code_block(o, (sm.y >> (8u * k)) & 255u);
+        b.at = at;
+        if (lane < n) place(b, (1ull << n) - 1u, tiles);
+        return false;
       }
     }
+    if (mine) {
+      asm volatile("");  // (a branch of its own: as one condition with the next it is six instructions more in every step)
+      if (own_step == s) {
+        if constexpr (PAIR) own = *own_lds;
+        place(own, mine, tiles);
+      }
+    }
+    return false;
   };
   auto decode_escapes = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
       const uint32_t meta = (Bn[k].meta >> 4) & 255u;
-      uint32_t o[3], n[3] = {0, 0, 0};
+      if (!__builtin_amdgcn_ballot_w64(meta >= kBlockEscape)) continue;
+      uint32_t o[3];
       block_octets(Bn[k].w[0], Bn[k].w[1], Bn[k].w[2] << 1, o);
-      const BlockEscape e = block_escape(o, meta);
-      o[0] = e.w0;
-      const int c = (int)e.win - 3;
-      const uint32_t odd = (uint32_t)c & 1u;
-#pragma unroll
-      for (uint32_t q = 0; q < 24u; ++q) {
-        const int v = nibble_at(o[q >> 3], q & 7u) + c - (q == e.at ? 16 : 0);
-        n[q >> 3] |= ((uint32_t)(((e.negative ? -v : v) - (int)odd) >> 1) & 15u) << (4u * (q & 7u));
-      }
-      const ValueBlock b = value_block(n, odd, scale_of(e.slot << 3));
+      const ValueBlock b = code_block(o, meta);
       if (meta >= kBlockEscape) {
         Bn[k].w[0] = b.d0;
         Bn[k].w[1] = b.d1;
@@ -785,7 +839,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       }
     }
   };
-  auto round = [&](uint32_t buffer, uint32_t next, uint32_t last, uint32_t s, auto round_j) __attribute__((always_inline)) {
+  auto round = [&](uint32_t buffer, uint32_t next, uint32_t last, uint32_t s, auto round_j, auto left_t, bool& decode) __attribute__((always_inline)) {
     constexpr uint32_t j = decltype(round_j)::value, jn = j < 2u ? j + 1u : 0u;  // of the products, and of what is unpacked
     constexpr uint32_t kParts = (PAIR && j == 1u ? 8u : 4u) * RF / CF;  // (PAIR: T is read anew behind its last use)
     u32x4_t to[kTerms][RF];
@@ -806,6 +860,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       if (j == 0u && c == (uint32_t)CF / 2u) {
         wide_wait<kLoads>();
         wide_barrier();
+        if constexpr (std::is_same<decltype(left_t), std::true_type>::value) read_codes(s + 1u, next);
       }
 #pragma unroll
       for (int p = (int)kTerms - 1; p >= 0; --p)
@@ -825,6 +880,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
           if (after & 1u) asm volatile("" : "+v"(pick[p].at), "+v"(pick[p].high));
           else asm volatile("" : "+v"(to[p][(after - 1u) >> 2]));
         }
+      if (j == 2u && c < 3u) to_next_step(c);
       if (j == 1u) {
         if (c == CF / 2u) {
 #pragma unroll
@@ -843,7 +899,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (j == 0u) place_escapes(s + 1u, next);
+    if (j == 0u) decode = place_escapes(left_t, s + 1u, next);
     if (j == 1u && decode) decode_escapes();
 #pragma unroll
     for (uint32_t p = 0; p < kTerms; ++p)
@@ -883,8 +939,8 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       const uint32_t from = min(i * 64u + lane, n_listed - 1u);
       const u32x4_t e = raw[from];
       const uint32_t step = (e.w >> 10) & 0x3FFFFu;
-      read_codes |= __builtin_amdgcn_ballot_w64(e.w == ~0u) != 0u;
-      const bool valid = i * 64u + lane < n_listed && e.w != 0u && step >= s0 && step < s1;
+      if (__builtin_amdgcn_ballot_w64(e.w == ~0u)) left_steps = ~0u;
+      const bool valid = i * 64u + lane < n_listed && e.w != 0u && e.w != ~0u && step >= s0 && step < s1;
       const uint64_t there = __builtin_amdgcn_ballot_w64(valid);
       const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(there >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)there, 0u));
       if (valid && at < 64u) {
@@ -892,21 +948,30 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
         kept_tile[at] = from / slots;
       }
       n += (uint32_t)__builtin_popcountll(there);
+      for (uint64_t over = __builtin_amdgcn_ballot_w64(valid && at >= 64u); over; over &= over - 1u) {
+        const uint32_t bit = (uint32_t)__builtin_amdgcn_readlane((int)step, (uint32_t)__builtin_ctzll(over)) - s0;
+        left_steps |= lane == ((bit >> 5) & 63u) ? 1u << (bit & 31u) : 0u;
+      }
     }
-    read_codes |= n > 64u;
     wave_lds_order();
-    if (n && !read_codes) {
+    if (n) {
       const u32x4_t e = kept[lane];
       const uint32_t tile_of = kept_tile[lane], row = e.w >> 28, blk = (e.w >> 9) & 0x7FFFFu, nibbles[3] = {e.x, e.y, e.z};
       own = value_block(nibbles, (e.w >> 8) & 1u, scale_of((e.w & 31u) << 3));
-      own.at = (tile_of * 256u + (row >> 3) * 128u + (row & 7u) * 16u + (blk & 1u) * 8u) | (512u * RF + tile_of * 128u + (row & 7u) * 16u + (row >> 3) * 8u) << 12 | (blk & 3u) << 24;
+      own.at = tile_place(tile_of, row, blk);
       own_step = lane < n ? blk >> 1 : ~0u;
       if constexpr (PAIR) *own_lds = own;
+      if (n > kWaveValues) {  // perhaps more of one step than there is room for
+        uint32_t same = 0;
+        for (uint32_t i = 0; i < min(n, 64u); ++i) same += (uint32_t)__builtin_amdgcn_readlane((int)own_step, i) == own_step ? 1u : 0u;
+        if (__builtin_amdgcn_ballot_w64(lane < n && same > kWaveValues)) left_steps = ~0u;
+      }
     }
   }
+  some_left = __builtin_amdgcn_ballot_w64(left_steps != 0u) != 0u;
   wide_wait<2 * kLoads>();
   lds_barrier();
-  place_escapes(s0, 0);
+  const bool decode_first = place_escapes(some_left, s0, 0);
   read_w(0);
   read_x(0, 0);
 #pragma unroll
@@ -914,7 +979,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
     read_values(k);
     assemble(k);
   }
-  if (decode) decode_escapes();
+  if (decode_first) decode_escapes();
 #pragma unroll
   for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
     B[k] = Bn[k];
@@ -937,26 +1002,33 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) sum[k][c][e] = 0.;
   }
-  uint32_t buffer = 0, next = kBuf, last = 3u * kBuf, s = s0;
-  do {  // (a split has at least one step)
-    round(buffer, next, last, s, std::integral_constant<uint32_t, 0>{});
-    round(buffer, next, last, s, std::integral_constant<uint32_t, 1>{});
-    round(buffer, next, last, s, std::integral_constant<uint32_t, 2>{});
-    last = buffer;
-    buffer = next;
-    next = next + kBuf == kWideDepth * kBuf ? 0u : next + kBuf;
-    if constexpr (PAIR) {
+  auto steps = [&](auto left_t) __attribute__((always_inline)) {
+    uint32_t buffer = 0, next = kBuf, last = 3u * kBuf, s = s0;
+    bool decode = false;
+    do {  // (a split has at least one step)
+      round(buffer, next, last, s, std::integral_constant<uint32_t, 0>{}, left_t, decode);
+      round(buffer, next, last, s, std::integral_constant<uint32_t, 1>{}, left_t, decode);
+      round(buffer, next, last, s, std::integral_constant<uint32_t, 2>{}, left_t, decode);
+      last = buffer;
+      buffer = next;
+      next = next + kBuf == kWideDepth * kBuf ? 0u : next + kBuf;
+      if constexpr (PAIR) {
 #pragma unroll
-      for (int k = 0; k < RF; ++k)
+        for (int k = 0; k < RF; ++k)
 #pragma unroll
-        for (int c = 0; c < CF; ++c) {
+          for (int c = 0; c < CF; ++c) {
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            sum[k][c][e] += (double)acc[k][c][e];
+            for (int e = 0; e < 16; ++e) {
+              sum[k][c][e] += (double)acc[k][c][e];
+            }
           }
-        }
-    }
-  } while (++s < s1);
+      }
+    } while (++s < s1);
+  };
+  // (Two loops: what the rare one needs costs the other 2 % where they are one.  With PAIR two would not fit the registers.)
+  if constexpr (PAIR) steps(some_left);
+  else if (some_left) steps(std::true_type{});
+  else steps(std::false_type{});
   if constexpr (PAIR) {
 #pragma unroll
     for (int k = 0; k < RF; ++k)

@@ -23,7 +23,8 @@ static bool round_trip(const int (&v)[24], uint32_t gain, uint32_t shell) {
   if (!block_encode(n, odd, gain, shell, c)) return false;
   if (c.meta > 255u || (c.s & ~0x11111111u)) return false;
   escapes += c.meta >= kBlockEscape;
-  uint32_t w[3], win = c.meta & 7u, slot = c.meta >> 3, negative = 0, far = 24;
+  uint32_t w[3], win = c.meta & 7u, slot = c.meta >> 3, negative = 0, far = 24, picks[3] = {0, 0, 0};
+  EscapePick pick{8, 0};
   block_octets(c.d0, c.d1, c.s << 3, w);
   if (c.meta >= kBlockEscape) {
     const BlockEscape e = block_escape(w, c.meta);
@@ -32,10 +33,18 @@ static bool round_trip(const int (&v)[24], uint32_t gain, uint32_t shell) {
     slot = e.slot;
     negative = e.negative;
     far = e.at;
+    std::memcpy(picks, w, sizeof w);
+    pick = escape_pick(picks, e);
+    if (far < 24 ? pick.index > 7 : pick.index != 8) return false;
+  } else {
+    std::memcpy(picks, w, sizeof w);
   }
   for (uint32_t i = 0; i < 24; ++i) {
     const int got = nibble_at(w[i / 8], i % 8) + (int)win - 3 - (i == far ? 16 : 0);
     if ((negative ? -got : got) != v[i]) return false;
+    const uint32_t index = (picks[i / 8] >> (4 * (i % 8) + 1)) & 7u;  // the same looked up
+    const int looked = index == pick.index ? pick.value : 2 * ((int)index < 4 ? (int)index : (int)index - 8) + (int)win - 3;
+    if ((negative ? -looked : looked) != v[i] || (picks[i / 8] & 0x11111111u)) return false;
   }
   return shell == 0 || slot == gain * 12u + shell - 2u;
 }

@@ -1,0 +1,85 @@
+"""Wide batched products whose escapes (block codes that say kBlockEscape or more) are not all in what a wavefront keeps of its tiles'
+lists: lists that overflow, more than 64 in a wavefront's share, more than sixteen in a step, beside tiles and steps with few or
+none.  Against the oracle's decoded matrix, through every form of the kernel; and that such matrices are not many times as slow."""
+import numpy as np
+import pytest
+
+from llvq_amd import artifact, synth
+from test_gpu_escapes import _far
+from test_gpu_gemm import _reference, _x16
+
+pytestmark = pytest.mark.gpu
+
+
+def _with_escapes(orc, d_out, nb, tail, share, full=()):
+    """share: of all blocks that are escapes by hand, besides 0.08 % by chance; full: rows of nothing else."""
+    raw = synth.make_matrix(f"model.layers.0.lists.{d_out}x{nb}.weight", d_out, nb * 24 + tail, seed=nb + tail)
+    rng = np.random.default_rng(nb + d_out)
+    idx, gains = raw.unpack()
+    idx = np.array(idx, np.uint64)
+    at = rng.random(idx.size) < share
+    for row in full:
+        at[row * nb:(row + 1) * nb] = True
+    far = _far(orc, 12)
+    idx[at] = rng.choice(far, int(at.sum()))
+    return artifact.RawMatrix(raw.name, d_out, raw.d_in, 12, raw.centroids, raw.row_scales, raw.tail, artifact.pack_codes(idx, gains, artifact.index_bits(12)))
+
+
+# Forms: 384 x 128 (10000 by 1000, 12000 by 1000), 256 x 256 (16384 by 700), 256 x 128 split over the columns (2560 by 500), both terms
+# of the weights split (tail 1) and whole (rows off their boundary).  nb: 17 and 25 blocks, lists of eight, 0.01 is some three a
+# tile and overflows one in thirty; 200 (lists of 16, 96 rows of them) and 541 (lists of 24, 64 rows): 0.004 and 0.0027 are more than 64
+# for most wavefronts, in lists that hold and lists that do not; rows full of them: more than sixteen of a step in one wavefront.
+@pytest.mark.parametrize("d_out,nb,tail,M,off,share,full", [
+    (10000, 17, 8, 1000, 0, 0.01, ()), (12000, 200, 0, 1000, 0, 0.004, range(96, 130)), (16384, 25, 16, 700, 0, 0.01, range(40, 60)),
+    (2560, 405, 0, 500, 0, 0.003, range(7)), (1000, 541, 0, 1024, 0, 0.0027, ()), (700, 200, 1, 130, 0, 0.004, range(70, 90)), (500, 541, 8, 100, 1, 0.0027, range(9))])
+def test_escapes_past_the_lists(gpu_rt, orc, d_out, nb, tail, M, off, share, full):
+    import torch
+
+    raw = _with_escapes(orc, d_out, nb, tail, share, full)
+    X = synth.make_activation(raw.d_in, seed=nb, rows=M)
+    pick = sorted({0, 1, 31, 32, M // 2, M - 2, M - 1})
+    Y_ref, A_ref = _reference(orc, raw, X[pick])
+    proj = gpu_rt.upload(raw)
+    try:
+        buf = torch.empty(M * raw.d_in + 8, dtype=torch.float16, device="cuda")
+        x = buf[off:off + M * raw.d_in].view(M, raw.d_in)
+        x.copy_(_x16(X))
+        y, again = (torch.empty((M, d_out), dtype=torch.float32, device="cuda") for _ in range(2))
+        gpu_rt.forward_batched_into(proj, x, y)
+        gpu_rt.forward_batched_into(proj, x, again)
+    finally:
+        gpu_rt.free(proj)
+    assert torch.equal(y, again)
+    y = y[pick].double().cpu().numpy()
+    if off or tail % 8:  # both terms: the bar of test_gpu_tiles.py's rows off their boundaries
+        assert np.linalg.norm(y - Y_ref) / np.linalg.norm(Y_ref) < 8 * 2.0 ** -24
+    else:  # weights are rounded to binary16, 2^-11 of each at the most; the sums in binary32 beside that
+        assert np.all(np.abs(y - Y_ref) <= 1.05 * 2.0 ** -11 * A_ref + 1e-7)
+
+
+def test_one_escape_in_a_hundred_blocks_does_not_double_the_time(gpu_rt, orc):
+    """Gate and up of a 4B layer at 512 rows, 81 us with the escapes of uniform codes: with twelve times as many, which no tile's list
+    holds, it took 192 us when every step of such a tile was read by every lane, and 124 where a lane reads each."""
+    import torch
+
+    def time(share):
+        proj = gpu_rt.upload(_with_escapes(orc, 9728, 106, 16, share))
+        x = torch.randn(512, 2560, device="cuda").half()
+        ys = [torch.empty((512, 9728), dtype=torch.float16, device="cuda") for _ in range(2)]
+        took = []
+        try:
+            for _ in range(8):
+                begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                begin.record()
+                for _ in range(10):
+                    gpu_rt.forward_batched_group_into([proj, proj], x, ys)
+                end.record()
+                torch.cuda.synchronize()
+                took.append(begin.elapsed_time(end))
+        finally:
+            gpu_rt.free(proj)
+        return sorted(took)[3]
+
+    usual, many = time(0.0), time(0.01)
+    print(f"OBSERVED {usual * 100:.1f} us, {many * 100:.1f} us with one escape in a hundred blocks")
+    assert many < 1.95 * usual
