@@ -532,7 +532,9 @@ struct StoreEach {
 // blocks) ahead.
 // PAIR: both terms of the weights against the same activations, 2 CF more products a round; every step's sums go to f64
 // ones (512 registers: CF = 4, RF = 2 and one wavefront on a SIMD).  2.5 us a step, of which moving those sums in and out of the
-// accumulator registers is most; 13000 x 5121 at 600 rows 115 -> 250 to 280 us.
+// accumulator registers is most; 13000 x 5121 at 600 rows 115 -> 252 us.  (With arithmetic for the look-ups that loop was as fast over
+// 13 bytes a block, 250 us; small products took 1.5 to 2.5 us less, without lists of escapes to wait for and read: 4096 x 4097 at
+// 130 rows 45.3 us, 47.9 now.)
 // Launches with too few tiles to fill the chip split the columns (`splits`): partial sums go to the workspace and
 // gemm_reduce_kernel adds them in order; otherwise the tile is finished here.
 // Gate and up of an 8B layer (24576 x 4096) at 512 rows: 116 -> 110 us, 935 TFLOP/s (116 with 17 binary16 operations an octet and
@@ -738,13 +740,11 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
   ValueBlock own{};
   ValueBlock* const own_lds = reinterpret_cast<ValueBlock*>(smem + kWideDepth * kBuf) + tid;
   // What no lane keeps, because it is past 64 or of a list that does not count, is read from its code, and left_steps says in which
-  // steps that can be: there the codes are counted, and where they are more than lanes keep, every one of them goes to a lane, which reads
-  // it, some 250 instructions, and puts it in its own place likewise.  Steps with more than kWaveValues are for every lane to
-  // read its blocks, 200 instructions a fragment that has one.  Gate and up of a 4B layer at 512 rows, 81 us: with one tile whose
-  // list does not count 101 -> 87 us, with one escape in a hundred blocks 191 -> 124 us; 17408 x 17408 with the escapes of uniform
-  // codes, past 64 in one wavefront of six, 500 -> 360 us, without any 350 (before: from the first of these on every step was read by every
-  // lane, 500 instructions a fragment).
-  bool some_left = false;
+  // steps that can be: there the codes that no lane keeps go to a lane each, which reads it, some 250 instructions, and puts it in
+  // its own place likewise.  Steps with more than kWaveValues are for every lane to read its blocks, 200 instructions a fragment
+  // that has one.  Gate and up of a 4B layer at 512 rows, 81 us: with one tile whose list does not count 101 -> 87 us, with one
+  // escape in a hundred blocks 191 -> 124 us; 17408 x 17408 with the escapes of uniform codes, past 64 in one wavefront of six,
+  // 500 -> 360 us, without any 350 (before: from the first of these on every step was read by every lane, 500 instructions a fragment).
   uint32_t left_steps = 0;  // bit s of the 2048 in the lanes: step s0 + s (+ 2048 ...) may have one of those
   const uint32_t my_tiles = gemm_wide_x_bytes<CF>() + wave * kTileBytes;
   const auto tile_place = [&](uint32_t tile_of, uint32_t row, uint32_t blk) __attribute__((always_inline)) {
@@ -763,9 +763,9 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
     }
     return b;
   };
-  // b of the lanes in `there`, 16 at the most, into the tiles.
-  const auto place = [&](const ValueBlock& b, uint64_t there, uint8_t* tiles) __attribute__((always_inline)) {
-    const uint32_t v = kBlockEscape + wave * kWaveValues + __builtin_amdgcn_mbcnt_hi((uint32_t)(there >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)there, 0u));
+  // b of the lanes in `there` into the tiles, its weights from place `first` on of the wavefront's sixteen.
+  const auto place = [&](const ValueBlock& b, uint64_t there, uint32_t first, uint8_t* tiles) __attribute__((always_inline)) {
+    const uint32_t v = kBlockEscape + wave * kWaveValues + first + __builtin_amdgcn_mbcnt_hi((uint32_t)(there >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)there, 0u));
     *reinterpret_cast<u32x2_t*>(tiles + (b.at & 0xFFFu)) = u32x2_t{b.d0, b.d1};
     uint32_t* const meta = reinterpret_cast<uint32_t*>(tiles + ((b.at >> 12) & 0xFFFu));
     const uint32_t k = b.at >> 24;
@@ -775,58 +775,67 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
     reinterpret_cast<u32x4_t*>(wide_smem)[v] = b.t.hi;
     if constexpr (PAIR) reinterpret_cast<u32x4_t*>(wide_smem + kValueBytes)[v] = b.t.lo;
   };
-  uint32_t codes[RF];  // the lane's blocks' of the step after
+  auto place_escapes = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) {
+    const uint64_t mine = __builtin_amdgcn_ballot_w64(own_step == s);
+    if (PAIR ? mine != 0u : __builtin_expect(mine != 0u, 0)) {
+      asm volatile("");  // (a branch of its own: as one condition with the next it is six instructions more in every step)
+      if (own_step == s) {
+        if constexpr (PAIR) own = *own_lds;
+        place(own, mine, 0, smem + buffer + my_tiles);
+      }
+    }
+  };
+  const auto some_left = [&](uint32_t s) __attribute__((always_inline)) {
+    return s < s1 && ((uint32_t)__builtin_amdgcn_readlane((int)left_steps, ((s - s0) >> 5) & 63u) >> ((s - s0) & 31u) & 1u) != 0u;
+  };
+  // A step's codes, and those that place_escapes left: placed too (1), for every lane to read its own if there are more than
+  // places (2), or none (0).
+  uint32_t codes[RF];
+  uint64_t left[RF];
   const auto read_codes = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) {
 #pragma unroll
     for (uint32_t k = 0; k < (uint32_t)RF; ++k) codes[k] = (smem + (buffer + meta_at) + k * 256u + 4u)[2u * (s & 1u) + h];
   };
-  auto place_escapes = [&](auto left_t, uint32_t s, uint32_t buffer) __attribute__((always_inline)) -> bool {  // whether the step is read by every lane
-    const uint64_t mine = __builtin_amdgcn_ballot_w64(own_step == s);
+  const auto place_left = [&](uint32_t s, uint32_t buffer) __attribute__((always_inline)) -> uint32_t {
     uint8_t* const tiles = smem + buffer + my_tiles;
-    const uint32_t bit = s - s0;
-    if (left_t && s < s1 && ((uint32_t)__builtin_amdgcn_readlane((int)left_steps, (bit >> 5) & 63u) >> (bit & 31u) & 1u)) {
-      if constexpr (!std::is_same<decltype(left_t), std::true_type>::value) read_codes(s, buffer);
-      // lane i's the i-th of the step's escapes: fragment, row and half of a step
-      uint32_t n = 0, at = 0;
 #pragma unroll
-      for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
-        for (uint64_t left = __builtin_amdgcn_ballot_w64(codes[k] >= kBlockEscape); left; left &= left - 1u) {
-          const uint32_t l = (uint32_t)__builtin_ctzll(left);
-          at = lane == n ? tile_place(2u * k + ((l & 31u) >> 4), l & 15u, 2u * (s & 1u) + (l >> 5)) : at;
-          ++n;
-        }
-      }
-      if (n > kWaveValues) return true;
-      if (n != (uint32_t)__builtin_popcountll(mine)) {
-        at = lane < n ? at : tile_place(0u, 0u, 0u);
-        const u32x2_t d = *reinterpret_cast<const u32x2_t*>(tiles + (at & 0xFFFu)), sm = *reinterpret_cast<const u32x2_t*>(tiles + ((at >> 12) & 0xFFFu));
-        const uint32_t k = at >> 24;
-        uint32_t o[3];
-        block_octets(d.x, d.y, sm.x << (3u - k), o);
-        ValueBlock b = code_block(o, (sm.y >> (8u * k)) & 255u);
-        b.at = at;
-        if (lane < n) place(b, (1ull << n) - 1u, tiles);
-        return false;
-      }
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k) left[k] = __builtin_amdgcn_ballot_w64(codes[k] >= kBlockEscape);
+    const uint64_t mine = __builtin_amdgcn_ballot_w64(own_step == s);
+    const uint32_t first = (uint32_t)__builtin_popcountll(mine);
+    const uint32_t mine_at = PAIR ? own_lds->at : own.at;
+    for (uint64_t m = mine; m; m &= m - 1u) {
+      const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)mine_at, (uint32_t)__builtin_ctzll(m));
+#pragma unroll
+      for (uint32_t k = 0; k < (uint32_t)RF; ++k)
+        left[k] &= ((at >> 9) & 7u) == k ? ~(1ull << (((at >> 8) & 1u) * 16u + ((at >> 7) & 1u) * 8u + ((at >> 4) & 7u) + ((at >> 3) & 1u) * 32u)) : ~0ull;
     }
-    if (mine) {
-      asm volatile("");  // (a branch of its own: as one condition with the next it is six instructions more in every step)
-      if (own_step == s) {
-        if constexpr (PAIR) own = *own_lds;
-        place(own, mine, tiles);
+    // lane i's the i-th of them: fragment, row and half of a step
+    uint32_t n = 0, at = tile_place(0u, 0u, 0u);
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k)
+      for (uint64_t m = left[k]; m; m &= m - 1u) {
+        const uint32_t l = (uint32_t)__builtin_ctzll(m);
+        at = lane == n ? tile_place(2u * k + ((l & 31u) >> 4), l & 15u, 2u * (s & 1u) + (l >> 5)) : at;
+        ++n;
       }
-    }
-    return false;
+    if (n == 0u || first + n > kWaveValues) return n ? 2u : 0u;
+    const u32x2_t d = *reinterpret_cast<const u32x2_t*>(tiles + (at & 0xFFFu)), sm = *reinterpret_cast<const u32x2_t*>(tiles + ((at >> 12) & 0xFFFu));
+    const uint32_t k = at >> 24;
+    uint32_t o[3];
+    block_octets(d.x, d.y, sm.x << (3u - k), o);
+    ValueBlock b = code_block(o, (sm.y >> (8u * k)) & 255u);
+    b.at = at;
+    if (lane < n) place(b, (1ull << n) - 1u, first, tiles);
+    return 1u;
   };
   auto decode_escapes = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
-      const uint32_t meta = (Bn[k].meta >> 4) & 255u;
-      if (!__builtin_amdgcn_ballot_w64(meta >= kBlockEscape)) continue;
+      if (__builtin_expect(!left[k], 1)) continue;
       uint32_t o[3];
       block_octets(Bn[k].w[0], Bn[k].w[1], Bn[k].w[2] << 1, o);
-      const ValueBlock b = code_block(o, meta);
-      if (meta >= kBlockEscape) {
+      const ValueBlock b = code_block(o, (Bn[k].meta >> 4) & 255u);
+      if (left[k] >> lane & 1u) {
         Bn[k].w[0] = b.d0;
         Bn[k].w[1] = b.d1;
         Bn[k].w[2] = (b.d0 & 0x11111111u) | (b.d1 & 0x11111111u) << 1 | b.s << 2;
@@ -839,7 +848,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       }
     }
   };
-  auto round = [&](uint32_t buffer, uint32_t next, uint32_t last, uint32_t s, auto round_j, auto left_t, bool& decode) __attribute__((always_inline)) {
+  auto round = [&](uint32_t buffer, uint32_t next, uint32_t last, uint32_t s, auto round_j, auto left_t, uint32_t& found) __attribute__((always_inline)) {
     constexpr uint32_t j = decltype(round_j)::value, jn = j < 2u ? j + 1u : 0u;  // of the products, and of what is unpacked
     constexpr uint32_t kParts = (PAIR && j == 1u ? 8u : 4u) * RF / CF;  // (PAIR: T is read anew behind its last use)
     u32x4_t to[kTerms][RF];
@@ -860,7 +869,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       if (j == 0u && c == (uint32_t)CF / 2u) {
         wide_wait<kLoads>();
         wide_barrier();
-        if constexpr (std::is_same<decltype(left_t), std::true_type>::value) read_codes(s + 1u, next);
+        if constexpr (decltype(left_t)::value) read_codes(s + 1u, next);
       }
 #pragma unroll
       for (int p = (int)kTerms - 1; p >= 0; --p)
@@ -899,8 +908,10 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (j == 0u) decode = place_escapes(left_t, s + 1u, next);
-    if (j == 1u && decode) decode_escapes();
+    if (j == 0u) place_escapes(s + 1u, next);
+    if constexpr (decltype(left_t)::value && j == 0u) found = some_left(s + 1u) ? place_left(s + 1u, next) : 0u;
+    if constexpr (decltype(left_t)::value && j == 1u)
+      if (found == 2u) decode_escapes();
 #pragma unroll
     for (uint32_t p = 0; p < kTerms; ++p)
 #pragma unroll
@@ -965,29 +976,40 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
         uint32_t same = 0;
         for (uint32_t i = 0; i < min(n, 64u); ++i) same += (uint32_t)__builtin_amdgcn_readlane((int)own_step, i) == own_step ? 1u : 0u;
         if (__builtin_amdgcn_ballot_w64(lane < n && same > kWaveValues)) left_steps = ~0u;
+        if (same > kWaveValues) own_step = ~0u;
       }
     }
   }
-  some_left = __builtin_amdgcn_ballot_w64(left_steps != 0u) != 0u;
+  const bool any_left = __builtin_amdgcn_ballot_w64(left_steps != 0u) != 0u;
   wide_wait<2 * kLoads>();
   lds_barrier();
-  const bool decode_first = place_escapes(some_left, s0, 0);
-  read_w(0);
-  read_x(0, 0);
+  // A step from its tiles in LDS: the first, and with PAIR those that something was left of, whose first octet is unpacked already.
+  auto begin = [&](uint32_t buffer, bool all, auto first) __attribute__((always_inline)) {
+    read_w(buffer);
+    if constexpr (decltype(first)::value) read_x(buffer, 0);
 #pragma unroll
-  for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
-    read_values(k);
-    assemble(k);
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
+      read_values(k);
+      assemble(k);
+    }
+    if (__builtin_expect(all, 0)) decode_escapes();
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
+      B[k] = Bn[k];
+      if constexpr (!PAIR) T[k][0] = Tn[k];
+      ValuePick pick[kTerms];
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; ++i) unpack_part(std::integral_constant<uint32_t, 0>{}, 4u * k + i, pick, w);
+    }
+  };
+  // (What is rare is said to be: it then stands behind the rest of the kernel, and 6000 x 1000 at 130 rows takes 28.9 us, not 29.5.)
+  place_escapes(s0, 0);
+  uint32_t found = 0;
+  if (__builtin_expect(any_left && some_left(s0), 0)) {
+    read_codes(s0, 0);
+    found = place_left(s0, 0);
   }
-  if (decode_first) decode_escapes();
-#pragma unroll
-  for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
-    B[k] = Bn[k];
-    if constexpr (!PAIR) T[k][0] = Tn[k];
-    ValuePick pick[kTerms];
-#pragma unroll
-    for (uint32_t i = 0; i < 4u; ++i) unpack_part(std::integral_constant<uint32_t, 0>{}, 4u * k + i, pick, w);
-  }
+  begin(0, found == 2u, std::true_type{});
 #pragma unroll
   for (int k = 0; k < RF; ++k)
 #pragma unroll
@@ -1002,13 +1024,12 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) sum[k][c][e] = 0.;
   }
-  auto steps = [&](auto left_t) __attribute__((always_inline)) {
-    uint32_t buffer = 0, next = kBuf, last = 3u * kBuf, s = s0;
-    bool decode = false;
+  uint32_t buffer = 0, next = kBuf, last = 3u * kBuf, s = s0;
+  auto steps_to = [&](uint32_t end, auto left_t) __attribute__((always_inline)) {
     do {  // (a split has at least one step)
-      round(buffer, next, last, s, std::integral_constant<uint32_t, 0>{}, left_t, decode);
-      round(buffer, next, last, s, std::integral_constant<uint32_t, 1>{}, left_t, decode);
-      round(buffer, next, last, s, std::integral_constant<uint32_t, 2>{}, left_t, decode);
+      round(buffer, next, last, s, std::integral_constant<uint32_t, 0>{}, left_t, found);
+      round(buffer, next, last, s, std::integral_constant<uint32_t, 1>{}, left_t, found);
+      round(buffer, next, last, s, std::integral_constant<uint32_t, 2>{}, left_t, found);
       last = buffer;
       buffer = next;
       next = next + kBuf == kWideDepth * kBuf ? 0u : next + kBuf;
@@ -1023,12 +1044,26 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
             }
           }
       }
-    } while (++s < s1);
+    } while (++s < end);
   };
-  // (Two loops: what the rare one needs costs the other 2 % where they are one.  With PAIR two would not fit the registers.)
-  if constexpr (PAIR) steps(some_left);
-  else if (some_left) steps(std::true_type{});
-  else steps(std::false_type{});
+  // (What the rare steps need costs the others 2 to 3 % where it stands in the same loop.  A second loop with PAIR would not fit the
+  // registers, 36 too many: there the loop ends in front of such a step and begins again with it.  12288 x 4099 at 500 rows 199 -> 194 us,
+  // 13000 x 5121 at 600 rows 259 -> 252; two loops without PAIR are as fast as that and need half the time for a rare step.)
+  if constexpr (PAIR) {
+    for (;;) {
+      uint32_t end = any_left ? s + 1u : s1;
+      while (end < s1 && !some_left(end)) ++end;
+      steps_to(end, std::false_type{});
+      if (s == s1) break;
+      read_codes(s, buffer);
+      found = place_left(s, buffer);
+      if (found) begin(buffer, found == 2u, std::false_type{});
+    }
+  } else if (__builtin_expect(!any_left, 1)) {
+    steps_to(s1, std::false_type{});
+  } else {
+    steps_to(s1, std::true_type{});
+  }
   if constexpr (PAIR) {
 #pragma unroll
     for (int k = 0; k < RF; ++k)
