@@ -29,6 +29,7 @@
 #pragma once
 
 #include "block_code.h"
+#include "escape_list.h"
 #include "step_sums.h"
 
 namespace llvq {
@@ -36,7 +37,6 @@ namespace llvq {
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
-constexpr uint32_t kTileRows = 16;
 constexpr uint32_t kUnitBytes = 640;
 constexpr uint32_t kTileTableBytes = kScaleSlots * 4;
 
@@ -44,16 +44,6 @@ constexpr uint32_t kTileTableBytes = kScaleSlots * 4;
 __host__ __device__ inline uint32_t tail_depth(uint32_t tail_w) { return (tail_w + 3u) >> 2; }
 __host__ __device__ inline uint32_t tile_head_bytes(uint32_t tail_w) { return 128u + 256u * tail_depth(tail_w); }
 __host__ __device__ inline uint32_t tile_units(uint32_t nb) { return (nb + 3u) >> 2; }
-// Places in a tile's list, a multiple of eight: of uniformly drawn points of shells 2..12 0.08 % are escapes (with shell 13
-// 0.4 %), so as many as a tile has of them on average and four deviations more.  (Shell 13 takes no batched products, whose
-// kernels have room for 32.)
-constexpr uint32_t kMaxListSlots = 32, kMaxListSlots13 = 64;
-__host__ inline uint32_t list_slots(uint32_t nb, bool shell13) {
-  if (nb == 0) return 0u;
-  const double mean = kTileRows * (double)nb * (shell13 ? 4.1e-3 : 0.85e-3), want = mean + 4. * std::sqrt(mean) + 8.;
-  const uint32_t most = shell13 ? kMaxListSlots13 : kMaxListSlots;
-  return want < most ? (uint32_t)want / 8u * 8u : most;
-}
 // bytes of one tile of sixteen rows, a multiple of 128
 __host__ __device__ inline uint32_t tile_stride(uint32_t nb, uint32_t tail_w, uint32_t slots) {
   return tile_head_bytes(tail_w) + tile_units(nb) * kUnitBytes + slots * 16u;
@@ -129,8 +119,9 @@ __global__ __launch_bounds__(512) void transcode_kernel(GlobalTables g, const ui
   }
 }
 
-// The lists in order, behind transcode_kernel, whose lanes put an escape wherever there was room: a wavefront per tile, a
-// lane per escape, which goes where as many lie before it.
+// The lists in order, behind transcode_kernel, whose lanes put an escape wherever there was room: a wavefront per tile, two
+// escapes a lane, which go where as many lie before them.
+static_assert(kMaxListSlots13 <= 128 && kMaxListSlots <= kMaxListSlots13, "two places of a list to a lane");
 __global__ __launch_bounds__(256) void sort_lists_kernel(uint8_t* __restrict__ tiles, uint32_t n_tiles, uint32_t stride, uint32_t slots) {
   const uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
   if (tile >= n_tiles) return;
@@ -141,11 +132,21 @@ __global__ __launch_bounds__(256) void sort_lists_kernel(uint8_t* __restrict__ t
     if (lane == 0) list[0].w = 0xFFFFFFFFu;  // for those who read the list alone
     return;
   }
-  const uint4 mine = list[min(lane, slots - 1u)];
-  uint32_t before = 0;
-  for (uint32_t e = 0; e < count; ++e) before += (uint32_t)__shfl((int)mine.w, (int)e) < mine.w ? 1u : 0u;
-  if (lane < count) list[before] = mine;
-  else if (lane < slots) list[lane] = make_uint4(0, 0, 0, 0);
+  uint4 mine[2];
+  uint32_t before[2] = {0, 0};
+#pragma unroll
+  for (uint32_t i = 0; i < 2; ++i) mine[i] = list[min(i * 64u + lane, slots - 1u)];
+  for (uint32_t e = 0; e < count; ++e) {
+    const uint32_t key = (uint32_t)__shfl((int)(e < 64u ? mine[0].w : mine[1].w), (int)(e & 63u));
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) before[i] += key < mine[i].w ? 1u : 0u;
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < 2; ++i) {
+    const uint32_t at = i * 64u + lane;
+    if (at < count) list[before[i]] = mine[i];
+    else if (at < slots) list[at] = make_uint4(0, 0, 0, 0);
+  }
 }
 
 // Row scales, the escapes' counters (zero) and tail columns into the tiles' heads (zeros for rows past the last and columns that are not there), the
@@ -800,13 +801,7 @@ __device__ __forceinline__ float tile_extras(const TileExtras& X, const uint8_t*
   const uint32_t count = (uint32_t)__builtin_amdgcn_readfirstlane((int)X.count);
   if (count == 0u) return t;
   float sum = 0.f;
-  auto add = [&](const uint32_t (&w)[3], uint32_t key, uint32_t n) {  // the escapes of lanes 0 .. n - 1
-    const uint32_t blk = (key >> 9) & 0x7FFFFu;
-    int x[3 * DIG];
-    load_planes<DIG>(L.planes + plane_at<DIG>(blk), x);
-    const u32x2_t ss = *reinterpret_cast<const u32x2_t*>(L.planes + plane_sum_at<DIG>(blk));
-    const int v = (digits_sum<DIG>(w, x, 0) << 1) + ((key >> 8) & 1u ? (int)ss.x : 0);
-    const float f = (float)v * (scale_at((key & 31u) << 3, table) * __uint_as_float(ss.y));
+  auto to_rows = [&](float f, uint32_t key, uint32_t n) {  // those of lanes 0 .. n - 1
     for (uint32_t e = 0; e < n; ++e) {
       const uint32_t row = (uint32_t)__builtin_amdgcn_readlane((int)key, (int)e) >> 28;
       const float p = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), (int)e));
@@ -814,21 +809,50 @@ __device__ __forceinline__ float tile_extras(const TileExtras& X, const uint8_t*
     }
   };
   if (count <= slots) {
-    const bool mine = lane < count;  // (the others: any block that is there)
-    add({X.escape.x, X.escape.y, X.escape.z}, mine ? X.escape.w : 0u, count);
-  } else {  // more than there was room for: the tile's blocks one row after the other, 64 at a time
+    u32x4_t e = X.escape;
 #pragma unroll 1
-    for (uint32_t r = 0; r < kTileRows; ++r)
+    for (uint32_t first = 0; first < count; first += 64u) {
+      if (first) e = *reinterpret_cast<const u32x4_t*>(rec + list_at(nb, tail_w) + min(first + lane, slots - 1u) * 16u);
+      const uint32_t key = first + lane < count ? e.w : 0u, blk = (key >> 9) & 0x7FFFFu, w[3] = {e.x, e.y, e.z};  // (the others: any block that is there)
+      int x[3 * DIG];
+      load_planes<DIG>(L.planes + plane_at<DIG>(blk), x);
+      const u32x2_t ss = *reinterpret_cast<const u32x2_t*>(L.planes + plane_sum_at<DIG>(blk));
+      const int v = (digits_sum<DIG>(w, x, 0) << 1) + ((key >> 8) & 1u ? (int)ss.x : 0);
+      to_rows((float)v * (scale_at((key & 31u) << 3, table) * __uint_as_float(ss.y)), key, min(count - first, 64u));
+    }
+  } else {
+    // More than there was room for: the tile's meta dwords, kWalkSteps steps of them at a time, and of the escapes they show one to a lane.
+    // (Every block of one row after the other, a load to wait for each 64, took 25 us in a launch of 6.5.)
+    const uint32_t steps = tile_steps(nb), units = tile_units(nb), head = tile_head_bytes(tail_w);
 #pragma unroll 1
-      for (uint32_t b0 = 0; b0 < nb; b0 += 64u) {
-        const uint32_t blk = min(b0 + lane, nb - 1u), k = blk & 3u;
-        const uint8_t* unit = rec + tile_head_bytes(tail_w) + (blk >> 2) * kUnitBytes + (r & 7u) * 16u;
+    for (uint32_t s0 = 0; s0 < steps; s0 += kWalkSteps) {
+      uint32_t lo[kWalkSteps], hi[kWalkSteps];
+#pragma unroll
+      for (uint32_t i = 0; i < kWalkSteps; ++i) {
+        const uint8_t* piece = rec + step_offset(s0 + i, units, head, lane) + 512u;
+        lo[i] = reinterpret_cast<const uint32_t*>(piece)[1];
+        hi[i] = reinterpret_cast<const uint32_t*>(piece)[3];
+      }
+#pragma unroll
+      for (uint32_t i = 0; i < kWalkSteps; ++i) lo[i] = (s0 + i) * kStepUnits + (lane >> 3) < units ? walk_mask(lo[i], hi[i]) : 0u;
+      uint32_t n;
+      do {
+        uint32_t key = 0;  // (the lanes without one: any block that is there)
+        n = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kWalkSteps; ++i)
+          for (uint64_t left; n < 64u && (left = __builtin_amdgcn_ballot_w64(lo[i] != 0u)) != 0u; ++n) {
+            const uint32_t of = (uint32_t)__builtin_ctzll(left), mask = (uint32_t)__builtin_amdgcn_readlane((int)lo[i], of);
+            key = lane == n ? walk_key(s0 + i, of, (uint32_t)__builtin_ctz(mask)) : key;
+            lo[i] = lane == of ? mask & (mask - 1u) : lo[i];
+          }
+        const uint32_t blk = key & 0xFFFFFFFu, r = key >> 28, k = blk & 3u;
+        const uint8_t* unit = rec + head + (blk >> 2) * kUnitBytes + (r & 7u) * 16u;
         const u32x2_t d = *reinterpret_cast<const u32x2_t*>(unit + ((r >> 3) * 2u + (k >> 1)) * 128u + (k & 1u) * 8u);
         const u32x2_t sm = *reinterpret_cast<const u32x2_t*>(unit + 512u + (r >> 3) * 8u);
-        const uint32_t meta = (sm.y >> (8u * k)) & 255u;
         uint32_t w[3];
         block_octets(d.x, d.y, sm.x << (3u - k), w);
-        const BlockEscape e = block_escape(w, meta);
+        const BlockEscape e = block_escape(w, (sm.y >> (8u * k)) & 255u);
         w[0] = e.w0;
         int x[3 * DIG];
         load_planes<DIG>(L.planes + plane_at<DIG>(blk), x);
@@ -836,13 +860,9 @@ __device__ __forceinline__ float tile_extras(const TileExtras& X, const uint8_t*
         const uint32_t bit = 1u << (4u * (e.at & 7u));  // the coordinate that is 16 below, by itself
         const uint32_t one[3] = {e.at < 8u ? bit : 0u, (e.at >> 3) == 1u ? bit : 0u, (e.at >> 3) == 2u ? bit : 0u};
         const int v = digits_sum<DIG>(w, x, ((int)e.win - 3) * (int)ss.x) - (digits_sum<DIG>(one, x, 0) << 4);
-        const float f = (float)(e.negative ? -v : v) * (scale_at(e.slot << 3, table) * __uint_as_float(ss.y));
-        const bool mine = meta >= kBlockEscape && b0 + lane < nb;
-        for (uint64_t left = __builtin_amdgcn_ballot_w64(mine); left; left &= left - 1u) {
-          const float p = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), __builtin_ctzll(left)));
-          sum += lane_row(lane) == r ? p : 0.f;
-        }
-      }
+        to_rows((float)(e.negative ? -v : v) * (scale_at(e.slot << 3, table) * __uint_as_float(ss.y)), key, n);
+      } while (n == 64u);
+    }
   }
   return fmaf(sum, X.scale, t);
 }

@@ -83,3 +83,64 @@ def test_one_escape_in_a_hundred_blocks_does_not_double_the_time(gpu_rt, orc):
     usual, many = time(0.0), time(0.01)
     print(f"OBSERVED {usual * 100:.1f} us, {many * 100:.1f} us with one escape in a hundred blocks")
     assert many < 1.95 * usual
+
+
+@pytest.mark.parametrize("extra", [25, 60])
+def test_lists_of_more_than_a_lane_each(gpu_rt, orc, extra):
+    """The widest rows of shells up to 13: 88 places, in which 25 escapes a tile besides the 50 by chance are more than 64; 60 are too many
+    for some tiles and not for others."""
+    import torch
+
+    nb, tail, d_out = 1000, 8, 36
+    raw = synth.make_matrix("model.layers.0.lists13.weight", d_out, nb * 24 + tail, seed=extra, shell_cap=13)
+    rng = np.random.default_rng(extra)
+    idx, gains = raw.unpack()
+    idx = np.array(idx, np.uint64)
+    at = rng.random(idx.size) < extra / (16 * nb)
+    idx[at] = rng.choice(_far(orc, 13), int(at.sum()))
+    raw = artifact.RawMatrix(raw.name, d_out, raw.d_in, 13, raw.centroids, raw.row_scales, raw.tail, artifact.pack_codes(idx, gains, artifact.index_bits(13)))
+    X = synth.make_activation(raw.d_in, seed=1, rows=1)
+    Y_ref, A_ref = _reference(orc, raw, X)
+    proj = gpu_rt.upload(raw)
+    try:
+        x = _x16(X)[0]
+        y = gpu_rt.forward(proj, x, out_dtype=torch.float32).reshape(-1)
+        seq = gpu_rt.plan_sequence([([proj], x, False)], out_dtype=torch.float32)
+        seq.run()
+        seq.status()
+        assert torch.equal(y, seq.outputs[0][0].reshape(-1))
+        seq.close()
+    finally:
+        gpu_rt.free(proj)
+    assert np.max(np.abs(y.double().cpu().numpy() - Y_ref[0]) / A_ref[0]) < 1e-5
+
+
+def test_a_list_that_overflows_does_not_double_a_batch1_launch(gpu_rt, orc):
+    """One tile of a 9728 x 2560 product with twenty escapes, where its list has eight places: the launch of 6.5 us took 30 when each row of
+    the tile was walked 64 blocks at a time."""
+    import torch
+
+    raw = synth.make_matrix("model.layers.0.lists1.weight", 9728, 2560, seed=3)
+    idx, gains = raw.unpack()
+    idx = np.array(idx, np.uint64)
+    idx[106 * np.arange(20) % (16 * 106) + np.arange(20)] = _far(orc, 12)[:20]  # (rows 0 to 15, each a block or two)
+    many = artifact.RawMatrix(raw.name, 9728, 2560, 12, raw.centroids, raw.row_scales, raw.tail, artifact.pack_codes(idx, gains, artifact.index_bits(12)))
+    x = torch.randn(2560, device="cuda").half()
+    projs = [gpu_rt.upload(m) for m in (raw, many)]
+    took = [[], []]
+    try:
+        for _ in range(8):
+            for (launch, _), t in zip([gpu_rt.plan_group([proj], x) for proj in projs], took):
+                begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                begin.record()
+                for _ in range(100):
+                    launch()
+                end.record()
+                torch.cuda.synchronize()
+                t.append(begin.elapsed_time(end))
+    finally:
+        for proj in projs:
+            gpu_rt.free(proj)
+    usual, one = (sorted(t)[3] for t in took)
+    print(f"OBSERVED {usual * 10:.2f} us, {one * 10:.2f} us with a list that overflows")
+    assert one < 1.8 * usual
