@@ -9,8 +9,6 @@
 
 namespace llvq {
 
-constexpr uint32_t kTileRows = 16;
-
 // Of uniformly drawn points of shells 2..12 0.078 % are escapes, of shells 2..13 0.316 % (2 M draws of each).
 constexpr double kEscapeShare = 0.78e-3, kEscapeShare13 = 3.16e-3;
 // Places, a multiple of eight: as many as a tile of such points has but for one in 30 000, whose codes are read.  (At 2560 columns

@@ -1,5 +1,5 @@
-// Where the sums of a tile's steps lie in LDS between the wavefronts that leave them there and the one that adds them up
-// (gemv_tiles_kernel): plain integer arithmetic, compiled for gfx950 and for the host.
+// What a batch-1 product keeps in LDS (gemv_tiles_kernel): the activation's planes, and the sums of a tile's steps between the
+// wavefronts that leave them there and the one that adds them up.  Plain integer arithmetic, compiled for gfx950 and for the host.
 #pragma once
 #include <cstdint>
 
@@ -7,6 +7,7 @@
 
 namespace llvq {
 
+constexpr uint32_t kTileRows = 16;
 constexpr uint32_t kStepUnits = 8;
 constexpr uint32_t kStepBlocks = 4 * kStepUnits;
 LLVQ_HD uint32_t tile_steps(uint32_t nb) { return (nb + kStepBlocks - 1u) / kStepBlocks; }
@@ -34,6 +35,23 @@ LLVQ_HD uint32_t sums_at(uint32_t round, uint32_t team_index, uint32_t team, boo
 LLVQ_HD uint32_t sums_read(uint32_t i, uint32_t c, uint32_t steps) {
   const uint32_t s = 4u * i + c, last = steps ? steps - 1u : 0u;
   return s < last ? s : last;
+}
+
+// In LDS the four blocks of a unit lie together: 3 dwords per digit and block, then each block's sum of its integers
+// (v = 2 n + b: sum v x = 2 sum n x + b sum x) and scale.  The pad spreads the eight units of a step over the banks.
+template <int DIG> struct XPlanes {
+  static constexpr uint32_t kBlock = 3 * DIG, kSums = 4 * kBlock, kDwords = kSums + 8 + (DIG == 6 ? 4 : 0);
+};
+// Units of the planes in LDS: whole steps, and a step of zeros behind them for the wavefronts whose steps end early.
+LLVQ_HD uint32_t gemv_plane_units(uint32_t nb) { return (tile_steps(nb) + 1u) * kStepUnits; }
+
+LLVQ_HD uint32_t gemv_lds_fixed() { return 128u + 64u; }
+// The rotated activation and the sums share their place: rows of 20480 columns with f32 results, 24576 with binary16, are the widest that
+// fit (160 KB).  One behind the other, 19456 and 20480 columns with f32 results and 23552 with binary16 took a launch more, 3.6 to 4 us.
+inline uint64_t gemv_tiles_lds_bytes(uint32_t nb, uint32_t d_in, bool f32_out, bool rotated) {
+  const uint64_t planes = (uint64_t)gemv_plane_units(nb) * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
+  const uint64_t sums = kGemvRounds * sums_steps(gemv_wide(nb)) * kTileRows * 4, values = rotated ? ((uint64_t)d_in * 4 + 31) / 16 * 16 : 0;
+  return gemv_lds_fixed() + planes + (sums > values ? sums : values);
 }
 
 }  // namespace llvq

@@ -186,11 +186,6 @@ __device__ __forceinline__ T* uniform_global(T* p) {
 // largest, a sixteenth of the half ulp such a result carries anyway), six for f32 results (2^22: every binary16 value
 // within 2^12 of its block's largest is exact).  An 8-wide 4-bit dot product then takes one digit of eight columns
 // against a dword of weights, exactly.
-// In LDS the four blocks of a unit lie together: 3 dwords per digit and block, then each block's sum of its integers
-// (v = 2 n + b: sum v x = 2 sum n x + b sum x) and scale.  The pad spreads the eight units of a step over the banks.
-template <int DIG> struct XPlanes {
-  static constexpr uint32_t kBlock = 3 * DIG, kSums = 4 * kBlock, kDwords = kSums + 8 + (DIG == 6 ? 4 : 0);
-};
 template <int DIG>
 __device__ __forceinline__ uint32_t plane_at(uint32_t blk) { return (blk >> 2) * XPlanes<DIG>::kDwords + (blk & 3u) * XPlanes<DIG>::kBlock; }
 template <int DIG>
@@ -271,9 +266,6 @@ __device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub
 }
 
 // ---- batch-1 product ------------------------------------------------------------------------------
-// Units of the planes in LDS: whole steps, and a step of zeros behind them for the wavefronts whose steps end early.
-__host__ __device__ inline uint32_t gemv_plane_units(uint32_t nb) { return (tile_steps(nb) + 1u) * kStepUnits; }
-
 // What a launch's activation is made from.
 enum : int { kSrcF16 = 0, kSrcRotated = 1, kSrcSiluMul = 2, kSrcAddRmsNorm = 3 };
 
@@ -296,23 +288,16 @@ struct GemvLds {
   float* red;        // [16]
   uint32_t* planes;  // [plane units][XPlanes::kDwords]
   float* part;       // [kGemvRounds][sums_steps][16 rows]
-  float* xf;         // [d_in] f32 values of a rotated activation
+  float* xf;         // [d_in] f32 values of a rotated activation, in the same place: they are in the planes before there are sums
 };
-__host__ __device__ inline uint32_t gemv_lds_fixed() { return 128u + 64u; }
-__host__ __device__ inline size_t gemv_tiles_lds_bytes(uint32_t nb, uint32_t d_in, bool f32_out, bool rotated) {
-  const size_t planes = (size_t)gemv_plane_units(nb) * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
-  const size_t sums = kGemvRounds * kGemvMaxWaves * kTileRows * 4;
-  return gemv_lds_fixed() + planes + (gemv_wide(nb) ? kGemvWideSteps : 1u) * sums + (rotated ? ((size_t)d_in * 4 + 31) / 16 * 16 : 0);
-}
-template <int DIG, bool WIDE>
+template <int DIG>
 __device__ __forceinline__ GemvLds gemv_lds(uint8_t* smem, uint32_t plane_units) {
-  constexpr uint32_t kSums = kGemvRounds * kGemvMaxWaves * kTileRows;
   GemvLds L;
   L.xtail = reinterpret_cast<float*>(smem);
   L.red = L.xtail + 32;
   L.planes = reinterpret_cast<uint32_t*>(L.red + 16);
   L.part = reinterpret_cast<float*>(L.planes + (size_t)plane_units * XPlanes<DIG>::kDwords);
-  L.xf = L.part + kSums * (WIDE ? kGemvWideSteps : 1u);
+  L.xf = L.part;
   return L;
 }
 
@@ -918,7 +903,7 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
   constexpr int DIG = std::is_same<OutT, __half>::value ? 4 : 6;
   constexpr uint32_t kSteps = WIDE ? kGemvWideSteps : 1u;
   extern __shared__ __align__(16) uint8_t smem[];
-  const GemvLds L = gemv_lds<DIG, WIDE>(smem, gemv_plane_units(a.nb));
+  const GemvLds L = gemv_lds<DIG>(smem, gemv_plane_units(a.nb));
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), waves = blockDim.x >> 6;
   const uint32_t team = wave / a.team, w = wave - team * a.team, n_teams = a.teams * gridDim.x;

@@ -1,4 +1,4 @@
-// Every place of LDS that the batch-1 product's sums over a tile's steps are read from (step_sums.h), for every row length, round
+// What a batch-1 product keeps in LDS (step_sums.h): how wide a row may be, and every place that the batch-1 product's sums over a tile's steps are read from, for every row length, round
 // and team of a workgroup: one that the tile's own wavefronts wrote.  Prints the first that is not and returns 1.
 #include "step_sums.h"
 
@@ -21,5 +21,13 @@ int main() {
             }
           }
   }
+  // The rotated rows that are rotated in their product's launch, which has 160 KB: of the widths a rotation can have these are the widest.
+  const struct { uint32_t width; bool f32, fits; } rotated[] = {{19456, true, true},  {20480, true, true},  {21504, true, false},
+                                                                {23552, false, true}, {24576, false, true}, {17408, true, true}};
+  for (const auto& r : rotated)
+    if ((gemv_tiles_lds_bytes(r.width / kDim, r.width, r.f32, true) <= 160u * 1024u) != r.fits) {
+      std::printf("%u columns rotated: %u bytes\n", r.width, (unsigned)gemv_tiles_lds_bytes(r.width / kDim, r.width, r.f32, true));
+      return 1;
+    }
   return 0;
 }

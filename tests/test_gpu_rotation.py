@@ -158,9 +158,9 @@ def test_a_power_of_two_goes_through_a_rotated_product_unchanged(gpu_rt, k, d_in
 
 
 def test_rows_too_wide_to_be_rotated_in_the_launch(gpu_rt, orc):
-    """20 480 columns with f32 results and 24 576 with either do not fit LDS beside their digit planes: the activation is
-    rotated by a kernel of its own, into memory that belongs to the rotation.  An upload between two products (which
-    brings another such rotation) changes nothing about the first."""
+    """24 576 columns with f32 results do not fit LDS beside their digit planes: the activation is rotated by a kernel of its own,
+    into memory that belongs to the rotation.  An upload between two products (which brings another such rotation) changes
+    nothing about the first, nor about rows that are rotated in their launch."""
     import torch
 
     first = _rotated("model.layers.0.wide.0.weight", 9, 20480, 3, 41)
@@ -181,6 +181,34 @@ def test_rows_too_wide_to_be_rotated_in_the_launch(gpu_rt, orc):
     finally:
         for p in projs:
             gpu_rt.free(p)
+
+
+# The widest rows that are rotated in their product's launch (f32 up to 20480, binary16 up to 24576 columns), whose partial sums lie
+# where the rotated row was, with more tiles than a round of a launch has; and past them, between uploads of another such rotation.
+@pytest.mark.parametrize("n,out", [(19456, "f32"), (20480, "f32"), (23552, "f16"), (24576, "f16"), (24576, "f32")])
+def test_widest_rotated_rows(gpu_rt, orc, n, out):
+    import torch
+
+    d_out = 16 * 256 + 9 if n == 20480 or out == "f16" else 40
+    raw = _rotated(f"model.layers.0.widest.{n}.weight", d_out, n, 3, 51)
+    x = synth.make_activation(n, seed=n)[0]
+    proj = gpu_rt.upload(raw)
+    dt = torch.float32 if out == "f32" else torch.float16
+    try:
+        one = gpu_rt.forward(proj, _x16(x), out_dtype=dt).reshape(-1)
+        other = gpu_rt.upload(_rotated("model.layers.0.widest.other.weight", 9, n, 4, 52))
+        gpu_rt.forward(other, _x16(x), out_dtype=dt)
+        again = gpu_rt.forward(proj, _x16(x), out_dtype=dt).reshape(-1)
+        gpu_rt.free(other)
+        apart = gpu_rt.forward_rotated(proj, gpu_rt.rotate(proj, _x16(x)), out_dtype=dt).reshape(-1)
+    finally:
+        gpu_rt.free(proj)
+    assert torch.equal(one, again) and torch.equal(one, apart)
+    om, _ = orc.read_matrix_raw(artifact.write_matrix_raw(raw))
+    y_ref, a_ref = om.fused_product(x.astype(np.float64))
+    err = np.abs(one.double().cpu().numpy() - y_ref)
+    # (binary16 results: the activation to 2^-15 of its block's largest value, which is less than five times their mean, and the result's rounding)
+    assert np.all(err <= (1e-5 * a_ref if out == "f32" else 5 * 2.0 ** -15 * a_ref + 2.0 ** -11 * np.abs(y_ref)))
 
 
 # Rows that are rotated straight to the products' octets, in a call of its own, against the rotated rows of a group too large for
