@@ -9,9 +9,9 @@
 //   * Independent items: a workgroup takes one contiguous run of tiles, the runs equal in bytes, so that it meets two or
 //     three items of a model's 144 and streams the rest.  What bounds it is HBM: 10.x bytes per block, 252 matrices
 //     of a 4B model 387 -> 265 us, 5.1 -> 5.8 TB/s (13 bytes before, in lines shared between loads).  A wavefront takes
-//     up to four steps of a tile at a time (a task); a step's registers are loaded again, piece by piece, for its next
+//     up to four steps of a tile at a time (a task; two where a launch is short); a step's registers are loaded again, piece by piece, for its next
 //     step, in this task or the one after, as soon as they have been used: sixteen wavefronts x 5 KB in flight per CU.
-//     Rows of up to four steps (128 blocks) are a wavefront's own; of wider ones the sums of the steps meet in LDS, the
+//     Rows of one task are a wavefront's own; of wider ones the sums of the steps meet in LDS, the
 //     wavefront that arrives last at a tile's counter adds them up and stores, and a barrier every kSeqDrift tasks
 //     bounds how far the wavefronts drift apart.
 //   * Ordered items (`wait_item`): a step is a task, the tiles are dealt out evenly; before a workgroup reads an activation
@@ -28,8 +28,6 @@
 namespace llvq {
 
 constexpr uint32_t kSeqNoWait = 0xFFFFFFFFu;
-constexpr uint32_t kSeqWaves = 16;
-constexpr uint32_t kSeqTaskSteps = 4;  // steps of a task of independent items
 constexpr uint32_t kSeqDrift = 4;      // tasks of a wavefront between two barriers, where tiles are shared
 // Tiles whose sums may be pending between two barriers, when a tile is `tasks` >= 2 tasks: those that begin there, and one
 // that is cut at either end.

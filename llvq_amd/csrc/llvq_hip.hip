@@ -1219,6 +1219,7 @@ static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) 
   // of them; a unit is what a workgroup has of a matrix.  Ordered ones are spread over all workgroups as a launch of their
   // own would be, unit after unit: everyone waits for the slowest.
   uint32_t grid = (uint32_t)std::min<uint64_t>(n_tiles, grid_cap);
+  const uint32_t task_steps = dependent ? 1u : seq_task_steps(bytes, grid);
   std::vector<uint32_t> runs{0};
   uint64_t done = 0;
   for (int i = 0; i < n; ++i) {
@@ -1238,7 +1239,7 @@ static int seq_create(llvq_rt* rt, const SeqSpec* specs, int n, llvq_seq** out) 
     I.first_unit = (uint32_t)units.size();
     I.wait_item = sp.after_previous ? (uint32_t)(i - 1) : kSeqNoWait;
     I.signals = (i + 1 < n && specs[i + 1].after_previous) ? 1u : 0u;
-    I.tasks = std::max(1u, dependent ? steps : (steps + kSeqTaskSteps - 1u) / kSeqTaskSteps);
+    I.tasks = seq_tasks(steps, task_steps);
     I.inv_tasks = I.tasks > 1u ? (uint32_t)(((1ull << 32) + I.tasks - 1u) / I.tasks) : 0u;
     const size_t ysz = f32 ? 4 : 2;
     for (int j = 0; j < sp.n; ++j) {

@@ -8,6 +8,7 @@
 namespace llvq {
 
 constexpr uint32_t kTileRows = 16;
+constexpr uint32_t kUnitBytes = 640;
 constexpr uint32_t kStepUnits = 8;
 constexpr uint32_t kStepBlocks = 4 * kStepUnits;
 LLVQ_HD uint32_t tile_steps(uint32_t nb) { return (nb + kStepBlocks - 1u) / kStepBlocks; }
@@ -53,5 +54,17 @@ inline uint64_t gemv_tiles_lds_bytes(uint32_t nb, uint32_t d_in, bool f32_out, b
   const uint64_t sums = kGemvRounds * sums_steps(gemv_wide(nb)) * kTileRows * 4, values = rotated ? ((uint64_t)d_in * 4 + 31) / 16 * 16 : 0;
   return gemv_lds_fixed() + planes + (sums > values ? sums : values);
 }
+
+// ---- lists of products as one launch (gemv_seq.h) ----
+constexpr uint32_t kSeqWaves = 16;
+// Steps of a task of independent items, `bytes` of tiles on `grid` workgroups.  Two where a wavefront has sixteen steps or fewer: with few
+// tiles to a workgroup tasks of four leave wavefronts without one, and with many the sums through LDS cost more than that.  One layer of a 4B
+// model (2 steps a wavefront) 17.1 us with four, 14.8 with two, 14.6 with one; four layers (9) 38.1, 37.4, 38.0; six (13) 51.7, 50.2,
+// 52.0; twelve (26) 91.2, 93.2, 97.4.
+constexpr uint32_t kSeqTaskSteps = 4, kSeqShortTaskSteps = 2, kSeqShortSteps = 16;
+LLVQ_HD uint32_t seq_task_steps(uint64_t bytes, uint32_t grid) {
+  return bytes > (uint64_t)kSeqShortSteps * kSeqWaves * kStepUnits * kUnitBytes * grid ? kSeqTaskSteps : kSeqShortTaskSteps;
+}
+LLVQ_HD uint32_t seq_tasks(uint32_t steps, uint32_t task_steps) { return steps ? (steps + task_steps - 1u) / task_steps : 1u; }
 
 }  // namespace llvq

@@ -37,7 +37,6 @@ namespace llvq {
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
-constexpr uint32_t kUnitBytes = 640;
 constexpr uint32_t kTileTableBytes = kScaleSlots * 4;
 
 // Floats of a row's tail columns that a lane of its four holds: column c is the (c / 4)-th of lane class c % 4.

@@ -1,5 +1,6 @@
-// What a batch-1 product keeps in LDS (step_sums.h): how wide a row may be, and every place that the batch-1 product's sums over a tile's steps are read from, for every row length, round
-// and team of a workgroup: one that the tile's own wavefronts wrote.  Prints the first that is not and returns 1.
+// What a batch-1 product keeps in LDS (step_sums.h): how wide a row may be, and every place that its sums over a tile's steps are read
+// from, for every row length, round and team of a workgroup: one that the tile's own wavefronts wrote.  And how a list of products is
+// shared out.  Prints the first that is not so and returns 1.
 #include "step_sums.h"
 
 #include <cstdio>
@@ -29,5 +30,18 @@ int main() {
       std::printf("%u columns rotated: %u bytes\n", r.width, (unsigned)gemv_tiles_lds_bytes(r.width / kDim, r.width, r.f32, true));
       return 1;
     }
+  // A layer of a 4B model as one launch of 256 workgroups: each has tasks for its wavefronts (but for two), whichever matrix its share is of.
+  const struct { uint32_t rows, width; } layer[] = {{6144, 2560}, {2560, 4096}, {19456, 2560}, {2560, 9728}};
+  uint64_t bytes = 0;
+  for (const auto& m : layer) bytes += (uint64_t)m.rows / 16 * ((m.width / kDim + 3) / 4) * kUnitBytes;
+  for (const auto& m : layer) {
+    const uint64_t tiles = bytes / 256 / ((uint64_t)(m.width / kDim + 3) / 4 * kUnitBytes);
+    const uint32_t tasks = seq_tasks(tile_steps(m.width / kDim), seq_task_steps(bytes, 256));
+    if (tiles * tasks < kSeqWaves - 2) {
+      std::printf("%u columns: %u tasks of a workgroup\n", m.width, (unsigned)tiles * tasks);
+      return 1;
+    }
+  }
+  if (seq_task_steps(36 * bytes, 256) != kSeqTaskSteps) return 1;
   return 0;
 }

@@ -188,3 +188,23 @@ def test_sequence_refusals(gpu_rt):
     finally:
         for q in (p, pr, po):
             gpu_rt.free(q)
+
+
+def test_long_lists_and_short_ones_give_the_same_bits(gpu_rt):
+    """Lists of more than 335 MB of tiles share them out in tasks of four steps (128 blocks), shorter ones in tasks of two: widths of one to
+    thirteen steps, each matrix many times over."""
+    shapes = [(6000, 24 * 30), (6000, 24 * 60 + 7), (6000, 24 * 90), (6000, 24 * 128), (6000, 24 * 160 + 1), (3000, 9728)]
+    projs = [gpu_rt.upload(synth.make_matrix(f"model.layers.{i}.long.weight", do, di, i)) for i, (do, di) in enumerate(shapes)]
+    try:
+        xs = [_x16(synth.make_activation(di, seed=di)[0]) for _, di in shapes]
+        want = [gpu_rt.forward(p, x) for p, x in zip(projs, xs)]
+        for times in (1, 14):
+            seq = gpu_rt.plan_sequence([([p], x, False) for p, x in zip(projs, xs)] * times)
+            seq.run()
+            seq.status()
+            for i, ys in enumerate(seq.outputs):
+                assert _same_bits(ys[0].reshape(-1), want[i % len(projs)].reshape(-1)), (times, i)
+            seq.close()
+    finally:
+        for p in projs:
+            gpu_rt.free(p)

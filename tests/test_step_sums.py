@@ -1,4 +1,5 @@
-"""The batch-1 product's sums over a tile's steps stay in their place in LDS: tests/step_sums.cpp walks every row length, round and team."""
+"""The batch-1 product's sums over a tile's steps stay in their place in LDS, and its work is shared out over all wavefronts:
+tests/step_sums.cpp walks every row length, round and team."""
 import os
 import shutil
 import subprocess
