@@ -93,7 +93,10 @@ int main(int argc, char** argv) {
   auto rank = [&](uint64_t idx) {
     int8_t p[24];
     int shell = 0;
-    if (!host_decode(idx, p, &shell)) return;
+    if (!host_decode(idx, p, &shell)) {
+      std::fprintf(stderr, "rank %llu has no point\n", (unsigned long long)idx);
+      std::exit(1);
+    }
     for (int i = 0; i < 24; ++i) v[i] = p[i];
     for (uint32_t gain = 0; gain < 2; ++gain)
       if (!round_trip(v, gain, (uint32_t)shell)) fail(v, "rank");
@@ -104,6 +107,10 @@ int main(int argc, char** argv) {
   for (int i = 0; i < 400000; ++i) {
     z ^= z << 13; z ^= z >> 7; z ^= z << 17;
     rank(z % (kN13 + 1));
+  }
+  if (shapes == 0 || seen == 0 || escapes == 0 || ranks != 400000 + (size_t)(argc - 1)) {
+    std::fprintf(stderr, "%zu shapes, %zu of them escapes; %zu ranks, %zu escapes\n", shapes, seen / 4, ranks, escapes / 2);
+    return 1;
   }
   std::printf("ok: %zu shapes, %zu of them escapes; %zu ranks, %zu escapes\n", shapes, seen / 4, ranks, escapes / 2);
   return 0;
