@@ -62,9 +62,9 @@ def test_the_batched_kernel_does_not_spill_either(usage):
 
 def test_the_wide_batched_kernel_keeps_its_workgroups_on_a_cu(usage):
     """Four wavefronts to a workgroup, one on each SIMD: two workgroups share a CU's 512 registers a lane where a tile has
-    128 activation rows, one has them for itself at 256 rows or with both terms of the weights."""
-    wide = {k: v for k, v in usage.items() if "gemm_wide_kernel" in k}
-    bound = {"ILi4ELb0E": 256, "ILi4ELb1E": 512, "ILi8ELb0E": 512}
+    128 activation rows, one has them for itself at 256 rows, with tiles of 384 weight rows or with both terms of the weights."""
+    wide = {k: v for k, v in usage.items() if "gemm_wide_kernel" in k or "gemm_tall_kernel" in k}
+    bound = {"ILi4ELb0E": 256, "ILi4ELb1E": 512, "ILi8ELb0E": 512, "gemm_tall_kernel": 512}
     assert len(wide) == len(bound)
     for name, u in wide.items():
         limit = next(v for k, v in bound.items() if k in name)
