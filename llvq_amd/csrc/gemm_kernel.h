@@ -1083,7 +1083,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
   // (From the lane's number anew: nothing of this may occupy registers during the loop.)
   const uint32_t lane_e = lane_offset(lane), l32e = lane_e & 31u, he = lane_e >> 5;
   const uint32_t m0 = mt * kCols + l32e;
-  if (a.splits > 1u) {
+  if (RF == 2 && a.splits > 1u) {  // (gemm_plan splits no tiles of 384 rows)
     const uint32_t n_rows = a.n_tiles * kRows;
     float* out = a.ws + (size_t)split * a.m_pad * n_rows;
 #pragma unroll

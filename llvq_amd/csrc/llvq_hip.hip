@@ -1472,10 +1472,10 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
   // place holds the octets of either plan, and needs no partial sums for rows that hardly ever come.)
   const uint32_t steps = (nb + 1u) / 2u, most = pair && mats[0]->d_in % 8 == 0 ? 1u : 16u;
   double best = 1e30;
-  const auto weigh = [&](uint32_t rf, uint32_t cf, size_t ws_cap) {
+  const auto weigh = [&](uint32_t rf, uint32_t cf, uint32_t most) {
     const uint32_t rows = 128u * rf, n_tiles = tiles_of(rows), m_tiles = (M + 32u * cf - 1u) / (32u * cf), m_pad = m_tiles * 32u * cf;
     const size_t one = (size_t)m_pad * n_tiles * rows * sizeof(float);
-    for (uint32_t sp = 1; sp <= most && (sp == 1u || (steps / sp >= 8u && one * sp <= ws_cap)); ++sp) {
+    for (uint32_t sp = 1; sp <= most && (sp == 1u || (steps / sp >= 8u && one * sp <= kGemmWsCap)); ++sp) {
       const uint32_t per = (steps + sp - 1u) / sp, wgs = n_tiles * m_tiles * ((steps + per - 1u) / per), per_cu = (wgs + cus - 1u) / cus;
       const double step = pair ? kWidePairStep : rf == 3u ? kTallStep : cf == 8u ? kWideStep : per_cu == 1u ? kWideHalfStepAlone : kWideHalfStep;
       const double cost = per_cu * step * per + (sp > 1u ? 3.0 + 2.0 * (double)one * sp / 4e6 : 0.0);
@@ -1493,10 +1493,10 @@ static GemmPlan gemm_plan(const llvq_rt* rt, const llvq_mat* const* mats, int n,
       }
     }
   };
-  if (!pair) weigh(2u, 8u, kGemmWsCap);
-  weigh(2u, 4u, kGemmWsCap);
-  // (384 rows never with more workspace than the best of 256: where a call has to fit a given one it fits as before)
-  if (!pair) weigh(3u, 4u, p.ws_bytes);
+  if (!pair) weigh(2u, 8u, most);
+  weigh(2u, 4u, most);
+  // (384 rows are not split: of 150 000 drawn shapes none would be, and no call needs more workspace for them.)
+  if (!pair) weigh(3u, 4u, 1u);
   p.xt_bytes = (size_t)p.n_oct * p.m_pad * 16;
   return p;
 }
@@ -2313,7 +2313,7 @@ int llvq_hip_decoder_create(llvq_rt* rt, const llvq_decoder_desc* c, llvq_decode
   d->eps = (float)c->rms_eps;
   d->kv_q8 = c->kv_mode == LLVQ_KV_Q8;
   d->proj.assign(c->projections, c->projections + (size_t)c->n_layers * 7);
-  d->head_grid = kHeadGroups;
+  d->head_grid = kHeadGroups * (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
   while (d->head_grid > 1 && (uint64_t)d->head_grid * (kHeadThreads / 64) > c->vocab) d->head_grid >>= 1;
 
   // RoPE tables exactly as Rotary::new builds them (model.rs:163-179): f32 inverse
