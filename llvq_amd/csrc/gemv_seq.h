@@ -28,13 +28,6 @@
 namespace llvq {
 
 constexpr uint32_t kSeqNoWait = 0xFFFFFFFFu;
-constexpr uint32_t kSeqDrift = 4;      // tasks of a wavefront between two barriers, where tiles are shared
-// Tiles whose sums may be pending between two barriers, when a tile is `tasks` >= 2 tasks: those that begin there, and one
-// that is cut at either end.
-__host__ __device__ inline uint32_t seq_slots(uint32_t tasks) { return kSeqDrift * kSeqWaves / tasks + 2u; }
-// Sixteen rows of sums for each of their steps: at the most 4 tasks (64 / tasks + 2) with tasks <= 8.
-constexpr uint32_t kSeqPartSteps = 4 * (kSeqDrift * kSeqWaves + 2 * 8), kSeqMaxSlots = kSeqDrift * kSeqWaves / 2 + 2;
-
 struct SeqUnit {           // consecutive tiles of one matrix
   const uint8_t* rec;      // the first tile
   const uint32_t* table;   // the matrix's scales

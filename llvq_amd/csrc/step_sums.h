@@ -29,15 +29,14 @@ LLVQ_HD bool gemv_wide(uint32_t nb) { return nb > kStepBlocks * kGemvMaxWaves; }
 // ... and so that there is a wavefront for each of the workgroup's
 LLVQ_HD uint32_t gemv_batch(uint32_t team) { return team < kGemvRounds ? team : kGemvRounds; }
 
-// The array: kGemvRounds rounds of as many steps as a workgroup's teams take together.  Tile `team_index` of a round begins here.
+// The array: kGemvRounds rounds of as many steps as a workgroup's teams take together, and room behind them for what a sum reads past
+// its tile's steps and does not use: the places to read are then the same for every tile.  (Each held back by the number of steps,
+// which is twelve instructions in front of the first product, took 0.08 us of every launch.)  Tile `team_index` of a round begins here.
 LLVQ_HD uint32_t sums_steps(bool wide) { return kGemvMaxWaves * (wide ? kGemvWideSteps : 1u); }
 LLVQ_HD uint32_t sums_at(uint32_t round, uint32_t team_index, uint32_t team, bool wide) { return round * sums_steps(wide) + team_index * team; }
-// The step of a tile of `steps` that a lane of class c reads as its i-th: past the tile's last that one again (a row may have none).
-LLVQ_HD uint32_t sums_read(uint32_t i, uint32_t c, uint32_t steps) {
-  const uint32_t s = 4u * i + c, last = steps ? steps - 1u : 0u;
-  return s < last ? s : last;
-}
-
+LLVQ_HD uint32_t sums_room(bool wide) { return kGemvRounds * sums_steps(wide) + (wide ? 0u : kGemvMaxWaves); }
+// The step that a lane of class c reads as its i-th.
+LLVQ_HD uint32_t sums_read(uint32_t i, uint32_t c) { return 4u * i + c; }
 // In LDS the four blocks of a unit lie together: 3 dwords per digit and block, then each block's sum of its integers
 // (v = 2 n + b: sum v x = 2 sum n x + b sum x) and scale.  The pad spreads the eight units of a step over the banks.
 template <int DIG> struct XPlanes {
@@ -51,7 +50,7 @@ LLVQ_HD uint32_t gemv_lds_fixed() { return 128u + 64u; }
 // fit (160 KB).  One behind the other, 19456 and 20480 columns with f32 results and 23552 with binary16 took a launch more, 3.6 to 4 us.
 inline uint64_t gemv_tiles_lds_bytes(uint32_t nb, uint32_t d_in, bool f32_out, bool rotated) {
   const uint64_t planes = (uint64_t)gemv_plane_units(nb) * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
-  const uint64_t sums = kGemvRounds * sums_steps(gemv_wide(nb)) * kTileRows * 4, values = rotated ? ((uint64_t)d_in * 4 + 31) / 16 * 16 : 0;
+  const uint64_t sums = sums_room(gemv_wide(nb)) * kTileRows * 4, values = rotated ? ((uint64_t)d_in * 4 + 31) / 16 * 16 : 0;
   return gemv_lds_fixed() + planes + (sums > values ? sums : values);
 }
 
@@ -66,5 +65,12 @@ LLVQ_HD uint32_t seq_task_steps(uint64_t bytes, uint32_t grid) {
   return bytes > (uint64_t)kSeqShortSteps * kSeqWaves * kStepUnits * kUnitBytes * grid ? kSeqTaskSteps : kSeqShortTaskSteps;
 }
 LLVQ_HD uint32_t seq_tasks(uint32_t steps, uint32_t task_steps) { return steps ? (steps + task_steps - 1u) / task_steps : 1u; }
+
+constexpr uint32_t kSeqDrift = 4;      // tasks of a wavefront between two barriers, where tiles are shared
+// Tiles whose sums may be pending between two barriers, when a tile is `tasks` >= 2 tasks: those that begin there, and one
+// that is cut at either end.
+LLVQ_HD uint32_t seq_slots(uint32_t tasks) { return kSeqDrift * kSeqWaves / tasks + 2u; }
+// Sixteen rows of sums for each of their steps: at the most 4 tasks (64 / tasks + 2) with tasks <= 8.
+constexpr uint32_t kSeqPartSteps = 4 * (kSeqDrift * kSeqWaves + 2 * 8), kSeqMaxSlots = kSeqDrift * kSeqWaves / 2 + 2;
 
 }  // namespace llvq

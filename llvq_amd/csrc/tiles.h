@@ -286,7 +286,7 @@ struct GemvLds {
   float* xtail;      // [32]
   float* red;        // [16]
   uint32_t* planes;  // [plane units][XPlanes::kDwords]
-  float* part;       // [kGemvRounds][sums_steps][16 rows]
+  float* part;       // [sums_room][16 rows]
   float* xf;         // [d_in] f32 values of a rotated activation, in the same place: they are in the planes before there are sums
 };
 template <int DIG>
@@ -858,7 +858,7 @@ __device__ __forceinline__ float steps_sum(const float* part, uint32_t steps, ui
 #pragma unroll
   for (uint32_t i = 0; i < MAX / 4; ++i) {
     const uint32_t s = 4u * i + lane_class(lane);
-    v[i] = part[sums_read(i, lane_class(lane), steps) * kTileRows + lane_row(lane)];
+    v[i] = part[sums_read(i, lane_class(lane)) * kTileRows + lane_row(lane)];
     v[i] = s < steps ? v[i] : 0.f;
   }
 #pragma unroll
