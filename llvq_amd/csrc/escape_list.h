@@ -32,7 +32,6 @@ inline uint32_t list_slots(uint32_t nb, bool shell13) {
 // A tile's codes: eight units to a step and lane (l, q) = (lane % 8, lane / 8) at piece l of the step's unit q, which has four
 // blocks each of rows l and l + 8.  Their meta dwords give a mask with bit 8 k for block k of row l and bit 8 k + 1 for row l + 8;
 // taken lane after lane and bit after bit, a row's blocks come in their order.
-constexpr uint32_t kWalkSteps = 4;  // steps whose masks are read together
 LLVQ_HD uint32_t walk_mask(uint32_t meta_lo, uint32_t meta_hi) {  // (bytes of kBlockEscape = 192 or more: the two top bits)
   return (meta_lo & meta_lo << 1 & 0x80808080u) >> 7 | (meta_hi & meta_hi << 1 & 0x80808080u) >> 6;
 }

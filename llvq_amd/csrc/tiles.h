@@ -792,44 +792,48 @@ __device__ __forceinline__ float tile_extras(const TileExtras& X, const uint8_t*
       sum += lane_row(lane) == row ? p : 0.f;
     }
   };
-  if (count <= slots) {
+  if (__builtin_expect(count <= slots, 1)) {
     u32x4_t e = X.escape;
+    uint32_t first = 0;
 #pragma unroll 1
-    for (uint32_t first = 0; first < count; first += 64u) {
-      if (first) e = *reinterpret_cast<const u32x4_t*>(rec + list_at(nb, tail_w) + min(first + lane, slots - 1u) * 16u);
+    for (;;) {
       const uint32_t key = first + lane < count ? e.w : 0u, blk = (key >> 9) & 0x7FFFFu, w[3] = {e.x, e.y, e.z};  // (the others: any block that is there)
       int x[3 * DIG];
       load_planes<DIG>(L.planes + plane_at<DIG>(blk), x);
       const u32x2_t ss = *reinterpret_cast<const u32x2_t*>(L.planes + plane_sum_at<DIG>(blk));
       const int v = (digits_sum<DIG>(w, x, 0) << 1) + ((key >> 8) & 1u ? (int)ss.x : 0);
       to_rows((float)v * (scale_at((key & 31u) << 3, table) * __uint_as_float(ss.y)), key, min(count - first, 64u));
+      first += 64u;
+      if (__builtin_expect(first >= count, 1)) break;
+      asm volatile("" : "+s"(nb), "+s"(tail_w));  // (as below)
+      e = *reinterpret_cast<const u32x4_t*>(rec + list_at(nb, tail_w) + min(first + lane, slots - 1u) * 16u);
     }
   } else {
-    // More than there was room for: the tile's meta dwords, kWalkSteps steps of them at a time, and of the escapes they show one to a lane.
-    // (Every block of one row after the other, a load to wait for each 64, took 25 us in a launch of 6.5.)
+    // More than there was room for: the tile's meta dwords step by step, the next one's on their way, and of the escapes they show one to a
+    // lane; those are read 64 at a time.  A launch of 5.6 us takes 10.5 with a tile of twenty (every block of one row after the other, a load
+    // to wait for each 64: 30; four steps' dwords together, each with loops of its own: 8.3, and 3 KB more of each of these kernels, which is
+    // up to 1 % of a decoded token).
+    asm volatile("" : "+s"(nb), "+s"(tail_w), "+v"(lane));  // (what is made of them is made here, and not ahead of the launch's tiles)
     const uint32_t steps = tile_steps(nb), units = tile_units(nb), head = tile_head_bytes(tail_w);
+    auto masks = [&](uint32_t s) {
+      const uint32_t* piece = reinterpret_cast<const uint32_t*>(rec + step_offset(s, units, head, lane) + 512u);
+      return u32x2_t{piece[1], piece[3]};
+    };
+    u32x2_t next = masks(0);
+    uint32_t step = 0, mask = 0, key = 0, n = 0;  // (key: of the lanes without one any block that is there)
 #pragma unroll 1
-    for (uint32_t s0 = 0; s0 < steps; s0 += kWalkSteps) {
-      uint32_t lo[kWalkSteps], hi[kWalkSteps];
-#pragma unroll
-      for (uint32_t i = 0; i < kWalkSteps; ++i) {
-        const uint8_t* piece = rec + step_offset(s0 + i, units, head, lane) + 512u;
-        lo[i] = reinterpret_cast<const uint32_t*>(piece)[1];
-        hi[i] = reinterpret_cast<const uint32_t*>(piece)[3];
-      }
-#pragma unroll
-      for (uint32_t i = 0; i < kWalkSteps; ++i) lo[i] = (s0 + i) * kStepUnits + (lane >> 3) < units ? walk_mask(lo[i], hi[i]) : 0u;
-      uint32_t n;
-      do {
-        uint32_t key = 0;  // (the lanes without one: any block that is there)
-        n = 0;
-#pragma unroll
-        for (uint32_t i = 0; i < kWalkSteps; ++i)
-          for (uint64_t left; n < 64u && (left = __builtin_amdgcn_ballot_w64(lo[i] != 0u)) != 0u; ++n) {
-            const uint32_t of = (uint32_t)__builtin_ctzll(left), mask = (uint32_t)__builtin_amdgcn_readlane((int)lo[i], of);
-            key = lane == n ? walk_key(s0 + i, of, (uint32_t)__builtin_ctz(mask)) : key;
-            lo[i] = lane == of ? mask & (mask - 1u) : lo[i];
-          }
+    for (;;) {
+      const uint64_t left = __builtin_amdgcn_ballot_w64(mask != 0u);
+      if (left != 0u && n < 64u) {
+        const uint32_t of = (uint32_t)__builtin_ctzll(left), m = (uint32_t)__builtin_amdgcn_readlane((int)mask, of);
+        key = lane == n ? walk_key(step - 1u, of, (uint32_t)__builtin_ctz(m)) : key;
+        mask = lane == of ? m & (m - 1u) : mask;
+        ++n;
+      } else if (left == 0u && step < steps) {
+        mask = step * kStepUnits + (lane >> 3) < units ? walk_mask(next.x, next.y) : 0u;
+        ++step;
+        next = masks(step);  // (past the last: units that are there)
+      } else {
         const uint32_t blk = key & 0xFFFFFFFu, r = key >> 28, k = blk & 3u;
         const uint8_t* unit = rec + head + (blk >> 2) * kUnitBytes + (r & 7u) * 16u;
         const u32x2_t d = *reinterpret_cast<const u32x2_t*>(unit + ((r >> 3) * 2u + (k >> 1)) * 128u + (k & 1u) * 8u);
@@ -845,7 +849,9 @@ __device__ __forceinline__ float tile_extras(const TileExtras& X, const uint8_t*
         const uint32_t one[3] = {e.at < 8u ? bit : 0u, (e.at >> 3) == 1u ? bit : 0u, (e.at >> 3) == 2u ? bit : 0u};
         const int v = digits_sum<DIG>(w, x, ((int)e.win - 3) * (int)ss.x) - (digits_sum<DIG>(one, x, 0) << 4);
         to_rows((float)(e.negative ? -v : v) * (scale_at(e.slot << 3, table) * __uint_as_float(ss.y)), key, n);
-      } while (n == 64u);
+        if (left == 0u) break;
+        key = n = 0;
+      }
     }
   }
   return fmaf(sum, X.scale, t);
