@@ -16,8 +16,9 @@ constexpr double kEscapeShare = 0.78e-3, kEscapeShare13 = 3.16e-3;
 // every product.)  Shell 13 takes no batched products, whose kernels have room for 32.
 constexpr double kListMisses = 1. / 30000;
 constexpr uint32_t kMaxListSlots = 32, kMaxListSlots13 = 96;
+constexpr uint32_t kMaxListBlocks = 1u << 19;  // what an entry has bits for; rows of more have no list, and their codes are read
 inline uint32_t list_slots(uint32_t nb, bool shell13) {
-  if (nb == 0) return 0u;
+  if (nb == 0 || nb > kMaxListBlocks) return 0u;
   const double mean = (double)kTileRows * nb * (shell13 ? kEscapeShare13 : kEscapeShare);
   const uint32_t most = shell13 ? kMaxListSlots13 : kMaxListSlots;
   double term = std::exp(-mean), within = term;

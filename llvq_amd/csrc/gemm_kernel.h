@@ -411,7 +411,7 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
 #pragma unroll
     for (int k = 0; k < RG; ++k) {
       b[k] = gemm_block(W[k].d.x, W[k].d.y, W[k].m.x, W[k].m.y, g, table);
-      // Escapes from the tiles' lists, where those count: 30 instructions and not 120.  (One of twenty units has one, but so
+      // Escapes from the tiles' lists, where those count: 30 instructions and not 120 (what the codes take here, block_escape with them).  (One of twenty units has one, but so
       // has nearly every workgroup, and waits for it: 0.1 us of 6.5.)
       if (__builtin_amdgcn_ballot_w64(is_escape(b[k]))) {
         if (read_codes) {
@@ -753,7 +753,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
   // that has one.  Gate and up of a 4B layer at 512 rows, 81 us: with one tile whose list does not count 101 -> 87 us, with one
   // escape in a hundred blocks 191 -> 124 us; 17408 x 17408 with the escapes of uniform codes, past 64 in one wavefront of six,
   // 500 -> 360 us, without any 350 (before: from the first of these on every step was read by every lane, 500 instructions a fragment).
-  uint32_t left_steps = 0;  // bit s of the 2048 in the lanes: step s0 + s (+ 2048 ...) may have one of those
+  uint32_t left_steps = t.slots ? 0u : ~0u;  // bit s of the 2048 in the lanes: step s0 + s (+ 2048 ...) may have one of those
   const uint32_t my_tiles = gemm_wide_x_bytes<CF>() + wave * kTileBytes;
   const auto tile_place = [&](uint32_t tile_of, uint32_t row, uint32_t blk) __attribute__((always_inline)) {
     return (tile_of * 256u + (row >> 3) * 128u + (row & 7u) * 16u + (blk & 1u) * 8u) | (512u * RF + tile_of * 128u + (row & 7u) * 16u + (row >> 3) * 8u) << 12 | (blk & 3u) << 24;

@@ -48,6 +48,8 @@ int main() {
     }
   }
   if (list_slots(0, false) || list_slots(0, true)) fail("places of no block", 0, 0);
+  for (uint32_t nb : {1u << 19, (1u << 19) + 1u})  // (an entry has 19 bits for the block)
+    if (list_slots(nb, false) != (nb >> 19 << 19 == nb ? kMaxListSlots : 0u)) fail("places of the widest rows", nb, list_slots(nb, false));
   for (uint32_t byte = 0; byte < 256; ++byte)
     for (uint32_t k = 0; k < 4; ++k) {
       const uint32_t lo = byte << (8 * k) | (0x7F7F7F7Fu & ~(255u << (8 * k))), want = byte >= kBlockEscape ? 1u << (8 * k) : 0u;

@@ -144,3 +144,27 @@ def test_a_list_that_overflows_is_not_many_times_a_batch1_launch(gpu_rt, orc):
     usual, one = (sorted(t)[3] for t in took)
     print(f"OBSERVED {usual * 10:.2f} us, {one * 10:.2f} us with a list that overflows")
     assert one < 2.5 * usual
+
+
+@pytest.mark.parametrize("M", [2, 65])
+def test_rows_of_more_blocks_than_an_entry_has_bits_for(gpu_rt, orc, M):
+    """Past 2^19 blocks (12.6 M columns) a tile has no list: its codes are read.  With lists, the escapes past that block were added to
+    other rows."""
+    import torch
+
+    nb, d_out = (1 << 19) + 300, 2
+    rng = np.random.default_rng(3)
+    few = synth.make_matrix("model.layers.0.widest.weight", d_out, 24, seed=2)
+    codes = artifact.pack_codes(rng.integers(0, orc.N12 + 1, d_out * nb).astype(np.uint64), rng.integers(0, 2, d_out * nb).astype(np.uint8), artifact.index_bits(12))
+    raw = artifact.RawMatrix(few.name, d_out, nb * 24, 12, few.centroids, few.row_scales, few.tail, codes)
+    X = rng.standard_normal((2, raw.d_in), dtype=np.float32).astype(np.float16)
+    Y_ref, _ = _reference(orc, raw, X)
+    proj = gpu_rt.upload(raw)
+    try:
+        x = _x16(X)[torch.arange(M, device="cuda") % 2]
+        y = gpu_rt.forward_batched(proj, x, out_dtype=torch.float32).double().cpu().numpy()
+    finally:
+        gpu_rt.free(proj)
+    # weights are rounded to binary16 one by one: 2^-12 of each on average, whose sum over 12.6 M columns goes with the root of their number
+    for m in range(M):
+        assert np.linalg.norm(y[m] - Y_ref[m % 2]) < 1e-3 * np.linalg.norm(Y_ref[m % 2])
