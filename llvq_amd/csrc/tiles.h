@@ -118,8 +118,8 @@ __global__ __launch_bounds__(512) void transcode_kernel(GlobalTables g, const ui
   }
 }
 
-// The lists in order, behind transcode_kernel, whose lanes put an escape wherever there was room: a wavefront per tile, two
-// escapes a lane, which go where as many lie before them.
+// The lists in order, behind transcode_kernel, whose lanes put an escape wherever there was room: a wavefront per tile, an
+// escape a lane, or two where there are places for more, which go where as many lie before them.
 static_assert(kMaxListSlots13 <= 128 && kMaxListSlots <= kMaxListSlots13, "two places of a list to a lane");
 __global__ __launch_bounds__(256) void sort_lists_kernel(uint8_t* __restrict__ tiles, uint32_t n_tiles, uint32_t stride, uint32_t slots) {
   const uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
@@ -129,6 +129,14 @@ __global__ __launch_bounds__(256) void sort_lists_kernel(uint8_t* __restrict__ t
   uint4* list = reinterpret_cast<uint4*>(t + stride - slots * 16u);
   if (count > slots) {
     if (lane == 0) list[0].w = 0xFFFFFFFFu;  // for those who read the list alone
+    return;
+  }
+  if (slots <= 64u) {
+    const uint4 mine = list[min(lane, slots - 1u)];
+    uint32_t before = 0;
+    for (uint32_t e = 0; e < count; ++e) before += (uint32_t)__shfl((int)mine.w, (int)e) < mine.w ? 1u : 0u;
+    if (lane < count) list[before] = mine;
+    else if (lane < slots) list[lane] = make_uint4(0, 0, 0, 0);
     return;
   }
   uint4 mine[2];
