@@ -801,20 +801,18 @@ __device__ __forceinline__ float tile_extras(const TileExtras& X, const uint8_t*
     }
   };
   if (__builtin_expect(count <= slots, 1)) {
-    u32x4_t e = X.escape;
-    uint32_t first = 0;
-#pragma unroll 1
-    for (;;) {
-      const uint32_t key = first + lane < count ? e.w : 0u, blk = (key >> 9) & 0x7FFFFu, w[3] = {e.x, e.y, e.z};  // (the others: any block that is there)
+    auto listed = [&](const u32x4_t& e, uint32_t n) __attribute__((always_inline)) {
+      const uint32_t key = lane < n ? e.w : 0u, blk = (key >> 9) & 0x7FFFFu, w[3] = {e.x, e.y, e.z};  // (the others: any block that is there)
       int x[3 * DIG];
       load_planes<DIG>(L.planes + plane_at<DIG>(blk), x);
       const u32x2_t ss = *reinterpret_cast<const u32x2_t*>(L.planes + plane_sum_at<DIG>(blk));
       const int v = (digits_sum<DIG>(w, x, 0) << 1) + ((key >> 8) & 1u ? (int)ss.x : 0);
-      to_rows((float)v * (scale_at((key & 31u) << 3, table) * __uint_as_float(ss.y)), key, min(count - first, 64u));
-      first += 64u;
-      if (__builtin_expect(first >= count, 1)) break;
+      to_rows((float)v * (scale_at((key & 31u) << 3, table) * __uint_as_float(ss.y)), key, n);
+    };
+    listed(X.escape, min(count, 64u));
+    if (__builtin_expect(count > 64u, 0)) {  // (a loop instead: 0.1 us of every launch)
       asm volatile("" : "+s"(nb), "+s"(tail_w));  // (as below)
-      e = *reinterpret_cast<const u32x4_t*>(rec + list_at(nb, tail_w) + min(first + lane, slots - 1u) * 16u);
+      listed(*reinterpret_cast<const u32x4_t*>(rec + list_at(nb, tail_w) + min(64u + lane, slots - 1u) * 16u), count - 64u);
     }
   } else {
     // More than there was room for: the tile's meta dwords step by step, the next one's on their way, and of the escapes they show one to a
