@@ -2,7 +2,7 @@
 // product with a few logical instructions.  Compiled for gfx950 and for the host.
 //
 // The coordinates v of a point are all even or all odd and lie, but for 0.08 % of uniformly drawn points of shells 2..12
-// (0.4 % with shell 13), in a window [b, b + 14] with -11 <= b <= -4 of their parity: v = 2 j + b with j of 3 bits.
+// (0.32 % of shells 2..13), in a window [b, b + 14] with -11 <= b <= -4 of their parity: v = 2 j + b with j of 3 bits.
 // Nothing is rounded.
 //
 // An octet of coordinates is a dword of eight nibbles, two's complement, 2 (j - 4) in each: their lowest bits are free.

@@ -1045,8 +1045,9 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
 }
 
 // Enqueues x' = Q x for `rows` activation rows of width rot->n.
-// Rows up to which a rotation writes octets: a column of them is m_pad x 16 bytes, so the rows' stores share no lines.  2048 x
-// 4096 at 20 rows 17.2 -> 16.1 us with it, q/k/v of a 14B layer at 130 rows 43.2 -> 41.7, 5120 x 4096 at 300 rows 42.1 -> 43.0.
+// Rows up to which a rotation writes octets, as many as there are workgroups at once: a column of them is m_pad x 16 bytes, so the rows'
+// stores share no lines, and a second turn waits for them.  From 1024 x 2560 to 13000 x 12288: at 3 rows 1.5 to 2.6 us less with it, at 64
+// 0.5 to 1.7, at 200 and 256 0.1 to 1.7; at 300 rows 0.4 to 5.5 us more, at 600 1.2 to 11.
 constexpr int kRotOctetRows = 256;
 static RotArgs rot_args(const llvq_rt::DevRotation* rot, const void* x_f16, void* out) {
   RotArgs a{};

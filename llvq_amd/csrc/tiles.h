@@ -25,7 +25,8 @@
 // Eight units are a step of a wavefront, 5120 consecutive bytes: lane (l, q) = (lane % 8, lane / 8) loads the five pieces l
 // of unit q.  Every line of memory is asked for by one load, whole, and marked as not to be kept: read like that the card
 // delivers 6.9 TB/s (a loop of nothing else, 8 or 16 wavefronts on a CU), without the mark 6.1, and 5.9 where 12-byte
-// pieces and their bytes of meta are asked for by two loads that share lines (there the mark makes it 5.4).
+// pieces and their bytes of meta are asked for by two loads that share lines (there the mark makes it 5.4).  A 4B model as one
+// launch takes 257 us with the mark and 291 without; four layers by themselves, which the 256 MB cache holds, 38.0 and 36.2.
 #pragma once
 
 #include "block_code.h"
