@@ -238,9 +238,9 @@ __global__ __launch_bounds__(1024) void gemv_seq_kernel(SeqArgs s) {
     auto ask = [&] { if constexpr (!kWaits) request(); };
     constexpr int kPasses = kWide ? 4 : 2;
     const bool resid = u == I.first_unit;
-    if (kPro && I.prologue == kPrologueSiluMul) stage_x<DIG, kSrcSiluMul, kPasses, kWaits>(in, nb, tail_w, L, resid, ask);
-    else if (kPro && I.prologue == kPrologueAddRmsNorm) stage_x<DIG, kSrcAddRmsNorm, kPasses, kWaits>(in, nb, tail_w, L, resid, ask);
-    else stage_x<DIG, kSrcF16, kPasses, kWaits>(in, nb, tail_w, L, false, ask);
+    if (kPro && I.prologue == kPrologueSiluMul) stage_x<DIG, kSrcSiluMul, kPasses, kWaits>(in, nb, tail_w, kSeqWaves, stage_passes(nb, kSeqWaves), L, resid, ask);
+    else if (kPro && I.prologue == kPrologueAddRmsNorm) stage_x<DIG, kSrcAddRmsNorm, kPasses, kWaits>(in, nb, tail_w, kSeqWaves, stage_passes(nb, kSeqWaves), L, resid, ask);
+    else stage_x<DIG, kSrcF16, kPasses, kWaits>(in, nb, tail_w, kSeqWaves, stage_passes(nb, kSeqWaves), L, false, ask);
     lds_barrier();
 
     auto store_rows = [&](const Task& t, float v) {

@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -1036,10 +1037,14 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
   a.teams = std::min((a.n_tiles + cus - 1u) / cus, kGemvMaxWaves / a.team);
   const uint32_t grid = std::min(cus, (a.n_tiles + a.teams - 1u) / a.teams);
-  const uint32_t waves = rotated || gemv_wide(a.nb) ? kGemvMaxWaves : a.teams * a.team;
+  a.grid = grid;
+  a.waves = rotated || gemv_wide(a.nb) ? kGemvMaxWaves : a.teams * a.team;
+  a.passes = stage_passes(a.nb, a.waves);
+  a.inv_team = (65536u + a.team - 1u) / a.team;
+  a.inv_teams = (65536u + a.teams - 1u) / a.teams;
   const int src = rotated ? kSrcRotated : a.in.prologue == kPrologueSiluMul ? kSrcSiluMul : a.in.prologue == kPrologueAddRmsNorm ? kSrcAddRmsNorm : kSrcF16;
   void* params[] = {&a};
-  HIP_TRY(hipLaunchKernel(gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(grid), dim3(waves * 64u), params,
+  HIP_TRY(hipLaunchKernel(gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(grid), dim3(a.waves * 64u), params,
                           gemv_tiles_lds_bytes(a.nb, m0->d_in, f32, rot != nullptr), rt->stream));
   return LLVQ_OK;
 }

@@ -25,6 +25,8 @@ LLVQ_HD uint32_t gemv_team(uint32_t nb) {
   const uint32_t steps = tile_steps(nb);
   return steps > kGemvMaxWaves ? kGemvMaxWaves : steps ? steps : 1u;
 }
+// How often the quads of that many wavefronts pass over a row's blocks, whole steps of them.
+LLVQ_HD uint32_t stage_passes(uint32_t nb, uint32_t waves) { return (tile_steps(nb) * kStepBlocks + waves * 16u - 1u) / (waves * 16u); }
 LLVQ_HD bool gemv_wide(uint32_t nb) { return nb > kStepBlocks * kGemvMaxWaves; }
 // ... and so that there is a wavefront for each of the workgroup's
 LLVQ_HD uint32_t gemv_batch(uint32_t team) { return team < kGemvRounds ? team : kGemvRounds; }
