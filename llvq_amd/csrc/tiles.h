@@ -210,28 +210,27 @@ __device__ __forceinline__ int quad_sum(int v) {
 }
 
 // Eight values of a block (columns 8 sub .. 8 sub + 7 of it), sub = lane % 4; the quad's fourth lane passes zeros and
-// only takes part in the exchange.  Writes the block's planes at xb, its sum and scale at xs.  About 90 instructions for the quad's 24 values.
-template <int DIG>
-__device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub, uint32_t* xb, uint32_t* xs) {
+// only takes part in the exchange.  m: what the f32 bits of the quad's values have for a largest magnitude (a NaN is larger than
+// anything); value(j, up, magic): value j times up plus magic, fused.  Writes the block's planes at xb, its sum and scale at xs.
+// Every wavefront of a workgroup quantises and every workgroup does it for itself, so that its instructions count: about 50 from binary16 values
+// (converted as they are multiplied), 60 from f32 ones; with a value at a time 100, and a token of a 4B model 1535 us, not 1516.
+template <int DIG, class Value>
+__device__ __forceinline__ void quantize_scaled(uint32_t m, Value&& value, uint32_t sub, uint32_t* xb, uint32_t* xs) {
   constexpr int kBits = DIG == 4 ? 14 : 22;
   constexpr uint32_t kMagic = 0x4B400000u;  // 1.5 2^23: adding it leaves the rounded integer in the low mantissa bits
-  uint32_t m = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) m = max(m, __float_as_uint(v[j]) & 0x7FFFFFFFu);
-  m = quad_max(m);
   // Biased exponent of the block's largest, at least the one below which `scale` would leave the normal range (2^-105 with
   // six digits, 2^-113 with four): smaller blocks are quantised at that scale.
   const uint32_t e = max(m >> 23, (uint32_t)kBits);
-  const bool bad = m >= 0x7F800000u;     // inf or NaN: the block's products are NaN
-  const float up = bad ? 0.f : __uint_as_float((253u + (uint32_t)kBits - e) << 23);
+  const bool bad = m >= 0x7F800000u;     // inf or NaN: the block's products are NaN, whatever the digits
+  const float up = __uint_as_float((253u + (uint32_t)kBits - e) << 23);
   const float scale = bad ? __builtin_nanf("") : __uint_as_float((e + 1u - (uint32_t)kBits) << 23);
-  uint32_t t[8];
+  uint32_t t[8], total = 0;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) t[j] = __float_as_uint(fmaf(bad ? 0.f : v[j], up, __uint_as_float(kMagic)));
-  int sum = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) sum += (int)(t[j] - kMagic);
-  sum = quad_sum(sum);
+  for (int j = 0; j < 8; ++j) {
+    t[j] = __float_as_uint(value(j, up, __uint_as_float(kMagic)));
+    total += t[j];
+  }
+  const int sum = quad_sum((int)(total - 8u * kMagic));
   uint32_t lo[DIG / 2], hi[DIG / 2];  // byte k of the values in slots 0..3 and 4..7: columns 0, 4, 1, 5 and 2, 6, 3, 7
   if constexpr (DIG == 4) {
     uint32_t p[4];  // two 16-bit values each; adding 8 to every digit and flipping its top bit makes the digits balanced
@@ -271,6 +270,32 @@ __device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub
     xs[0] = (uint32_t)sum;
     xs[1] = __float_as_uint(scale);
   }
+}
+
+// f32 values.  kAny: they may be any; else one of them is not finite only if none of the lane's is (a rotation's).
+template <int DIG, bool kAny>
+__device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub, uint32_t* xb, uint32_t* xs) {
+  uint32_t m = 0;
+  if constexpr (kAny) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = max(m, __float_as_uint(v[j]) & 0x7FFFFFFFu);
+  } else {
+    float f = 0.f;  // (of NaN and another value v_max3_f32 gives the other)
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(f) : "v"(v[j]), "v"(v[j + 1]));
+    m = __float_as_uint(f);
+  }
+  quantize_scaled<DIG>(quad_max(m), [&](int j, float up, float magic) { return fmaf(v[j], up, magic); }, sub, xb, xs);
+}
+// binary16 values, in pairs
+template <int DIG>
+__device__ __forceinline__ void quantize_halves(const uint32_t (&w)[4], uint32_t sub, uint32_t* xb, uint32_t* xs) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  us2 two = __builtin_bit_cast(us2, w[0] & 0x7FFF7FFFu);
+#pragma unroll
+  for (int j = 1; j < 4; ++j) two = __builtin_elementwise_max(two, __builtin_bit_cast(us2, w[j] & 0x7FFF7FFFu));
+  const uint32_t m = quad_max(max((uint32_t)two.x, (uint32_t)two.y));
+  quantize_scaled<DIG>(__float_as_uint(half_lo(m)), [&](int j, float up, float magic) { return fmaf(j & 1 ? half_hi(w[j >> 1]) : half_lo(w[j >> 1]), up, magic); }, sub, xb, xs);
 }
 
 // ---- batch-1 product ------------------------------------------------------------------------------
@@ -319,6 +344,9 @@ __device__ __forceinline__ GemvLds gemv_lds(uint8_t* smem, uint32_t plane_units)
   return L;
 }
 
+__device__ __forceinline__ uint32_t pack_halves(float lo, float hi) {
+  return (uint32_t)__half_as_ushort(__float2half_rn(lo)) | (uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16;
+}
 __device__ __forceinline__ float round_half(float v) { return __half2float(__float2half_rn(v)); }
 __device__ __forceinline__ float silu_mul(float gate, float up) { return round_half(round_half(gate / (1.0f + __expf(-gate))) * up); }
 
@@ -352,7 +380,6 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
   const uint32_t tid = threadIdx.x, n_thr = waves * 64u, lane = tid & 63u, wave = tid >> 6;
   const uint32_t sub = tid & 3u, quad = tid >> 2, quads = n_thr >> 2;
   const uint32_t pad = tile_steps(nb) * kStepBlocks, d_in = nb * kDim + tail_w;
-  auto quantize = [&](const float (&v)[8], uint32_t blk) { quantize_octet<DIG>(v, sub, L.planes + plane_at<DIG>(blk), L.planes + plane_sum_at<DIG>(blk)); };
   auto zeros = [&]() {  // past the tail, and the step of zeros
     if (tid < 32u) L.xtail[tid] = 0.f;
     for (uint32_t i = tid; i < kStepUnits * XPlanes<DIG>::kDwords; i += n_thr) L.planes[plane_at<DIG>(pad) + i] = 0u;
@@ -393,7 +420,6 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
             sg[i] = signs[from >> 3];
           }
         };
-        auto pack = [](float lo, float hi) { return (uint32_t)__half_as_ushort(__float2half_rn(lo)) | (uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16; };
         load_tile(wave);
         if constexpr (PMAX <= 2) request();
         __builtin_amdgcn_sched_barrier(0);
@@ -410,7 +436,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
                 lo = round_half(lo + half_lo(b[i].w[j]));
                 hi = round_half(hi + half_hi(b[i].w[j]));
               }
-              a[i].w[j] = pack(lo, hi);
+              a[i].w[j] = pack_halves(lo, hi);
               ss = fmaf(lo, lo, fmaf(hi, hi, ss));
             }
             if (in.resid_out && store_resid) *reinterpret_cast<HalfOctet*>(in.resid_out + rot_octet_at(wave, i)) = a[i];
@@ -425,11 +451,11 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
             if (silu) {
 #pragma unroll
               for (int j = 0; j < 4; ++j)
-                a[i].w[j] = pack(silu_mul(half_lo(b[i].w[j]), half_lo(a[i].w[j])), silu_mul(half_hi(b[i].w[j]), half_hi(a[i].w[j])));
+                a[i].w[j] = pack_halves(silu_mul(half_lo(b[i].w[j]), half_lo(a[i].w[j])), silu_mul(half_hi(b[i].w[j]), half_hi(a[i].w[j])));
             } else if (norm) {
 #pragma unroll
               for (int j = 0; j < 4; ++j)
-                a[i].w[j] = pack(half_lo(a[i].w[j]) * inv * half_lo(g[i].w[j]), half_hi(a[i].w[j]) * inv * half_hi(g[i].w[j]));
+                a[i].w[j] = pack_halves(half_lo(a[i].w[j]) * inv * half_lo(g[i].w[j]), half_hi(a[i].w[j]) * inv * half_hi(g[i].w[j]));
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) a[i].w[j] = rot_octet_at(tile, i) < d_in ? flip_signs(a[i].w[j], sg[i], j) : 0u;
@@ -468,17 +494,22 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
       float v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = 0.f;
-      if (blk < nb && sub < 3u) {
-        const uint32_t at = blk * kDim + sub * 8u;
-        if (in.x_f32) {
+      const bool ok = blk < nb && sub < 3u;
+      const uint32_t at = blk * kDim + sub * 8u;
+      uint32_t *const xb = L.planes + plane_at<DIG>(blk), *const xs = L.planes + plane_sum_at<DIG>(blk);
+      if (in.x_f32) {
+        if (ok) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[j] = in.x_f32[at + j];
-        } else {
+        }
+        quantize_octet<DIG, true>(v, sub, xb, xs);
+      } else {
+        if (ok) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[j] = xf[at + j];
         }
+        quantize_octet<DIG, false>(v, sub, xb, xs);
       }
-      quantize(v, blk);
     }
     if (tid < tail_w) L.xtail[tid] = in.x_f32 ? in.x_f32[nb * kDim + tid] : xf[nb * kDim + tid];
   } else {
@@ -487,10 +518,6 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
     // second puts the block's planes (or, when two passes are all, in the registers).
     constexpr int kChunk = PMAX > 2 && DIG == 6 ? 1 : 2;
     const __half* second = SRC == kSrcAddRmsNorm ? (in.x2 ? in.x2 : in.x) : in.x2;
-    const uint32_t t_at = min(nb * kDim + tid, d_in - 1u);
-    float t0 = __half2float(load_half<kDeviceScope>(in.x + t_at)), t1 = 0.f, tg = 0.f;
-    if constexpr (SRC != kSrcF16) t1 = __half2float(load_half<kDeviceScope>(second + t_at));
-    if constexpr (SRC == kSrcAddRmsNorm) tg = __half2float(in.norm_w[t_at]);
     uint32_t a[kChunk][4], b[kChunk][4], g[kChunk][4];
     auto block_of = [&](uint32_t p) { return quad + p * quads; };
     auto load_operands = [&](uint32_t p0) {
@@ -509,23 +536,22 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
     };
     auto emit = [&](int k, uint32_t blk, float inv) {  // a[k] (and b, g) -> the planes of block blk
       const bool ok = blk < nb && sub < 3u;
-      float v[8];
+      uint32_t w[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        float lo = half_lo(a[k][j]), hi = half_hi(a[k][j]);
-        if constexpr (SRC == kSrcSiluMul) {
-          lo = silu_mul(half_lo(b[k][j]), lo);
-          hi = silu_mul(half_hi(b[k][j]), hi);
-        } else if constexpr (SRC == kSrcAddRmsNorm) {
-          lo = round_half(lo * inv * half_lo(g[k][j]));
-          hi = round_half(hi * inv * half_hi(g[k][j]));
-        }
-        v[2 * j] = ok ? lo : 0.f;
-        v[2 * j + 1] = ok ? hi : 0.f;
+        const float lo = half_lo(a[k][j]), hi = half_hi(a[k][j]);
+        w[j] = a[k][j];
+        if constexpr (SRC == kSrcSiluMul) w[j] = pack_halves(silu_mul(half_lo(b[k][j]), lo), silu_mul(half_hi(b[k][j]), hi));
+        if constexpr (SRC == kSrcAddRmsNorm) w[j] = pack_halves(lo * inv * half_lo(g[k][j]), hi * inv * half_hi(g[k][j]));
+        w[j] = ok ? w[j] : 0u;
       }
-      quantize(v, blk);
+      quantize_halves<DIG>(w, sub, L.planes + plane_at<DIG>(blk), L.planes + plane_sum_at<DIG>(blk));
     };
     load_operands(0);
+    const uint32_t t_at = min(nb * kDim + tid, d_in - 1u);
+    float t0 = __half2float(load_half<kDeviceScope>(in.x + t_at)), t1 = 0.f, tg = 0.f;
+    if constexpr (SRC != kSrcF16) t1 = __half2float(load_half<kDeviceScope>(second + t_at));
+    if constexpr (SRC == kSrcAddRmsNorm) tg = __half2float(in.norm_w[t_at]);
     request();
     __builtin_amdgcn_sched_barrier(0);
     zeros();
@@ -544,7 +570,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
                 lo = round_half(lo + half_lo(b[k][j]));
                 hi = round_half(hi + half_hi(b[k][j]));
               }
-              a[k][j] = (uint32_t)__half_as_ushort(__float2half_rn(lo)) | (uint32_t)__half_as_ushort(__float2half_rn(hi)) << 16;
+              a[k][j] = pack_halves(lo, hi);
               ss = fmaf(lo, lo, fmaf(hi, hi, ss));
             }
             if (in.resid_out && store_resid) {
