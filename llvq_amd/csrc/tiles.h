@@ -280,9 +280,10 @@ __device__ __forceinline__ void quantize_octet(const float (&v)[8], uint32_t sub
 #pragma unroll
     for (int j = 0; j < 8; ++j) m = max(m, __float_as_uint(v[j]) & 0x7FFFFFFFu);
   } else {
-    float f = 0.f;  // (of NaN and another value v_max3_f32 gives the other)
+    float f;  // (of a NaN and another value these give the other)
+    asm("v_max_f32 %0, |%1|, |%2|" : "=v"(f) : "v"(v[0]), "v"(v[1]));
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(f) : "v"(v[j]), "v"(v[j + 1]));
+    for (int j = 2; j < 8; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(f) : "v"(v[j]), "v"(v[j + 1]));
     m = __float_as_uint(f);
   }
   quantize_scaled<DIG>(quad_max(m), [&](int j, float up, float magic) { return fmaf(v[j], up, magic); }, sub, xb, xs);

@@ -231,3 +231,32 @@ def test_rotated_rows_to_octets(gpu_rt, n, rows):
             gpu_rt.free(p)
     for y, z in zip(ys, alone):
         assert torch.isfinite(z).all() and torch.equal(y, z)
+
+
+# around what the lane moves reach (columns of 32 values, m = 64 .. 1024), above and below it; k up to 9 as scalars (whole columns to a lane,
+# parts of a column to the wavefronts), above on the matrix cores
+@pytest.mark.parametrize("m,k", [(32, 9), (64, 1), (64, 3), (64, 9), (64, 11), (128, 5), (256, 7), (256, 31), (512, 1), (512, 9), (512, 11), (1024, 1), (1024, 3),
+                                 (1024, 9), (1024, 17), (2048, 1), (2048, 5), (4096, 3), (8192, 1)])
+def test_rotation_of_every_kind_of_width(gpu_rt, orc, m, k):
+    import torch
+
+    n = m * k
+    raw = _rotated(f"model.layers.0.rw{n}.weight", 16, n, 1, n)
+    x = synth.make_activation(n, seed=n)[0]
+    proj = gpu_rt.upload(raw)
+    try:
+        xr = gpu_rt.rotate(proj, _x16(x))
+        got = xr.cpu().numpy().reshape(-1)
+        want = orc.Rotation(n, n).apply(x.astype(np.float64))
+        # f32: a rounding for each of log2 m levels, for the k terms of a sum and for the two factors
+        assert np.linalg.norm(got - want) <= (np.log2(m) + k + 2) * 2.0**-24 * np.linalg.norm(want)
+        assert np.array_equal(gpu_rt.forward(proj, _x16(x), out_dtype=torch.float32).cpu().numpy().reshape(-1),
+                              gpu_rt.forward_rotated(proj, xr, out_dtype=torch.float32).cpu().numpy().reshape(-1))
+        # one value that is not finite is in all of them
+        for value in (float("nan"), float("inf"), float("-inf")):
+            bad = _x16(x)
+            bad[n // 2] = value
+            for dtype in (torch.float16, torch.float32):
+                assert not torch.isfinite(gpu_rt.forward(proj, bad, out_dtype=dtype)).any()
+    finally:
+        gpu_rt.free(proj)
