@@ -183,7 +183,7 @@ struct ActivationIn {
   uint32_t prologue;   // kPrologue*
   // the basis of the matrices, when they are stored rotated and the launch rotates its own activation (see rotate_lds)
   const uint32_t* rot_signbits;
-  const void* rot_fragments;  // [64] RotFragments
+  const void* rot_fragments;  // RotTable
   float rot_inv;
   uint32_t rot_m, rot_k;
 };
@@ -205,24 +205,31 @@ __device__ __forceinline__ float half_hi(uint32_t w) { return __half2float(__ush
 //
 // Every workgroup of a batch-1 product rotates its own activation, and with sixteen wavefronts on a CU an instruction of
 // each costs 7 ns: what bounds a rotation is their number.  (With a value per lane and load, lane exchanges through LDS and a
-// pass over LDS per level above 512 a 2560 x 9728 product took 19.2 us; it takes 12.7.)  So:
+// pass over LDS per level above 512 a 2560 x 9728 product took 19.2 us; with the levels at 48 instructions, sixteen wavefronts'
+// operands asked for where ten have any, and every k on the matrix cores 12.6; it takes 11.6, and 5120 x 5120 9.0 where it was 11.5.)  So:
 //  * The five lowest levels are two matrix-core steps: what is rotated is binary16, the entries of H are 0 and +-1, so
 //    the products are exact and the sums f32, as butterflies would have them.  A wavefront takes 1024 values; a column of
 //    its 32 x 32 result is 32 neighbouring ones, requested by two lanes as two octets each (with their signs).
-//  * The next four are lane moves between columns, on the sixteen results a lane holds; the values meet LDS once.
-//  * The levels above 512 are passes over LDS, three levels to a pass, the k x k block is f32 matrix-core steps (rotate_rest).
-// A lane's parts of both matrices lie together in a table (RotFragments).
+//  * The next five are lane moves between columns, on the sixteen results a lane holds, an instruction to a result and level
+//    (lane_level); the values meet LDS once.
+//  * The levels above 1024 are passes over LDS, three levels to a pass, the k x k block is products of scalars for k up to 9, else f32
+//    matrix-core steps (rotate_rest).
+// A lane's parts of both matrices lie together in a table (RotFragments), the k x k block as it is behind it (RotTable).
 // Where an octet spans groups (m < 8) the signed values are put into LDS instead and every level is a pass there.
 constexpr uint32_t kRotOctetM = 8;    // the narrowest m that takes the octets
-constexpr uint32_t kRotRun = 512;     // values that the levels before LDS reach across
-constexpr uint32_t kRotTile = 1024;   // values of a wavefront
+constexpr uint32_t kRotTile = 1024;   // values of a wavefront, and how far the levels before LDS reach
 typedef _Float16 rot_h8_t __attribute__((ext_vector_type(8)));
 typedef float rot_acc_t __attribute__((ext_vector_type(16)));
-struct RotFragments {   // of lane l: (l32, lh) = (l % 32, l / 32)
+struct __attribute__((aligned(16))) RotFragments {   // of lane l: (l32, lh) = (l % 32, l / 32)
   float s[kRotKMax / 2];  // S[l32][2 i + lh], zero past k
   rot_h8_t h[2];          // H[l32][16 i + 8 lh + e], H the transform inside groups of min(m, 32)
 };
 static_assert(sizeof(RotFragments) == 96, "six 16-byte loads");
+constexpr uint32_t kRotScalarK = 9;  // the largest k whose block is multiplied as scalars: rows of it are padded to that, with zeros
+struct RotTable {
+  RotFragments lane[64];
+  float rows[kRotScalarK][kRotScalarK + 3];  // S[g][i]
+};
 __device__ __forceinline__ float flip_sign(float v, uint32_t bits, int j) {  // bit j of `bits` is the sign of D
   return __uint_as_float(__float_as_uint(v) ^ (((bits >> j) & 1u) << 31));
 }
@@ -235,45 +242,99 @@ __device__ __forceinline__ uint32_t rot_octet_at(uint32_t tile, uint32_t i) {
   const uint32_t lane = threadIdx.x & 63u;
   return tile * kRotTile + (lane & 31u) * 32u + i * 16u + (lane >> 5) * 8u;
 }
-// Sum and difference with the lane L away: lower lanes get own + other, upper ones other - own (sgn = -1 there).
+// A level between lanes that are L apart: v + g * the other lane's v with g = -1 in the lower lane, 1 in the upper one, so that the lower
+// one has the difference and the upper one the sum: what lane l holds in the end belongs to column l with the bits of all such
+// levels turned over.  The compiler makes a move and a multiply-add of it (v_fmac_f32 takes the move as an operand, but is not
+// folded): 16 instructions a level as they stand here, and with a product for the sign, as they were, 48 with the waits in between.  (What a
+// lane move reads has to be written two instructions before.)
 template <int L>
-__device__ __forceinline__ void lane_level(rot_acc_t& v, uint32_t lane, uint32_t m) {
-  if (m < 64u * (uint32_t)L) return;
-  const float sgn = (lane & (uint32_t)L) ? -1.f : 1.f;
+__device__ __forceinline__ void lane_level(rot_acc_t& v, uint32_t lane) {
+  const float g = (lane & (uint32_t)L) ? 1.f : -1.f;
+  if constexpr (L == 1) {  // behind the matrix cores, whose results the compiler waits for
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int i = (int)__float_as_uint(v[r]);
-    int o = i;
-    if constexpr (L == 1) o = __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, true);
-    if constexpr (L == 2) o = __builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, true);
-    if constexpr (L == 4) {  // lane ^ 7, then lane ^ 3
-      o = __builtin_amdgcn_update_dpp(0, i, 0x141, 0xF, 0xF, true);
-      o = __builtin_amdgcn_update_dpp(0, o, 0x1B, 0xF, 0xF, true);
-    }
-    if constexpr (L == 8) o = __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, true);
-    v[r] = __uint_as_float((uint32_t)o) + sgn * v[r];  // (exact product)
+    for (int r = 0; r < 16; ++r) v[r] = fmaf(__uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v[r]), 0xB1, 0xF, 0xF, true)), g, v[r]);
+    return;
   }
+  float a[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) a[r] = v[r];
+#define LEVEL(r, move) "v_fmac_f32_dpp %" #r ", %" #r ", %16 " move " row_mask:0xf bank_mask:0xf\n\t"
+#define LEVELS(move) "s_nop 1\n\t" LEVEL(0, move) LEVEL(1, move) LEVEL(2, move) LEVEL(3, move) LEVEL(4, move) LEVEL(5, move) LEVEL(6, move) LEVEL(7, move) \
+  LEVEL(8, move) LEVEL(9, move) LEVEL(10, move) LEVEL(11, move) LEVEL(12, move) LEVEL(13, move) LEVEL(14, move) LEVEL(15, move) "s_nop 1"
+#define SIXTEEN "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), \
+  "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15])
+  if constexpr (L == 2) asm(LEVELS("quad_perm:[2,3,0,1]") : SIXTEEN : "v"(g));
+  if constexpr (L == 8) asm(LEVELS("row_ror:8") : SIXTEEN : "v"(g));
+  if constexpr (L == 4) {  // lane ^ 7, then lane ^ 3
+    float t0, t1, t2, t3;
+#define MIRROR(t, r) "v_mov_b32_dpp %" #t ", %" #r " row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+#define TURN(r, t) "v_fmac_f32_dpp %" #r ", %" #t ", %20 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf\n\t"
+#define FOUR(r0, r1, r2, r3) MIRROR(16, r0) MIRROR(17, r1) MIRROR(18, r2) MIRROR(19, r3) TURN(r0, 16) TURN(r1, 17) TURN(r2, 18) TURN(r3, 19)
+    asm("s_nop 1\n\t" FOUR(0, 1, 2, 3) FOUR(4, 5, 6, 7) FOUR(8, 9, 10, 11) FOUR(12, 13, 14, 15) "s_nop 1"
+        : SIXTEEN, "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3) : "v"(g));
+#undef FOUR
+#undef TURN
+#undef MIRROR
+  }
+#undef SIXTEEN
+#undef LEVELS
+#undef LEVEL
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r] = a[r];
 }
-// The levels below min(m, 512) of a tile whose signed octets a lane holds (zeros past n), into LDS.
-__device__ __forceinline__ void rotate_tile_to(float* v, const uint32_t (&x0)[4], const uint32_t (&x1)[4], const RotFragments& F, uint32_t tile,
+// The levels below min(m, 1024) of a tile whose signed octets a lane holds (zeros past n), into LDS.
+__device__ __forceinline__ void rotate_tile_to(float* v, const uint32_t (&x0)[4], const uint32_t (&x1)[4], const rot_h8_t (&h)[2], uint32_t tile,
                                                uint32_t n, uint32_t m, uint32_t k, float inv) {
   const uint32_t lane = threadIdx.x & 63u;
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   rot_acc_t acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F.h[0], __builtin_bit_cast(rot_h8_t, u4{x0[0], x0[1], x0[2], x0[3]}), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(F.h[1], __builtin_bit_cast(rot_h8_t, u4{x1[0], x1[1], x1[2], x1[3]}), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(h[0], __builtin_bit_cast(rot_h8_t, u4{x0[0], x0[1], x0[2], x0[3]}), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(h[1], __builtin_bit_cast(rot_h8_t, u4{x1[0], x1[1], x1[2], x1[3]}), acc, 0, 0, 0);
   // acc[r] is value 8 (r / 4) + 4 lh + r % 4 of column l32
-  lane_level<1>(acc, lane, m);
-  lane_level<2>(acc, lane, m);
-  lane_level<4>(acc, lane, m);
-  lane_level<8>(acc, lane, m);
-  if (k == 1 && m <= kRotRun) {  // nothing follows but the factor
+  uint32_t turned = 0;
+  if (m >= 64u) {
+    lane_level<1>(acc, lane);
+    turned = 1u;
+  }
+  if (m >= 128u) {
+    lane_level<2>(acc, lane);
+    turned = 3u;
+  }
+  if (m >= 256u) {
+    lane_level<4>(acc, lane);
+    turned = 7u;
+  }
+  if (m >= 512u) {
+    lane_level<8>(acc, lane);
+    turned = 15u;
+  }
+  const bool done = k == 1 && m <= kRotTile;  // nothing follows but the factor
+  if (m >= 1024u) {
+    // Between the two rows of sixteen lanes results change places, eight against eight: a row has one eight of both, and forms its sums
+    // (column below 16) and differences (that one and 16).
+    const uint32_t row = (lane >> 4) & 1u, at = tile * kRotTile + ((lane & 15u) ^ turned) * 32u + row * 16u + (lane >> 5) * 4u;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[r]), __float_as_uint(acc[r + 8]), false, false);
+      acc[r] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+      acc[r + 8] = __uint_as_float(p[0]) - __uint_as_float(p[1]);
+    }
+    if (done) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] *= inv;
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q)  // (such a tile is whole)
+      *reinterpret_cast<float4*>(v + at + 8u * (q & 1u) + 512u * (q >> 1)) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+    return;
+  }
+  if (done) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] *= inv;
   }
-  const uint32_t at = tile * kRotTile + (lane & 31u) * 32u + (lane >> 5) * 4u;
+  const uint32_t at = tile * kRotTile + ((lane & 31u) ^ turned) * 32u + (lane >> 5) * 4u;
 #pragma unroll
   for (uint32_t q = 0; q < 4u; ++q)
     if (at + 8u * q < n) *reinterpret_cast<float4*>(v + at + 8u * q) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
@@ -301,14 +362,57 @@ __device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t lg,
   }
 }
 
-// What is left once the levels below 512 are in LDS (every level, `put_levels`, where the octets were not taken): the values
+// The k x k block of K x K numbers as products of scalars: a lane takes whole columns, or where there are fewer than lanes the
+// wavefronts share the rows of a column, and read it before any of them writes.  K * K multiply-adds a column, where the matrix cores
+// multiply 32 x 32: 5120 values, k = 5, 2.3 us of a launch with the latter.
+template <uint32_t K>
+__device__ __forceinline__ void rotate_columns(float* v, uint32_t m, float inv, const float* rows) {
+  typedef const float __attribute__((address_space(4))) scalar_f;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lg = 31u - (uint32_t)__builtin_clz(m);
+  const uint32_t parts = m < 1024u ? 1024u >> lg : 1u, part = m < 1024u ? wave >> (lg - 6u) : 0u;  // (m >= 64: a part is whole wavefronts)
+  const uint32_t g0 = K * part / parts, g1 = K * (part + 1u) / parts;
+#pragma unroll 1
+  for (uint32_t j = threadIdx.x & (m - 1u); j < m; j += 1024u) {
+    float c[K];
+#pragma unroll
+    for (uint32_t i = 0; i < K; ++i) c[i] = v[i * m + j] * inv;
+    if (parts > 1u) lds_barrier();
+#pragma unroll 1
+    for (uint32_t g = g0; g < g1; ++g) {
+      scalar_f* s = (scalar_f*)(rows + g * (kRotScalarK + 3u));
+      float t = s[0] * c[0];
+#pragma unroll
+      for (uint32_t i = 1; i < K; ++i) t = fmaf(s[i], c[i], t);
+      v[g * m + j] = t;
+    }
+  }
+}
+// What rotate_rest needs of the k x k block in registers; its loads are to be out in front of the barrier that rotate_rest is behind.
+struct RotBlock { float s[kRotKMax / 2]; };
+__device__ __forceinline__ bool rot_scalars(uint32_t m, uint32_t k) { return m >= 64u && k <= kRotScalarK; }
+__device__ __forceinline__ RotBlock rot_block(const RotTable* table, uint32_t m, uint32_t k) {
+  RotBlock b{};
+  const uint32_t lane = threadIdx.x & 63u;
+  if (!rot_scalars(m, k)) {
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q) {
+      if (8u * q >= k) break;
+      const float4 f = *reinterpret_cast<const float4*>(table->lane[lane].s + 4u * q);
+      b.s[4 * q] = f.x;
+      b.s[4 * q + 1] = f.y;
+      b.s[4 * q + 2] = f.z;
+      b.s[4 * q + 3] = f.w;
+    }
+  }
+  return b;
+}
+// What is left once the levels below 1024 are in LDS (every level, `put_levels`, where the octets were not taken): the values
 // are final after the caller's next barrier.  Called behind a barrier.
-__device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, uint32_t k, float inv,
-                                            const float (&S)[kRotKMax / 2], bool put_levels) {
+__device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, uint32_t k, float inv, const RotTable* table, const RotBlock& B, bool put_levels) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
   // three levels to a pass, what is over in the last
-  for (uint32_t lg = put_levels ? 0u : 31u - (uint32_t)__builtin_clz(kRotRun); (1u << lg) < m; lg += 3u) {
+  for (uint32_t lg = put_levels ? 0u : 31u - (uint32_t)__builtin_clz(kRotTile); (1u << lg) < m; lg += 3u) {
     const bool last = (8u << lg) >= m;
     const float factor = last && k == 1 ? inv : 1.f;
     if ((m >> lg) >= 8u) rotate_levels<8>(v, n, lg, factor);
@@ -320,6 +424,14 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
     if (tid == 0) v[0] *= inv;
   }
   if (k == 1) return;
+  if (rot_scalars(m, k)) {
+    const float* rows = &table->rows[0][0];
+    if (k == 3u) rotate_columns<3>(v, m, inv, rows);
+    else if (k == 5u) rotate_columns<5>(v, m, inv, rows);
+    else if (k == 7u) rotate_columns<7>(v, m, inv, rows);
+    else rotate_columns<9>(v, m, inv, rows);
+    return;
+  }
   // S (k x k) . C (k x m), the 1 / sqrt m factor first: a wavefront takes 32 columns of C at a time as f32 matrix-core
   // steps of depth 2 (S padded with zeros to 32 x 32; lanes past a narrow m repeat its first column); it reads its columns
   // whole before it writes them, and no other wavefront touches them.
@@ -344,7 +456,7 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
         if (s0 + i >= steps) break;
         float x = c[i] * inv;
         if (s0 + i + 1u == steps) x = lh ? 0.f : x;
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(S[s0 + i], x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(B.s[s0 + i], x, acc, 0, 0, 0);
       }
     }
     // acc[r] is row 8 (r / 4) + 4 lh + r % 4 of column j
@@ -397,7 +509,7 @@ struct RotArgs {
   const __half* x;        // [rows, n]
   void* out;              // [rows, n] f32 or f16
   const uint32_t* signbits;
-  const void* fragments;  // [64] RotFragments
+  const void* fragments;  // RotTable
   uint32_t n, m, k;
   float inv;
   // to the batched kernels' octets (gemm_kernel.h): `rows` of them, `out` takes the columns from `kcols` on
@@ -422,8 +534,9 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
     if (blockIdx.x >= a.rows) return;
   }
   const __half* x = a.x + (size_t)blockIdx.x * n;
-  const RotFragments F = reinterpret_cast<const RotFragments*>(a.fragments)[tid & 63u];
+  const RotTable* table = reinterpret_cast<const RotTable*>(a.fragments);
   if (m >= kRotOctetM) {
+    const rot_h8_t h[2] = {table->lane[tid & 63u].h[0], table->lane[tid & 63u].h[1]};
     const uint8_t* signs = reinterpret_cast<const uint8_t*>(a.signbits);
 #pragma unroll 1
     for (uint32_t tile = tid >> 6; tile * kRotTile < n; tile += 16u) {
@@ -439,13 +552,14 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
       for (uint32_t i = 0; i < 2u; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[i].w[j] = rot_octet_at(tile, i) < n ? flip_signs(o[i].w[j], sg[i], j) : 0u;
-      rotate_tile_to(rot_s, o[0].w, o[1].w, F, tile, n, m, k, a.inv);
+      rotate_tile_to(rot_s, o[0].w, o[1].w, h, tile, n, m, k, a.inv);
     }
   } else {
     for (uint32_t i = tid; i < n; i += 1024) rot_s[i] = flip_sign(__half2float(x[i]), a.signbits[i >> 5] >> (i & 31u), 0);
   }
+  const RotBlock block = rot_block(table, m, k);
   __syncthreads();
-  rotate_rest(rot_s, n, m, k, a.inv, F.s, m < kRotOctetM);
+  rotate_rest(rot_s, n, m, k, a.inv, table, block, m < kRotOctetM);
   __syncthreads();
   constexpr bool kOctets = std::is_same<OutT, RotOctets>::value, kHalf = kOctets || std::is_same<OutT, __half>::value;
   typedef typename std::conditional<kHalf, __half, float>::type out_t;
@@ -494,7 +608,7 @@ struct llvq_rt {
     uint64_t seed = 0;
     float inv = 1.f;
     uint32_t* signbits = nullptr;
-    void* fragments = nullptr;  // [64] RotFragments
+    void* fragments = nullptr;  // RotTable
     float* scratch = nullptr;   // one rotated activation, f32, where rows are too wide to be rotated in a product's launch
   };
   std::vector<DevRotation*> rotations;
@@ -705,7 +819,12 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
   r->n = t.n; r->m = t.m; r->k = t.k; r->seed = seed; r->inv = t.inv;
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&r->signbits), t.signbits.size() * 4);
   if (e == hipSuccess) e = hipMemcpy(r->signbits, t.signbits.data(), t.signbits.size() * 4, hipMemcpyHostToDevice);
-  std::vector<RotFragments> frag(64);
+  std::vector<RotTable> host(1);
+  std::memset(static_cast<void*>(host.data()), 0, sizeof(RotTable));
+  RotFragments* const frag = host[0].lane;
+  if (t.k <= kRotScalarK)
+    for (uint32_t g = 0; g < t.k; ++g)
+      for (uint32_t i = 0; i < t.k; ++i) host[0].rows[g][i] = t.small[(size_t)g * t.k + i];
   const uint32_t inside = std::min(t.m, 32u) - 1u;  // the bits of a column that the transform mixes
   for (uint32_t l = 0; l < 64u; ++l) {
     const uint32_t row = l & 31u, lh = l >> 5;
@@ -720,8 +839,8 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
         frag[l].h[i][e8] = (_Float16)(!same ? 0.f : __builtin_popcount(row & c & inside) & 1 ? -1.f : 1.f);
       }
   }
-  if (e == hipSuccess) e = hipMalloc(&r->fragments, frag.size() * sizeof(RotFragments));
-  if (e == hipSuccess) e = hipMemcpy(r->fragments, frag.data(), frag.size() * sizeof(RotFragments), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMalloc(&r->fragments, sizeof(RotTable));
+  if (e == hipSuccess) e = hipMemcpy(r->fragments, host.data(), sizeof(RotTable), hipMemcpyHostToDevice);
   // (f32 results have the larger planes: where those fit, all do)
   if (e == hipSuccess && !gemv_fits(n, true, true)) e = hipMalloc(reinterpret_cast<void**>(&r->scratch), (size_t)n * sizeof(float));
   if (e != hipSuccess) {

@@ -393,35 +393,40 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
     if (in.x_f32) {
       request();
     } else {
-      const RotFragments F = reinterpret_cast<const RotFragments*>(in.rot_fragments)[lane];
+      const RotTable* table = reinterpret_cast<const RotTable*>(in.rot_fragments);
       const bool norm = in.prologue == kPrologueAddRmsNorm, silu = in.prologue == kPrologueSiluMul;
       auto norm_scale = [&](float ss) {
         ss = wave_sum(ss);
         if (lane == 0) L.red[wave] = ss;
         lds_barrier();
         float total = 0.f;
-        for (uint32_t w = 0; w < waves; ++w) total += L.red[w];
+        for (uint32_t w = 0; w < 16u; ++w) total += L.red[w];
         return 1.0f / sqrtf(total / (float)d_in + in.eps);
       };
       if (in.rot_m >= kRotOctetM) {
-        // Every operand of a wavefront's tile is requested before the first is used; one that is not there reads x.
+        // Every operand of a wavefront's tile is requested before the first is used.
         // (Rows past sixteen tiles: a second turn.  Those have no norm in front: a decoder's hidden size ends at 8192.)
-        const __half* second = in.x2 ? in.x2 : in.x;
-        const __half* third = norm ? in.norm_w : in.x;
         const uint8_t* signs = reinterpret_cast<const uint8_t*>(in.rot_signbits);
-        HalfOctet a[2], b[2], g[2];
-        uint32_t sg[2];
+        HalfOctet a[2] = {}, b[2] = {}, g[2] = {};
+        uint32_t sg[2] = {0, 0};
+        rot_h8_t h[2] = {};
         auto load_tile = [&](uint32_t tile) {
 #pragma unroll
           for (uint32_t i = 0; i < 2u; ++i) {
             const uint32_t from = rot_octet_at(tile, i) < d_in ? rot_octet_at(tile, i) : 0u;
+            if (norm) g[i] = *reinterpret_cast<const HalfOctet*>(in.norm_w + from);
+            if (in.x2) b[i] = *reinterpret_cast<const HalfOctet*>(in.x2 + from);
             a[i] = *reinterpret_cast<const HalfOctet*>(in.x + from);
-            b[i] = *reinterpret_cast<const HalfOctet*>(second + from);
-            g[i] = *reinterpret_cast<const HalfOctet*>(third + from);
             sg[i] = signs[from >> 3];
           }
         };
-        load_tile(wave);
+        // (A wavefront without a tile asks for none: loads of sixteen wavefronts that nobody uses are a microsecond in front of the weights'.)
+        const bool has_tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave) * kRotTile < d_in;
+        if (has_tile) {
+          load_tile(wave);
+          h[0] = table->lane[lane].h[0];
+          h[1] = table->lane[lane].h[1];
+        }
         if constexpr (PMAX <= 2) request();
         __builtin_amdgcn_sched_barrier(0);
         float inv = 0.f;
@@ -446,7 +451,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
         }
 #pragma unroll 1
         for (uint32_t tile = wave; tile * kRotTile < d_in; tile += 16u) {
-          if (tile != wave) load_tile(tile);
+          uint32_t x[2][4];
 #pragma unroll
           for (uint32_t i = 0; i < 2u; ++i) {
             if (silu) {
@@ -459,9 +464,10 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
                 a[i].w[j] = pack_halves(half_lo(a[i].w[j]) * inv * half_lo(g[i].w[j]), half_hi(a[i].w[j]) * inv * half_hi(g[i].w[j]));
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a[i].w[j] = rot_octet_at(tile, i) < d_in ? flip_signs(a[i].w[j], sg[i], j) : 0u;
+            for (int j = 0; j < 4; ++j) x[i][j] = rot_octet_at(tile, i) < d_in ? flip_signs(a[i].w[j], sg[i], j) : 0u;
           }
-          rotate_tile_to(xf, a[0].w, a[1].w, F, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
+          if ((tile + 16u) * kRotTile < d_in) load_tile(tile + 16u);  // (on their way beside this tile's levels)
+          rotate_tile_to(xf, x[0], x[1], h, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
         }
         if constexpr (PMAX > 2) request();  // (no registers for a wide step beside the operands)
       } else {
@@ -484,8 +490,9 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
           request();
         }
       }
+      const RotBlock block = rot_block(table, in.rot_m, in.rot_k);
       lds_barrier();
-      rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, F.s, in.rot_m < kRotOctetM);
+      rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, table, block, in.rot_m < kRotOctetM);
       lds_barrier();
     }
 #pragma unroll 1
