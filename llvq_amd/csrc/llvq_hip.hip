@@ -1157,7 +1157,7 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   a.teams = std::min((a.n_tiles + cus - 1u) / cus, kGemvMaxWaves / a.team);
   const uint32_t grid = std::min(cus, (a.n_tiles + a.teams - 1u) / a.teams);
   a.grid = grid;
-  a.waves = rotated || gemv_wide(a.nb) ? kGemvMaxWaves : a.teams * a.team;
+  a.waves = rotated || gemv_wide(a.nb) ? kGemvMaxWaves : gemv_waves(a.team, a.teams, (a.n_tiles + grid - 1u) / grid);
   a.passes = stage_passes(a.nb, a.waves);
   a.inv_team = (65536u + a.team - 1u) / a.team;
   a.inv_teams = (65536u + a.teams - 1u) / a.teams;

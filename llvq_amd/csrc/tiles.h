@@ -982,8 +982,10 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
   StepWords W[kSteps];
   constexpr uint32_t kFirst = SRC == kSrcRotated ? 1u : kSteps;  // (beside a rotation's operands there are registers for one)
   uint32_t table;
-  // The tile that this wavefront finishes of those whose rounds begin with r0.
-  const uint32_t batch = gemv_batch(a.team), my_round = (wave * a.inv_teams) >> 16, my_team = wave - my_round * a.teams;
+  // The tile that this wavefront finishes of those whose rounds begin with r0: the last wavefronts see to the first tiles, since what a tile
+  // has besides its steps (tile_extras, 0.8 us for one wavefront) is then not in front of anybody's products where there are
+  // wavefronts without any.
+  const uint32_t fin = a.waves - 1u - wave, batch = gemv_batch(a.team), my_round = (fin * a.inv_teams) >> 16, my_team = fin - my_round * a.teams;
   TileExtras extras;
   uint32_t extras_table;
   auto finished = [&](uint32_t r0) { return my_round < batch ? (r0 + my_round) * n_teams + my_team * a.grid + blockIdx.x : 0xFFFFFFFFu; };
