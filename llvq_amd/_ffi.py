@@ -155,6 +155,22 @@ def lib():
     return L
 
 
+_calls = None
+
+
+def calls():
+    """The operator's calls as one native step each (csrc/bind.cpp), bound to the library that is loaded here; None where that module was
+    not built for this interpreter: fused.py then makes them itself.  torch has to be imported."""
+    global _calls
+    if _calls is None and os.path.exists(os.path.join(_HERE, "_calls.so")):
+        from . import _calls as module
+
+        L = lib()
+        module.bind_library(*(C.cast(f, C.c_void_p).value for f in (L.llvq_hip_gemv, L.llvq_hip_gemv_group, L.llvq_hip_gemm, L.llvq_hip_gemm_group)))
+        _calls = module
+    return _calls
+
+
 def check(rc):
     if rc != 0:
         raise LlvqError(rc, (lib().llvq_hip_last_error() or b"").decode("utf-8", "replace"))

@@ -90,6 +90,7 @@ class FusedProj:
     def __init__(self, rt, handle, fm: FusedMatrix):
         self._rt = rt
         self.handle = handle
+        self._at = handle.value  # 0 once freed (_calls reads it)
         self.name = fm.name
         self.d_out, self.d_in = fm.d_out, fm.d_in
         self.nblocks, self.tail_w = fm.nblocks, fm.tail_w
@@ -143,6 +144,8 @@ class FusedRuntime:
         h = C.c_void_p()
         _ffi.check(L.llvq_hip_runtime_create(device, C.c_void_p(stream.cuda_stream), C.byref(h)))
         self.handle = h
+        self._at = h.value
+        self._calls = _ffi.calls()
         self.projs = []
         if model is not None:
             for fm in model.matrices:
@@ -179,6 +182,7 @@ class FusedRuntime:
         if proj.handle:
             _ffi.lib().llvq_hip_matrix_free(self.handle, proj.handle)
             proj.handle = None
+            proj._at = 0
 
     # -- the operator ---------------------------------------------------------------
     def _f16(self, x, proj):
@@ -235,6 +239,10 @@ class FusedRuntime:
 
     def forward(self, proj: FusedProj, x, out_dtype=None):
         """Proj::forward (model.rs:337-345): rotate + forward_rotated in one call."""
+        if self._calls is not None:  # the usual tensors; None: not one of those
+            y = self._calls.forward(self, proj, x, out_dtype)
+            if y is not None:
+                return y
         torch = self._torch
         x = self._f16(x, proj)
         if x.numel() != proj.d_in:
@@ -249,6 +257,10 @@ class FusedRuntime:
 
     def forward_group(self, projs, x, out_dtype=None):
         """group_forward (llvq-llm/src/model.rs:497-536) for projections sharing one activation."""
+        if self._calls is not None:
+            ys = self._calls.forward_group(self, projs, x, out_dtype)
+            if ys is not None:
+                return ys
         launch, ys = self.plan_group(projs, x, out_dtype)
         launch()
         return ys
@@ -308,6 +320,10 @@ class FusedRuntime:
     def forward_batched(self, proj: FusedProj, x, out_dtype=None):
         """Rows of `x` [M, d_in] through one projection (the row loop of model.rs:521-529).  M >= 2: weights are rounded to
         binary16 once where d_in is a multiple of 8 and x starts on a 16-byte boundary; otherwise as exact as `forward`."""
+        if self._calls is not None:
+            y = self._calls.forward_batched(self, proj, x, out_dtype)
+            if y is not None:
+                return y
         torch = self._torch
         if x.dim() != 2 or x.shape[1] != proj.d_in:
             raise ValueError(f"{proj.name} expects [M, {proj.d_in}], got {list(x.shape)}")
@@ -351,6 +367,8 @@ class FusedRuntime:
         """Rows of `x` [M, d_in] through the projections of one group (q/k/v, gate/up) into caller-owned
         [M, d_out_i] tensors of one dtype: one batched launch per run of projections that share a basis
         (the row loop of group_forward, model.rs:497-536)."""
+        if self._calls is not None and self._calls.forward_batched_group_into(self, projs, x, ys):
+            return ys
         torch = self._torch
         if len(projs) != len(ys) or not projs:
             raise ValueError("one output per projection")
@@ -399,6 +417,7 @@ class FusedRuntime:
                 self.free(p)
             _ffi.lib().llvq_hip_runtime_destroy(self.handle)
             self.handle = None
+            self._at = 0
 
     def __del__(self):
         try:
