@@ -266,7 +266,15 @@ struct GemmArgs {
   uint32_t ldx, tail_w;
   uint32_t M, m_pad, nb;
   uint32_t m_tiles, splits, steps_per_split;  // the wide kernel's grid
+  // Where gemm_tiles_kernel finds octet j of block k of unit q of row m: xs + q * xs_unit + k * xs_block + j * xs_octet + m * xs_row, rows
+  // past xs_last being that one.
+  const uint8_t* xs;
+  uint32_t xs_unit, xs_block, xs_octet, xs_row, xs_last;
 };
+// All arguments asked for at once (as touch_args does for the batch-1 products').
+__device__ __forceinline__ void touch_args(const GemmArgs& a) {
+  asm volatile("" ::"s"(a.ws), "s"(a.mat[1].base), "s"(a.mat[3].base), "s"(a.M), "s"(a.xs_last));
+}
 
 struct GemmTile {
   const uint8_t* base;
@@ -308,7 +316,8 @@ __device__ __forceinline__ uint32_t lane_offset(uint32_t v) {
 // flight while the step before is multiplied, and the sixteen partial sums meet in LDS: no workspace, no second kernel.
 // RG = 1, MT = 1: up to 16 rows of activations; RG = 2, MT = 4: up to 64 (two row groups share the activation
 // fragments, whose way from L2 would bind otherwise).
-// 2560 x 2560 at 5 rows: 35.9 -> 10.4 us; rotated q, k, v of 2560 columns at 64 rows, rotation included: 58.1 -> 21.7 us
+// Of few rows the octets are read from the rows themselves (gemm_direct in llvq_hip.hip has the rule, and both sides' times).
+// 2560 x 2560 at 5 rows: 35.9 -> 10.4 us (6.7 -> 4.7 with that, between the native calls); rotated q, k, v of 2560 columns at 64 rows, rotation included: 58.1 -> 21.7 us
 // (before: codes unranked in the product, partial sums through memory).
 // PAIR: both terms of the weights (dequant_octet_pair), 32 columns to a product sum that starts from zero, those added in
 // f64; RG = 1 always, two row groups would not fit the registers.  4097 columns, 1024 rows by 64: 16 -> 14 us (twice the
@@ -316,6 +325,7 @@ __device__ __forceinline__ uint32_t lane_offset(uint32_t v) {
 template <int RG, int MT, bool PAIR>
 __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   extern __shared__ __align__(16) uint8_t smem[];
+  touch_args(a);
   constexpr uint32_t kRows = RG * 16, kCols = MT * 16;
   float* part = reinterpret_cast<float*>(smem);           // [16 wavefronts][RG][MT][64 lanes][4]
   float* tw = part + 16 * RG * MT * 256;                  // [kRows][24] tail weights
@@ -332,7 +342,7 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   const float entry = __uint_as_float(scale_table(t.base, lane));
   const uint32_t d_off = head + (m16 & 7u) * 16u + ((m16 >> 3) * 2u + (g >> 1)) * 128u + (g & 1u) * 8u;
   const uint32_t m_off = head + (m16 & 7u) * 16u + 512u + (m16 >> 3) * 8u;
-  const uint32_t x_off = (g * 3u * a.m_pad + m16) * 16u, x_oct = a.m_pad * 16u;
+  const uint32_t x_row = MT == 1 ? min(m16, a.xs_last) * a.xs_row : m16 * 16u, x_off = x_row + g * a.xs_block;
 
   struct Words { u32x2_t d, m; } W[RG];
   u32x4_t X[3][MT];
@@ -347,10 +357,15 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
   };
   auto load_x = [&](uint32_t j, uint32_t q, bool live) {
     const uint32_t keep = live ? 0xFFFFFFFFu : 0u;
-    const uint8_t* p = uniform_global(reinterpret_cast<const uint8_t*>(a.xt) + ((size_t)(q * 12u + j) * x_oct & (size_t)(int64_t)(int32_t)keep));
-    const uint32_t off = lane_offset(x_off & keep);
+    const uint8_t* p = uniform_global(a.xs + (((size_t)q * a.xs_unit + j * a.xs_octet) & (size_t)(int64_t)(int32_t)keep));
+    uint32_t off = x_off;
+    if (MT == 1 && 4u * q + 4u > nb) off = x_row + min(g, nb - 1u - min(4u * q, nb - 1u)) * a.xs_block;  // (in the last unit: a block that is there)
+    off = lane_offset(off & keep);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) X[j][mt] = *reinterpret_cast<const u32x4_t*>(p + off + (uint32_t)mt * 256u);
+    for (int mt = 0; mt < MT; ++mt) {
+      const HalfOctet o = *reinterpret_cast<const HalfOctet*>(p + off + (uint32_t)mt * 256u);
+      X[j][mt] = u32x4_t{o.w[0], o.w[1], o.w[2], o.w[3]};
+    }
   };
   // The row scales and the tail's operands, needed at the end: asked for first.
   const uint32_t op_row = tid % kRows, op_col = tid / kRows;  // column 24: the row's scale
@@ -404,6 +419,11 @@ __global__ __launch_bounds__(1024) void gemm_tiles_kernel(GemmArgs a) {
     }
   }
   for (; q < n_quads; q += 16u) {
+    if (MT == 1 && 4u * q + 4u > nb) {  // octets of blocks that are not there are zero, and their weights are
+      const uint32_t there = 4u * q + g < nb ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+      for (uint32_t j = 0; j < 3; ++j) X[j][0] &= there;
+    }
     const uint32_t qn = q + 16u;
     const bool live = qn < n_quads;
     BlockScale s[RG];

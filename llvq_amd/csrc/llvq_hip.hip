@@ -1662,6 +1662,16 @@ static int reserve_batched(llvq_rt* rt, const llvq_mat* const* mats, int n, uint
   return rc;
 }
 
+// Whether gemm_tiles_kernel reads a small batch where it is, so that no launch makes octets of it (2.2 us).  A load of sixteen rows' pieces
+// then meets as many lines as there are rows, three of which cost nothing and each other one 0.065 us for each unit of a wavefront: direct /
+// by octets, in us, 4096 x 4096 at 2, 5, 10 and 16 rows 5.4 / 7.5, 5.4 / 7.5, 6.3 / 7.4, 7.4 / 7.5; 12288 x 4096 10.2 / 12.0, 11.3 / 12.1,
+// 14.1 / 12.1, 17.4 / 12.2; 2560 x 9728 7.7 / 10.0, 8.4 / 9.8, 10.5 / 9.9, 13.0 / 10.0; 5120 x 17408 19.6 / 21.7, 22.7 / 21.7.  Rows off 16-byte
+// boundaries, where a piece is two lines, gain at 2 rows (4096 x 4097 8.4 / 8.8) and lose from 4 (9.6 / 8.3).
+static bool gemm_direct(uint32_t M, uint32_t n_tiles, uint32_t nb, uint32_t cus, bool pair) {
+  if (pair || M > 16u) return false;
+  const uint32_t units = (n_tiles + cus - 1u) / cus * tile_units(nb);  // of the fullest CU
+  return M <= 3u || (M - 3u) * units < 20u * 16u;
+}
 // One launch over n <= kGemmMaxGroup matrices of equal d_in that take the same activations
 // (already in the matrices' basis), M <= kGemmMaxM rows.  from: rows that are rotated on the way to the octets, their tail
 // columns to x.
@@ -1698,6 +1708,13 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   a.m_tiles = p.m_tiles;
   a.splits = p.splits;
   a.steps_per_split = p.steps_per_split;
+  const bool direct = !from && p.small == 1u && gemm_direct(M, a.n_tiles, a.nb, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), pair);
+  a.xs = direct ? reinterpret_cast<const uint8_t*>(x) : reinterpret_cast<const uint8_t*>(xt_buf);
+  a.xs_octet = direct ? 16u : p.m_pad * 16u;
+  a.xs_block = 3u * a.xs_octet;
+  a.xs_unit = 4u * a.xs_block;
+  a.xs_row = direct ? a.ldx * 2u : 16u;
+  a.xs_last = direct ? M - 1u : 15u;
   if (from) {
     RotArgs ra = rot_args(m0->rot, from, const_cast<void*>(x));
     ra.xt = reinterpret_cast<uint4*>(xt_buf);
@@ -1706,7 +1723,7 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
     ra.n_oct = p.n_oct;
     ra.kcols = a.nb * kDim;
     hipLaunchKernelGGL(rotate_kernel<RotOctets>, dim3(p.m_pad), dim3(1024), (size_t)ra.n * sizeof(float), rt->stream, ra);
-  } else {
+  } else if (!direct) {
     const uint32_t oct_waves = (p.n_oct + 7u) / 8u * (p.m_pad / 8u);
     hipLaunchKernelGGL(tile_activations_kernel, dim3((oct_waves + 3u) / 4u), dim3(256), 0, rt->stream, xh, M, a.ldx, a.nb * 24u, p.m_pad, p.n_oct,
                        reinterpret_cast<uint4*>(xt_buf));

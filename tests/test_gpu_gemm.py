@@ -393,3 +393,30 @@ def test_gemm_wide_stores_into_an_output_that_is_only_element_aligned(gpu_rt, d_
             assert bool(torch.isnan(buf[0])) and bool(torch.isnan(buf[1 + M * d_out:]).all())
     finally:
         gpu_rt.free(proj)
+
+
+# rows read where they are (up to three whatever the size; more of small products): 1, 2, 3, 4, 5 blocks (a unit of four, whole and not), units
+# for all sixteen wavefronts and one over, two tiles and a ragged one, and a product on either side of the rule's line
+@pytest.mark.parametrize("d_out,d_in", [(16, 24), (24, 64), (40, 72), (16, 96), (33, 136), (48, 1536), (16, 1568), (72, 2560)])
+@pytest.mark.parametrize("rows", [2, 3, 4, 13, 16])
+def test_small_batches_read_their_rows_and_no_others(gpu_rt, orc, d_out, d_in, rows):
+    import torch
+
+    raw = synth.make_matrix(f"model.layers.0.d{d_out}.{d_in}.weight", d_out, d_in, seed=d_in)
+    proj = gpu_rt.upload(raw)
+    try:
+        X = synth.make_activation(d_in, seed=rows, rows=rows)
+        x = _x16(X)
+        Y_ref, A_ref = _reference(orc, raw, X)
+        clean = gpu_rt.forward_batched(proj, x, out_dtype=torch.float32)
+        _check(clean.cpu().numpy(), Y_ref, A_ref)
+        # what lies behind a row, whatever it is, reaches nothing of it
+        for first in (0, 1):
+            dirty = x.clone()
+            dirty[first::2] = float("nan")
+            dirty[first::4] = float("inf")
+            got = gpu_rt.forward_batched(proj, dirty, out_dtype=torch.float32)
+            assert torch.equal(got[1 - first::2], clean[1 - first::2])
+            assert not torch.isfinite(got[first::2]).any()
+    finally:
+        gpu_rt.free(proj)
