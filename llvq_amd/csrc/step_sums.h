@@ -44,6 +44,15 @@ LLVQ_HD uint32_t gemv_waves(uint32_t team, uint32_t teams, uint32_t tiles) {
 LLVQ_HD uint32_t sums_steps(bool wide) { return kGemvMaxWaves * (wide ? kGemvWideSteps : 1u); }
 LLVQ_HD uint32_t sums_at(uint32_t round, uint32_t team_index, uint32_t team, bool wide) { return round * sums_steps(wide) + team_index * team; }
 LLVQ_HD uint32_t sums_room(bool wide) { return kGemvRounds * sums_steps(wide) + (wide ? 0u : kGemvMaxWaves); }
+// Gate and up as one result (tiles_product, GATED): where the scales and extras of a wavefront's sixteen rows are, and how many teams a
+// workgroup has for `slots` tiles.  A pair's two tiles are finished together, so the teams' tiles of a batch of rounds are an even number.
+LLVQ_HD uint32_t gated_at(bool wide) { return sums_room(wide) * kTileRows; }
+constexpr uint32_t kGatedFloats = kGemvMaxWaves * kTileRows * 2;
+LLVQ_HD uint32_t gated_teams(uint32_t slots, uint32_t team) {
+  const uint32_t most = kGemvMaxWaves / team, teams = slots < most ? slots : most;
+  if (!((gemv_batch(team) * teams) & 1u)) return teams;
+  return teams < most ? teams + 1u : teams - 1u;  // (such a team is of seven wavefronts at the most: most >= 2)
+}
 // The step that a lane of class c reads as its i-th.
 LLVQ_HD uint32_t sums_read(uint32_t i, uint32_t c) { return 4u * i + c; }
 // In LDS the four blocks of a unit lie together: 3 dwords per digit and block, then each block's sum of its integers
@@ -57,9 +66,9 @@ LLVQ_HD uint32_t gemv_plane_units(uint32_t nb) { return (tile_steps(nb) + 1u) * 
 LLVQ_HD uint32_t gemv_lds_fixed() { return 128u + 64u; }
 // The rotated activation and the sums share their place: rows of 20480 columns with f32 results, 24576 with binary16, are the widest that
 // fit (160 KB).  One behind the other, 19456 and 20480 columns with f32 results and 23552 with binary16 took a launch more, 3.6 to 4 us.
-inline uint64_t gemv_tiles_lds_bytes(uint32_t nb, uint32_t d_in, bool f32_out, bool rotated) {
+inline uint64_t gemv_tiles_lds_bytes(uint32_t nb, uint32_t d_in, bool f32_out, bool rotated, bool gated = false) {
   const uint64_t planes = (uint64_t)gemv_plane_units(nb) * (f32_out ? XPlanes<6>::kDwords : XPlanes<4>::kDwords) * 4;
-  const uint64_t sums = sums_room(gemv_wide(nb)) * kTileRows * 4, values = rotated ? ((uint64_t)d_in * 4 + 31) / 16 * 16 : 0;
+  const uint64_t sums = sums_room(gemv_wide(nb)) * kTileRows * 4 + (gated ? kGatedFloats * 4 : 0), values = rotated ? ((uint64_t)d_in * 4 + 31) / 16 * 16 : 0;
   return gemv_lds_fixed() + planes + (sums > values ? sums : values);
 }
 

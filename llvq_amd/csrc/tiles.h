@@ -315,8 +315,9 @@ struct GemvArgs {
   uint32_t nb, tail_w, n_mats, n_tiles;
   uint32_t team, teams;  // wavefronts of a team, teams of a workgroup (more wavefronts only stage the activation)
   // What the host knows as well, so that no wavefront works it out: its workgroup's wavefronts, the workgroups, how often the former
-  // pass over the activation, 2^16 / team and 2^16 / teams, rounded up (exact for the sixteen numbers that are divided).
+  // pass over the activation, 2^16 / team and 2^16 / teams, rounded up (exact for the seventeen numbers that are divided).
   uint32_t waves, grid, passes, inv_team, inv_teams;
+  uint32_t rounds;  // tiles of a team, at the most
   TileMat m[kMaxGroup];
 };
 // Asks for all of a launch's arguments at once: each of their cache lines is a miss of its own, and the compiler would load
@@ -954,8 +955,13 @@ __device__ __forceinline__ void tile_mat(const GemvArgs& a, uint32_t tile, const
 // the two rows a lane has.  The sums over a team's wavefronts wait in LDS for one barrier per gemv_batch tiles, behind which
 // every wavefront finishes one.  The host spreads teams over the CUs first, tiles over teams so that the last, partial round
 // meets every CU.
-template <typename OutT, int SRC, bool WIDE>
-__global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
+//
+// GATED: the two matrices are a layer's gate and up, and what is stored is f16(f16(silu(gate)) up) of their rows, both rounded to
+// binary16 first (model.rs:831): the bits that the product behind it makes of the two results otherwise, in every one of its workgroups
+// (two passes of an exponential and a division for 9728 columns, 2.4 us).  A row's two tiles are neighbouring slots of one workgroup; the
+// wavefront of the up tile leaves its scales and extras in LDS in front of the barrier that is there anyway.
+template <typename OutT, int SRC, bool WIDE, bool GATED>
+__device__ __forceinline__ void tiles_product(const GemvArgs& a) {
   constexpr int DIG = std::is_same<OutT, __half>::value ? 4 : 6;
   constexpr uint32_t kSteps = WIDE ? kGemvWideSteps : 1u;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -967,18 +973,29 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
   const uint32_t nb = a.nb, n_steps = tile_steps(nb), units = tile_units(nb), head = tile_head_bytes(a.tail_w);
 
   struct Record { const uint8_t* rec; const uint8_t* base; uint32_t slots; };
-  auto record_of = [&](uint32_t t) {
+  // A workgroup's slot i of tiles is tile i * grid + its number; with GATED that tile of pairs of slots, the even one in the first matrix.
+  const uint32_t n_tiles = GATED ? a.m[1].tile_begin : a.n_tiles;
+  auto tile_of = [&](uint32_t slot) { return (GATED ? slot >> 1 : slot) * a.grid + blockIdx.x; };
+  auto record_of = [&](uint32_t t, uint32_t slot) {
     const uint8_t* base;
     void* y;
     uint32_t row0, d_out, stride, slots;
-    tile_mat(a, t, base, y, row0, d_out, stride, slots);
+    if constexpr (GATED) {
+      const bool up = slot & 1u;
+      base = up ? a.m[1].base : a.m[0].base;
+      stride = up ? a.m[1].stride : a.m[0].stride;
+      slots = up ? a.m[1].slots : a.m[0].slots;
+      row0 = t * kTileRows;
+    } else {
+      tile_mat(a, t, base, y, row0, d_out, stride, slots);
+    }
     return Record{base + kTileTableBytes + (size_t)(row0 / kTileRows) * stride, base, slots};
   };
   uint32_t off[kSteps];  // (where a wavefront has no step, or no next tile, its loads repeat one: one cache line, and no branch)
 #pragma unroll
   for (uint32_t j = 0; j < kSteps; ++j) off[j] = step_offset(w + j * kGemvMaxWaves, units, head, lane);
-  uint32_t tile = team < a.teams ? team * a.grid + blockIdx.x : 0xFFFFFFFFu;
-  Record cur = record_of(min(tile, a.n_tiles - 1u));
+  uint32_t tile = team < a.teams ? tile_of(team) : 0xFFFFFFFFu;
+  Record cur = record_of(min(tile, n_tiles - 1u), team);
   StepWords W[kSteps];
   constexpr uint32_t kFirst = SRC == kSrcRotated ? 1u : kSteps;  // (beside a rotation's operands there are registers for one)
   uint32_t table;
@@ -988,39 +1005,42 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
   const uint32_t fin = a.waves - 1u - wave, batch = gemv_batch(a.team), my_round = (fin * a.inv_teams) >> 16, my_team = fin - my_round * a.teams;
   TileExtras extras;
   uint32_t extras_table;
-  auto finished = [&](uint32_t r0) { return my_round < batch ? (r0 + my_round) * n_teams + my_team * a.grid + blockIdx.x : 0xFFFFFFFFu; };
+  auto finished = [&](uint32_t r0) { return my_round < batch ? tile_of(r0 * a.teams + fin) : 0xFFFFFFFFu; };
   auto load_finish = [&](uint32_t r0) {
     const uint32_t t = finished(r0);
-    const Record r = record_of(min(t, a.n_tiles - 1u));
-    extras = load_extras(r.rec, nb, a.tail_w, r.slots, t < a.n_tiles, lane);
+    const Record r = record_of(min(t, n_tiles - 1u), fin);  // (a batch of rounds has an even number of slots where that matters: gated_teams)
+    extras = load_extras(r.rec, nb, a.tail_w, r.slots, t < n_tiles, lane);
     extras_table = scale_table(r.base, lane);
   };
   stage_x<DIG, SRC, WIDE ? 4 : 2>(a.in, nb, a.tail_w, a.waves, a.passes, L, blockIdx.x == 0, [&]() {
     if constexpr (SRC != kSrcRotated) load_finish(0);  // little, and it has a use while the pieces come
     table = scale_table(cur.base, lane);
     const uint8_t* base = scalar_base(cur.rec);
-    const uint32_t keep = tile < a.n_tiles ? 0xFFFFFFFFu : 0u;
+    const uint32_t keep = tile < n_tiles ? 0xFFFFFFFFu : 0u;
 #pragma unroll
     for (uint32_t j = 0; j < kFirst; ++j) load_step(W[j], base, off[j] & keep);
   });
-  if constexpr (kFirst != kSteps) load_step(W[1], scalar_base(cur.rec), off[1] & (tile < a.n_tiles ? 0xFFFFFFFFu : 0u));
+  if constexpr (kFirst != kSteps) load_step(W[1], scalar_base(cur.rec), off[1] & (tile < n_tiles ? 0xFFFFFFFFu : 0u));
   if constexpr (SRC == kSrcRotated) load_finish(0);
   lds_barrier();
 
-  const uint32_t rounds = (a.n_tiles + n_teams - 1u) / n_teams;
+  // (In a rotated basis there is no scalar register to keep it in: 2560 x 9728 takes 11.5 us like this, 11.8 with the argument.)
+  const uint32_t rounds = SRC == kSrcRotated ? (a.n_tiles + n_teams - 1u) / n_teams : a.rounds;
   for (uint32_t r0 = 0; r0 < rounds; r0 += batch) {
     const uint32_t r1 = min(r0 + batch, rounds), o_tile = finished(r0);
     const float o_scale = extras.scale;
     float o_extra = 0.f;
-    if (o_tile < a.n_tiles) {
-      const Record r = record_of(o_tile);
+    if (o_tile < n_tiles) {
+      const Record r = record_of(o_tile, fin);
       o_extra = tile_extras<DIG>(extras, r.rec, nb, a.tail_w, r.slots, extras_table, L, lane);
     }
+    if constexpr (GATED)
+      if ((fin & 1u) && lane_class(lane) == 0u) *reinterpret_cast<float2*>(L.part + gated_at(WIDE) + (fin * kTileRows + lane_row(lane)) * 2u) = make_float2(o_scale, o_extra);
     if (r1 != rounds) load_finish(r1);
-    for (uint32_t rd = r0; rd < r1 && tile < a.n_tiles; ++rd) {
-      const uint32_t next = tile + n_teams;
-      const bool more = next < a.n_tiles;
-      const Record nx = record_of(min(next, a.n_tiles - 1u));
+    for (uint32_t rd = r0; rd < r1 && tile < n_tiles; ++rd) {
+      const uint32_t next = GATED ? tile_of((rd + 1u) * a.teams + team) : tile + n_teams;
+      const bool more = next < n_tiles;
+      const Record nx = record_of(min(next, n_tiles - 1u), (rd + 1u) * a.teams + team);
       const uint32_t lanes_table = table, keep = more ? 0xFFFFFFFFu : 0u;
       const uint8_t* base = scalar_base(nx.rec);
       float* const part = L.part + sums_at(rd - r0, team, a.team, WIDE) * kTileRows;
@@ -1038,7 +1058,18 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
     }
     // A wavefront per tile of these rounds: everything but the sums themselves is scalar.
     lds_barrier();
-    if (o_tile < a.n_tiles) {
+    if constexpr (GATED) {
+      if (o_tile < n_tiles && !(fin & 1u)) {
+        auto sum_of = [&](uint32_t slot) {
+          const uint32_t round = (slot * a.inv_teams) >> 16;
+          return steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(round, slot - round * a.teams, a.team, WIDE) * kTileRows, n_steps, lane);
+        };
+        const float2 up_scale = *reinterpret_cast<const float2*>(L.part + gated_at(WIDE) + ((fin + 1u) * kTileRows + lane_row(lane)) * 2u);
+        const float gate = fmaf(sum_of(fin), o_scale, o_extra), up = fmaf(sum_of(fin + 1u), up_scale.x, up_scale.y);
+        const uint32_t row = o_tile * kTileRows + lane_row(lane);
+        if (lane_class(lane) == 0u && row < a.m[0].d_out) store_out<OutT>(a.m[0].y, row, silu_mul(round_half(gate), round_half(up)));
+      }
+    } else if (o_tile < n_tiles) {
       const uint8_t* o_base;
       void* o_y;
       uint32_t o_row0, o_d_out, o_stride, o_slots;
@@ -1050,6 +1081,11 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) {
     if (r1 != rounds) lds_barrier();
   }
 }
+
+template <typename OutT, int SRC, bool WIDE>
+__global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) { tiles_product<OutT, SRC, WIDE, false>(a); }
+// gate and up; y of the first matrix takes the result.
+__global__ __launch_bounds__(1024) void gated_product_kernel(GemvArgs a) { tiles_product<__half, kSrcAddRmsNorm, false, true>(a); }
 
 template <typename OutT, bool WIDE>
 __host__ const void* gemv_kernel_of(int src) {
@@ -1066,6 +1102,7 @@ __host__ inline const void* gemv_kernel(bool f32, int src, bool wide) {
 }
 template <class Fn>
 __host__ void for_each_gemv_kernel(Fn&& fn) {
+  fn(reinterpret_cast<const void*>(gated_product_kernel));
   for (int src = kSrcF16; src <= kSrcAddRmsNorm; ++src)
     for (int v = 0; v < 4; ++v) fn(gemv_kernel(v & 1, src, v & 2));
 }

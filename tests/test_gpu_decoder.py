@@ -695,3 +695,28 @@ def test_head_rows_and_chunks(gpu_rt, hidden, vocab, int8):
             assert best == int(np.argmax(got))
     finally:
         dec.close()
+
+
+# a team of 1, 2, 3 (odd: teams are made even), 5, 7 and 11 wavefronts (one team: rounds are), rows past the last tile, one and two pairs of
+# tiles to a workgroup, several batches of rounds
+@pytest.mark.parametrize("hidden,inter", [(200, 24), (1032, 4400), (1632, 40), (1632, 4400), (2408, 328), (3600, 328), (5208, 4104), (8192, 72), (200, 24000)])
+def test_gate_and_up_as_one_result(gpu_rt, hidden, inter):
+    """silu(gate) up formed where gate and up are finished, against the two results taken apart again by down_proj's launch (as sequences of
+    one item do): the same bits."""
+    from llvq_amd import _ffi
+
+    cfg = decoder.Qwen3Config(num_hidden_layers=1, hidden_size=hidden, num_attention_heads=2, num_key_value_heads=1, head_dim=64, intermediate_size=inter,
+                              vocab_size=96, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=8, tie_word_embeddings=True)
+    raws = decoder.synthetic_projections(cfg, hidden + inter)
+    weights = decoder.synthetic_weights(cfg, 3)
+    projs = [[gpu_rt.upload(m) for m in layer] for layer in raws]
+    decs = [decoder.Decoder(gpu_rt, cfg, projs, weights, launch_mode=m) for m in (_ffi.LAUNCH_PER_GROUP, _ffi.LAUNCH_SINGLE)]
+    try:
+        for t in (5, 95, 0):
+            (a, ta), (b, tb) = (d.forward_token(t) for d in decs)
+            assert ta == tb and np.isfinite(a).all() and np.array_equal(a, b)
+    finally:
+        for d in decs:
+            d.close()
+        for p in projs[0]:
+            gpu_rt.free(p)
