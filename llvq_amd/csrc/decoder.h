@@ -205,6 +205,8 @@ struct AttnNew {
 
 constexpr int kAttnThreads = 256;
 constexpr int kAttnWaves = kAttnThreads / 64;
+constexpr uint32_t kAttnClasses = 4 * kAttnWaves;  // position classes of a workgroup, 16 lanes each
+constexpr int kAttnRows = 4;                       // positions of a class whose rows are requested together
 constexpr int kAttnMaxSplits = 64;  // the cache is cut into at most this many ranges (host picks by length; 128 was measured slower at 8188 positions)
 constexpr int kAttnMaxGroup = 8;    // query heads per kv head
 constexpr int kAttnInlineSplits = 16;  // up to this many ranges, the workgroup that finishes last merges them itself
@@ -639,17 +641,15 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
                                                                    const __half* __restrict__ vcache, KvQ8 q8,
                                                                    __half* __restrict__ ctx,
                                                                    float* part, uint32_t* __restrict__ counters,
-                                                                   uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
+                                                                   uint32_t groups, uint32_t chunk, uint32_t head_dim,
                                                                    uint32_t T, uint32_t max_pos, float scale, uint32_t n_splits,
                                                                    uint32_t merge_inline) {
   extern __shared__ __align__(16) float att_smem[];
   __shared__ uint32_t arrived;
   __shared__ float stage[kAttnWaves][256];  // one head per wavefront while it is normed and rotated
   __shared__ float knew[256], vnew[256];    // the new position's k and v as the cache returns them
-  const uint32_t kvh = blockIdx.x / n_splits, split = blockIdx.x % n_splits;
+  const uint32_t kvh = blockIdx.y, split = blockIdx.x;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t groups = n_heads / n_kv;  // <= kAttnMaxGroup (checked by the host)
-  const uint32_t chunk = (T + n_splits - 1) / n_splits;
   const uint32_t j0 = min(T, split * chunk), j1 = min(T, j0 + chunk), nj = j1 - j0;
   float* qs = att_smem;                         // [groups][head_dim]
   float* cls = qs + groups * head_dim;          // the wavefronts' results
@@ -668,7 +668,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
   const bool has_new = nj > 0 && j1 == T;
   const uint32_t newj = has_new ? pos : 0xFFFFFFFFu;
   // Lane (pj, sub) = (lane / 16, lane % 16) of wavefront w holds dims [8 sub, 8 sub + 8) of the
-  // positions of class c = 4 w + pj: jj = c, c + 16, ...  U rows of K and of V are requested
+  // positions of class c = 4 w + pj: jj = c, c + kAttnClasses, ...  U rows of K and of V are requested
   // together.  The loads are unconditional (a lane with no row, or with the row this launch
   // appends, re-reads a valid one and ignores it): a guarded load would be waited for where it
   // is issued, and the first batch is issued here, ahead of the work on the query heads, which
@@ -676,13 +676,13 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
   const uint32_t sub = lane & 15u, pj = lane >> 4, i0 = sub * 8u, c = wave * 4u + pj;
   const bool active = i0 < head_dim;
   const uint32_t i0c = active ? i0 : 0u;
-  constexpr int U = 4;
+  constexpr int U = kAttnRows;
   uint4 kraw[U], vraw[U];
   float ksc[U], kbi[U], vsc[U], vbi[U];
   auto request = [&](uint32_t jb) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint32_t j = min(j0 + jb + 16u * u, pos);
+      const uint32_t j = min(j0 + jb + kAttnClasses * u, pos);
       if constexpr (Q8) {
         const uint2 kc = *reinterpret_cast<const uint2*>(Kq + (size_t)j * head_dim + i0c);
         const uint2 vc = *reinterpret_cast<const uint2*>(Vq + (size_t)j * head_dim + i0c);
@@ -798,11 +798,11 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
       qv[g][t] = ((uint32_t)g < groups && active) ? qs[g * head_dim + i0 + t] : 0.f;
     }
   }
-  for (uint32_t jb = c; jb < nj; jb += 16u * U) {
+  for (uint32_t jb = c; jb < nj; jb += kAttnClasses * U) {
     float sc[U][G], vfs[U][8];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint32_t jj = jb + 16u * u;
+      const uint32_t jj = jb + kAttnClasses * u;
       // A row past the range is one of the row this launch is about to write: whatever an earlier use of the cache left.
       // Its weight is zero, and its values have to be as well: 0 x infinity would reach the sums.
       if (jj >= nj) {
@@ -842,14 +842,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
         sc[u][g] = row16_sum(d);
       }
     }
-    if (jb + 16u * U < nj) request(jb + 16u * U);
+    if (jb + kAttnClasses * U < nj) request(jb + kAttnClasses * U);
     // the batch's maximum first, so that its exponentials do not wait for each other
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       float mn = m[g];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        sc[u][g] = jb + 16u * u < nj ? sc[u][g] : -INFINITY;
+        sc[u][g] = jb + kAttnClasses * u < nj ? sc[u][g] : -INFINITY;
         mn = fmaxf(mn, sc[u][g]);
       }
       const float e0 = __expf(m[g] - mn);  // 0 on the first batch (m = -inf)
@@ -871,9 +871,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
   }
   // A wavefront's four classes meet by lane moves; every sixteen lanes then hold the sums, and lanes 16 (g mod 4) on put
   // head g's down.  (A class with no position: maximum -inf, weight 0.)
-  float* wmax = cls;                                       // [4 wavefronts][groups] running maximum,
+  float* wmax = cls;                                       // [wavefronts][groups] running maximum,
   float* wsum = wmax + kAttnWaves * groups;                // sum of exponentials,
-  float* wacc = qs + ((groups * head_dim + 2u * kAttnWaves * groups + 3u) & ~3u);  // [4][groups][head_dim] weighted V sums
+  float* wacc = qs + ((groups * head_dim + 2u * kAttnWaves * groups + 3u) & ~3u);  // [wavefronts][groups][head_dim] weighted V sums
   // (Heads four at a time: a move across half the wavefront leaves each half two heads of both, one across a quarter
   // each quarter its own head of all four.)
   auto swap32 = [](float a, float b, auto op) {

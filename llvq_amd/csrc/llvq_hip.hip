@@ -2201,8 +2201,8 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     nw.vcache = vc;
     nw.eps = d->eps;
     auto attend = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(d->n_kv * n_splits), dim3(kAttnThreads), attn_lds, st, nw, kc, vc, lq8, d->ctx, d->attn_part,
-                         d->attn_counters, d->n_heads, d->n_kv, d->head_dim, T, d->max_pos, 1.0f / sqrtf((float)d->head_dim), n_splits,
+      hipLaunchKernelGGL(kernel, dim3(n_splits, d->n_kv), dim3(kAttnThreads), attn_lds, st, nw, kc, vc, lq8, d->ctx, d->attn_part,
+                         d->attn_counters, groups_per_kv, (T + n_splits - 1) / n_splits, d->head_dim, T, d->max_pos, 1.0f / sqrtf((float)d->head_dim), n_splits,
                          merge_inline);
     };
     if (d->kv_q8) {
