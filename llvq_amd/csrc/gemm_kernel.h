@@ -30,17 +30,24 @@ constexpr uint32_t kGemmTileRowsSmall = 16; // weight rows of a fragment there
 
 // ---- activations as column octets ----------------------------------------------------------------
 // One lane per octet; a wavefront takes eight octets of eight rows: 128 consecutive bytes of a row read, 128 of the copy
-// written.  Rows from M on and columns from kcols on are zero.
-__global__ __launch_bounds__(256) void tile_activations_kernel(const __half* __restrict__ x, uint32_t M, uint32_t ldx, uint32_t kcols,
-                                                               uint32_t m_pad, uint32_t n_oct, uint4* __restrict__ xt) {
+// written.  Rows from M on and columns from kcols on are zero.  gate: the activations are f16(silu(gate)) x, and their tail columns
+// go to `rows` (octets past the copy's have lanes of their own).
+__global__ __launch_bounds__(256) void tile_activations_kernel(const __half* __restrict__ x, const __half* __restrict__ gate, __half* __restrict__ rows,
+                                                               uint32_t M, uint32_t ldx, uint32_t kcols, uint32_t m_pad, uint32_t n_oct, uint4* __restrict__ xt) {
   const uint32_t lane = threadIdx.x & 63u, wave = blockIdx.x * 4u + (threadIdx.x >> 6);
   const uint32_t groups_m = m_pad >> 3;
   const uint32_t gc = wave / groups_m, gm = wave - gc * groups_m;
   const uint32_t c = gc * 8u + (lane & 7u), m = gm * 8u + (lane >> 3);
   uint4 v = make_uint4(0, 0, 0, 0);
-  if (m < M && c * 8u < kcols) {
-    const HalfOctet o = *reinterpret_cast<const HalfOctet*>(x + (size_t)m * ldx + c * 8u);
-    v = make_uint4(o.w[0], o.w[1], o.w[2], o.w[3]);
+  if (m < M && c * 8u < (gate ? ldx : kcols)) {
+    HalfOctet o = *reinterpret_cast<const HalfOctet*>(x + (size_t)m * ldx + c * 8u);
+    if (gate) {
+      const HalfOctet g = *reinterpret_cast<const HalfOctet*>(gate + (size_t)m * ldx + c * 8u);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o.w[j] = pack_halves(silu_mul(half_lo(g.w[j]), half_lo(o.w[j])), silu_mul(half_hi(g.w[j]), half_hi(o.w[j])));
+    }
+    if (c * 8u < kcols) v = make_uint4(o.w[0], o.w[1], o.w[2], o.w[3]);
+    else *reinterpret_cast<HalfOctet*>(rows + (size_t)m * ldx + c * 8u) = o;
   }
   // the copy wants eight rows of one octet together: lane (octet, row) <- lane (row, octet)
   const int from = (int)(((lane & 7u) * 8u + (lane >> 3)) * 4u);

@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <utility>
@@ -517,6 +518,17 @@ struct RotArgs {
   uint32_t rows, m_pad, n_oct, kcols;
 };
 struct RotOctets {};  // in place of an output type
+// Where a kernel that makes a batch's rows leaves them for a batched product: xt as the octets gemm_kernel.h describes (`rows` of them, zeros
+// behind and past the column kcols), tail columns in the rows themselves.
+struct Octets {
+  uint4* xt;
+  uint32_t rows, m_pad, n_oct, kcols;
+};
+// The row of workgroup b where a workgroup writes a row's octets: eight rows share the lines of those, and workgroups go to the eight XCDs in
+// turn, so rows that share lines are eight apart and a line is made in one L2.  (As they come, every line is written in parts by
+// eight of them.  Rotated q, k, v of 64 rows 17.26 -> 16.78 us; and where it paid only up to 256 rows to write octets, it does for all:
+// 4096 x 4096 at 300 rows 38.6 us by rows and tile_activations_kernel, 36.4 so, 13000 x 12288 at 1024 310 and 303, 2560 x 9728 94 and 89.)
+__device__ __forceinline__ uint32_t octet_row(uint32_t b, uint32_t m_pad) { return m_pad & 63u ? b : (b & ~63u) | (b & 7u) << 3 | ((b >> 3) & 7u); }
 
 // the identity rotation: binary16 -> f32
 __global__ __launch_bounds__(256) void widen_kernel(const __half* __restrict__ x, float* __restrict__ out, uint32_t n) {
@@ -528,12 +540,14 @@ template <typename OutT>
 __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
   extern __shared__ __align__(16) float rot_s[];
   const uint32_t tid = threadIdx.x, n = a.n, m = a.m, k = a.k;
+  uint32_t row = blockIdx.x;
   if constexpr (std::is_same<OutT, RotOctets>::value) {
-    const uint32_t live = blockIdx.x < a.rows ? a.kcols / 8u : 0u;  // octets from there on are zero
-    for (uint32_t o = live + tid; o < a.n_oct; o += 1024) a.xt[(size_t)o * a.m_pad + blockIdx.x] = make_uint4(0, 0, 0, 0);
-    if (blockIdx.x >= a.rows) return;
+    row = octet_row(row, a.m_pad);
+    const uint32_t live = row < a.rows ? a.kcols / 8u : 0u;  // octets from there on are zero
+    for (uint32_t o = live + tid; o < a.n_oct; o += 1024) a.xt[(size_t)o * a.m_pad + row] = make_uint4(0, 0, 0, 0);
+    if (row >= a.rows) return;
   }
-  const __half* x = a.x + (size_t)blockIdx.x * n;
+  const __half* x = a.x + (size_t)row * n;
   const RotTable* table = reinterpret_cast<const RotTable*>(a.fragments);
   if (m >= kRotOctetM) {
     const rot_h8_t h[2] = {table->lane[tid & 63u].h[0], table->lane[tid & 63u].h[1]};
@@ -563,7 +577,7 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
   __syncthreads();
   constexpr bool kOctets = std::is_same<OutT, RotOctets>::value, kHalf = kOctets || std::is_same<OutT, __half>::value;
   typedef typename std::conditional<kHalf, __half, float>::type out_t;
-  out_t* out = reinterpret_cast<out_t*>(a.out) + (size_t)blockIdx.x * n;
+  out_t* out = reinterpret_cast<out_t*>(a.out) + (size_t)row * n;
   if constexpr (kHalf) {
     if (kOctets || m >= kRotOctetM) {
       for (uint32_t i = tid * 8u; i < n; i += 8192) {
@@ -571,7 +585,7 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           o.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(rot_s[i + 2 * j])) | (uint32_t)__half_as_ushort(__float2half_rn(rot_s[i + 2 * j + 1])) << 16;
-        if (kOctets && i < a.kcols) a.xt[(size_t)(i / 8u) * a.m_pad + blockIdx.x] = make_uint4(o.w[0], o.w[1], o.w[2], o.w[3]);
+        if (kOctets && i < a.kcols) a.xt[(size_t)(i / 8u) * a.m_pad + row] = make_uint4(o.w[0], o.w[1], o.w[2], o.w[3]);
         else *reinterpret_cast<HalfOctet*>(out + i) = o;
       }
       return;
@@ -1179,10 +1193,6 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
 }
 
 // Enqueues x' = Q x for `rows` activation rows of width rot->n.
-// Rows up to which a rotation writes octets, as many as there are workgroups at once: a column of them is m_pad x 16 bytes, so the rows'
-// stores share no lines, and a second turn waits for them.  From 1024 x 2560 to 13000 x 12288: at 3 rows 1.5 to 2.6 us less with it, at 64
-// 0.5 to 1.7, at 200 and 256 0.1 to 1.7; at 300 rows 0.4 to 5.5 us more, at 600 1.2 to 11.
-constexpr int kRotOctetRows = 256;
 static RotArgs rot_args(const llvq_rt::DevRotation* rot, const void* x_f16, void* out) {
   RotArgs a{};
   a.x = reinterpret_cast<const __half*>(x_f16);
@@ -1692,8 +1702,9 @@ static bool gemm_direct(uint32_t M, uint32_t n_tiles, uint32_t nb, uint32_t cus,
 // One launch over n <= kGemmMaxGroup matrices of equal d_in that take the same activations
 // (already in the matrices' basis), M <= kGemmMaxM rows.  from: rows that are rotated on the way to the octets, their tail
 // columns to x.
+// make: launches what makes the rows, as octets (and their tail columns in x).
 static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, uint32_t M, void* const* y,
-                       int y_dtype, bool pair, GemmWorkspace* wsp = nullptr, const void* from = nullptr) {
+                       int y_dtype, bool pair, GemmWorkspace* wsp = nullptr, const void* from = nullptr, const std::function<void(const Octets&)>* make = nullptr) {
   const llvq_mat* m0 = mats[0];
   const __half* xh = reinterpret_cast<const __half*>(x);
   const GemmPlan p = gemm_plan(rt, mats, n, M, pair);
@@ -1725,7 +1736,7 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   a.m_tiles = p.m_tiles;
   a.splits = p.splits;
   a.steps_per_split = p.steps_per_split;
-  const bool direct = !from && p.small == 1u && gemm_direct(M, a.n_tiles, a.nb, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), pair);
+  const bool direct = !from && !make && p.small == 1u && gemm_direct(M, a.n_tiles, a.nb, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), pair);
   a.xs = direct ? reinterpret_cast<const uint8_t*>(x) : reinterpret_cast<const uint8_t*>(xt_buf);
   a.xs_octet = direct ? 16u : p.m_pad * 16u;
   a.xs_block = 3u * a.xs_octet;
@@ -1740,10 +1751,12 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
     ra.n_oct = p.n_oct;
     ra.kcols = a.nb * kDim;
     hipLaunchKernelGGL(rotate_kernel<RotOctets>, dim3(p.m_pad), dim3(1024), (size_t)ra.n * sizeof(float), rt->stream, ra);
+  } else if (make) {
+    (*make)(Octets{reinterpret_cast<uint4*>(xt_buf), M, p.m_pad, p.n_oct, a.nb * kDim});
   } else if (!direct) {
     const uint32_t oct_waves = (p.n_oct + 7u) / 8u * (p.m_pad / 8u);
-    hipLaunchKernelGGL(tile_activations_kernel, dim3((oct_waves + 3u) / 4u), dim3(256), 0, rt->stream, xh, M, a.ldx, a.nb * 24u, p.m_pad, p.n_oct,
-                       reinterpret_cast<uint4*>(xt_buf));
+    hipLaunchKernelGGL(tile_activations_kernel, dim3((oct_waves + 3u) / 4u), dim3(256), 0, rt->stream, xh, (const __half*)nullptr, (__half*)nullptr, M,
+                       a.ldx, a.nb * 24u, p.m_pad, p.n_oct, reinterpret_cast<uint4*>(xt_buf));
   }
   const dim3 wide_grid(a.n_tiles * p.m_tiles * p.splits);
   auto product = [&](auto pair) {
@@ -1783,6 +1796,14 @@ static size_t static_admission_bytes(const llvq_rt* rt, const llvq_mat* m, uint3
   const uint32_t band0 = kparts == 1 ? share.shared0 : 0u;
   const size_t sums = (size_t)(bands - (band0 < bands ? band0 : bands)) * share.max_pieces * kparts * M * 64 * sizeof(float);
   return ((sums + 255) & ~(size_t)255) + (size_t)spb * 12 * ((M + 63) / 64 * 64) * 64;
+}
+
+// Whether one launch takes M rows that come as octets through these matrices (what gemm_same_basis asks of rows in their own basis).
+static bool gemm_takes_octets(const llvq_mat* const* mats, int n, uint32_t M) {
+  if (n > kGemmMaxGroup || M < 2u || !mats[0]->nblocks || mats[0]->d_in % 8 != 0 || M > gemm_chunk(mats[0]->nblocks, false)) return false;
+  for (int i = 0; i < n; ++i)
+    if (mats[i]->has_rotation || mats[i]->record_bits != 48 || mats[i]->d_in != mats[0]->d_in) return false;
+  return true;
 }
 
 // Matrices [0, n) of one group: same d_in, same basis.  What such a call has always been good to decides its way:
@@ -1834,7 +1855,7 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
     const int rc0 = workspace_take(rt, wsp, reinterpret_cast<void**>(&rt->rot_rows), &rt->rot_rows_bytes,
                                    (size_t)M * m0->d_in * sizeof(__half), &rows);
     if (rc0) return rc0;
-    if (n <= kGemmMaxGroup && M <= kRotOctetRows && M <= chunk && m0->rot->m >= kRotOctetM)
+    if (n <= kGemmMaxGroup && M <= chunk && m0->rot->m >= kRotOctetM)
       return launch_gemm(rt, mats, n, rows, (uint32_t)M, y, y_dtype, pair, wsp, x);
     const int rc = launch_rotate(rt, m0->rot, x, (uint32_t)M, rows, true);
     if (rc) return rc;
@@ -2171,7 +2192,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     if (pro.kind == kPrologueAddRmsNorm) {
       hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, x, reinterpret_cast<const __half*>(pro.x2),
                          reinterpret_cast<const __half*>(pro.norm_w), reinterpret_cast<__half*>(pro.resid_out), d->normed,
-                         d->hidden, pro.eps);
+                         d->hidden, pro.eps, Octets{});
       staged = d->normed;
     } else {
       hipLaunchKernelGGL(silu_mul_kernel, dim3((d->inter / 8 + 256) / 256), dim3(256), 0, st, reinterpret_cast<const __half*>(pro.x2),
@@ -2287,7 +2308,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   }
   phase_mark(d);
   if (want_logits) {
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, h, d->down, d->fnorm, h, d->normed, d->hidden, d->eps);
+    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, h, d->down, d->fnorm, h, d->normed, d->hidden, d->eps, Octets{});
     launch_head(d, history_slot, record);
   }
   HIP_TRY(hipGetLastError());
@@ -2333,16 +2354,23 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     hipLaunchKernelGGL(embed_kernel, dim3((d->hidden + 255) / 256, n), dim3(256), 0, st, d->embed, d->ptokens, 0u, d->vocab, d->hidden, ph);
   const size_t cache_layer = (size_t)d->n_kv * d->max_pos * d->head_dim, group_layer = cache_layer / kKvGroup;
   const float scale = 1.0f / sqrtf((float)d->head_dim);
-  auto rows = [&](const llvq_mat* m, const __half* x, __half* y) { return llvq_hip_gemm(rt, m, x, (int)n, y, LLVQ_F16); };
+  // Rows that `make` launches what makes, through projections that share them: straight to the product's octets where one launch takes them
+  // all in their own basis, else to x first.
+  const auto product = [&](const llvq_mat* const* mats, int n_mats, const __half* x, void* const* y, const std::function<void(const Octets&)>& make) {
+    if (gemm_takes_octets(mats, n_mats, n)) return launch_gemm(rt, mats, n_mats, x, n, y, LLVQ_F16, false, nullptr, nullptr, &make);
+    make(Octets{});
+    return llvq_hip_gemm_group(rt, mats, n_mats, x, (int)n, y, LLVQ_F16);
+  };
   for (uint32_t L = 0; L < d->n_layers; ++L) {
     const llvq_mat* const* P = d->proj.data() + (size_t)L * 7;
     // residual + previous MLP branch, then the input norm (the branch of layer 0 is absent)
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(n), dim3(norm_threads(d->hidden)), 0, st, ph, L ? d->pdown : (const __half*)nullptr,
-                       d->ln1 + (size_t)L * d->hidden, L ? ph_alt : (__half*)nullptr, d->pnormed, d->hidden, d->eps);
-    if (L) std::swap(ph, ph_alt);
     void* const qkv[3] = {d->pq, d->pk, d->pv};
-    int rc = llvq_hip_gemm_group(rt, P, 3, d->pnormed, (int)n, qkv, LLVQ_F16);
+    int rc = product(P, 3, d->pnormed, qkv, [&](const Octets& to) {
+      hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(to.xt ? to.m_pad : n), dim3(norm_threads(d->hidden)), 0, st, ph, L ? d->pdown : (const __half*)nullptr,
+                         d->ln1 + (size_t)L * d->hidden, L ? ph_alt : (__half*)nullptr, d->pnormed, d->hidden, d->eps, to);
+    });
     if (rc) return rc;
+    if (L) std::swap(ph, ph_alt);
     KvQ8 lq8 = d->q8;
     if (d->kv_q8) {
       lq8.kq += L * cache_layer; lq8.vq += L * cache_layer;
@@ -2359,6 +2387,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     nw.vcache = vc;
     nw.eps = d->eps;
     const dim3 hgrid((d->n_heads + 2 * d->n_kv + 3) / 4, n), agrid(d->n_kv, n);
+    Octets ctx_to{};
     auto attend = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, agrid, dim3(64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->head_dim, d->pos, d->max_pos, scale);
     };
@@ -2368,8 +2397,9 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     const bool on_mfma = d->head_dim == 128 && grp <= (uint32_t)kAttnMaxGroup;
     const dim3 mgrid(d->n_kv, (n + kAttnTile - 1) / kAttnTile);
     auto attend_mfma = [&](auto kernel, uint32_t waves) {
-      hipLaunchKernelGGL(kernel, mgrid, dim3(waves * 64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->pos, n, d->max_pos, scale);
+      hipLaunchKernelGGL(kernel, mgrid, dim3(waves * 64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->pos, n, d->max_pos, scale, ctx_to);
     };
+    const auto attention = [&]() {
     if (d->kv_q8) {
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<true>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos);
@@ -2395,23 +2425,42 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       else if (grp <= 5) attend(attn_rows_kernel<false, 5>);
       else attend(attn_rows_kernel<false, kAttnMaxGroup>);
     }
-    rc = rows(P[3], d->pctx, d->po);
+    };
+    void* const o_out[1] = {d->po};
+    if (on_mfma) {
+      rc = product(P + 3, 1, d->pctx, o_out, [&](const Octets& to) {
+        ctx_to = to;
+        attention();
+      });
+    } else {
+      attention();
+      rc = llvq_hip_gemm(rt, P[3], d->pctx, (int)n, d->po, LLVQ_F16);
+    }
     if (rc) return rc;
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(n), dim3(norm_threads(d->hidden)), 0, st, ph, d->po, d->ln2 + (size_t)L * d->hidden, ph_alt,
-                       d->pnormed, d->hidden, d->eps);
-    std::swap(ph, ph_alt);
     void* const gate_up[2] = {d->pgate, d->pup};
-    rc = llvq_hip_gemm_group(rt, P + 4, 2, d->pnormed, (int)n, gate_up, LLVQ_F16);
+    rc = product(P + 4, 2, d->pnormed, gate_up, [&](const Octets& to) {
+      hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(to.xt ? to.m_pad : n), dim3(norm_threads(d->hidden)), 0, st, ph, d->po, d->ln2 + (size_t)L * d->hidden,
+                         ph_alt, d->pnormed, d->hidden, d->eps, to);
+    });
     if (rc) return rc;
-    const uint32_t na = n * d->inter;
-    hipLaunchKernelGGL(silu_mul_kernel, dim3(std::min((na / 8u + 256u) / 256u, 4096u)), dim3(256), 0, st, d->pgate, d->pup, d->pact, na);
-    rc = rows(P[6], d->pact, d->pdown);
+    std::swap(ph, ph_alt);
+    void* const down[1] = {d->pdown};
+    rc = product(P + 6, 1, d->pact, down, [&](const Octets& to) {
+      if (to.xt) {
+        const uint32_t waves = (std::max(to.n_oct, d->inter / 8u) + 7u) / 8u * (to.m_pad / 8u);
+        hipLaunchKernelGGL(tile_activations_kernel, dim3((waves + 3u) / 4u), dim3(256), 0, st, d->pup, d->pgate, d->pact, n, d->inter, to.kcols, to.m_pad,
+                           to.n_oct, to.xt);
+        return;
+      }
+      const uint32_t na = n * d->inter;
+      hipLaunchKernelGGL(silu_mul_kernel, dim3(std::min((na / 8u + 256u) / 256u, 4096u)), dim3(256), 0, st, d->pgate, d->pup, d->pact, na);
+    });
     if (rc) return rc;
   }
   if (want_logits) {
     const size_t last = (size_t)(n - 1) * d->hidden;
     hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, ph + last, d->pdown + last, d->fnorm, d->h, d->normed,
-                       d->hidden, d->eps);
+                       d->hidden, d->eps, Octets{});
     launch_head(d, history_slot, record);
   }
   HIP_TRY(hipGetLastError());

@@ -720,3 +720,25 @@ def test_gate_and_up_as_one_result(gpu_rt, hidden, inter):
             d.close()
         for p in projs[0]:
             gpu_rt.free(p)
+
+
+@pytest.mark.parametrize("kv_mode", ["f16", "q8"])
+def test_prompt_rows_straight_to_octets(gpu_rt, orc, kv_mode):
+    """A pass's rows go to the products' octets where they are made (norm, attention, silu).  Widths with tail columns, of which two have more
+    octets than whole units do (208 = 8 blocks + 16, 112 = 4 blocks + 16) and one fewer (256 = 10 blocks + 16); rows around the
+    paddings of 16, 64, 128 and 256; what a pass of other rows left in the octets reaches nothing."""
+    cfg = decoder.Qwen3Config(num_hidden_layers=2, hidden_size=208, num_attention_heads=2, num_key_value_heads=1, head_dim=128, intermediate_size=112,
+                              vocab_size=300, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=160, tie_word_embeddings=True, kv_mode=kv_mode)
+    dec, ref = _build(gpu_rt, orc, cfg, 21, prefill_rows=256)
+    try:
+        tokens = np.random.default_rng(21).integers(0, cfg.vocab_size, size=140)
+        want = [ref.forward_token(int(t)) for t in tokens]
+        for rows in (130, 1, 2, 16, 17, 64, 65, 128, 129, 33):
+            dec.reset()
+            got, best = dec.prefill(tokens[:rows])
+            after, _ = dec.forward_token(int(tokens[rows]))
+            assert best == int(np.argmax(got))
+            for g, w in ((got, want[rows - 1]), (after, want[rows])):
+                assert np.abs(g - w).max() < 2e-3 * np.abs(w).max(), (rows, np.abs(g - w).max() / np.abs(w).max())
+    finally:
+        dec.close()

@@ -260,3 +260,10 @@ def test_rotation_of_every_kind_of_width(gpu_rt, orc, m, k):
                 assert not torch.isfinite(gpu_rt.forward(proj, bad, out_dtype=dtype)).any()
     finally:
         gpu_rt.free(proj)
+
+
+# up to the rows of a launch every batch's rotation writes octets: past 256, off and on the padding of 128 and 256 rows, and the last count
+# (widths whose columns no plan splits: the same sums)
+@pytest.mark.parametrize("n,rows", [(31 * 8, 300), (31 * 8, 700), (1024, 512), (3 * 128, 1000), (31 * 8, 1024), (31 * 8, 1025)])
+def test_many_rotated_rows_to_octets(gpu_rt, n, rows):
+    test_rotated_rows_to_octets(gpu_rt, n, rows)
