@@ -2238,7 +2238,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
       else attend(attn_decode_kernel<false, kAttnMaxGroup>);
     }
     if (!merge_inline)
-      hipLaunchKernelGGL(attn_merge_kernel, dim3(d->n_heads), dim3(128), 0, st, d->attn_part, d->ctx, d->head_dim, n_splits);
+      hipLaunchKernelGGL(attn_merge_kernel, dim3(d->n_heads), dim3(kMergeParts * 128), 0, st, d->attn_part, d->ctx, d->head_dim, n_splits);
   };
   if (!d->seqs.empty() && d->seq_chained) {
     // the projections between two attention launches are one persistent launch each
