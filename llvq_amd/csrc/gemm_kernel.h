@@ -1216,25 +1216,23 @@ __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmArgs a) { wide_pr
 // kReduceM activation rows, so that the row's tail is read once for them.
 // What bounds it is how many round trips to memory a lane makes: the sums and the tail columns are read four splits and
 // eight columns at a time, the activations' tail comes to LDS with the first of them.  (One by one 11.3 us for 500
-// rows of 2560 with 8 or 16 tail columns and 14.9 for 6144; so 9.0 and 10.3.)
+// rows of 2560 with 8 or 16 tail columns and 14.9 for 6144; so 9.0 and 10.3; and a microsecond less with a workgroup's lanes a tile's rows,
+// which needs no division, and loads of the splits there are alone.)
 constexpr uint32_t kReduceM = 8;
 constexpr uint32_t kReduceSplits = 4;
-struct GemmReduceArgs {
-  GemmArgs g;
-  uint32_t rows_per_tile, row_chunks;
-};
-// With PAIR the splits are added in f64 and the tail by itself.
+// With PAIR the splits are added in f64 and the tail by itself.  Grid (tiles of 256 weight rows, the only ones that are split; kReduceM
+// activation rows).
+constexpr uint32_t kReduceRows = 256;
+static_assert(kReduceRows == gemm_wide_rows<2>(), "a workgroup's lanes are a tile's rows");
 template <bool PAIR>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a) {
   typedef typename std::conditional<PAIR, double, float>::type sum_t;
   __shared__ float x_tail[kReduceM][32];
   static_assert(kReduceM * 32u == 256u && kDim <= 32, "a value of the activations' tail per lane");
-  const GemmArgs& a = ra.g;
-  const uint32_t n_rows = a.n_tiles * ra.rows_per_tile;
-  const uint32_t chunk = blockIdx.x % ra.row_chunks, m0 = blockIdx.x / ra.row_chunks * kReduceM;
-  const uint32_t mine = chunk * 256u + threadIdx.x, out_row = min(mine, n_rows - 1u);  // lanes past the last row repeat it
-  const GemmTile t = gemm_tile_at(a, out_row / ra.rows_per_tile, ra.rows_per_tile);
-  const uint32_t my_row = t.row0 + out_row % ra.rows_per_tile, row = min(my_row, t.d_out - 1u);
+  touch_args(a);
+  const uint32_t n_rows = a.n_tiles * kReduceRows, m0 = blockIdx.y * kReduceM, out_row = blockIdx.x * kReduceRows + threadIdx.x;
+  const GemmTile t = gemm_tile_at(a, blockIdx.x, kReduceRows);
+  const uint32_t my_row = t.row0 + threadIdx.x, row = min(my_row, t.d_out - 1u);  // lanes past the last row repeat it
   const uint32_t stride = t.stride;
   const uint8_t* rec = t.base + kTileTableBytes + (size_t)(row / kTileRows) * stride;
   const uint32_t r = row & 15u, tail_w = a.tail_w;
@@ -1257,14 +1255,17 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
   for (uint32_t p0 = 0; p0 < a.splits; p0 += kReduceSplits) {
     float v[kReduceSplits][kReduceM];
 #pragma unroll
-    for (uint32_t p = 0; p < kReduceSplits; ++p)
+    for (uint32_t p = 0; p < kReduceSplits; ++p) {
+      if (p0 + p >= a.splits) break;
 #pragma unroll
-      for (uint32_t k = 0; k < kReduceM; ++k)
-        v[p][k] = a.ws[((size_t)min(p0 + p, a.splits - 1u) * a.m_pad + min(m0 + k, a.M - 1u)) * n_rows + out_row];
+      for (uint32_t k = 0; k < kReduceM; ++k) v[p][k] = uniform_global(a.ws + ((size_t)(p0 + p) * a.m_pad + min(m0 + k, a.M - 1u)) * n_rows)[out_row];
+    }
 #pragma unroll
-    for (uint32_t p = 0; p < kReduceSplits; ++p)
+    for (uint32_t p = 0; p < kReduceSplits; ++p) {
+      if (p0 + p >= a.splits) break;
 #pragma unroll
-      for (uint32_t k = 0; k < kReduceM; ++k) s[k] = p0 + p < a.splits ? s[k] + (sum_t)v[p][k] : s[k];
+      for (uint32_t k = 0; k < kReduceM; ++k) s[k] += (sum_t)v[p][k];
+    }
   }
   float out[kReduceM];
 #pragma unroll
@@ -1284,7 +1285,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmReduceArgs ra) {
           }
     }
   }
-  if (mine < n_rows && my_row < t.d_out) {
+  if (my_row < t.d_out) {
 #pragma unroll
     for (uint32_t k = 0; k < kReduceM; ++k)
       if (m0 + k < a.M) store_y(t.y, (size_t)(m0 + k) * t.d_out + row, PAIR ? fmaf((float)s[k], scale, out[k]) : out[k], a.y_f32);

@@ -1717,8 +1717,7 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   rc = workspace_take(rt, wsp, reinterpret_cast<void**>(&rt->gemm_xt), &rt->gemm_xt_bytes, p.xt_bytes, &xt_buf);
   if (rc) return rc;
   if (wsp) wsp->used = mark;
-  GemmReduceArgs r{};
-  GemmArgs& a = r.g;
+  GemmArgs a{};
   a.xt = reinterpret_cast<const uint4*>(xt_buf);
   a.x = xh;
   a.ws = reinterpret_cast<float*>(ws_buf);
@@ -1772,11 +1771,9 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   if (pair) product(std::true_type{});
   else product(std::false_type{});
   if (p.splits > 1u) {
-    r.rows_per_tile = p.rows_per_tile;
-    r.row_chunks = (a.n_tiles * p.rows_per_tile + 255u) / 256u;
-    const dim3 grid(r.row_chunks * ((M + kReduceM - 1u) / kReduceM));
-    if (pair) hipLaunchKernelGGL(gemm_reduce_kernel<true>, grid, dim3(256), 0, rt->stream, r);
-    else hipLaunchKernelGGL(gemm_reduce_kernel<false>, grid, dim3(256), 0, rt->stream, r);
+    const dim3 grid(a.n_tiles, (M + kReduceM - 1u) / kReduceM);
+    if (pair) hipLaunchKernelGGL(gemm_reduce_kernel<true>, grid, dim3(kReduceRows), 0, rt->stream, a);
+    else hipLaunchKernelGGL(gemm_reduce_kernel<false>, grid, dim3(kReduceRows), 0, rt->stream, a);
   }
   HIP_TRY(hipGetLastError());
   return LLVQ_OK;
