@@ -222,14 +222,14 @@ constexpr uint32_t kRotTile = 1024;   // values of a wavefront, and how far the 
 typedef _Float16 rot_h8_t __attribute__((ext_vector_type(8)));
 typedef float rot_acc_t __attribute__((ext_vector_type(16)));
 struct __attribute__((aligned(16))) RotFragments {   // of lane l: (l32, lh) = (l % 32, l / 32)
-  float s[kRotKMax / 2];  // S[l32][2 i + lh], zero past k
+  float s[kRotKMax / 2];  // (S / sqrt m)[l32][2 i + lh], zero past k
   rot_h8_t h[2];          // H[l32][16 i + 8 lh + e], H the transform inside groups of min(m, 32)
 };
 static_assert(sizeof(RotFragments) == 96, "six 16-byte loads");
 constexpr uint32_t kRotScalarK = 9;  // the largest k whose block is multiplied as scalars: rows of it are padded to that, with zeros
 struct RotTable {
   RotFragments lane[64];
-  float rows[kRotScalarK][kRotScalarK + 3];  // S[g][i]
+  float rows[kRotScalarK][kRotScalarK + 3];  // (S / sqrt m)[g][i]
 };
 __device__ __forceinline__ float flip_sign(float v, uint32_t bits, int j) {  // bit j of `bits` is the sign of D
   return __uint_as_float(__float_as_uint(v) ^ (((bits >> j) & 1u) << 31));
@@ -367,7 +367,7 @@ __device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t lg,
 // wavefronts share the rows of a column, and read it before any of them writes.  K * K multiply-adds a column, where the matrix cores
 // multiply 32 x 32: 5120 values, k = 5, 2.3 us of a launch with the latter.
 template <uint32_t K>
-__device__ __forceinline__ void rotate_columns(float* v, uint32_t m, float inv, const float* rows) {
+__device__ __forceinline__ void rotate_columns(float* v, uint32_t m, const float* rows) {
   typedef const float __attribute__((address_space(4))) scalar_f;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lg = 31u - (uint32_t)__builtin_clz(m);
   const uint32_t parts = m < 1024u ? 1024u >> lg : 1u, part = m < 1024u ? wave >> (lg - 6u) : 0u;  // (m >= 64: a part is whole wavefronts)
@@ -376,7 +376,7 @@ __device__ __forceinline__ void rotate_columns(float* v, uint32_t m, float inv, 
   for (uint32_t j = threadIdx.x & (m - 1u); j < m; j += 1024u) {
     float c[K];
 #pragma unroll
-    for (uint32_t i = 0; i < K; ++i) c[i] = v[i * m + j] * inv;
+    for (uint32_t i = 0; i < K; ++i) c[i] = v[i * m + j];
     if (parts > 1u) lds_barrier();
 #pragma unroll 1
     for (uint32_t g = g0; g < g1; ++g) {
@@ -427,13 +427,13 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
   if (k == 1) return;
   if (rot_scalars(m, k)) {
     const float* rows = &table->rows[0][0];
-    if (k == 3u) rotate_columns<3>(v, m, inv, rows);
-    else if (k == 5u) rotate_columns<5>(v, m, inv, rows);
-    else if (k == 7u) rotate_columns<7>(v, m, inv, rows);
-    else rotate_columns<9>(v, m, inv, rows);
+    if (k == 3u) rotate_columns<3>(v, m, rows);
+    else if (k == 5u) rotate_columns<5>(v, m, rows);
+    else if (k == 7u) rotate_columns<7>(v, m, rows);
+    else rotate_columns<9>(v, m, rows);
     return;
   }
-  // S (k x k) . C (k x m), the 1 / sqrt m factor first: a wavefront takes 32 columns of C at a time as f32 matrix-core
+  // S (k x k, with the factor 1 / sqrt m) . C (k x m): a wavefront takes 32 columns of C at a time as f32 matrix-core
   // steps of depth 2 (S padded with zeros to 32 x 32; lanes past a narrow m repeat its first column); it reads its columns
   // whole before it writes them, and no other wavefront touches them.
 #pragma unroll 1
@@ -442,7 +442,7 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
     asm volatile("" : "+s"(k), "+s"(m));
     const uint32_t steps = (k + 1u) >> 1;  // k is odd: the last one has no row for the upper half
     const uint32_t j = tile * 32u + l32;
-    const float* col = v + (j < m ? j : 0u);
+    const float *at = v + (j < m ? j : 0u), *col = at + lh * m;
     rot_acc_t acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -451,11 +451,14 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
       if (s0 >= steps) break;
       float c[8];
 #pragma unroll
-      for (uint32_t i = 0; i < 8u; ++i) c[i] = col[min((2u * (s0 + i) + lh) * m, (k - 1u) * m)];  // always valid, so the reads go out together
+      for (uint32_t i = 0; i < 8u; ++i) {
+        if (s0 + i >= steps) break;
+        c[i] = s0 + i + 1u == steps ? at[(k - 1u) * m] : col[2u * (s0 + i) * m];
+      }
 #pragma unroll
       for (uint32_t i = 0; i < 8u; ++i) {
         if (s0 + i >= steps) break;
-        float x = c[i] * inv;
+        float x = c[i];
         if (s0 + i + 1u == steps) x = lh ? 0.f : x;
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(B.s[s0 + i], x, acc, 0, 0, 0);
       }
@@ -836,15 +839,17 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
   std::vector<RotTable> host(1);
   std::memset(static_cast<void*>(host.data()), 0, sizeof(RotTable));
   RotFragments* const frag = host[0].lane;
+  const double unit = 1. / std::sqrt((double)t.m);
+  auto scaled = [&](uint32_t g, uint32_t i) { return (float)((double)t.small[(size_t)g * t.k + i] * unit); };
   if (t.k <= kRotScalarK)
     for (uint32_t g = 0; g < t.k; ++g)
-      for (uint32_t i = 0; i < t.k; ++i) host[0].rows[g][i] = t.small[(size_t)g * t.k + i];
+      for (uint32_t i = 0; i < t.k; ++i) host[0].rows[g][i] = scaled(g, i);
   const uint32_t inside = std::min(t.m, 32u) - 1u;  // the bits of a column that the transform mixes
   for (uint32_t l = 0; l < 64u; ++l) {
     const uint32_t row = l & 31u, lh = l >> 5;
     for (uint32_t i = 0; i < kRotKMax / 2; ++i) {
       const uint32_t c = 2u * i + lh;
-      frag[l].s[i] = row < t.k && c < t.k ? t.small[(size_t)row * t.k + c] : 0.f;
+      frag[l].s[i] = row < t.k && c < t.k ? scaled(row, c) : 0.f;
     }
     for (uint32_t i = 0; i < 2u; ++i)
       for (uint32_t e8 = 0; e8 < 8u; ++e8) {
