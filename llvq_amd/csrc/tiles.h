@@ -372,8 +372,11 @@ __device__ __forceinline__ void load_halves(const __half* p, uint32_t (&w)[4]) {
 }
 
 // Fills the planes and the tail values in LDS from `in`, by every lane of the workgroup.
-// `request` is called once, right behind the loads of the activation's operands: the first weights go out there.  (With a
-// barrier in front, so that no wavefront's operands come behind the others' weights, a decode step took 3 % longer.)
+// `request` is called once, behind the loads of the activation's operands: the first weights go out there.  (With a
+// barrier in front, so that no wavefront's operands come behind the others' weights, a decode step took 3 % longer.  A
+// rotation in octets has it behind the levels in registers: loads come back in order, and with the weights right behind the
+// operands the first wavefronts' weights kept the last ones' operands waiting.  2560 x 9728 on the card: 11.35 us, and 11.1
+// so; a rotated 14B decode of 8 tokens 4365 and 4265 us; behind the first barrier of rotate_rest, 4335.)
 // PMAX: how often the workgroup's quads pass over the padded blocks, at most; `waves`, `passes`: its wavefronts and how often that is
 // (stage_passes).  store_resid: this workgroup is the one that stores the new residual.  Ends without a barrier.
 template <int DIG, int SRC, int PMAX, bool kDeviceScope = false, class Request>
@@ -428,7 +431,6 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
           h[0] = table->lane[lane].h[0];
           h[1] = table->lane[lane].h[1];
         }
-        if constexpr (PMAX <= 2) request();
         __builtin_amdgcn_sched_barrier(0);
         float inv = 0.f;
         if (norm) {
@@ -470,7 +472,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
           if ((tile + 16u) * kRotTile < d_in) load_tile(tile + 16u);  // (on their way beside this tile's levels)
           rotate_tile_to(xf, x[0], x[1], h, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
         }
-        if constexpr (PMAX > 2) request();  // (no registers for a wide step beside the operands)
+        request();
       } else {
         auto put = [&](uint32_t i, float v) { xf[i] = flip_sign(v, in.rot_signbits[i >> 5] >> (i & 31u), 0); };
         if (norm) {
