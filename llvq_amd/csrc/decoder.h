@@ -1042,7 +1042,7 @@ __global__ __launch_bounds__(kMergeParts * 128) void attn_merge_kernel(const flo
   const uint32_t head = blockIdx.x, tid = threadIdx.x, lane = tid & 63u, i = tid & 127u;
   const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 7)), stride = head_dim + 2u;
   const float* src = part + (size_t)head * n_splits * stride;
-  // Everything is asked for at once (past the last range: the last again, of weight zero).
+  // Everything is asked for at once (past the last range: the last again, not added).
   const uint32_t mine = min(lane, n_splits - 1u) * stride, col = 2u + min(i, head_dim - 1u);
   const float m = src[mine], l = src[mine + 1u];
   float v[kRanges];
@@ -1056,7 +1056,10 @@ __global__ __launch_bounds__(kMergeParts * 128) void attn_merge_kernel(const flo
   const float L = wave_sum(lane < n_splits ? l * w : 0.f);
   float A = 0.f;
 #pragma unroll
-  for (uint32_t u = 0; u < kRanges; ++u) A = fmaf(v[u], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), p * kRanges + u)), A);
+  for (uint32_t u = 0; u < kRanges; ++u) {
+    const float sum = fmaf(v[u], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), p * kRanges + u)), A);
+    A = p * kRanges + u < n_splits ? sum : A;  // (0 x infinity, of the last range's repeats, would reach the sums)
+  }
   sums[p][i] = A;
   __syncthreads();
   if (tid >= head_dim) return;
@@ -1239,39 +1242,71 @@ __global__ __launch_bounds__(kHeadThreads) void lm_head_q8_kernel(QuantRows e, c
   head_rows(QuantHead{e, hidden, (hidden + kEmbedGroup - 1) / kEmbedGroup}, h, vocab, hidden, hs, logits, best_val, best_idx);
 }
 
-// token = argmax over the wavefront winners; lowest row on ties
-__global__ __launch_bounds__(1024) void argmax_final_kernel(const float* __restrict__ best_val, const uint32_t* __restrict__ best_idx,
-                                                            uint32_t n, uint32_t* __restrict__ token_out,
-                                                            uint32_t* __restrict__ history, uint32_t slot) {
-  __shared__ float sv[1024];
-  __shared__ uint32_t si[1024];
+// token = argmax over the wavefront winners; lowest row on ties.  Where the caller wants the results, workgroup 0 leaves the token in pinned host
+// memory as well, and the others, 4096 values each, the logits: a copy enqueued behind the launch is the copy engine's, which waits
+// for the launch by a signal.  (Eight tokens of a 4B model with 151936 logits each 11 640 us with that copy, 11 425 so; four 14B layers 4280 and
+// 4110.  Stored by the head itself, a row at a time, they would be writes of four bytes.)
+// What bounds workgroup 0 is its round trips: its values are asked for together, and meet in lane moves and one pass over LDS.
+constexpr int kFinalThreads = 1024;
+constexpr uint32_t kFinalCopy = 4u * kFinalThreads;  // logits of a workgroup
+constexpr int kFinalRounds = 4;                      // values of a lane that are asked for together
+struct HostResults {  // pinned memory, each null where it is not wanted
+  float* logits;
+  uint32_t* token;
+};
+__global__ __launch_bounds__(kFinalThreads) void argmax_final_kernel(const float* __restrict__ best_val, const uint32_t* __restrict__ best_idx,
+                                                                     uint32_t n, uint32_t* __restrict__ token_out, uint32_t* __restrict__ history,
+                                                                     uint32_t slot, const float* __restrict__ logits, uint32_t vocab, HostResults host) {
+  if (blockIdx.x) {
+    const uint32_t at = (blockIdx.x - 1u) * kFinalCopy + threadIdx.x * 4u;
+    if (at + 4u <= vocab) *reinterpret_cast<float4*>(host.logits + at) = *reinterpret_cast<const float4*>(logits + at);
+    else
+      for (uint32_t i = at; i < vocab; ++i) host.logits[i] = logits[i];
+    return;
+  }
+  __shared__ float sv[kFinalThreads / 64];
+  __shared__ uint32_t si[kFinalThreads / 64];
   float bv = -INFINITY;
   uint32_t bi = 0xFFFFFFFFu;
-  for (uint32_t i = threadIdx.x; i < n; i += 1024) {
-    const float v = best_val[i];
-    const uint32_t id = best_idx[i];
-    if (v > bv || (v == bv && id < bi)) {
-      bv = v;
-      bi = id;
+  const auto take = [&](float v, uint32_t id) {
+    const bool better = v > bv || (v == bv && id < bi);
+    bv = better ? v : bv;
+    bi = better ? id : bi;
+  };
+  const auto wavefront = [&]() {
+#pragma unroll
+    for (int k = 1; k < 64; k <<= 1) {
+      const float v = __shfl_xor(bv, k);
+      const uint32_t id = (uint32_t)__shfl_xor((int)bi, k);
+      take(v, id);
     }
+  };
+  for (uint32_t i0 = threadIdx.x; i0 < n; i0 += kFinalRounds * kFinalThreads) {
+    float v[kFinalRounds];
+    uint32_t id[kFinalRounds];
+#pragma unroll
+    for (int u = 0; u < kFinalRounds; ++u) {  // (past the last: the last again)
+      const uint32_t i = min(i0 + u * kFinalThreads, n - 1u);
+      v[u] = best_val[i];
+      id[u] = best_idx[i];
+    }
+#pragma unroll
+    for (int u = 0; u < kFinalRounds; ++u) take(v[u], id[u]);
   }
-  sv[threadIdx.x] = bv;
-  si[threadIdx.x] = bi;
+  wavefront();
+  if ((threadIdx.x & 63u) == 0) {
+    sv[threadIdx.x >> 6] = bv;
+    si[threadIdx.x >> 6] = bi;
+  }
   __syncthreads();
-  for (uint32_t s = 512; s >= 1; s >>= 1) {
-    if (threadIdx.x < s) {
-      const float v = sv[threadIdx.x + s];
-      const uint32_t id = si[threadIdx.x + s];
-      if (v > sv[threadIdx.x] || (v == sv[threadIdx.x] && id < si[threadIdx.x])) {
-        sv[threadIdx.x] = v;
-        si[threadIdx.x] = id;
-      }
-    }
-    __syncthreads();
-  }
+  if (threadIdx.x >= 64) return;
+  bv = sv[threadIdx.x % (kFinalThreads / 64)];
+  bi = si[threadIdx.x % (kFinalThreads / 64)];
+  wavefront();
   if (threadIdx.x == 0) {
-    *token_out = si[0];
-    if (history) history[slot] = si[0];
+    *token_out = bi;
+    if (history) history[slot] = bi;
+    if (host.token) *host.token = bi;
   }
 }
 

@@ -1986,8 +1986,8 @@ struct llvq_decoder {
   __half *kcache = nullptr, *vcache = nullptr;  // [n_layers][n_kv][max_pos][head_dim]
   __half *h = nullptr, *h_alt = nullptr, *normed = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *ctx = nullptr, *o = nullptr;
   __half *gate = nullptr, *up = nullptr, *act = nullptr, *down = nullptr;
-  float* logits = nullptr;      // [vocab], and the chosen token behind them: one copy takes both to the host
-  float* host_out = nullptr;    // pinned memory for that copy (null where there is none to be had: the copy goes to the caller's memory)
+  float* logits = nullptr;      // [vocab], and the chosen token behind them
+  float* host_out = nullptr;    // [vocab + 1] pinned memory: a step's last launch leaves logits and token there (null where there is none to be had: copies to the caller's memory)
   float* best_val = nullptr;
   uint32_t* best_idx = nullptr;
   uint32_t* token = nullptr;    // logits + vocab: the token the next step embeds
@@ -2025,8 +2025,8 @@ void phase_mark(llvq_decoder* d) {
   if (d->marks && d->next_mark < d->marks->size()) (void)hipEventRecord((*d->marks)[d->next_mark++], d->rt->stream);
 }
 
-// The head over dec->normed and the argmax, which overwrites *dec->token (and history[slot] when recording).
-void launch_head(llvq_decoder* d, uint32_t history_slot, bool record) {
+// The head over dec->normed and the argmax, which overwrites *dec->token (and history[slot] when recording) and leaves what `host` asks for there.
+void launch_head(llvq_decoder* d, uint32_t history_slot, bool record, const HostResults& host) {
   hipStream_t st = d->rt->stream;
   if (d->head_q8)
     hipLaunchKernelGGL(lm_head_q8_kernel, dim3(d->head_grid), dim3(kHeadThreads), d->hidden * sizeof(float), st, d->head_q, d->normed,
@@ -2035,8 +2035,9 @@ void launch_head(llvq_decoder* d, uint32_t history_slot, bool record) {
     hipLaunchKernelGGL(lm_head_kernel, dim3(d->head_grid), dim3(kHeadThreads), d->hidden * sizeof(float), st, d->head, d->normed,
                        d->vocab, d->hidden, d->logits, d->best_val, d->best_idx);
   phase_mark(d);
-  hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(1024), 0, st, d->best_val, d->best_idx,
-                     d->head_grid * (kHeadThreads / 64), d->token, record ? d->history : (uint32_t*)nullptr, history_slot);
+  const uint32_t copies = host.logits ? (d->vocab + kFinalCopy - 1u) / kFinalCopy : 0u;
+  hipLaunchKernelGGL(argmax_final_kernel, dim3(1u + copies), dim3(kFinalThreads), 0, st, d->best_val, d->best_idx, d->head_grid * (kHeadThreads / 64),
+                     d->token, record ? d->history : (uint32_t*)nullptr, history_slot, d->logits, d->vocab, host);
   phase_mark(d);
 }
 
@@ -2158,7 +2159,7 @@ int decoder_check_sequences(llvq_decoder* d) {
 
 // Enqueues one position: embeds *fed (host memory, read here) or, without it, *dec->token, runs the layers at position dec->pos,
 // and (want_logits) the head and the argmax, which overwrites *dec->token.
-int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool record, const uint32_t* fed = nullptr) {
+int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool record, const uint32_t* fed = nullptr, const HostResults& host = {}) {
   llvq_rt* rt = d->rt;
   hipStream_t st = rt->stream;
   if (d->pos >= d->max_pos) return fail(LLVQ_ERR_INVALID_ARGUMENT, "decoder: position " + std::to_string(d->pos) + " is past max_positions");
@@ -2311,16 +2312,21 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   phase_mark(d);
   if (want_logits) {
     hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, h, d->down, d->fnorm, h, d->normed, d->hidden, d->eps, Octets{});
-    launch_head(d, history_slot, record);
+    launch_head(d, history_slot, record, host);
   }
   HIP_TRY(hipGetLastError());
   d->pos += 1;
   return LLVQ_OK;
 }
-// The logits and the chosen token to the host, and the wait for them.  A copy straight to the caller's (pageable) memory
-// is staged by the runtime, one for each result, and begins when the stream has been waited for.  One copy to pinned
-// memory is enqueued behind the step instead, and while the step runs the pages that the results go to are touched,
-// which for fresh memory is most of what moving them costs: a token through four 14B layers takes 686 us, not 712.
+// Where a step's last launch leaves what the caller wants of it: in pinned memory, if there is any.
+HostResults host_results(llvq_decoder* d, const float* logits_host, const uint32_t* argmax_host) {
+  if (!d->host_out) return {};
+  return {logits_host ? d->host_out : nullptr, argmax_host ? reinterpret_cast<uint32_t*>(d->host_out + d->vocab) : nullptr};
+}
+// The wait for a step's results, and their way to the caller's memory.  A copy straight to that (pageable) memory is staged by the
+// runtime, one for each result, and begins when the stream has been waited for.  With pinned memory they are there when the
+// step ends, and while it runs the pages that they go to are touched, which for fresh memory is most of what moving
+// them costs: a token through four 14B layers takes 686 us, not 712.
 int decoder_results(llvq_decoder* d, float* logits_host, uint32_t* argmax_host) {
   hipStream_t st = d->rt->stream;
   const size_t bytes = (size_t)d->vocab * sizeof(float);
@@ -2330,8 +2336,6 @@ int decoder_results(llvq_decoder* d, float* logits_host, uint32_t* argmax_host) 
     HIP_TRY(hipStreamSynchronize(st));
     return LLVQ_OK;
   }
-  if (logits_host) HIP_TRY(hipMemcpyAsync(d->host_out, d->logits, bytes + sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  else if (argmax_host) HIP_TRY(hipMemcpyAsync(d->host_out + d->vocab, d->token, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
   if (logits_host) {
     volatile char* page = reinterpret_cast<volatile char*>(logits_host);
     for (size_t at = 0; at < bytes; at += 4096) page[at] = 0;
@@ -2345,7 +2349,7 @@ int decoder_results(llvq_decoder* d, float* logits_host, uint32_t* argmax_host) 
 
 // n <= prefill_rows positions at once, starting at dec->pos: tokens from dec->ptokens.
 // With want_logits the head runs on the last row and leaves its argmax in *dec->token.
-int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t history_slot, bool record) {
+int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t history_slot, bool record, const HostResults& host) {
   llvq_rt* rt = d->rt;
   hipStream_t st = rt->stream;
   if (d->pos + n > d->max_pos) return fail(LLVQ_ERR_INVALID_ARGUMENT, "decoder_prefill: positions past max_positions");
@@ -2463,7 +2467,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     const size_t last = (size_t)(n - 1) * d->hidden;
     hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, ph + last, d->pdown + last, d->fnorm, d->h, d->normed,
                        d->hidden, d->eps, Octets{});
-    launch_head(d, history_slot, record);
+    launch_head(d, history_slot, record, host);
   }
   HIP_TRY(hipGetLastError());
   d->pos += n;
@@ -2471,12 +2475,12 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
 }
 
 // The prompt through decoder_prefill_pass, prefill_rows positions at a time; the head runs after the last one.
-int decoder_prefill(llvq_decoder* d, const uint32_t* tokens, size_t n, uint32_t history_slot, bool record) {
+int decoder_prefill(llvq_decoder* d, const uint32_t* tokens, size_t n, uint32_t history_slot, bool record, const HostResults& host = {}) {
   if (!d->prefill_rows) return fail(LLVQ_ERR_UNSUPPORTED, "decoder_prefill: the decoder was created with prefill_rows = 0");
   for (size_t at = 0; at < n; at += d->prefill_rows) {
     const uint32_t c = (uint32_t)(n - at < d->prefill_rows ? n - at : d->prefill_rows);
     HIP_TRY(hipMemcpyAsync(d->ptokens, tokens + at, c * sizeof(uint32_t), hipMemcpyHostToDevice, d->rt->stream));
-    const int rc = decoder_prefill_pass(d, c, at + c == n, history_slot, record);
+    const int rc = decoder_prefill_pass(d, c, at + c == n, history_slot, record, host);
     if (rc) return rc;
   }
   return LLVQ_OK;
@@ -2690,7 +2694,7 @@ int llvq_hip_decoder_forward_token(llvq_decoder* d, uint32_t token, float* logit
   if (!d) return fail(LLVQ_ERR_INVALID_ARGUMENT, "decoder_forward_token: null decoder");
   if (token >= d->vocab) return fail(LLVQ_ERR_INVALID_ARGUMENT, "decoder_forward_token: token " + std::to_string(token) + " is outside the vocabulary");
   HIP_TRY(hipSetDevice(d->rt->device));
-  const int rc = decoder_step(d, true, 0, false, &token);
+  const int rc = decoder_step(d, true, 0, false, &token, host_results(d, logits_host, argmax_host));
   if (rc) return rc;
   {
     const int rc1 = decoder_results(d, logits_host, argmax_host);
@@ -2788,7 +2792,7 @@ int llvq_hip_decoder_prefill(llvq_decoder* d, const uint32_t* tokens, size_t n, 
   for (size_t i = 0; i < n; ++i)
     if (tokens[i] >= d->vocab) return fail(LLVQ_ERR_INVALID_ARGUMENT, "decoder_prefill: token outside the vocabulary");
   HIP_TRY(hipSetDevice(d->rt->device));
-  const int rc = decoder_prefill(d, tokens, n, 0, false);
+  const int rc = decoder_prefill(d, tokens, n, 0, false, host_results(d, logits_host, argmax_host));
   if (rc) return rc;
   {
     const int rc1 = decoder_results(d, logits_host, argmax_host);

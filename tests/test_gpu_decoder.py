@@ -742,3 +742,30 @@ def test_prompt_rows_straight_to_octets(gpu_rt, orc, kv_mode):
                 assert np.abs(g - w).max() < 2e-3 * np.abs(w).max(), (rows, np.abs(g - w).max() / np.abs(w).max())
     finally:
         dec.close()
+
+
+# fewer logits than a 16-byte store has and than a wavefront has lanes, a workgroup's 4096 and one more or less, several with a remainder
+@pytest.mark.parametrize("vocab", [2, 63, 4095, 4096, 4097, 8195, 20001])
+def test_results_where_the_last_launch_leaves_them(gpu_rt, orc, vocab):
+    """Logits of every vocabulary size come whole, with the token or without it, a prompt's as well as a step's, and are those of their own step."""
+    cfg = decoder.Qwen3Config(num_hidden_layers=1, hidden_size=64, num_attention_heads=2, num_key_value_heads=1, head_dim=64, intermediate_size=48,
+                              vocab_size=vocab, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=16, tie_word_embeddings=True)
+    dec, ref = _build(gpu_rt, orc, cfg, 31, prefill_rows=8)
+    try:
+        tokens = np.random.default_rng(vocab).integers(0, vocab, size=5)
+        want = [ref.forward_token(int(t)) for t in tokens]
+        first = []
+        for t, w in zip(tokens, want):
+            got, best = dec.forward_token(int(t))
+            first.append(best)
+            assert got.shape == (vocab,) and best == int(np.argmax(got))
+            assert np.abs(got - w).max() < 2e-3 * np.abs(w).max()
+        dec.reset()
+        for t, best in zip(tokens, first):
+            got, again = dec.forward_token(int(t), want_logits=False)
+            assert got is None and again == best
+        dec.reset()
+        got, best = dec.prefill(tokens)
+        assert best == int(np.argmax(got)) and np.abs(got - want[-1]).max() < 2e-3 * np.abs(want[-1]).max()
+    finally:
+        dec.close()
