@@ -1187,6 +1187,7 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   }
   a.rounds = (slots + a.teams - 1u) / a.teams;
   a.waves = rotated || gemv_wide(a.nb) ? kGemvMaxWaves : gemv_waves(a.team, a.teams, slots);
+  if (a.in.prologue == kPrologueAddRmsNorm) a.waves = std::max(a.waves, gemv_norm_waves(a.nb));
   a.passes = stage_passes(a.nb, a.waves);
   a.inv_team = (65536u + a.team - 1u) / a.team;
   a.inv_teams = (65536u + a.teams - 1u) / a.teams;

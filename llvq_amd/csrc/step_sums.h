@@ -37,6 +37,11 @@ LLVQ_HD uint32_t gemv_waves(uint32_t team, uint32_t teams, uint32_t tiles) {
   const uint32_t at_a_time = gemv_batch(team) * teams, finish = tiles < at_a_time ? tiles : at_a_time;
   return team * teams + finish < kGemvMaxWaves ? team * teams + finish : kGemvMaxWaves;
 }
+// Wavefronts below which a launch that norms its row does not go.  A row's squares are added a wavefront at a time, each over its sixteen blocks
+// of every pass, and the wavefronts' sums in order: with a wavefront for every sixteen blocks, or with all sixteen, as sequences have them, that
+// is one order whatever shares the launch.  (With fewer, 2560 columns in five wavefronts for instance, one row in eight had another norm than in
+// a sequence, in its last bit.)
+LLVQ_HD uint32_t gemv_norm_waves(uint32_t nb) { return 2u * tile_steps(nb) < kGemvMaxWaves ? 2u * tile_steps(nb) : kGemvMaxWaves; }
 
 // The array: kGemvRounds rounds of as many steps as a workgroup's teams take together, and room behind them for what a sum reads past
 // its tile's steps and does not use: the places to read are then the same for every tile.  (Each held back by the number of steps,

@@ -769,3 +769,33 @@ def test_results_where_the_last_launch_leaves_them(gpu_rt, orc, vocab):
         assert best == int(np.argmax(got)) and np.abs(got - want[-1]).max() < 2e-3 * np.abs(want[-1]).max()
     finally:
         dec.close()
+
+
+# Two passes of the launch's quads over the row where it has as many wavefronts as its tiles ask for, one with sixteen (2560: 5 wavefronts to 128
+# blocks, 1200: 3 to 64, 5208: 9 to 224), and two whatever it has (8192: 352 blocks)
+@pytest.mark.parametrize("hidden,n", [(1200, 60), (2560, 60), (5208, 30), (8192, 60)])
+def test_a_norm_does_not_depend_on_what_shares_its_launch(gpu_rt, hidden, n):
+    """The f32 sum of a row's squares is formed in one order, however many wavefronts a launch has: the last bit of the norm, and with it binary16
+    values of the normed row, would differ between the launch modes for about one row in eight."""
+    from llvq_amd import _ffi
+
+    cfg = decoder.Qwen3Config(num_hidden_layers=2, hidden_size=hidden, num_attention_heads=2, num_key_value_heads=1, head_dim=64, intermediate_size=72,
+                              vocab_size=96, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=64, tie_word_embeddings=True)
+    weights = decoder.synthetic_weights(cfg, hidden)
+    projs = [[gpu_rt.upload(m) for m in layer] for layer in decoder.synthetic_projections(cfg, hidden)]
+    decs = [decoder.Decoder(gpu_rt, cfg, projs, weights, launch_mode=m) for m in (_ffi.LAUNCH_PER_GROUP, _ffi.LAUNCH_SINGLE, _ffi.LAUNCH_CHAINED)]
+    try:
+        apart = []
+        for i, t in enumerate(np.random.default_rng(hidden).permutation(cfg.vocab_size)[:n]):
+            first, *others = [d.forward_token(int(t))[0] for d in decs]
+            assert np.isfinite(first).all()
+            apart += [i for o in others if not np.array_equal(first, o)]
+            for d in decs:  # (each token by itself)
+                d.reset()
+        assert not apart, f"{len(apart)} of {2 * n} logits differ, first at token {apart[0]}"
+    finally:
+        for d in decs:
+            d.close()
+        for layer in projs:
+            for p in layer:
+                gpu_rt.free(p)
