@@ -1705,6 +1705,16 @@ static bool gemm_direct(uint32_t M, uint32_t n_tiles, uint32_t nb, uint32_t cus,
   const uint32_t units = (n_tiles + cus - 1u) / cus * tile_units(nb);  // of the fullest CU
   return M <= 3u || (M - 3u) * units < 20u * 16u;
 }
+// Whether one of the results lies over the rows, be it in part.  Such rows are not read where they are: octets are whole before the
+// product that stores begins.
+static bool stored_over_rows(const void* x, size_t x_bytes, const llvq_mat* const* mats, int n, uint32_t M, void* const* y, int y_dtype) {
+  const uintptr_t x0 = reinterpret_cast<uintptr_t>(x);
+  for (int i = 0; i < n; ++i) {
+    const uintptr_t y0 = reinterpret_cast<uintptr_t>(y[i]);
+    if (y0 < x0 + x_bytes && x0 < y0 + (size_t)M * mats[i]->d_out * (y_dtype == LLVQ_F32 ? 4u : 2u)) return true;
+  }
+  return false;
+}
 // One launch over n <= kGemmMaxGroup matrices of equal d_in that take the same activations
 // (already in the matrices' basis), M <= kGemmMaxM rows.  from: rows that are rotated on the way to the octets, their tail
 // columns to x.
@@ -1741,7 +1751,8 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   a.m_tiles = p.m_tiles;
   a.splits = p.splits;
   a.steps_per_split = p.steps_per_split;
-  const bool direct = !from && !make && p.small == 1u && gemm_direct(M, a.n_tiles, a.nb, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), pair);
+  const bool direct = !from && !make && p.small == 1u && gemm_direct(M, a.n_tiles, a.nb, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), pair) &&
+                      !stored_over_rows(x, (size_t)M * m0->d_in * 2u, mats, n, M, y, y_dtype);
   a.xs = direct ? reinterpret_cast<const uint8_t*>(x) : reinterpret_cast<const uint8_t*>(xt_buf);
   a.xs_octet = direct ? 16u : p.m_pad * 16u;
   a.xs_block = 3u * a.xs_octet;

@@ -420,3 +420,36 @@ def test_small_batches_read_their_rows_and_no_others(gpu_rt, orc, d_out, d_in, r
             assert not torch.isfinite(got[first::2]).any()
     finally:
         gpu_rt.free(proj)
+
+
+# more tiles than are on the card at once, where the last would read what the first have stored; one tile to a CU and less; the wide kernel
+@pytest.mark.parametrize("width,rows", [(9600, 2), (9600, 3), (9600, 4), (2400, 5), (2400, 16), (96, 7), (2400, 17), (2400, 65)])
+def test_results_stored_over_the_rows(gpu_rt, width, rows):
+    """Rows of whole blocks are taken as octets before a result is stored over them: all of the rows, a part, by one of a group's matrices."""
+    import torch
+
+    projs = [gpu_rt.upload(synth.make_matrix(f"model.layers.0.o{i}.weight", width, width, seed=width + i)) for i in range(2)]
+    try:
+        x = _x16(synth.make_activation(width, seed=rows, rows=rows))
+        want = [gpu_rt.forward_batched(p, x) for p in projs]
+        y = x.clone()
+        gpu_rt.forward_batched_into(projs[0], y, y)
+        assert torch.equal(y, want[0])
+        want = gpu_rt.forward_batched_group_into(projs, x, [torch.empty_like(x) for _ in projs])  # (a group's columns may be split otherwise)
+        both, other = x.clone(), torch.empty_like(x)
+        gpu_rt.forward_batched_group_into(projs, both, [other, both])
+        assert torch.equal(other, want[0]) and torch.equal(both, want[1])
+        want = gpu_rt.forward_batched(projs[0], x)
+        for rows_in, rows_out in ((slice(0, rows), slice(1, rows + 1)), (slice(1, rows + 1), slice(0, rows))):
+            buf = torch.zeros(rows + 1, width, dtype=torch.float16, device="cuda")
+            buf[rows_in] = x
+            gpu_rt.forward_batched_into(projs[0], buf[rows_in], buf[rows_out])
+            assert torch.equal(buf[rows_out], want)
+        wide = torch.zeros(2 * rows, width, dtype=torch.float16, device="cuda")
+        wide[rows // 2:rows // 2 + rows] = x
+        want32 = gpu_rt.forward_batched(projs[0], x, out_dtype=torch.float32)
+        gpu_rt.forward_batched_into(projs[0], wide[rows // 2:rows // 2 + rows], wide.view(torch.float32).view(rows, width))
+        assert torch.equal(wide.view(torch.float32).view(rows, width), want32)
+    finally:
+        for p in projs:
+            gpu_rt.free(p)
