@@ -155,20 +155,46 @@ def lib():
     return L
 
 
-_calls = None
+_CALLS = os.path.join(_HERE, "_calls.so")
+_calls = _NOT_ASKED = object()
+
+
+def _built_for():
+    """What csrc/bind.cpp has to have been built for (its Makefile writes the same into it)."""
+    import sysconfig
+
+    import torch
+
+    return f"{torch.__version__}/{sysconfig.get_config_var('SOABI')}"
 
 
 def calls():
     """The operator's calls as one native step each (csrc/bind.cpp), bound to the library that is loaded here; None where that module was
-    not built for this interpreter: fused.py then makes them itself.  torch has to be imported."""
+    not built, or (with a warning) not for this interpreter and this torch: fused.py then makes them itself.  torch has to be imported."""
     global _calls
-    if _calls is None and os.path.exists(os.path.join(_HERE, "_calls.so")):
-        from . import _calls as module
+    if _calls is _NOT_ASKED:
+        _calls = None
+        if os.path.exists(_CALLS):
+            try:
+                _calls = _load_calls()
+            except (ImportError, SystemError, AttributeError) as e:
+                import warnings
 
-        L = lib()
-        module.bind_library(*(C.cast(f, C.c_void_p).value for f in (L.llvq_hip_gemv, L.llvq_hip_gemv_group, L.llvq_hip_gemm, L.llvq_hip_gemm_group)))
-        _calls = module
+                warnings.warn(f"{_CALLS} is not used: {e}; rebuild it with `make -B -C {os.path.join(_HERE, 'csrc')} ../_calls.so`", RuntimeWarning)
     return _calls
+
+
+def _load_calls():
+    import importlib.util
+
+    spec = importlib.util.spec_from_file_location(__package__ + "._calls", _CALLS)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    if module.built_for != _built_for():
+        raise ImportError(f"it was built for {module.built_for}, this is {_built_for()}")
+    L = lib()
+    module.bind_library(*(C.cast(f, C.c_void_p).value for f in (L.llvq_hip_gemv, L.llvq_hip_gemv_group, L.llvq_hip_gemm, L.llvq_hip_gemm_group)))
+    return module
 
 
 def check(rc):

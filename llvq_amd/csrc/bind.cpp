@@ -247,5 +247,8 @@ PyMODINIT_FUNC PyInit__calls() {
   g_handle = PyUnicode_InternFromString("_at");
   g_d_in = PyUnicode_InternFromString("d_in");
   g_d_out = PyUnicode_InternFromString("d_out");
-  return g_handle && g_d_in && g_d_out ? PyModule_Create(&kModule) : nullptr;
+  PyObject* module = g_handle && g_d_in && g_d_out ? PyModule_Create(&kModule) : nullptr;
+  // the torch and the interpreter of the build: _ffi.py makes no call here under others
+  if (module && PyModule_AddStringConstant(module, "built_for", LLVQ_BUILT_FOR)) Py_CLEAR(module);
+  return module;
 }
