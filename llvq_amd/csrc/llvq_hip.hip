@@ -1259,9 +1259,9 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
 
 // Whether a layer's gate and up are one launch that leaves silu(gate) up.  Not in a rotated basis, where down_proj's rotation forms it, a
 // sixteenth in each wavefront: 4831 us against 4879 for eight tokens through four 14B layers, since pairs of tiles spread less evenly.
+// (Rows of up to 8192 columns, a decoder's widest, have as many steps as there are wavefronts at the most, and the sums of pairs fit LDS.)
 static bool gated_fits(const llvq_mat* gate, const llvq_mat* up) {
-  return !gate->has_rotation && !up->has_rotation && gate->nblocks && !gemv_wide(gate->nblocks) &&
-         gemv_tiles_lds_bytes(gate->nblocks, gate->d_in, false, false, true) <= 160 * 1024;
+  return !gate->has_rotation && !up->has_rotation && gate->nblocks;
 }
 
 static int launch_gemv(llvq_rt* rt, const llvq_mat* m, const void* x, void* y, int y_dtype) {

@@ -30,6 +30,8 @@ int main() {
       }
     }
   }
+  // A decoder's widest row: gate and up as one result fit, rows of one step to a wavefront.
+  if (gemv_wide(8192 / kDim) || gemv_tiles_lds_bytes(8192 / kDim, 8192, false, false, true) > 160u * 1024u) return 1;
   // The rotated rows that are rotated in their product's launch, which has 160 KB: of the widths a rotation can have these are the widest.
   const struct { uint32_t width; bool f32, fits; } rotated[] = {{19456, true, true},  {20480, true, true},  {21504, true, false},
                                                                 {23552, false, true}, {24576, false, true}, {17408, true, true}};

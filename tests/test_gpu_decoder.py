@@ -799,3 +799,32 @@ def test_a_norm_does_not_depend_on_what_shares_its_launch(gpu_rt, hidden, n):
         for layer in projs:
             for p in layer:
                 gpu_rt.free(p)
+
+
+# gate and up rotated, one of them, or of rows without a block; down in the natural basis, narrow and past 512 blocks (the wide form), with tail columns
+@pytest.mark.parametrize("hidden,inter,rotated", [(256, 328, (4, 5)), (256, 12328, (4, 5)), (256, 328, (5,)), (256, 12328, (4,)), (16, 328, ()), (16, 12328, ()),
+                                                  (8, 72, ())])
+def test_silu_formed_by_down_projections_launch(gpu_rt, orc, hidden, inter, rotated):
+    """Where gate and up are not one launch, down_proj's forms silu(gate) up from the two results."""
+    from oracle import qwen3_oracle
+
+    cfg = decoder.Qwen3Config(num_hidden_layers=2, hidden_size=hidden, num_attention_heads=4, num_key_value_heads=2, head_dim=32, intermediate_size=inter,
+                              vocab_size=100, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=16, tie_word_embeddings=True)
+    raws = decoder.synthetic_projections(cfg, inter)
+    for li, layer in enumerate(raws):
+        for i in rotated:
+            layer[i].rotation_seed = 100 * li + 7
+    weights = decoder.synthetic_weights(cfg, inter)
+    dense = [[orc.read_matrix_raw(artifact.write_matrix_raw(m))[0].decode_matrix() for m in layer] for layer in raws]
+    ref, dec = qwen3_oracle.Qwen3Oracle(cfg, dense, weights), decoder.Decoder(gpu_rt, cfg, raws, weights)
+    try:
+        worst = 0.0
+        for t in np.random.default_rng(hidden).integers(0, cfg.vocab_size, size=8):
+            want = ref.forward_token(int(t))
+            got, best = dec.forward_token(int(t))
+            assert best == int(np.argmax(got))
+            worst = max(worst, float(np.abs(got - want).max() / np.abs(want).max()))
+        print(f"OBSERVED silu_by_down {hidden}/{inter}/{rotated}: {worst:.3e}")
+        assert worst < BAR_SMALL  # (1.3e-4 observed)
+    finally:
+        dec.close()
