@@ -1165,36 +1165,17 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   a.nb = m0->nblocks;
   a.tail_w = m0->tail_w;
   a.n_mats = (uint32_t)n;
-  a.team = gemv_team(m0->nblocks);
   for (int i = 0; i < n; ++i) {
     a.m[i] = TileMat{mats[i]->tiles, gated ? y[0] : y[i], mats[i]->d_out, a.n_tiles, mats[i]->stride, mats[i]->slots};
     a.n_tiles += tile_count(mats[i]->d_out);
   }
-  // Teams go to as many CUs as there are tiles for, then to the same CU, up to sixteen wavefronts: a small launch
-  // is short because every CU has a part of it, a large one because a CU keeps sixteen wavefronts' loads in flight.
-  // The in-launch rotation and the wide rows are written for a full workgroup, whatever of it has a tile.
-  const uint32_t cus = (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
-  uint32_t slots;  // tiles of the fullest workgroup
-  if (gated) {
-    const uint32_t pairs = a.m[1].tile_begin;
-    a.grid = std::min(cus, pairs);
-    slots = 2u * ((pairs + a.grid - 1u) / a.grid);
-    a.teams = gated_teams(slots, a.team);
-  } else {
-    a.teams = std::min((a.n_tiles + cus - 1u) / cus, kGemvMaxWaves / a.team);
-    a.grid = std::min(cus, (a.n_tiles + a.teams - 1u) / a.teams);
-    slots = (a.n_tiles + a.grid - 1u) / a.grid;
-  }
-  a.rounds = (slots + a.teams - 1u) / a.teams;
-  a.waves = rotated || gemv_wide(a.nb) ? kGemvMaxWaves : gemv_waves(a.team, a.teams, slots);
-  if (a.in.prologue == kPrologueAddRmsNorm) a.waves = std::max(a.waves, gemv_norm_waves(a.nb));
-  a.passes = stage_passes(a.nb, a.waves);
-  a.inv_team = (65536u + a.team - 1u) / a.team;
-  a.inv_teams = (65536u + a.teams - 1u) / a.teams;
+  // (The in-launch rotation and the wide rows are written for a full workgroup, whatever of it has a tile.)
+  a.g = gemv_grid(a.nb, gated ? a.m[1].tile_begin : a.n_tiles, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), gated, rotated || gemv_wide(a.nb),
+                  a.in.prologue == kPrologueAddRmsNorm);
   const int src = rotated ? kSrcRotated : a.in.prologue == kPrologueSiluMul ? kSrcSiluMul : a.in.prologue == kPrologueAddRmsNorm ? kSrcAddRmsNorm : kSrcF16;
   void* params[] = {&a};
-  HIP_TRY(hipLaunchKernel(gated ? reinterpret_cast<const void*>(gated_product_kernel) : gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(a.grid),
-                          dim3(a.waves * 64u), params, gemv_tiles_lds_bytes(a.nb, m0->d_in, f32, rot != nullptr, gated), rt->stream));
+  HIP_TRY(hipLaunchKernel(gated ? reinterpret_cast<const void*>(gated_product_kernel) : gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(a.g.grid),
+                          dim3(a.g.waves * 64u), params, gemv_tiles_lds_bytes(a.nb, m0->d_in, f32, rot != nullptr, gated), rt->stream));
   return LLVQ_OK;
 }
 

@@ -58,6 +58,40 @@ LLVQ_HD uint32_t gated_teams(uint32_t slots, uint32_t team) {
   if (!((gemv_batch(team) * teams) & 1u)) return teams;
   return teams < most ? teams + 1u : teams - 1u;  // (such a team is of seven wavefronts at the most: most >= 2)
 }
+// A launch's workgroups, their teams and wavefronts, as the host lays them out.  Slot i of a workgroup is tile i * grid + its number (gated: of
+// pairs of slots); round r of team t is slot r * teams + t.
+struct GemvGrid {
+  uint32_t team, teams;          // wavefronts of a team, teams of a workgroup
+  uint32_t waves, grid, passes;  // wavefronts (those that no team has only stage the activation); workgroups; how often the former pass over the activation
+  uint32_t inv_team, inv_teams;  // 2^16 / team and 2^16 / teams, rounded up: exact for the seventeen numbers that are divided
+  uint32_t rounds;               // tiles of a team, at the most
+};
+// tiles: of all matrices, or pairs of them (gated).  full: sixteen wavefronts whatever there is for them.  norm: the launch norms its row.
+// Teams go to as many CUs as there are tiles for, then to the same CU, up to sixteen wavefronts: a small launch
+// is short because every CU has a part of it, a large one because a CU keeps sixteen wavefronts' loads in flight.
+inline GemvGrid gemv_grid(uint32_t nb, uint32_t tiles, uint32_t cus, bool gated, bool full, bool norm) {
+  GemvGrid g{};
+  g.team = gemv_team(nb);
+  uint32_t slots;  // tiles of the fullest workgroup
+  if (gated) {
+    g.grid = cus < tiles ? cus : tiles;
+    slots = 2u * ((tiles + g.grid - 1u) / g.grid);
+    g.teams = gated_teams(slots, g.team);
+  } else {
+    const uint32_t each = (tiles + cus - 1u) / cus, most = kGemvMaxWaves / g.team;
+    g.teams = each < most ? each : most;
+    const uint32_t filled = (tiles + g.teams - 1u) / g.teams;
+    g.grid = cus < filled ? cus : filled;
+    slots = (tiles + g.grid - 1u) / g.grid;
+  }
+  g.rounds = (slots + g.teams - 1u) / g.teams;
+  g.waves = full ? kGemvMaxWaves : gemv_waves(g.team, g.teams, slots);
+  if (norm && g.waves < gemv_norm_waves(nb)) g.waves = gemv_norm_waves(nb);
+  g.passes = stage_passes(nb, g.waves);
+  g.inv_team = (65536u + g.team - 1u) / g.team;
+  g.inv_teams = (65536u + g.teams - 1u) / g.teams;
+  return g;
+}
 // The step that a lane of class c reads as its i-th.
 LLVQ_HD uint32_t sums_read(uint32_t i, uint32_t c) { return 4u * i + c; }
 // In LDS the four blocks of a unit lie together: 3 dwords per digit and block, then each block's sum of its integers

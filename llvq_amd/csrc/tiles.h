@@ -313,11 +313,7 @@ struct TileMat {
 struct GemvArgs {
   ActivationIn in;
   uint32_t nb, tail_w, n_mats, n_tiles;
-  uint32_t team, teams;  // wavefronts of a team, teams of a workgroup (more wavefronts only stage the activation)
-  // What the host knows as well, so that no wavefront works it out: its workgroup's wavefronts, the workgroups, how often the former
-  // pass over the activation, 2^16 / team and 2^16 / teams, rounded up (exact for the seventeen numbers that are divided).
-  uint32_t waves, grid, passes, inv_team, inv_teams;
-  uint32_t rounds;  // tiles of a team, at the most
+  GemvGrid g;  // what the host knows as well, so that no wavefront works it out
   TileMat m[kMaxGroup];
 };
 // Asks for all of a launch's arguments at once: each of their cache lines is a miss of its own, and the compiler would load
@@ -971,13 +967,13 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
   const GemvLds L = gemv_lds<DIG>(smem, gemv_plane_units(a.nb));
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-  const uint32_t team = (wave * a.inv_team) >> 16, w = wave - team * a.team, n_teams = a.teams * a.grid;
+  const uint32_t team = (wave * a.g.inv_team) >> 16, w = wave - team * a.g.team, n_teams = a.g.teams * a.g.grid;
   const uint32_t nb = a.nb, n_steps = tile_steps(nb), units = tile_units(nb), head = tile_head_bytes(a.tail_w);
 
   struct Record { const uint8_t* rec; const uint8_t* base; uint32_t slots; };
   // A workgroup's slot i of tiles is tile i * grid + its number; with GATED that tile of pairs of slots, the even one in the first matrix.
   const uint32_t n_tiles = GATED ? a.m[1].tile_begin : a.n_tiles;
-  auto tile_of = [&](uint32_t slot) { return (GATED ? slot >> 1 : slot) * a.grid + blockIdx.x; };
+  auto tile_of = [&](uint32_t slot) { return (GATED ? slot >> 1 : slot) * a.g.grid + blockIdx.x; };
   auto record_of = [&](uint32_t t, uint32_t slot) {
     const uint8_t* base;
     void* y;
@@ -996,7 +992,7 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
   uint32_t off[kSteps];  // (where a wavefront has no step, or no next tile, its loads repeat one: one cache line, and no branch)
 #pragma unroll
   for (uint32_t j = 0; j < kSteps; ++j) off[j] = step_offset(w + j * kGemvMaxWaves, units, head, lane);
-  uint32_t tile = team < a.teams ? tile_of(team) : 0xFFFFFFFFu;
+  uint32_t tile = team < a.g.teams ? tile_of(team) : 0xFFFFFFFFu;
   Record cur = record_of(min(tile, n_tiles - 1u), team);
   StepWords W[kSteps];
   constexpr uint32_t kFirst = SRC == kSrcRotated ? 1u : kSteps;  // (beside a rotation's operands there are registers for one)
@@ -1004,17 +1000,17 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
   // The tile that this wavefront finishes of those whose rounds begin with r0: the last wavefronts see to the first tiles, since what a tile
   // has besides its steps (tile_extras, 0.8 us for one wavefront) is then not in front of anybody's products where there are
   // wavefronts without any.
-  const uint32_t fin = a.waves - 1u - wave, batch = gemv_batch(a.team), my_round = (fin * a.inv_teams) >> 16, my_team = fin - my_round * a.teams;
+  const uint32_t fin = a.g.waves - 1u - wave, batch = gemv_batch(a.g.team), my_round = (fin * a.g.inv_teams) >> 16, my_team = fin - my_round * a.g.teams;
   TileExtras extras;
   uint32_t extras_table;
-  auto finished = [&](uint32_t r0) { return my_round < batch ? tile_of(r0 * a.teams + fin) : 0xFFFFFFFFu; };
+  auto finished = [&](uint32_t r0) { return my_round < batch ? tile_of(r0 * a.g.teams + fin) : 0xFFFFFFFFu; };
   auto load_finish = [&](uint32_t r0) {
     const uint32_t t = finished(r0);
     const Record r = record_of(min(t, n_tiles - 1u), fin);  // (a batch of rounds has an even number of slots where that matters: gated_teams)
     extras = load_extras(r.rec, nb, a.tail_w, r.slots, t < n_tiles, lane);
     extras_table = scale_table(r.base, lane);
   };
-  stage_x<DIG, SRC, WIDE ? 4 : 2>(a.in, nb, a.tail_w, a.waves, a.passes, L, blockIdx.x == 0, [&]() {
+  stage_x<DIG, SRC, WIDE ? 4 : 2>(a.in, nb, a.tail_w, a.g.waves, a.g.passes, L, blockIdx.x == 0, [&]() {
     if constexpr (SRC != kSrcRotated) load_finish(0);  // little, and it has a use while the pieces come
     table = scale_table(cur.base, lane);
     const uint8_t* base = scalar_base(cur.rec);
@@ -1027,7 +1023,7 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
   lds_barrier();
 
   // (In a rotated basis there is no scalar register to keep it in: 2560 x 9728 takes 11.5 us like this, 11.8 with the argument.)
-  const uint32_t rounds = SRC == kSrcRotated ? (a.n_tiles + n_teams - 1u) / n_teams : a.rounds;
+  const uint32_t rounds = SRC == kSrcRotated ? (a.n_tiles + n_teams - 1u) / n_teams : a.g.rounds;
   for (uint32_t r0 = 0; r0 < rounds; r0 += batch) {
     const uint32_t r1 = min(r0 + batch, rounds), o_tile = finished(r0);
     const float o_scale = extras.scale;
@@ -1040,12 +1036,12 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
       if ((fin & 1u) && lane_class(lane) == 0u) *reinterpret_cast<float2*>(L.part + gated_at(WIDE) + (fin * kTileRows + lane_row(lane)) * 2u) = make_float2(o_scale, o_extra);
     if (r1 != rounds) load_finish(r1);
     for (uint32_t rd = r0; rd < r1 && tile < n_tiles; ++rd) {
-      const uint32_t next = GATED ? tile_of((rd + 1u) * a.teams + team) : tile + n_teams;
+      const uint32_t next = GATED ? tile_of((rd + 1u) * a.g.teams + team) : tile + n_teams;
       const bool more = next < n_tiles;
-      const Record nx = record_of(min(next, n_tiles - 1u), (rd + 1u) * a.teams + team);
+      const Record nx = record_of(min(next, n_tiles - 1u), (rd + 1u) * a.g.teams + team);
       const uint32_t lanes_table = table, keep = more ? 0xFFFFFFFFu : 0u;
       const uint8_t* base = scalar_base(nx.rec);
-      float* const part = L.part + sums_at(rd - r0, team, a.team, WIDE) * kTileRows;
+      float* const part = L.part + sums_at(rd - r0, team, a.g.team, WIDE) * kTileRows;
       table = scale_table(nx.base, lane);  // in front of the pieces, so that the next round waits for it alone
 #pragma unroll
       for (uint32_t j = 0; j < kSteps; ++j) {
@@ -1063,8 +1059,8 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
     if constexpr (GATED) {
       if (o_tile < n_tiles && !(fin & 1u)) {
         auto sum_of = [&](uint32_t slot) {
-          const uint32_t round = (slot * a.inv_teams) >> 16;
-          return steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(round, slot - round * a.teams, a.team, WIDE) * kTileRows, n_steps, lane);
+          const uint32_t round = (slot * a.g.inv_teams) >> 16;
+          return steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(round, slot - round * a.g.teams, a.g.team, WIDE) * kTileRows, n_steps, lane);
         };
         const float2 up_scale = *reinterpret_cast<const float2*>(L.part + gated_at(WIDE) + ((fin + 1u) * kTileRows + lane_row(lane)) * 2u);
         const float gate = fmaf(sum_of(fin), o_scale, o_extra), up = fmaf(sum_of(fin + 1u), up_scale.x, up_scale.y);
@@ -1076,7 +1072,7 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
       void* o_y;
       uint32_t o_row0, o_d_out, o_stride, o_slots;
       tile_mat(a, o_tile, o_base, o_y, o_row0, o_d_out, o_stride, o_slots);
-      const float v = steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(my_round, my_team, a.team, WIDE) * kTileRows, n_steps, lane);
+      const float v = steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(my_round, my_team, a.g.team, WIDE) * kTileRows, n_steps, lane);
       const uint32_t row = o_row0 + lane_row(lane);
       if (lane_class(lane) == 0u && row < o_d_out) store_out<OutT>(o_y, row, fmaf(v, o_scale, o_extra));
     }
