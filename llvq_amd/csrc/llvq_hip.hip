@@ -1238,8 +1238,9 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
   return LLVQ_OK;
 }
 
-// Whether a layer's gate and up are one launch that leaves silu(gate) up.  Not in a rotated basis, where down_proj's rotation forms it, a
-// sixteenth in each wavefront: 4831 us against 4879 for eight tokens through four 14B layers, since pairs of tiles spread less evenly.
+// Whether a layer's gate and up are one launch that leaves silu(gate) up: 37.8, 44.9 and 63.8 us a layer and token of a decode of four layers at the widths of
+// 4B, 8B and 14B models, 38.7, 45.9 and 65.0 as two results that down_proj's launch takes.  Not in a rotated basis, which has no such kernel: down_proj's
+// rotation forms it there, a sixteenth in each wavefront.  (One for it would pay as well: 51.0, 56.2 and 78.0 us are 49.6, 54.6 and 77.3 with it.)
 // (Rows of up to 8192 columns, a decoder's widest, have as many steps as there are wavefronts at the most, and the sums of pairs fit LDS.)
 static bool gated_fits(const llvq_mat* gate, const llvq_mat* up) {
   return !gate->has_rotation && !up->has_rotation && gate->nblocks;
@@ -2318,8 +2319,8 @@ HostResults host_results(llvq_decoder* d, const float* logits_host, const uint32
 }
 // The wait for a step's results, and their way to the caller's memory.  A copy straight to that (pageable) memory is staged by the
 // runtime, one for each result, and begins when the stream has been waited for.  With pinned memory they are there when the
-// step ends, and while it runs the pages that they go to are touched, which for fresh memory is most of what moving
-// them costs: a token through four 14B layers takes 686 us, not 712.
+// step ends (argmax_final_kernel has the times), and while it runs the pages that they go to are touched, which for fresh memory is most of
+// what moving them costs.
 int decoder_results(llvq_decoder* d, float* logits_host, uint32_t* argmax_host) {
   hipStream_t st = d->rt->stream;
   const size_t bytes = (size_t)d->vocab * sizeof(float);
