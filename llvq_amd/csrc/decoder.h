@@ -38,8 +38,9 @@ __global__ __launch_bounds__(256) void embed_kernel(const __half* __restrict__ t
 // wavefronts where one has work, 500 rows of 2560 took 5.2 us.
 // (A prompt's passes: the launches that brought rows into octets are gone, 500 tokens through twelve 4B layers 3215 -> 3067 us.)
 // to: the normed rows go there as octets (a workgroup for each of m_pad rows), and only their tail columns to `normed`.
+// sums: delta is what a product left in parts, added up and rounded here.
 __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(const __half* h, const __half* __restrict__ delta, const __half* __restrict__ w,
-                                                           __half* h_out, __half* __restrict__ normed, uint32_t n, float eps, Octets to) {
+                                                           __half* h_out, __half* __restrict__ normed, uint32_t n, float eps, Octets to, GemmSums sums) {
   __shared__ float red[16];
   const uint32_t at = threadIdx.x * 8u, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   uint32_t m = blockIdx.x;
@@ -53,8 +54,16 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(const __half* h, cons
   const uint32_t from = in ? at : 0u;
   HalfOctet x = *reinterpret_cast<const HalfOctet*>(h + row + from);
   const HalfOctet g = *reinterpret_cast<const HalfOctet*>(w + from);
-  if (delta) {  // the residual stream is binary16
-    const HalfOctet d = *reinterpret_cast<const HalfOctet*>(delta + row + from);
+  if (delta || sums.ws) {  // the residual stream is binary16
+    HalfOctet d;
+    if (sums.ws) {
+      float v[8];
+      parts_read(sums, m, sums.first[0] + from, v);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d.w[j] = pack_halves(v[2 * j], v[2 * j + 1]);
+    } else {
+      d = *reinterpret_cast<const HalfOctet*>(delta + row + from);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       x.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(half_lo(x.w[j]) + half_lo(d.w[j]))) |
@@ -224,29 +233,69 @@ constexpr int kAttnInlineSplits = 16;  // up to this many ranges, the workgroup 
 // One wavefront per (head, row), four to a workgroup: q heads are normed and rotated in place, k heads are
 // normed, rotated and appended to the cache at position pos0 + row, v heads are appended.
 // Grid (a quarter of n_heads + 2 n_kv, rows).  Same arithmetic as the one-position path.
+// sums: heads of 128 come as what the product left in parts, and are added up and rounded here.
 template <bool Q8>
 __global__ __launch_bounds__(256) void norm_rope_append_rows_kernel(__half* __restrict__ q, const __half* __restrict__ k,
                                                                    const __half* __restrict__ v, AttnNew nw, KvQ8 q8,
                                                                    uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
-                                                                   uint32_t pos0, uint32_t max_pos) {
+                                                                   uint32_t pos0, uint32_t max_pos, GemmSums sums) {
   __shared__ float stages[4][256];
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t head = blockIdx.x * 4u + wave, row = blockIdx.y, lane = threadIdx.x & 63u;
   if (head >= n_heads + 2u * n_kv) return;
   float* stage = stages[wave];
   const uint32_t pos = pos0 + row, kvgroups = head_dim / kKvGroup;
+  __half x1{}, x2{};  // of sums: elements lane and lane + 64
+  const auto from_sums = [&](const __half* w) {
+    const RopeAngle a{nw.cos_t[(size_t)pos * 64 + lane], nw.sin_t[(size_t)pos * 64 + lane]};
+    const float2 r = norm_rope_128(HeadOperands{x1, x2, w[lane], w[lane + 64]}, a, nw.eps);
+    stage[lane] = r.x;
+    stage[lane + 64] = r.y;
+    wave_lds_sync();
+  };
+  if (sums.ws) {
+    const uint32_t of = head < n_heads ? head : head < n_heads + n_kv ? head - n_heads : head - n_heads - n_kv;
+    const uint32_t first = head < n_heads ? sums.first[0] : head < n_heads + n_kv ? sums.first[1] : sums.first[2];
+    const float* from = uniform_global(sums.ws + (size_t)row * sums.ld + first + of * 128u);
+    const size_t step = (size_t)sums.m_pad * sums.ld;
+    float a = 0.f, b = 0.f;
+    for (uint32_t p0 = 0; p0 < sums.splits; p0 += kReduceSplits) {
+      float va[kReduceSplits], vb[kReduceSplits];
+#pragma unroll
+      for (uint32_t p = 0; p < kReduceSplits; ++p) {
+        const float* at = from + min(p0 + p, sums.splits - 1u) * step;
+        va[p] = at[lane];
+        vb[p] = at[lane + 64u];
+      }
+#pragma unroll
+      for (uint32_t p = 0; p < kReduceSplits; ++p) {
+        if (p0 + p >= sums.splits) break;
+        a += va[p];
+        b += vb[p];
+      }
+    }
+    x1 = __float2half_rn(a);
+    x2 = __float2half_rn(b);
+  }
   if (head < n_heads) {
     __half* qh = q + ((size_t)row * n_heads + head) * head_dim;
-    norm_rope_wave(qh, nw.qn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage, lane);
+    if (sums.ws) from_sums(nw.qn);
+    else norm_rope_wave(qh, nw.qn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage, lane);
     for (uint32_t i = lane; i < head_dim; i += 64) qh[i] = __float2half_rn(stage[i]);
     return;
   }
   const bool is_k = head < n_heads + n_kv;
   const uint32_t kvh = is_k ? head - n_heads : head - n_heads - n_kv;
   const __half* src = (is_k ? k : v) + ((size_t)row * n_kv + kvh) * head_dim;
-  if (is_k) norm_rope_wave(src, nw.kn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage, lane);
+  if (is_k && sums.ws) from_sums(nw.kn);
+  else if (is_k) norm_rope_wave(src, nw.kn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage, lane);
   else {
-    for (uint32_t i = lane; i < head_dim; i += 64) stage[i] = __half2float(src[i]);
+    if (sums.ws) {
+      stage[lane] = __half2float(x1);
+      stage[lane + 64] = __half2float(x2);
+    } else {
+      for (uint32_t i = lane; i < head_dim; i += 64) stage[i] = __half2float(src[i]);
+    }
     wave_lds_sync();
   }
   const size_t crow = (size_t)kvh * max_pos + pos;

@@ -283,6 +283,46 @@ __device__ __forceinline__ void touch_args(const GemmArgs& a) {
   asm volatile("" ::"s"(a.ws), "s"(a.mat[1].base), "s"(a.mat[3].base), "s"(a.M), "s"(a.xs_last));
 }
 
+// What a product whose columns are split leaves for the launch behind it: value r of activation row m of matrix i is the sum, in order, of
+// ws[(p m_pad + m) ld + first[i] + r] over the splits p.  No splits: the results are where they belong.  (A prompt's norms and its heads' norms
+// read them: a launch of 9 us less for q/k/v, o and down of each layer, and results that do not go through memory a second time.  500 tokens of
+// twelve 4B layers 2916 -> 2697 us with it and what is said at the product's end.)
+struct GemmSums {
+  const float* ws;
+  uint32_t splits, m_pad, ld;
+  uint32_t first[kGemmMaxGroup];
+};
+constexpr uint32_t kReduceSplits = 4;  // whose values are asked for together
+// N values of row m from place `at` on (at a multiple of four)
+template <uint32_t N>
+__device__ __forceinline__ void parts_read(const GemmSums& s, uint32_t m, uint32_t at, float (&out)[N]) {
+  static_assert(N % 4 == 0, "in sixteens of bytes");
+#pragma unroll
+  for (uint32_t i = 0; i < N; ++i) out[i] = 0.f;
+  const size_t step = (size_t)s.m_pad * s.ld;
+  const float* from = s.ws + (size_t)m * s.ld + at;
+  for (uint32_t p0 = 0; p0 < s.splits; p0 += kReduceSplits) {
+    float4 v[kReduceSplits][N / 4];
+#pragma unroll
+    for (uint32_t p = 0; p < kReduceSplits; ++p) {  // (past the last: the last again)
+      const float4* q = reinterpret_cast<const float4*>(from + min(p0 + p, s.splits - 1u) * step);
+#pragma unroll
+      for (uint32_t i = 0; i < N / 4; ++i) v[p][i] = q[i];
+    }
+#pragma unroll
+    for (uint32_t p = 0; p < kReduceSplits; ++p) {
+      if (p0 + p >= s.splits) break;
+#pragma unroll
+      for (uint32_t i = 0; i < N / 4; ++i) {
+        out[4 * i] += v[p][i].x;
+        out[4 * i + 1] += v[p][i].y;
+        out[4 * i + 2] += v[p][i].z;
+        out[4 * i + 3] += v[p][i].w;
+      }
+    }
+  }
+}
+
 struct GemmTile {
   const uint8_t* base;
   void* y;
@@ -518,37 +558,71 @@ template <int RG, int MT>
 __host__ constexpr size_t gemm_small_lds() { return (size_t)(16 * RG * MT * 256 + RG * 16 * 25 + MT * 16 * 24) * 4; }
 static_assert(gemm_small_lds<2, 4>() <= 160 * 1024, "partial sums of sixteen wavefronts fit a CU's LDS");
 
-// A lane's sixteen results of one activation row (weight rows row + 8 g + 4 h .. + 3, g < 4) into y + at: where y and its
-// rows lie on 16-byte boundaries, and one by one.
+// A fragment's results on their way to y, ld values from an activation row's to the next: a lane has sixteen of one activation row (weight rows
+// 8 g + 4 h .. + 3, g < 4).  Where y and its rows lie on 16-byte boundaries they go through LDS (`turn`, a wavefront's own), so that a store
+// takes whole lines, eight lanes to a row: as the lanes have them a store is sixteen bytes each of 32 rows, and the partial results of a 4B layer's
+// products of 500 rows took 2 us longer each.  Else one by one.
+// wave_lds_order: what a wavefront has read of LDS has come before it writes there, and the other way round.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+template <int RF>
+__host__ __device__ constexpr uint32_t turn_bytes() { return 32u * (64u * RF + 16u) > 32u * 144u ? 32u * (64u * RF + 16u) : 32u * 144u; }
+// What a store of fragment (k, c) needs: the first activation row of c, rows there are, the wavefront's first weight row in a row of y.
+struct StoreAt {
+  void* y;
+  size_t ld;
+  uint32_t m, m_end, row, d_out;  // (d_out: of rows from `row` on, those below it are stored)
+  uint8_t* turn;
+};
+template <int RF>
 struct StoreF32 {
-  static __device__ __forceinline__ void store(void* y, size_t at, uint32_t row, uint32_t h, uint32_t, const acc16_t& v) {
-    float* out = reinterpret_cast<float*>(y) + at + row + 4u * h;
+  static __device__ __forceinline__ void store(const StoreAt& t, uint32_t k, uint32_t lane, const acc16_t& v) {
+    const uint32_t l32 = lane & 31u, h = lane >> 5, r = lane >> 3, q = lane & 7u;
+    float* const to = reinterpret_cast<float*>(t.turn) + l32 * 36u + h * 4u;
+    wave_lds_order();
 #pragma unroll
-    for (int g = 0; g < 4; ++g) *reinterpret_cast<float4*>(out + g * 8) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+    for (int g = 0; g < 4; ++g) *reinterpret_cast<float4*>(to + g * 8) = make_float4(v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]);
+    wave_lds_order();
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) {
+      const float4 o = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(t.turn) + (i * 8u + r) * 36u + q * 4u);
+      const uint32_t m = t.m + i * 8u + r;
+      if (m < t.m_end) *reinterpret_cast<float4*>(reinterpret_cast<float*>(t.y) + (size_t)m * t.ld + t.row + k * 32u + q * 4u) = o;
+    }
   }
 };
-struct StoreF16 {
-  static __device__ __forceinline__ void store(void* y, size_t at, uint32_t row, uint32_t h, uint32_t, const acc16_t& v) {
-    uint32_t p[8];
+template <int RF>
+struct StoreF16 {  // (all fragments of an activation row with the last of them)
+  static __device__ __forceinline__ void store(const StoreAt& t, uint32_t k, uint32_t lane, const acc16_t& v) {
+    constexpr uint32_t kPitch = 64u * RF + 16u, kPieces = 4u * RF;  // bytes of a row in LDS, and 16-byte pieces of it
+    const uint32_t l32 = lane & 31u, h = lane >> 5;
+    if (k == 0u) wave_lds_order();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) p[i] = __builtin_bit_cast(uint32_t, half2_t{(_Float16)v[2 * i], (_Float16)v[2 * i + 1]});
-    _Float16* out = reinterpret_cast<_Float16*>(y) + at + row;
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<u32x2_t*>(t.turn + l32 * kPitch + k * 64u + (uint32_t)g * 16u + h * 8u) =
+          u32x2_t{__builtin_bit_cast(uint32_t, half2_t{(_Float16)v[4 * g], (_Float16)v[4 * g + 1]}), __builtin_bit_cast(uint32_t, half2_t{(_Float16)v[4 * g + 2], (_Float16)v[4 * g + 3]})};
+    if (k + 1u != (uint32_t)RF) return;
+    wave_lds_order();
 #pragma unroll
-    for (int g = 0; g < 4; g += 2) {  // the upper half's group g for the lower half's group g + 1: eight rows in a row each
-      const auto a = __builtin_amdgcn_permlane32_swap(p[2 * g], p[2 * g + 2], false, false);
-      const auto b = __builtin_amdgcn_permlane32_swap(p[2 * g + 1], p[2 * g + 3], false, false);
-      *reinterpret_cast<u32x4_t*>(out + (g + h) * 8u) = u32x4_t{a[0], b[0], a[1], b[1]};
+    for (uint32_t i = 0; i < 2u * RF; ++i) {
+      const uint32_t p = i * 64u + lane, r = p / kPieces, q = p - r * kPieces, m = t.m + r;
+      const u32x4_t o = *reinterpret_cast<const u32x4_t*>(t.turn + r * kPitch + q * 16u);
+      if (m < t.m_end) *reinterpret_cast<u32x4_t*>(reinterpret_cast<_Float16*>(t.y) + (size_t)m * t.ld + t.row + q * 8u) = o;
     }
   }
 };
 template <typename Y>
 struct StoreEach {
-  static __device__ __forceinline__ void store(void* y, size_t at, uint32_t row, uint32_t h, uint32_t d_out, const acc16_t& v) {
-    Y* out = reinterpret_cast<Y*>(y) + at;
+  static __device__ __forceinline__ void store(const StoreAt& t, uint32_t k, uint32_t lane, const acc16_t& v) {
+    const uint32_t m = t.m + (lane & 31u);
+    Y* out = reinterpret_cast<Y*>(t.y) + (size_t)m * t.ld;
+    if (m >= t.m_end) return;
 #pragma unroll
     for (uint32_t e = 0; e < 16; ++e) {
-      const uint32_t r = row + 8u * (e >> 2) + 4u * h + (e & 3u);
-      if (r < d_out) out[r] = (Y)v[e];
+      const uint32_t r = t.row + k * 32u + 8u * (e >> 2) + 4u * (lane >> 5) + (e & 3u);
+      if (r < t.d_out) out[r] = (Y)v[e];
     }
   }
 };
@@ -570,8 +644,8 @@ struct StoreEach {
 // accumulator registers is most; 13000 x 5121 at 600 rows 115 -> 252 us.  (With arithmetic for the look-ups that loop was as fast over
 // 13 bytes a block, 250 us; small products took 1.5 to 2.5 us less, without lists of escapes to wait for and read: 4096 x 4097 at
 // 130 rows 45.3 us, 47.9 now.)
-// Launches with too few tiles to fill the chip split the columns (`splits`): partial sums go to the workspace and
-// gemm_reduce_kernel adds them in order; otherwise the tile is finished here.
+// Launches with too few tiles to fill the chip split the columns (`splits`): partial results go to the workspace and are added in order by
+// gemm_sum_kernel or by the launch that takes them (GemmSums), with PAIR partial sums by gemm_reduce_pair_kernel; otherwise the tile is finished here.
 // Gate and up of an 8B layer (24576 x 4096) at 512 rows: 116 -> 110 us, 935 TFLOP/s (116 with 17 binary16 operations an octet and
 // 13 bytes a block; 121 with those and ten); a plain f16 product of that size by the vendor's library runs at 1159 on this card.
 template <int RF>
@@ -594,8 +668,8 @@ template <int RF>
 __host__ __device__ constexpr uint32_t gemm_wide_lists() { return 2u * RF * kMaxListSlots * 16u; }
 static_assert(gemm_wide_buf<2, 4>() >= 4u * (gemm_wide_lists<2>() + 64u * 20u) && gemm_wide_buf<3, 4>() >= 4u * (gemm_wide_lists<3>() + 64u * 20u), "the lists fit a buffer");
 template <int RF, int CF>
-__host__ constexpr bool gemm_wide_tail_fits() { return kWideDepth * gemm_wide_buf<RF, CF>() >= (gemm_wide_rows<RF>() + 32u * CF) * kDim * 4u; }
-static_assert(gemm_wide_tail_fits<2, 4>() && gemm_wide_tail_fits<2, 8>() && gemm_wide_tail_fits<3, 4>(), "the tail's operands fit the buffers");
+__host__ constexpr bool gemm_wide_tail_fits() { return kWideDepth * gemm_wide_buf<RF, CF>() >= ((gemm_wide_rows<RF>() + 32u * CF) * kDim + gemm_wide_rows<RF>()) * 4u + 4u * turn_bytes<RF>(); }
+static_assert(gemm_wide_tail_fits<2, 4>() && gemm_wide_tail_fits<2, 8>() && gemm_wide_tail_fits<3, 4>(), "what the end has in LDS fits the buffers");
 
 // 16 bytes per lane from base + offset to LDS, lane after lane from `lds` on.  In assembly because the compiler, which
 // cannot tell the buffers apart, would have every read of LDS wait for all of these; the counting is done by hand
@@ -622,11 +696,6 @@ __device__ __forceinline__ void load_tiles_to_lds(uint32_t lds, const uint32_t (
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\ts_mov_b32 exec_hi, 0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4 offset:1024\n\t"
                  "s_mov_b32 exec_hi, 0xffff\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %5 offset:1536\n\ts_mov_b32 exec_hi, -1"
                  : : "{m0}"(lds), "v"(o[0]), "v"(o[1]), "v"(o[2]), "s"(d), "s"(m) : "memory");
-}
-// What a wavefront has read of LDS has come before it writes there, and the other way round.
-__device__ __forceinline__ void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
 }
 // A barrier by itself: what LDS reads of a wavefront are in flight it has not begun to need, and what they read stays.
 __device__ __forceinline__ void wide_barrier() {
@@ -701,9 +770,22 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
 #pragma unroll
     for (uint32_t part = 0; part < 3u; ++part) to_next_step(part);
   };
+  // What the end needs from the tiles' heads: the row scales, a lane's own, and (so that they are in L2 then) the lines of the tail columns.
+  // (Asked for there they were two to three waits for memory in every workgroup.  With that, operands a fragment ahead and stores of whole lines the
+  // end takes 6.5 us of a tile of 384 rows and sixteen tail columns where it took 11: 12288 + 12288 x 4096 at 512 rows 111.3 -> 108.8 us.)
+  float my_scale[(RF + 1) / 2];
+#pragma unroll
+  for (uint32_t i = 0; i < (uint32_t)(RF + 1) / 2u; ++i) {
+    const uint32_t row = row0 + min(i * 64u + lane, 32u * RF - 1u);
+    my_scale[i] = reinterpret_cast<const float*>(rec0 + record(row))[row & 15u];
+  }
+  const uint32_t touched = *reinterpret_cast<const uint32_t*>(rec0 + record(t.row0 + min(tid / 9u, kRows / 16u - 1u) * 16u) + min(tid % 9u, (head >> 7) - 1u) * 128u);
   acc16_t acc[RF][CF];
   double sum[PAIR ? RF : 1][PAIR ? CF : 1][16];  // of the steps, with PAIR
   const float unit = table_unit(entry_f), table = entry_f * (1.f / unit);
+#pragma unroll
+  for (int i = 0; i < (RF + 1) / 2; ++i) asm volatile("" : "+v"(my_scale[i]));
+  asm volatile("" ::"v"(touched));
   const auto scale_of = [&](uint32_t meta) __attribute__((always_inline)) {
     return __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)meta, (int)__float_as_uint(table)));
   };
@@ -1117,25 +1199,32 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
   // A lane's activation row is l32 of a fragment; element e is weight row 8 (e / 4) + 4 h + e % 4 of it.
   // (From the lane's number anew: nothing of this may occupy registers during the loop.)
   const uint32_t lane_e = lane_offset(lane), l32e = lane_e & 31u, he = lane_e >> 5;
-  const uint32_t m0 = mt * kCols + l32e;
-  if (RF == 2 && a.splits > 1u) {  // (gemm_plan splits no tiles of 384 rows)
-    const uint32_t n_rows = a.n_tiles * kRows;
-    float* out = a.ws + (size_t)split * a.m_pad * n_rows;
+  const bool in_parts = RF == 2 && a.splits > 1u;  // (gemm_plan splits no tiles of 384 rows)
+  const uint32_t n_rows = a.n_tiles * kRows;
+  float* const parts = a.ws + (size_t)split * a.m_pad * n_rows;
+  uint8_t* const turn_at = smem + ((kRows + 32u * CF) * kDim + kRows) * 4u + wave * turn_bytes<RF>();
+  if (PAIR && in_parts) {
+    __syncthreads();
 #pragma unroll
-    for (int c = 0; c < CF; ++c)
-      if (m0 + (uint32_t)c * 32u < a.M) {
+    for (uint32_t c = 0; c < (uint32_t)CF; ++c)
 #pragma unroll
-        for (int k = 0; k < RF; ++k)
-          StoreF32::store(out, (size_t)(m0 + (uint32_t)c * 32u) * n_rows, tile * kRows + wave * (32u * RF) + (uint32_t)k * 32u, he, 0, acc[k][c] * unit);
-      }
+      for (uint32_t k = 0; k < (uint32_t)RF; ++k)
+        StoreF32<RF>::store(StoreAt{parts, n_rows, mt * kCols + c * 32u, a.M, tile * kRows + wave * (32u * RF), 0u, turn_at}, k, lane_e, acc[k][c] * unit);
     return;
   }
-  // The tail's operands to LDS, columns of all rows: a lane would wait for each of its loads in turn.
-  float* w_tail = reinterpret_cast<float*>(smem);
+  // The tail columns this workgroup adds: of a split its share of them, in pairs.
+  const uint32_t tail_w = a.tail_w, tail_parts = in_parts ? a.splits : 1u, tail_part = in_parts ? split : 0u;
+  const uint32_t tail0 = PAIR ? 0u : (tail_w / 2u * tail_part / tail_parts) * 2u, tail1 = PAIR ? tail_w : (tail_w / 2u * (tail_part + 1u) / tail_parts) * 2u;
+  // The tail's operands to LDS: a lane would wait for each of its loads in turn.
+  float* const scales = reinterpret_cast<float*>(smem) + wave * (32u * RF);
+  float* w_tail = reinterpret_cast<float*>(smem) + kRows;
   float* x_tail = w_tail + kRows * kDim;
-  if (a.tail_w) {
-    __syncthreads();
-    for (uint32_t c0 = 0; c0 < a.tail_w; c0 += 8u) {
+  __syncthreads();
+#pragma unroll
+  for (uint32_t i = 0; i < (uint32_t)(RF + 1) / 2u; ++i)
+    if (i * 64u + lane < 32u * RF) scales[i * 64u + lane] = my_scale[i] * unit;
+  if constexpr (PAIR) {
+    for (uint32_t c0 = 0; c0 < tail_w; c0 += 8u) {
       float v[8];
       const uint32_t m = mt * kCols + tid % kCols;
       const __half* tx = a.x + (size_t)min(m, a.M - 1u) * a.ldx + nb * kDim;
@@ -1144,89 +1233,142 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
         const uint32_t row = min(r0 + tid, kRows - 1u);
         const float* rec = reinterpret_cast<const float*>(rec0 + record(t.row0 + row));
 #pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) v[i] = rec[tail_at(row & 15u, min(c0 + i, a.tail_w - 1u), a.tail_w)];
+        for (uint32_t i = 0; i < 8; ++i) v[i] = rec[tail_at(row & 15u, min(c0 + i, tail_w - 1u), tail_w)];
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i)
-          if (r0 + tid < kRows && c0 + i < a.tail_w) w_tail[(c0 + i) * kRows + row] = v[i];
+          if (r0 + tid < kRows && c0 + i < tail_w) w_tail[(c0 + i) * kRows + row] = v[i];
       }
 #pragma unroll
-      for (uint32_t i = 0; i < 8; ++i) v[i] = __half2float(tx[min(c0 + i, a.tail_w - 1u)]);
+      for (uint32_t i = 0; i < 8; ++i) v[i] = __half2float(tx[min(c0 + i, tail_w - 1u)]);
 #pragma unroll
       for (uint32_t i = 0; i < 8; ++i)
-        if (tid < kCols && c0 + i < a.tail_w) x_tail[(c0 + i) * kCols + tid] = v[i];
+        if (tid < kCols && c0 + i < tail_w) x_tail[(c0 + i) * kCols + tid] = v[i];
     }
-    __syncthreads();
-  }
-  auto finish = [&](auto to) __attribute__((always_inline)) {
+  } else if (tail0 != tail1) {
+    // Eight or sixteen columns: the heads as they are, 16 bytes a lane, and the activations by octets.
+    constexpr uint32_t kW = (kRows + 255u) / 256u * 4u, kX = 2u * kCols / 256u;
+    const uint32_t pieces = tail_depth(tail_w) * 16u;  // of a tile
+    u32x4_t w[kW];
+    HalfOctet x[kX];
 #pragma unroll
-    for (int k = 0; k < RF; ++k) {
-      const uint32_t row = row0 + (uint32_t)k * 32u;
-      float scale[16];
+    for (uint32_t i = 0; i < kW; ++i) {
+      const uint32_t k = min(i * 256u + tid, kRows / 16u * pieces - 1u), of = k / pieces;
+      w[i] = *reinterpret_cast<const u32x4_t*>(rec0 + record(t.row0 + of * 16u) + 128u + (k - of * pieces) * 16u);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kX; ++i) {
+      const uint32_t k = i * 256u + tid, m = mt * kCols + k % kCols, c = k / kCols * 8u;
+      x[i] = *reinterpret_cast<const HalfOctet*>(a.x + (size_t)min(m, a.M - 1u) * a.ldx + nb * kDim + (c < tail_w ? c : 0u));
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kW; ++i) reinterpret_cast<u32x4_t*>(w_tail)[min(i * 256u + tid, kRows / 16u * pieces - 1u)] = w[i];
+#pragma unroll
+    for (uint32_t i = 0; i < kX; ++i) {
+      const uint32_t k = i * 256u + tid, c = k / kCols * 8u;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        x_tail[(c + 2u * j) * kCols + k % kCols] = half_lo(x[i].w[j]);
+        x_tail[(c + 2u * j + 1u) * kCols + k % kCols] = half_hi(x[i].w[j]);
+      }
+    }
+  }
+  __syncthreads();
+  // ld, from: values from one of the results' activation rows to the next, and where this wavefront's first weight row is in one.
+  // A fragment's tail columns, two at a time (the halves hold one each), are a chain of f32 products of 64 cycles, beside which the fragment in
+  // front of it is converted and stored; its operands are read a fragment ahead.
+  auto finish = [&](auto to, void* y, size_t ld, uint32_t from) __attribute__((always_inline)) {
+    constexpr uint32_t kPairs = PAIR ? 1u : 8u, kFragments = RF * CF;  // pairs of tail columns
+    const uint32_t pairs = (tail1 - tail0) >> 1;
+    float scale[RF][16], tw[RF][kPairs], tx[kPairs];
+#pragma unroll
+    for (uint32_t k = 0; k < (uint32_t)RF; ++k) {
 #pragma unroll
       for (uint32_t g = 0; g < 4u; ++g) {
-        const float4 v = *reinterpret_cast<const float4*>(rec0 + record(row + g * 8u) + (g & 1u) * 32u + he * 16u);
-        scale[4 * g] = v.x * unit;
-        scale[4 * g + 1] = v.y * unit;
-        scale[4 * g + 2] = v.z * unit;
-        scale[4 * g + 3] = v.w * unit;
+        const float4 v = *reinterpret_cast<const float4*>(scales + k * 32u + g * 8u + he * 4u);
+        scale[k][4 * g] = v.x;
+        scale[k][4 * g + 1] = v.y;
+        scale[k][4 * g + 2] = v.z;
+        scale[k][4 * g + 3] = v.w;
       }
+      if constexpr (!PAIR) {
+        const uint32_t row = wave * (32u * RF) + k * 32u + l32e;
+        const float* at = w_tail + (row >> 4) * 64u * tail_depth(tail_w);
 #pragma unroll
-      for (int c = 0; c < CF; ++c) {
-        // f32 tail columns, two at a time: the halves hold one each.  (One by one on top of the blocks' sum each costs that a
-        // rounding: with PAIR they are summed by themselves and meet it last.)
-        acc16_t v;
+        for (uint32_t i = 0; i < kPairs; ++i) tw[k][i] = at[tail_at(row & 15u, min(tail0 + 2u * i + he, 15u), tail_w) - 32u];  // (past the last: not used)
+      }
+    }
+    auto read_c = [&](uint32_t c) __attribute__((always_inline)) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = PAIR ? 0.f : acc[k][c][e] * scale[e];
-        for (uint32_t i = 0; i < a.tail_w; i += 2u) {
-          // (Without PAIR they are an even number.  With it a column past the last is zero in both operands: zero times the last
-          // one again is not zero where that is infinite.)
-          const uint32_t col = PAIR ? min(i + he, a.tail_w - 1u) : i + he;
-          const bool there = !PAIR || i + he < a.tail_w;
-          const float tw = w_tail[col * kRows + wave * (32u * RF) + (uint32_t)k * 32u + l32e], tx = x_tail[col * kCols + (uint32_t)c * 32u + l32e];
-          v = __builtin_amdgcn_mfma_f32_32x32x2f32(there ? tw : 0.f, there ? tx : 0.f, v, 0, 0, 0);
+      for (uint32_t i = 0; i < kPairs; ++i) tx[i] = x_tail[min(tail0 + 2u * i + he, 15u) * kCols + c * 32u + l32e];
+    };
+    auto put = [&](uint32_t i, const acc16_t& v) __attribute__((always_inline)) {
+      decltype(to)::store(StoreAt{y, ld, mt * kCols + i / RF * 32u, a.M, from, t.d_out, turn_at}, i % RF, lane_e, v);
+    };
+    acc16_t before;
+    if constexpr (!PAIR) read_c(0);
+#pragma unroll
+    for (uint32_t i = 0; i < kFragments; ++i) {
+      const uint32_t k = i % RF, c = i / RF;
+      acc16_t v;
+      if constexpr (PAIR) {
+        // (One by one on top of the blocks' sum each column costs that a rounding: they are summed by themselves and meet it last.  A column past
+        // the last is zero in both operands: zero times the last one again is not zero where that is infinite.)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = 0.f;
+        for (uint32_t j = 0; j < tail_w; j += 2u) {
+          const uint32_t col = min(j + he, tail_w - 1u);
+          const float w = w_tail[col * kRows + wave * (32u * RF) + k * 32u + l32e], x1 = x_tail[col * kCols + c * 32u + l32e];
+          v = __builtin_amdgcn_mfma_f32_32x32x2f32(j + he < tail_w ? w : 0.f, j + he < tail_w ? x1 : 0.f, v, 0, 0, 0);
         }
-        if constexpr (PAIR) {
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            float y = fmaf(acc[k][c][e], scale[e], v[e]);
-            asm("" : "+v"(y));  // (an f32 value in every store: where they convert one by one it would be one operation, rounded once)
-            v[e] = y;
-          }
+        for (int e = 0; e < 16; ++e) {
+          float r = fmaf(acc[k][c][e], scale[k][e], v[e]);
+          asm("" : "+v"(r));  // (an f32 value in every store: where they convert one by one it would be one operation, rounded once)
+          v[e] = r;
         }
-        const uint32_t m = m0 + (uint32_t)c * 32u;
-        if (m < a.M) decltype(to)::store(t.y, (size_t)m * t.d_out, row, he, t.d_out, v);
+        put(i, v);
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = acc[k][c][e] * scale[k][e];
+#pragma unroll
+        for (uint32_t j = 0; j < kPairs; ++j)
+          if (j < pairs) v = __builtin_amdgcn_mfma_f32_32x32x2f32(tw[k][j], tx[j], v, 0, 0, 0);
+        if (k + 1u == (uint32_t)RF && c + 1u < (uint32_t)CF) read_c(c + 1u);
+        if (i) put(i - 1u, before);
+        before = v;
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if constexpr (!PAIR) put(kFragments - 1u, before);
   };
   const bool whole = row0 + 32u * RF <= t.d_out && ((reinterpret_cast<uintptr_t>(t.y) | t.d_out * (a.y_f32 ? 4u : 2u)) & 15u) == 0;
-  if (a.y_f32) {
-    if (whole) finish(StoreF32{});
-    else finish(StoreEach<float>{});
+  if (!PAIR && in_parts) {
+    finish(StoreF32<RF>{}, parts, n_rows, tile * kRows + wave * (32u * RF));
+  } else if (a.y_f32) {
+    if (whole) finish(StoreF32<RF>{}, t.y, t.d_out, row0);
+    else finish(StoreEach<float>{}, t.y, t.d_out, row0);
   } else {
-    if (whole) finish(StoreF16{});
-    else finish(StoreEach<_Float16>{});
+    if (whole) finish(StoreF16<RF>{}, t.y, t.d_out, row0);
+    else finish(StoreEach<_Float16>{}, t.y, t.d_out, row0);
   }
 }
 template <int CF, bool PAIR>
 __global__ __launch_bounds__(256, CF == 8 || PAIR ? 1 : 2) void gemm_wide_kernel(GemmArgs a) { wide_product<2, CF, PAIR>(a); }
 __global__ __launch_bounds__(256, 1) void gemm_tall_kernel(GemmArgs a) { wide_product<3, 4, false>(a); }
 
-// The partial sums of the column splits, added in order; row scale and tail columns.  A lane takes one weight row and
+// PAIR: the partial sums of the column splits, added in order; row scale and tail columns.  A lane takes one weight row and
 // kReduceM activation rows, so that the row's tail is read once for them.
 // What bounds it is how many round trips to memory a lane makes: the sums and the tail columns are read four splits and
 // eight columns at a time, the activations' tail comes to LDS with the first of them.  (One by one 11.3 us for 500
 // rows of 2560 with 8 or 16 tail columns and 14.9 for 6144; so 9.0 and 10.3; and a microsecond less with a workgroup's lanes a tile's rows,
 // which needs no division, and loads of the splits there are alone.)
 constexpr uint32_t kReduceM = 8;
-constexpr uint32_t kReduceSplits = 4;
-// With PAIR the splits are added in f64 and the tail by itself.  Grid (tiles of 256 weight rows, the only ones that are split; kReduceM
+// The splits are added in f64 and the tail by itself.  Grid (tiles of 256 weight rows, the only ones that are split; kReduceM
 // activation rows).
 constexpr uint32_t kReduceRows = 256;
 static_assert(kReduceRows == gemm_wide_rows<2>(), "a workgroup's lanes are a tile's rows");
-template <bool PAIR>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a) {
-  typedef typename std::conditional<PAIR, double, float>::type sum_t;
+__global__ __launch_bounds__(256) void gemm_reduce_pair_kernel(GemmArgs a) {
   __shared__ float x_tail[kReduceM][32];
   static_assert(kReduceM * 32u == 256u && kDim <= 32, "a value of the activations' tail per lane");
   touch_args(a);
@@ -1249,7 +1391,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a) {
     for (uint32_t c = 0; c < 4u; ++c) tw[c] = *reinterpret_cast<const F4*>(reinterpret_cast<const float*>(rec) + tail_at(r, 4u * i0 + c, tail_w));
   };
   if (tail_w) read_tail(0);
-  sum_t s[kReduceM];
+  double s[kReduceM];
 #pragma unroll
   for (uint32_t k = 0; k < kReduceM; ++k) s[k] = 0;
   for (uint32_t p0 = 0; p0 < a.splits; p0 += kReduceSplits) {
@@ -1264,12 +1406,12 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a) {
     for (uint32_t p = 0; p < kReduceSplits; ++p) {
       if (p0 + p >= a.splits) break;
 #pragma unroll
-      for (uint32_t k = 0; k < kReduceM; ++k) s[k] += (sum_t)v[p][k];
+      for (uint32_t k = 0; k < kReduceM; ++k) s[k] += (double)v[p][k];
     }
   }
   float out[kReduceM];
 #pragma unroll
-  for (uint32_t k = 0; k < kReduceM; ++k) out[k] = PAIR ? 0.f : (float)s[k] * scale;
+  for (uint32_t k = 0; k < kReduceM; ++k) out[k] = 0.f;
   if (tail_w) {
     lds_barrier();
     const uint32_t depth = tail_depth(tail_w);
@@ -1288,7 +1430,53 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a) {
   if (my_row < t.d_out) {
 #pragma unroll
     for (uint32_t k = 0; k < kReduceM; ++k)
-      if (m0 + k < a.M) store_y(t.y, (size_t)(m0 + k) * t.d_out + row, PAIR ? fmaf((float)s[k], scale, out[k]) : out[k], a.y_f32);
+      if (m0 + k < a.M) store_y(t.y, (size_t)(m0 + k) * t.d_out + row, fmaf((float)s[k], scale, out[k]), a.y_f32);
+  }
+}
+
+// The partial results of the column splits (each has its row scale, the last the tail columns), added in order, where no launch behind the
+// product takes them as they are (GemmSums).  A lane takes four weight rows of kSumM activation rows, kReduceSplits splits at a time.  (The launch that
+// also had scales and tails to see to took 8.8 us for 500 rows of 2560; 6000 x 1000 at 130 rows 28.1 -> 25.4 us, 4096 x 4096 at 300 33.8 -> 32.1.)
+constexpr uint32_t kSumM = 2;
+__device__ __forceinline__ void add_four(float (&s)[4], const float4& v) {
+  s[0] += v.x;
+  s[1] += v.y;
+  s[2] += v.z;
+  s[3] += v.w;
+}
+__global__ __launch_bounds__(256) void gemm_sum_kernel(GemmArgs a) {
+  touch_args(a);
+  const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const GemmTile t = gemm_tile_at(a, blockIdx.x, kReduceRows);
+  const uint32_t n_rows = a.n_tiles * kReduceRows, m0 = (blockIdx.y * 4u + wave) * kSumM, row = t.row0 + lane * 4u;
+  if (m0 >= a.M) return;
+  float s[kSumM][4] = {};
+  for (uint32_t p0 = 0; p0 < a.splits; p0 += kReduceSplits) {
+    float4 v[kReduceSplits][kSumM];
+#pragma unroll
+    for (uint32_t p = 0; p < kReduceSplits; ++p) {
+      if (p0 + p >= a.splits) break;
+#pragma unroll
+      for (uint32_t k = 0; k < kSumM; ++k)
+        v[p][k] = reinterpret_cast<const float4*>(uniform_global(a.ws + ((size_t)(p0 + p) * a.m_pad + min(m0 + k, a.M - 1u)) * n_rows + blockIdx.x * kReduceRows))[lane];
+    }
+#pragma unroll
+    for (uint32_t p = 0; p < kReduceSplits; ++p) {
+      if (p0 + p >= a.splits) break;
+#pragma unroll
+      for (uint32_t k = 0; k < kSumM; ++k) add_four(s[k], v[p][k]);
+    }
+  }
+  const bool whole = row + 4u <= t.d_out && ((reinterpret_cast<uintptr_t>(t.y) | (size_t)t.d_out * (a.y_f32 ? 4u : 2u)) & (a.y_f32 ? 15u : 7u)) == 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kSumM; ++k) {
+    if (m0 + k >= a.M) break;
+    const size_t at = (size_t)(m0 + k) * t.d_out + row;
+    if (whole && a.y_f32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(t.y) + at) = make_float4(s[k][0], s[k][1], s[k][2], s[k][3]);
+    else if (whole) *reinterpret_cast<uint2*>(reinterpret_cast<__half*>(t.y) + at) = make_uint2(pack_halves(s[k][0], s[k][1]), pack_halves(s[k][2], s[k][3]));
+    else
+      for (uint32_t i = 0; i < 4u; ++i)
+        if (row + i < t.d_out) store_y(t.y, at + i, s[k][i], a.y_f32);
   }
 }
 

@@ -1700,9 +1700,11 @@ static bool stored_over_rows(const void* x, size_t x_bytes, const llvq_mat* cons
 // One launch over n <= kGemmMaxGroup matrices of equal d_in that take the same activations
 // (already in the matrices' basis), M <= kGemmMaxM rows.  from: rows that are rotated on the way to the octets, their tail
 // columns to x.
-// make: launches what makes the rows, as octets (and their tail columns in x).
+// make: launches what makes the rows, as octets (and their tail columns in x).  left: takes the results where they are partial ones, to be
+// added up by a launch that is enqueued before the next product's (no results in y then).
 static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, uint32_t M, void* const* y,
-                       int y_dtype, bool pair, GemmWorkspace* wsp = nullptr, const void* from = nullptr, const std::function<void(const Octets&)>* make = nullptr) {
+                       int y_dtype, bool pair, GemmWorkspace* wsp = nullptr, const void* from = nullptr, const std::function<void(const Octets&)>* make = nullptr,
+                       GemmSums* left = nullptr) {
   const llvq_mat* m0 = mats[0];
   const __half* xh = reinterpret_cast<const __half*>(x);
   const GemmPlan p = gemm_plan(rt, mats, n, M, pair);
@@ -1769,10 +1771,13 @@ static int launch_gemm(llvq_rt* rt, const llvq_mat* const* mats, int n, const vo
   };
   if (pair) product(std::true_type{});
   else product(std::false_type{});
-  if (p.splits > 1u) {
-    const dim3 grid(a.n_tiles, (M + kReduceM - 1u) / kReduceM);
-    if (pair) hipLaunchKernelGGL(gemm_reduce_kernel<true>, grid, dim3(kReduceRows), 0, rt->stream, a);
-    else hipLaunchKernelGGL(gemm_reduce_kernel<false>, grid, dim3(kReduceRows), 0, rt->stream, a);
+  if (p.splits > 1u && pair) {
+    hipLaunchKernelGGL(gemm_reduce_pair_kernel, dim3(a.n_tiles, (M + kReduceM - 1u) / kReduceM), dim3(kReduceRows), 0, rt->stream, a);
+  } else if (p.splits > 1u && left) {
+    *left = GemmSums{a.ws, p.splits, p.m_pad, a.n_tiles * p.rows_per_tile, {}};
+    for (int i = 0; i < n; ++i) left->first[i] = a.mat[i].tile_begin * p.rows_per_tile;
+  } else if (p.splits > 1u) {
+    hipLaunchKernelGGL(gemm_sum_kernel, dim3(a.n_tiles, (M + 4u * kSumM - 1u) / (4u * kSumM)), dim3(256), 0, rt->stream, a);
   }
   HIP_TRY(hipGetLastError());
   return LLVQ_OK;
@@ -1812,7 +1817,7 @@ static bool gemm_takes_octets(const llvq_mat* const* mats, int n, uint32_t M) {
 //     binary16, a row by itself in f32; such widths end at 124), matrices without a whole block, and cap-13 matrices,
 //     whose rows keep the bits of the single-row product.
 static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, int M, void* const* y, int y_dtype,
-                           GemmWorkspace* wsp = nullptr) {
+                           GemmWorkspace* wsp = nullptr, GemmSums* left = nullptr) {
   const llvq_mat* m0 = mats[0];
   const size_t esz = y_dtype == LLVQ_F32 ? 4 : 2;
   const uint8_t* xb = reinterpret_cast<const uint8_t*>(x);
@@ -1852,7 +1857,7 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
                                    (size_t)M * m0->d_in * sizeof(__half), &rows);
     if (rc0) return rc0;
     if (n <= kGemmMaxGroup && M <= chunk && m0->rot->m >= kRotOctetM)
-      return launch_gemm(rt, mats, n, rows, (uint32_t)M, y, y_dtype, pair, wsp, x);
+      return launch_gemm(rt, mats, n, rows, (uint32_t)M, y, y_dtype, pair, wsp, x, nullptr, left);
     const int rc = launch_rotate(rt, m0->rot, x, (uint32_t)M, rows, true);
     if (rc) return rc;
     xb = reinterpret_cast<const uint8_t*>(rows);
@@ -1863,7 +1868,8 @@ static int gemm_same_basis(llvq_rt* rt, const llvq_mat* const* mats, int n, cons
       const int cnt = n - i0 < kGemmMaxGroup ? n - i0 : kGemmMaxGroup;
       void* ys[kGemmMaxGroup];
       for (int i = 0; i < cnt; ++i) ys[i] = reinterpret_cast<uint8_t*>(y[i0 + i]) + (size_t)m_lo * mats[i0 + i]->d_out * esz;
-      const int rc = launch_gemm(rt, mats + i0, cnt, xb + (size_t)m_lo * m0->d_in * 2, mc, ys, y_dtype, pair, wsp);
+      const int rc = launch_gemm(rt, mats + i0, cnt, xb + (size_t)m_lo * m0->d_in * 2, mc, ys, y_dtype, pair, wsp, nullptr, nullptr,
+                                 cnt == n && (int)mc == M ? left : nullptr);
       if (rc) return rc;
     }
   }
@@ -2189,7 +2195,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     if (pro.kind == kPrologueAddRmsNorm) {
       hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, x, reinterpret_cast<const __half*>(pro.x2),
                          reinterpret_cast<const __half*>(pro.norm_w), reinterpret_cast<__half*>(pro.resid_out), d->normed,
-                         d->hidden, pro.eps, Octets{});
+                         d->hidden, pro.eps, Octets{}, GemmSums{});
       staged = d->normed;
     } else {
       hipLaunchKernelGGL(silu_mul_kernel, dim3((d->inter / 8 + 256) / 256), dim3(256), 0, st, reinterpret_cast<const __half*>(pro.x2),
@@ -2305,7 +2311,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   }
   phase_mark(d);
   if (want_logits) {
-    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, h, d->down, d->fnorm, h, d->normed, d->hidden, d->eps, Octets{});
+    hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, h, d->down, d->fnorm, h, d->normed, d->hidden, d->eps, Octets{}, GemmSums{});
     launch_head(d, history_slot, record, host);
   }
   HIP_TRY(hipGetLastError());
@@ -2356,19 +2362,31 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
   const float scale = 1.0f / sqrtf((float)d->head_dim);
   // Rows that `make` launches what makes, through projections that share them: straight to the product's octets where one launch takes them
   // all in their own basis, else to x first.
-  const auto product = [&](const llvq_mat* const* mats, int n_mats, const __half* x, void* const* y, const std::function<void(const Octets&)>& make) {
-    if (gemm_takes_octets(mats, n_mats, n)) return launch_gemm(rt, mats, n_mats, x, n, y, LLVQ_F16, false, nullptr, nullptr, &make);
+  // left: where the launch that takes the results adds up what the product leaves in parts (the workspace that those are in is as large as any
+  // product of a pass needs it, llvq_hip_decoder_create, and is not touched before the next product).
+  const auto product = [&](const llvq_mat* const* mats, int n_mats, const __half* x, void* const* y, const std::function<void(const Octets&)>& make,
+                           GemmSums* left = nullptr) {
+    if (gemm_takes_octets(mats, n_mats, n)) return launch_gemm(rt, mats, n_mats, x, n, y, LLVQ_F16, false, nullptr, nullptr, &make, left);
     make(Octets{});
+    bool one_basis = true;
+    for (int i = 1; i < n_mats; ++i) one_basis &= same_basis(mats[0], mats[i]);
+    if (left && one_basis) return gemm_same_basis(rt, mats, n_mats, x, (int)n, y, LLVQ_F16, nullptr, left);
     return llvq_hip_gemm_group(rt, mats, n_mats, x, (int)n, y, LLVQ_F16);
   };
+  GemmSums down_sums{};  // of the layer before
   for (uint32_t L = 0; L < d->n_layers; ++L) {
     const llvq_mat* const* P = d->proj.data() + (size_t)L * 7;
+    const uint32_t grp = d->n_heads / d->n_kv;
+    // 32 rows per workgroup on the matrix cores where the head width is the one that kernel is built for, the cache walked
+    // by two sets of wavefronts (more than five heads to a set leave it too few registers for that)
+    const bool on_mfma = d->head_dim == 128 && grp <= (uint32_t)kAttnMaxGroup;
+    GemmSums qkv_sums{}, o_sums{};
     // residual + previous MLP branch, then the input norm (the branch of layer 0 is absent)
     void* const qkv[3] = {d->pq, d->pk, d->pv};
     int rc = product(P, 3, d->pnormed, qkv, [&](const Octets& to) {
       hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(to.xt ? to.m_pad : n), dim3(norm_threads(d->hidden)), 0, st, ph, L ? d->pdown : (const __half*)nullptr,
-                         d->ln1 + (size_t)L * d->hidden, L ? ph_alt : (__half*)nullptr, d->pnormed, d->hidden, d->eps, to);
-    });
+                         d->ln1 + (size_t)L * d->hidden, L ? ph_alt : (__half*)nullptr, d->pnormed, d->hidden, d->eps, to, down_sums);
+    }, d->head_dim == 128 ? &qkv_sums : nullptr);
     if (rc) return rc;
     if (L) std::swap(ph, ph_alt);
     KvQ8 lq8 = d->q8;
@@ -2391,10 +2409,6 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     auto attend = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, agrid, dim3(64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->head_dim, d->pos, d->max_pos, scale);
     };
-    const uint32_t grp = d->n_heads / d->n_kv;
-    // 32 rows per workgroup on the matrix cores where the head width is the one that kernel is built for, the cache walked
-    // by two sets of wavefronts (more than five heads to a set leave it too few registers for that)
-    const bool on_mfma = d->head_dim == 128 && grp <= (uint32_t)kAttnMaxGroup;
     const dim3 mgrid(d->n_kv, (n + kAttnTile - 1) / kAttnTile);
     auto attend_mfma = [&](auto kernel, uint32_t waves) {
       hipLaunchKernelGGL(kernel, mgrid, dim3(waves * 64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->pos, n, d->max_pos, scale, ctx_to);
@@ -2402,7 +2416,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     const auto attention = [&]() {
     if (d->kv_q8) {
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<true>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
-                         d->head_dim, d->pos, d->max_pos);
+                         d->head_dim, d->pos, d->max_pos, qkv_sums);
       if (on_mfma) {
         if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<true, 2, 2>, 2 * 2);
         else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<true, 4, 2>, 2 * 4);
@@ -2414,7 +2428,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       else attend(attn_rows_kernel<true, kAttnMaxGroup>);
     } else {
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<false>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
-                         d->head_dim, d->pos, d->max_pos);
+                         d->head_dim, d->pos, d->max_pos, qkv_sums);
       if (on_mfma) {
         if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<false, 2, 2>, 2 * 2);
         else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<false, 4, 2>, 2 * 4);
@@ -2431,7 +2445,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       rc = product(P + 3, 1, d->pctx, o_out, [&](const Octets& to) {
         ctx_to = to;
         attention();
-      });
+      }, &o_sums);
     } else {
       attention();
       rc = llvq_hip_gemm(rt, P[3], d->pctx, (int)n, d->po, LLVQ_F16);
@@ -2440,11 +2454,12 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     void* const gate_up[2] = {d->pgate, d->pup};
     rc = product(P + 4, 2, d->pnormed, gate_up, [&](const Octets& to) {
       hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(to.xt ? to.m_pad : n), dim3(norm_threads(d->hidden)), 0, st, ph, d->po, d->ln2 + (size_t)L * d->hidden,
-                         ph_alt, d->pnormed, d->hidden, d->eps, to);
+                         ph_alt, d->pnormed, d->hidden, d->eps, to, o_sums);
     });
     if (rc) return rc;
     std::swap(ph, ph_alt);
     void* const down[1] = {d->pdown};
+    down_sums = GemmSums{};
     rc = product(P + 6, 1, d->pact, down, [&](const Octets& to) {
       if (to.xt) {
         const uint32_t waves = (std::max(to.n_oct, d->inter / 8u) + 7u) / 8u * (to.m_pad / 8u);
@@ -2454,13 +2469,14 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       }
       const uint32_t na = n * d->inter;
       hipLaunchKernelGGL(silu_mul_kernel, dim3(std::min((na / 8u + 256u) / 256u, 4096u)), dim3(256), 0, st, d->pgate, d->pup, d->pact, na);
-    });
+    }, &down_sums);
     if (rc) return rc;
   }
   if (want_logits) {
     const size_t last = (size_t)(n - 1) * d->hidden;
+    if (down_sums.ws) down_sums.ws += (size_t)(n - 1) * down_sums.ld;
     hipLaunchKernelGGL(add_rmsnorm_kernel, dim3(1), dim3(norm_threads(d->hidden)), 0, st, ph + last, d->pdown + last, d->fnorm, d->h, d->normed,
-                       d->hidden, d->eps, Octets{});
+                       d->hidden, d->eps, Octets{}, down_sums);
     launch_head(d, history_slot, record, host);
   }
   HIP_TRY(hipGetLastError());

@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
 BAR_SMALL = 5e-4    # 1.2e-4: hidden 256, heads of 64
 BAR_RAGGED = 2e-3   # 5.3e-4: hidden 200, heads of 32, every projection with tail columns; few logits, so a binary16 step weighs more
 BAR_Q8 = 9e-4       # 1.3e-4 position by position, 2.3e-4 after a batched prompt: int8 KV cache
+BAR_PARTS = 2.5e-4  # 6.3e-5, before products left parts and after: rows of 1032 and 1024, a prompt of 66 to 200
 
 
 def _bar(cfg):
@@ -826,5 +827,36 @@ def test_silu_formed_by_down_projections_launch(gpu_rt, orc, hidden, inter, rota
             worst = max(worst, float(np.abs(got - want).max() / np.abs(want).max()))
         print(f"OBSERVED silu_by_down {hidden}/{inter}/{rotated}: {worst:.3e}")
         assert worst < BAR_SMALL  # (1.3e-4 observed)
+    finally:
+        dec.close()
+
+
+# Rows long enough that a prompt's products are split over their columns: 43 and 42 blocks and 16 tail columns, 64 blocks and 8
+PARTS = decoder.Qwen3Config(num_hidden_layers=2, hidden_size=1032, num_attention_heads=8, num_key_value_heads=2, head_dim=128, intermediate_size=1544,
+                            vocab_size=600, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=210, tie_word_embeddings=True)
+
+
+@pytest.mark.parametrize("hidden,inter,kv_mode,rotate", [(1032, 1544, "f16", False), (1032, 1544, "q8", False), (1024, 1536, "f16", True)])
+@pytest.mark.parametrize("n", [66, 129, 200])
+def test_prompt_results_left_in_parts(gpu_rt, orc, hidden, inter, kv_mode, rotate, n):
+    """What products of a prompt leave in parts is added up by the launches behind them (norms; heads' norms and rotations, cache rows): one
+    pass, and two, of which the last's rows have the head behind them."""
+    import dataclasses
+
+    cfg = dataclasses.replace(PARTS, hidden_size=hidden, intermediate_size=inter, kv_mode=kv_mode)
+    dec, ref = _build(gpu_rt, orc, cfg, 31, rotate=rotate, prefill_rows=130)
+    try:
+        tokens = np.random.default_rng(n).integers(0, cfg.vocab_size, size=n)
+        for t in tokens[:-1]:
+            ref.forward_token(int(t))
+        want = ref.forward_token(int(tokens[-1]))
+        got, _ = dec.prefill(tokens)
+        worst = float(np.abs(got - want).max() / np.abs(want).max())
+        for t in (3, 77):  # over the rows that the pass left in the cache
+            want = ref.forward_token(t)
+            got, _ = dec.forward_token(t)
+            worst = max(worst, float(np.abs(got - want).max() / np.abs(want).max()))
+        print(f"OBSERVED parts {hidden}/{kv_mode}/{rotate}/{n}: {worst:.3e}")
+        assert worst < BAR_PARTS, f"max |dlogit| / max|logit| = {worst:.3e}"
     finally:
         dec.close()

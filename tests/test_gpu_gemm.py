@@ -453,3 +453,29 @@ def test_results_stored_over_the_rows(gpu_rt, width, rows):
     finally:
         for p in projs:
             gpu_rt.free(p)
+
+
+@pytest.mark.parametrize("d_outs,d_in,M", [
+    ((260,), 2400, 70),          # no tail columns; the last tile a row group short
+    ((1023, 5), 2408, 129),      # eight of them; rows of y off 16-byte boundaries
+    ((514, 256, 30), 4096, 300),  # sixteen; three matrices, whose tiles are not full
+    ((768,), 808, 513),          # 33 blocks: two splits of unequal steps
+    ((4,), 5008, 65),
+])
+def test_columns_split_over_workgroups(gpu_rt, orc, d_outs, d_in, M):
+    """Few tiles of long rows: the columns are split, every split leaves rows times their scales with its share of the tail columns, and
+    those are added up."""
+    import torch
+
+    X = synth.make_activation(d_in, seed=M, rows=M)
+    raws = [synth.make_matrix(f"model.layers.0.split{i}.{d}x{d_in}.weight", d, d_in, seed=d + i) for i, d in enumerate(d_outs)]
+    projs = [gpu_rt.upload(r) for r in raws]
+    try:
+        for dtype in (torch.float32, torch.float16):
+            ys = [torch.empty((M, d), dtype=dtype, device="cuda") for d in d_outs]
+            gpu_rt.forward_batched_group_into(projs, _x16(X), ys)
+            for raw, y in zip(raws, ys):
+                _check(y.cpu().numpy(), *_reference(orc, raw, X), out_rounding=0.0 if dtype == torch.float32 else 2**-11)
+    finally:
+        for p in projs:
+            gpu_rt.free(p)
