@@ -465,8 +465,10 @@ __global__ __launch_bounds__(64) void attn_rows_kernel(const __half* __restrict_
 //   O^T += V^T P^T   8 x the same MFMA; B = the probabilities just computed, rounded to
 //                    binary16 in the lanes that hold them (no cross-lane movement: the K
 //                    index of the product is permuted to match, V^T is stored in that order).
-// H = 2: a second set of wavefronts walks every other tile, and the two sets' sums are joined at the end: the walk is a
-// chain (16 tiles for the last rows of a 500-row prompt), and a prompt's workgroups leave CUs idle.  31 -> 22 us for 500 rows of 32 heads.
+// H sets of wavefronts walk every H-th tile each, and their sums are joined at the end: the walk is a chain (16 tiles for the last rows of a
+// 500-row prompt).  A workgroup takes G heads of a kv head's (blockIdx.x: the ceil(heads / G) of each kv head), all of them or, where that leaves
+// CUs idle, two.  500 rows of 32 heads: 31 us with one set, 22 with two, 17.5 with four and two heads to a workgroup (500 tokens of
+// twelve 4B layers 2665 -> 2605 us).
 // Scores, maxima, sums and O stay in f32; the context is rounded once.  The next tile's K and
 // V rows are requested before the current tile is multiplied.  Positions past the pass's last
 // row are read as that row.  Inside a tile a masked position has probability zero and is multiplied
@@ -489,15 +491,15 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
     _Float16 v[kDimH * kAttnVPitch];
   };
   __shared__ Tile tiles[H];
-  static_assert(H == 1 || (H == 2 && sizeof(tiles) >= G * 64 * 16 * sizeof(float)), "the parts meet in the tiles' memory");
-  const uint32_t kvh = blockIdx.x, row0 = blockIdx.y * kAttnTile;
+  static_assert(sizeof(tiles) >= (H - 1) * G * 64 * 16 * sizeof(float), "the parts meet in the tiles' memory");
+  const uint32_t groups = n_heads / n_kv, of_kv = (groups + G - 1u) / G;
+  const uint32_t kvh = blockIdx.x / of_kv, head0 = (blockIdx.x - kvh * of_kv) * G, row0 = blockIdx.y * kAttnTile;
   const uint32_t part = H == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kThreads));
   const uint32_t tid = threadIdx.x - part * kThreads, lane = tid & 63u, wave = tid >> 6;
   _Float16 *kt = tiles[part].k, *vt = tiles[part].v;
-  const uint32_t groups = n_heads / n_kv;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
-  const bool has_head = wave < groups;
-  const uint32_t head = kvh * groups + min(wave, groups - 1u);
+  const bool has_head = head0 + wave < groups;
+  const uint32_t head = kvh * groups + min(head0 + wave, groups - 1u);
   const uint32_t my_row = min(row0 + l32, n_rows - 1u);      // rows past the pass repeat its last row and store nothing
   const uint32_t qpos = pos0 + my_row;
   const uint32_t last_pos = pos0 + n_rows - 1u;              // last cached position
@@ -581,7 +583,7 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
     deposit();
     __syncthreads();
     if (tile + H < n_tiles + part) request(tile + H);
-    if (H == 2 && tile >= n_tiles) continue;  // past every row of this block: nothing of it may reach their sums, not even times zero
+    if (H > 1 && tile >= n_tiles) continue;  // past every row of this block: nothing of it may reach their sums, not even times zero
     // S^T = K Q^T
     f16v sacc;
 #pragma unroll
@@ -628,32 +630,45 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
       }
     }
   }
-  if constexpr (H == 2) {  // the second part's sums join the first's, a quarter of the dims at a time
-    float* meet = reinterpret_cast<float*>(tiles) + wave * 1024u + lane;
+  if constexpr (H > 1) {  // the other parts' sums join the first's in order, a quarter of the dims at a time
+    float* const meet = reinterpret_cast<float*>(tiles) + wave * 1024u + lane;
+    float* const mine = meet + (part ? part - 1u : 0u) * (G * 1024u);
     __syncthreads();
     if (part) {
-      meet[0] = m_run;
-      meet[64] = l_run;
+      mine[0] = m_run;
+      mine[64] = l_run;
     }
     __syncthreads();
-    float w0 = 1.f, w1 = 0.f;
-    if (!part) {
-      const float m1 = meet[0], l1 = meet[64], m = fmaxf(m_run, m1);  // the first part has seen position 0
-      w0 = __expf(m_run - m);
-      w1 = __expf(m1 - m);
-      l_run = fmaf(l_run, w0, l1 * w1);
+    float w[H];
+    if (!part) {  // (a part that met no tile of these rows: maximum -inf, weight 0; the first has seen position 0)
+      float m = m_run;
+#pragma unroll
+      for (uint32_t k = 1; k < (uint32_t)H; ++k) m = fmaxf(m, meet[(k - 1u) * (G * 1024u)]);
+      w[0] = __expf(m_run - m);
+      float l = l_run * w[0];
+#pragma unroll
+      for (uint32_t k = 1; k < (uint32_t)H; ++k) {
+        w[k] = __expf(meet[(k - 1u) * (G * 1024u)] - m);
+        l = fmaf(meet[(k - 1u) * (G * 1024u) + 64u], w[k], l);
+      }
+      l_run = l;
     }
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
       __syncthreads();
       if (part) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) meet[j * 64] = o[dt][j];
+        for (int j = 0; j < 16; ++j) mine[j * 64] = o[dt][j];
       }
       __syncthreads();
       if (!part) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) o[dt][j] = fmaf(o[dt][j], w0, meet[j * 64] * w1);
+        for (int j = 0; j < 16; ++j) {
+          float v = o[dt][j] * w[0];
+#pragma unroll
+          for (uint32_t k = 1; k < (uint32_t)H; ++k) v = fmaf(meet[(k - 1u) * (G * 1024u) + (uint32_t)j * 64u], w[k], v);
+          o[dt][j] = v;
+        }
       }
     }
     if (part) return;
@@ -683,7 +698,7 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
       }
   }
   // columns past the blocks are zero (rows past the pass: nobody has a result of theirs)
-  if (to.xt && kvh == 0u && part == 0u && wave == 0u) {
+  if (to.xt && blockIdx.x == 0u && part == 0u && wave == 0u) {
     if (row_e < n_rows)
       for (uint32_t o = to.kcols / 8u + (lane_e >> 5); o < to.n_oct; o += 2u) to.xt[(size_t)o * to.m_pad + row_e] = make_uint4(0, 0, 0, 0);
   }

@@ -2409,19 +2409,21 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     auto attend = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, agrid, dim3(64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->head_dim, d->pos, d->max_pos, scale);
     };
-    const dim3 mgrid(d->n_kv, (n + kAttnTile - 1) / kAttnTile);
-    auto attend_mfma = [&](auto kernel, uint32_t waves) {
-      hipLaunchKernelGGL(kernel, mgrid, dim3(waves * 64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->pos, n, d->max_pos, scale, ctx_to);
+    const uint32_t row_blocks = (n + kAttnTile - 1) / kAttnTile;
+    // two heads to a workgroup where one for each kv head and 32 rows would leave half of the CUs without any
+    const bool by_two = grp > 2u && 2u * d->n_kv * row_blocks <= (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
+    auto attend_mfma = [&](auto kernel, uint32_t heads, uint32_t sets) {
+      hipLaunchKernelGGL(kernel, dim3(d->n_kv * ((grp + heads - 1u) / heads), row_blocks), dim3(heads * sets * 64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->pos, n, d->max_pos, scale, ctx_to);
     };
     const auto attention = [&]() {
     if (d->kv_q8) {
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<true>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos, qkv_sums);
       if (on_mfma) {
-        if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<true, 2, 2>, 2 * 2);
-        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<true, 4, 2>, 2 * 4);
-        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<true, 5, 2>, 2 * 5);
-        else attend_mfma(attn_rows_mfma_kernel<true, kAttnMaxGroup, 1>, kAttnMaxGroup);
+        if (grp <= 2 || by_two) attend_mfma(attn_rows_mfma_kernel<true, 2, 4>, 2, 4);
+        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<true, 4, 2>, 4, 2);
+        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<true, 5, 2>, 5, 2);
+        else attend_mfma(attn_rows_mfma_kernel<true, kAttnMaxGroup, 1>, kAttnMaxGroup, 1);
       } else if (grp <= 2) attend(attn_rows_kernel<true, 2>);
       else if (grp <= 4) attend(attn_rows_kernel<true, 4>);
       else if (grp <= 5) attend(attn_rows_kernel<true, 5>);
@@ -2430,10 +2432,10 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<false>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos, qkv_sums);
       if (on_mfma) {
-        if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<false, 2, 2>, 2 * 2);
-        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<false, 4, 2>, 2 * 4);
-        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<false, 5, 2>, 2 * 5);
-        else attend_mfma(attn_rows_mfma_kernel<false, kAttnMaxGroup, 1>, kAttnMaxGroup);
+        if (grp <= 2 || by_two) attend_mfma(attn_rows_mfma_kernel<false, 2, 4>, 2, 4);
+        else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<false, 4, 2>, 4, 2);
+        else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<false, 5, 2>, 5, 2);
+        else attend_mfma(attn_rows_mfma_kernel<false, kAttnMaxGroup, 1>, kAttnMaxGroup, 1);
       } else if (grp <= 2) attend(attn_rows_kernel<false, 2>);
       else if (grp <= 4) attend(attn_rows_kernel<false, 4>);
       else if (grp <= 5) attend(attn_rows_kernel<false, 5>);
