@@ -2,7 +2,7 @@
 //
 // A product of a few microseconds is shorter than its call from Python: checks, torch.empty, ctypes and the launch take 6.6 us for one
 // projection and 11.5 for a group of three (three results to allocate), where the kernels take 3.8 and 4.9.  Here the same checks, the
-// results' allocation and the library's entry point are one call: 3.9 and 5.4, most of it the launch.  What is not such a tensor gets None back, and takes fused.py's own
+// results' allocation and the library's entry point are one call: 3.5 and 4.4, most of it the launch.  What is not such a tensor gets None back, and takes fused.py's own
 // lines: they convert, or refuse, as ever; so does a call that the library refuses.
 //
 // Tensors that only look like one on the device (subclasses, those of a transformation or a tracer), and calls under a mode that wants to
@@ -10,14 +10,19 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/EmptyTensor.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/Tensor.h>
-#include <ATen/ops/empty.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/llvq_hip.h"
+
+namespace at::cuda {
+c10::Allocator* getCUDADeviceAllocator();  // (ATen/cuda/CUDAContextLight.h, whose other declarations want the device's libraries' headers)
+}
 
 namespace {
 
@@ -91,10 +96,12 @@ Py_ssize_t projs_of(PyObject* obj, Proj (&p)[kMost]) {
     if (!proj_of(PySequence_Fast_GET_ITEM(obj, i), &p[i])) return 0;
   return n;
 }
+// On the current device, which is x's (c10::DeviceGuard).  (What at::empty does behind its dispatch and the guards of its own, which are most of an
+// allocation's time: a group of three results 5.4 -> 4.4 us of host time a call, 5.48 -> 4.58 a pass.)
 at::Tensor result_like(const at::Tensor& x, int64_t d_out, at::ScalarType type) {
   c10::SmallVector<int64_t, 4> dims(x.sizes().begin(), x.sizes().end());
   dims.back() = d_out;
-  return at::empty(dims, x.options().dtype(type));
+  return at::Tensor(at::detail::empty_generic(dims, at::cuda::getCUDADeviceAllocator(), c10::DispatchKeySet(c10::DispatchKey::CUDA), type, std::nullopt));
 }
 
 // A C++ exception of the allocation is fused.py's to raise: its own lines meet it again.
@@ -118,6 +125,7 @@ PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::ScalarType type;
     if (!plain_call() || !runtime_of(args[0], &rt) || !proj_of(args[1], &p) || !plain_tensor(args[2], at::kHalf, &x) || !out_type(args[3], &type)) return nullptr;
     if (x->dim() < 1 || x->numel() != p.d_in || x->size(-1) != p.d_in) return nullptr;
+    const c10::DeviceGuard on(x->device());
     at::Tensor y = result_like(*x, p.d_out, type);
     const void* in = x->const_data_ptr();
     void* out = y.mutable_data_ptr();
@@ -139,6 +147,7 @@ PyObject* forward_group(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!plain_call() || !runtime_of(args[0], &rt) || !plain_tensor(args[2], at::kHalf, &x) || !out_type(args[3], &type)) return nullptr;
     const Py_ssize_t n = projs_of(args[1], p);
     if (n < 1 || x->dim() < 1 || x->numel() != p[0].d_in || x->size(-1) != p[0].d_in) return nullptr;
+    const c10::DeviceGuard on(x->device());
     at::Tensor y[kMost];
     const llvq_mat* mats[kMost];
     void* outs[kMost];
@@ -172,6 +181,7 @@ PyObject* forward_batched(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::ScalarType type;
     if (!plain_call() || !runtime_of(args[0], &rt) || !proj_of(args[1], &p) || !plain_tensor(args[2], at::kHalf, &x) || !out_type(args[3], &type)) return nullptr;
     if (x->dim() != 2 || x->size(1) != p.d_in || x->size(0) < 1 || x->size(0) > INT_MAX) return nullptr;
+    const c10::DeviceGuard on(x->device());
     at::Tensor y = result_like(*x, p.d_out, type);
     const void* in = x->const_data_ptr();
     void* out = y.mutable_data_ptr();
