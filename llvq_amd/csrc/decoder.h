@@ -105,14 +105,10 @@ struct KvQ8 {
   __half* vb;
 };
 
-// One group of 64 values held one per lane -> code, scale, bias.
+// One group of 64 values held one per lane -> code, scale, bias.  (The extremes by lane moves: by __shfl_xor, an LDS instruction each, the twelve
+// steps of a group were a microsecond of the decode attention's launch.)
 __device__ __forceinline__ uint8_t kv_quantize_group(float x, __half* s_out, __half* b_out) {
-  float mn = x, mx = x;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    mn = fminf(mn, __shfl_xor(mn, o, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-  }
+  const float mn = wave_best(x, [](float a, float b) { return fminf(a, b); }), mx = wave_best(x, [](float a, float b) { return fmaxf(a, b); });
   const __half sh = __float2half_rn(__fdiv_rn(__fsub_rn(mx, mn), 255.0f));
   const __half bh = __float2half_rn(mn);
   const float s = __half2float(sh), b = __half2float(bh);
@@ -123,8 +119,9 @@ __device__ __forceinline__ uint8_t kv_quantize_group(float x, __half* s_out, __h
   return (uint8_t)q;
 }
 
+// (q s is exact in f32, 8 bits by 11: the fused operation rounds where the sum alone did.)
 __device__ __forceinline__ float kv_dequant(uint32_t q, float s, float b) {
-  return __half2float(__float2half_rn(__fadd_rn(__fmul_rn((float)q, s), b)));
+  return __half2float(__float2half_rn(fmaf((float)q, s, b)));
 }
 
 // One wavefront: per-head RMSNorm of a q or k head (model.rs:800-808), then RoPE at
@@ -704,8 +701,360 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
   }
 }
 
-// Attention of one query position over the cache (model.rs:812-822), split over
-// the cache: workgroup (kv head, split) takes a contiguous range of positions
+// Attention of one query position over the cache (model.rs:812-822), heads of 128: workgroup (range, kv head) takes the positions
+// [range * chunk, + chunk) for all query heads that share the kv head, sixteen positions (a tile) to a wavefront at a time.
+//
+// What bounds it: round trips to memory (operands and the first rows; partials, the counter and the partials again), so that the rest has to be
+// short.  On the vector ALUs a tile was 500 instructions at four query heads (each lane eight columns of a row for every head, sixteen-lane
+// sums of the scores); here scores are four matrix instructions (16 positions x 16 columns, of which the query heads take the
+// first) and the weighted sum of V eight, beside about 100 others (250 with an int8 cache).  The first product leaves a head's scores in the lanes that
+// the second takes its weights from: column lane % 16 is the head, 4 (lane / 16) + i the position.  V lies in a lane by rows, four of them, which
+// a byte permute turns into pairs of positions.  Weights keep their 24 bits: 2^14 times a weight is two binary16 terms, which are the two halves of one
+// instruction's contraction.  Maxima, sums and scores are f32; K, V and the rotated queries are binary16 values already.  Error
+// against 64 bits before the context is rounded, in the mean over 3 to 8100 positions, both caches: 1.11e-7; on the vector ALUs 1.14e-7.
+// Per launch, before -> now: 513 positions of a 4B layer 8.4 -> 6.8 us, 8100 of a 14B layer with an int8 cache 19.9 (4.7 of them a merge
+// launch) -> 11.0.
+//
+// The workgroup that arrives last at the kv head's counter merges the ranges' partials in their order and rounds the context once;
+// partials go to memory and back at device scope (past the XCDs' own L2s), not between fences, which write back and empty an L2.
+constexpr uint32_t kDecodeTile = 16;    // positions of a wavefront at a time
+constexpr uint32_t kDecodeWaves = 8;
+constexpr uint32_t kDecodeMaxGroup = kAttnMaxGroup;
+constexpr uint32_t kDecodeFetch = 32;   // ranges whose partials are asked for together
+// log2(e) / sqrt(128), to 9e-9 of itself: scores are exponents of two, with one rounding of a score's difference to the maximum where the scaled
+// score, the difference and __expf's product with log2(e) are three.
+constexpr float kDecodeScale = 0.127517432f;
+// Ranges of T positions: a tile to a wavefront, until the kv heads' workgroups fill a card of 256 CUs.  (513 positions of a 4B layer: 6.8 us with 128 a
+// range, 7.5 with 64, 7.8 with 256; 8100 of a 14B layer with an int8 cache: 11.0 us in 32 ranges, 12.4 in 16.)
+__host__ __device__ inline uint32_t decode_ranges(uint32_t T, uint32_t n_kv) {
+  const uint32_t n = (T + kDecodeTile * kDecodeWaves - 1u) / (kDecodeTile * kDecodeWaves), fill = (256u + n_kv - 1u) / n_kv;
+  return min(n, min(fill, (uint32_t)kAttnMaxSplits));
+}
+constexpr uint32_t kDecodeCounter = 64;   // counters are lines of their own: 256 workgroups' additions to one line, behind each other, took 1.5 us
+
+template <bool Q8>
+__global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(AttnNew nw, const __half* __restrict__ kcache, const __half* __restrict__ vcache,
+                                                                             KvQ8 q8, __half* __restrict__ ctx, float* part, uint32_t* __restrict__ counters,
+                                                                             uint32_t groups, uint32_t chunk, uint32_t T, uint32_t max_pos, uint32_t n_splits) {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  constexpr uint32_t D = 128, kThreads = kDecodeWaves * 64, kvgroups = D / kKvGroup;
+  constexpr uint32_t kQuarter = 32 + 4, kAccPitch = 4 * kQuarter + 4;  // a head's sums in LDS: four quarters of 32 columns, on banks of their own
+  __shared__ __align__(16) __half qh[kDecodeMaxGroup][D + 8];  // the query heads, normed and rotated
+  __shared__ __align__(16) __half knew[D], vnew[D];            // the new position's k and v, or their codes
+  __shared__ uint32_t knew_s, knew_b, vnew_s, vnew_b;          // scales and biases of those, a group to a half
+  __shared__ __align__(16) float wmax[kDecodeMaxGroup][kDecodeWaves], wsum[kDecodeMaxGroup][kDecodeWaves];
+  __shared__ __align__(16) float wacc[kDecodeWaves][kDecodeMaxGroup][kAccPitch];
+  __shared__ uint32_t arrived;
+  const uint32_t kvh = blockIdx.y, split = blockIdx.x, tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t j0 = min(T, split * chunk), j1 = min(T, j0 + chunk), nj = j1 - j0;
+  const uint32_t pos = T - 1u;  // the position being decoded
+  const bool has_new = nj > 0 && j1 == T;
+  const uint32_t n16 = lane & 15u, quarter = lane >> 4;
+  const size_t rows = (size_t)kvh * max_pos;
+
+  // A tile's rows: K of position lane % 16, columns 8 (quarter + 4 m) + 0 .. 7 of matrix instruction m (int8: 16 (quarter + 4 m) + 0 .. 15 of
+  // 2 m and 2 m + 1); V of positions 4 quarter + u, columns 8 (lane % 16) + 0 .. 7.  Unconditional: past the end the position being
+  // decoded is read, whose row this launch writes, and not used.
+  uint4 kraw[Q8 ? 2 : 4], vraw[4];
+  uint32_t ks = 0, kb = 0;
+  __half vs[4], vb[4];
+  auto request = [&](uint32_t tile) {
+    const uint32_t kp = min(j0 + tile * kDecodeTile + n16, pos);
+    if constexpr (Q8) {
+      const uint8_t* k = q8.kq + (rows + kp) * D + quarter * 16u;
+#pragma unroll
+      for (int m = 0; m < 2; ++m) kraw[m] = *reinterpret_cast<const uint4*>(k + m * 64);
+      ks = *reinterpret_cast<const uint32_t*>(q8.ks + (rows + kp) * kvgroups);
+      kb = *reinterpret_cast<const uint32_t*>(q8.kb + (rows + kp) * kvgroups);
+    } else {
+      const __half* k = kcache + (rows + kp) * D + quarter * 8u;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) kraw[m] = *reinterpret_cast<const uint4*>(k + m * 32);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t vp = min(j0 + tile * kDecodeTile + quarter * 4u + (uint32_t)u, pos);
+      if constexpr (Q8) {
+        const uint2 v = *reinterpret_cast<const uint2*>(q8.vq + (rows + vp) * D + n16 * 8u);
+        vraw[u] = make_uint4(v.x, v.y, 0, 0);
+        vs[u] = q8.vs[(rows + vp) * kvgroups + (n16 >> 3)];
+        vb[u] = q8.vb[(rows + vp) * kvgroups + (n16 >> 3)];
+      } else {
+        vraw[u] = *reinterpret_cast<const uint4*>(vcache + (rows + vp) * D + n16 * 8u);
+      }
+    }
+  };
+  // operands of the wavefront's query head and of the new k and v, in front of the rows (a wavefront without a head: the last one's)
+  const RopeAngle angle{nw.cos_t[pos * 64u + lane], nw.sin_t[pos * 64u + lane]};
+  const HeadOperands qop = head_operands_128(nw.q_raw + (size_t)(kvh * groups + min(wave, groups - 1u)) * D, nw.qn, lane, lane + 64u);
+  const HeadOperands kop = head_operands_128(nw.k_raw + (size_t)kvh * D, nw.kn, lane, lane + 64u);
+  const __half v1 = nw.v_raw[(size_t)kvh * D + lane], v2 = nw.v_raw[(size_t)kvh * D + lane + 64u];
+  request(wave);
+  static_assert(kDecodeMaxGroup <= kDecodeWaves, "a query head to a wavefront");
+  if (wave < groups) {
+    const float2 r = norm_rope_128(qop, angle, nw.eps);
+    qh[wave][lane] = __float2half_rn(r.x);  // (exact)
+    qh[wave][lane + 64u] = __float2half_rn(r.y);
+  }
+  // The range that ends at the new position owns its k and v: they go to the cache for later positions, and to LDS for this one.
+  const auto quantized = [&](float x, uint32_t g, uint8_t* codes, __half* s_row, __half* b_row, __half* fresh, uint32_t* fresh_s, uint32_t* fresh_b) {
+    __half sh, bh;
+    const uint8_t code = kv_quantize_group(x, &sh, &bh);
+    codes[(rows + pos) * D + g * kKvGroup + lane] = code;
+    reinterpret_cast<uint8_t*>(fresh)[g * kKvGroup + lane] = code;
+    if (lane == 0) {
+      s_row[(rows + pos) * kvgroups + g] = sh;
+      b_row[(rows + pos) * kvgroups + g] = bh;
+      reinterpret_cast<__half*>(fresh_s)[g] = sh;
+      reinterpret_cast<__half*>(fresh_b)[g] = bh;
+    }
+  };
+  if (has_new && wave == kDecodeWaves - 1u) {
+    const float2 r = norm_rope_128(kop, angle, nw.eps);
+    if constexpr (Q8) {
+      quantized(r.x, 0, q8.kq, q8.ks, q8.kb, knew, &knew_s, &knew_b);
+      quantized(r.y, 1, q8.kq, q8.ks, q8.kb, knew, &knew_s, &knew_b);
+    } else {
+      nw.kcache[(rows + pos) * D + lane] = knew[lane] = __float2half_rn(r.x);
+      nw.kcache[(rows + pos) * D + lane + 64u] = knew[lane + 64u] = __float2half_rn(r.y);
+    }
+  }
+  if (has_new && wave == kDecodeWaves - 2u) {
+    if constexpr (Q8) {
+      quantized(__half2float(v1), 0, q8.vq, q8.vs, q8.vb, vnew, &vnew_s, &vnew_b);
+      quantized(__half2float(v2), 1, q8.vq, q8.vs, q8.vb, vnew, &vnew_s, &vnew_b);
+    } else {
+      nw.vcache[(rows + pos) * D + lane] = vnew[lane] = v1;
+      nw.vcache[(rows + pos) * D + lane + 64u] = vnew[lane + 64u] = v2;
+    }
+  }
+  __syncthreads();
+
+  h8 qf[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const uint32_t col = Q8 ? (quarter + 4u * (m >> 1)) * 16u + (m & 1) * 8u : (quarter + 4u * m) * 8u;
+    qf[m] = *reinterpret_cast<const h8*>(&qh[min(n16, groups - 1u)][col]);  // (columns past the heads: the last head again, not used)
+  }
+  f4 acc[8];  // [t]: columns 8 (4 quarter + i) + t of head lane % 16
+#pragma unroll
+  for (int t = 0; t < 8; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;  // the head's maximum so far; the lane's positions' sum of exponentials
+  const auto lane_max = [](float v) {    // over the quarters
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  };
+  const auto lane_sum = [](float v) {
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  };
+  const auto half_of = [](uint32_t w, uint32_t i) { return __half2float(__ushort_as_half((unsigned short)(w >> (16u * i)))); };
+#pragma unroll 1
+  for (uint32_t tile = wave; tile * kDecodeTile < nj; tile += kDecodeWaves) {
+    const uint32_t left = nj - tile * kDecodeTile;  // positions from the tile's first on
+    if (left <= kDecodeTile) {                      // the range's last tile
+      if (has_new) {                                // ends in the row that this launch appends
+        if (n16 == left - 1u) {
+#pragma unroll
+          for (int m = 0; m < (Q8 ? 2 : 4); ++m)
+            kraw[m] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(knew) + (quarter + 4u * m) * 16u);
+          if constexpr (Q8) {
+            ks = knew_s;
+            kb = knew_b;
+          }
+        }
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) {
+        const uint32_t at = quarter * 4u + u;
+        if (has_new && at == left - 1u) {
+          if constexpr (Q8) {
+            const uint2 v = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(vnew) + n16 * 8u);
+            vraw[u] = make_uint4(v.x, v.y, 0, 0);
+            vs[u] = __ushort_as_half((unsigned short)(vnew_s >> (16u * (n16 >> 3))));
+            vb[u] = __ushort_as_half((unsigned short)(vnew_b >> (16u * (n16 >> 3))));
+          } else {
+            vraw[u] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(vnew) + n16 * 16u);
+          }
+        }
+        // A row past the range is whatever an earlier use of the cache left.  Its weight is zero, and its values have to be
+        // as well: 0 x infinity would reach the sums.
+        if (at >= left) {
+          vraw[u] = make_uint4(0, 0, 0, 0);
+          vs[u] = vb[u] = __ushort_as_half(0);
+        }
+      }
+    }
+    // scores
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    f4 quad[4];  // (each from zero: one behind the other they round more, and wait for each other)
+    uint32_t va[8][2];  // [t]: column t of positions 0, 1 and of 2, 3
+    if constexpr (Q8) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const float sc = half_of(ks, m), bi = half_of(kb, m);
+        const uint32_t w[4] = {kraw[m].x, kraw[m].y, kraw[m].z, kraw[m].w};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          h8 k;
+#pragma unroll
+          for (int t = 0; t < 8; ++t) k[t] = (_Float16)fmaf((float)((w[2 * h + (t >> 2)] >> (8 * (t & 3))) & 0xFFu), sc, bi);  // kv_dequant
+          quad[2 * m + h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k, qf[2 * m + h], zero, 0, 0, 0);
+        }
+      }
+      float fs[4], fb[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        fs[u] = __half2float(vs[u]);
+        fb[u] = __half2float(vb[u]);
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = fmaf((float)(((t < 4 ? vraw[u].x : vraw[u].y) >> (8 * (t & 3))) & 0xFFu), fs[u], fb[u]);
+        va[t][0] = __builtin_bit_cast(uint32_t, (h2){(_Float16)v[0], (_Float16)v[1]});
+        va[t][1] = __builtin_bit_cast(uint32_t, (h2){(_Float16)v[2], (_Float16)v[3]});
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) quad[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kraw[m]), qf[m], zero, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const auto word = [&](int u) { return t < 2 ? vraw[u].x : t < 4 ? vraw[u].y : t < 6 ? vraw[u].z : vraw[u].w; };
+        const uint32_t pick = t & 1 ? 0x07060302u : 0x05040100u;
+        va[t][0] = __builtin_amdgcn_perm(word(1), word(0), pick);
+        va[t][1] = __builtin_amdgcn_perm(word(3), word(2), pick);
+      }
+    }
+    if ((tile + kDecodeWaves) * kDecodeTile < nj) request(tile + kDecodeWaves);
+    float s[4], mt = -INFINITY;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      s[i] = quarter * 4u + i < left ? (quad[0][i] + quad[1][i]) + (quad[2][i] + quad[3][i]) : -INFINITY;
+      mt = fmaxf(mt, s[i]);
+    }
+    const float mn = fmaxf(m_run, lane_max(mt) * kDecodeScale);
+    if (__builtin_amdgcn_ballot_w64(mn != m_run) != 0u) {  // (most tiles of a long range raise nobody's maximum)
+      const float e0 = __builtin_amdgcn_exp2f(m_run - mn);  // 0 at the first tile (m_run = -inf)
+      m_run = mn;
+      l_run *= e0;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) acc[t] *= e0;
+    }
+    h8 pw;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p = __builtin_amdgcn_exp2f(fmaf(s[i], kDecodeScale, -mn)), w = p * 16384.f;
+      l_run += p;
+      pw[i] = (_Float16)w;
+      pw[4 + i] = (_Float16)(w - (float)pw[i]);
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const uint4 v = make_uint4(va[t][0], va[t][1], va[t][0], va[t][1]);
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, v), pw, acc[t], 0, 0, 0);
+    }
+  }
+  // The wavefronts' results meet in LDS.  (One without a position: maximum -inf, weight 0.)
+  const float l_all = lane_sum(l_run);
+  if (n16 < groups) {
+    if (quarter == 0) {
+      wmax[n16][wave] = m_run;
+      wsum[n16][wave] = l_all;
+    }
+    float* dst = &wacc[wave][n16][quarter * kQuarter];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<float4*>(dst + 8 * i) = make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]);
+      *reinterpret_cast<float4*>(dst + 8 * i + 4) = make_float4(acc[4][i], acc[5][i], acc[6][i], acc[7][i]);
+    }
+  }
+  __syncthreads();
+  // ---- this workgroup's partial: the wavefronts merged in order, two neighbouring columns to a lane ----
+  // part: [head][range][column] weighted sums, behind those of every head's [head][range] {maximum, sum of exponentials}
+  float* const part_ml = part + (size_t)gridDim.y * groups * kAttnMaxSplits * D;
+  auto put = [&](float* at, float a, float b) {  // read by another workgroup of this launch
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(at), (uint64_t)__float_as_uint(a) | (uint64_t)__float_as_uint(b) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (wave < groups) {
+    float w[kDecodeWaves], M = -INFINITY, L = 0.f, A = 0.f, B = 0.f;
+#pragma unroll
+    for (uint32_t k = 0; k < kDecodeWaves; ++k) {
+      w[k] = wmax[wave][k];
+      M = fmaxf(M, w[k]);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kDecodeWaves; ++k) {
+      w[k] = w[k] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(w[k] - M);
+      const float2 a = *reinterpret_cast<const float2*>(&wacc[k][wave][quarter * kQuarter + n16 * 2u]);
+      L = fmaf(wsum[wave][k], w[k], L);
+      A = fmaf(a.x, w[k], A);
+      B = fmaf(a.y, w[k], B);
+    }
+    const uint32_t head = kvh * groups + wave;
+    if (n_splits == 1u) {
+      reinterpret_cast<__half2*>(ctx + (size_t)head * D)[lane] = __floats2half2_rn(A * 0x1p-14f / L, B * 0x1p-14f / L);
+    } else {
+      put(part + ((size_t)head * n_splits + split) * D + lane * 2u, A * 0x1p-14f, B * 0x1p-14f);
+      if (lane == 0) put(part_ml + (head * n_splits + split) * 2u, M, L);  // (-inf for an empty range)
+    }
+  }
+  if (n_splits == 1u) return;
+  // Let the last workgroup of this kv head merge: a lane's partials have arrived in memory before it reaches the barrier,
+  // and only then is the workgroup counted.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) arrived = __hip_atomic_fetch_add(&counters[kvh * kDecodeCounter], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (arrived != n_splits - 1u) return;
+  // A head to a wavefront: its lanes hold the ranges' maxima and sums, and its weights; then two neighbouring columns each.  The first ranges'
+  // partials are requested together with those, every load unconditional (past the last range: the last again, not added).  Sums run in range order.
+  static_assert(kAttnMaxSplits <= 64, "a range to a lane");
+  if (wave < groups) {
+    const uint32_t head = kvh * groups + wave;
+    auto load2 = [&](const float* at) { return __hip_atomic_load(reinterpret_cast<const uint64_t*>(at), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    const uint64_t pair = load2(part_ml + (head * n_splits + min(lane, n_splits - 1u)) * 2u);
+    uint64_t v[kDecodeFetch];
+    auto fetch = [&](uint32_t from) {
+#pragma unroll
+      for (uint32_t u = 0; u < kDecodeFetch; ++u)
+        if (from + (u & ~7u) < n_splits) v[u] = load2(part + ((size_t)head * n_splits + min(from + u, n_splits - 1u)) * D + lane * 2u);
+    };
+    fetch(0);
+    const float mx = lane < n_splits ? __uint_as_float((uint32_t)pair) : -INFINITY;
+    const float M = wave_best(mx, [](float a, float b) { return fmaxf(a, b); });
+    const float w = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mx - M);  // 0 for an empty range too
+    const float L = wave_sum(lane < n_splits ? w * __uint_as_float((uint32_t)(pair >> 32)) : 0.f);
+    float A = 0.f, B = 0.f;
+#pragma unroll 1
+    for (uint32_t from = 0;; from += kDecodeFetch) {
+#pragma unroll
+      for (uint32_t u0 = 0; u0 < kDecodeFetch; u0 += 8u)
+        if (from + u0 < n_splits)
+#pragma unroll
+          for (uint32_t u = u0; u < u0 + 8u; ++u) {
+            const float of = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), (int)(from + u)));
+            const float a = fmaf(__uint_as_float((uint32_t)v[u]), of, A), b = fmaf(__uint_as_float((uint32_t)(v[u] >> 32)), of, B);
+            A = from + u < n_splits ? a : A;  // (0 x infinity, of the last range's repeats, would reach the sums)
+            B = from + u < n_splits ? b : B;
+          }
+      if (from + kDecodeFetch >= n_splits) break;
+      fetch(from + kDecodeFetch);
+    }
+    reinterpret_cast<__half2*>(ctx + (size_t)(kvh * groups + wave) * D + lane * 2u)[0] = __floats2half2_rn(A / L, B / L);
+  }
+  if (tid == 0) counters[kvh * kDecodeCounter] = 0;  // ready for the next launch
+}
+
+// The same for heads of another width than 128, split over the cache: workgroup (kv head, split) takes a contiguous range of positions
 // for all query heads that share the kv head, so every K and V row is fetched
 // (and, for the int8 cache, rebuilt) once per group.  The range is walked once:
 // sixteen position classes (four per wavefront, 16 lanes x 8 dims each) keep a
@@ -784,31 +1133,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
       }
     }
   };
-  // head_dim = 128: the operands of the wavefront's query heads and of the new k and v, in front of the rows
-  constexpr int kHeads = (G + kAttnWaves - 1) / kAttnWaves;  // query heads of a wavefront
-  const bool d128 = head_dim == 128u;
-  // (of another width: what these read is valid, and not used)
-  const uint32_t lane_a = d128 ? lane : 0u, lane_b = d128 ? lane + 64u : 0u, angle_at = d128 ? pos * 64u + lane : 0u;
-  const RopeAngle angle{nw.cos_t[angle_at], nw.sin_t[angle_at]};
-  HeadOperands qop[kHeads];
-#pragma unroll
-  for (int i = 0; i < kHeads; ++i)
-    qop[i] = head_operands_128(nw.q_raw + (size_t)(kvh * groups + min(wave + (uint32_t)i * kAttnWaves, groups - 1u)) * head_dim, nw.qn, lane_a, lane_b);
-  const HeadOperands kop = head_operands_128(nw.k_raw + (size_t)kvh * head_dim, nw.kn, lane_a, lane_b);
-  const uint16_t v1 = reinterpret_cast<const uint16_t*>(nw.v_raw)[(size_t)kvh * head_dim + lane_a], v2 = reinterpret_cast<const uint16_t*>(nw.v_raw)[(size_t)kvh * head_dim + lane_b];
   request(c);
   // the query heads of this kv head: norm, rotate, scale
-  if (d128) {
-#pragma unroll
-    for (int i = 0; i < kHeads; ++i) {
-      const uint32_t g = wave + (uint32_t)i * kAttnWaves;
-      if (g < groups) {
-        const float2 r = norm_rope_128(qop[i], angle, nw.eps);
-        qs[g * 128u + lane] = r.x * scale;
-        qs[g * 128u + 64u + lane] = r.y * scale;
-      }
-    }
-  } else for (uint32_t g = wave; g < groups; g += kAttnWaves) {
+  for (uint32_t g = wave; g < groups; g += kAttnWaves) {
     norm_rope_wave(nw.q_raw + (size_t)(kvh * groups + g) * head_dim, nw.qn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps,
                    stage[wave], lane);
     for (uint32_t i = lane; i < head_dim; i += 64) qs[g * head_dim + i] = stage[wave][i] * scale;
@@ -818,14 +1145,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
   // cache for later positions, and to LDS, in the form the cache gives back,
   // for this one (nothing else reads that cache row during this launch).
   if (has_new && wave == 0) {
-    if (d128) {
-      const float2 r = norm_rope_128(kop, angle, nw.eps);
-      stage[0][lane] = r.x;
-      stage[0][lane + 64] = r.y;
-      wave_lds_sync();
-    } else {
-      norm_rope_wave(nw.k_raw + (size_t)kvh * head_dim, nw.kn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage[0], lane);
-    }
+    norm_rope_wave(nw.k_raw + (size_t)kvh * head_dim, nw.kn, nw.cos_t, nw.sin_t, pos, head_dim, nw.eps, stage[0], lane);
     const size_t row = (size_t)kvh * max_pos + pos;
     if constexpr (Q8) {
       for (uint32_t g = 0; g < kvgroups; ++g) {
@@ -849,7 +1169,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
     const size_t row = (size_t)kvh * max_pos + pos;
     if constexpr (Q8) {
       for (uint32_t g = 0; g < kvgroups; ++g) {
-        const float x = d128 ? __half2float(__ushort_as_half(g ? v2 : v1)) : __half2float(nw.v_raw[(size_t)kvh * head_dim + g * kKvGroup + lane]);
+        const float x = __half2float(nw.v_raw[(size_t)kvh * head_dim + g * kKvGroup + lane]);
         __half sh, bh;
         const uint8_t code = kv_quantize_group(x, &sh, &bh);
         q8.vq[row * head_dim + g * kKvGroup + lane] = code;
@@ -861,7 +1181,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnNew nw, c
       }
     } else {
       for (uint32_t i = lane; i < head_dim; i += 64) {
-        const __half x = __ushort_as_half(d128 ? (i < 64u ? v1 : v2) : __half_as_ushort(nw.v_raw[(size_t)kvh * head_dim + i]));
+        const __half x = nw.v_raw[(size_t)kvh * head_dim + i];
         nw.vcache[row * head_dim + i] = x;
         vnew[i] = __half2float(x);
       }

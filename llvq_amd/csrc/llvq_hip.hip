@@ -117,6 +117,19 @@ __device__ __forceinline__ float wave_sum(float v) {
          __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32)) + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
 }
 
+// The largest or smallest of the wavefront, the same value in every lane.
+template <class Op>
+__device__ __forceinline__ float wave_best(float v, Op&& op) {
+  v = op(v, dpp_move<0xB1>(v));
+  v = op(v, dpp_move<0x4E>(v));
+  v = op(v, dpp_move<0x141>(v));
+  v = op(v, dpp_move<0x140>(v));
+  auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+
 constexpr uint32_t kDenseBits = 49;  // bits per block at shell cap 13: a 48-bit index and the gain bit
 
 // ---- parity probe: unrank records to points -----------------------------------
@@ -1995,7 +2008,7 @@ struct llvq_decoder {
   float* attn_part = nullptr;   // [n_heads][kAttnMaxSplits][head_dim + 2] partial attention sums
   bool kv_q8 = false;           // int8 KV cache (kvq.rs) instead of binary16
   KvQ8 q8{};                    // layer 0's arrays; a layer's are at + layer * (cache_layer or cache_layer / 64 groups)
-  uint32_t* attn_counters = nullptr;  // [n_kv], zero between launches
+  uint32_t* attn_counters = nullptr;  // [n_kv][kDecodeCounter], zero between launches
   uint32_t pos = 0;
   uint32_t head_grid = 0;
   // rows of positions at once (llvq_hip_decoder_prefill): [prefill_rows, width] buffers, one allocation
@@ -2175,7 +2188,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
   phase_mark(d);
   const size_t cache_layer = (size_t)d->n_kv * d->max_pos * d->head_dim;
   const uint32_t T = d->pos + 1;
-  // about 64 cached positions per workgroup (one batch of four per position class), at most kAttnMaxSplits ranges
+  // heads of another width than 128: about 64 cached positions per workgroup (one batch of four per position class), at most kAttnMaxSplits ranges
   uint32_t n_splits = (T + 63) / 64;
   if (n_splits > (uint32_t)kAttnMaxSplits) n_splits = kAttnMaxSplits;
   const uint32_t groups_per_kv = d->n_heads / d->n_kv;
@@ -2224,6 +2237,12 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     nw.kcache = kc;
     nw.vcache = vc;
     nw.eps = d->eps;
+    if (d->head_dim == 128u) {
+      const uint32_t n = decode_ranges(T, d->n_kv);
+      hipLaunchKernelGGL(d->kv_q8 ? attn_decode_mfma_kernel<true> : attn_decode_mfma_kernel<false>, dim3(n, d->n_kv), dim3(kDecodeWaves * 64u), 0, st, nw, kc, vc, lq8, d->ctx,
+                         d->attn_part, d->attn_counters, groups_per_kv, (T + n - 1u) / n, T, d->max_pos, n);
+      return;
+    }
     auto attend = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(n_splits, d->n_kv), dim3(kAttnThreads), attn_lds, st, nw, kc, vc, lq8, d->ctx, d->attn_part,
                          d->attn_counters, groups_per_kv, (T + n_splits - 1) / n_splits, d->head_dim, T, d->max_pos, 1.0f / sqrtf((float)d->head_dim), n_splits,
@@ -2589,7 +2608,7 @@ int llvq_hip_decoder_create(llvq_rt* rt, const llvq_decoder_desc* c, llvq_decode
   const size_t n_best = (size_t)d->head_grid * (kHeadThreads / 64);
   const size_t o_bv = take(n_best * sizeof(float)), o_bi = take(n_best * sizeof(uint32_t));
   const size_t o_hist = take((size_t)c->max_positions * sizeof(uint32_t));
-  const size_t o_ap = take((size_t)c->n_heads * kAttnMaxSplits * (c->head_dim + 2) * sizeof(float)), o_ac = take((size_t)c->n_kv_heads * sizeof(uint32_t));
+  const size_t o_ap = take((size_t)c->n_heads * kAttnMaxSplits * (c->head_dim + 2) * sizeof(float)), o_ac = take((size_t)c->n_kv_heads * kDecodeCounter * sizeof(uint32_t));
   const size_t o_seqst = take(256);
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&d->blob), total);
   if (e != hipSuccess) { delete d; return hip_fail(e, "hipMalloc(decoder)"); }

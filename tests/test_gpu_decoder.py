@@ -177,6 +177,24 @@ def test_generate_with_batched_prefill_matches_token_by_token(gpu_rt, orc):
         dec.close()
 
 
+@pytest.mark.parametrize("heads,kv,kv_mode", [(1, 1, "q8"), (3, 1, "f16"), (8, 1, "f16"), (10, 2, "q8")])
+def test_decode_attention_at_every_length(gpu_rt, orc, heads, kv, kv_mode):
+    """Heads of 128, one to eight of them to a kv head (all columns of a matrix instruction but for those are other heads' again): every
+    position of the first tiles, of the second range and of its first tiles, each against the oracle."""
+    import dataclasses
+
+    cfg = dataclasses.replace(_wide(heads, kv, kv_mode), num_hidden_layers=1, vocab_size=200)
+    cfg.max_positions = 163
+    dec, ref = _build(gpu_rt, orc, cfg, 31)
+    try:
+        for n, t in enumerate(np.random.default_rng(32).integers(0, cfg.vocab_size, size=cfg.max_positions)):
+            want, got = ref.forward_token(int(t)), dec.forward_token(int(t))[0]
+            # Both round at the same places, and the attention differs by 1e-6 before its result is rounded: a binary16 step of single logits is 1e-3.
+            assert np.abs(got - want).max() < 1e-3 * np.abs(want).max(), n
+    finally:
+        dec.close()
+
+
 def test_long_cache_takes_the_merge_kernel(gpu_rt, orc):
     """Past 1024 cached positions the attention partials (more than 16 ranges of 64) are merged
     by a kernel of their own; the logits must keep agreeing with the oracle across the switch."""
