@@ -1185,6 +1185,7 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   // (The in-launch rotation and the wide rows are written for a full workgroup, whatever of it has a tile.)
   a.g = gemv_grid(a.nb, gated ? a.m[1].tile_begin : a.n_tiles, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), gated, rotated || gemv_wide(a.nb),
                   a.in.prologue == kPrologueAddRmsNorm);
+  if (gemv_wide(a.nb)) spread_into(a.g, gemv_spread(a.nb, a.n_tiles, a.g.grid));
   const int src = rotated ? kSrcRotated : a.in.prologue == kPrologueSiluMul ? kSrcSiluMul : a.in.prologue == kPrologueAddRmsNorm ? kSrcAddRmsNorm : kSrcF16;
   void* params[] = {&a};
   HIP_TRY(hipLaunchKernel(gated ? reinterpret_cast<const void*>(gated_product_kernel) : gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(a.g.grid),

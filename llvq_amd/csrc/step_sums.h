@@ -18,7 +18,7 @@ constexpr uint32_t kGemvWideSteps = 2;  // steps of a wavefront where a row has 
 constexpr uint32_t kGemvRounds = 8;     // tiles per team between two sums over the team's wavefronts, at the most
 constexpr uint32_t kGemvMaxBlocks = kStepBlocks * kGemvMaxWaves * kGemvWideSteps;
 
-// A tile's steps go to a team of wavefronts, one each (two each past sixteen).  A row is added up in an order that does not
+// A tile's steps go to a team of wavefronts, one each (past sixteen: GemvSpread).  A row is added up in an order that does not
 // depend on that: the lanes of a step (rows_sum), the steps of equal number mod 4 one behind the other, those four sums;
 // so a matrix gives the same bits whatever it shares a launch with.
 LLVQ_HD uint32_t gemv_team(uint32_t nb) {
@@ -92,6 +92,27 @@ inline GemvGrid gemv_grid(uint32_t nb, uint32_t tiles, uint32_t cus, bool gated,
   g.inv_teams = (65536u + g.teams - 1u) / g.teams;
   return g;
 }
+// Rows of more than sixteen steps: a workgroup's steps, its slots' one behind the other, go to its sixteen wavefronts in turn, one at a time.
+// (As a team that takes a tile's steps two at a time: of the 23 steps of a 14B down_proj nine wavefronts then have no second one.)
+struct GemvSpread {
+  uint32_t slots, full;  // tiles of a workgroup, one fewer from workgroup `full` on
+  uint32_t batch;        // tiles whose sums are in LDS together and finished together, a wavefront each
+};
+LLVQ_HD uint32_t spread_batch(uint32_t steps) {  // (of the last one as many places are read as the widest row has steps)
+  const uint32_t most = (sums_room(true) - sums_steps(true)) / steps + 1u;
+  return most < kGemvMaxWaves ? most : kGemvMaxWaves;
+}
+inline GemvSpread gemv_spread(uint32_t nb, uint32_t tiles, uint32_t grid) {
+  const uint32_t more = tiles % grid;
+  return {tiles / grid + (more ? 1u : 0u), more ? more : grid, spread_batch(tile_steps(nb))};
+}
+// The arguments of a launch are four lines of memory and no more: such a launch has its numbers in the places of those that only teams use.
+inline void spread_into(GemvGrid& g, const GemvSpread& s) {
+  g.rounds = s.slots;
+  g.teams = s.full;
+  g.inv_teams = s.batch;
+}
+LLVQ_HD GemvSpread spread_of(const GemvGrid& g) { return {g.rounds, g.teams, g.inv_teams}; }
 // The step that a lane of class c reads as its i-th.
 LLVQ_HD uint32_t sums_read(uint32_t i, uint32_t c) { return 4u * i + c; }
 // In LDS the four blocks of a unit lie together: 3 dwords per digit and block, then each block's sum of its integers

@@ -947,12 +947,18 @@ __device__ __forceinline__ void tile_mat(const GemvArgs& a, uint32_t tile, const
 //
 // What bounds it: at 10 bytes per block and about 35 vector instructions the weights' way from memory; in a launch of
 // a few microseconds the chain launch -> activation -> planes -> product -> store.  So: a team of wavefronts takes a tile of
-// sixteen rows, a wavefront a fixed step of it (two of rows past 512 blocks); a tile's loads are all in flight before the
+// sixteen rows, a wavefront a fixed step of it; a tile's loads are all in flight before the
 // planes are ready, and each piece's registers are loaded again for the team's next tile as soon as they have been used,
 // without a branch, so that every wait is for the oldest load only.  The planes of a unit are read from LDS once for
 // the two rows a lane has.  The sums over a team's wavefronts wait in LDS for one barrier per gemv_batch tiles, behind which
 // every wavefront finishes one.  The host spreads teams over the CUs first, tiles over teams so that the last, partial round
 // meets every CU.
+//
+// WIDE, rows past 512 blocks, more steps than wavefronts: a workgroup's steps go to its wavefronts in turn (GemvSpread), across the ends of
+// tiles.  (As a team with two steps of a tile each, 23 steps were 32, both steps' registers were waited for together and a second tile began
+// when both were done: 5120 x 17408 14.4 -> 12.0 us, 4096 x 17408 10.8 -> 8.6, 18000 x 14000 25.7 -> 20.6, rotated 5120 x 17408 21.6 -> 19.7.
+// Narrower rows gain nothing from it, or 3 to 7 % where rows of nine to thirteen steps leave a team's workgroup wavefronts without one and
+// there are many, and lose up to 7 % elsewhere: 18000 x 4096 8.35 -> 8.95 us, their last wavefronts having steps beside the first tiles' ends.)
 //
 // GATED: the two matrices are a layer's gate and up, and what is stored is f16(f16(silu(gate)) up) of their rows, both rounded to
 // binary16 first (model.rs:831): the bits that the product behind it makes of the two results otherwise, in every one of its workgroups
@@ -961,7 +967,7 @@ __device__ __forceinline__ void tile_mat(const GemvArgs& a, uint32_t tile, const
 template <typename OutT, int SRC, bool WIDE, bool GATED>
 __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
   constexpr int DIG = std::is_same<OutT, __half>::value ? 4 : 6;
-  constexpr uint32_t kSteps = WIDE ? kGemvWideSteps : 1u;
+  static_assert(!(WIDE && GATED), "a pair's tiles are a team's");
   extern __shared__ __align__(16) uint8_t smem[];
   touch_args(a);
   const GemvLds L = gemv_lds<DIG>(smem, gemv_plane_units(a.nb));
@@ -989,21 +995,27 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
     }
     return Record{base + kTileTableBytes + (size_t)(row0 / kTileRows) * stride, base, slots};
   };
-  uint32_t off[kSteps];  // (where a wavefront has no step, or no next tile, its loads repeat one: one cache line, and no branch)
-#pragma unroll
-  for (uint32_t j = 0; j < kSteps; ++j) off[j] = step_offset(w + j * kGemvMaxWaves, units, head, lane);
-  uint32_t tile = team < a.g.teams ? tile_of(team) : 0xFFFFFFFFu;
+  // Teams: step w of every tile of the wavefront's is its own (of n_steps and more: none).  WIDE: step `step` of slot `slot`, the sixteenth
+  // behind it the next time.  Where a wavefront has no step, or no next one, its loads repeat one: one cache line, and no branch.
+  const GemvSpread spread = spread_of(a.g);
+  const uint32_t slots = WIDE ? spread.slots - (blockIdx.x < spread.full ? 0u : 1u) : 0u;
+  uint32_t off = step_offset(w, units, head, lane);
+  uint32_t tile = team < (WIDE ? slots : a.g.teams) ? tile_of(team) : 0xFFFFFFFFu;
   Record cur = record_of(min(tile, n_tiles - 1u), team);
-  StepWords W[kSteps];
-  constexpr uint32_t kFirst = SRC == kSrcRotated ? 1u : kSteps;  // (beside a rotation's operands there are registers for one)
+  StepWords W;
   uint32_t table;
   // The tile that this wavefront finishes of those whose rounds begin with r0: the last wavefronts see to the first tiles, since what a tile
   // has besides its steps (tile_extras, 0.8 us for one wavefront) is then not in front of anybody's products where there are
   // wavefronts without any.
-  const uint32_t fin = a.g.waves - 1u - wave, batch = gemv_batch(a.g.team), my_round = (fin * a.g.inv_teams) >> 16, my_team = fin - my_round * a.g.teams;
+  const uint32_t fin = a.g.waves - 1u - wave, batch = WIDE ? spread.batch : gemv_batch(a.g.team);
+  const uint32_t my_round = WIDE ? fin : (fin * a.g.inv_teams) >> 16, my_team = WIDE ? 0u : fin - my_round * a.g.teams;
   TileExtras extras;
   uint32_t extras_table;
-  auto finished = [&](uint32_t r0) { return my_round < batch ? tile_of(r0 * a.g.teams + fin) : 0xFFFFFFFFu; };
+  // r0: the first of a batch of rounds, or of slots
+  auto finished = [&](uint32_t r0) {
+    if constexpr (WIDE) return my_round < batch && r0 + fin < slots ? tile_of(r0 + fin) : 0xFFFFFFFFu;
+    else return my_round < batch ? tile_of(r0 * a.g.teams + fin) : 0xFFFFFFFFu;
+  };
   auto load_finish = [&](uint32_t r0) {
     const uint32_t t = finished(r0);
     const Record r = record_of(min(t, n_tiles - 1u), fin);  // (a batch of rounds has an even number of slots where that matters: gated_teams)
@@ -1014,16 +1026,14 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
     if constexpr (SRC != kSrcRotated) load_finish(0);  // little, and it has a use while the pieces come
     table = scale_table(cur.base, lane);
     const uint8_t* base = scalar_base(cur.rec);
-    const uint32_t keep = tile < n_tiles ? 0xFFFFFFFFu : 0u;
-#pragma unroll
-    for (uint32_t j = 0; j < kFirst; ++j) load_step(W[j], base, off[j] & keep);
+    load_step(W, base, off & (tile < n_tiles ? 0xFFFFFFFFu : 0u));
   });
-  if constexpr (kFirst != kSteps) load_step(W[1], scalar_base(cur.rec), off[1] & (tile < n_tiles ? 0xFFFFFFFFu : 0u));
   if constexpr (SRC == kSrcRotated) load_finish(0);
   lds_barrier();
 
   // (In a rotated basis there is no scalar register to keep it in: 2560 x 9728 takes 11.5 us like this, 11.8 with the argument.)
-  const uint32_t rounds = SRC == kSrcRotated ? (a.n_tiles + n_teams - 1u) / n_teams : a.g.rounds;
+  const uint32_t rounds = WIDE ? slots : SRC == kSrcRotated ? (a.n_tiles + n_teams - 1u) / n_teams : a.g.rounds;
+  uint32_t slot = 0, step = w;  // (WIDE: every wavefront's first step is one of the first slot)
   for (uint32_t r0 = 0; r0 < rounds; r0 += batch) {
     const uint32_t r1 = min(r0 + batch, rounds), o_tile = finished(r0);
     const float o_scale = extras.scale;
@@ -1035,32 +1045,38 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
     if constexpr (GATED)
       if ((fin & 1u) && lane_class(lane) == 0u) *reinterpret_cast<float2*>(L.part + gated_at(WIDE) + (fin * kTileRows + lane_row(lane)) * 2u) = make_float2(o_scale, o_extra);
     if (r1 != rounds) load_finish(r1);
-    for (uint32_t rd = r0; rd < r1 && tile < n_tiles; ++rd) {
-      const uint32_t next = GATED ? tile_of((rd + 1u) * a.g.teams + team) : tile + n_teams;
-      const bool more = next < n_tiles;
-      const Record nx = record_of(min(next, n_tiles - 1u), (rd + 1u) * a.g.teams + team);
-      const uint32_t lanes_table = table, keep = more ? 0xFFFFFFFFu : 0u;
-      const uint8_t* base = scalar_base(nx.rec);
-      float* const part = L.part + sums_at(rd - r0, team, a.g.team, WIDE) * kTileRows;
-      table = scale_table(nx.base, lane);  // in front of the pieces, so that the next round waits for it alone
-#pragma unroll
-      for (uint32_t j = 0; j < kSteps; ++j) {
-        const uint32_t step = w + j * kGemvMaxWaves;
-        float lo, hi;
-        step_product<DIG>(W[j], L.planes + (min(step, n_steps) * kStepUnits + (lane >> 3)) * XPlanes<DIG>::kDwords, lanes_table, lo, hi,
-                          [&](auto piece) __attribute__((always_inline)) { load_piece<decltype(piece)::value>(W[j], base, off[j] & keep); });
-        const float v = rows_sum(lo, hi);
-        if (lane_class(lane) == 0u) part[step * kTileRows + lane_row(lane)] = v;
+    for (uint32_t rd = r0; WIDE ? slot < r1 : rd < r1 && tile < n_tiles; ++rd) {
+      uint32_t next_slot = slot, next_step = step;
+      if constexpr (WIDE) {
+        next_step += kGemvMaxWaves;
+        if (next_step >= n_steps) {
+          next_step -= n_steps;
+          ++next_slot;
+        }
       }
+      const uint32_t next = WIDE ? (next_slot < slots ? tile_of(next_slot) : 0xFFFFFFFFu) : GATED ? tile_of((rd + 1u) * a.g.teams + team) : tile + n_teams;
+      const Record nx = record_of(min(next, n_tiles - 1u), WIDE ? next_slot : (rd + 1u) * a.g.teams + team);
+      const uint32_t lanes_table = table, keep = next < n_tiles ? 0xFFFFFFFFu : 0u;
+      const uint8_t* base = scalar_base(nx.rec);
+      float* const part = L.part + (WIDE ? (slot - r0) * n_steps : sums_at(rd - r0, team, a.g.team, false)) * kTileRows;
+      table = scale_table(nx.base, lane);  // in front of the pieces, so that the next round waits for it alone
+      if constexpr (WIDE) off = step_offset(next_step, units, head, lane);
+      float lo, hi;
+      step_product<DIG>(W, L.planes + (min(step, n_steps) * kStepUnits + (lane >> 3)) * XPlanes<DIG>::kDwords, lanes_table, lo, hi,
+                        [&](auto piece) __attribute__((always_inline)) { load_piece<decltype(piece)::value>(W, base, off & keep); });
+      const float v = rows_sum(lo, hi);
+      if (lane_class(lane) == 0u) part[step * kTileRows + lane_row(lane)] = v;
       tile = next;
+      slot = next_slot;
+      step = next_step;
     }
     // A wavefront per tile of these rounds: everything but the sums themselves is scalar.
     lds_barrier();
     if constexpr (GATED) {
       if (o_tile < n_tiles && !(fin & 1u)) {
-        auto sum_of = [&](uint32_t slot) {
-          const uint32_t round = (slot * a.g.inv_teams) >> 16;
-          return steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(round, slot - round * a.g.teams, a.g.team, WIDE) * kTileRows, n_steps, lane);
+        auto sum_of = [&](uint32_t of) {
+          const uint32_t round = (of * a.g.inv_teams) >> 16;
+          return steps_sum<kGemvMaxWaves>(L.part + sums_at(round, of - round * a.g.teams, a.g.team, false) * kTileRows, n_steps, lane);
         };
         const float2 up_scale = *reinterpret_cast<const float2*>(L.part + gated_at(WIDE) + ((fin + 1u) * kTileRows + lane_row(lane)) * 2u);
         const float gate = fmaf(sum_of(fin), o_scale, o_extra), up = fmaf(sum_of(fin + 1u), up_scale.x, up_scale.y);
@@ -1072,7 +1088,7 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
       void* o_y;
       uint32_t o_row0, o_d_out, o_stride, o_slots;
       tile_mat(a, o_tile, o_base, o_y, o_row0, o_d_out, o_stride, o_slots);
-      const float v = steps_sum<kGemvMaxWaves * kSteps>(L.part + sums_at(my_round, my_team, a.g.team, WIDE) * kTileRows, n_steps, lane);
+      const float v = steps_sum<kGemvMaxWaves * (WIDE ? kGemvWideSteps : 1u)>(L.part + (WIDE ? fin * n_steps : sums_at(my_round, my_team, a.g.team, false)) * kTileRows, n_steps, lane);
       const uint32_t row = o_row0 + lane_row(lane);
       if (lane_class(lane) == 0u && row < o_d_out) store_out<OutT>(o_y, row, fmaf(v, o_scale, o_extra));
     }

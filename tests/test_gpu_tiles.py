@@ -36,6 +36,36 @@ def test_single_row_products(gpu_rt, orc, nb, tail, d_out):
         assert torch.equal(y.reshape(1, -1), y32)  # the same split, whatever shares the launch
 
 
+# Rows past sixteen steps, whose steps go to the wavefronts across the ends of tiles: the fewest and the most of them, one tile to a workgroup
+# and one more, as many as are finished together (fourteen and eight of them) and one more.
+@pytest.mark.parametrize("nb,tail,tiles", [(513, 1, 257), (513, 0, 256 * 14 + 1), (725, 8, 320), (1024, 0, 256), (1024, 0, 256 * 8 + 3)])
+def test_tiles_of_a_large_launch_are_those_of_a_small_one(gpu_rt, nb, tail, tiles):
+    import torch
+
+    from llvq_amd import artifact
+
+    d_in, d_out = nb * 24 + tail, tiles * 16
+    rng = np.random.default_rng(nb + tiles)
+    codes = rng.integers(0, 2 * (artifact.N12 + 1), size=(d_out, nb), dtype=np.uint64).astype(">u8").view(np.uint8).reshape(d_out, nb, 8)[:, :, 2:]
+    scales = np.exp(-4.0 + 0.3 * rng.standard_normal(d_out))
+    tails = (0.02 * rng.standard_normal((d_out, tail))).astype(np.float32)
+    few = np.unique([t for t in (0, 1, 255, 256, 256 * 8 - 1, 256 * 8, 256 * 13 + 5, tiles - 2, tiles - 1) if t < tiles])
+    rows = (few[:, None] * 16 + np.arange(16)).ravel()
+
+    def matrix(name, r):
+        return artifact.RawMatrix(name, len(r), d_in, 12, (0.8, 1.25), scales[r], tails[r].ravel(), codes[r].reshape(-1))
+
+    x = _x16(synth.make_activation(d_in, seed=nb)[:1])[0]
+    projs = [gpu_rt.upload(matrix("model.layers.0.all.weight", np.arange(d_out))), gpu_rt.upload(matrix("model.layers.0.few.weight", rows))]
+    try:
+        for dtype in (torch.float32, torch.float16):
+            whole, some = (gpu_rt.forward(p, x, out_dtype=dtype).reshape(-1) for p in projs)
+            assert torch.equal(whole[torch.from_numpy(rows).to(whole.device)], some)
+    finally:
+        for p in projs:
+            gpu_rt.free(p)
+
+
 # Rows of activations: 16, 64 and 128 close a variant or a tile; columns: products of four blocks, of two, steps of
 # the last split that are short, a block beyond them, tails and row strides of any parity; few rows split the columns.
 # (Tails of 8 and 16 columns keep the rows on 16-byte boundaries: weights of one term.  Other tails: of two.)
