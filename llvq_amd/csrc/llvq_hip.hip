@@ -611,6 +611,124 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
     for (uint32_t i = tid; i < n; i += 1024) out[i] = (out_t)rot_s[i];
 }
 
+// One row by kRotSplit workgroups, f32.  Both factors of I_k (x) H_m mix a row's values by bits of their own: workgroup p makes the p-th
+// m / 32 values of every group, all of H's five highest bits at once as the sums of its sign p over the row (every value of it, once), then
+// the others, lane by lane, and the k x k block over the groups' values, which it has all of.
+// What bounds it is latency: the launch, a row's way from memory, three barriers; 3.4 to 4.2 us whatever the width.  In the product's launch, where
+// every workgroup does all of it, wide rows are several turns of what sixteen wavefronts can at once, and a k x k block past 9 is 32 x 32 on the
+// matrix cores: a rotated product of 2560 x 9728 takes 11.2 us there, 10.1 so; 5120 x 17408 19.7 and 16.6, 4096 x 20480 16.0 and 14.0, 4096 x 14336 13.0
+// and 12.1, 4096 x 11264 (k = 11) 12.9 and 10.6, 4096 x 8704 (k = 17) 10.6 and 9.9, 4096 x 12288 11.6 and 11.4.  Not 4096 x 10240 (k = 5), 10.4 in both, 4096 x 9216 (k = 9), 9.3
+// and 9.8, and 2560 x 5632 (k = 11), 8.8 in both.
+constexpr uint32_t kRotSplit = 32, kRotSplitTile = 512;  // workgroups; values of a wavefront
+__host__ inline bool rot_split_pays(uint32_t n, uint32_t m, uint32_t k) {  // (m, n: what the kernel is written for)
+  return n >= (k > kRotScalarK ? 8192u : 10241u) && m >= 512u && m <= 4096u && n <= kRotSplit * 1024u;
+}
+__host__ inline size_t rot_split_lds(uint32_t n, uint32_t m) { return (size_t)(n / kRotSplitTile) * (m / kRotSplit) * sizeof(float); }
+__global__ __launch_bounds__(1024) void rotate_split_kernel(RotArgs a) {
+  extern __shared__ __align__(16) float part[];  // [tile][run]
+  __shared__ float mixed[1024];
+  asm volatile("" ::"s"(a.x), "s"(a.out), "s"(a.signbits), "s"(a.fragments), "s"(a.n), "s"(a.m), "s"(a.k), "s"(a.inv));  // (all asked for at once)
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, n = a.n, m = a.m, k = a.k, p = blockIdx.x;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t run = m / kRotSplit, lg = 31u - (uint32_t)__builtin_clz(run), tiles = n / kRotSplitTile;  // run: 16 .. 128
+  const uint8_t* signs = reinterpret_cast<const uint8_t*>(a.signbits);
+  HalfOctet o[4];
+  uint32_t sg[4];
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; ++i) {  // (n <= 64 tiles; a wavefront without one repeats the first)
+    const uint32_t tile = wave + 16u * i, at = (tile < tiles ? tile : 0u) * kRotSplitTile + lane * 8u;
+    o[i] = *reinterpret_cast<const HalfOctet*>(a.x + at);
+    sg[i] = signs[at >> 3];
+  }
+  const uint32_t g = tid >> lg, b = tid & (run - 1u);  // the lane's result: value p * run + b of group g, where g < k
+  const RotTable* table = reinterpret_cast<const RotTable*>(a.fragments);
+  float s[kRotKMax];
+  if (k > 1u) {
+#pragma unroll
+    for (uint32_t lh = 0; lh < 2u; ++lh)
+#pragma unroll
+      for (uint32_t q = 0; q < 4u; ++q) {
+        const float4 f = *reinterpret_cast<const float4*>(table->lane[lh * 32u + (g & 31u)].s + 4u * q);
+        s[8 * q + lh] = f.x;
+        s[8 * q + 2 + lh] = f.y;
+        s[8 * q + 4 + lh] = f.z;
+        s[8 * q + 6 + lh] = f.w;
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; ++i) {
+    const uint32_t tile = wave + 16u * i;
+    if (tile >= tiles) break;
+    const uint32_t at = tile * kRotSplitTile + lane * 8u;
+    const uint32_t bits = sg[i] ^ (__builtin_popcount(((at & (m - 1u)) >> lg) & p) & 1u ? 0xFFu : 0u);
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t w = flip_signs(o[i].w[j], bits, j);
+      v[2 * j] = half_lo(w);
+      v[2 * j + 1] = half_hi(w);
+    }
+    // over the lanes that hold other runs' values of the same places: halves of the wavefront, then rows of sixteen lanes, each
+    // going on with half of the values
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[j]), __float_as_uint(v[j + 4]), false, false);
+      v[j] = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[j]), __float_as_uint(v[j + 2]), false, false);
+      float u = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+      if (run <= 64u) u += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(u), 0x128, 0xF, 0xF, false));  // row_ror 8, 4, 2
+      if (run <= 32u) u += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(u), 0x124, 0xF, 0xF, false));
+      if (run <= 16u) u += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(u), 0x122, 0xF, 0xF, false));
+      v[j] = u;
+    }
+    if ((lane & 15u) * 8u < run)
+      *reinterpret_cast<float2*>(part + tile * run + (lane & 15u) * 8u + (lane >> 5) * 4u + ((lane >> 4) & 1u) * 2u) = make_float2(v[0], v[1]);
+  }
+  __syncthreads();
+  const uint32_t each = m / kRotSplitTile;  // tiles of a group
+  float v = 0.f;
+  if (g < k)
+    for (uint32_t t = 0; t < each; ++t) v += part[(g * each + t) * run + b];
+  // H's other bits: the upper value of a pair has the difference
+  auto level = [&](uint32_t l, float other) __attribute__((always_inline)) { v = b & l ? other - v : other + v; };
+  auto lane_move = [&](auto ctrl, float u) __attribute__((always_inline)) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(u), decltype(ctrl)::value, 0xF, 0xF, false));
+  };
+  level(1u, lane_move(std::integral_constant<int, 0xB1>{}, v));
+  level(2u, lane_move(std::integral_constant<int, 0x4E>{}, v));
+  level(4u, lane_move(std::integral_constant<int, 0x1B>{}, lane_move(std::integral_constant<int, 0x141>{}, v)));  // lane ^ 7, then ^ 3
+  level(8u, lane_move(std::integral_constant<int, 0x128>{}, v));
+  if (run >= 32u) level(16u, __shfl_xor(v, 16));
+  if (run >= 64u) level(32u, __shfl_xor(v, 32));
+  if (run >= 128u) {
+    mixed[tid] = v;
+    __syncthreads();
+    level(64u, mixed[tid ^ 64u]);
+    __syncthreads();
+  }
+  if (k == 1u) {
+    v *= a.inv;
+  } else {
+    mixed[tid] = v;
+    __syncthreads();
+    v = 0.f;
+#pragma unroll
+    for (uint32_t q = 0; q < kRotKMax; q += 8u) {
+      if (q >= k) break;
+      float c[8];
+#pragma unroll
+      for (uint32_t i = 0; i < 8u; ++i) c[i] = mixed[(min(q + i, k - 1u) << lg) + b];  // (past k: meets zeros)
+#pragma unroll
+      for (uint32_t i = 0; i < 8u; ++i) v = fmaf(s[q + i], c[i], v);
+    }
+  }
+  if (g < k) reinterpret_cast<float*>(a.out)[g * m + p * run + b] = v;
+}
+
 }  // namespace llvq
 
 #include "tiles.h"
@@ -639,7 +757,7 @@ struct llvq_rt {
     float inv = 1.f;
     uint32_t* signbits = nullptr;
     void* fragments = nullptr;  // RotTable
-    float* scratch = nullptr;   // one rotated activation, f32, where rows are too wide to be rotated in a product's launch
+    float* scratch = nullptr;   // one rotated activation, f32, where that is not made in the product's launch: a call's launches use it one behind the other on the runtime's stream
   };
   std::vector<DevRotation*> rotations;
   __half* rot_rows = nullptr;     // rotated batch rows, f16 (matrix-core path)
@@ -874,7 +992,7 @@ static int runtime_rotation(llvq_rt* rt, uint32_t n, uint64_t seed, const llvq_r
   if (e == hipSuccess) e = hipMalloc(&r->fragments, sizeof(RotTable));
   if (e == hipSuccess) e = hipMemcpy(r->fragments, host.data(), sizeof(RotTable), hipMemcpyHostToDevice);
   // (f32 results have the larger planes: where those fit, all do)
-  if (e == hipSuccess && !gemv_fits(n, true, true)) e = hipMalloc(reinterpret_cast<void**>(&r->scratch), (size_t)n * sizeof(float));
+  if (e == hipSuccess && (!gemv_fits(n, true, true) || rot_split_pays(t.n, t.m, t.k))) e = hipMalloc(reinterpret_cast<void**>(&r->scratch), (size_t)n * sizeof(float));
   if (e != hipSuccess) {
     (void)hipFree(r->signbits);
     (void)hipFree(r->fragments);
@@ -1155,7 +1273,7 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
                         const llvq_rt::DevRotation* rot = nullptr, bool gated = false) {
   const llvq_mat* m0 = mats[0];
   if (y_dtype != LLVQ_F32 && y_dtype != LLVQ_F16) return fail(LLVQ_ERR_INVALID_ARGUMENT, "gemv: unknown output dtype");
-  const bool f32 = y_dtype == LLVQ_F32, rotated = rot || x_f32;
+  const bool f32 = y_dtype == LLVQ_F32, rotated = rot != nullptr;
   if (!gemv_fits(m0->d_in, f32, rot != nullptr))
     return fail(LLVQ_ERR_UNSUPPORTED, m0->name + ": d_in " + std::to_string(m0->d_in) + " does not fit the LDS activation tile");
   GemvArgs a{};
@@ -1186,9 +1304,9 @@ static int launch_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const v
   a.g = gemv_grid(a.nb, gated ? a.m[1].tile_begin : a.n_tiles, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256), gated, rotated || gemv_wide(a.nb),
                   a.in.prologue == kPrologueAddRmsNorm);
   if (gemv_wide(a.nb)) spread_into(a.g, gemv_spread(a.nb, a.n_tiles, a.g.grid));
-  const int src = rotated ? kSrcRotated : a.in.prologue == kPrologueSiluMul ? kSrcSiluMul : a.in.prologue == kPrologueAddRmsNorm ? kSrcAddRmsNorm : kSrcF16;
+  const int src = x_f32 ? kSrcFinished : rotated ? kSrcRotated : a.in.prologue == kPrologueSiluMul ? kSrcSiluMul : a.in.prologue == kPrologueAddRmsNorm ? kSrcAddRmsNorm : kSrcF16;
   void* params[] = {&a};
-  HIP_TRY(hipLaunchKernel(gated ? reinterpret_cast<const void*>(gated_product_kernel) : gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(a.g.grid),
+  HIP_TRY(hipLaunchKernel(gated ? gated_kernel(rotated) : gemv_kernel(f32, src, gemv_wide(a.nb)), dim3(a.g.grid),
                           dim3(a.g.waves * 64u), params, gemv_tiles_lds_bytes(a.nb, m0->d_in, f32, rot != nullptr, gated), rt->stream));
   return LLVQ_OK;
 }
@@ -1216,6 +1334,15 @@ static int launch_rotate(llvq_rt* rt, const llvq_rt::DevRotation* rot, const voi
   return LLVQ_OK;
 }
 
+// One row, to f32 (with and without a launch of its own a call has the same bits in either form, llvq_hip_rotate).
+static int launch_rotate_row(llvq_rt* rt, const llvq_rt::DevRotation* rot, const void* x_f16, float* out) {
+  if (!rot_split_pays(rot->n, rot->m, rot->k)) return launch_rotate(rt, rot, x_f16, 1, out, false);
+  const RotArgs a = rot_args(rot, x_f16, out);
+  hipLaunchKernelGGL(rotate_split_kernel, dim3(kRotSplit), dim3(1024), rot_split_lds(a.n, a.m), rt->stream, a);
+  HIP_TRY(hipGetLastError());
+  return LLVQ_OK;
+}
+
 static bool same_basis(const llvq_mat* a, const llvq_mat* b) {
   return a->has_rotation == b->has_rotation && (!a->has_rotation || a->rotation_seed == b->rotation_seed);
 }
@@ -1223,8 +1350,9 @@ static bool same_basis(const llvq_mat* a, const llvq_mat* b) {
 // One activation through projections that share it: consecutive matrices in the
 // same basis go out as one launch (at most kMaxGroup).  A launch in a rotated basis
 // rotates the activation itself (`pro`, when given, derives it first); rows too wide
-// for that get it rotated once, into the rotation's scratch, by a kernel of its own
-// (never together with `pro`: the caller stages the activation first then).
+// for that, or wide enough that it pays (rot_split_pays), get it rotated once, into the
+// rotation's scratch, by a kernel of its own (the former never together with `pro`: the
+// caller stages the activation first then).
 static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const void* x, void* const* y, int y_dtype,
                          const Prologue* pro = nullptr) {
   int i = 0;
@@ -1232,7 +1360,7 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
     int j = i + 1;
     while (j < n && j - i < kMaxGroup && same_basis(mats[i], mats[j])) ++j;
     const float* xr = nullptr;
-    if (mats[i]->has_rotation && gemv_fits(mats[i]->d_in, y_dtype == LLVQ_F32, true)) {
+    if (mats[i]->has_rotation && gemv_fits(mats[i]->d_in, y_dtype == LLVQ_F32, true) && (pro || !rot_split_pays(mats[i]->rot->n, mats[i]->rot->m, mats[i]->rot->k))) {
       const int rc = launch_group(rt, mats + i, j - i, x, y + i, y_dtype, pro, nullptr, mats[i]->rot);
       if (rc) return rc;
       i = j;
@@ -1241,7 +1369,7 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
     if (pro && mats[i]->has_rotation) return fail(LLVQ_ERR_UNSUPPORTED, mats[i]->name + ": prologue with a rotation outside the launch");
     if (mats[i]->has_rotation) {
       // the scratch may still hold this very rotation if the previous run used it; rotating again is cheap and always right
-      const int rc = launch_rotate(rt, mats[i]->rot, x, 1, mats[i]->rot->scratch, false);
+      const int rc = launch_rotate_row(rt, mats[i]->rot, x, mats[i]->rot->scratch);
       if (rc) return rc;
       xr = mats[i]->rot->scratch;
     }
@@ -1253,11 +1381,11 @@ static int forward_group(llvq_rt* rt, const llvq_mat* const* mats, int n, const 
 }
 
 // Whether a layer's gate and up are one launch that leaves silu(gate) up: 37.8, 44.9 and 63.8 us a layer and token of a decode of four layers at the widths of
-// 4B, 8B and 14B models, 38.7, 45.9 and 65.0 as two results that down_proj's launch takes.  Not in a rotated basis, which has no such kernel: down_proj's
-// rotation forms it there, a sixteenth in each wavefront.  (One for it would pay as well: 51.0, 56.2 and 78.0 us are 49.6, 54.6 and 77.3 with it.)
+// 4B, 8B and 14B models, 38.7, 45.9 and 65.0 as two results that down_proj's launch takes.  In a rotated basis, where down_proj's activation is then as wide as
+// rotate_split_kernel wants it and binary16: 50.3, 56.6 and 71.9 us, 53.1, 58.6 and 76.7 with both as parts of down_proj's launch.
 // (Rows of up to 8192 columns, a decoder's widest, have as many steps as there are wavefronts at the most, and the sums of pairs fit LDS.)
 static bool gated_fits(const llvq_mat* gate, const llvq_mat* up) {
-  return !gate->has_rotation && !up->has_rotation && gate->nblocks;
+  return same_basis(gate, up) && gate->nblocks && (!gate->has_rotation || gemv_fits(gate->d_in, false, true));
 }
 
 static int launch_gemv(llvq_rt* rt, const llvq_mat* m, const void* x, void* y, int y_dtype) {
@@ -1273,7 +1401,7 @@ int llvq_hip_gemv(llvq_rt* rt, const llvq_mat* m, const void* x, void* y, int y_
 int llvq_hip_rotate(llvq_rt* rt, const llvq_mat* m, const void* x_f16_dev, float* xr_f32_dev) {
   if (!rt || !m || !x_f16_dev || !xr_f32_dev) return fail(LLVQ_ERR_INVALID_ARGUMENT, "rotate: null argument");
   HIP_TRY(hipSetDevice(rt->device));
-  if (m->has_rotation) return launch_rotate(rt, m->rot, x_f16_dev, 1, xr_f32_dev, false);
+  if (m->has_rotation) return launch_rotate_row(rt, m->rot, x_f16_dev, xr_f32_dev);
   hipLaunchKernelGGL(widen_kernel, dim3((m->d_in + 255) / 256), dim3(256), 0, rt->stream,
                      reinterpret_cast<const __half*>(x_f16_dev), xr_f32_dev, m->d_in);
   HIP_TRY(hipGetLastError());
@@ -2314,7 +2442,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     void* d_out[1] = {d->down};
     if (gated_fits(P[4], P[5])) {
       void* act_out[1] = {d->act};
-      rc = launch_group(rt, P + 4, 2, h, act_out, LLVQ_F16, &ln2, nullptr, nullptr, true);
+      rc = launch_group(rt, P + 4, 2, h, act_out, LLVQ_F16, &ln2, nullptr, P[4]->rot, true);
       if (!rc) rc = forward_group(rt, P + 6, 1, d->act, d_out, LLVQ_F16);
     } else {
       void* gu_out[2] = {d->gate, d->up};

@@ -301,7 +301,7 @@ __device__ __forceinline__ void quantize_halves(const uint32_t (&w)[4], uint32_t
 
 // ---- batch-1 product ------------------------------------------------------------------------------
 // What a launch's activation is made from.
-enum : int { kSrcF16 = 0, kSrcRotated = 1, kSrcSiluMul = 2, kSrcAddRmsNorm = 3 };
+enum : int { kSrcF16 = 0, kSrcRotated = 1, kSrcSiluMul = 2, kSrcAddRmsNorm = 3, kSrcFinished = 4 };  // (the last: f32 values, in.x_f32)
 
 struct TileMat {
   const uint8_t* base;  // the matrix (table, then records)
@@ -386,114 +386,110 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
     for (uint32_t i = tid; i < kStepUnits * XPlanes<DIG>::kDwords; i += n_thr) L.planes[plane_at<DIG>(pad) + i] = 0u;
   };
   if constexpr (SRC == kSrcRotated) {
-    // The activation is rotated into LDS and quantised from there (a finished f32 one from where it is).
+    // The activation is rotated into LDS and quantised from there (what it is made of is binary16).
     // A launch in a rotated basis has 1024 lanes.
     float* xf = L.xf;
     zeros();
-    if (in.x_f32) {
+    const RotTable* table = reinterpret_cast<const RotTable*>(in.rot_fragments);
+    const bool norm = in.prologue == kPrologueAddRmsNorm, silu = in.prologue == kPrologueSiluMul;
+    auto norm_scale = [&](float ss) {
+      ss = wave_sum(ss);
+      if (lane == 0) L.red[wave] = ss;
+      lds_barrier();
+      float total = 0.f;
+      for (uint32_t w = 0; w < 16u; ++w) total += L.red[w];
+      return 1.0f / sqrtf(total / (float)d_in + in.eps);
+    };
+    if (in.rot_m >= kRotOctetM) {
+      // Every operand of a wavefront's tile is requested before the first is used.
+      // (Rows past sixteen tiles: a second turn.  Those have no norm in front: a decoder's hidden size ends at 8192.)
+      const uint8_t* signs = reinterpret_cast<const uint8_t*>(in.rot_signbits);
+      HalfOctet a[2] = {}, b[2] = {}, g[2] = {};
+      uint32_t sg[2] = {0, 0};
+      rot_h8_t h[2] = {};
+      auto load_tile = [&](uint32_t tile) {
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i) {
+          const uint32_t from = rot_octet_at(tile, i) < d_in ? rot_octet_at(tile, i) : 0u;
+          if (norm) g[i] = *reinterpret_cast<const HalfOctet*>(in.norm_w + from);
+          if (in.x2) b[i] = *reinterpret_cast<const HalfOctet*>(in.x2 + from);
+          a[i] = *reinterpret_cast<const HalfOctet*>(in.x + from);
+          sg[i] = signs[from >> 3];
+        }
+      };
+      // (A wavefront without a tile asks for none: loads of sixteen wavefronts that nobody uses are a microsecond in front of the weights'.)
+      const bool has_tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave) * kRotTile < d_in;
+      if (has_tile) {
+        load_tile(wave);
+        h[0] = table->lane[lane].h[0];
+        h[1] = table->lane[lane].h[1];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      float inv = 0.f;
+      if (norm) {
+        float ss = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i) {
+          if (rot_octet_at(wave, i) >= d_in) continue;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float lo = half_lo(a[i].w[j]), hi = half_hi(a[i].w[j]);
+            if (in.x2) {
+              lo = round_half(lo + half_lo(b[i].w[j]));
+              hi = round_half(hi + half_hi(b[i].w[j]));
+            }
+            a[i].w[j] = pack_halves(lo, hi);
+            ss = fmaf(lo, lo, fmaf(hi, hi, ss));
+          }
+          if (in.resid_out && store_resid) *reinterpret_cast<HalfOctet*>(in.resid_out + rot_octet_at(wave, i)) = a[i];
+        }
+        inv = norm_scale(ss);
+      }
+#pragma unroll 1
+      for (uint32_t tile = wave; tile * kRotTile < d_in; tile += 16u) {
+        uint32_t x[2][4];
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i) {
+          if (silu) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              a[i].w[j] = pack_halves(silu_mul(half_lo(b[i].w[j]), half_lo(a[i].w[j])), silu_mul(half_hi(b[i].w[j]), half_hi(a[i].w[j])));
+          } else if (norm) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              a[i].w[j] = pack_halves(half_lo(a[i].w[j]) * inv * half_lo(g[i].w[j]), half_hi(a[i].w[j]) * inv * half_hi(g[i].w[j]));
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) x[i][j] = rot_octet_at(tile, i) < d_in ? flip_signs(a[i].w[j], sg[i], j) : 0u;
+        }
+        if ((tile + 16u) * kRotTile < d_in) load_tile(tile + 16u);  // (on their way beside this tile's levels)
+        rotate_tile_to(xf, x[0], x[1], h, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
+      }
       request();
     } else {
-      const RotTable* table = reinterpret_cast<const RotTable*>(in.rot_fragments);
-      const bool norm = in.prologue == kPrologueAddRmsNorm, silu = in.prologue == kPrologueSiluMul;
-      auto norm_scale = [&](float ss) {
-        ss = wave_sum(ss);
-        if (lane == 0) L.red[wave] = ss;
-        lds_barrier();
-        float total = 0.f;
-        for (uint32_t w = 0; w < 16u; ++w) total += L.red[w];
-        return 1.0f / sqrtf(total / (float)d_in + in.eps);
-      };
-      if (in.rot_m >= kRotOctetM) {
-        // Every operand of a wavefront's tile is requested before the first is used.
-        // (Rows past sixteen tiles: a second turn.  Those have no norm in front: a decoder's hidden size ends at 8192.)
-        const uint8_t* signs = reinterpret_cast<const uint8_t*>(in.rot_signbits);
-        HalfOctet a[2] = {}, b[2] = {}, g[2] = {};
-        uint32_t sg[2] = {0, 0};
-        rot_h8_t h[2] = {};
-        auto load_tile = [&](uint32_t tile) {
-#pragma unroll
-          for (uint32_t i = 0; i < 2u; ++i) {
-            const uint32_t from = rot_octet_at(tile, i) < d_in ? rot_octet_at(tile, i) : 0u;
-            if (norm) g[i] = *reinterpret_cast<const HalfOctet*>(in.norm_w + from);
-            if (in.x2) b[i] = *reinterpret_cast<const HalfOctet*>(in.x2 + from);
-            a[i] = *reinterpret_cast<const HalfOctet*>(in.x + from);
-            sg[i] = signs[from >> 3];
-          }
-        };
-        // (A wavefront without a tile asks for none: loads of sixteen wavefronts that nobody uses are a microsecond in front of the weights'.)
-        const bool has_tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave) * kRotTile < d_in;
-        if (has_tile) {
-          load_tile(wave);
-          h[0] = table->lane[lane].h[0];
-          h[1] = table->lane[lane].h[1];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        float inv = 0.f;
-        if (norm) {
-          float ss = 0.f;
-#pragma unroll
-          for (uint32_t i = 0; i < 2u; ++i) {
-            if (rot_octet_at(wave, i) >= d_in) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              float lo = half_lo(a[i].w[j]), hi = half_hi(a[i].w[j]);
-              if (in.x2) {
-                lo = round_half(lo + half_lo(b[i].w[j]));
-                hi = round_half(hi + half_hi(b[i].w[j]));
-              }
-              a[i].w[j] = pack_halves(lo, hi);
-              ss = fmaf(lo, lo, fmaf(hi, hi, ss));
-            }
-            if (in.resid_out && store_resid) *reinterpret_cast<HalfOctet*>(in.resid_out + rot_octet_at(wave, i)) = a[i];
-          }
-          inv = norm_scale(ss);
-        }
-#pragma unroll 1
-        for (uint32_t tile = wave; tile * kRotTile < d_in; tile += 16u) {
-          uint32_t x[2][4];
-#pragma unroll
-          for (uint32_t i = 0; i < 2u; ++i) {
-            if (silu) {
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                a[i].w[j] = pack_halves(silu_mul(half_lo(b[i].w[j]), half_lo(a[i].w[j])), silu_mul(half_hi(b[i].w[j]), half_hi(a[i].w[j])));
-            } else if (norm) {
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                a[i].w[j] = pack_halves(half_lo(a[i].w[j]) * inv * half_lo(g[i].w[j]), half_hi(a[i].w[j]) * inv * half_hi(g[i].w[j]));
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) x[i][j] = rot_octet_at(tile, i) < d_in ? flip_signs(a[i].w[j], sg[i], j) : 0u;
-          }
-          if ((tile + 16u) * kRotTile < d_in) load_tile(tile + 16u);  // (on their way beside this tile's levels)
-          rotate_tile_to(xf, x[0], x[1], h, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
+      auto put = [&](uint32_t i, float v) { xf[i] = flip_sign(v, in.rot_signbits[i >> 5] >> (i & 31u), 0); };
+      if (norm) {
+        float ss = 0.f;
+        for (uint32_t i = tid; i < d_in; i += n_thr) {
+          float r = __half2float(in.x[i]);
+          if (in.x2) r = round_half(r + __half2float(in.x2[i]));
+          if (in.resid_out && store_resid) in.resid_out[i] = __float2half_rn(r);
+          xf[i] = r;
+          ss += r * r;
         }
         request();
+        const float inv = norm_scale(ss);
+        for (uint32_t i = tid; i < d_in; i += n_thr) put(i, round_half(xf[i] * inv * __half2float(in.norm_w[i])));
       } else {
-        auto put = [&](uint32_t i, float v) { xf[i] = flip_sign(v, in.rot_signbits[i >> 5] >> (i & 31u), 0); };
-        if (norm) {
-          float ss = 0.f;
-          for (uint32_t i = tid; i < d_in; i += n_thr) {
-            float r = __half2float(in.x[i]);
-            if (in.x2) r = round_half(r + __half2float(in.x2[i]));
-            if (in.resid_out && store_resid) in.resid_out[i] = __float2half_rn(r);
-            xf[i] = r;
-            ss += r * r;
-          }
-          request();
-          const float inv = norm_scale(ss);
-          for (uint32_t i = tid; i < d_in; i += n_thr) put(i, round_half(xf[i] * inv * __half2float(in.norm_w[i])));
-        } else {
-          for (uint32_t i = tid; i < d_in; i += n_thr)
-            put(i, silu ? silu_mul(__half2float(in.x2[i]), __half2float(in.x[i])) : __half2float(in.x[i]));
-          request();
-        }
+        for (uint32_t i = tid; i < d_in; i += n_thr)
+          put(i, silu ? silu_mul(__half2float(in.x2[i]), __half2float(in.x[i])) : __half2float(in.x[i]));
+        request();
       }
-      const RotBlock block = rot_block(table, in.rot_m, in.rot_k);
-      lds_barrier();
-      rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, table, block, in.rot_m < kRotOctetM);
-      lds_barrier();
     }
+    const RotBlock block = rot_block(table, in.rot_m, in.rot_k);
+    lds_barrier();
+    rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, table, block, in.rot_m < kRotOctetM);
+    lds_barrier();
 #pragma unroll 1
     for (uint32_t p = 0; p < passes; ++p) {
       const uint32_t blk = quad + p * quads;
@@ -501,24 +497,43 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
       float v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = 0.f;
-      const bool ok = blk < nb && sub < 3u;
-      const uint32_t at = blk * kDim + sub * 8u;
-      uint32_t *const xb = L.planes + plane_at<DIG>(blk), *const xs = L.planes + plane_sum_at<DIG>(blk);
-      if (in.x_f32) {
-        if (ok) {
+      if (blk < nb && sub < 3u) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = in.x_f32[at + j];
-        }
-        quantize_octet<DIG, true>(v, sub, xb, xs);
-      } else {
-        if (ok) {
+        for (int j = 0; j < 8; ++j) v[j] = xf[blk * kDim + sub * 8u + j];
+      }
+      quantize_octet<DIG, false>(v, sub, L.planes + plane_at<DIG>(blk), L.planes + plane_sum_at<DIG>(blk));
+    }
+    if (tid < tail_w) L.xtail[tid] = xf[nb * kDim + tid];
+  } else if constexpr (SRC == kSrcFinished) {
+    // Every value is asked for in front of the weights: loads come back in order.
+    struct __attribute__((packed, aligned(4))) Four { float v[4]; };
+    float v[PMAX][8] = {};
+    if (nb) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = xf[at + j];
+      for (int p = 0; p < PMAX; ++p) {
+        const uint32_t blk = quad + (uint32_t)p * quads, at = blk < nb && sub < 3u ? blk * kDim + sub * 8u : 0u;
+        const Four a = *reinterpret_cast<const Four*>(in.x_f32 + at), b = *reinterpret_cast<const Four*>(in.x_f32 + at + 4u);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[p][j] = a.v[j];
+          v[p][4 + j] = b.v[j];
         }
-        quantize_octet<DIG, false>(v, sub, xb, xs);
       }
     }
-    if (tid < tail_w) L.xtail[tid] = in.x_f32 ? in.x_f32[nb * kDim + tid] : xf[nb * kDim + tid];
+    const float t = in.x_f32[min(nb * kDim + tid, d_in - 1u)];
+    __builtin_amdgcn_sched_barrier(0);
+    request();
+    __builtin_amdgcn_sched_barrier(0);
+    zeros();
+#pragma unroll
+    for (int p = 0; p < PMAX; ++p) {
+      const uint32_t blk = quad + (uint32_t)p * quads;
+      if (blk >= pad) break;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[p][j] = blk < nb && sub < 3u ? v[p][j] : 0.f;
+      quantize_octet<DIG, true>(v[p], sub, L.planes + plane_at<DIG>(blk), L.planes + plane_sum_at<DIG>(blk));
+    }
+    if (tid < tail_w) L.xtail[tid] = t;
   } else {
     // One or two passes at a time, every operand requested before the first is used; a lane without columns reads the
     // row's first.  The norm's sum comes between two walks: the first leaves the summed values, as binary16, where the
@@ -1032,7 +1047,7 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
   lds_barrier();
 
   // (In a rotated basis there is no scalar register to keep it in: 2560 x 9728 takes 11.5 us like this, 11.8 with the argument.)
-  const uint32_t rounds = WIDE ? slots : SRC == kSrcRotated ? (a.n_tiles + n_teams - 1u) / n_teams : a.g.rounds;
+  const uint32_t rounds = WIDE ? slots : SRC == kSrcRotated && !GATED ? (a.n_tiles + n_teams - 1u) / n_teams : a.g.rounds;
   uint32_t slot = 0, step = w;  // (WIDE: every wavefront's first step is one of the first slot)
   for (uint32_t r0 = 0; r0 < rounds; r0 += batch) {
     const uint32_t r1 = min(r0 + batch, rounds), o_tile = finished(r0);
@@ -1099,11 +1114,20 @@ __device__ __forceinline__ void tiles_product(const GemvArgs& a) {
 template <typename OutT, int SRC, bool WIDE>
 __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvArgs a) { tiles_product<OutT, SRC, WIDE, false>(a); }
 // gate and up; y of the first matrix takes the result.
-__global__ __launch_bounds__(1024) void gated_product_kernel(GemvArgs a) { tiles_product<__half, kSrcAddRmsNorm, false, true>(a); }
+template <int SRC>
+__global__ __launch_bounds__(1024) void gated_product_kernel(GemvArgs a) { tiles_product<__half, SRC, false, true>(a); }
+__host__ inline const void* gated_kernel(bool rotated) {
+  return rotated ? reinterpret_cast<const void*>(gated_product_kernel<kSrcRotated>) : reinterpret_cast<const void*>(gated_product_kernel<kSrcAddRmsNorm>);
+}
+
+// of a finished activation
+template <typename OutT, bool WIDE>
+__global__ __launch_bounds__(1024) void finished_product_kernel(GemvArgs a) { tiles_product<OutT, kSrcFinished, WIDE, false>(a); }
 
 template <typename OutT, bool WIDE>
 __host__ const void* gemv_kernel_of(int src) {
   switch (src) {
+    case kSrcFinished: return reinterpret_cast<const void*>(finished_product_kernel<OutT, WIDE>);
     case kSrcF16: return reinterpret_cast<const void*>(gemv_tiles_kernel<OutT, kSrcF16, WIDE>);
     case kSrcRotated: return reinterpret_cast<const void*>(gemv_tiles_kernel<OutT, kSrcRotated, WIDE>);
     case kSrcSiluMul: return reinterpret_cast<const void*>(gemv_tiles_kernel<OutT, kSrcSiluMul, WIDE>);
@@ -1116,8 +1140,8 @@ __host__ inline const void* gemv_kernel(bool f32, int src, bool wide) {
 }
 template <class Fn>
 __host__ void for_each_gemv_kernel(Fn&& fn) {
-  fn(reinterpret_cast<const void*>(gated_product_kernel));
-  for (int src = kSrcF16; src <= kSrcAddRmsNorm; ++src)
+  for (int rotated = 0; rotated < 2; ++rotated) fn(gated_kernel(rotated != 0));
+  for (int src = kSrcF16; src <= kSrcFinished; ++src)
     for (int v = 0; v < 4; ++v) fn(gemv_kernel(v & 1, src, v & 2));
 }
 

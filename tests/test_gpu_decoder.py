@@ -849,6 +849,35 @@ def test_silu_formed_by_down_projections_launch(gpu_rt, orc, hidden, inter, rota
         dec.close()
 
 
+# Gate, up and down in rotated bases: silu(gate) up in their launch (groups of 1 x 256, 5 x 64, 1 x 1024; more pairs of tiles than a workgroup has
+# teams), down's activation by rotate_split_kernel (groups of 512, 1024, 2048 and 4096; one group; the most groups and tiles of sizes that are
+# products) and in its own launch below that and past it.
+@pytest.mark.parametrize("hidden,inter", [(256, 8704), (320, 9216), (256, 10240), (1024, 12288), (256, 20480), (256, 23552), (256, 14848), (320, 4096), (256, 8192)])
+def test_rotated_gate_up_and_wide_down(gpu_rt, orc, hidden, inter):
+    from oracle import qwen3_oracle
+
+    cfg = decoder.Qwen3Config(num_hidden_layers=2, hidden_size=hidden, num_attention_heads=4, num_key_value_heads=2, head_dim=32, intermediate_size=inter,
+                              vocab_size=100, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=16, tie_word_embeddings=True)
+    raws = decoder.synthetic_projections(cfg, inter)
+    for li, layer in enumerate(raws):
+        for i, seed in ((4, 7), (5, 7), (6, 9)):
+            layer[i].rotation_seed = 100 * li + seed
+    weights = decoder.synthetic_weights(cfg, inter)
+    dense = [[orc.read_matrix_raw(artifact.write_matrix_raw(m))[0].decode_matrix() for m in layer] for layer in raws]
+    ref, dec = qwen3_oracle.Qwen3Oracle(cfg, dense, weights), decoder.Decoder(gpu_rt, cfg, raws, weights)
+    try:
+        worst = 0.0
+        for t in np.random.default_rng(hidden + inter).integers(0, cfg.vocab_size, size=6):
+            want = ref.forward_token(int(t))
+            got, best = dec.forward_token(int(t))
+            assert best == int(np.argmax(got))
+            worst = max(worst, float(np.abs(got - want).max() / np.abs(want).max()))
+        print(f"OBSERVED rotated_wide_down {hidden}/{inter}: {worst:.3e}")
+        assert worst < BAR_SMALL
+    finally:
+        dec.close()
+
+
 # Rows long enough that a prompt's products are split over their columns: 43 and 42 blocks and 16 tail columns, 64 blocks and 8
 PARTS = decoder.Qwen3Config(num_hidden_layers=2, hidden_size=1032, num_attention_heads=8, num_key_value_heads=2, head_dim=128, intermediate_size=1544,
                             vocab_size=600, rope_theta=1e6, rms_norm_eps=1e-6, max_positions=210, tie_word_embeddings=True)

@@ -267,3 +267,9 @@ def test_rotation_of_every_kind_of_width(gpu_rt, orc, m, k):
 @pytest.mark.parametrize("n,rows", [(31 * 8, 300), (31 * 8, 700), (1024, 512), (3 * 128, 1000), (31 * 8, 1024), (31 * 8, 1025)])
 def test_many_rotated_rows_to_octets(gpu_rt, n, rows):
     test_rotated_rows_to_octets(gpu_rt, n, rows)
+
+
+# widths whose rotation goes to many workgroups (rot_split_pays): every m, few and many groups, one and several tiles a wavefront
+@pytest.mark.parametrize("m,k", [(512, 17), (512, 31), (1024, 11), (1024, 23), (2048, 7), (2048, 11), (4096, 3), (4096, 5)])
+def test_rotation_by_many_workgroups(gpu_rt, orc, m, k):
+    test_rotation_of_every_kind_of_width(gpu_rt, orc, m, k)
