@@ -296,7 +296,22 @@ __device__ __forceinline__ void lane_level(rot_acc_t& v, uint32_t lane) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = a[r];
 }
+// Where value p of a row under rotation is in LDS: at p, or PLACED.  A lane's results are four neighbours in each of several groups of 32 values, a lane's groups 128 bytes from the
+// next one's: eight lanes to a bank.  From m = 512 on, fours of a group change places by the group's number (bits 6 to 8 of p), so that sixteen
+// lanes have banks of their own; multiples of m, and of 1024, are added as they are.  (Two thirds of the LDS cycles of rotate_kernel were
+// conflicts: rotated q, k, v of 4096 columns at 64 rows 15.2 -> 15.0 us.  In the products' launches, all of whose workgroups do it, what it takes to find
+// the places is as long: 2560 x 2560 6.57 -> 6.54, 2560 x 320 5.54 -> 5.60.)
+template <bool PLACED>
+__device__ __forceinline__ uint32_t rot_place(uint32_t p, uint32_t m) { return PLACED && m >= 512u ? p ^ ((p >> 4) & 0x1Cu) : p; }
+// Eight values from p (a multiple of eight) on, PLACED.
+__device__ __forceinline__ void rot_octet(const float* v, uint32_t p, uint32_t m, float (&out)[8]) {
+  const uint32_t at = rot_place<true>(p, m);
+  const float4 a = *reinterpret_cast<const float4*>(v + at), b = *reinterpret_cast<const float4*>(v + (at ^ 4u));
+  out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
+  out[4] = b.x; out[5] = b.y; out[6] = b.z; out[7] = b.w;
+}
 // The levels below min(m, 1024) of a tile whose signed octets a lane holds (zeros past n), into LDS.
+template <bool PLACED>
 __device__ __forceinline__ void rotate_tile_to(float* v, const uint32_t (&x0)[4], const uint32_t (&x1)[4], const rot_h8_t (&h)[2], uint32_t tile,
                                                uint32_t n, uint32_t m, uint32_t k, float inv) {
   const uint32_t lane = threadIdx.x & 63u;
@@ -328,7 +343,7 @@ __device__ __forceinline__ void rotate_tile_to(float* v, const uint32_t (&x0)[4]
   if (m >= 1024u) {
     // Between the two rows of sixteen lanes results change places, eight against eight: a row has one eight of both, and forms its sums
     // (column below 16) and differences (that one and 16).
-    const uint32_t row = (lane >> 4) & 1u, at = tile * kRotTile + ((lane & 15u) ^ turned) * 32u + row * 16u + (lane >> 5) * 4u;
+    const uint32_t row = (lane >> 4) & 1u, at = rot_place<PLACED>(tile * kRotTile + ((lane & 15u) ^ turned) * 32u + row * 16u + (lane >> 5) * 4u, m);
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[r]), __float_as_uint(acc[r + 8]), false, false);
@@ -341,24 +356,24 @@ __device__ __forceinline__ void rotate_tile_to(float* v, const uint32_t (&x0)[4]
     }
 #pragma unroll
     for (uint32_t q = 0; q < 4u; ++q)  // (such a tile is whole)
-      *reinterpret_cast<float4*>(v + at + 8u * (q & 1u) + 512u * (q >> 1)) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+      *reinterpret_cast<float4*>(v + (at ^ 8u * (q & 1u)) + 512u * (q >> 1)) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
     return;
   }
   if (done) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] *= inv;
   }
-  const uint32_t at = tile * kRotTile + ((lane & 31u) ^ turned) * 32u + (lane >> 5) * 4u;
+  const uint32_t at = tile * kRotTile + ((lane & 31u) ^ turned) * 32u + (lane >> 5) * 4u, place = rot_place<PLACED>(at, m);
 #pragma unroll
   for (uint32_t q = 0; q < 4u; ++q)
-    if (at + 8u * q < n) *reinterpret_cast<float4*>(v + at + 8u * q) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+    if (at + 8u * q < n) *reinterpret_cast<float4*>(v + (place ^ 8u * q)) = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
 }
 // log2 R levels from 2^lg on, by all lanes: butterflies over R values 2^lg apart.
-template <uint32_t R>
-__device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t lg, float factor) {
+template <uint32_t R, bool PLACED>
+__device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t m, uint32_t lg, float factor) {
 #pragma unroll 1
   for (uint32_t p = threadIdx.x; p < n / R; p += 1024u) {
-    float* at = v + (p >> lg) * (R << lg) + (p & ((1u << lg) - 1u));
+    float* at = v + rot_place<PLACED>((p >> lg) * (R << lg) + (p & ((1u << lg) - 1u)), m);
     float r[R];
 #pragma unroll
     for (uint32_t i = 0; i < R; ++i) r[i] = at[i << lg];
@@ -379,7 +394,7 @@ __device__ __forceinline__ void rotate_levels(float* v, uint32_t n, uint32_t lg,
 // The k x k block of K x K numbers as products of scalars: a lane takes whole columns, or where there are fewer than lanes the
 // wavefronts share the rows of a column, and read it before any of them writes.  K * K multiply-adds a column, where the matrix cores
 // multiply 32 x 32: 5120 values, k = 5, 2.3 us of a launch with the latter.
-template <uint32_t K>
+template <uint32_t K, bool PLACED>
 __device__ __forceinline__ void rotate_columns(float* v, uint32_t m, const float* rows) {
   typedef const float __attribute__((address_space(4))) scalar_f;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lg = 31u - (uint32_t)__builtin_clz(m);
@@ -387,9 +402,10 @@ __device__ __forceinline__ void rotate_columns(float* v, uint32_t m, const float
   const uint32_t g0 = K * part / parts, g1 = K * (part + 1u) / parts;
 #pragma unroll 1
   for (uint32_t j = threadIdx.x & (m - 1u); j < m; j += 1024u) {
+    const uint32_t place = rot_place<PLACED>(j, m);
     float c[K];
 #pragma unroll
-    for (uint32_t i = 0; i < K; ++i) c[i] = v[i * m + j];
+    for (uint32_t i = 0; i < K; ++i) c[i] = v[i * m + place];
     if (parts > 1u) lds_barrier();
 #pragma unroll 1
     for (uint32_t g = g0; g < g1; ++g) {
@@ -397,7 +413,7 @@ __device__ __forceinline__ void rotate_columns(float* v, uint32_t m, const float
       float t = s[0] * c[0];
 #pragma unroll
       for (uint32_t i = 1; i < K; ++i) t = fmaf(s[i], c[i], t);
-      v[g * m + j] = t;
+      v[g * m + place] = t;
     }
   }
 }
@@ -422,6 +438,7 @@ __device__ __forceinline__ RotBlock rot_block(const RotTable* table, uint32_t m,
 }
 // What is left once the levels below 1024 are in LDS (every level, `put_levels`, where the octets were not taken): the values
 // are final after the caller's next barrier.  Called behind a barrier.
+template <bool PLACED>
 __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, uint32_t k, float inv, const RotTable* table, const RotBlock& B, bool put_levels) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
@@ -429,9 +446,9 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
   for (uint32_t lg = put_levels ? 0u : 31u - (uint32_t)__builtin_clz(kRotTile); (1u << lg) < m; lg += 3u) {
     const bool last = (8u << lg) >= m;
     const float factor = last && k == 1 ? inv : 1.f;
-    if ((m >> lg) >= 8u) rotate_levels<8>(v, n, lg, factor);
-    else if ((m >> lg) == 4u) rotate_levels<4>(v, n, lg, factor);
-    else rotate_levels<2>(v, n, lg, factor);
+    if ((m >> lg) >= 8u) rotate_levels<8, PLACED>(v, n, m, lg, factor);
+    else if ((m >> lg) == 4u) rotate_levels<4, PLACED>(v, n, m, lg, factor);
+    else rotate_levels<2, PLACED>(v, n, m, lg, factor);
     if (!last || k > 1) lds_barrier();
   }
   if (k == 1 && m == 1) {  // (a row of one value)
@@ -440,10 +457,10 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
   if (k == 1) return;
   if (rot_scalars(m, k)) {
     const float* rows = &table->rows[0][0];
-    if (k == 3u) rotate_columns<3>(v, m, rows);
-    else if (k == 5u) rotate_columns<5>(v, m, rows);
-    else if (k == 7u) rotate_columns<7>(v, m, rows);
-    else rotate_columns<9>(v, m, rows);
+    if (k == 3u) rotate_columns<3, PLACED>(v, m, rows);
+    else if (k == 5u) rotate_columns<5, PLACED>(v, m, rows);
+    else if (k == 7u) rotate_columns<7, PLACED>(v, m, rows);
+    else rotate_columns<9, PLACED>(v, m, rows);
     return;
   }
   // S (k x k, with the factor 1 / sqrt m) . C (k x m): a wavefront takes 32 columns of C at a time as f32 matrix-core
@@ -455,7 +472,7 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
     asm volatile("" : "+s"(k), "+s"(m));
     const uint32_t steps = (k + 1u) >> 1;  // k is odd: the last one has no row for the upper half
     const uint32_t j = tile * 32u + l32;
-    const float *at = v + (j < m ? j : 0u), *col = at + lh * m;
+    const float *at = v + rot_place<PLACED>(j < m ? j : 0u, m), *col = at + lh * m;
     rot_acc_t acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -478,7 +495,7 @@ __device__ __forceinline__ void rotate_rest(float* v, uint32_t n, uint32_t m, ui
     }
     // acc[r] is row 8 (r / 4) + 4 lh + r % 4 of column j
     if (j < m) {
-      float* out = v + j + lh * 4u * m;
+      float* out = v + rot_place<PLACED>(j, m) + lh * 4u * m;
 #pragma unroll
       for (uint32_t r = 0; r < 16; ++r) {
         const uint32_t g = 8u * (r >> 2) + (r & 3u);
@@ -582,14 +599,14 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
       for (uint32_t i = 0; i < 2u; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[i].w[j] = rot_octet_at(tile, i) < n ? flip_signs(o[i].w[j], sg[i], j) : 0u;
-      rotate_tile_to(rot_s, o[0].w, o[1].w, h, tile, n, m, k, a.inv);
+      rotate_tile_to<true>(rot_s, o[0].w, o[1].w, h, tile, n, m, k, a.inv);
     }
   } else {
     for (uint32_t i = tid; i < n; i += 1024) rot_s[i] = flip_sign(__half2float(x[i]), a.signbits[i >> 5] >> (i & 31u), 0);
   }
   const RotBlock block = rot_block(table, m, k);
   __syncthreads();
-  rotate_rest(rot_s, n, m, k, a.inv, table, block, m < kRotOctetM);
+  rotate_rest<true>(rot_s, n, m, k, a.inv, table, block, m < kRotOctetM);
   __syncthreads();
   constexpr bool kOctets = std::is_same<OutT, RotOctets>::value, kHalf = kOctets || std::is_same<OutT, __half>::value;
   typedef typename std::conditional<kHalf, __half, float>::type out_t;
@@ -598,9 +615,11 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
     if (kOctets || m >= kRotOctetM) {
       for (uint32_t i = tid * 8u; i < n; i += 8192) {
         HalfOctet o;
+        float v[8];
+        rot_octet(rot_s, i, m, v);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          o.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(rot_s[i + 2 * j])) | (uint32_t)__half_as_ushort(__float2half_rn(rot_s[i + 2 * j + 1])) << 16;
+          o.w[j] = (uint32_t)__half_as_ushort(__float2half_rn(v[2 * j])) | (uint32_t)__half_as_ushort(__float2half_rn(v[2 * j + 1])) << 16;
         if (kOctets && i < a.kcols) a.xt[(size_t)(i / 8u) * a.m_pad + row] = make_uint4(o.w[0], o.w[1], o.w[2], o.w[3]);
         else *reinterpret_cast<HalfOctet*>(out + i) = o;
       }
@@ -608,7 +627,7 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
     }
   }
   if constexpr (!kOctets)
-    for (uint32_t i = tid; i < n; i += 1024) out[i] = (out_t)rot_s[i];
+    for (uint32_t i = tid; i < n; i += 1024) out[i] = (out_t)rot_s[rot_place<true>(i, m)];
 }
 
 // One row by kRotSplit workgroups, f32.  Both factors of I_k (x) H_m mix a row's values by bits of their own: workgroup p makes the p-th

@@ -463,7 +463,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
           for (int j = 0; j < 4; ++j) x[i][j] = rot_octet_at(tile, i) < d_in ? flip_signs(a[i].w[j], sg[i], j) : 0u;
         }
         if ((tile + 16u) * kRotTile < d_in) load_tile(tile + 16u);  // (on their way beside this tile's levels)
-        rotate_tile_to(xf, x[0], x[1], h, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
+        rotate_tile_to<false>(xf, x[0], x[1], h, tile, d_in, in.rot_m, in.rot_k, in.rot_inv);
       }
       request();
     } else {
@@ -488,7 +488,7 @@ __device__ __forceinline__ void stage_x(const ActivationIn& in, uint32_t nb, uin
     }
     const RotBlock block = rot_block(table, in.rot_m, in.rot_k);
     lds_barrier();
-    rotate_rest(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, table, block, in.rot_m < kRotOctetM);
+    rotate_rest<false>(xf, d_in, in.rot_m, in.rot_k, in.rot_inv, table, block, in.rot_m < kRotOctetM);
     lds_barrier();
 #pragma unroll 1
     for (uint32_t p = 0; p < passes; ++p) {
