@@ -635,8 +635,8 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
 // the others, lane by lane, and the k x k block over the groups' values, which it has all of.
 // What bounds it is latency: the launch, a row's way from memory, three barriers; 3.4 to 4.2 us whatever the width.  In the product's launch, where
 // every workgroup does all of it, wide rows are several turns of what sixteen wavefronts can at once, and a k x k block past 9 is 32 x 32 on the
-// matrix cores: a rotated product of 2560 x 9728 takes 11.2 us there, 10.1 so; 5120 x 17408 19.7 and 16.6, 4096 x 20480 16.0 and 14.0, 4096 x 14336 13.0
-// and 12.1, 4096 x 11264 (k = 11) 12.9 and 10.6, 4096 x 8704 (k = 17) 10.6 and 9.9, 4096 x 12288 11.6 and 11.4.  Not 4096 x 10240 (k = 5), 10.4 in both, 4096 x 9216 (k = 9), 9.3
+// matrix cores: a rotated product of 2560 x 9728 takes 11.2 us there, 10.2 so; 5120 x 17408 19.7 and 16.7, 4096 x 20480 16.0 and 14.2, 4096 x 14336 13.0
+// and 12.4, 4096 x 11264 (k = 11) 12.9 and 10.7, 4096 x 8704 (k = 17) 10.6 and 10.0, 4096 x 12288 11.6 and 11.5.  Not 4096 x 10240 (k = 5), 10.4 in both, 4096 x 9216 (k = 9), 9.3
 // and 9.8, and 2560 x 5632 (k = 11), 8.8 in both.
 constexpr uint32_t kRotSplit = 32, kRotSplitTile = 512;  // workgroups; values of a wavefront
 __host__ inline bool rot_split_pays(uint32_t n, uint32_t m, uint32_t k) {  // (m, n: what the kernel is written for)
@@ -734,15 +734,28 @@ __global__ __launch_bounds__(1024) void rotate_split_kernel(RotArgs a) {
   } else {
     mixed[tid] = v;
     __syncthreads();
-    v = 0.f;
+    // Few terms in f64, many as four sums (0.1 us of a call): a rotated row is 6 to 28 % nearer to its values in 64 bits than one that a workgroup rotates by
+    // itself, ten widths from 8704 to 23552 (17408: 7.4e-8 of its norm, 8.9e-8 there); as one f32 chain it was up to 0.9 % further.
+    if (k <= kRotScalarK) {
+      double t = 0.;
 #pragma unroll
-    for (uint32_t q = 0; q < kRotKMax; q += 8u) {
-      if (q >= k) break;
-      float c[8];
+      for (uint32_t i = 0; i < kRotScalarK; ++i) {
+        if (i >= k) break;
+        t = fma((double)s[i], (double)mixed[(i << lg) + b], t);
+      }
+      v = (float)t;
+    } else {
+      float t[4] = {};
 #pragma unroll
-      for (uint32_t i = 0; i < 8u; ++i) c[i] = mixed[(min(q + i, k - 1u) << lg) + b];  // (past k: meets zeros)
+      for (uint32_t q = 0; q < kRotKMax; q += 8u) {
+        if (q >= k) break;
+        float c[8];
 #pragma unroll
-      for (uint32_t i = 0; i < 8u; ++i) v = fmaf(s[q + i], c[i], v);
+        for (uint32_t i = 0; i < 8u; ++i) c[i] = mixed[(min(q + i, k - 1u) << lg) + b];  // (past k: meets zeros)
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) t[i & 3u] = fmaf(s[q + i], c[i], t[i & 3u]);
+      }
+      v = (t[0] + t[1]) + (t[2] + t[3]);
     }
   }
   if (g < k) reinterpret_cast<float*>(a.out)[g * m + p * run + b] = v;
