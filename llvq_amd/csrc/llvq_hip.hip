@@ -217,10 +217,11 @@ __device__ __forceinline__ float half_hi(uint32_t w) { return __half2float(__ush
 // The rotation x' = (S (x) I_m)(I_k (x) H_m / sqrt m) D x of an activation of n = k m values, by a workgroup of 1024
 // lanes (llvq-quant/src/rotation.rs:97-105; f32 like the reference's device rotation, llvq-cuda/kernels/llvq_rot.cuh).
 //
-// Every workgroup of a batch-1 product rotates its own activation, and with sixteen wavefronts on a CU an instruction of
+// Every workgroup of a batch-1 product rotates its own activation (rows up to those of rot_split_pays), and with sixteen wavefronts on a CU an instruction of
 // each costs 7 ns: what bounds a rotation is their number.  (With a value per lane and load, lane exchanges through LDS and a
 // pass over LDS per level above 512 a 2560 x 9728 product took 19.2 us; with the levels at 48 instructions, sixteen wavefronts'
-// operands asked for where ten have any, and every k on the matrix cores 12.6; it takes 11.1, and 5120 x 5120 9.0 where it was 11.5.)  So:
+// operands asked for where ten have any, and every k on the matrix cores 12.6; 11.1 after that, and 5120 x 5120 8.2 where it was 11.5.  Rows as wide as the former are rotated by
+// rotate_split_kernel now, which has both times.)  So:
 //  * The five lowest levels are two matrix-core steps: what is rotated is binary16, the entries of H are 0 and +-1, so
 //    the products are exact and the sums f32, as butterflies would have them.  A wavefront takes 1024 values; a column of
 //    its 32 x 32 result is 32 neighbouring ones, requested by two lanes as two octets each (with their signs).
