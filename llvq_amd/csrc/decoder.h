@@ -707,13 +707,16 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
 // What bounds it: round trips to memory (operands and the first rows; partials, the counter and the partials again), so that the rest has to be
 // short.  On the vector ALUs a tile was 500 instructions at four query heads (each lane eight columns of a row for every head, sixteen-lane
 // sums of the scores); here scores are four matrix instructions (16 positions x 16 columns, of which the query heads take the
-// first) and the weighted sum of V eight, beside about 100 others (250 with an int8 cache).  The first product leaves a head's scores in the lanes that
-// the second takes its weights from: column lane % 16 is the head, 4 (lane / 16) + i the position.  V lies in a lane by rows, four of them, which
-// a byte permute turns into pairs of positions.  Weights keep their 24 bits: 2^14 times a weight is two binary16 terms, which are the two halves of one
-// instruction's contraction.  Maxima, sums and scores are f32; K, V and the rotated queries are binary16 values already.  Error
-// against 64 bits before the context is rounded, in the mean over 3 to 8100 positions, both caches: 1.11e-7; on the vector ALUs 1.14e-7.
-// Per launch, before -> now: 513 positions of a 4B layer 8.4 -> 6.8 us, 8100 of a 14B layer with an int8 cache 19.9 (4.7 of them a merge
-// launch) -> 11.0.
+// first), the weighted sum of V 32 for every four heads, beside about 130 others (280 with an int8 cache).  The first product leaves a head's scores in the lanes that
+// the second takes its weights from: column lane % 16 is head lane % (4 SETS), 4 (lane / 16) + i the position.  V lies in a lane by rows, four of them, eight columns each; in
+// the second product a position and column of a lane meet the weights of its four neighbours' heads (16 blocks of 4 heads x 4 columns, 8 cycles each), and every
+// quarter of the wavefront has the sums of its own positions until the range ends.  Weights, maxima, sums and scores are f32; K, V and the rotated queries are binary16
+// values already.  (Weights as two binary16 terms, of sixteen positions in one instruction, take 6.9 and 11.1 us where these take 7.4 and 12.6, but have no bits below 2^-38
+// of the largest, up to 18 % of weights of 2^-37, and where the second term is zero an infinite V is NaN.  f32 products with sixteen columns for the heads, of which
+// they are a quarter: 7.9 and 12.8.)  Relative error of the context against 64 bits before it is rounded, in the mean over 3 to 8100 positions, four to eight heads
+// and both caches: 1.46e-7; on the vector ALUs 1.58e-7.
+// Per launch, on the vector ALUs -> now: 513 positions of a 4B layer 8.3 -> 7.4 us, 8100 of a 14B layer with an int8 cache 19.9 (4.6 of them a merge
+// launch) -> 12.6.
 //
 // The workgroup that arrives last at the kv head's counter merges the ranges' partials in their order and rounds the context once;
 // partials go to memory and back at device scope (past the XCDs' own L2s), not between fences, which write back and empty an L2.
@@ -732,20 +735,19 @@ __host__ __device__ inline uint32_t decode_ranges(uint32_t T, uint32_t n_kv) {
 }
 constexpr uint32_t kDecodeCounter = 64;   // counters are lines of their own: 256 workgroups' additions to one line, behind each other, took 1.5 us
 
-template <bool Q8>
+// SETS: of up to four query heads each.
+template <bool Q8, int SETS>
 __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(AttnNew nw, const __half* __restrict__ kcache, const __half* __restrict__ vcache,
                                                                              KvQ8 q8, __half* __restrict__ ctx, float* part, uint32_t* __restrict__ counters,
                                                                              uint32_t groups, uint32_t chunk, uint32_t T, uint32_t max_pos, uint32_t n_splits) {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   typedef float f4 __attribute__((ext_vector_type(4)));
-  constexpr uint32_t D = 128, kThreads = kDecodeWaves * 64, kvgroups = D / kKvGroup;
-  constexpr uint32_t kQuarter = 32 + 4, kAccPitch = 4 * kQuarter + 4;  // a head's sums in LDS: four quarters of 32 columns, on banks of their own
+  constexpr uint32_t D = 128, kvgroups = D / kKvGroup;
   __shared__ __align__(16) __half qh[kDecodeMaxGroup][D + 8];  // the query heads, normed and rotated
   __shared__ __align__(16) __half knew[D], vnew[D];            // the new position's k and v, or their codes
   __shared__ uint32_t knew_s, knew_b, vnew_s, vnew_b;          // scales and biases of those, a group to a half
   __shared__ __align__(16) float wmax[kDecodeMaxGroup][kDecodeWaves], wsum[kDecodeMaxGroup][kDecodeWaves];
-  __shared__ __align__(16) float wacc[kDecodeWaves][kDecodeMaxGroup][kAccPitch];
+  __shared__ __align__(16) float wacc[kDecodeWaves][4 * SETS][D];
   __shared__ uint32_t arrived;
   const uint32_t kvh = blockIdx.y, split = blockIdx.x, tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -793,7 +795,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(Att
   const HeadOperands kop = head_operands_128(nw.k_raw + (size_t)kvh * D, nw.kn, lane, lane + 64u);
   const __half v1 = nw.v_raw[(size_t)kvh * D + lane], v2 = nw.v_raw[(size_t)kvh * D + lane + 64u];
   request(wave);
-  static_assert(kDecodeMaxGroup <= kDecodeWaves, "a query head to a wavefront");
+  static_assert(kDecodeMaxGroup <= kDecodeWaves && kDecodeMaxGroup <= 8, "a query head to a wavefront, two sets of them");
   if (wave < groups) {
     const float2 r = norm_rope_128(qop, angle, nw.eps);
     qh[wave][lane] = __float2half_rn(r.x);  // (exact)
@@ -837,11 +839,19 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(Att
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
     const uint32_t col = Q8 ? (quarter + 4u * (m >> 1)) * 16u + (m & 1) * 8u : (quarter + 4u * m) * 8u;
-    qf[m] = *reinterpret_cast<const h8*>(&qh[min(n16, groups - 1u)][col]);  // (columns past the heads: the last head again, not used)
+    qf[m] = *reinterpret_cast<const h8*>(&qh[min(n16 % (4u * SETS), groups - 1u)][col]);  // (past the heads: the last head again, not used)
   }
-  f4 acc[8];  // [t]: columns 8 (4 quarter + i) + t of head lane % 16
+  f4 acc[SETS][8];  // [set][t]: column 8 (lane % 16) + t of heads 4 set + i, of the lane's quarter's positions
 #pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+  for (int set = 0; set < SETS; ++set)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[set][t] = f4{0.f, 0.f, 0.f, 0.f};
+  // Of a value that lane has for head lane % (4 SETS), that of head 4 set + lane % 4.
+  const auto of_set = [](int set, float v) {
+    if constexpr (SETS == 1) return v;
+    const int b = __float_as_int(v);  // quads 1 and 3 take what is in those in front of them; 0 and 2 those behind
+    return __int_as_float(set == 0 ? __builtin_amdgcn_update_dpp(b, b, 0x114, 0xF, 0xA, false) : __builtin_amdgcn_update_dpp(b, b, 0x104, 0xF, 0x5, false));
+  };
   float m_run = -INFINITY, l_run = 0.f;  // the head's maximum so far; the lane's positions' sum of exponentials
   const auto lane_max = [](float v) {    // over the quarters
     auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -895,7 +905,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(Att
     // scores
     const f4 zero = {0.f, 0.f, 0.f, 0.f};
     f4 quad[4];  // (each from zero: one behind the other they round more, and wait for each other)
-    uint32_t va[8][2];  // [t]: column t of positions 0, 1 and of 2, 3
+    float va[4][8];  // [u][t]: column t of position u
     if constexpr (Q8) {
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
@@ -916,22 +926,20 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(Att
         fb[u] = __half2float(vb[u]);
       }
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        float v[4];
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = fmaf((float)(((t < 4 ? vraw[u].x : vraw[u].y) >> (8 * (t & 3))) & 0xFFu), fs[u], fb[u]);
-        va[t][0] = __builtin_bit_cast(uint32_t, (h2){(_Float16)v[0], (_Float16)v[1]});
-        va[t][1] = __builtin_bit_cast(uint32_t, (h2){(_Float16)v[2], (_Float16)v[3]});
-      }
+        for (int t = 0; t < 8; ++t) va[u][t] = kv_dequant(((t < 4 ? vraw[u].x : vraw[u].y) >> (8 * (t & 3))) & 0xFFu, fs[u], fb[u]);
     } else {
 #pragma unroll
       for (int m = 0; m < 4; ++m) quad[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kraw[m]), qf[m], zero, 0, 0, 0);
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const auto word = [&](int u) { return t < 2 ? vraw[u].x : t < 4 ? vraw[u].y : t < 6 ? vraw[u].z : vraw[u].w; };
-        const uint32_t pick = t & 1 ? 0x07060302u : 0x05040100u;
-        va[t][0] = __builtin_amdgcn_perm(word(1), word(0), pick);
-        va[t][1] = __builtin_amdgcn_perm(word(3), word(2), pick);
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t w[4] = {vraw[u].x, vraw[u].y, vraw[u].z, vraw[u].w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          va[u][2 * t] = half_lo(w[t]);
+          va[u][2 * t + 1] = half_hi(w[t]);
+        }
       }
     }
     if ((tile + kDecodeWaves) * kDecodeTile < nj) request(tile + kDecodeWaves);
@@ -947,35 +955,48 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(Att
       m_run = mn;
       l_run *= e0;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) acc[t] *= e0;
-    }
-    h8 pw;
+      for (int set = 0; set < SETS; ++set) {
+        const int b = __float_as_int(of_set(set, e0));
+        const f4 e = {__int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x00, 0xF, 0xF, false)), __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x55, 0xF, 0xF, false)),
+                      __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0xAA, 0xF, 0xF, false)), __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0xFF, 0xF, 0xF, false))};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float p = __builtin_amdgcn_exp2f(fmaf(s[i], kDecodeScale, -mn)), w = p * 16384.f;
+        for (int t = 0; t < 8; ++t) acc[set][t] *= e;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float p = __builtin_amdgcn_exp2f(fmaf(s[u], kDecodeScale, -mn));
       l_run += p;
-      pw[i] = (_Float16)w;
-      pw[4 + i] = (_Float16)(w - (float)pw[i]);
-    }
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const uint4 v = make_uint4(va[t][0], va[t][1], va[t][0], va[t][1]);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, v), pw, acc[t], 0, 0, 0);
+      for (int set = 0; set < SETS; ++set) {
+        const float ps = of_set(set, p);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) acc[set][t] = __builtin_amdgcn_mfma_f32_4x4x1f32(ps, va[u][t], acc[set][t], 0, 0, 0);
+      }
     }
   }
   // The wavefronts' results meet in LDS.  (One without a position: maximum -inf, weight 0.)
   const float l_all = lane_sum(l_run);
-  if (n16 < groups) {
-    if (quarter == 0) {
-      wmax[n16][wave] = m_run;
-      wsum[n16][wave] = l_all;
-    }
-    float* dst = &wacc[wave][n16][quarter * kQuarter];
+  if (n16 < groups && quarter == 0) {
+    wmax[n16][wave] = m_run;
+    wsum[n16][wave] = l_all;
+  }
+  // The quarters' sums meet by lane moves: a move across half the wavefront leaves each half two columns of four, one across a quarter each quarter one.
+  const auto quarters = [](float a, float b, float c, float d) {
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(c), false, false);
+    const float lo = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    p = __builtin_amdgcn_permlane32_swap(__float_as_uint(b), __float_as_uint(d), false, false);
+    const float hi = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    p = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *reinterpret_cast<float4*>(dst + 8 * i) = make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]);
-      *reinterpret_cast<float4*>(dst + 8 * i + 4) = make_float4(acc[4][i], acc[5][i], acc[6][i], acc[7][i]);
-    }
+  for (uint32_t g = 0; g < 4u * SETS; ++g) {
+    if (g >= groups) break;
+    const f4(&a)[8] = acc[g / 4u];
+    const uint32_t i = g % 4u;
+    const float x = quarters(a[0][i], a[2][i], a[4][i], a[6][i]), y = quarters(a[1][i], a[3][i], a[5][i], a[7][i]);
+    *reinterpret_cast<float2*>(&wacc[wave][g][n16 * 8u + quarter * 2u]) = make_float2(x, y);
   }
   __syncthreads();
   // ---- this workgroup's partial: the wavefronts merged in order, two neighbouring columns to a lane ----
@@ -994,16 +1015,16 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(Att
 #pragma unroll
     for (uint32_t k = 0; k < kDecodeWaves; ++k) {
       w[k] = w[k] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(w[k] - M);
-      const float2 a = *reinterpret_cast<const float2*>(&wacc[k][wave][quarter * kQuarter + n16 * 2u]);
+      const float2 a = *reinterpret_cast<const float2*>(&wacc[k][wave][lane * 2u]);
       L = fmaf(wsum[wave][k], w[k], L);
       A = fmaf(a.x, w[k], A);
       B = fmaf(a.y, w[k], B);
     }
     const uint32_t head = kvh * groups + wave;
     if (n_splits == 1u) {
-      reinterpret_cast<__half2*>(ctx + (size_t)head * D)[lane] = __floats2half2_rn(A * 0x1p-14f / L, B * 0x1p-14f / L);
+      reinterpret_cast<__half2*>(ctx + (size_t)head * D)[lane] = __floats2half2_rn(A / L, B / L);
     } else {
-      put(part + ((size_t)head * n_splits + split) * D + lane * 2u, A * 0x1p-14f, B * 0x1p-14f);
+      put(part + ((size_t)head * n_splits + split) * D + lane * 2u, A, B);
       if (lane == 0) put(part_ml + (head * n_splits + split) * 2u, M, L);  // (-inf for an empty range)
     }
   }

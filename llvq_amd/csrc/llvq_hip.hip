@@ -2401,7 +2401,9 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     nw.eps = d->eps;
     if (d->head_dim == 128u) {
       const uint32_t n = decode_ranges(T, d->n_kv);
-      hipLaunchKernelGGL(d->kv_q8 ? attn_decode_mfma_kernel<true> : attn_decode_mfma_kernel<false>, dim3(n, d->n_kv), dim3(kDecodeWaves * 64u), 0, st, nw, kc, vc, lq8, d->ctx,
+      const auto kernel = groups_per_kv <= 4u ? (d->kv_q8 ? attn_decode_mfma_kernel<true, 1> : attn_decode_mfma_kernel<false, 1>)
+                                              : (d->kv_q8 ? attn_decode_mfma_kernel<true, 2> : attn_decode_mfma_kernel<false, 2>);
+      hipLaunchKernelGGL(kernel, dim3(n, d->n_kv), dim3(kDecodeWaves * 64u), 0, st, nw, kc, vc, lq8, d->ctx,
                          d->attn_part, d->attn_counters, groups_per_kv, (T + n - 1u) / n, T, d->max_pos, n);
       return;
     }

@@ -12,7 +12,7 @@ reference's own runner comparison excuses, llvq-llm/src/bin/fusedrun.rs:263-278)
 import numpy as np
 import pytest
 
-from llvq_amd import artifact, decoder
+from llvq_amd import artifact, decoder, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -191,6 +191,54 @@ def test_decode_attention_at_every_length(gpu_rt, orc, heads, kv, kv_mode):
             want, got = ref.forward_token(int(t)), dec.forward_token(int(t))[0]
             # Both round at the same places, and the attention differs by 1e-6 before its result is rounded: a binary16 step of single logits is 1e-3.
             assert np.abs(got - want).max() < 1e-3 * np.abs(want).max(), n
+    finally:
+        dec.close()
+
+
+@pytest.mark.parametrize("kv_mode", ["f16", "q8"])
+def test_small_attention_weights_keep_their_bits(gpu_rt, orc, kv_mode):
+    """Positions with weights of 2^-37 to 2^-25 of the largest, which every sixteen positions have one of, and the only V that is not zero: the context is
+    theirs alone, 7e-6 to 0.01.  Every projection is tail columns, so that embeddings, queries, keys and values are exact: rows of 16 columns with a
+    single one become 4, heads are of equal magnitudes, and the frequencies of the upper 32 pairs turn nothing.  (Weights in steps of 2^-38 of the
+    largest were off by up to 18 %.)"""
+    from oracle import qwen3_oracle
+
+    hidden, hd, queries = 16, 128, 6
+    cfg = decoder.Qwen3Config(num_hidden_layers=1, hidden_size=hidden, num_attention_heads=1, num_key_value_heads=1, head_dim=hd, intermediate_size=24,
+                              vocab_size=16, rope_theta=1e30, rms_norm_eps=1e-6, max_positions=128, tie_word_embeddings=False, kv_mode=kv_mode)
+    dense = [np.zeros((do, di), np.float32) for _, do, di in cfg.shapes()]
+    slow = np.arange(hd) % 64 >= 32
+    dense[0][:] = 0.25
+    for c in range(queries):  # query token c differs from the small keys in 4 c of 64 signs less
+        dense[0][np.flatnonzero(slow)[: 2 * c], 1 + c] = -0.25
+    dense[1][:] = 0.25
+    dense[1][:, 0] = -0.25
+    dense[2][120:, 0] = 16000.0   # V of the small positions: 64000 in the columns that o_proj has as its tail
+    dense[3][15, 120:] = 1e4 / 8
+    raws = []
+    for m, (site, do, di) in zip(dense, cfg.shapes()):
+        r = synth.make_matrix(f"model.layers.0.{site}.weight", do, di, 3)
+        r.row_scales = np.full_like(r.row_scales, 1e-30)
+        r.tail = np.ascontiguousarray(m[:, di - di % 24:]).ravel()
+        raws.append(r)
+    one = np.ones((1, hidden), np.float16)
+    gains = np.where(slow, 1.0, 0.0).astype(np.float16)[None]
+    embed = np.eye(16, hidden, dtype=np.float16)
+    weights = decoder.DecoderWeights(one, one, gains, (2.25 * gains).astype(np.float16), one[0], embed, embed)
+    ref = qwen3_oracle.Qwen3Oracle(cfg, [[orc.read_matrix_raw(artifact.write_matrix_raw(r))[0].decode_matrix() for r in raws]], weights, kv_mode=kv_mode)
+    dec = decoder.Decoder(gpu_rt, cfg, [raws], weights)
+    try:
+        for i, t in enumerate(([1] + [0] * 15) * 6 + list(range(1, 1 + queries))):
+            with np.errstate(all="ignore"):  # (the first small position's result is past binary16, and nobody's but its own)
+                want = ref.forward_token(t)
+            got = dec.forward_token(t)[0]
+            if i < 96:
+                continue
+            # column 15 of the residual against the token's own, which is one: 10^4 times the context
+            ratio, mine = float(want[15]) / float(want[t]), float(got[15]) / float(got[t])
+            print(f"OBSERVED small_weights {kv_mode} {ratio / 1e4:.3e}: {mine / ratio - 1.0:.3e}")
+            # a binary16 step of the context (2^-24 of those below 2^-14), and of o_proj's result, the residual and two logits
+            assert abs(mine / ratio - 1.0) < 2.0 ** -24 / (ratio / 1e4) + 5 * 2.0 ** -11
     finally:
         dec.close()
 
