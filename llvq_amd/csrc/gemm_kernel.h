@@ -791,13 +791,11 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
     const uint32_t row = row0 + min(i * 64u + lane, 32u * RF - 1u);
     my_scale[i] = reinterpret_cast<const float*>(rec0 + record(row))[row & 15u];
   }
-  const uint32_t touched = *reinterpret_cast<const uint32_t*>(rec0 + record(t.row0 + min(tid / 9u, kRows / 16u - 1u) * 16u) + min(tid % 9u, (head >> 7) - 1u) * 128u);
+  uint32_t touched = 0;
+  if (a.tail_w) touched = *reinterpret_cast<const uint32_t*>(rec0 + record(t.row0 + min(tid / 9u, kRows / 16u - 1u) * 16u) + min(tid % 9u, (head >> 7) - 1u) * 128u);
   acc16_t acc[RF][CF];
   double sum[PAIR ? RF : 1][PAIR ? CF : 1][16];  // of the steps, with PAIR
   const float unit = table_unit(entry_f), table = entry_f * (1.f / unit);
-#pragma unroll
-  for (int i = 0; i < (RF + 1) / 2; ++i) asm volatile("" : "+v"(my_scale[i]));
-  asm volatile("" ::"v"(touched));
   const auto scale_of = [&](uint32_t meta) __attribute__((always_inline)) {
     return __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)meta, (int)__float_as_uint(table)));
   };
@@ -1110,6 +1108,12 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
     }
   }
   const bool any_left = __builtin_amdgcn_ballot_w64(left_steps != 0u) != 0u;
+  // The end's operands, behind the first steps' loads: what waits for the one waits for the other.  (In front of them these came a way from memory later.
+  // With that, and the tail operands read where there are none: 2612 x 672 at 96 rows 17.9 us with f32 results, 17.4 so, 1000 x 408 at 600 17.3 with binary16
+  // ones and 16.5, 12288 x 4096 at 512 65.3 and 64.7, 9728 x 2560 at 500 43.6 and 43.0.)
+#pragma unroll
+  for (int i = 0; i < (RF + 1) / 2; ++i) asm volatile("" : "+v"(my_scale[i]));
+  asm volatile("" ::"v"(touched));
   wide_wait<2 * kLoads>();
   lds_barrier();
   // A step from its tiles in LDS: the first, and with PAIR those that something was left of, whose first octet is unpacked already.
@@ -1302,7 +1306,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
         scale[k][4 * g + 2] = v.z;
         scale[k][4 * g + 3] = v.w;
       }
-      if constexpr (!PAIR) {
+      if (!PAIR && pairs) {
         const uint32_t row = wave * (32u * RF) + k * 32u + l32e;
         const float* at = w_tail + (row >> 4) * 64u * tail_depth(tail_w);
 #pragma unroll
@@ -1317,7 +1321,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
       decltype(to)::store(StoreAt{y, ld, mt * kCols + i / RF * 32u, a.M, from, t.d_out, turn_at}, i % RF, lane_e, v);
     };
     acc16_t before;
-    if constexpr (!PAIR) read_c(0);
+    if (!PAIR && pairs) read_c(0);
 #pragma unroll
     for (uint32_t i = 0; i < kFragments; ++i) {
       const uint32_t k = i % RF, c = i / RF;
@@ -1346,7 +1350,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
 #pragma unroll
         for (uint32_t j = 0; j < kPairs; ++j)
           if (j < pairs) v = __builtin_amdgcn_mfma_f32_32x32x2f32(tw[k][j], tx[j], v, 0, 0, 0);
-        if (k + 1u == (uint32_t)RF && c + 1u < (uint32_t)CF) read_c(c + 1u);
+        if (pairs && k + 1u == (uint32_t)RF && c + 1u < (uint32_t)CF) read_c(c + 1u);
         if (i) put(i - 1u, before);
         before = v;
         __builtin_amdgcn_sched_barrier(0);
