@@ -573,7 +573,8 @@ static_assert(gemm_small_lds<2, 4>() <= 160 * 1024, "partial sums of sixteen wav
 // A fragment's results on their way to y, ld values from an activation row's to the next: a lane has sixteen of one activation row (weight rows
 // 8 g + 4 h .. + 3, g < 4).  Where y and its rows lie on 16-byte boundaries they go through LDS (`turn`, a wavefront's own), so that a store
 // takes whole lines, eight lanes to a row: as the lanes have them a store is sixteen bytes each of 32 rows, and the partial results of a 4B layer's
-// products of 500 rows took 2 us longer each.  Else one by one.
+// products of 500 rows took 2 us longer each; f32 results without splits 12000 x 1000 at 600 rows 32.1 us and 30.6 so, 13000 x 408 at 600 21.9 and 20.6,
+// 12288 x 4096 at 512 and others of long rows the same.  Else one by one.
 // wave_lds_order: what a wavefront has read of LDS has come before it writes there, and the other way round.
 __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -602,6 +603,25 @@ struct StoreF32 {
       const float4 o = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(t.turn) + (i * 8u + r) * 36u + q * 4u);
       const uint32_t m = t.m + i * 8u + r;
       if (m < t.m_end) *reinterpret_cast<float4*>(reinterpret_cast<float*>(t.y) + (size_t)m * t.ld + t.row + k * 32u + q * 4u) = o;
+    }
+  }
+};
+// As the lanes have them, the halves exchanged so that a lane has eight rows in a row: binary16 results with PAIR, whose fragments are not converted and
+// stored beside each other's products, and wait for LDS by themselves.  (9728 x 700 at 350 rows 40.0 us through LDS, 39.5 so, at 90 38.8 and 38.2, 12288 x 4099 at 500 175.7
+// and 175.1, other shapes the same; f32 results take a whole microsecond more: 1000 x 409 at 600 29.9 and 30.8.)
+struct StoreF16Direct {
+  static __device__ __forceinline__ void store(const StoreAt& t, uint32_t k, uint32_t lane, const acc16_t& v) {
+    const uint32_t m = t.m + (lane & 31u), h = lane >> 5;
+    if (m >= t.m_end) return;
+    uint32_t p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = __builtin_bit_cast(uint32_t, half2_t{(_Float16)v[2 * i], (_Float16)v[2 * i + 1]});
+    _Float16* out = reinterpret_cast<_Float16*>(t.y) + (size_t)m * t.ld + t.row + k * 32u;
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+      const auto a = __builtin_amdgcn_permlane32_swap(p[2 * g], p[2 * g + 2], false, false);
+      const auto b = __builtin_amdgcn_permlane32_swap(p[2 * g + 1], p[2 * g + 3], false, false);
+      *reinterpret_cast<u32x4_t*>(out + (g + h) * 8u) = u32x4_t{a[0], b[0], a[1], b[1]};
     }
   }
 };
@@ -1365,7 +1385,7 @@ __device__ __forceinline__ void wide_product(const GemmArgs& a) {
     if (whole) finish(StoreF32<RF>{}, t.y, t.d_out, row0);
     else finish(StoreEach<float>{}, t.y, t.d_out, row0);
   } else {
-    if (whole) finish(StoreF16<RF>{}, t.y, t.d_out, row0);
+    if (whole) finish(typename std::conditional<PAIR, StoreF16Direct, StoreF16<RF>>::type{}, t.y, t.d_out, row0);
     else finish(StoreEach<_Float16>{}, t.y, t.d_out, row0);
   }
 }
