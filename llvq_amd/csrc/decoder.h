@@ -463,8 +463,8 @@ __global__ __launch_bounds__(64) void attn_rows_kernel(const __half* __restrict_
 //                    binary16 in the lanes that hold them (no cross-lane movement: the K
 //                    index of the product is permuted to match, V^T is stored in that order).
 // H sets of wavefronts walk every H-th tile each, and their sums are joined at the end: the walk is a chain (16 tiles for the last rows of a
-// 500-row prompt).  A workgroup takes G heads of a kv head's (blockIdx.x: the ceil(heads / G) of each kv head), all of them or, where that leaves
-// CUs idle, two.  500 rows of 32 heads: 31 us with one set, 22 with two, 17.5 with four and two heads to a workgroup (500 tokens of
+// 500-row prompt).  A workgroup takes G heads of a kv head's (blockIdx.x: the ceil(heads / G) of each kv head), all of them or two
+// (prompt_heads_by_two).  500 rows of 32 heads: 31 us with one set, 22 with two, 17.5 with four and two heads to a workgroup (500 tokens of
 // twelve 4B layers 2665 -> 2605 us).
 // Scores, maxima, sums and O stay in f32; the context is rounded once.  The next tile's K and
 // V rows are requested before the current tile is multiplied.  Positions past the pass's last
@@ -699,6 +699,22 @@ __global__ __launch_bounds__(G * H * 64) void attn_rows_mfma_kernel(const __half
     if (row_e < n_rows)
       for (uint32_t o = to.kcols / 8u + (lane_e >> 5); o < to.n_oct; o += 2u) to.xt[(size_t)o * to.m_pad + row_e] = make_uint4(0, 0, 0, 0);
   }
+}
+
+// Whether a prompt's workgroups take two query heads and the cache by four sets of wavefronts, where else they take all of a kv head's by two sets (one
+// past five heads).  Every workgroup brings a kv head's tiles to LDS for itself, so this pays where CUs would be idle, and where the walk is long enough for
+// four sets.  us a layer, all heads -> by two, binary16 and int8 caches:
+//   up to as many workgroups as CUs: 32 heads of 8, 500 rows at 0 95 -> 91, 102 -> 98, at 2000 154 -> 133, 178 -> 156, at 7600 315 -> 251, 388 -> 313; 40 heads
+//     of 8, 300 rows at 500 106 -> 96, 116 -> 105, 256 at 7600 352 -> 245, 431 -> 304; 64 of 8, 256 at 500 115 -> 98, 125 -> 105; 16 of 2, 500 at 0 96 -> 85, 102 -> 89;
+//   past that with three to five heads: 40 of 8, 340 rows at 0 92 -> 95, 98 -> 100, 500 at 3000 204 -> 224, 242 -> 276, at 7600 363 -> 422, 447 -> 540;
+//   with six to eight: 64 of 8, 300 rows at 0 96 -> 98, 102 -> 105, 400 104 -> 105, 112 -> 115, 500 112 -> 109, 120 -> 118, 300 at 500 118 -> 119, 129 -> 132, 500 135 -> 128,
+//     149 -> 145, at 3000 247 -> 231, 294 -> 285;
+//   up to 128 positions: 32 of 8, 24 rows at 0 47.7 -> 48.5, 52.9 -> 54.1, 64 53.5 -> 53.8, 55.5 -> 57.1; one and two heads 49.6 -> 50.7, 50.5 -> 51.5
+//     (130 rows at 0: within half a us of each other).
+inline bool prompt_heads_by_two(uint32_t n_kv, uint32_t groups, uint32_t row_blocks, uint32_t last_pos, uint32_t cus) {
+  if (last_pos < 128u) return false;
+  if (groups <= 2u || n_kv * ((groups + 1u) / 2u) * row_blocks <= cus) return true;
+  return groups > 5u && 2u * n_kv * row_blocks <= cus && last_pos >= 448u;
 }
 
 // Attention of one query position over the cache (model.rs:812-822), heads of 128: workgroup (range, kv head) takes the positions

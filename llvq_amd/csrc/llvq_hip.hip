@@ -2561,7 +2561,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
     const llvq_mat* const* P = d->proj.data() + (size_t)L * 7;
     const uint32_t grp = d->n_heads / d->n_kv;
     // 32 rows per workgroup on the matrix cores where the head width is the one that kernel is built for, the cache walked
-    // by two sets of wavefronts (more than five heads to a set leave it too few registers for that)
+    // by two sets of wavefronts, four of two heads each (more than five heads to a set leave it too few registers for a second)
     const bool on_mfma = d->head_dim == 128 && grp <= (uint32_t)kAttnMaxGroup;
     GemmSums qkv_sums{}, o_sums{};
     // residual + previous MLP branch, then the input norm (the branch of layer 0 is absent)
@@ -2593,8 +2593,7 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(kernel, agrid, dim3(64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->head_dim, d->pos, d->max_pos, scale);
     };
     const uint32_t row_blocks = (n + kAttnTile - 1) / kAttnTile;
-    // two heads to a workgroup where one for each kv head and 32 rows would leave half of the CUs without any
-    const bool by_two = grp > 2u && 2u * d->n_kv * row_blocks <= (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256);
+    const bool by_two = prompt_heads_by_two(d->n_kv, grp, row_blocks, d->pos + n - 1u, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256));
     auto attend_mfma = [&](auto kernel, uint32_t heads, uint32_t sets) {
       hipLaunchKernelGGL(kernel, dim3(d->n_kv * ((grp + heads - 1u) / heads), row_blocks), dim3(heads * sets * 64), 0, st, d->pq, kc, vc, lq8, d->pctx, d->n_heads, d->n_kv, d->pos, n, d->max_pos, scale, ctx_to);
     };
@@ -2603,7 +2602,8 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<true>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos, qkv_sums);
       if (on_mfma) {
-        if (grp <= 2 || by_two) attend_mfma(attn_rows_mfma_kernel<true, 2, 4>, 2, 4);
+        if (by_two) attend_mfma(attn_rows_mfma_kernel<true, 2, 4>, 2, 4);
+        else if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<true, 2, 2>, 2, 2);
         else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<true, 4, 2>, 4, 2);
         else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<true, 5, 2>, 5, 2);
         else attend_mfma(attn_rows_mfma_kernel<true, kAttnMaxGroup, 1>, kAttnMaxGroup, 1);
@@ -2615,7 +2615,8 @@ int decoder_prefill_pass(llvq_decoder* d, uint32_t n, bool want_logits, uint32_t
       hipLaunchKernelGGL(norm_rope_append_rows_kernel<false>, hgrid, dim3(256), 0, st, d->pq, d->pk, d->pv, nw, lq8, d->n_heads, d->n_kv,
                          d->head_dim, d->pos, d->max_pos, qkv_sums);
       if (on_mfma) {
-        if (grp <= 2 || by_two) attend_mfma(attn_rows_mfma_kernel<false, 2, 4>, 2, 4);
+        if (by_two) attend_mfma(attn_rows_mfma_kernel<false, 2, 4>, 2, 4);
+        else if (grp <= 2) attend_mfma(attn_rows_mfma_kernel<false, 2, 2>, 2, 2);
         else if (grp <= 4) attend_mfma(attn_rows_mfma_kernel<false, 4, 2>, 4, 2);
         else if (grp <= 5) attend_mfma(attn_rows_mfma_kernel<false, 5, 2>, 5, 2);
         else attend_mfma(attn_rows_mfma_kernel<false, kAttnMaxGroup, 1>, kAttnMaxGroup, 1);
