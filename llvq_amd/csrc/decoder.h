@@ -743,11 +743,15 @@ constexpr uint32_t kDecodeFetch = 32;   // ranges whose partials are asked for t
 // log2(e) / sqrt(128), to 9e-9 of itself: scores are exponents of two, with one rounding of a score's difference to the maximum where the scaled
 // score, the difference and __expf's product with log2(e) are three.
 constexpr float kDecodeScale = 0.127517432f;
-// Ranges of T positions: a tile to a wavefront, until the kv heads' workgroups fill a card of 256 CUs.  (513 positions of a 4B layer: 6.8 us with 128 a
-// range, 7.5 with 64, 7.8 with 256; 8100 of a 14B layer with an int8 cache: 11.0 us in 32 ranges, 12.4 in 16.)
-__host__ __device__ inline uint32_t decode_ranges(uint32_t T, uint32_t n_kv) {
-  const uint32_t n = (T + kDecodeTile * kDecodeWaves - 1u) / (kDecodeTile * kDecodeWaves), fill = (256u + n_kv - 1u) / n_kv;
-  return min(n, min(fill, (uint32_t)kAttnMaxSplits));
+// Ranges of T positions: a tile to a wavefront, until the kv heads' workgroups fill the CUs.  us a launch by the number of ranges, on 256 CUs (* the rule's):
+//   32 heads of 8, binary16       300: 1 7.3, 2 7.7, 3* 7.1, 8 6.6    1000: 4 8.4, 8* 7.1, 16 7.2, 32 8.7    4000: 8 11.2, 16 9.4, 32* 9.4, 64 16.6    8100: 16 12.4, 32* 12.2, 64 17.7
+//   40 heads of 8, int8           300: 1 10.6, 2 9.7, 3* 8.7, 8 7.7   1000: 4 11.1, 8* 8.8, 16 8.3, 32 9.4   4000: 8 16.2, 16 12.1, 32* 10.9, 64 21.3   8100: 16 17.0, 32* 13.8, 64 23.7
+//   8 heads of 1, binary16        300: 1 8.4, 2 8.8, 3* 8.2, 8 8.0    1000: 4 10.4, 8* 8.7, 16 8.6, 32 10.0  4000: 8 14.0, 16 11.3, 32* 11.2, 64 12.4   8100: 16 14.4, 32 12.6, 64* 13.0
+//   64 heads of 32, binary16      300: 1 6.9, 2 7.3, 3* 6.8, 8 7.4    1000: 4 8.6, 8* 7.8, 16 13.0, 32 22.0  4000: 4 16.9, 8* 14.9, 16 18.0
+// (One range has nobody to wait for: 130 positions 5.7 us in one and 7.0 in two.)
+inline uint32_t decode_ranges(uint32_t T, uint32_t n_kv, uint32_t cus) {
+  const uint32_t n = (T + kDecodeTile * kDecodeWaves - 1u) / (kDecodeTile * kDecodeWaves), fill = (cus + n_kv - 1u) / n_kv;
+  return std::min(n, std::min(fill, (uint32_t)kAttnMaxSplits));
 }
 constexpr uint32_t kDecodeCounter = 64;   // counters are lines of their own: 256 workgroups' additions to one line, behind each other, took 1.5 us
 

@@ -2400,7 +2400,7 @@ int decoder_step(llvq_decoder* d, bool want_logits, uint32_t history_slot, bool 
     nw.vcache = vc;
     nw.eps = d->eps;
     if (d->head_dim == 128u) {
-      const uint32_t n = decode_ranges(T, d->n_kv);
+      const uint32_t n = decode_ranges(T, d->n_kv, (uint32_t)(rt->cu_count > 0 ? rt->cu_count : 256));
       const auto kernel = groups_per_kv <= 4u ? (d->kv_q8 ? attn_decode_mfma_kernel<true, 1> : attn_decode_mfma_kernel<false, 1>)
                                               : (d->kv_q8 ? attn_decode_mfma_kernel<true, 2> : attn_decode_mfma_kernel<false, 2>);
       hipLaunchKernelGGL(kernel, dim3(n, d->n_kv), dim3(kDecodeWaves * 64u), 0, st, nw, kc, vc, lq8, d->ctx,
