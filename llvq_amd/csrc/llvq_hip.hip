@@ -632,7 +632,7 @@ __global__ __launch_bounds__(1024) void rotate_kernel(RotArgs a) {
 }
 
 // One row by kRotSplit workgroups, f32.  Both factors of I_k (x) H_m mix a row's values by bits of their own: workgroup p makes the p-th
-// m / 32 values of every group, all of H's five highest bits at once as the sums of its sign p over the row (every value of it, once), then
+// m / 32 values of every group (of three and more, by rot_split_pays), all of H's five highest bits at once as the sums of its sign p over the row (every value of it, once), then
 // the others, lane by lane, and the k x k block over the groups' values, which it has all of.
 // What bounds it is latency: the launch, a row's way from memory, three barriers; 3.4 to 4.2 us whatever the width.  In the product's launch, where
 // every workgroup does all of it, wide rows are several turns of what sixteen wavefronts can at once, and a k x k block past 9 is 32 x 32 on the
@@ -647,7 +647,7 @@ __host__ inline size_t rot_split_lds(uint32_t n, uint32_t m) { return (size_t)(n
 __global__ __launch_bounds__(1024) void rotate_split_kernel(RotArgs a) {
   extern __shared__ __align__(16) float part[];  // [tile][run]
   __shared__ float mixed[1024];
-  asm volatile("" ::"s"(a.x), "s"(a.out), "s"(a.signbits), "s"(a.fragments), "s"(a.n), "s"(a.m), "s"(a.k), "s"(a.inv));  // (all asked for at once)
+  asm volatile("" ::"s"(a.x), "s"(a.out), "s"(a.signbits), "s"(a.fragments), "s"(a.n), "s"(a.m), "s"(a.k));  // (all asked for at once)
   const uint32_t tid = threadIdx.x, lane = tid & 63u, n = a.n, m = a.m, k = a.k, p = blockIdx.x;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t run = m / kRotSplit, lg = 31u - (uint32_t)__builtin_clz(run), tiles = n / kRotSplitTile;  // run: 16 .. 128
@@ -663,18 +663,16 @@ __global__ __launch_bounds__(1024) void rotate_split_kernel(RotArgs a) {
   const uint32_t g = tid >> lg, b = tid & (run - 1u);  // the lane's result: value p * run + b of group g, where g < k
   const RotTable* table = reinterpret_cast<const RotTable*>(a.fragments);
   float s[kRotKMax];
-  if (k > 1u) {
 #pragma unroll
-    for (uint32_t lh = 0; lh < 2u; ++lh)
+  for (uint32_t lh = 0; lh < 2u; ++lh)
 #pragma unroll
-      for (uint32_t q = 0; q < 4u; ++q) {
-        const float4 f = *reinterpret_cast<const float4*>(table->lane[lh * 32u + (g & 31u)].s + 4u * q);
-        s[8 * q + lh] = f.x;
-        s[8 * q + 2 + lh] = f.y;
-        s[8 * q + 4 + lh] = f.z;
-        s[8 * q + 6 + lh] = f.w;
-      }
-  }
+    for (uint32_t q = 0; q < 4u; ++q) {
+      const float4 f = *reinterpret_cast<const float4*>(table->lane[lh * 32u + (g & 31u)].s + 4u * q);
+      s[8 * q + lh] = f.x;
+      s[8 * q + 2 + lh] = f.y;
+      s[8 * q + 4 + lh] = f.z;
+      s[8 * q + 6 + lh] = f.w;
+    }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (uint32_t i = 0; i < 4u; ++i) {
@@ -730,34 +728,30 @@ __global__ __launch_bounds__(1024) void rotate_split_kernel(RotArgs a) {
     level(64u, mixed[tid ^ 64u]);
     __syncthreads();
   }
-  if (k == 1u) {
-    v *= a.inv;
-  } else {
-    mixed[tid] = v;
-    __syncthreads();
-    // Few terms in f64, many as four sums (0.1 us of a call): a rotated row is 6 to 28 % nearer to its values in 64 bits than one that a workgroup rotates by
-    // itself, ten widths from 8704 to 23552 (17408: 7.4e-8 of its norm, 8.9e-8 there); as one f32 chain it was up to 0.9 % further.
-    if (k <= kRotScalarK) {
-      double t = 0.;
+  mixed[tid] = v;
+  __syncthreads();
+  // Few terms in f64, many as four sums (0.1 us of a call): a rotated row is 6 to 28 % nearer to its values in 64 bits than one that a workgroup rotates by
+  // itself, ten widths from 8704 to 23552 (17408: 7.4e-8 of its norm, 8.9e-8 there); as one f32 chain it was up to 0.9 % further.
+  if (k <= kRotScalarK) {
+    double t = 0.;
 #pragma unroll
-      for (uint32_t i = 0; i < kRotScalarK; ++i) {
-        if (i >= k) break;
-        t = fma((double)s[i], (double)mixed[(i << lg) + b], t);
-      }
-      v = (float)t;
-    } else {
-      float t[4] = {};
-#pragma unroll
-      for (uint32_t q = 0; q < kRotKMax; q += 8u) {
-        if (q >= k) break;
-        float c[8];
-#pragma unroll
-        for (uint32_t i = 0; i < 8u; ++i) c[i] = mixed[(min(q + i, k - 1u) << lg) + b];  // (past k: meets zeros)
-#pragma unroll
-        for (uint32_t i = 0; i < 8u; ++i) t[i & 3u] = fmaf(s[q + i], c[i], t[i & 3u]);
-      }
-      v = (t[0] + t[1]) + (t[2] + t[3]);
+    for (uint32_t i = 0; i < kRotScalarK; ++i) {
+      if (i >= k) break;
+      t = fma((double)s[i], (double)mixed[(i << lg) + b], t);
     }
+    v = (float)t;
+  } else {
+    float t[4] = {};
+#pragma unroll
+    for (uint32_t q = 0; q < kRotKMax; q += 8u) {
+      if (q >= k) break;
+      float c[8];
+#pragma unroll
+      for (uint32_t i = 0; i < 8u; ++i) c[i] = mixed[(min(q + i, k - 1u) << lg) + b];  // (past k: meets zeros)
+#pragma unroll
+      for (uint32_t i = 0; i < 8u; ++i) t[i & 3u] = fmaf(s[q + i], c[i], t[i & 3u]);
+    }
+    v = (t[0] + t[1]) + (t[2] + t[3]);
   }
   if (g < k) reinterpret_cast<float*>(a.out)[g * m + p * run + b] = v;
 }

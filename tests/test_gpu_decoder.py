@@ -898,8 +898,8 @@ def test_silu_formed_by_down_projections_launch(gpu_rt, orc, hidden, inter, rota
 
 
 # Gate, up and down in rotated bases: silu(gate) up in their launch (groups of 1 x 256, 5 x 64, 1 x 1024; more pairs of tiles than a workgroup has
-# teams), down's activation by rotate_split_kernel (groups of 512, 1024, 2048 and 4096; one group; the most groups and tiles of sizes that are
-# products) and in its own launch below that and past it.
+# teams), down's activation by rotate_split_kernel (groups of 512, 1024, 2048 and 4096, the most groups and tiles of sizes that are products) and in its
+# own launch: fewer columns than that pays for, and 8192 as one group.
 @pytest.mark.parametrize("hidden,inter", [(256, 8704), (320, 9216), (256, 10240), (1024, 12288), (256, 20480), (256, 23552), (256, 14848), (320, 4096), (256, 8192)])
 def test_rotated_gate_up_and_wide_down(gpu_rt, orc, hidden, inter):
     from oracle import qwen3_oracle

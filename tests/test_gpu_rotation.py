@@ -273,3 +273,17 @@ def test_many_rotated_rows_to_octets(gpu_rt, n, rows):
 @pytest.mark.parametrize("m,k", [(512, 17), (512, 31), (1024, 11), (1024, 23), (2048, 7), (2048, 11), (4096, 3), (4096, 5)])
 def test_rotation_by_many_workgroups(gpu_rt, orc, m, k):
     test_rotation_of_every_kind_of_width(gpu_rt, orc, m, k)
+
+
+# rows wider than a batch-1 product takes, rotated by themselves: as many tiles as the wavefronts' last turn begins with, and nearly all of it
+@pytest.mark.parametrize("m,k", [(4096, 7), (1024, 31)])
+def test_rotation_of_rows_past_the_products(gpu_rt, orc, m, k):
+    n = m * k
+    proj = gpu_rt.upload(_rotated(f"model.layers.0.rw{n}.weight", 16, n, 1, n))
+    x = synth.make_activation(n, seed=n)[0]
+    try:
+        got = gpu_rt.rotate(proj, _x16(x)).cpu().numpy().reshape(-1)
+        want = orc.Rotation(n, n).apply(x.astype(np.float64))
+        assert np.linalg.norm(got - want) <= (np.log2(m) + k + 2) * 2.0**-24 * np.linalg.norm(want)  # (as above)
+    finally:
+        gpu_rt.free(proj)
