@@ -243,6 +243,63 @@ def test_small_attention_weights_keep_their_bits(gpu_rt, orc, kv_mode):
         dec.close()
 
 
+def _attention_alone(gpu_rt, orc, heads, kv, head_dim, kv_mode, marked, seed):
+    """One layer whose logits are the attention's: embeddings are rows of the unit matrix, q, k and v tail columns (a token's 4 times the column, exactly), half
+    of every head's columns are ones that no position turns, the MLP is nothing and the head is the unit matrix.  marked: the positions that have a V, and what becomes of a single one of them
+    shows in the logits by its share."""
+    from oracle import qwen3_oracle
+
+    cfg = decoder.Qwen3Config(num_hidden_layers=1, hidden_size=16, num_attention_heads=heads, num_key_value_heads=kv, head_dim=head_dim, intermediate_size=24,
+                              vocab_size=16, rope_theta=1e30, rms_norm_eps=1e-6, max_positions=len(marked), tie_word_embeddings=False, kv_mode=kv_mode)
+    rng = np.random.default_rng(seed)
+    raws = []
+    for i, (site, do, di) in enumerate(cfg.shapes()):
+        r = synth.make_matrix(f"model.layers.0.{site}.weight", do, di, seed)
+        if i < 2:
+            r.tail = rng.choice(np.float32([-0.25, 0.25]), size=r.tail.size)
+        elif i == 2:
+            r.tail = rng.standard_normal((do, di)).astype(np.float32)
+            r.tail[:, 0] = 0.0
+            r.tail = r.tail.ravel()
+        elif i == 3:
+            r.row_scales, r.tail = r.row_scales * 64.0, r.tail * 512.0
+        else:
+            r.row_scales, r.tail = r.row_scales * 1e-20, r.tail * 0.0
+        raws.append(r)
+    one, gains = np.ones((1, 16), np.float16), np.where(np.arange(head_dim) % (head_dim // 2) >= head_dim // 4, 1.5, 0.0).astype(np.float16)[None]
+    eye = np.eye(16, dtype=np.float16)
+    weights = decoder.DecoderWeights(one, one, gains, gains, one[0], eye, eye)
+    dense = [[orc.read_matrix_raw(artifact.write_matrix_raw(r))[0].decode_matrix() for r in raws]]
+    dec = decoder.Decoder(gpu_rt, cfg, [raws], weights, prefill_rows=512)
+    tokens = np.where(marked, rng.integers(1, 16, size=len(marked)), 0)
+    return dec, qwen3_oracle.Qwen3Oracle(cfg, dense, weights, kv_mode=kv_mode), tokens
+
+
+def _worst_of_last(dec, ref, tokens, first):
+    """A batched prompt of `first` tokens, then the others one by one: the largest difference of their logits from the oracle's."""
+    try:
+        ref.prefill_rows(tokens[:first])
+        dec.prefill(tokens[:first], want_logits=False)
+        worst = 0.0
+        for t in tokens[first:]:
+            want, (got, _) = ref.forward_token(int(t)), dec.forward_token(int(t))
+            worst = max(worst, float(np.abs(got - want).max() / np.abs(want).max()))
+        return worst
+    finally:
+        dec.close()
+
+
+@pytest.mark.parametrize("heads,kv,kv_mode,first", [(5, 1, "f16", 1018), (4, 2, "f16", 4090), (5, 1, "q8", 4090)])
+def test_long_caches_of_heads_of_64(gpu_rt, orc, heads, kv, kv_mode, first):
+    """Heads of another width than 128, whose decode attention is attn_decode_kernel: where its ranges go to attn_merge_kernel (past 1024 positions; 17
+    ranges, and 64), and past 4096, where a range has a 65th position and its classes a second batch.  The positions that have a V are those, and
+    the last twelve (without one of them the logits move by 2 % in the median)."""
+    at = np.arange(first + 12)
+    worst = _worst_of_last(*_attention_alone(gpu_rt, orc, heads, kv, 64, kv_mode, (at % 65 == 64) | (at >= first), 33), first)
+    print(f"OBSERVED heads_of_64 {heads}/{kv}/{kv_mode}/{first}: {worst:.3e}")
+    assert worst < 2e-3
+
+
 def test_long_cache_takes_the_merge_kernel(gpu_rt, orc):
     """Past 1024 cached positions the attention partials (more than 16 ranges of 64) are merged
     by a kernel of their own; the logits must keep agreeing with the oracle across the switch."""
