@@ -300,6 +300,19 @@ def test_long_caches_of_heads_of_64(gpu_rt, orc, heads, kv, kv_mode, first):
     assert worst < 2e-3
 
 
+@pytest.mark.parametrize("heads,kv,kv_mode,first,last", [(128, 128, "f16", 254, 290), (128, 128, "q8", 254, 290), (160, 32, "f16", 1028, 1042), (160, 32, "q8", 1028, 1042)])
+def test_decode_attention_past_a_tile_for_every_wavefront(gpu_rt, orc, heads, kv, kv_mode, first, last):
+    """Kv heads enough that the ranges are as many as the CUs take (two, eight) before every wavefront has a tile of sixteen positions: the first ones
+    have a second tile, loaded over the first's registers, in which some heads' maxima rise, and the new position is its first row, one in its
+    middle, its last (every one of them at two ranges), with the rows behind it past the range.  All positions have a V (without one the logits move by
+    7e-3 in the median), or those around the beginning of a second tile and the last (6 %)."""
+    at = np.arange(last)
+    marked = at >= 0 if kv == 128 else (at % 129 >= 126) | (at >= first)
+    worst = _worst_of_last(*_attention_alone(gpu_rt, orc, heads, kv, 128, kv_mode, marked, 33), first)
+    print(f"OBSERVED second_tiles {heads}/{kv}/{kv_mode}: {worst:.3e}")
+    assert worst < 2e-3
+
+
 def test_long_cache_takes_the_merge_kernel(gpu_rt, orc):
     """Past 1024 cached positions the attention partials (more than 16 ranges of 64) are merged
     by a kernel of their own; the logits must keep agreeing with the oracle across the switch."""
