@@ -1104,10 +1104,10 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void attn_decode_mfma_kernel(Att
 // four classes meet by lane moves, the wavefronts in LDS, and the workgroup
 // leaves an unnormalised partial per query head.  The workgroup that arrives
 // last at the kv head's counter merges the partials in split order and rounds
-// the context once.  At the lengths of a chat (one batch of rows per class) a
+// the context once (past 16 ranges attn_merge_kernel does).  At the lengths of a chat (one batch of rows per class) a
 // launch is a chain of round trips: operands and rows, partials to memory, the
-// counter, partials from memory.  So all operands of the new position's heads
-// are requested in front of the rows, and partials are stored and loaded at
+// counter, partials from memory.  So the first rows are requested in front of the
+// work on the new position's heads, and partials are stored and loaded at
 // device scope (past the XCDs' own L2s) instead of between fences, which write
 // back and empty an L2.  Scores, softmax and sums stay in
 // f32.  head_dim <= 128, a multiple of 8; G >= query heads per kv head sizes

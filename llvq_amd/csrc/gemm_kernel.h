@@ -1470,7 +1470,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_pair_kernel(GemmArgs a) {
   }
 }
 
-// The partial results of the column splits (each has its row scale, the last the tail columns), added in order, where no launch behind the
+// The partial results of the column splits (each has its row scale and its share of the tail columns), added in order, where no launch behind the
 // product takes them as they are (GemmSums).  A lane takes four weight rows of kSumM activation rows, kReduceSplits splits at a time.  (The launch that
 // also had scales and tails to see to took 8.8 us for 500 rows of 2560; 6000 x 1000 at 130 rows 28.1 -> 25.4 us, 4096 x 4096 at 300 33.8 -> 32.1.)
 constexpr uint32_t kSumM = 2;

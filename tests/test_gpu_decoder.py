@@ -337,7 +337,7 @@ def test_long_cache_takes_the_merge_kernel(gpu_rt, orc):
 def test_context_of_8192_positions_int8_cache(gpu_rt):
     """BASELINE config 4's regime for the attention: an int8 KV cache filled to 8192 positions, heads of
     128, 5 query heads per kv head (a small model otherwise, so that the oracle can follow).  The cache is
-    filled once position by position (split-KV attention over up to 64 ranges and the merge kernel) and once
+    filled once position by position (split-KV attention over up to 64 ranges, merged in the launch) and once
     by the batched path (matrix-core attention over up to 256 cache tiles, int8 rows rebuilt in LDS); the
     logits of the last prompt position and of six more positions are compared with the oracle's, which are
     a fixture (tests/golden/qwen3_small_q8kv_8192_logits.npz, written by make_long_context_logits.py: the
@@ -379,9 +379,9 @@ def test_context_of_8192_positions_int8_cache(gpu_rt):
 
 def test_config4_as_stated_14b_int8_cache_8192_positions(gpu_rt):
     """BASELINE config 4 as stated, in one run: the 40-layer model at the Qwen3-14B widths (280 LLVQ
-    matrices, 3.3 GB of codes resident), int8 KV cache, batch 1 at 8186+ cached positions — past 1024
-    positions the split attention leaves more than 16 partials per head, so the chip-wide merge kernel is
-    the path taken at every decoded position here.  The CPU oracle cannot follow at this size (hours), so
+    matrices, 3.3 GB of codes resident), int8 KV cache, batch 1 at 8186+ cached positions, where the decode
+    attention has as many ranges as the CUs take (32 of two tiles to every wavefront, merged in its own launch).
+    The CPU oracle cannot follow at this size (hours), so
     the checks are properties the reference states for its own cache (llvq-llm/tests/kv_cache.rs:222-262:
     split prefill == whole prefill; llvq-llm/src/bin/run.rs:4-7: cached generation is repeatable):
       * the cache filled by the batched path in passes of 512 rows and in passes of 384 rows gives the same
@@ -601,9 +601,8 @@ def test_prompt_attention_on_the_matrix_cores(gpu_rt, orc, heads, kv, kv_mode, s
 @pytest.mark.parametrize("heads,kv,kv_mode", [(4, 2, "f16"), (8, 2, "q8"), (10, 2, "f16"), (8, 1, "q8")])
 def test_attention_where_its_split_turns(gpu_rt, orc, heads, kv, kv_mode):
     """Prompts that end a row block or a cache tile, one short of it and one past it (an odd count of tiles leaves the second
-    set of wavefronts one that is masked whole), and decoded positions where another range begins (64, 128) and where the
-    ranges leave the merge inside the launch (1024): the prompt path against the position-by-position path, whose
-    attention kernels share nothing."""
+    set of wavefronts one that is masked whole), from 129 positions on by two heads and four sets of wavefronts; and decoded positions, where
+    another range begins every 128: the prompt path against the position-by-position path, whose attention kernels share nothing."""
     cfg = _wide(heads, kv, kv_mode)
     cfg.max_positions = 1040
     dec, _ = _build(gpu_rt, orc, cfg, 21, prefill_rows=512)
@@ -693,7 +692,7 @@ def test_config4_widths_and_context_against_the_oracle(gpu_rt):
     heads over 8 kv heads of 128, 17 408-wide down_proj rows — the lean-image kernel variant), int8 KV cache, 8192
     cached positions; 2 layers and a vocabulary of 2048 so that the oracle can follow (its logits are the fixture
     tests/golden/qwen3_14b_widths_q8kv_8192_logits.npz, written by make_config4_logits.py).  The device fills the
-    cache position by position (split-KV attention over 64 ranges and the merge kernel) and by the batched path
+    cache position by position (split-KV attention over up to 32 ranges, merged in the launch) and by the batched path
     (512 rows a pass); the logits of the last prompt position and of six more are compared.  Bar: 1e-3 of the
     largest logit, i.e. one binary16 step: logits are binary16 values on both sides, a step of the largest one is
     between 4.9e-4 and 9.8e-4 of it, and a different summation order can move a logit across one rounding boundary
